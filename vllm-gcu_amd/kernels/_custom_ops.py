@@ -8,6 +8,13 @@ extension has defined the name already (the reference's ``findSchema`` guard,
 torch_bindings.cpp:114-117); the implementation is registered for the GPU
 dispatch key ("CUDA" is the HIP device on PyTorch-ROCm).  Every implementation
 converts tensors to raw pointers and calls the C ABI of ``libmi355q.so``.
+
+The operators without a weight (norms, activations, quantisers, routing, sums)
+are implemented natively (csrc/host/activation_ops.cpp).  For the ones with a
+weight the wrappers and the quantization methods first offer their operands to
+``_runtime.host`` (csrc/host/module.cpp), which runs them when the kernels can
+read them as they are and returns None otherwise; the functions here convert,
+check and raise.
 """
 from typing import List, Optional, Tuple
 
@@ -21,8 +28,6 @@ from .quantization import rearrange
 
 # start of the shared scratch reserved for arrival counters (they must stay zero between launches)
 _WS_COUNTER_BYTES = 1 << 20
-
-_lib.load()          # fail at import time when the HIP library is missing
 
 _libs = {
     "_C": torch.library.Library("_C", "FRAGMENT"),
@@ -40,11 +45,19 @@ def _schema_exists(qualname: str) -> bool:
         return False
 
 
-def _register(ns: str, name: str, schema: str, fn, tags=()):
+def _register(ns: str, name: str, schema: str, fn=None, tags=()):
+    """``fn`` None: the implementation is native and registered at the end of this module."""
     SCHEMAS[f"{ns}::{name}"] = name + schema
     if not _schema_exists(f"{ns}::{name}"):
         _libs[ns].define(name + schema, tags=tags)
-    _libs[ns].impl(name, fn, "CUDA")
+    if fn is not None:
+        _libs[ns].impl(name, fn, "CUDA")
+
+
+def eager() -> bool:
+    """Whether a call may go straight to the native host path: not while a graph is being traced, where the
+    operator itself has to be seen."""
+    return not torch.compiler.is_compiling()
 
 
 # ---------------------------------------------------------------------------
@@ -134,6 +147,10 @@ def w4a16_gemm(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     """out[M, N] = x[M, K] @ dequant(qweight) (+ bias); allocates the output
     like gptq_gemm_gcu (csrc/src/gptq_gemm_gcu.cpp:35) unless the caller brings
     a contiguous ``out [M, N]`` of the activation dtype."""
+    if not (split_k or family) and out is None:
+        fast = rt.host.w4a16(x, qweight, zeros, scales, None, bias, int(group_size))
+        if fast is not None:
+            return fast
     rt.require_gpu(x, qweight, scales, zeros, bias)
     if x.dim() < 1:
         raise RuntimeError(f"w4a16_gemm expects activations [.., K], got {tuple(x.shape)}")
@@ -223,6 +240,10 @@ _register("_C", "awq_gemm_gcu",
 # for scales / zeros are swapped relative to the schema, positions are kept)
 def awq_gemm_gcu(input: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Tensor,
                  scales: torch.Tensor, split_k_iters: int, bias=None, group_size=128) -> torch.Tensor:
+    if eager():
+        out = rt.host.w4a16(input, qweight, scales, qzeros, None, bias, group_size)
+        if out is not None:
+            return out
     return torch.ops._C.awq_gemm_gcu(input, qweight, qzeros, scales, split_k_iters, bias, group_size)
 
 
@@ -238,6 +259,10 @@ def gptq_gemm_gcu(a: torch.Tensor, b_q_weight: torch.Tensor, b_gptq_qzeros: torc
                   group_size=128) -> torch.Tensor:
     assert bit in [4, 8]
     if bit == 4:
+        if eager():
+            out = rt.host.w4a16(a, b_q_weight, b_gptq_qzeros, b_gptq_scales, b_g_idx, bias, group_size)
+            if out is not None:
+                return out
         out_shape = a.shape[:-1] + (b_q_weight.shape[-1],)
         reshaped_a = a.reshape(-1, a.shape[-1])
         output = torch.ops._C.gptq_gemm_gcu(reshaped_a, b_q_weight, b_gptq_qzeros, b_gptq_scales,
@@ -263,32 +288,6 @@ def _gptq_gemm_gcu_fake(a, b_q_weight, b_gptq_qzeros, b_gptq_scales, b_g_idx, bi
 # W8A8 int8 (csrc/torch_bindings.cpp:734-766, 1002-1019)
 # ---------------------------------------------------------------------------
 _INT8_STREAM_MAX_M = 64      # measured on MI355X (K 8192, N 28672): 40-51 us against 90 us for the MFMA tile kernel
-
-
-def _int8_stream_rows(K: int, N: int) -> int:
-    """Up to how many rows the weight-streaming kernel takes a kslab layer (measured on MI355X, us,
-    streaming / MFMA tile kernel).  The streaming kernel gives a layer of few columns 32 or 16 columns per
-    workgroup, so every CU streams a share; the tile kernel's wavefronts without rows only copy, and on
-    layers of at most 128 column tiles it cuts K into ranges that fill the chip.  The streaming kernel's
-    time grows with the rows (in steps at 17, 33), the split tile kernel's hardly does: they cross at
-    25..32 rows behind a very long K -- 28672 x 8192: M = 24 45.4 / 50.5, M = 32 51.5 / 50.7, M = 64 67.1 / 49.7;
-    at 33..40 where K >= 2 N -- 16384 x 7168: M = 32 26.2 / 29.6, M = 40 31.0 / 30.3; 14336 x 4096: M = 32 19.5 / 20.1,
-    M = 40 24.4 / 20.2; at 41..48 for other K >= 7168 -- 7168 x 4096: M = 40 14.9 / 15.9, M = 48 16.2 / 16.1;
-    8192 x 8192: M = 48 19.5 / 21.3, M = 64 23.0 / 22.0; on wide layers (128 column tiles or more, no split)
-    -- 8192 x 28672: M = 40 49.8 / 52.3, M = 48 51.9 / 49.1; a short K stays with the streaming kernel --
-    4096 x 4096: M = 64 13.4 / 15.6."""
-    top = _INT8_STREAM_MAX_M
-    if N % 128 != 0:
-        return top
-    if N >= 128 * 128:
-        return top * 5 // 8
-    if K >= 24576:
-        return top * 3 // 8
-    if K >= 2 * N and K >= 7168:
-        return top // 2
-    if K >= 7168:
-        return top * 5 // 8
-    return top
 
 
 def _int8_weight_nk(weight: torch.Tensor):
@@ -347,7 +346,7 @@ def _scaled_int8_mm(out, x, weight, x_scale, w_scale, bias, acc_out=None):
             bias = bias.to(torch.float32)
             bias_f32 = 1
         bias = bias.contiguous()
-    stream_rows = _int8_stream_rows(K, N)
+    stream_rows = rt.host.int8_stream_rows(K, N, _INT8_STREAM_MAX_M)
     # (row-major [N, K] weights: the tile kernel with its K ranges is level with the streaming kernel on
     # large layers -- 8192 x 28672 at M = 16: 54 against 58 us -- and behind it on small ones up to 32
     # rows: 4096 x 4096 at M = 16: 13.8 against 7.7 us)
@@ -441,37 +440,6 @@ def _dot_bias_quant_impl(out, lhs, rhs, scale, bias):
     _scaled_int8_mm(out, lhs, rhs, None, scale, bias)
 
 
-def _dynamic_scaled_int8_quant_impl(output, input, scales, azp):
-    rt.require_gpu(output, input, scales)
-    if azp is not None:
-        raise RuntimeError("dynamic_scaled_int8_quant: asymmetric quantisation (azp) is not supported")
-    if input.numel() == 0:
-        return
-    x = input.contiguous()
-    K = x.shape[-1]
-    M = x.numel() // K
-    if not output.is_contiguous() or not scales.is_contiguous() or scales.dtype != torch.float32:
-        raise RuntimeError("dynamic_scaled_int8_quant: output and fp32 scales must be contiguous")
-    with torch.cuda.device(x.device):
-        _lib.call("mi355q_dynamic_int8_quant", output.data_ptr(), scales.data_ptr(), x.data_ptr(), M, K,
-                  rt.dtype_code(x.dtype), 0, rt.stream_ptr())
-
-
-def _static_scaled_int8_quant_impl(result, input, scale, azp):
-    rt.require_gpu(result, input, scale)
-    if input.numel() == 0:
-        return
-    x = input.contiguous()
-    K = x.shape[-1]
-    M = x.numel() // K
-    sc = scale.to(torch.float32).reshape(-1).contiguous()
-    if sc.numel() not in (1, K):
-        raise RuntimeError(f"static_scaled_int8_quant: scale must have 1 or K={K} entries, got {sc.numel()}")
-    with torch.cuda.device(x.device):
-        _lib.call("mi355q_static_int8_quant", result.data_ptr(), x.data_ptr(), sc.data_ptr(),
-                  int(sc.numel() > 1), M, K, rt.dtype_code(x.dtype), rt.stream_ptr())
-
-
 _register("_C", "cutlass_scaled_mm",
           "(Tensor! out, Tensor x, Tensor weight, Tensor x_scale, Tensor w_scale, Tensor? bias) -> ()",
           _cutlass_scaled_mm_impl, tags=(torch.Tag.flexible_layout,))
@@ -480,9 +448,9 @@ _register("_C", "dot_bias_quant", "(Tensor! out, Tensor lhs, Tensor rhs, Tensor 
 # `azp` is a plain Tensor in the reference's schema and Python passes None for
 # it (modular_experts.py:246); when this module owns the schema it is optional
 _register("_C", "dynamic_scaled_int8_quant",
-          "(Tensor! output, Tensor input, Tensor! scales, Tensor? azp) -> ()", _dynamic_scaled_int8_quant_impl)
+          "(Tensor! output, Tensor input, Tensor! scales, Tensor? azp) -> ()")
 _register("_C", "static_scaled_int8_quant",
-          "(Tensor! result, Tensor input, Tensor scale, Tensor? azp) -> ()", _static_scaled_int8_quant_impl)
+          "(Tensor! result, Tensor input, Tensor scale, Tensor? azp) -> ()")
 
 
 def scaled_int8_quant(input: torch.Tensor, scale: Optional[torch.Tensor] = None,
@@ -525,112 +493,27 @@ def int8_gemm_accumulators(x: torch.Tensor, weight: torch.Tensor) -> torch.Tenso
 # MoE routing / align (csrc/torch_bindings.cpp:803-809, 1052-1063, 1178-1189,
 # 1390-1431)
 # ---------------------------------------------------------------------------
-def _topk_softmax_impl(topk_weights, topk_indices, token_expert_indices, gating_output):
-    rt.require_gpu(topk_weights, topk_indices, token_expert_indices, gating_output)
-    if gating_output.numel() == 0:
-        return
-    g = gating_output.contiguous()
-    M, E = g.shape
-    k = topk_weights.shape[-1]
-    if topk_weights.dtype != torch.float32 or topk_indices.dtype != torch.int32:
-        raise RuntimeError("topk_softmax: topk_weights must be float32 and topk_indices int32")
-    if not (topk_weights.is_contiguous() and topk_indices.is_contiguous()):
-        raise RuntimeError("topk_softmax: outputs must be contiguous")
-    tei = token_expert_indices
-    if tei is not None and (tei.dtype != torch.int32 or not tei.is_contiguous()):
-        raise RuntimeError("topk_softmax: token_expert_indices must be contiguous int32")
-    with torch.cuda.device(g.device):
-        _lib.call("mi355q_topk_softmax", topk_weights.data_ptr(), topk_indices.data_ptr(), rt.ptr(tei),
-                  g.data_ptr(), M, E, k, 0, rt.dtype_code(g.dtype), rt.stream_ptr())
-
-
-def _fused_grouped_topk_impl(topk_weights, topk_ids, gating_output, topk, renormalize, num_expert_group,
-                             topk_group, e_score_correction_bias, scoring_func):
-    rt.require_gpu(topk_weights, topk_ids, gating_output, e_score_correction_bias)
-    if gating_output.numel() == 0:
-        return
-    if scoring_func not in ("softmax", "sigmoid"):
-        raise RuntimeError(f"fused_grouped_topk: unsupported scoring function {scoring_func!r}")
-    g = gating_output.contiguous()
-    M, E = g.shape
-    bias = e_score_correction_bias
-    if bias is not None:
-        bias = bias.to(torch.float32).contiguous()
-    if topk_weights.dtype != torch.float32 or topk_ids.dtype != torch.int32:
-        raise RuntimeError("fused_grouped_topk: topk_weights must be float32 and topk_ids int32")
-    with torch.cuda.device(g.device):
-        _lib.call("mi355q_grouped_topk", topk_weights.data_ptr(), topk_ids.data_ptr(), g.data_ptr(),
-                  rt.ptr(bias), M, E, int(topk), int(bool(renormalize)), int(num_expert_group),
-                  int(topk_group), int(scoring_func == "sigmoid"), rt.dtype_code(g.dtype), rt.stream_ptr())
-
-
-def _align(topk_ids, valid_rows, num_experts, block_size, expert_map, sorted_token_ids, experts_ids,
-           num_tokens_post_pad):
-    rt.require_gpu(topk_ids, valid_rows, expert_map, sorted_token_ids, experts_ids, num_tokens_post_pad)
-    ids = topk_ids.contiguous()
-    if ids.dtype not in (torch.int32, torch.int64):
-        raise RuntimeError(f"moe_align_block_size: topk_ids must be int32 or int64, got {ids.dtype}")
-    numel = ids.numel()
-    top = ids.shape[-1] if ids.dim() > 1 else 1
-    cap = numel + num_experts * (block_size - 1)
-    if sorted_token_ids.numel() < cap or experts_ids.numel() < cap // block_size:
-        raise RuntimeError("moe_align_block_size: output buffers are smaller than "
-                           "numel + num_experts * (block_size - 1)")
-    for t in (sorted_token_ids, experts_ids, num_tokens_post_pad):
-        if t.dtype != torch.int32 or not t.is_contiguous():
-            raise RuntimeError("moe_align_block_size: outputs must be contiguous int32")
-    if valid_rows is not None and valid_rows.dtype != torch.int32:
-        valid_rows = valid_rows.to(torch.int32)
-    if expert_map is not None:
-        expert_map = expert_map.to(torch.int32).contiguous()
-    with torch.cuda.device(ids.device):
-        _lib.call("mi355q_moe_align_block_size", ids.data_ptr(), int(ids.dtype == torch.int64), numel, top,
-                  rt.ptr(valid_rows), int(num_experts), int(block_size), rt.ptr(expert_map),
-                  sorted_token_ids.data_ptr(), experts_ids.data_ptr(), num_tokens_post_pad.data_ptr(),
-                  rt.stream_ptr())
-
-
-def _moe_align_block_size_impl(topk_ids, num_experts, block_size, sorted_token_ids, experts_ids,
-                               num_tokens_post_pad):
-    _align(topk_ids, None, num_experts, block_size, None, sorted_token_ids, experts_ids, num_tokens_post_pad)
-
-
-def _moe_align_block_size_pad_impl(topk_ids, topk_ids_size, num_experts, block_size, sorted_token_ids,
-                                   experts_ids, num_tokens_post_pad):
-    _align(topk_ids, topk_ids_size, num_experts, block_size, None, sorted_token_ids, experts_ids,
-           num_tokens_post_pad)
-
-
-def _exts_moe_align_block_size_impl(sorted_token_ids, experts_ids, num_tokens_post_pad, topk_ids,
-                                    real_token_num, expert_map, num_experts, block_size):
-    _align(topk_ids, real_token_num, num_experts, block_size, expert_map, sorted_token_ids, experts_ids,
-           num_tokens_post_pad)
-
-
 _register("_moe_C", "topk_softmax",
-          "(Tensor! topk_weights, Tensor! topk_indices, Tensor! token_expert_indices, Tensor gating_output) -> ()",
-          _topk_softmax_impl)
+          "(Tensor! topk_weights, Tensor! topk_indices, Tensor! token_expert_indices, Tensor gating_output) -> ()")
 # e_score_correction_bias is a plain Tensor in the reference and Python passes
 # None (fused_moe.py:256-266); optional where this module owns the schema
 _register("_C", "fused_grouped_topk",
           "(Tensor! topk_weights, Tensor! topk_ids, Tensor gating_output, SymInt topk, bool renormalize, "
-          "SymInt num_expert_group, SymInt topk_group, Tensor? e_score_correction_bias, str scoring_func) -> ()",
-          _fused_grouped_topk_impl)
+          "SymInt num_expert_group, SymInt topk_group, Tensor? e_score_correction_bias, str scoring_func) -> ()")
 _register("_moe_C", "moe_align_block_size",
           "(Tensor topk_ids, int num_experts, int block_size, Tensor! sorted_token_ids, Tensor! experts_ids, "
-          "Tensor! num_tokens_post_pad) -> ()", _moe_align_block_size_impl)
+          "Tensor! num_tokens_post_pad) -> ()")
 _register("_moe_C", "sgl_moe_align_block_size",
           "(Tensor topk_ids, int num_experts, int block_size, Tensor! sorted_token_ids, Tensor! experts_ids, "
-          "Tensor! num_tokens_post_pad) -> ()", _moe_align_block_size_impl)
+          "Tensor! num_tokens_post_pad) -> ()")
 # registered from a C++ function pointer in the reference, hence positional-only
 # callers (torch_bindings.cpp:803-809, moe_align_block_size_pad.cpp:43-47)
 _register("_C", "moe_align_block_size_pad",
           "(Tensor topk_ids, Tensor topk_ids_size, int num_experts, int block_size, Tensor! sorted_token_ids, "
-          "Tensor! experts_ids, Tensor! num_tokens_post_pad) -> ()", _moe_align_block_size_pad_impl)
+          "Tensor! experts_ids, Tensor! num_tokens_post_pad) -> ()")
 _register("_C", "exts_moe_align_block_size",
           "(Tensor(a!) sorted_token_ids, Tensor(a!) experts_ids, Tensor(a!) num_tokens_post_pad, Tensor topk_ids, "
-          "Tensor real_token_num, Tensor expert_map, int num_experts, int block_size) -> ()",
-          _exts_moe_align_block_size_impl)
+          "Tensor real_token_num, Tensor expert_map, int num_experts, int block_size) -> ()")
 
 
 def topk_softmax(topk_weights, topk_ids, token_expert_indices, gating_output) -> None:
@@ -640,6 +523,10 @@ def topk_softmax(topk_weights, topk_ids, token_expert_indices, gating_output) ->
 def fused_topk(hidden_states: torch.Tensor, gating_output: torch.Tensor, topk: int, renormalize: bool):
     """vLLM's ``fused_topk`` as used by ``FusedMoE.select_experts``
     (moe_wna16.py:612-623): softmax -> top-k (descending) -> optional renorm."""
+    if eager():
+        routed = rt.host.fused_topk(gating_output, topk, bool(renormalize))
+        if routed is not None:
+            return routed
     M = gating_output.shape[0]
     topk_weights = torch.empty(M, topk, dtype=torch.float32, device=gating_output.device)
     topk_ids = torch.empty(M, topk, dtype=torch.int32, device=gating_output.device)
@@ -685,189 +572,25 @@ def moe_align_block_size_pad(topk_ids, topk_ids_size, num_experts, block_size, s
 # activation glue (csrc/torch_bindings.cpp:163-175, 291, 714-766, 1083-1153,
 # 1404-1410)
 # ---------------------------------------------------------------------------
-def _rows_last(t: torch.Tensor):
-    return t.numel() // t.shape[-1], t.shape[-1]
-
-
-def _silu_and_mul_common(out, input, size, rows_per_count=1):
-    rt.require_gpu(out, input, size)
-    if input.numel() == 0:
-        return
-    x = input.contiguous()
-    rows, d2 = _rows_last(x)
-    if not out.is_contiguous() or out.shape[-1] * 2 != d2 or out.dtype != x.dtype:
-        raise RuntimeError("silu_and_mul: out must be contiguous [..., d] of the input dtype for input [..., 2d]")
-    with torch.cuda.device(x.device):
-        _lib.call("mi355q_silu_and_mul", out.data_ptr(), x.data_ptr(), rows, d2 // 2, rt.dtype_code(x.dtype),
-                  rt.ptr(size), rows_per_count, rt.stream_ptr())
-
-
-def _silu_and_mul_impl(result, input):
-    _silu_and_mul_common(result, input, None)
-
-
-def _leading_rows_to_flat(t: torch.Tensor, size: torch.Tensor):
-    """``size`` counts entries of the leading dimension (tokens); the kernels work on rows flattened
-    over every dimension but the last.  -> (count tensor, rows per counted entry): the product is
-    taken inside the kernel, so a captured graph whose count tensor is rewritten between replays
-    sees the new value."""
-    if size.dtype != torch.int32:
-        size = size.to(torch.int32)
-    lead = t.shape[0]
-    inner = (t.numel() // t.shape[-1]) // max(lead, 1)
-    return size, max(int(inner), 1)
-
-
-def _silu_and_mul_pad_impl(out, input, size):
-    _silu_and_mul_common(out, input, *_leading_rows_to_flat(input, size))
-
-
-def _fp8_out_ok(out, shape):
-    if out.dtype not in (torch.float8_e4m3fn, torch.uint8) or not out.is_contiguous() or tuple(out.shape) != tuple(shape):
-        raise RuntimeError(f"fp8 output must be a contiguous float8_e4m3fn tensor of shape {tuple(shape)}")
-
-
-def _group_quant_common(out, scale, input, real_size, group_size, fuse, rows_per_count=1):
-    rt.require_gpu(out, scale, input, real_size)
-    if input.numel() == 0:
-        return
-    x = input.contiguous()
-    rows, kin = _rows_last(x)
-    K = kin // 2 if fuse else kin
-    _fp8_out_ok(out, x.shape[:-1] + (K,))
-    if scale.dtype != torch.float32 or not scale.is_contiguous() or scale.numel() != rows * (K // group_size):
-        raise RuntimeError("per-token-group quant: scale must be contiguous float32 [..., K / group_size]")
-    if real_size is not None and real_size.dtype != torch.int32:
-        real_size = real_size.to(torch.int32)
-    with torch.cuda.device(x.device):
-        _lib.call("mi355q_fp8_group_quant", out.data_ptr(), scale.data_ptr(), x.data_ptr(), rows, K,
-                  int(group_size), int(fuse), rt.dtype_code(x.dtype), rt.ptr(real_size), rows_per_count,
-                  rt.stream_ptr())
-
-
-def _dynamic_per_token_group_fp8_quant_impl(out, scale, input, group_size):
-    _group_quant_common(out, scale, input, None, group_size, False)
-
-
-def _dynamic_per_token_group_fp8_quant_with_size_impl(out, scale, input, real_size, group_size):
-    cnt, rpc = _leading_rows_to_flat(input, real_size)
-    _group_quant_common(out, scale, input, cnt, group_size, False, rpc)
-
-
-def _silu_mul_per_token_group_quant_impl(out, scale, input, group_size):
-    _group_quant_common(out, scale, input, None, group_size, True)
-
-
-def _silu_mul_per_token_group_quant_with_size_impl(out, scale, input, size, group_size):
-    cnt, rpc = _leading_rows_to_flat(input, size)
-    _group_quant_common(out, scale, input, cnt, group_size, True, rpc)
-
-
-def _dynamic_per_token_scaled_fp8_quant_impl(result, input, scale, scale_ub):
-    # scale_ub is ignored, as in the reference (dynamic_per_token_scaled_fp8_quant.cpp:32-34)
-    rt.require_gpu(result, input, scale)
-    if input.numel() == 0:
-        return
-    x = input.contiguous()
-    rows, K = _rows_last(x)
-    _fp8_out_ok(result, x.shape)
-    with torch.cuda.device(x.device):
-        _lib.call("mi355q_fp8_token_quant", result.data_ptr(), scale.data_ptr(), x.data_ptr(), rows, K,
-                  rt.dtype_code(x.dtype), 0, rt.stream_ptr())
-
-
-def _static_fp8_common(out, input, scale, real_rows, fuse, rows_per_count=1):
-    rt.require_gpu(out, input, scale, real_rows)
-    if input.numel() == 0:
-        return
-    x = input.contiguous()
-    rows, kin = _rows_last(x)
-    K = kin // 2 if fuse else kin
-    _fp8_out_ok(out, x.shape[:-1] + (K,))
-    sc = scale.to(torch.float32).reshape(-1)
-    if sc.numel() != 1:
-        raise RuntimeError("static fp8 quant takes a single scale")
-    with torch.cuda.device(x.device):
-        _lib.call("mi355q_fp8_static_quant", out.data_ptr(), x.data_ptr(), sc.data_ptr(), rows, K, int(fuse),
-                  rt.dtype_code(x.dtype), rt.ptr(real_rows), rows_per_count, rt.stream_ptr())
-
-
-def _static_scaled_fp8_quant_impl(result, input, scale):
-    _static_fp8_common(result, input, scale, None, 0)
-
-
-def _silu_mul_static_fp8_quant_impl(out, input, scale, real_num_tokens):
-    cnt, rpc = _leading_rows_to_flat(input, real_num_tokens)
-    _static_fp8_common(out, input, scale, cnt, 1, rpc)
-
-
-def _mul_static_fp8_quant_impl(out, input, scale, real_num_tokens):
-    cnt, rpc = _leading_rows_to_flat(input, real_num_tokens)
-    _static_fp8_common(out, input, scale, cnt, 2, rpc)
-
-
-def _silu_mul_static_int8_quant_impl(result, input, scale):
-    # csrc/src/silu_mul_static_int8_quant.cpp:11-28: a 0-d scale is per tensor,
-    # anything else per channel of the gated half
-    rt.require_gpu(result, input, scale)
-    if input.numel() == 0:
-        return
-    x = input.contiguous()
-    rows, kin = _rows_last(x)
-    d = kin // 2
-    if result.dtype != torch.int8 or tuple(result.shape) != tuple(x.shape[:-1]) + (d,) or not result.is_contiguous():
-        raise RuntimeError(f"silu_mul_static_int8_quant: result must be contiguous int8 {tuple(x.shape[:-1]) + (d,)}")
-    sc = scale.to(torch.float32).reshape(-1).contiguous()
-    if sc.numel() not in (1, d):
-        raise RuntimeError(f"silu_mul_static_int8_quant: scale must have 1 or {d} entries, got {sc.numel()}")
-    with torch.cuda.device(x.device):
-        _lib.call("mi355q_silu_mul_static_int8_quant", result.data_ptr(), x.data_ptr(), sc.data_ptr(),
-                  int(sc.numel() > 1), rows, d, rt.dtype_code(x.dtype), rt.stream_ptr())
-
-
-def _moe_sum_pad_impl(out, input, size, dim, keepdim):
-    rt.require_gpu(out, input, size)
-    if input.numel() == 0:
-        return
-    if input.dim() != 3 or dim != 1 or keepdim:
-        raise RuntimeError("moe_sum_pad: expects input [M, topk, K], dim=1, keepdim=False")
-    x = input.contiguous()
-    M, T, K = x.shape
-    if not out.is_contiguous() or tuple(out.shape) != (M, K):
-        raise RuntimeError("moe_sum_pad: out must be contiguous [M, K]")
-    with torch.cuda.device(x.device):
-        _lib.call("mi355q_moe_sum", out.data_ptr(), x.data_ptr(), M, T, K, rt.dtype_code(x.dtype),
-                  rt.dtype_code(out.dtype), rt.ptr(None if size is None else size.to(torch.int32)),
-                  rt.stream_ptr())
-
-
-_register("_C", "silu_and_mul", "(Tensor! result, Tensor input) -> ()", _silu_and_mul_impl)
-_register("_C", "silu_and_mul_pad", "(Tensor(a!) out, Tensor input, Tensor size) -> ()", _silu_and_mul_pad_impl)
+_register("_C", "silu_and_mul", "(Tensor! result, Tensor input) -> ()")
+_register("_C", "silu_and_mul_pad", "(Tensor(a!) out, Tensor input, Tensor size) -> ()")
 _register("_C", "dynamic_per_token_group_fp8_quant",
-          "(Tensor! out, Tensor! scale, Tensor input, int group_size) -> ()",
-          _dynamic_per_token_group_fp8_quant_impl)
+          "(Tensor! out, Tensor! scale, Tensor input, int group_size) -> ()")
 _register("_C", "dynamic_per_token_group_fp8_quant_with_size",
-          "(Tensor! out, Tensor! scale, Tensor input, Tensor real_size, int group_size) -> ()",
-          _dynamic_per_token_group_fp8_quant_with_size_impl)
+          "(Tensor! out, Tensor! scale, Tensor input, Tensor real_size, int group_size) -> ()")
 _register("_C", "silu_mul_per_token_group_quant",
-          "(Tensor! out, Tensor! scale, Tensor input, int group_size) -> ()", _silu_mul_per_token_group_quant_impl)
+          "(Tensor! out, Tensor! scale, Tensor input, int group_size) -> ()")
 _register("_C", "silu_mul_per_token_group_quant_with_size",
-          "(Tensor(a!) out, Tensor(a!) scale, Tensor input, Tensor size, int group_size) -> ()",
-          _silu_mul_per_token_group_quant_with_size_impl)
+          "(Tensor(a!) out, Tensor(a!) scale, Tensor input, Tensor size, int group_size) -> ()")
 _register("_C", "dynamic_per_token_scaled_fp8_quant",
-          "(Tensor! result, Tensor input, Tensor! scale, Tensor? scale_ub) -> ()",
-          _dynamic_per_token_scaled_fp8_quant_impl)
-_register("_C", "static_scaled_fp8_quant", "(Tensor! result, Tensor input, Tensor scale) -> ()",
-          _static_scaled_fp8_quant_impl)
+          "(Tensor! result, Tensor input, Tensor! scale, Tensor? scale_ub) -> ()")
+_register("_C", "static_scaled_fp8_quant", "(Tensor! result, Tensor input, Tensor scale) -> ()")
 _register("_C", "mul_static_fp8_quant",
-          "(Tensor(a!) out, Tensor input, Tensor scale, Tensor real_num_tokens) -> ()", _mul_static_fp8_quant_impl)
-_register("_C", "silu_mul_static_int8_quant", "(Tensor(a!) result, Tensor input, Tensor scale) -> ()",
-          _silu_mul_static_int8_quant_impl)
+          "(Tensor(a!) out, Tensor input, Tensor scale, Tensor real_num_tokens) -> ()")
+_register("_C", "silu_mul_static_int8_quant", "(Tensor(a!) result, Tensor input, Tensor scale) -> ()")
 _register("_C", "silu_mul_static_fp8_quant",
-          "(Tensor(a!) out, Tensor input, Tensor scale, Tensor real_num_tokens) -> ()",
-          _silu_mul_static_fp8_quant_impl)
-_register("_moe_C", "moe_sum_pad", "(Tensor(a!) out, Tensor input, Tensor size, int dim, bool keepdim) -> ()",
-          _moe_sum_pad_impl)
+          "(Tensor(a!) out, Tensor input, Tensor scale, Tensor real_num_tokens) -> ()")
+_register("_moe_C", "moe_sum_pad", "(Tensor(a!) out, Tensor input, Tensor size, int dim, bool keepdim) -> ()")
 
 
 # ---------------------------------------------------------------------------
@@ -875,94 +598,21 @@ _register("_moe_C", "moe_sum_pad", "(Tensor(a!) out, Tensor input, Tensor size, 
 # (csrc/torch_bindings.cpp:254-317, 852-871, 1124-1143; the fused operators are
 # what vllm_gcu/compilation/fusion.py:104-127 substitutes for norm -> quantiser)
 # ---------------------------------------------------------------------------
-def _rms_common(out, out_scales, input, residual, weight, scale, epsilon, quant_mode, group_size=0):
-    rt.require_gpu(out, out_scales, input, residual, weight, scale)
-    if input.numel() == 0:
-        return
-    if input.dtype not in (torch.float16, torch.bfloat16):
-        raise RuntimeError(f"rms_norm: input must be f16/bf16, got {input.dtype}")
-    if not input.is_contiguous() or not out.is_contiguous():
-        raise RuntimeError("rms_norm: input and output must be contiguous")
-    rows, K = _rows_last(input)
-    if weight.numel() != K:
-        raise RuntimeError(f"rms_norm: weight has {weight.numel()} elements for rows of {K}")
-    if tuple(out.shape) != tuple(input.shape):
-        raise RuntimeError(f"rms_norm: output shape {tuple(out.shape)} != input shape {tuple(input.shape)}")
-    want = {0: input.dtype, 1: torch.float8_e4m3fn, 2: torch.float8_e4m3fn, 3: torch.int8}[quant_mode]
-    if out.dtype != want:
-        raise RuntimeError(f"rms_norm: output must be {want}, got {out.dtype}")
-    if residual is not None and (residual.dtype != input.dtype or tuple(residual.shape) != tuple(input.shape)
-                                 or not residual.is_contiguous()):
-        raise RuntimeError("rms_norm: residual must match the input (dtype, shape, contiguous)")
-    w = weight.to(input.dtype).contiguous()
-    sc = None
-    if quant_mode in (1, 3):
-        sc = scale.to(torch.float32).reshape(-1)
-        if sc.numel() != 1:
-            raise RuntimeError("rms_norm + static quant takes a single scale")
-    if quant_mode == 2:
-        if out_scales.dtype != torch.float32 or not out_scales.is_contiguous() or \
-                out_scales.numel() != rows * (K // group_size):
-            raise RuntimeError("rms_norm + group quant: scales must be contiguous f32 [.., K / group_size]")
-    with torch.cuda.device(input.device):
-        _lib.call("mi355q_rms_norm", out.data_ptr(), rt.ptr(out_scales), input.data_ptr(), rt.ptr(residual),
-                  w.data_ptr(), rt.ptr(sc), float(epsilon), rows, K, quant_mode, int(group_size),
-                  rt.dtype_code(input.dtype), rt.stream_ptr())
-
-
-def _rms_norm_impl(result, input, weight, epsilon):
-    _rms_common(result, None, input, None, weight, None, epsilon, 0)
-
-
-def _fused_add_rms_norm_impl(input, residual, weight, epsilon):
-    _rms_common(input, None, input, residual, weight, None, epsilon, 0)
-
-
-def _rms_norm_static_fp8_quant_impl(result, input, weight, scale, epsilon):
-    _rms_common(result, None, input, None, weight, scale, epsilon, 1)
-
-
-def _fused_add_rms_norm_static_fp8_quant_impl(result, input, residual, weight, scale, epsilon):
-    _rms_common(result, None, input, residual, weight, scale, epsilon, 1)
-
-
-def _rms_norm_per_token_group_quant_fp8_impl(out, scale, input, weight, epsilon, group_size):
-    _rms_common(out, scale, input, None, weight, None, epsilon, 2, group_size)
-
-
-def _fused_add_rms_norm_per_token_group_quant_fp8_impl(out, residual, scale, input, weight, epsilon, group_size):
-    _rms_common(out, scale, input, residual, weight, None, epsilon, 2, group_size)
-
-
-def _rms_norm_static_int8_quant_impl(result, input, weight, scale, epsilon):
-    _rms_common(result, None, input, None, weight, scale, epsilon, 3)
-
-
-def _fused_add_rms_norm_static_int8_quant_impl(result, input, residual, weight, epsilon, scale):
-    _rms_common(result, None, input, residual, weight, scale, epsilon, 3)
-
-
-_register("_C", "rms_norm", "(Tensor! result, Tensor input, Tensor weight, float epsilon) -> ()", _rms_norm_impl)
-_register("_C", "fused_add_rms_norm", "(Tensor! input, Tensor! residual, Tensor weight, float epsilon) -> ()",
-          _fused_add_rms_norm_impl)
+_register("_C", "rms_norm", "(Tensor! result, Tensor input, Tensor weight, float epsilon) -> ()")
+_register("_C", "fused_add_rms_norm", "(Tensor! input, Tensor! residual, Tensor weight, float epsilon) -> ()")
 _register("_C", "rms_norm_static_fp8_quant",
-          "(Tensor! result, Tensor input, Tensor weight, Tensor scale, float epsilon) -> ()",
-          _rms_norm_static_fp8_quant_impl)
+          "(Tensor! result, Tensor input, Tensor weight, Tensor scale, float epsilon) -> ()")
 _register("_C", "fused_add_rms_norm_static_fp8_quant",
-          "(Tensor! result, Tensor input, Tensor! residual, Tensor weight, Tensor scale, float epsilon) -> ()",
-          _fused_add_rms_norm_static_fp8_quant_impl)
+          "(Tensor! result, Tensor input, Tensor! residual, Tensor weight, Tensor scale, float epsilon) -> ()")
 _register("_C", "rms_norm_per_token_group_quant_fp8",
-          "(Tensor! out, Tensor! scale, Tensor input, Tensor weight, float epsilon, int group_size) -> ()",
-          _rms_norm_per_token_group_quant_fp8_impl)
+          "(Tensor! out, Tensor! scale, Tensor input, Tensor weight, float epsilon, int group_size) -> ()")
 _register("_C", "fused_add_rms_norm_per_token_group_quant_fp8",
           "(Tensor! out, Tensor! residual, Tensor! scale, Tensor input, Tensor weight, float epsilon, "
-          "int group_size) -> ()", _fused_add_rms_norm_per_token_group_quant_fp8_impl)
+          "int group_size) -> ()")
 _register("_C", "rms_norm_static_int8_quant",
-          "(Tensor(a!) result, Tensor input, Tensor weight, Tensor scale, float epsilon) -> ()",
-          _rms_norm_static_int8_quant_impl)
+          "(Tensor(a!) result, Tensor input, Tensor weight, Tensor scale, float epsilon) -> ()")
 _register("_C", "fused_add_rms_norm_static_int8_quant",
-          "(Tensor(a!) result, Tensor input, Tensor(a!) residual, Tensor weight, float epsilon, Tensor scale) -> ()",
-          _fused_add_rms_norm_static_int8_quant_impl)
+          "(Tensor(a!) result, Tensor input, Tensor(a!) residual, Tensor weight, float epsilon, Tensor scale) -> ()")
 
 
 # 8bit (vllm_gcu/kernels/_custom_ops.py:298-317)
@@ -1243,13 +893,7 @@ def _kcontig(out, a, w, a_scale, w_scale, bias, mode, group):
                   layout, rt.stream_ptr())
 
 
-# the MFMA tile kernel beats the weight-streaming kernel above 64 rows once its tiles fill a good part of
-# the chip (measured, K 8192 N 28672 = 224 tiles: M 65..128 69..73 us against 87..119 us, M 64 68 us
-# against 73 us for the streamer's last single-block size; K 7168 N 4096 = 32 tiles: 52 us against
-# 37..53 us at M 65..128, so few tiles stay with the streamer).  The tile kernel needs about 1 us
-# per K block however few tiles there are; the streamer's time grows with the rows: they cross at
-# 48..64 tiles (K 7168 N 4096: 32 tiles 56 against 31 us, 64 tiles 55 against 58 us, 96 tiles 56
-# against 85 us; the same on K 4096 N 4096, K 2048 N 7168 and K 7168 N 2048)
+# which kernel takes a block-scaled fp8 layer (the rule: fp8_tile_plan in csrc/host/module.cpp)
 _FP8_TILE_MIN_M = 64
 _FP8_STAGE_SCALES = True      # room in the workspace for the activation scales in K block major order (tile kernel)
 _FP8_TILE_MIN_TILES = 64
@@ -1263,16 +907,8 @@ def _linear_quant_impl(out, lhs, rhs, bias, lhs_scale, rhs_scale):
     if lhs.dtype != torch.float8_e4m3fn or rhs.dtype != torch.float8_e4m3fn:
         raise RuntimeError("linear_quant: operands must be float8_e4m3fn")
     M, N, K = lhs.numel() // lhs.shape[-1], rhs.shape[0], lhs.shape[-1]
-    tiles = -(-M // 256) * (N // 128)               # 256 x 128 output tiles, one workgroup each
-    # (from 33 rows on a layer of 128 tiles or more: the tile kernel's wavefronts without rows only copy,
-    # K 8192 x N 28672 at M = 40 / 48 / 64: 59.0 / 62.3 / 68.7 -> 55.5 / 56.3 / 53.6 us; 112 tiles: the streamer stays ahead)
-    # (and, whatever the tile count, where the library plans K ranges side by side that fill the chip:
-    # from 65 rows, and from 25 / 33 rows on where K is long, see fp8_split_min_rows)
-    need = _lib.load().mi355q_fp8_gemm_workspace_bytes(M, N, K) \
-        if M > _FP8_TILE_MIN_M // 4 and N % 128 == 0 and K % 128 == 0 else 0
-    if (need or (M > _FP8_TILE_MIN_M and tiles >= _FP8_TILE_MIN_TILES)
-            or (M > _FP8_TILE_MIN_M // 2 and tiles >= 2 * _FP8_TILE_MIN_TILES)) \
-            and N % 128 == 0 and K % 128 == 0 \
+    need = rt.host.fp8_tile_plan(M, N, K, _FP8_TILE_MIN_M, _FP8_TILE_MIN_TILES)
+    if need >= 0 \
             and out.dtype in (torch.float16, torch.bfloat16) \
             and rhs.dim() == 2 and rhs.is_contiguous() and out.is_contiguous():
         # prefill-sized M: the MFMA tile kernel (the weight-streaming kernel re-reads the weights per 64 rows)
@@ -1401,3 +1037,6 @@ def w8a8_block_fp8_matmul(A: torch.Tensor, B: torch.Tensor, As: torch.Tensor, Bs
     C = A.new_empty(C_shape, dtype=output_dtype)
     torch.ops._C.linear_quant(C, A, B, bias, As, Bs)
     return C
+
+
+rt.host.register_activation_ops()

@@ -1,8 +1,15 @@
 """Small runtime helpers shared by the operator wrappers: stream handle,
-dtype codes, the per-(device, stream) split-K workspace."""
+dtype codes, the per-(device, stream) split-K workspace, the native host path."""
 import torch
 
 from .. import _lib
+
+_lib.load()          # fail at import time when the HIP library is missing
+try:
+    from .. import _mi355q_host as host
+except ImportError as e:
+    raise ImportError("the native host path vllm-gcu_amd/_mi355q_host.so is missing or does not fit this torch: build "
+                      "it with `python -c 'import __graft_entry__ as g; g.build()'`") from e
 
 _DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _lib.F32}
 
@@ -61,3 +68,6 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor:
         buf = torch.zeros(max(nbytes, WORKSPACE_BYTES), dtype=torch.uint8, device=device)
         _workspaces[key] = buf
     return buf
+
+
+host.set_workspace(workspace)

@@ -10,6 +10,7 @@ from typing import Any, Dict, List, Optional, Tuple
 import torch
 
 from . import _custom_ops as ops
+from . import _runtime as rt
 
 
 # Rows per expert from which the fp8 block-scaled and int8 grouped GEMMs take blocks of 128 and of 256 slots, i.e.
@@ -82,6 +83,11 @@ def grouped_topk(hidden_states: torch.Tensor, gating_output: torch.Tensor, topk:
                  num_expert_group: int = 0, topk_group: int = 0, scoring_func: str = "softmax",
                  e_score_correction_bias: Optional[torch.Tensor] = None):
     assert hidden_states.shape[0] == gating_output.shape[0], "Number of tokens mismatch"
+    if scoring_func in ("softmax", "sigmoid") and ops.eager():
+        routed = rt.host.grouped_topk(gating_output, topk, bool(renormalize), num_expert_group, topk_group,
+                                      scoring_func == "sigmoid", e_score_correction_bias)
+        if routed is not None:
+            return routed
     topk_weights = torch.empty((gating_output.shape[0], topk), device=gating_output.device, dtype=torch.float32)
     topk_ids = torch.empty((gating_output.shape[0], topk), device=gating_output.device, dtype=torch.int32)
     if hidden_states.numel() == 0:

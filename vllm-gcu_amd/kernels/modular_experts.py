@@ -12,6 +12,8 @@ from typing import Optional
 
 import torch
 
+from .. import _lib
+from . import _runtime as rt
 from .fused_moe import get_default_config, invoke_fused_moe_kernel, moe_align_block_size
 
 
@@ -69,6 +71,26 @@ class TritonExpertsPad:
         workspace2 = (M, topk, max(N, K))
         output = (M, K)
         return (workspace1, workspace2, output, a.dtype)
+
+    def apply_native(self, output, hidden_states, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, w1_zp, w2_zp) -> bool:
+        """The whole sequence, activation quantisation included, in one native call on its own scratch: int4
+        experts, and block-scaled fp8 and per-token int8 experts whose activations are quantised on the fly.  For
+        calls in which every row counts and every expert is local.  False (nothing done) where the operands
+        need the general path."""
+        if self.use_int4_w4a16:
+            mode, group = _lib.Q_W4A16, self.block_shape[1]
+        elif self.use_fp8_w8a8 and w1.dtype == torch.float8_e4m3fn and self.block_shape is not None \
+                and list(self.block_shape) == [128, 128]:
+            mode, group = _lib.Q_FP8_BLOCK, 128
+        elif self.use_int8_w8a8 and self.per_act_token_quant:
+            mode, group = _lib.Q_INT8, 1
+        else:
+            return False
+        E, M, N, K, top_k = moe_problem_size(hidden_states, w1, w2, topk_ids, self.use_int4_w4a16)
+        config = get_default_config(M=M, E=E, N=N, K=K, topk=top_k, dtype="int8_w8a8" if self.use_int8_w8a8 else None,
+                                    is_marlin=False, block_shape=self.block_shape)
+        return rt.host.fused_experts(mode, group, config["BLOCK_SIZE_M"], hidden_states, w1, w2, w1_scale, w2_scale, w1_zp,
+                                     w2_zp, topk_weights, topk_ids, output) is not None
 
     def apply(self, output, hidden_states, w1, w2, topk_weights, topk_ids, activation, global_num_experts,
               expert_map, w1_scale, w2_scale, w1_zp, w2_zp, a1q_scale, a2_scale, workspace13, workspace2,

@@ -11,7 +11,9 @@ from typing import Optional
 
 import torch
 
-from .modular_experts import moe_problem_size
+from . import _custom_ops as ops
+from .modular_experts import TritonExpertsPad, moe_problem_size
+from .prepare_finalize import MoEPrepareAndFinalizeNoEP
 
 
 def fused_moe_chunk_size() -> int:
@@ -51,10 +53,15 @@ class FusedMoEModularKernel(torch.nn.Module):
         E, M, N, K, top_k = moe_problem_size(a1, w1, w2, topk_ids, fe.use_int4_w4a16)
         if global_num_experts == -1:
             global_num_experts = E
+        chunk = fused_moe_chunk_size() if fe.supports_chunking() else M
+        if M <= chunk and type(fe) is TritonExpertsPad and type(self.prepare_finalize) is MoEPrepareAndFinalizeNoEP \
+                and self.prepare_finalize.shared_experts is None and activation == "silu" and global_num_experts == E \
+                and expert_map is None and a1_scale is None and a2_scale is None and not apply_router_weight_on_input \
+                and ops.eager() and fe.apply_native(output, a1, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, w1_zp, w2_zp):
+            return output
         a1q, a1q_scale, expert_num_tokens, _ids, _w, shared_output = self.prepare_finalize.prepare(
             a1, a1_scale, a2_scale, topk_weights, topk_ids, global_num_experts, expert_map,
             apply_router_weight_on_input, fe.quant_config)
-        chunk = fused_moe_chunk_size() if fe.supports_chunking() else M
         num_chunks = -(-M // chunk)
         if num_chunks > 1:
             # output shape from the full M, workspaces from one chunk (modular_kernel.py:176-186)

@@ -11,6 +11,7 @@ import torch
 from torch.nn import Parameter
 
 from .. import _custom_ops as ops
+from .. import _runtime as rt
 from . import rearrange
 from .utils import register_gcu_quantization_config
 
@@ -63,6 +64,10 @@ class AWQGCULinearMethod:
         layer.qzeros = Parameter(qzeros, requires_grad=False)
 
     def apply(self, layer, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+        if ops.eager():
+            out = rt.host.w4a16_layer(layer, x, bias, self.quant_config.group_size)
+            if out is not None:
+                return out
         if x.numel() == 0:
             return torch.empty([0, layer.qweight.shape[-1]], dtype=x.dtype, device=x.device)
         out_shape = x.shape[:-1] + (layer.qweight.shape[-1],)

@@ -13,6 +13,7 @@ from typing import List, Optional
 import torch
 
 from .. import _custom_ops as ops
+from .. import _runtime as rt
 from ..fused_moe import select_experts
 from ..modular_experts import TritonExpertsPad
 from ..modular_kernel import FusedMoEModularKernel
@@ -127,7 +128,15 @@ class Fp8GCULinearMethod:
     def apply(self, layer, x: torch.Tensor, bias: Optional[torch.Tensor] = None,
               x_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
         if not self.block_quant:
+            if ops.eager():
+                out = rt.host.fp8_scaled_layer(layer, x, bias)
+                if out is not None:
+                    return out
             return self._apply_scaled_mm(layer, x, bias)
+        if bias is None and ops.eager():
+            out = rt.host.fp8_block_layer(layer, x, x_scale, ops._FP8_TILE_MIN_M, ops._FP8_TILE_MIN_TILES, ops._FP8_STAGE_SCALES)
+            if out is not None:
+                return out
         return apply_w8a8_block_fp8_linear(input=x, weight=layer.weight,
                                            block_size=self.quant_config.weight_block_size,
                                            weight_scale=layer.weight_scale_inv,

@@ -14,6 +14,7 @@ import torch
 from torch.nn import Parameter
 
 from .. import _custom_ops as ops
+from .. import _runtime as rt
 from . import rearrange
 from .utils import register_gcu_quantization_config
 
@@ -91,6 +92,10 @@ class GPTQGCULinearMethod:
                 layer.scales = Parameter(layer.scales.data.squeeze(0), requires_grad=False)
 
     def apply(self, layer, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+        if self.quant_config.weight_bits == 4 and ops.eager():
+            out = rt.host.w4a16_layer(layer, x, bias, self.quant_config.group_size)
+            if out is not None:
+                return out
         n_out = layer.qweight.shape[-1] if self.quant_config.weight_bits == 4 else layer.qweight.shape[0]
         if x.numel() == 0:
             return torch.empty([0, n_out], dtype=x.dtype, device=x.device)

@@ -123,37 +123,22 @@ def unpack_slab(packed: torch.Tensor) -> torch.Tensor:
     return dst
 
 
-# kslab allocations by (device index, address) -> byte size: the flag has to survive views
-# (``weight.t()`` is what the int8 operators receive), which drop Python attributes
-_KSLAB_ALLOCS = {}           # (device, address) -> [bytes, live tensor objects that carry the flag]
-
-
-def _unregister_kslab(key) -> None:
-    ent = _KSLAB_ALLOCS.get(key)
-    if ent is not None:
-        ent[1] -= 1
-        if ent[1] <= 0:
-            del _KSLAB_ALLOCS[key]
-
-
+# The kslab flag has to survive views (``weight.t()`` is what the int8 operators receive), which drop Python
+# attributes: the native host path keeps the address ranges of flagged tensors by (device, address), with the
+# number of live tensor objects that carry the flag on each.
 def _register_kslab(t: torch.Tensor) -> None:
     """Entries live as long as a flagged tensor object on that memory does (the tensor made by
     to_kslab, a Parameter wrapped around it and marked with mark_kslab, ...)."""
-    key = (t.device.index, t.data_ptr())
-    ent = _KSLAB_ALLOCS.setdefault(key, [t.numel() * t.element_size(), 0])
-    ent[0] = t.numel() * t.element_size()
-    ent[1] += 1
-    weakref.finalize(t, _unregister_kslab, key)
+    dev, addr = t.get_device(), t.data_ptr()
+    rt.host.kslab_register(dev, addr, t.numel() * t.element_size())
+    weakref.finalize(t, rt.host.kslab_unregister, dev, addr)
 
 
 def is_kslab(w: torch.Tensor) -> bool:
     """True for a tensor made by :func:`to_kslab`, for a Parameter / view marked with
     :func:`mark_kslab`, and for any view that starts at the address of such an allocation and
     covers all of it (e.g. ``w.t()``)."""
-    if getattr(w, "_mi355q_kslab", False):
-        return True
-    ent = _KSLAB_ALLOCS.get((w.device.index, w.data_ptr())) if w.is_cuda else None
-    return ent is not None and ent[0] == w.numel() * w.element_size()
+    return getattr(w, "_mi355q_kslab", False) or rt.host.is_kslab(w)
 
 
 def kslab_eligible(w: torch.Tensor) -> bool:

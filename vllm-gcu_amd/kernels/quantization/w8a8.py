@@ -14,6 +14,7 @@ import torch
 from torch.nn import Parameter
 
 from .. import _custom_ops as ops
+from .. import _runtime as rt
 from ..fused_moe import select_experts
 from ..modular_experts import TritonExpertsPad
 from ..modular_kernel import FusedMoEModularKernel
@@ -63,6 +64,10 @@ class W8A8LinearMethod:
         rearrange.kslab_parameters_(layer, ("weight",))
 
     def apply(self, layer, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+        if ops.eager():
+            out = rt.host.w8a8_static_layer(layer, x, bias, ops._INT8_STREAM_MAX_M)
+            if out is not None:
+                return out
         if x.dtype in self.quant_config.get_supported_act_dtypes():
             x = ops.scaled_int8_quant(x, layer.in_scales)[0]
         assert x.dtype == torch.int8
@@ -81,6 +86,10 @@ class CompressedTensorMMLinearKernel:
         rearrange.kslab_parameters_(layer, ("weight",))
 
     def apply_weights(self, layer, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+        if ops.eager():
+            out = rt.host.int8_dynamic_layer(layer, x, bias, ops._INT8_STREAM_MAX_M)
+            if out is not None:
+                return out
         x_q, x_s, _ = ops.scaled_int8_quant(x.contiguous(), getattr(layer, "input_scale", None))
         x_2d = x_q.reshape(-1, x_q.shape[-1])
         out = ops.cutlass_scaled_mm(x_2d, layer.weight.t(), x_s, layer.weight_scale, x.dtype, bias)
