@@ -221,6 +221,10 @@ int mi355q_dynamic_int8_quant(int8_t* out, float* scales, const void* x, int M, 
  * with the reciprocal rounded to the input dtype; scale is one value or [K]. */
 int mi355q_static_int8_quant(int8_t* out, const void* x, const float* scale, int per_channel, int M,
                              int K, int dtype, void* stream);
+/* The same with the scales as stored: scale_dtype is F32 or `dtype` (checkpoints keep them in the
+ * activation type, vllm_gcu/kernels/quantization/w8a8.py:157-171). */
+int mi355q_static_int8_quant_typed(int8_t* out, const void* x, const void* scale, int scale_dtype, int per_channel,
+                                   int M, int K, int dtype, void* stream);
 
 /* Replaces topsvllmSiluMulQuant as called by silu_mul_static_int8_quant
  * (csrc/src/silu_mul_static_int8_quant.cpp:11-28): x is [rows, 2d];

@@ -1,0 +1,80 @@
+"""The row-in-registers quantisers and norms at the edges of their launch shapes: rows that end inside a piece, one
+piece short of and past a whole number of pieces, fewer and more rows than the rule's steps, rows too long for
+registers and rows whose address or length needs the one-element loops."""
+import pytest
+import torch
+
+from vllm_gcu_amd.kernels import _custom_ops  # noqa: F401  (registers the ops)
+
+pytestmark = pytest.mark.gpu
+SHAPES = [(1, 8), (3, 13), (2, 2040), (2, 2056), (700, 2048), (1100, 1032), (3, 8192 + 8), (600, 16384), (2, 65536), (2, 65544)]
+
+
+def over(a, b):
+    """a / b as one division (torch multiplies by the reciprocal where one side is a plain number)"""
+    t = a if torch.is_tensor(a) else b
+    return (a if torch.is_tensor(a) else torch.full_like(t, a)) / (b if torch.is_tensor(b) else torch.full_like(t, b))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,K", SHAPES)
+def test_dynamic_row_quantisers(rows, K, dtype):
+    print(f"case row quantisers {rows} x {K} {dtype}", flush=True)
+    torch.manual_seed(rows * K)
+    x = torch.randn(rows, K, device="cuda").to(dtype)
+    x[0] = 0
+    flat = torch.empty(rows * K + 1, dtype=dtype, device="cuda")
+    flat[1:] = x.view(-1)
+    for src in (x, flat[1:].view(rows, K)):                      # the second one off the 16-byte grid
+        q, s = torch.empty(rows, K, dtype=torch.int8, device="cuda"), torch.empty(rows, 1, device="cuda")
+        torch.ops._C.dynamic_scaled_int8_quant(q, src, s, None)
+        mx = x.float().abs().amax(dim=1, keepdim=True)
+        assert torch.equal(s, over(mx, 127.0))
+        want = torch.nan_to_num(x.float() * over(127.0, mx), nan=0.0).round().clamp(-128, 127).to(torch.int8)
+        assert torch.equal(q, want)
+        f, fs = torch.empty(rows, K, dtype=torch.float8_e4m3fn, device="cuda"), torch.empty(rows, 1, device="cuda")
+        torch.ops._C.dynamic_per_token_scaled_fp8_quant(f, src, fs, None)
+        assert torch.equal(fs, over(mx.clamp_min(1e-10), 448.0))
+        assert torch.equal(f.view(torch.uint8), (x.float() / fs).clamp(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,K", [(1, 8), (3, 13), (5, 2056), (300, 520)])
+def test_static_int8_quant_with_scales_of_either_type(rows, K, dtype):
+    print(f"case static int8 {rows} x {K} {dtype}", flush=True)
+    torch.manual_seed(rows * K)
+    x = torch.randn(rows, K, device="cuda").to(dtype)
+    sc = (torch.rand(K, device="cuda") * 0.03 + 0.01).to(dtype)
+    want = (x.float() * (1.0 / sc.float()).to(dtype).float()).round().clamp(-128, 127).to(torch.int8)
+    for scale in (sc, sc.float()):
+        q = torch.empty(rows, K, dtype=torch.int8, device="cuda")
+        torch.ops._C.static_scaled_int8_quant(q, x, scale, None)
+        assert torch.equal(q, want)
+        torch.ops._C.static_scaled_int8_quant(q, x, scale[:1], None)
+        one = (x.float() * (1.0 / sc[:1].float()).to(dtype).float()).round().clamp(-128, 127).to(torch.int8)
+        assert torch.equal(q, one)
+
+
+@pytest.mark.parametrize("rows,d", [(1, 8), (3, 1544), (700, 1408), (2048, 2048)])
+def test_silu_and_sum_index_arithmetic(rows, d):
+    print(f"case silu / sum {rows} x {d}", flush=True)
+    torch.manual_seed(rows + d)
+    x = torch.randn(rows, 2 * d, device="cuda").half()
+    out = torch.full((rows, d), float("nan"), device="cuda").half()
+    torch.ops._C.silu_and_mul(out, x)
+    want = torch.nn.functional.silu(x[:, :d].float()) * x[:, d:].float()
+    torch.testing.assert_close(out.float(), want, rtol=2e-3, atol=2e-3)
+    x3 = torch.randn(rows, 3, d, device="cuda").half()
+    n = torch.tensor([max(1, rows - 1)], dtype=torch.int32, device="cuda")
+    total = torch.full((rows, d), float("nan"), device="cuda").half()
+    torch.ops._moe_C.moe_sum_pad(total, x3, n, 1, False)
+    m = int(n)
+    torch.testing.assert_close(total[:m].float(), x3[:m].float().sum(1), rtol=2e-3, atol=2e-3)
+    assert torch.isnan(total[m:]).all()
+    if d % 128 == 0:
+        q = torch.empty(rows, d, dtype=torch.float8_e4m3fn, device="cuda")
+        s = torch.empty(rows, d // 128, device="cuda")
+        torch.ops._C.silu_mul_per_token_group_quant(q, s, x, 128)
+        g = out.float().view(rows, d // 128, 128)
+        assert torch.equal(s, over(g.abs().amax(-1).clamp_min(1e-10), 448.0))
+        assert torch.equal(q.view(torch.uint8), (g / s[..., None]).clamp(-448, 448).view(rows, d).to(torch.float8_e4m3fn).view(torch.uint8))

@@ -6,6 +6,8 @@
 // without a host synchronisation.
 #include "common.h"
 
+#include <algorithm>
+
 namespace mi355q {
 namespace {
 
@@ -74,21 +76,22 @@ struct SharedDivisor {
 };
 
 // ---- silu_and_mul: out[r, :d] = silu(x[r, :d]) * x[r, d:] -------------------
+// (row and piece of an item by multiplication: a 64-bit division per 16-byte piece was a quarter of these kernels'
+// instructions, and they are bound by issue as much as by HBM)
 template <int DT>
 __global__ void __launch_bounds__(256)
-silu_and_mul_kernel(uint16_t* out, const uint16_t* x, long rows, int d, const int* valid_rows, int rpc) {
-  const long nrow = valid_rows ? min(rows, (long)max(0, *valid_rows) * rpc) : rows;
-  const int chunks = d / 8;
-  const long total = nrow * chunks;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long)gridDim.x * 256) {
-    const long r = i / chunks;
-    const int c = (int)(i - r * chunks);
+silu_and_mul_kernel(uint16_t* out, const uint16_t* x, uint32_t rows, int d, FastDiv chunks, const int* valid_rows, int rpc) {
+  const long nrow = valid_rows ? min((long)rows, (long)max(0, *valid_rows) * rpc) : rows;
+  const uint32_t total = (uint32_t)nrow * chunks.d;
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+    const uint32_t r = chunks.div(i), c = i - r * chunks.d;
+    const uint16_t* xr = x + (size_t)r * 2 * d + 8 * c;
     float a[8], b[8], y[8];
-    unpack8<DT>(*(const u4*)(x + r * 2 * d + 8 * c), a);
-    unpack8<DT>(*(const u4*)(x + r * 2 * d + d + 8 * c), b);
+    unpack8<DT>(*(const u4*)xr, a);
+    unpack8<DT>(*(const u4*)(xr + d), b);
 #pragma unroll
     for (int e = 0; e < 8; ++e) y[e] = silu_mul(a[e], b[e]);
-    *(u4*)(out + r * d + 8 * c) = pack8<DT>(y);
+    *(u4*)(out + (size_t)r * d + 8 * c) = pack8<DT>(y);
   }
 }
 
@@ -96,28 +99,26 @@ silu_and_mul_kernel(uint16_t* out, const uint16_t* x, long rows, int d, const in
 // A group of `gs` elements is handled by gs/8 adjacent lanes (gs in 64,128,256,512).
 template <int DT, bool SILU>
 __global__ void __launch_bounds__(256)
-group_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, long rows, int K, int gs,
+group_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, uint32_t rows, int K, FastDiv chunks, int lpg,
                        const int* valid_rows, int rpc) {
-  const long nrow = valid_rows ? min(rows, (long)max(0, *valid_rows) * rpc) : rows;
-  const int chunks = K / 8;                      // 8-element chunks per output row
-  const int lpg = gs / 8;                        // lanes per group (power of two <= 64)
-  const long total = nrow * chunks;
-  const long stride = (long)gridDim.x * 256;
-  for (long i0 = (long)blockIdx.x * 256; i0 < total; i0 += stride) {
-    const long i = i0 + threadIdx.x;
+  const long nrow = valid_rows ? min((long)rows, (long)max(0, *valid_rows) * rpc) : rows;
+  const uint32_t total = (uint32_t)nrow * chunks.d;     // 8-element pieces; lpg (a power of two <= 64) lanes per group
+  const int lg = 31 - __clz(lpg);
+  for (uint32_t i0 = blockIdx.x * 256; i0 < total; i0 += gridDim.x * 256) {
+    const uint32_t i = i0 + threadIdx.x;
     const bool live = i < total;
-    const long r = live ? i / chunks : 0;
-    const int c = live ? (int)(i - r * chunks) : 0;
+    const uint32_t r = live ? chunks.div(i) : 0, c = live ? i - r * chunks.d : 0;
     float y[8];
     if (SILU) {
+      const uint16_t* xr = x + (size_t)r * 2 * K + 8 * c;
       float a[8], b[8];
-      unpack8<DT>(*(const u4*)(x + r * 2 * K + 8 * c), a);
-      unpack8<DT>(*(const u4*)(x + r * 2 * K + K + 8 * c), b);
+      unpack8<DT>(*(const u4*)xr, a);
+      unpack8<DT>(*(const u4*)(xr + K), b);
       // the unfused sequence stores the gate output in the activation dtype
 #pragma unroll
       for (int e = 0; e < 8; ++e) y[e] = round_act<DT>(silu_mul(a[e], b[e]));
     } else {
-      unpack8<DT>(*(const u4*)(x + r * K + 8 * c), y);
+      unpack8<DT>(*(const u4*)(x + (size_t)r * K + 8 * c), y);
     }
     float mx = 0.f;
 #pragma unroll
@@ -130,25 +131,63 @@ group_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, long rows
 #pragma unroll
     for (int e = 0; e < 8; ++e) q[e] = clamp448(by_s.div(y[e]));
     if (live) {
-      *(u2*)(out + r * K + 8 * c) = to_fp8x8(q);
-      if ((c % lpg) == 0) scales[r * (K / gs) + c / lpg] = s;
+      *(u2*)(out + (size_t)r * K + 8 * c) = to_fp8x8(q);
+      // (a row is a whole number of groups: the groups of the matrix count through)
+      if ((c & (lpg - 1)) == 0) scales[i >> lg] = s;
     }
   }
 }
 
 // ---- per-token fp8 (one workgroup per row) and static fp8 --------------------
+// Bound by latency up to some hundred rows, by HBM above: the row is read once, P pieces of 16 bytes per lane with
+// all loads in flight together, and quantised from registers.
+template <int DT, int P>
+__global__ void __launch_bounds__(1024)
+token_fp8_quant_row_kernel(uint8_t* out, float* scales, const uint16_t* x, int K, const int* valid_rows) {
+  const long row = blockIdx.x;
+  if (valid_rows && row >= *valid_rows) return;
+  __shared__ float red[16];
+  const int chunks = K / 8, nt = blockDim.x;
+  const uint16_t* xr = x + row * K;
+  u4 v[P];
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const int c = threadIdx.x + nt * i;
+    v[i] = *(const u4*)(xr + 8 * (c < chunks ? c : 0));     // (past the end: the first piece again, for the maximum)
+  }
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    float y[8];
+    unpack8<DT>(v[i], y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(y[e]));
+  }
+  mx = block_max(mx, red);
+  const float s = fmaxf(mx, 1e-10f) / FP8_MAX;
+  if (threadIdx.x == 0) scales[row] = s;
+  const SharedDivisor by_s(s);
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const int c = threadIdx.x + nt * i;
+    float y[8];
+    unpack8<DT>(v[i], y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = clamp448(by_s.div(y[e]));
+    if (c < chunks) *(u2*)(out + row * K + 8 * c) = to_fp8x8(y);
+  }
+}
+
+// any row length and alignment, one element at a time
 template <int DT>
 __global__ void __launch_bounds__(256)
 token_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, int K, const int* valid_rows) {
   const long row = blockIdx.x;
   if (valid_rows && row >= *valid_rows) return;
-  __shared__ float red[4];
+  __shared__ float red[16];
   float mx = 0.f;
   for (int k = threadIdx.x; k < K; k += 256) mx = fmaxf(mx, fabsf(Elem<DT>::to_f32(x[row * K + k])));
-  mx = wave_max(mx);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  mx = block_max(mx, red);
   const float s = fmaxf(mx, 1e-10f) / FP8_MAX;
   if (threadIdx.x == 0) scales[row] = s;
   const SharedDivisor by_s(s);
@@ -156,6 +195,19 @@ token_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, int K, co
     const float y = clamp448(by_s.div(Elem<DT>::to_f32(x[row * K + k])));
     int w = __builtin_amdgcn_cvt_pk_fp8_f32(y, y, 0, false);
     out[row * K + k] = (uint8_t)(w & 0xff);
+  }
+}
+
+template <int DT>
+void launch_token_quant(long rows, int K, hipStream_t st, uint8_t* out, float* scales, const uint16_t* x, const int* valid_rows) {
+  const RowShape s = row_shape(rows, K, (((uintptr_t)x & 15) | ((uintptr_t)out & 7)) == 0, device_cu_count());
+  const dim3 grid((unsigned)rows), block(s.threads);
+  switch (s.pieces) {
+    case 1: hipLaunchKernelGGL((token_fp8_quant_row_kernel<DT, 1>), grid, block, 0, st, out, scales, x, K, valid_rows); break;
+    case 2: hipLaunchKernelGGL((token_fp8_quant_row_kernel<DT, 2>), grid, block, 0, st, out, scales, x, K, valid_rows); break;
+    case 4: hipLaunchKernelGGL((token_fp8_quant_row_kernel<DT, 4>), grid, block, 0, st, out, scales, x, K, valid_rows); break;
+    case 8: hipLaunchKernelGGL((token_fp8_quant_row_kernel<DT, 8>), grid, block, 0, st, out, scales, x, K, valid_rows); break;
+    default: hipLaunchKernelGGL((token_fp8_quant_kernel<DT>), grid, dim3(256), 0, st, out, scales, x, K, valid_rows); break;
   }
 }
 
@@ -209,13 +261,12 @@ static_fp8_quant_kernel(uint8_t* out, const uint16_t* x, const float* scale, lon
 // ---- moe_sum: out[m, :] = sum_t in[m, t, :] in fp32 --------------------------
 template <int DT_IN, int DT_OUT>
 __global__ void __launch_bounds__(256)
-moe_sum_kernel(void* out, const uint16_t* in, long rows, int T, int K, const int* valid_rows) {
-  const long nrow = valid_rows ? min(rows, (long)max(0, *valid_rows)) : rows;
-  const int chunks = K / 8;
-  const long total = nrow * chunks;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long)gridDim.x * 256) {
-    const long r = i / chunks;
-    const int c = (int)(i - r * chunks);
+moe_sum_kernel(void* out, const uint16_t* in, uint32_t rows, int T, int K, FastDiv chunks, const int* valid_rows) {
+  const long nrow = valid_rows ? min((long)rows, (long)max(0, *valid_rows)) : rows;
+  const uint32_t total = (uint32_t)nrow * chunks.d;
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+    const long r = chunks.div(i);
+    const int c = (int)(i - (uint32_t)r * chunks.d);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int t = 0; t < T; ++t) {
       float v[8];
@@ -318,64 +369,62 @@ rms_norm_kernel(void* out, float* out_scales, const uint16_t* x, uint16_t* resid
   }
 }
 
-// The same operator for rows of up to 8192 elements: the row (and the weight vector) is loaded once,
-// up to four 16-byte pieces per lane with all loads in flight together, and both passes run from
-// registers -- the loop version above waits for one piece at a time and reads the row twice.  Same
-// arithmetic in the same order per element; the sum of squares adds the lane's pieces in the same
-// order too, so the results are bit-identical.
-template <int DT, bool ADD, int QM>
-__global__ void __launch_bounds__(256)
+// The same operator with the row (and the weight vector) loaded once, P pieces of 16 bytes per lane with all loads in
+// flight together, and both passes run from registers -- the loop version above waits for one piece at a time and
+// reads the row twice.  Same arithmetic per element; only the order in which the squares are added differs.
+template <int DT, bool ADD, int QM, int P>
+__global__ void __launch_bounds__(1024)
 rms_norm_row_kernel(void* out, float* out_scales, const uint16_t* x, uint16_t* residual, const uint16_t* weight,
-                    const float* scale, float eps, int K, int gs) {
+                    const float* scale, float eps, int K, int lpg) {
   const long row = blockIdx.x;
-  const int chunks = K / 8;
+  const int chunks = K / 8, nt = blockDim.x;
   const uint16_t* xr = x + row * K;
   uint16_t* rr = ADD ? residual + row * K : nullptr;
-  __shared__ float red[4];
-  u4 xv[4], rv[4], wv[4];
-  bool live[4];
+  __shared__ float red[16];
+  u4 xv[P], rv[P], wv[P];
+  bool live[P];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c0 = threadIdx.x + 256 * i;
+  for (int i = 0; i < P; ++i) {
+    const int c0 = threadIdx.x + nt * i;
     live[i] = c0 < chunks;
     const int c = live[i] ? c0 : 0;
     xv[i] = *(const u4*)(xr + 8 * c);
     if (ADD) rv[i] = *(const u4*)(rr + 8 * c);
     wv[i] = *(const u4*)(weight + 8 * c);
   }
-  float v[4][8];
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    unpack8<DT>(xv[i], v[i]);
+  for (int i = 0; i < P; ++i) {
+    float v[8];
+    unpack8<DT>(xv[i], v);
     if (ADD) {
       float r[8];
       unpack8<DT>(rv[i], r);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[i][e] = round_act<DT>(v[i][e] + r[e]);
-      if (live[i]) *(u4*)(rr + 8 * (threadIdx.x + 256 * i)) = pack8<DT>(v[i]);
+      for (int e = 0; e < 8; ++e) v[e] = round_act<DT>(v[e] + r[e]);
+      xv[i] = pack8<DT>(v);
+      // (what follows starts from the stored 16-bit values in both variants: from known values the compiler takes other
+      // instructions for the sum and the first rounding, and the operators would differ in the last place)
+      asm("" : "+v"(xv[i]));
+      if (live[i]) *(u4*)(rr + 8 * (threadIdx.x + nt * i)) = xv[i];
+      unpack8<DT>(xv[i], v);
     }
-    if (live[i]) {
+    float s = ss;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ss += v[i][e] * v[i][e];
-    }
+    for (int e = 0; e < 8; ++e) s = __builtin_fmaf(v[e], v[e], s);
+    ss = live[i] ? s : ss;
   }
-  ss = wave_sum(ss);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  ss = (red[0] + red[1]) + (red[2] + red[3]);
+  ss = block_sum(ss, red);
   const float rs = rsqrtf(ss / (float)K + eps);
   float qs = 1.f;
   if (QM == 1) qs = *scale;
   if (QM == 3) qs = round_act<DT>(1.0f / *scale);
-  const int lpg = QM == 2 ? gs / 8 : 1;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (256 * i >= chunks) break;                       // (uniform: every lane stays for the group shuffles)
-    const int c = threadIdx.x + 256 * i;
-    float w[8];
+  for (int i = 0; i < P; ++i) {
+    const int c = threadIdx.x + nt * i;                 // (every lane stays for the group shuffles)
+    float w[8], y[8];
+    unpack8<DT>(xv[i], y);
     unpack8<DT>(wv[i], w);
-    float* y = v[i];
 #pragma unroll
     for (int e = 0; e < 8; ++e) y[e] = round_act<DT>(round_act<DT>(y[e] * rs) * w[e]);
     if (QM == 0) {
@@ -398,7 +447,7 @@ rms_norm_row_kernel(void* out, float* out_scales, const uint16_t* x, uint16_t* r
       for (int e = 0; e < 8; ++e) q[e] = clamp448(by_sg.div(y[e]));
       if (live[i]) {
         *(u2*)((uint8_t*)out + row * K + 8 * c) = to_fp8x8(q);
-        if ((c % lpg) == 0) out_scales[row * (K / gs) + c / lpg] = sg;
+        if ((c & (lpg - 1)) == 0) out_scales[(row * chunks + c) >> (31 - __clz(lpg))] = sg;
       }
     } else {
       uint32_t lo = 0, hi = 0;
@@ -414,26 +463,34 @@ rms_norm_row_kernel(void* out, float* out_scales, const uint16_t* x, uint16_t* r
   }
 }
 
-template <int DT, bool ADD>
-void launch_rms(int qm, long rows, hipStream_t st, void* out, float* out_scales, const uint16_t* x,
-                uint16_t* residual, const uint16_t* weight, const float* scale, float eps, int K, int gs) {
+template <int DT, bool ADD, int QM>
+void launch_rms_mode(long rows, hipStream_t st, void* out, float* out_scales, const uint16_t* x, uint16_t* residual,
+                     const uint16_t* weight, const float* scale, float eps, int K, int gs) {
   const dim3 grid((unsigned)rows);
-  if (K <= 8192) {
-    switch (qm) {
-      case 0: hipLaunchKernelGGL((rms_norm_row_kernel<DT, ADD, 0>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
-      case 1: hipLaunchKernelGGL((rms_norm_row_kernel<DT, ADD, 1>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
-      case 2: hipLaunchKernelGGL((rms_norm_row_kernel<DT, ADD, 2>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
-      default: hipLaunchKernelGGL((rms_norm_row_kernel<DT, ADD, 3>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
-    }
-    return;
-  }
-  switch (qm) {
-    case 0: hipLaunchKernelGGL((rms_norm_kernel<DT, ADD, 0>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
-    case 1: hipLaunchKernelGGL((rms_norm_kernel<DT, ADD, 1>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
-    case 2: hipLaunchKernelGGL((rms_norm_kernel<DT, ADD, 2>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
-    default: hipLaunchKernelGGL((rms_norm_kernel<DT, ADD, 3>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
+  const RowShape s = row_shape(rows, K, true, device_cu_count());      // (the operator asks for 16-byte rows)
+  const dim3 block(s.threads);
+  const int lpg = QM == 2 ? gs / 8 : 1;
+  switch (s.pieces) {
+    case 1: hipLaunchKernelGGL((rms_norm_row_kernel<DT, ADD, QM, 1>), grid, block, 0, st, out, out_scales, x, residual, weight, scale, eps, K, lpg); break;
+    case 2: hipLaunchKernelGGL((rms_norm_row_kernel<DT, ADD, QM, 2>), grid, block, 0, st, out, out_scales, x, residual, weight, scale, eps, K, lpg); break;
+    case 4: hipLaunchKernelGGL((rms_norm_row_kernel<DT, ADD, QM, 4>), grid, block, 0, st, out, out_scales, x, residual, weight, scale, eps, K, lpg); break;
+    default: hipLaunchKernelGGL((rms_norm_kernel<DT, ADD, QM>), grid, dim3(256), 0, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
   }
 }
+
+template <int DT, bool ADD>
+void launch_rms(int qm, long rows, hipStream_t st, void* out, float* out_scales, const uint16_t* x, uint16_t* residual,
+                const uint16_t* weight, const float* scale, float eps, int K, int gs) {
+  switch (qm) {
+    case 0: launch_rms_mode<DT, ADD, 0>(rows, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
+    case 1: launch_rms_mode<DT, ADD, 1>(rows, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
+    case 2: launch_rms_mode<DT, ADD, 2>(rows, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
+    default: launch_rms_mode<DT, ADD, 3>(rows, st, out, out_scales, x, residual, weight, scale, eps, K, gs); break;
+  }
+}
+
+// rows per launch of the kernels that index their 16-byte pieces with 31 bits
+inline long rows_per_launch(int chunks) { return (long)0x7fff0000 / chunks; }
 
 inline unsigned grid_for(long items) {
   long b = (items + 255) / 256;
@@ -459,12 +516,20 @@ extern "C" int mi355q_silu_and_mul(void* out, const void* x, long rows, int d, i
   MQ_REQUIRE(rows >= 0 && d > 0 && d % 8 == 0, "silu_and_mul: bad shape rows=%ld d=%d (d %% 8 == 0)", rows, d);
   if (rows == 0) return 0;
   MQ_REQUIRE(out && x, "silu_and_mul: null pointer");
+  MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "silu_and_mul: dtype %d must be f16 or bf16", dtype);
+  MQ_REQUIRE(!valid_rows || rows <= rows_per_launch(d / 8), "silu_and_mul: too many rows with a row count");
   hipStream_t st = as_stream(stream);
-  unsigned g = grid_for(rows * (d / 8));
-  MQ_DISPATCH_16(dtype,
-    hipLaunchKernelGGL((silu_and_mul_kernel<MI355Q_F16>), dim3(g), dim3(256), 0, st, (uint16_t*)out, (const uint16_t*)x, rows, d, valid_rows, rows_per_count),
-    hipLaunchKernelGGL((silu_and_mul_kernel<MI355Q_BF16>), dim3(g), dim3(256), 0, st, (uint16_t*)out, (const uint16_t*)x, rows, d, valid_rows, rows_per_count),
-    "silu_and_mul");
+  const FastDiv chunks((uint32_t)(d / 8));
+  for (long r0 = 0; r0 < rows; r0 += rows_per_launch(d / 8)) {
+    const uint32_t n = (uint32_t)std::min(rows - r0, rows_per_launch(d / 8));
+    const unsigned g = grid_for((long)n * (d / 8));
+    uint16_t* o = (uint16_t*)out + r0 * d;
+    const uint16_t* xp = (const uint16_t*)x + r0 * 2 * d;
+    if (dtype == MI355Q_F16)
+      hipLaunchKernelGGL((silu_and_mul_kernel<MI355Q_F16>), dim3(g), dim3(256), 0, st, o, xp, n, d, chunks, valid_rows, rows_per_count);
+    else
+      hipLaunchKernelGGL((silu_and_mul_kernel<MI355Q_BF16>), dim3(g), dim3(256), 0, st, o, xp, n, d, chunks, valid_rows, rows_per_count);
+  }
   MQ_LAUNCH_CHECK("silu_and_mul");
   return 0;
 }
@@ -479,19 +544,27 @@ extern "C" int mi355q_fp8_group_quant(uint8_t* out, float* scales, const void* x
   MQ_REQUIRE(group_size == 64 || group_size == 128 || group_size == 256 || group_size == 512,
              "fp8_group_quant: group_size=%d must be 64, 128, 256 or 512", group_size);
   MQ_REQUIRE(K % group_size == 0, "fp8_group_quant: K=%d must be a multiple of group_size=%d", K, group_size);
+  MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "fp8_group_quant: dtype %d must be f16 or bf16", dtype);
+  MQ_REQUIRE(!valid_rows || rows <= rows_per_launch(K / 8), "fp8_group_quant: too many rows with a row count");
   hipStream_t st = as_stream(stream);
-  // whole groups must sit inside one workgroup pass: 256 lanes cover 2048 elements
-  unsigned g = grid_for(rows * (K / 8));
-  if (fuse_silu_mul) {
-    MQ_DISPATCH_16(dtype,
-      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_F16, true>), dim3(g), dim3(256), 0, st, out, scales, (const uint16_t*)x, rows, K, group_size, valid_rows, rows_per_count),
-      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_BF16, true>), dim3(g), dim3(256), 0, st, out, scales, (const uint16_t*)x, rows, K, group_size, valid_rows, rows_per_count),
-      "fp8_group_quant");
-  } else {
-    MQ_DISPATCH_16(dtype,
-      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_F16, false>), dim3(g), dim3(256), 0, st, out, scales, (const uint16_t*)x, rows, K, group_size, valid_rows, rows_per_count),
-      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_BF16, false>), dim3(g), dim3(256), 0, st, out, scales, (const uint16_t*)x, rows, K, group_size, valid_rows, rows_per_count),
-      "fp8_group_quant");
+  const FastDiv chunks((uint32_t)(K / 8));
+  const int lpg = group_size / 8;
+  const bool f16 = dtype == MI355Q_F16;
+  for (long r0 = 0; r0 < rows; r0 += rows_per_launch(K / 8)) {
+    const uint32_t n = (uint32_t)std::min(rows - r0, rows_per_launch(K / 8));
+    // whole groups must sit inside one workgroup pass: 256 lanes cover 2048 elements
+    const unsigned g = grid_for((long)n * (K / 8));
+    uint8_t* o = out + r0 * K;
+    float* sc = scales + r0 * (K / group_size);
+    const uint16_t* xp = (const uint16_t*)x + r0 * K * (fuse_silu_mul ? 2 : 1);
+    if (fuse_silu_mul && f16)
+      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_F16, true>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count);
+    else if (fuse_silu_mul)
+      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_BF16, true>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count);
+    else if (f16)
+      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_F16, false>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count);
+    else
+      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_BF16, false>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count);
   }
   MQ_LAUNCH_CHECK("fp8_group_quant");
   return 0;
@@ -504,8 +577,8 @@ extern "C" int mi355q_fp8_token_quant(uint8_t* out, float* scales, const void* x
   MQ_REQUIRE(out && scales && x, "fp8_token_quant: null pointer");
   hipStream_t st = as_stream(stream);
   MQ_DISPATCH_16(dtype,
-    hipLaunchKernelGGL((token_fp8_quant_kernel<MI355Q_F16>), dim3(rows), dim3(256), 0, st, out, scales, (const uint16_t*)x, K, valid_rows),
-    hipLaunchKernelGGL((token_fp8_quant_kernel<MI355Q_BF16>), dim3(rows), dim3(256), 0, st, out, scales, (const uint16_t*)x, K, valid_rows),
+    launch_token_quant<MI355Q_F16>(rows, K, st, out, scales, (const uint16_t*)x, valid_rows),
+    launch_token_quant<MI355Q_BF16>(rows, K, st, out, scales, (const uint16_t*)x, valid_rows),
     "fp8_token_quant");
   MQ_LAUNCH_CHECK("fp8_token_quant");
   return 0;
@@ -549,16 +622,22 @@ extern "C" int mi355q_moe_sum(void* out, const void* in, long rows, int topk, in
   MQ_REQUIRE(in_dtype == MI355Q_F16 || in_dtype == MI355Q_BF16, "moe_sum: input dtype %d must be f16 or bf16", in_dtype);
   MQ_REQUIRE(out_dtype == in_dtype || out_dtype == MI355Q_F32, "moe_sum: output dtype %d must equal the input's or be f32", out_dtype);
   hipStream_t st = as_stream(stream);
-  unsigned g = grid_for(rows * (K / 8));
-  const uint16_t* p = (const uint16_t*)in;
-  if (in_dtype == MI355Q_F16 && out_dtype == MI355Q_F16)
-    hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F16>), dim3(g), dim3(256), 0, st, out, p, rows, topk, K, valid_rows);
-  else if (in_dtype == MI355Q_F16)
-    hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F32>), dim3(g), dim3(256), 0, st, out, p, rows, topk, K, valid_rows);
-  else if (out_dtype == MI355Q_BF16)
-    hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_BF16>), dim3(g), dim3(256), 0, st, out, p, rows, topk, K, valid_rows);
-  else
-    hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_F32>), dim3(g), dim3(256), 0, st, out, p, rows, topk, K, valid_rows);
+  MQ_REQUIRE(!valid_rows || rows <= rows_per_launch(K / 8), "moe_sum: too many rows with a row count");
+  const FastDiv chunks((uint32_t)(K / 8));
+  for (long r0 = 0; r0 < rows; r0 += rows_per_launch(K / 8)) {
+    const uint32_t n = (uint32_t)std::min(rows - r0, rows_per_launch(K / 8));
+    const unsigned g = grid_for((long)n * (K / 8));
+    const uint16_t* p = (const uint16_t*)in + r0 * topk * K;
+    void* o = (char*)out + r0 * K * (out_dtype == MI355Q_F32 ? 4 : 2);
+    if (in_dtype == MI355Q_F16 && out_dtype == MI355Q_F16)
+      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F16>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows);
+    else if (in_dtype == MI355Q_F16)
+      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F32>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows);
+    else if (out_dtype == MI355Q_BF16)
+      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_BF16>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows);
+    else
+      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_F32>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows);
+  }
   MQ_LAUNCH_CHECK("moe_sum");
   return 0;
 }

@@ -170,6 +170,54 @@ __device__ __forceinline__ void zero_block_columns(uint16_t* out, const int* ids
   }
 }
 
+// n / d for a divisor known on the host and n < 2^31: a multiplication and two shifts, where the hardware-less 32- and
+// 64-bit divisions of a kernel's index arithmetic take 30 .. 100 instructions
+struct FastDiv {
+  uint32_t d, mul, shift;
+  FastDiv() = default;
+  explicit FastDiv(uint32_t div) : d(div) {
+    shift = 0;
+    while (shift < 31 && (1u << shift) < div) ++shift;                      // 2^shift >= d
+    mul = (uint32_t)(((uint64_t)1 << 32) * (((uint64_t)1 << shift) - div) / div + 1);
+  }
+  __device__ __forceinline__ uint32_t div(uint32_t n) const { return (__umulhi(n, mul) + n) >> shift; }
+};
+
+// Launch shape of the kernels that hold one row of K elements of 16 bits in registers (8 per lane and piece) between
+// two passes over it: threads per row and pieces per lane.  Four pieces per lane at most where there are rows
+// enough to fill the chip; with fewer rows than that a row is spread over more wavefronts, because the launch then
+// takes as long as one row does.  pieces == 0: the row is too long, not a whole number of pieces or not aligned.
+struct RowShape {
+  int threads, pieces;
+};
+inline RowShape row_shape(long rows, int K, bool aligned, int cus) {
+  const int chunks = K / 8;
+  if (!aligned || K % 8 != 0 || chunks > 8 * 1024) return {256, 0};
+  const int most = rows >= 4L * cus ? 4 : rows >= 2L * cus ? 2 : 1;
+  int threads = 256;
+  while (threads < 1024 && chunks > threads * most) threads *= 2;
+  const int p = (chunks + threads - 1) / threads;
+  return {threads, p <= 1 ? 1 : p <= 2 ? 2 : p <= 4 ? 4 : 8};
+}
+__device__ __forceinline__ float block_sum(float x, float* red) {
+  x = wave_sum(x);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  float s = red[0] + red[1];
+  const int n = (int)(blockDim.x >> 6);                                    // 4, 8 or 16 wavefronts
+  for (int i = 2; i < n; i += 2) s += red[i] + red[i + 1];
+  return s;
+}
+// maximum over the workgroup (up to 16 wavefronts, all lanes active); `red` is 16 floats of LDS
+__device__ __forceinline__ float block_max(float x, float* red) {
+  x = wave_max(x);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  float m = red[0];
+  for (int i = 1; i < (int)(blockDim.x >> 6); ++i) m = fmaxf(m, red[i]);
+  return m;
+}
+
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 int device_cu_count();

@@ -145,12 +145,12 @@ void static_int8(const Tensor& out, const Tensor& input, const Tensor& scale) {
   if (input.numel() == 0) return;
   const Tensor x = input.contiguous();
   const Rows r(x);
-  const Tensor sc = as(scale, at::kFloat);
+  const Tensor sc = as(scale, scale.scalar_type() == x.scalar_type() ? x.scalar_type() : at::kFloat);
   TORCH_CHECK(sc.numel() == 1 || sc.numel() == r.len, "static_scaled_int8_quant: scale must have 1 or K=", r.len,
               " entries, got ", sc.numel());
   const OnDevice on(x);
-  check(mi355q_static_int8_quant(static_cast<int8_t*>(out.data_ptr()), x.data_ptr(), static_cast<const float*>(sc.data_ptr()),
-                                 sc.numel() > 1, r.rows, r.len, require_dtype(x.scalar_type()), on.stream()),
+  check(mi355q_static_int8_quant_typed(static_cast<int8_t*>(out.data_ptr()), x.data_ptr(), sc.data_ptr(), dtype_code(sc.scalar_type()),
+                                       sc.numel() > 1, r.rows, r.len, require_dtype(x.scalar_type()), on.stream()),
         "static_int8_quant");
 }
 

@@ -297,9 +297,8 @@ PyObject* py_w8a8_static_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
     const NoGil free_gil;
     const Tensor q = empty({M, m.K}, at::kChar, x);
     out = empty(with_last(x, m.N), m.out_dtype, x);
-    const Tensor in_f32 = it->to(at::kFloat);
-    check(mi355q_static_int8_quant(static_cast<int8_t*>(q.data_ptr()), x.data_ptr(), static_cast<const float*>(in_f32.data_ptr()), 1, M,
-                                   m.K, dtype_code(x.scalar_type()), stream),
+    check(mi355q_static_int8_quant_typed(static_cast<int8_t*>(q.data_ptr()), x.data_ptr(), it->data_ptr(), dtype_code(x.scalar_type()),
+                                         1, M, m.K, dtype_code(x.scalar_type()), stream),
           "static_int8_quant");
     int8_mm(m, q, Tensor(), out, M, top, ws, stream);
   }

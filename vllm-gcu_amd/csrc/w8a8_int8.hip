@@ -534,66 +534,149 @@ __device__ __forceinline__ int8_t sat_rne_s8(float y) {
   return (int8_t)(int)y;
 }
 
-// one workgroup per token row: absmax -> scale = absmax / 127 -> q = rne(x * (127 / absmax))
+// the 8 values of a piece of 16-bit elements
 template <int DT>
-__global__ void __launch_bounds__(256)
-dynamic_int8_quant_kernel(int8_t* out, float* scales, const void* x, int K, const int* valid_rows) {
-  const int row = blockIdx.x;
-  if (valid_rows && row >= *valid_rows) return;
-  __shared__ float red[4];
-  float mx = 0.f;
-  // 16-bit inputs with K % 8 == 0: 16-byte loads, 8-byte stores (8 elements per lane and step)
-  const bool vec8 = DT != MI355Q_F32 && (K & 7) == 0;
-  const uint16_t* xr = (const uint16_t*)x + (long)row * K;
-  if (vec8) {
-    for (int c = threadIdx.x; c < (K >> 3); c += 256) {
-      const u4 v = *(const u4*)(xr + 8 * c);
+__device__ __forceinline__ void unpack_half8(const u4& v, float* f) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        mx = fmaxf(mx, fabsf(ld_half<DT>((uint16_t)(v[i] & 0xffffu))));
-        mx = fmaxf(mx, fabsf(ld_half<DT>((uint16_t)(v[i] >> 16))));
-      }
-    }
-  } else {
-    for (int k = threadIdx.x; k < K; k += 256) mx = fmaxf(mx, fabsf(ld_act<DT>(x, (long)row * K + k)));
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = ld_half<DT>((uint16_t)(v[i] & 0xffffu));
+    f[2 * i + 1] = ld_half<DT>((uint16_t)(v[i] >> 16));
   }
-  mx = wave_max(mx);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+__device__ __forceinline__ u2 pack_s8x8(const float* y) {
+  uint32_t q[2] = {0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) q[e >> 2] |= ((uint32_t)(uint8_t)sat_rne_s8(y[e])) << (8 * (e & 3));
+  return (u2){q[0], q[1]};
+}
+
+// one workgroup per token row: absmax -> scale = absmax / 127 -> q = rne(x * (127 / absmax)).  The row is read once,
+// P pieces of 16 bytes per lane with all loads in flight together, and quantised from registers: bound by HBM at
+// prefill sizes (the loop below reads every row twice, one piece at a time).
+template <int DT, int P>
+__global__ void __launch_bounds__(1024)
+dynamic_int8_quant_row_kernel(int8_t* out, float* scales, const uint16_t* x, int K, const int* valid_rows) {
+  const long row = blockIdx.x;
+  if (valid_rows && row >= *valid_rows) return;
+  __shared__ float red[16];
+  const int chunks = K >> 3, nt = blockDim.x;
+  const uint16_t* xr = x + row * K;
+  u4 v[P];
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    const int c = threadIdx.x + nt * i;
+    v[i] = *(const u4*)(xr + 8 * (c < chunks ? c : 0));     // (past the end: the first piece again, for the maximum)
+  }
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    float y[8];
+    unpack_half8<DT>(v[i], y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(y[e]));
+  }
+  mx = block_max(mx, red);
   if (threadIdx.x == 0) scales[row] = mx / 127.0f;
   const float inv = 127.0f / mx;                // inf for an all-zero row
-  if (vec8) {
-    for (int c = threadIdx.x; c < (K >> 3); c += 256) {
-      const u4 v = *(const u4*)(xr + 8 * c);    // the row was just read: an L2 hit
-      uint32_t q[2] = {0u, 0u};
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t w = v[e >> 1];
-        float y = ld_half<DT>((uint16_t)((e & 1) ? (w >> 16) : (w & 0xffffu))) * inv;
-        if (y != y) y = 0.f;                    // 0 * inf
-        q[e >> 2] |= ((uint32_t)(uint8_t)sat_rne_s8(y)) << (8 * (e & 3));
-      }
-      *(u2*)(out + (long)row * K + 8 * c) = (u2){q[0], q[1]};
+  for (int i = 0; i < P; ++i) {
+    const int c = threadIdx.x + nt * i;
+    float y[8];
+    unpack_half8<DT>(v[i], y);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      y[e] *= inv;
+      if (y[e] != y[e]) y[e] = 0.f;             // 0 * inf
     }
-    return;
-  }
-  for (int k = threadIdx.x; k < K; k += 256) {
-    float y = ld_act<DT>(x, (long)row * K + k) * inv;
-    if (y != y) y = 0.f;                        // 0 * inf
-    out[(long)row * K + k] = sat_rne_s8(y);
+    if (c < chunks) *(u2*)(out + row * K + 8 * c) = pack_s8x8(y);
   }
 }
 
-// static: the reciprocal of the scale is rounded to the input dtype first
+// any type, row length and alignment, one element at a time
 template <int DT>
 __global__ void __launch_bounds__(256)
-static_int8_quant_kernel(int8_t* out, const void* x, const float* scale, int per_channel, long total, int K) {
+dynamic_int8_quant_kernel(int8_t* out, float* scales, const void* x, int K, const int* valid_rows) {
+  const long row = blockIdx.x;
+  if (valid_rows && row >= *valid_rows) return;
+  __shared__ float red[16];
+  float mx = 0.f;
+  for (int k = threadIdx.x; k < K; k += 256) mx = fmaxf(mx, fabsf(ld_act<DT>(x, row * K + k)));
+  mx = block_max(mx, red);
+  if (threadIdx.x == 0) scales[row] = mx / 127.0f;
+  const float inv = 127.0f / mx;                // inf for an all-zero row
+  for (int k = threadIdx.x; k < K; k += 256) {
+    float y = ld_act<DT>(x, row * K + k) * inv;
+    if (y != y) y = 0.f;                        // 0 * inf
+    out[row * K + k] = sat_rne_s8(y);
+  }
+}
+
+template <int DT>
+void launch_dynamic_quant(int M, int K, hipStream_t st, int8_t* out, float* scales, const void* x, const int* valid_rows) {
+  const bool ok = DT != MI355Q_F32 && (((uintptr_t)x & 15) | ((uintptr_t)out & 7)) == 0;
+  const RowShape s = row_shape(M, K, ok, device_cu_count());
+  const dim3 grid((unsigned)M), block(s.threads);
+  constexpr int D = DT == MI355Q_F32 ? MI355Q_F16 : DT;
+  const uint16_t* xh = (const uint16_t*)x;
+  switch (s.pieces) {
+    case 1: hipLaunchKernelGGL((dynamic_int8_quant_row_kernel<D, 1>), grid, block, 0, st, out, scales, xh, K, valid_rows); break;
+    case 2: hipLaunchKernelGGL((dynamic_int8_quant_row_kernel<D, 2>), grid, block, 0, st, out, scales, xh, K, valid_rows); break;
+    case 4: hipLaunchKernelGGL((dynamic_int8_quant_row_kernel<D, 4>), grid, block, 0, st, out, scales, xh, K, valid_rows); break;
+    case 8: hipLaunchKernelGGL((dynamic_int8_quant_row_kernel<D, 8>), grid, block, 0, st, out, scales, xh, K, valid_rows); break;
+    default: hipLaunchKernelGGL((dynamic_int8_quant_kernel<DT>), grid, dim3(256), 0, st, out, scales, x, K, valid_rows); break;
+  }
+}
+
+// static: the reciprocal of the scale (in f32, or SDT = the input type where the scales are stored in it) is rounded to
+// the input dtype first.  One element per lane: any type, row length and alignment.
+template <int DT, int SDT>
+__global__ void __launch_bounds__(256)
+static_int8_quant_kernel(int8_t* out, const void* x, const void* scale, int per_channel, long total, int K) {
   long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
-  float inv = 1.0f / scale[per_channel ? (int)(i % K) : 0];
+  float inv = 1.0f / ld_act<SDT>(scale, per_channel ? (int)(i % K) : 0);
   if (DT != MI355Q_F32) inv = Elem<DT == MI355Q_F32 ? MI355Q_F16 : DT>::to_f32(Elem<DT == MI355Q_F32 ? MI355Q_F16 : DT>::from_f32(inv));
   out[i] = sat_rne_s8(ld_act<DT>(x, i) * inv);
+}
+
+// the same for 16-bit inputs with K % 8 == 0, eight elements per lane: 16-byte loads, 8-byte stores
+template <int DT, int SDT>
+__global__ void __launch_bounds__(256)
+static_int8_quant_vec_kernel(int8_t* out, const uint16_t* x, const void* scale, int per_channel, long pieces, int chunks) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= pieces) return;
+  const int c = (int)(i % chunks);
+  const u4 v = *(const u4*)(x + 8 * i);
+  float s[8];
+  if (!per_channel) {
+    const float one = ld_act<SDT>(scale, 0);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = one;
+  } else if (SDT == MI355Q_F32) {
+    const f4 a = *(const f4*)((const float*)scale + 8 * c), b = *(const f4*)((const float*)scale + 8 * c + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = a[e], s[4 + e] = b[e];
+  } else {
+    unpack_half8<DT>(*(const u4*)((const uint16_t*)scale + 8 * c), s);
+  }
+  float y[8];
+  unpack_half8<DT>(v, y);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] *= Elem<DT>::to_f32(Elem<DT>::from_f32(1.0f / s[e]));
+  *(u2*)(out + 8 * i) = pack_s8x8(y);
+}
+
+template <int DT, int SDT>
+void launch_static_quant(long total, int K, hipStream_t st, int8_t* out, const void* x, const void* scale, int per_channel) {
+  if constexpr (DT != MI355Q_F32) {
+    if (K % 8 == 0 && ((((uintptr_t)x | (uintptr_t)scale) & 15) | ((uintptr_t)out & 7)) == 0) {
+      hipLaunchKernelGGL((static_int8_quant_vec_kernel<DT, SDT>), dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0, st, out,
+                         (const uint16_t*)x, scale, per_channel, total / 8, K / 8);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((static_int8_quant_kernel<DT, SDT>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, out, x, scale,
+                     per_channel, total, K);
 }
 
 // silu(x[:, :d]) * x[:, d:] rounded to the input dtype, then quantised like
@@ -903,35 +986,45 @@ extern "C" int mi355q_dynamic_int8_quant(int8_t* out, float* scales, const void*
   MQ_REQUIRE(out && scales && x, "dynamic_int8_quant: null pointer");
   hipStream_t st = as_stream(stream);
   if (dtype == MI355Q_F16)
-    hipLaunchKernelGGL((dynamic_int8_quant_kernel<MI355Q_F16>), dim3(M), dim3(256), 0, st, out, scales, x, K, valid_rows);
+    launch_dynamic_quant<MI355Q_F16>(M, K, st, out, scales, x, valid_rows);
   else if (dtype == MI355Q_BF16)
-    hipLaunchKernelGGL((dynamic_int8_quant_kernel<MI355Q_BF16>), dim3(M), dim3(256), 0, st, out, scales, x, K, valid_rows);
+    launch_dynamic_quant<MI355Q_BF16>(M, K, st, out, scales, x, valid_rows);
   else if (dtype == MI355Q_F32)
-    hipLaunchKernelGGL((dynamic_int8_quant_kernel<MI355Q_F32>), dim3(M), dim3(256), 0, st, out, scales, x, K, valid_rows);
+    launch_dynamic_quant<MI355Q_F32>(M, K, st, out, scales, x, valid_rows);
   else
     MQ_REQUIRE(false, "dynamic_int8_quant: bad dtype %d", dtype);
   MQ_LAUNCH_CHECK("dynamic_int8_quant");
   return 0;
 }
 
-extern "C" int mi355q_static_int8_quant(int8_t* out, const void* x, const float* scale, int per_channel,
-                                        int M, int K, int dtype, void* stream) {
+extern "C" int mi355q_static_int8_quant_typed(int8_t* out, const void* x, const void* scale, int scale_dtype, int per_channel,
+                                              int M, int K, int dtype, void* stream) {
   MQ_REQUIRE(M >= 0 && K > 0, "static_int8_quant: bad shape M=%d K=%d", M, K);
   if (M == 0) return 0;
   MQ_REQUIRE(out && scale && x, "static_int8_quant: null pointer");
+  MQ_REQUIRE(scale_dtype == MI355Q_F32 || scale_dtype == dtype, "static_int8_quant: scales of type %d with inputs of type %d",
+             scale_dtype, dtype);
   const long total = (long)M * K;
-  const unsigned blocks = (unsigned)((total + 255) / 256);
   hipStream_t st = as_stream(stream);
-  if (dtype == MI355Q_F16)
-    hipLaunchKernelGGL((static_int8_quant_kernel<MI355Q_F16>), dim3(blocks), dim3(256), 0, st, out, x, scale, per_channel, total, K);
+  if (dtype == MI355Q_F16 && scale_dtype == MI355Q_F16)
+    launch_static_quant<MI355Q_F16, MI355Q_F16>(total, K, st, out, x, scale, per_channel);
+  else if (dtype == MI355Q_F16)
+    launch_static_quant<MI355Q_F16, MI355Q_F32>(total, K, st, out, x, scale, per_channel);
+  else if (dtype == MI355Q_BF16 && scale_dtype == MI355Q_BF16)
+    launch_static_quant<MI355Q_BF16, MI355Q_BF16>(total, K, st, out, x, scale, per_channel);
   else if (dtype == MI355Q_BF16)
-    hipLaunchKernelGGL((static_int8_quant_kernel<MI355Q_BF16>), dim3(blocks), dim3(256), 0, st, out, x, scale, per_channel, total, K);
+    launch_static_quant<MI355Q_BF16, MI355Q_F32>(total, K, st, out, x, scale, per_channel);
   else if (dtype == MI355Q_F32)
-    hipLaunchKernelGGL((static_int8_quant_kernel<MI355Q_F32>), dim3(blocks), dim3(256), 0, st, out, x, scale, per_channel, total, K);
+    launch_static_quant<MI355Q_F32, MI355Q_F32>(total, K, st, out, x, scale, per_channel);
   else
     MQ_REQUIRE(false, "static_int8_quant: bad dtype %d", dtype);
   MQ_LAUNCH_CHECK("static_int8_quant");
   return 0;
+}
+
+extern "C" int mi355q_static_int8_quant(int8_t* out, const void* x, const float* scale, int per_channel, int M, int K, int dtype,
+                                        void* stream) {
+  return mi355q_static_int8_quant_typed(out, x, scale, MI355Q_F32, per_channel, M, K, dtype, stream);
 }
 
 extern "C" int mi355q_moe_expert_int8_quant(int8_t* out, const void* x, const void* scale_rec,
