@@ -179,6 +179,12 @@ int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w, const flo
                               const void* bias, int M, int N, int K, long ldx, long ldw, long ldo,
                               int out_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
+/* No counterpart in the reference.  Whether an 8-bit layer in the kslab order with M rows is taken by the kernel for
+ * a few dozen to some hundred rows (csrc/q8_mid.hip) when mi355q_fp8_block_gemm_ws (kind 0), mi355q_fp8_scaled_gemm_ws
+ * (kind 1) or mi355q_w8a8_int8_gemm_ws (kind 2) is called with *workspace_bytes bytes of workspace (0: none needed).
+ * 1: it is, and those entry points are ahead of mi355q_kcontig_gemm; 0: it is not. */
+int mi355q_q8_mid_plan(int kind, int M, int N, int K, size_t* workspace_bytes);
+
 /* ---- W8A8 int8 -------------------------------------------------------------
  * Replaces topsatenDotBiasQuant as called by cutlass_scaled_mm
  * (csrc/src/cutlass_scaled_mm.cpp:12-36) and dot_bias_quant

@@ -1,0 +1,65 @@
+"""The 8-bit kernel for a few dozen to some hundred rows (csrc/q8_mid.hip) through the operators that choose it:
+row counts around every tile edge, column counts that are and are not a multiple of eight column tiles, odd numbers of K
+blocks, one and several K ranges, with and without bias.  int8 is exact; fp8 is compared with a float64 product."""
+import pytest
+import torch
+
+from vllm_gcu_amd import _lib
+from vllm_gcu_amd.kernels import _custom_ops as ops
+from vllm_gcu_amd.kernels import _runtime as rt
+from vllm_gcu_amd.kernels.quantization import rearrange
+
+pytestmark = pytest.mark.gpu
+# (M, N, K): tiles of 32, 64 and 128 rows, with and without K ranges
+SHAPES = [(17, 64, 384), (31, 320, 128), (33, 512, 1152), (48, 1024, 7168), (63, 640, 640), (64, 4096, 2048), (65, 1024, 1024),
+          (96, 3072, 3584), (127, 256, 4096), (129, 1024, 5120), (130, 4096, 7168), (200, 2048, 1408), (257, 4608, 3584),
+          (511, 4096, 4096), (512, 8192, 2048)]
+
+
+def _planned(kind, M, N, K):
+    want = rt.host.q8_mid_plan(kind, M, N, K)
+    print(f"case q8 mid kind={kind} M={M} N={N} K={K} workspace={want}", flush=True)
+    assert want >= 0, "another kernel takes this shape: the case tests nothing"
+
+
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_int8(M, N, K, with_bias):
+    _planned(_lib.Q_INT8, M, N, K)
+    torch.manual_seed(M + N + K)
+    x = torch.randint(-128, 128, (M, K), dtype=torch.int8, device="cuda")
+    w = torch.randint(-128, 128, (N, K), dtype=torch.int8, device="cuda")
+    xs, ws = torch.rand(M, 1, device="cuda") * 0.1, torch.rand(N, 1, device="cuda") * 0.01
+    bias = torch.randn(N, device="cuda").half() if with_bias else None
+    out = torch.full((M, N), float("nan"), device="cuda").half()
+    torch.ops._C.cutlass_scaled_mm(out, x, rearrange.to_kslab(w).t(), xs, ws, bias)
+    acc = (x.double() @ w.double().t()).float()              # exact: below 2^53, and below 2^24 where it matters not
+    want = acc * xs * ws.view(1, N)
+    if with_bias:
+        want = want + bias.float()
+    assert torch.equal(out, want.half())
+
+
+@pytest.mark.parametrize("M,N,K", [s for s in SHAPES if s[1] % 128 == 0])
+def test_fp8_block_and_scaled(M, N, K):
+    torch.manual_seed(M + N + K)
+    x = (torch.randn(M, K, device="cuda") * 40).to(torch.float8_e4m3fn)
+    w = (torch.randn(N, K, device="cuda") * 40).to(torch.float8_e4m3fn)
+    wk = rearrange.to_kslab(w)
+    xb, wb = torch.rand(M, K // 128, device="cuda") * 0.01 + 0.001, torch.rand(N // 128, K // 128, device="cuda") * 0.01 + 0.001
+    xd = x.double().view(M, K // 128, 128) * xb.double()[..., None]
+    wd = w.double().view(N // 128, 128, K // 128, 128) * wb.double()[:, None, :, None]
+    want = xd.view(M, K) @ wd.view(N, K).t()
+    _planned(_lib.Q_FP8_BLOCK, M, N, K)
+    for bias in (None, torch.randn(N, device="cuda").bfloat16()):
+        out = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+        torch.ops._C.linear_quant(out, x, wk, bias, xb, wb)
+        ref = want if bias is None else want + bias.double()
+        assert float((out.double() - ref).norm() / ref.norm()) < 3e-3        # one rounding to bf16
+    _planned(1, M, N, K)
+    for xs, ws in ((torch.rand(M, 1, device="cuda") * 0.01, torch.rand(N, 1, device="cuda") * 0.01),
+                   (torch.full((1,), 0.01, device="cuda"), torch.full((1,), 0.003, device="cuda"))):
+        out = torch.full((M, N), float("nan"), device="cuda").half()
+        torch.ops._C.cutlass_scaled_mm(out, x, wk.t(), xs, ws, None)
+        ref = (x.double() @ w.double().t()) * xs.double().view(-1, 1) * ws.double().view(1, -1)
+        assert float((out.double() - ref).norm() / ref.norm()) < 1e-3

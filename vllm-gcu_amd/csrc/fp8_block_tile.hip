@@ -33,6 +33,10 @@ namespace mi355q {
 int kcontig_fp8_pc_launch(void* out, const void* a, const void* w, const float* a_scale, int scale_per_row,
                           const float* w_scale, int scale_per_col, const void* bias, int M, int K, int N,
                           int out_dtype, int w_layout, hipStream_t st);
+bool q8_mid_wanted(int mode, int M, int N, int K, size_t* bytes);
+int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
+                  int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* partial,
+                  hipStream_t st);
 namespace {
 
 constexpr int FTM = 256, FTN = 128, FTKB = 128;
@@ -577,6 +581,8 @@ int fp8_scales_kmajor_launch(const float* xs, float* out, int rows, int KB, long
 constexpr size_t F8_SPLITK_BYTES = (size_t)64 << 20;
 constexpr size_t F8_WS_OFFSET = (size_t)1 << 20;     // the first MiB of a workspace belongs to the W4A16 arrival counters
 
+}  // namespace
+
 // K ranges for a shape: as many as put about one 256 x 128 tile on every CU, each at least eight K
 // blocks long, a divisor of the K block count, partial sums within 64 MiB.  1: no split.
 int fp8_ksplits(int M, int N, int K) {
@@ -589,6 +595,8 @@ int fp8_ksplits(int M, int N, int K) {
   while (s > 1 && (nt % s != 0 || (size_t)s * M * N * sizeof(float) > F8_SPLITK_BYTES)) --s;
   return s < 1 ? 1 : (int)s;
 }
+
+namespace {
 
 template <int DT, bool PC>
 int launch_f8(const F8Args& a, hipStream_t st);
@@ -763,6 +771,10 @@ extern "C" int mi355q_fp8_block_gemm_ws(void* out, const void* x, const void* w,
              "fp8_block_gemm: operands too large for 32-bit tile offsets (M=%d N=%d K=%d)", M, N, K);
   MQ_REQUIRE(ldo >= N && ldo % 4 == 0, "fp8_block_gemm: output row stride %ld must be >= N and a multiple of 4", ldo);
   MQ_REQUIRE(out_dtype == MI355Q_F16 || out_dtype == MI355Q_BF16, "fp8_block_gemm: bad out dtype %d", out_dtype);
+  size_t mid_bytes = 0;
+  if (kslab && q8_mid_wanted(0, M, N, K, &mid_bytes) && (mid_bytes == 0 || (workspace && workspace_bytes >= F8_WS_OFFSET + mid_bytes)))
+    return q8_mid_launch(0, out, x, w, x_scale, 0, w_scale, 0, bias, 0, M, N, K, ldx, ldo, out_dtype,
+                         mid_bytes ? (char*)workspace + F8_WS_OFFSET : nullptr, as_stream(stream));
   F8Args a;
   a.out = out; a.x = (const uint8_t*)x; a.w = (const uint8_t*)w; a.x_scale = x_scale; a.w_scale = w_scale;
   a.bias = bias; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldw = ldw; a.ldo = ldo;
@@ -796,6 +808,12 @@ extern "C" int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w
   MQ_REQUIRE(!kslab || N % 64 == 0, "fp8_scaled_gemm: weights in the kslab order need N=%d %% 64 == 0", N);
   MQ_REQUIRE(ldx >= K && (kslab || ldw >= K) && ldo >= N,
              "fp8_scaled_gemm: row strides (%ld, %ld, %ld) must cover K=%d / N=%d", ldx, ldw, ldo, K, N);
+  size_t mid_bytes = 0;
+  if (kslab && ldx % 16 == 0 && ldo % 4 == 0 && (size_t)128 * (size_t)ldx < ((size_t)1 << 32) &&
+      (out_dtype == MI355Q_F16 || out_dtype == MI355Q_BF16) && q8_mid_wanted(1, M, N, K, &mid_bytes) &&
+      (mid_bytes == 0 || (workspace && workspace_bytes >= F8_WS_OFFSET + mid_bytes)))
+    return q8_mid_launch(1, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, 0, M, N, K, ldx, ldo,
+                         out_dtype, mid_bytes ? (char*)workspace + F8_WS_OFFSET : nullptr, as_stream(stream));
   // the MFMA tile kernel from 65 rows on when its 256 x 128 tiles fill a good part of the chip; below
   // (and for shapes it does not take) the weight-streaming kernel, which wants dense operands
   const long tiles = (long)((M + FTM - 1) / FTM) * (N / FTN);

@@ -251,13 +251,13 @@ struct Int8Mm {
 };
 
 // q [M, K] int8 with one f32 scale per row (or none): GIL held on entry, `ws` is the stream's scratch
-void int8_mm(const Int8Mm& m, const Tensor& q, const Tensor& xs, const Tensor& out, int64_t M, int64_t top, const Scratch& ws,
-             void* stream) {
+void int8_mm(const Int8Mm& m, const Tensor& q, const Tensor& xs, const Tensor& out, int64_t M, int64_t top, bool mid,
+             const Scratch& ws, void* stream) {
   const float* xp = static_cast<const float*>(ptr(xs));
   const float* wp = static_cast<const float*>(m.ws.data_ptr());
   // decode-sized M: the weight-streaming kernel (same int32 sums, same epilogue order: bit-identical results)
   // reads kslab weights about twice as fast as the tile kernel
-  if (M <= int8_stream_rows(m.K, m.N, top)) {
+  if (!mid && M <= int8_stream_rows(m.K, m.N, top)) {
     check(mi355q_kcontig_gemm(out.data_ptr(), q.data_ptr(), m.w.data_ptr(), xp, wp, ptr(m.bias), 2, 0, M, m.K, m.N, MI355Q_F16,
                               dtype_code(m.out_dtype), 1, stream),
           "kcontig_gemm");
@@ -269,7 +269,11 @@ void int8_mm(const Int8Mm& m, const Tensor& q, const Tensor& xs, const Tensor& o
         "w8a8_int8_gemm");
 }
 
-size_t int8_scratch(const Int8Mm& m, int64_t M, int64_t top) {
+// bytes of scratch; mid: the kernel for some hundred rows takes the layer
+size_t int8_scratch(const Int8Mm& m, int64_t M, int64_t top, bool& mid) {
+  size_t need = 0;
+  mid = mi355q_q8_mid_plan(2, M, m.N, m.K, &need);
+  if (mid) return need;
   return M <= int8_stream_rows(m.K, m.N, top) ? 0 : mi355q_w8a8_int8_workspace_bytes(M, m.N, m.K);
 }
 
@@ -290,7 +294,8 @@ PyObject* py_w8a8_static_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
   const int64_t M = x.numel() / m.K;
   const OnDevice on(x);
   void* stream = on.stream();
-  const size_t need = int8_scratch(m, M, top);
+  bool mid;
+  const size_t need = int8_scratch(m, M, top, mid);
   const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
   Tensor out;
   {
@@ -300,7 +305,7 @@ PyObject* py_w8a8_static_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
     check(mi355q_static_int8_quant_typed(static_cast<int8_t*>(q.data_ptr()), x.data_ptr(), it->data_ptr(), dtype_code(x.scalar_type()),
                                          1, M, m.K, dtype_code(x.scalar_type()), stream),
           "static_int8_quant");
-    int8_mm(m, q, Tensor(), out, M, top, ws, stream);
+    int8_mm(m, q, Tensor(), out, M, top, mid, ws, stream);
   }
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -322,7 +327,8 @@ PyObject* py_int8_dynamic_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
   const int64_t M = x.numel() / m.K;
   const OnDevice on(x);
   void* stream = on.stream();
-  const size_t need = int8_scratch(m, M, top);
+  bool mid;
+  const size_t need = int8_scratch(m, M, top, mid);
   const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
   Tensor out;
   {
@@ -332,7 +338,7 @@ PyObject* py_int8_dynamic_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
     check(mi355q_dynamic_int8_quant(static_cast<int8_t*>(q.data_ptr()), static_cast<float*>(xs.data_ptr()), x.data_ptr(), M, m.K,
                                     dtype_code(x.scalar_type()), nullptr, stream),
           "dynamic_int8_quant");
-    int8_mm(m, q, xs, out, M, top, ws, stream);
+    int8_mm(m, q, xs, out, M, top, mid, ws, stream);
   }
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
@@ -384,14 +390,17 @@ PyObject* py_fp8_block_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
   if (x.size(-1) != K || K % 128 || N % 128 || wt->scalar_type() != at::kFloat8_e4m3fn || !is_kslab(*wt) ||
       !dense(*st, at::kFloat, N / 128 * (K / 128)) || (!quantise && !dense(xs, at::kFloat, M * (K / 128))))
     return no();
-  const int64_t need = fp8_tile_plan(M, N, K, PyLong_AsLongLong(a[3]), PyLong_AsLongLong(a[4]));
+  int64_t need = fp8_tile_plan(M, N, K, PyLong_AsLongLong(a[3]), PyLong_AsLongLong(a[4]));
+  size_t mid_need = 0;
+  const bool mid = mi355q_q8_mid_plan(0, M, N, K, &mid_need);
+  if (mid) need = mid_need;
   const at::ScalarType od = quantise ? x.scalar_type() : at::kBFloat16;
   const OnDevice on(x);
   void* stream = on.stream();
   Scratch ws{nullptr, 0};
   if (need >= 0) {
     // behind the partial sums of a K split (or the first MiB): room for the activation scales in K block major order
-    const int64_t stage = PyObject_IsTrue(a[5]) ? (M + 15) / 16 * 16 * (K / 128) * 4 : 0;
+    const int64_t stage = !mid && PyObject_IsTrue(a[5]) ? (M + 15) / 16 * 16 * (K / 128) * 4 : 0;
     const int64_t total = (need ? need : stage ? (1 << 20) : 0) + stage;
     if (total) ws = workspace(x, stream, total);
   }
@@ -438,7 +447,8 @@ PyObject* py_fp8_scaled_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
     return no();
   const OnDevice on(x);
   void* stream = on.stream();
-  const size_t need = mi355q_fp8_gemm_workspace_bytes(M, N, K);
+  size_t need = 0;
+  if (!mi355q_q8_mid_plan(1, M, N, K, &need)) need = mi355q_fp8_gemm_workspace_bytes(M, N, K);
   const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
   const int dt = dtype_code(x.scalar_type());
   Tensor out;
@@ -464,6 +474,13 @@ PyObject* py_fp8_scaled_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
   }
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
+}
+
+// (kind, M, N, K) -> bytes of workspace, or -1 where the kernel for some hundred rows does not take the layer
+PyObject* py_q8_mid_plan(PyObject*, PyObject* const* a, Py_ssize_t) {
+  size_t need = 0;
+  const bool mid = mi355q_q8_mid_plan(PyLong_AsLong(a[0]), PyLong_AsLong(a[1]), PyLong_AsLong(a[2]), PyLong_AsLong(a[3]), &need);
+  return PyLong_FromLongLong(mid ? static_cast<int64_t>(need) : -1);
 }
 
 // ---- fused MoE ---------------------------------------------------------------------------------------------
@@ -644,6 +661,7 @@ PyMethodDef kMethods[] = {
     MQ_FAST("fp8_block_layer", py_fp8_block_layer),
     MQ_FAST("fp8_scaled_layer", py_fp8_scaled_layer),
     MQ_FAST("fp8_tile_plan", py_fp8_tile_plan),
+    MQ_FAST("q8_mid_plan", py_q8_mid_plan),
     MQ_FAST("fused_topk", py_fused_topk),
     MQ_FAST("grouped_topk", py_grouped_topk),
     MQ_FAST("fused_experts", py_fused_experts),

@@ -20,6 +20,10 @@
 #include "common.h"
 
 namespace mi355q {
+bool q8_mid_wanted(int mode, int M, int N, int K, size_t* bytes);
+int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
+                  int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* partial,
+                  hipStream_t st);
 namespace {
 
 constexpr int TM = 256, TKB = 128;                // tile rows of x, bytes of K per LDS tile row
@@ -789,6 +793,8 @@ w8a8_splitk_epilogue_kernel(I8Args a) {
 constexpr size_t I8_SPLITK_BYTES = (size_t)64 << 20;
 constexpr size_t I8_WS_OFFSET = (size_t)1 << 20;     // the first MiB of a workspace belongs to the W4A16 arrival counters
 
+}  // namespace
+
 // K ranges for a shape: as many as put about one 256 x 128 tile on every CU, each at least eight K
 // tiles long, a divisor of the K tile count, partial sums within 64 MiB.  1: no split.
 int int8_ksplits(int M, int N, int K) {
@@ -820,6 +826,51 @@ int int8_ksplits_wide(int M, int N, int K) {
   return s < 2 ? 0 : (int)s;
 }
 
+// Tile width.  One workgroup per CU works through the output tiles in rounds; a last round that is
+// only part full idles the rest of the chip for a whole tile time.  Measured per round of 256 CUs on
+// K = 8192 (256 rows x TN columns per CU): TN = 256: 101 us, 224: 98.8 us, 128: 55 us -- the widest
+// tile is the cheapest per column.  So: as many FULL rounds of 256-wide tiles as the columns give, and
+// the remaining columns as a second launch with the width that wastes least (M 2048, N 28672: three
+// rounds of 256 and one of 128 instead of four of 224: 395 -> 387 us; under the profiler the two
+// launches last 315-337 us and 65-70 us, i.e. a round costs a little more when three follow each other
+// than the single-round figures above say).  A single width is kept where it is as good.
+struct Int8Tiles {
+  int width;                 // of the tiles: 128, 224 or 256
+  int split, tail_width;     // > 0: columns [split, N) as a second launch
+  double rounds256;          // price in rounds of 256-wide tiles
+};
+static Int8Tiles int8_tile_plan(int M, int N) {
+  const long cus = device_cu_count(), mtiles = (M + TM - 1) / TM;
+  auto rounds = [&](long cols, long w) { return (mtiles * ((cols + w - 1) / w) + cus - 1) / cus; };
+  const double c256 = 1.0, c224 = 0.978, c128 = 0.545;            // cost of one round, relative
+  const long t256 = mtiles * ((N + 255) / 256), t224 = mtiles * ((N + 223) / 224);
+  // a single row of tiles that leaves most CUs idle: tiles half as wide (the launch is bound by
+  // the weight stream, which then comes in over twice as many CUs)
+  const long t128 = mtiles * ((N + 127) / 128);
+  const long r224 = rounds(N, 224), r256 = rounds(N, 256);
+  if (mtiles == 1 && (t224 < r224 * 224 ? t224 : t256) * 3 <= cus * 2 && t128 > t224) return {128, 0, 0, rounds(N, 128) * c128};
+  Int8Tiles p = {256, 0, 0, r224 * c224 < r256 * c256 ? r224 * c224 : r256 * c256};
+  const long full = t256 / cus;                       // whole rounds of 256-wide tiles
+  if (full >= 1 && cus % mtiles == 0) {
+    const long ncols = full * (cus / mtiles) * 256;   // columns they cover
+    if (ncols < N) {
+      const long rest = N - ncols;
+      const double tails[3] = {rounds(rest, 128) * c128, rounds(rest, 224) * c224, rounds(rest, 256) * c256};
+      const int widths[3] = {128, 224, 256};
+      for (int i = 0; i < 3; ++i)
+        if (full * c256 + tails[i] < p.rounds256 - 0.05)   // (a second launch has to pay for itself)
+          p = {256, (int)ncols, widths[i], full * c256 + tails[i]};
+    }
+  }
+  if (!p.split && r224 * c224 < r256 * c256) p.width = 224;
+  return p;
+}
+
+// the price in rounds of 256 x 128 tiles
+double int8_tile_rounds(int M, int N) { return int8_tile_plan(M, N).rounds256 / 0.545; }
+
+namespace {
+
 template <int DT>
 int launch_gemm_splitk(const I8Args& a, int splits, void* workspace, hipStream_t st, bool wide = false) {
   I8Args b = a;
@@ -832,49 +883,17 @@ int launch_gemm_splitk(const I8Args& a, int splits, void* workspace, hipStream_t
   return 0;
 }
 
-// Tile width.  One workgroup per CU works through the output tiles in rounds; a last round that is
-// only part full idles the rest of the chip for a whole tile time.  Measured per round of 256 CUs on
-// K = 8192 (256 rows x TN columns per CU): TN = 256: 101 us, 224: 98.8 us, 128: 55 us -- the widest
-// tile is the cheapest per column.  So: as many FULL rounds of 256-wide tiles as the columns give, and
-// the remaining columns as a second launch with the width that wastes least (M 2048, N 28672: three
-// rounds of 256 and one of 128 instead of four of 224: 395 -> 387 us; under the profiler the two
-// launches last 315-337 us and 65-70 us, i.e. a round costs a little more when three follow each other
-// than the single-round figures above say).  A single width is kept where it is as good.
 template <int DT>
 int launch_gemm(const I8Args& a, hipStream_t st) {
-  const long cus = device_cu_count(), mtiles = (a.M + TM - 1) / TM;
-  auto rounds = [&](long cols, long w) { return (mtiles * ((cols + w - 1) / w) + cus - 1) / cus; };
-  const double c256 = 1.0, c224 = 0.978, c128 = 0.545;            // cost of one round, relative
-  const long t256 = mtiles * ((a.N + 255) / 256), t224 = mtiles * ((a.N + 223) / 224);
-  // a single row of tiles that leaves most CUs idle: tiles half as wide (the launch is bound by
-  // the weight stream, which then comes in over twice as many CUs)
-  const long t128 = mtiles * ((a.N + 127) / 128);
-  const long r224 = rounds(a.N, 224), r256 = rounds(a.N, 256);
-  if (mtiles == 1 && (t224 < r224 * 224 ? t224 : t256) * 3 <= cus * 2 && t128 > t224) return launch_tile<DT, 4, 2, 4, 4>(a, st);
-  double best = r224 * c224 < r256 * c256 ? r224 * c224 : r256 * c256;
-  int split = 0, tail_w = 0;
-  const long full = t256 / cus;                       // whole rounds of 256-wide tiles
-  if (full >= 1 && cus % mtiles == 0) {
-    const long ncols = full * (cus / mtiles) * 256;   // columns they cover
-    if (ncols < a.N) {
-      const long rest = a.N - ncols;
-      const double tails[3] = {rounds(rest, 128) * c128, rounds(rest, 224) * c224, rounds(rest, 256) * c256};
-      const int widths[3] = {128, 224, 256};
-      for (int i = 0; i < 3; ++i)
-        if (full * c256 + tails[i] < best - 0.05) {   // (a second launch has to pay for itself)
-          best = full * c256 + tails[i];
-          split = (int)ncols;
-          tail_w = widths[i];
-        }
-    }
+  const Int8Tiles p = int8_tile_plan(a.M, a.N);
+  if (p.split) {
+    if (int rc = launch_columns<DT, 2, 4, 4, 8>(a, 0, p.split, st)) return rc;
+    if (p.tail_width == 128) return launch_columns<DT, 4, 2, 4, 4>(a, p.split, a.N, st);
+    if (p.tail_width == 224) return launch_columns<DT, 4, 2, 7, 4>(a, p.split, a.N, st);
+    return launch_columns<DT, 2, 4, 4, 8>(a, p.split, a.N, st);
   }
-  if (split) {
-    if (int rc = launch_columns<DT, 2, 4, 4, 8>(a, 0, split, st)) return rc;
-    if (tail_w == 128) return launch_columns<DT, 4, 2, 4, 4>(a, split, a.N, st);
-    if (tail_w == 224) return launch_columns<DT, 4, 2, 7, 4>(a, split, a.N, st);
-    return launch_columns<DT, 2, 4, 4, 8>(a, split, a.N, st);
-  }
-  if (r224 * c224 < r256 * c256) return launch_tile<DT, 4, 2, 7, 4>(a, st);
+  if (p.width == 128) return launch_tile<DT, 4, 2, 4, 4>(a, st);
+  if (p.width == 224) return launch_tile<DT, 4, 2, 7, 4>(a, st);
   return launch_tile<DT, 2, 4, 4, 8>(a, st);
 }
 
@@ -957,6 +976,11 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
              "w8a8_int8_gemm: kslab weights need N=%d %% 64 == 0 and fewer than 4 Gi elements", N);
   MQ_REQUIRE(ldo >= N && ldo % 4 == 0, "w8a8_int8_gemm: output row stride %ld must be >= N and a multiple of 4", ldo);
   MQ_REQUIRE(out_dtype >= MI355Q_F16 && out_dtype <= MI355Q_F32, "w8a8_int8_gemm: bad out dtype %d", out_dtype);
+  size_t mid_bytes = 0;
+  if (kslab && !acc_out && (size_t)128 * (size_t)ldx < ((size_t)1 << 32) && q8_mid_wanted(2, M, N, K, &mid_bytes) &&
+      (mid_bytes == 0 || (workspace && workspace_bytes >= I8_WS_OFFSET + mid_bytes)))
+    return q8_mid_launch(2, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K, ldx,
+                         ldo, out_dtype, mid_bytes ? (char*)workspace + I8_WS_OFFSET : nullptr, as_stream(stream));
   I8Args a;
   a.out = out; a.acc_out = acc_out; a.x = x; a.w = w; a.x_scale = x_scale; a.w_scale = w_scale;
   a.bias = bias; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldw = ldw; a.ldo = ldo; a.ldacc = N;

@@ -346,7 +346,9 @@ def _scaled_int8_mm(out, x, weight, x_scale, w_scale, bias, acc_out=None):
             bias = bias.to(torch.float32)
             bias_f32 = 1
         bias = bias.contiguous()
-    stream_rows = rt.host.int8_stream_rows(K, N, _INT8_STREAM_MAX_M)
+    # kslab weights at some hundred rows: the kernel between the weight streamer and the 256-row tiles
+    mid = rt.host.q8_mid_plan(_lib.Q_INT8, M, N, K) if ldw == 0 and acc_out is None and _INT8_STREAM_MAX_M == 64 else -1
+    stream_rows = 0 if mid >= 0 else rt.host.int8_stream_rows(K, N, _INT8_STREAM_MAX_M)
     # (row-major [N, K] weights: the tile kernel with its K ranges is level with the streaming kernel on
     # large layers -- 8192 x 28672 at M = 16: 54 against 58 us -- and behind it on small ones up to 32
     # rows: 4096 x 4096 at M = 16: 13.8 against 7.7 us)
@@ -364,7 +366,7 @@ def _scaled_int8_mm(out, x, weight, x_scale, w_scale, bias, acc_out=None):
         return
     with torch.cuda.device(x.device):
         # (few output tiles behind a long K: K ranges side by side through the stream's workspace, bit-identical)
-        need = _lib.load().mi355q_w8a8_int8_workspace_bytes(M, N, K)
+        need = mid if mid >= 0 else _lib.load().mi355q_w8a8_int8_workspace_bytes(M, N, K)
         wsp = rt.workspace(x.device, need) if need else None
         _lib.call("mi355q_w8a8_int8_gemm_ws", out2.data_ptr(), rt.ptr(acc_out), x2.data_ptr(), w.data_ptr(),
                   rt.ptr(xs), xs_row, rt.ptr(ws), ws_col, rt.ptr(bias), bias_f32, M, N, K,
@@ -418,7 +420,8 @@ def _scaled_fp8_mm(out, x, weight, x_scale, w_scale, bias):
             raise RuntimeError(f"bias has {bias.numel()} entries for N={N}")
     with torch.cuda.device(x.device):
         # (few output tiles behind a long K: K ranges side by side through the stream's workspace)
-        need = _lib.load().mi355q_fp8_gemm_workspace_bytes(M, N, K)
+        mid = rt.host.q8_mid_plan(1, M, N, K) if ldw == 0 else -1
+        need = mid if mid >= 0 else _lib.load().mi355q_fp8_gemm_workspace_bytes(M, N, K)
         wsp = rt.workspace(x.device, need) if need else None
         _lib.call("mi355q_fp8_scaled_gemm_ws", out2.data_ptr(), x2.data_ptr(), w.data_ptr(), xs.data_ptr(),
                   int(xs.numel() > 1), ws.data_ptr(), int(ws.numel() > 1), rt.ptr(bias), M, N, K,
@@ -907,13 +910,16 @@ def _linear_quant_impl(out, lhs, rhs, bias, lhs_scale, rhs_scale):
     if lhs.dtype != torch.float8_e4m3fn or rhs.dtype != torch.float8_e4m3fn:
         raise RuntimeError("linear_quant: operands must be float8_e4m3fn")
     M, N, K = lhs.numel() // lhs.shape[-1], rhs.shape[0], lhs.shape[-1]
+    from .quantization import rearrange
     need = rt.host.fp8_tile_plan(M, N, K, _FP8_TILE_MIN_M, _FP8_TILE_MIN_TILES)
+    mid = rt.host.q8_mid_plan(0, M, N, K) if rearrange.is_kslab(rhs) else -1
+    if mid >= 0:
+        need = mid
     if need >= 0 \
             and out.dtype in (torch.float16, torch.bfloat16) \
             and rhs.dim() == 2 and rhs.is_contiguous() and out.is_contiguous():
         # prefill-sized M: the MFMA tile kernel (the weight-streaming kernel re-reads the weights per 64 rows)
         rt.require_gpu(out, lhs, rhs, bias, lhs_scale, rhs_scale)
-        from .quantization import rearrange
         a2 = lhs.reshape(M, K).contiguous()
         xs = lhs_scale.to(torch.float32).reshape(M, -1).contiguous()
         ws = rhs_scale.to(torch.float32).contiguous()
