@@ -1,0 +1,74 @@
+"""The W4A16 kernel for a few dozen to some hundred rows (csrc/w4a16_rows.hip): every tile it has at row counts around the
+tile's edges, odd and even numbers of K blocks (one range of a workgroup then holds one less, or none), K split over
+workgroups, column tiles that are and are not a multiple of eight, groups of 32 to K, every kind of zero-points, bias, and
+exact inputs bit for bit; then the choice the library makes by itself."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import w4 as ow4
+from vllm_gcu_amd.kernels import _custom_ops as ops
+from vllm_gcu_amd.kernels.quantization import rearrange
+
+pytestmark = pytest.mark.gpu
+TILES = [(2, 1), (3, 1), (4, 1), (2, 2), (3, 2), (4, 2), (5, 2), (6, 2)]     # rows / 16, columns / 64
+# (K, N, group, K ranges)
+SHAPES = [(128, 128, 128, 1), (384, 1024, 128, 1), (1280, 384, 256, 1), (2304, 640, 64, 2), (1152, 256, 32, 3), (1024, 512, 1024, 4)]
+
+
+def _case(seed, M, K, N, g, dtype, exact=False):
+    rng = np.random.default_rng(seed)
+    q = rng.integers(0, 16, size=(K, N), dtype=np.uint8)
+    z = rng.integers(0, 16, size=(K // g, N), dtype=np.uint8)
+    s = 2.0 ** -rng.integers(4, 8, size=(K // g, N)) if exact else rng.uniform(0.001, 0.01, size=(K // g, N))
+    x = rng.integers(-4, 5, size=(M, K)) if exact else rng.standard_normal((M, K))
+    return q, z, torch.from_numpy(s.astype(np.float32)).to(dtype), torch.from_numpy(x.astype(np.float32)).to(dtype)
+
+
+def _want(q, z, s, x, g, bias=None):
+    return ow4.w4a16_gemm(x.float().numpy(), q, z, s.float().numpy(), g, bias=None if bias is None else bias.float().numpy())
+
+
+def _run(q, z, s, x, g, bias=None, **kw):
+    w, zp = rearrange.rearrange_uint4_int32_gptq(torch.from_numpy(ow4.gptq_pack_weight(q)).cuda(),
+                                                 None if z is None else torch.from_numpy(ow4.gptq_pack_zeros(z)).cuda())
+    out = torch.full((x.shape[0], q.shape[1]), float("nan"), dtype=x.dtype, device="cuda")
+    return ops.w4a16_gemm(x.cuda(), w, s.cuda(), zp, None if bias is None else bias.cuda(), g, out=out, **kw).cpu()
+
+
+def _close(got, want):
+    np.testing.assert_allclose(got.float().numpy(), want, rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,N,g,splits", SHAPES)
+@pytest.mark.parametrize("mt,nt", TILES)
+def test_tiles(mt, nt, K, N, g, splits, dtype, monkeypatch):
+    kw = dict(family=4, split_k=splits | mt << 8 | nt << 16)
+    for M in (1, 16 * mt - 15, 16 * mt, 16 * mt + 1, 40 * mt):
+        print(f"case w4a16 rows {16 * mt}x{64 * nt} M={M} K={K} N={N} g={g} splits={splits} {dtype}", flush=True)
+        q, z, s, x = _case(M + K, M, K, N, g, dtype)
+        bias = torch.randn(N, generator=torch.Generator().manual_seed(M)).to(dtype)
+        _close(_run(q, z, s, x, g, bias, **kw), _want(q, z, s, x, g, bias))
+        _close(_run(q, None, s, x, g, **kw), _want(q, None, s, x, g))
+    # z * s in the activation type, as some checkpoints hold it: the kernel recovers the integer
+    monkeypatch.setattr(ops, "_RECOVER_INTEGER_ZEROS", False)
+    w, _ = rearrange.rearrange_uint4_int32_gptq(torch.from_numpy(ow4.gptq_pack_weight(q)).cuda(), None)
+    zs = (torch.from_numpy(z.astype(np.float32)) * s.float()).to(dtype)
+    _close(ops.w4a16_gemm(x.cuda(), w, s.cuda(), zs.cuda(), None, g, **kw).cpu(), _want(q, z, s, x, g))
+    q, z, s, x = _case(5, 16 * mt + 3, K, N, g, dtype, exact=True)
+    assert torch.equal(_run(q, z, s, x, g, **kw), torch.from_numpy(_want(q, z, s, x, g)).to(dtype))
+
+
+@pytest.mark.parametrize("M,K,N,g", [(5, 1024, 1024, 64), (20, 4096, 16384, 128), (24, 2048, 512, 32), (33, 1024, 128, 128),
+                                     (48, 4096, 1024, 128), (64, 2048, 4096, 128), (65, 3584, 512, 128), (96, 1024, 14336, 128),
+                                     (130, 2048, 1024, 64), (333, 1024, 2048, 128), (700, 1024, 1024, 128)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_automatic(M, K, N, g, dtype):
+    """What the library takes by itself equals this kernel's result (its sums are exact on these inputs, so they prove
+    that the numbers are right whatever it took)."""
+    print(f"case w4a16 rows automatic M={M} K={K} N={N} g={g} {dtype}", flush=True)
+    q, z, s, x = _case(M, M, K, N, g, dtype, exact=True)
+    want = torch.from_numpy(_want(q, z, s, x, g)).to(dtype)
+    assert torch.equal(_run(q, z, s, x, g), want)
+    assert torch.equal(_run(q, z, s, x, g, family=4), want)

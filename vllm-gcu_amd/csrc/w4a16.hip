@@ -2,6 +2,7 @@
 // streaming (small M) and the LDS-staged MFMA (large M) kernels.
 #include "common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace mi355q {
@@ -23,28 +24,31 @@ int w4a16_bf16_staged_launch(void* out, const void* x, const int32_t* qweight, c
 int w4a16_mid_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros,
                      int zeros_kind, const void* bias, int M, int K, int N, int group_size, int dtype,
                      void* workspace, size_t workspace_bytes, int splits, int tw, hipStream_t st);
+bool w4a16_rows_wanted(int M, int K, int N, int group_size, int zeros_kind, int dtype);
+size_t w4a16_rows_workspace_bytes(int M, int K, int N);
+int w4a16_rows_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
+                      const void* bias, int M, int K, int N, int group_size, int dtype, void* workspace, size_t workspace_bytes,
+                      int mt, int nt, int splits, hipStream_t st);
 }  // namespace mi355q
 
 using namespace mi355q;
 
 static constexpr size_t TILE_WS_OFFSET = (size_t)1 << 20;
 
-// streaming kernel up to 32 rows; 33..64 rows: the MFMA kernel where its pipelined loop exists
-// (fp16, integer zero-points; measured equal or up to 22 % faster there), else streaming again.
-// Groups of 64 and 32: the streaming kernel takes 32 rows per launch, so from 65 rows on the MFMA
-// kernel's plain loop with two or four groups per K block takes over.
-static int auto_family(int M, int group_size, int zeros_kind, int dtype) {
-  if (group_size % 128 != 0) return ((group_size == 64 || group_size == 32) && M > 64) ? 2 : 1;
-  const bool piped = dtype == MI355Q_F16 && zeros_kind != MI355Q_ZP_PRESCALED;
-  return (M <= 32 || (M <= 64 && !piped)) ? 1 : 2;
+// What is left when the kernel for a few dozen to some hundred rows does not take a problem (its rule stands with it): few
+// rows stream, many go to the MFMA kernels with larger tiles.  (Pre-scaled zero-points stream to 64 rows.)
+static int auto_family(int M, int K, int N, int group_size, int zeros_kind, int dtype) {
+  if (w4a16_rows_wanted(M, K, N, group_size, zeros_kind, dtype)) return 4;
+  if (group_size % 128 != 0 && group_size != 64 && group_size != 32) return 1;
+  return M <= 64 ? 1 : 2;
 }
 
 extern "C" size_t mi355q_w4a16_workspace_bytes(int M, int K, int N) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const size_t s = w4a16_stream_workspace_bytes(M > 64 ? 64 : M, N);
-  // the split-K partials of the MFMA kernel live behind the first MiB, which
+  // the split-K partials of the MFMA kernels live behind the first MiB, which
   // holds the streaming kernel's arrival counters (they must stay zero)
-  const size_t t = M > 32 ? w4a16_tile_workspace_bytes(M, K, N) : 0;
+  const size_t t = std::max<size_t>(M > 32 ? w4a16_tile_workspace_bytes(M, K, N) : 0, w4a16_rows_workspace_bytes(M, K, N));
   size_t tt = t ? t + TILE_WS_OFFSET : 0;
   // (this function does not see the dtype: room for the area that bf16 activations are staged in as
   // fp16 rows, behind the split-K partials -- a smaller workspace only means the bf16 loop runs instead)
@@ -94,9 +98,9 @@ extern "C" int mi355q_w4a16_gemm_ex(void* out, const void* x, const int32_t* qwe
   MQ_REQUIRE(zeros_kind >= MI355Q_ZP_NONE && zeros_kind <= MI355Q_ZP_PRESCALED,
              "w4a16_gemm: unknown zeros_kind %d", zeros_kind);
   MQ_REQUIRE(zeros_kind == MI355Q_ZP_NONE || zeros, "w4a16_gemm: zeros pointer missing");
-  MQ_REQUIRE(family >= 0 && family <= 3, "w4a16_gemm: unknown kernel family %d", family);
+  MQ_REQUIRE(family >= 0 && family <= 4, "w4a16_gemm: unknown kernel family %d", family);
   const int caller_family = family;       // 0: the library chooses, also between the two MFMA kernels
-  if (family == 0) family = auto_family(M, group_size, zeros_kind, dtype);
+  if (family == 0) family = auto_family(M, K, N, group_size, zeros_kind, dtype);
   MQ_REQUIRE(family != 2 || group_size % 128 == 0 || group_size == 64 || group_size == 32,
              "w4a16_gemm: the MFMA kernel needs a group size of 32, 64 or a multiple of 128, got %d", group_size);
   if (family == 1) {
@@ -115,6 +119,11 @@ extern "C" int mi355q_w4a16_gemm_ex(void* out, const void* x, const int32_t* qwe
     return 0;
   }
   const bool ws_ok = workspace && workspace_bytes > TILE_WS_OFFSET;
+  if (family == 2 && group_size % 128 != 0 && w4a16_rows_wanted(M, K, N, group_size, zeros_kind, dtype)) family = 4;
+  if (family == 4)
+    return w4a16_rows_launch(out, x, qweight, scales, zeros, zeros_kind, bias, M, K, N, group_size, dtype,
+                             ws_ok ? (char*)workspace + TILE_WS_OFFSET : nullptr, ws_ok ? workspace_bytes - TILE_WS_OFFSET : 0,
+                             (split_k >> 8) & 0xff, (split_k >> 16) & 0xff, split_k & 0xff, as_stream(stream));
   if (family == 3 && dtype == MI355Q_BF16) {
     // bf16 rows staged as fp16 in the workspace, ring workgroups of 256 (or, bits 8..15 = 4, 512) columns
     const int rc = w4a16_bf16_staged_launch(out, x, qweight, scales, zeros, zeros_kind, bias, M, K, N, group_size,
@@ -195,7 +204,7 @@ extern "C" int mi355q_w4a16_gemm_noalloc(void* out, const void* x, const int32_t
              gs, K);
   // what the plan of this shape needs, exactly -- the same plan mi355q_w4a16_gemm takes when its
   // workspace is large enough, so both entry points give bit-identical results
-  const int family = auto_family(M, gs, zeros_kind, dtype);
+  const int family = auto_family(M, K, N, gs, zeros_kind, dtype);
   size_t need;
   bool counters = false;
   if (family == 1) {
@@ -207,7 +216,13 @@ extern "C" int mi355q_w4a16_gemm_noalloc(void* out, const void* x, const int32_t
     }
     counters = need > 0;
   } else {
-    const size_t t = w4a16_tile_workspace_bytes(M, K, N);
+    // (which shapes are refused is part of the interface and goes by the 64-row tiles' K split, up to 128 rows by four ways of
+    // it at most, also where the kernel of family 4, whose partial sums always fit, takes the problem)
+    size_t t = w4a16_tile_workspace_bytes(M, K, N);
+    if (family == 4) {
+      if (M <= 128) t = std::min(t, (size_t)4 * M * N * sizeof(float));
+      t = M <= 32 ? w4a16_rows_workspace_bytes(M, K, N) : std::max(t, w4a16_rows_workspace_bytes(M, K, N));
+    }
     need = t ? t + TILE_WS_OFFSET : 0;
   }
   MQ_REQUIRE(need <= NOALLOC_SCRATCH_BYTES,

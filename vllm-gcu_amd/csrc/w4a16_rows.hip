@@ -1,0 +1,472 @@
+// W4A16 MFMA GEMM for a few dozen to some hundred rows.
+//
+// Between the decode kernel (up to 16 rows, 32 on some layers) and the prefill kernels the weights are still read about
+// once, so a launch is a stream of them with an LDS image of the activations beside it.  What bounds it: per K block of
+// 128 a CU moves 8 KiB of weights and 256 bytes per row into LDS, and its SIMDs issue nine vector instructions per packed
+// word to make operands of it; both take about as long (K 4096 x N 28672, 64 rows: 19.1 us for the copies alone, 19.5 for the
+// arithmetic alone).  Everything here is about running the two side by side:
+//   - wavefronts of their own copy (two per K range, one range per half of K): a copy instruction that waits for the
+//     address path holds up only its wavefront (the same loop with every wavefront copying its share: 27.2 us, with the copies
+//     spread between the matrix instructions 24.4, with copying wavefronts 23.5);
+//   - a wavefront that computes owns NT tiles of 16 columns x all rows of the workgroup, so no weight is dequantised twice
+//     in a workgroup, and A operands are read from LDS one K step ahead;
+//   - K is cut inside the workgroup (KS ranges, sums meet in LDS): as many wavefronts per SIMD as two workgroups
+//     give, without partial sums in memory;
+//   - tiles of 32..64 rows x 64 columns, two workgroups per CU, for layers of few columns, 32..96 x 128, one per CU,
+//     for wide ones.
+// Everything a stage needs travels from global memory straight into LDS by instructions issued from inline assembly
+// (the compiler, which does not see them, waits for the LDS reads alone); they are waited for by hand.
+//
+// B operands are the exact integers q - z in the activation type and the group scale multiplies the fp32 partial sum of
+// each group, as in the 64-row tile kernel: the only rounding is that of the fp32 additions, for fp16 and bf16 alike.
+//
+// Measured (us, fp16, groups of 128, weights cold; before -> here): 4096 x 4096 at 48 / 96 / 192 rows 12.0 / 15.5 / 23.1 ->
+// 9.1 / 9.4 / 12.2; 4096 x 6144 at 64 / 128 / 256 15.9 / 20.5 / 28.2 -> 9.5 / 13.2 / 18.6; 4096 x 28672 at 48 / 64 / 96
+// 29.9 / 32.7 / 41.7 -> 20.3 / 23.2 / 29.1; 14336 x 4096 at 48 / 96 / 192 20.3 / 27.5 / 39.0 -> 16.3 / 21.9 / 31.7.
+#include "common.h"
+
+#include <algorithm>
+#include <cmath>
+
+namespace mi355q {
+
+int w4a16_splitk_reduce_launch(void* out, const float* partial, const void* bias, int M, int N, int splits,
+                               int dtype, hipStream_t st);
+
+namespace {
+
+struct RowsArgs {
+  uint16_t* out;
+  const uint16_t* x;
+  const u4* qw;
+  const uint16_t* scales;
+  const char* zeros;          // packed int4, or z * s in the activation type
+  const uint16_t* bias;
+  int M, K, N;
+  int kper;                   // K blocks per range (blockIdx.y)
+  uint32_t gpk_magic;         // ceil(2^32 / K blocks per group), 0: a group is one K block or less
+  int mtiles, xcds;
+  float* partial;             // split K: f32 tiles [range][M][N]; null: write the output
+};
+
+__device__ __forceinline__ void rows_dma16(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr), "s"(more) : "memory", "scc");
+}
+template <int OFF>
+__device__ __forceinline__ void rows_dma16_next(uint32_t voff, const void* sbase) {   // the same m0; the offset counts on both sides
+  asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
+}
+
+struct RowsDq {
+  uint32_t magic, mlo, mhi;
+};
+template <int DT> struct RowsMma;
+template <> struct RowsMma<MI355Q_F16> {
+  static __device__ __forceinline__ f4 run(const u4& a, const u4& b, f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<h8>(a), bitcast<h8>(b), c, 0, 0, 0);
+  }
+  // one packed word -> 8 values q - z; zl = 1024 + z, zh = 64 + z
+  static __device__ __forceinline__ u4 dequant(uint32_t w, _Float16 zl, _Float16 zh, const RowsDq& k) {
+    const h2 zlo = {zl, zl}, zhi = {zh, zh}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
+    const uint32_t w8 = w >> 8;
+    const h2 r0 = bitcast<h2>((w & k.mlo) | k.magic) - zlo;                                          // 1024 + q
+    const h2 r1 = __builtin_elementwise_fma(bitcast<h2>((w & k.mhi) | k.magic), sixteenth, -zhi);    // 1024 + 16 q
+    const h2 r2 = bitcast<h2>((w8 & k.mlo) | k.magic) - zlo;
+    const h2 r3 = __builtin_elementwise_fma(bitcast<h2>((w8 & k.mhi) | k.magic), sixteenth, -zhi);
+    return (u4){bitcast<uint32_t>(r0), bitcast<uint32_t>(r1), bitcast<uint32_t>(r2), bitcast<uint32_t>(r3)};
+  }
+};
+template <> struct RowsMma<MI355Q_BF16> {
+  static __device__ __forceinline__ f4 run(const u4& a, const u4& b, f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<b8>(a), bitcast<b8>(b), c, 0, 0, 0);
+  }
+  // the same fp16 patterns through one mixed-precision multiply-add per weight (exact in fp32) and a packed conversion
+  static __device__ __forceinline__ uint32_t pair(h2 a, float m, _Float16 z) {
+    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+    const bf2 r = {(__bf16)__builtin_fmaf((float)a.x, m, -(float)z), (__bf16)__builtin_fmaf((float)a.y, m, -(float)z)};
+    return bitcast<uint32_t>(r);
+  }
+  static __device__ __forceinline__ u4 dequant(uint32_t w, _Float16 zl, _Float16 zh, const RowsDq& k) {
+    float one = 1.0f, sixteenth = 0.0625f;
+    asm volatile("" : "+s"(one));                     // (as a literal the multiplication folds away and the
+    asm volatile("" : "+s"(sixteenth));               //  conversion becomes an instruction of its own)
+    const uint32_t w8 = w >> 8;
+    return (u4){pair(bitcast<h2>((w & k.mlo) | k.magic), one, zl), pair(bitcast<h2>((w & k.mhi) | k.magic), sixteenth, zh),
+                pair(bitcast<h2>((w8 & k.mlo) | k.magic), one, zl), pair(bitcast<h2>((w8 & k.mhi) | k.magic), sixteenth, zh)};
+  }
+};
+
+// 16 MT rows x 64 NT columns; KS = 2 K ranges with NW wavefronts that compute and two that copy, and a ring of LDS stages,
+// each.  GPB: quantisation groups per K block (1 for group sizes that are multiples of 128, 2 / 4 for 64 / 32)
+template <int MT_, int NT_, int GPB_, int ZK>
+struct RowsCfg {
+  static constexpr int MT = MT_, NW = 4, NT = NT_, KS = 2, GPB = GPB_;
+  static constexpr int BM = 16 * MT, BN = 16 * NW * NT, CW = NW * KS, THREADS = 64 * (CW + 2 * KS);
+  static constexpr int A_BYTES = BM * 256, W_BYTES = 1024 * NW * NT, S_BYTES = 256 * GPB, Z_BYTES = (ZK == MI355Q_ZP_PRESCALED ? 256 : 64) * GPB;
+  static constexpr int W_OFF = A_BYTES, S_OFF = W_OFF + W_BYTES, Z_OFF = S_OFF + S_BYTES, STAGE = Z_OFF + Z_BYTES;
+  static constexpr int XC = A_BYTES / 2048, WC = NW * NT / 2, NC = XC + WC + 1;   // copies of a copying wavefront per stage
+  // two workgroups per CU where two stages fit so (deeper rings did not gain: the copies are bound by their rate)
+  static constexpr int PAIR = 2 * KS * STAGE <= 80 * 1024 ? 1 : 0, ROOM = (PAIR ? 80 : 159) * 1024 / (KS * STAGE);
+  static constexpr int D = ROOM < 4 ? ROOM : 4, RING = D * STAGE;
+  static_assert(XC * 2048 == A_BYTES && WC * 2 == NW * NT && WC <= 4 && D >= 2, "whole copies, a ring");
+  static_assert((D - 1) * NC < 64, "copies in flight that the wait can count");
+};
+
+template <int DT, int ZK, typename C>
+__global__ void __launch_bounds__(C::THREADS, (C::PAIR + 1) * C::THREADS / 256)
+w4a16_rows_kernel(RowsArgs a) {
+  typedef RowsMma<DT> MM;
+  constexpr int MT = C::MT, NW = C::NW, NT = C::NT, KS = C::KS, GPB = C::GPB, D = C::D, STAGE = C::STAGE;
+  // A operands one K step ahead where the registers are there (else the compiler places the reads, and spills nothing)
+  constexpr bool AHEAD = DT == MI355Q_F16 ? MT * NT <= 8 : MT * NT <= (C::PAIR ? 3 : 8);
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool copies = wg >= C::CW;
+  const int wave = copies ? (wg - C::CW) % 2 : wg % NW, ks = copies ? (wg - C::CW) / 2 : wg / NW;
+  const int c = lane & 15, kq = lane >> 4;
+  const int M = a.M, N = a.N, K = a.K, G = K >> 7;
+  int tm, tn;
+  if (a.xcds) {                                       // the row tiles of a column tile on one XCD: its weights pass one L2
+    const int j = blockIdx.x >> 3;
+    tm = j % a.mtiles;
+    tn = j / a.mtiles * 8 + (blockIdx.x & 7);
+  } else {
+    tm = blockIdx.x % a.mtiles;
+    tn = blockIdx.x / a.mtiles;
+  }
+  const int m0 = tm * C::BM;
+  const int slab = tn * NW * NT >> 3, t0 = tn * NW * NT & 7;           // 128-column slab, first of the workgroup's 16-column tiles in it
+  const int g0 = (int)blockIdx.y * a.kper, ng = min(G - g0, a.kper);   // K blocks of the workgroup
+  const int nk = (ng + KS - 1) / KS;                  // ... of each of its ranges (the last may hold fewer, even none)
+  const int mine = min(ng - ks * nk, nk);
+
+  f4 acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[mt][t] = (f4){0.f, 0.f, 0.f, 0.f};
+
+  if (copies) {
+    // x: 4 rows of 256 bytes per copy; lane = 16 * row + position, position p of row r receives chunk p ^ (r & 15)
+    uint32_t xo[C::XC];
+#pragma unroll
+    for (int p = 0; p < C::XC; ++p) {
+      const int r = 4 * (wave + 2 * p) + (lane >> 4);
+      xo[p] = ((uint32_t)min(m0 + r, M - 1) * (uint32_t)K + 8u * (uint32_t)((lane & 15) ^ (r & 15))) * 2u;
+    }
+    const uint32_t lane16 = (uint32_t)lane * 16u;
+    int kb = min(g0 + ks * nk, G - 1);                // the K block that the next copies are of
+    const int klast = max(g0 + ks * nk + mine - 1, kb);
+    const char* xg = (const char*)a.x + (size_t)kb * 256;
+    const char* qg = (const char*)a.qw + ((size_t)slab * G + kb) * 8192 + (t0 + wave * C::WC) * 1024;
+    // the first wavefront of the range copies the scales, the second the zero-points (without any, the scales again: both
+    // have the same number of copies to wait for)
+    const bool packed = ZK == MI355Q_ZP_PACKED && wave == 1, zwave = ZK != MI355Q_ZP_NONE && wave == 1;
+    const uint32_t szrow = packed ? (uint32_t)N / 2 : (uint32_t)N * 2;
+    const uint32_t szoff = packed ? (uint32_t)(lane & 3) * 16u + (uint32_t)(lane >> 2) * szrow
+                                  : (uint32_t)(lane & 15) * 16u + (uint32_t)(lane >> 4) * szrow;
+    const int szlanes = packed ? 4 * GPB : 16 * GPB;
+    const char* const szg = zwave ? a.zeros + (packed ? 64 : 256) * slab : (const char*)a.scales + 256 * slab;
+    const uint32_t szlds = zwave ? C::Z_OFF : C::S_OFF;
+    const uint32_t ring = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)lds) + ks * C::RING;
+    auto copy_stage = [&](int slot) {
+      const uint32_t sb = ring + (uint32_t)(slot * STAGE);
+#pragma unroll
+      for (int p = 0; p < C::XC; ++p) rows_dma16(xo[p], xg, sb, (uint32_t)((wave + 2 * p) * 1024));
+      rows_dma16(lane16, qg, sb, (uint32_t)(C::W_OFF + wave * C::WC * 1024));
+      if constexpr (C::WC > 1) rows_dma16_next<1024>(lane16, qg);
+      if constexpr (C::WC > 2) rows_dma16_next<2048>(lane16, qg);
+      if constexpr (C::WC > 3) rows_dma16_next<3072>(lane16, qg);
+      const uint32_t row = GPB > 1 ? (uint32_t)kb * GPB : a.gpk_magic ? (uint32_t)(((uint64_t)kb * a.gpk_magic) >> 32) : (uint32_t)kb;
+      if (lane < szlanes) rows_dma16(szoff, szg + (size_t)row * szrow, sb, szlds);
+      if (kb < klast) {                               // (past the end: a re-read into a stage nobody reads)
+        ++kb;
+        xg += 256;
+        qg += 8192;
+      }
+    };
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) copy_stage(d);
+    int slot = 0;
+    for (int i = 0; i < nk; ++i) {
+      asm volatile("s_waitcnt vmcnt(%0)" : : "n"((D - 2) * C::NC) : "memory");   // the copies of K block i have landed
+      __builtin_amdgcn_s_barrier();                   // ... everybody's, and nobody reads K block i - 1 any more
+      copy_stage(slot == 0 ? D - 1 : slot - 1);
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");   // no copy may still be writing LDS
+  } else {
+    uint32_t a_pos[4];
+#pragma unroll
+    for (int st = 0; st < 4; ++st) a_pos[st] = (uint32_t)(c * 256 + ((4 * st + kq) ^ c) * 16);
+    RowsDq dq = {0x64006400u, 0x000f000fu, 0x00f000f0u};
+    asm volatile("" : "+v"(dq.magic));
+    asm volatile("" : "+s"(dq.mlo));
+    asm volatile("" : "+s"(dq.mhi));
+    int slot = 0;
+    for (int i = 0; i < nk; ++i) {
+      asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");   // no LDS read of the stage before is open
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" : : : "memory");
+      if (i < mine) {
+        const unsigned char* st = lds + ks * C::RING + slot * STAGE;
+        u4 w[NT], av[2][MT];
+        float sc[NT][GPB];
+        _Float16 zlo[NT][GPB], zhi[NT][GPB];
+        uint32_t zw[GPB];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) w[t] = *(const u4*)(st + C::W_OFF + (wave * NT + t) * 1024 + lane * 16);
+#pragma unroll
+        for (int g = 0; g < GPB; ++g) zw[g] = ZK == MI355Q_ZP_PACKED ? *(const uint32_t*)(st + C::Z_OFF + 64 * g + c * 4) : 0x88888888u;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) av[0][mt] = *(const u4*)(st + a_pos[0] + mt * 4096);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const int tile = t0 + wave * NT + t;
+#pragma unroll
+          for (int g = 0; g < GPB; ++g) {
+            sc[t][g] = Elem<DT>::to_f32(*(const uint16_t*)(st + C::S_OFF + 256 * g + (8 * c + tile) * 2));
+            if constexpr (ZK == MI355Q_ZP_PRESCALED) {   // z * s rounded to the activation type -> the integer z
+              const float zf = __builtin_rintf(Elem<DT>::to_f32(*(const uint16_t*)(st + C::Z_OFF + 256 * g + (8 * c + tile) * 2)) / sc[t][g]);
+              zlo[t][g] = (_Float16)(1024.0f + zf);
+              zhi[t][g] = (_Float16)(64.0f + zf);
+            } else {                                     // fp16 bit patterns directly
+              const uint32_t z = (zw[g] >> (4 * tile)) & 15u;
+              zlo[t][g] = bitcast<_Float16>((uint16_t)(0x6400u | z));
+              zhi[t][g] = bitcast<_Float16>((uint16_t)(0x5400u | (z << 4)));
+            }
+          }
+        }
+        f4 part[MT][NT];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int g = s * GPB / 4;
+          if (!AHEAD && s > 0) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) av[s & 1][mt] = *(const u4*)(st + a_pos[s] + mt * 4096);
+          }
+          if (AHEAD && s < 3) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) av[(s + 1) & 1][mt] = *(const u4*)(st + a_pos[s + 1] + mt * 4096);
+          }
+          u4 b[NT];
+#pragma unroll
+          for (int t = 0; t < NT; ++t) b[t] = MM::dequant(w[t][s], zlo[t][g], zhi[t][g], dq);
+          if constexpr (AHEAD) asm volatile("" : : : "memory");   // (keeps the reads of the next K step above this one's matrix instructions)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              part[mt][t] = MM::run(av[s & 1][mt], b[t], s % (4 / GPB) == 0 ? (f4){0.f, 0.f, 0.f, 0.f} : part[mt][t]);
+          if ((s + 1) % (4 / GPB) == 0) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+              for (int t = 0; t < NT; ++t) acc[mt][t] += sc[t][g] * part[mt][t];
+          }
+        }
+      }
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+  }
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
+
+  // through LDS: a lane holds one column of 4 rows per row tile (columns 8 apart in memory), a wavefront's store should
+  // hold neighbours.  Tile column j = TC * c + tile is column 8 * (j / TC) + t0 + j % TC of the slab.
+  constexpr int EP = C::BN * 4 + 16, TC = NW * NT, Q = TC / 4;         // bytes per tile row; quads of columns per c
+  static_assert(C::BM * EP <= C::RING, "the output tile fits in the ring");
+  if (!copies) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *(float*)(lds + ks * C::RING + (mt * 16 + 4 * kq + i) * EP + (TC * c + wave * NT + t) * 4) = acc[mt][t][i];
+  }
+  __syncthreads();
+  constexpr int TPR = C::BN / 4;                      // threads per row
+  const int q = tid % TPR, n = 128 * slab + 8 * (q / Q) + t0 + 4 * (q % Q);
+  float bs[4] = {0.f, 0.f, 0.f, 0.f};
+  if (a.bias && !a.partial) {
+    const uint2 bw = *(const uint2*)(a.bias + n);
+    bs[0] = Elem<DT>::to_f32((uint16_t)(bw.x & 0xffffu)); bs[1] = Elem<DT>::to_f32((uint16_t)(bw.x >> 16));
+    bs[2] = Elem<DT>::to_f32((uint16_t)(bw.y & 0xffffu)); bs[3] = Elem<DT>::to_f32((uint16_t)(bw.y >> 16));
+  }
+  for (int r = tid / TPR; r < C::BM; r += C::THREADS / TPR) {
+    const int m = m0 + r;
+    if (m >= M) break;
+    f4 v = *(const f4*)(lds + r * EP + q * 16);
+#pragma unroll
+    for (int k = 1; k < KS; ++k) v += *(const f4*)(lds + k * C::RING + r * EP + q * 16);
+    if (a.partial) {
+      *(f4*)(a.partial + ((size_t)blockIdx.y * M + m) * N + n) = v;
+    } else {
+      uint2 o;
+      o.x = (uint32_t)Elem<DT>::from_f32(v[0] + bs[0]) | ((uint32_t)Elem<DT>::from_f32(v[1] + bs[1]) << 16);
+      o.y = (uint32_t)Elem<DT>::from_f32(v[2] + bs[2]) | ((uint32_t)Elem<DT>::from_f32(v[3] + bs[3]) << 16);
+      *(uint2*)(a.out + (size_t)m * N + n) = o;
+    }
+  }
+}
+
+template <int DT, int ZK, typename C>
+int launch_rows(RowsArgs a, int splits, const void* bias, int dtype, hipStream_t st) {
+  const int G = a.K / 128;
+  a.mtiles = (a.M + C::BM - 1) / C::BM;
+  a.xcds = (a.N / C::BN) % 8 == 0;
+  a.kper = (G + splits - 1) / splits;
+  splits = (G + a.kper - 1) / a.kper;                 // no empty ranges
+  if (splits <= 1) a.partial = nullptr;
+  const size_t shmem = (size_t)C::KS * C::RING;
+  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_rows_kernel<DT, ZK, C>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+  MQ_REQUIRE(attr == hipSuccess, "w4a16_gemm(rows): cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
+  hipLaunchKernelGGL((w4a16_rows_kernel<DT, ZK, C>), dim3((unsigned)(a.mtiles * (a.N / C::BN)), (unsigned)splits), dim3(C::THREADS), shmem, st, a);
+  MQ_LAUNCH_CHECK("w4a16_gemm(rows)");
+  if (splits > 1) return w4a16_splitk_reduce_launch(a.out, a.partial, bias, a.M, a.N, splits, dtype, st);
+  return 0;
+}
+
+template <int DT, int ZK, int GPB>
+int launch_rows_cfg(const RowsArgs& a, int mt, int nt, int splits, const void* bias, int dtype, hipStream_t st) {
+#define MQ_CFG(MT, NT) if (mt == MT && nt == NT) return launch_rows<DT, ZK, RowsCfg<MT, NT, GPB, ZK>>(a, splits, bias, dtype, st)
+  MQ_CFG(2, 1); MQ_CFG(3, 1); MQ_CFG(4, 1);
+  MQ_CFG(2, 2); MQ_CFG(3, 2); MQ_CFG(4, 2); MQ_CFG(5, 2); MQ_CFG(6, 2);
+#undef MQ_CFG
+  MQ_REQUIRE(false, "w4a16_gemm(rows): no tile of %d x %d", 16 * mt, 64 * nt);
+}
+
+// ---- the choice of tile and K split: the cheapest by a price model in microseconds.  Per tile: a K block of each of its two
+// ranges, for a workgroup alone on its CU and added for a second one beside it (tiles of 64 columns and 32 x 128 fit two).
+// Fitted to 3400 measurements (15 layer shapes, 20..2048 rows, 1..12 ranges, weights cold in the caches; rms error 5 %); the tile
+// taken by it is within 2 % of the best one on average over those points.
+struct RowsPrice {
+  int mt, nt;
+  double one, more;
+};
+constexpr RowsPrice kRows[] = {{2, 1, 0.419, 0.398}, {3, 1, 0.589, 0.480}, {4, 1, 0.716, 0}, {2, 2, 0.789, 0.578},
+                               {3, 2, 0.961, 0},     {4, 2, 1.147, 0},     {5, 2, 1.307, 0}, {6, 2, 1.520, 0}};
+constexpr double kRowsBase = 3.77, kRowsRound = 1.37, kRowsSplit = 2.36, kRowsSplitMN = 1.41;
+constexpr double kRowsAlone = 0.283;        // share of a step that goes away as the chip empties (the caches and memory are shared)
+constexpr double kRowsSecond = 0.345;       // share of the second workgroup's price that grows with how many CUs hold two
+constexpr double kRowsStream = 4.12e6;      // bytes of weights per microsecond
+
+struct RowsPlan {
+  int mt, nt, splits;
+  size_t bytes;                             // partial sums
+  double price;
+};
+
+RowsPlan rows_make_plan(int M, int K, int N, bool split) {
+  RowsPlan best = {0, 0, 1, 0, 1e30};
+  const int KB = K / 128;
+  const long cus = device_cu_count();
+  const double stream = std::pow((double)K * N / 2 / kRowsStream, 4);
+  for (const RowsPrice& p : kRows) {
+    const int bm = 16 * p.mt, bn = 64 * p.nt;
+    if (p.mt > 2 && M <= bm - 16) continue;
+    const long tiles = (long)((M + bm - 1) / bm) * (N / bn), res = p.more > 0 ? 2 : 1;
+    for (int s = 1; s <= (split ? 12 : 1); ++s) {
+      const int kper = (KB + s - 1) / s;
+      if (s > 1 && ((KB + kper - 1) / kper != s || kper < 8)) continue;
+      const size_t bytes = s > 1 ? (size_t)s * M * N * 4 : 0;
+      if (bytes > ((size_t)31 << 20)) continue;       // (fits the fixed scratch of callers that cannot allocate, too)
+      const long full = tiles * s / (res * cus), rest = tiles * s % (res * cus);
+      double steps = full * (p.one + p.more * (res - 1));
+      if (rest) steps += p.one * (1 - kRowsAlone * (1 - (double)std::min(rest, cus) / cus));
+      if (rest > cus) steps += p.more * ((double)(rest - cus) / cus * kRowsSecond + 1 - kRowsSecond);
+      double t = std::sqrt(std::sqrt(std::pow(steps * ((kper + 1) / 2), 4) + stream)) + kRowsBase + kRowsRound * (full + (rest > 0) - 1);
+      if (s > 1) t += kRowsSplit + kRowsSplitMN * 1e-6 * s * M * N;
+      if (t < best.price) best = {p.mt, p.nt, s, bytes, t};
+    }
+  }
+  return best;
+}
+
+// (a serving loop asks for the same few shapes again and again, from the host path and from the entry points)
+RowsPlan rows_plan(int M, int K, int N) {
+  struct Entry {
+    int M, N, K, cus;
+    RowsPlan plan;
+  };
+  static thread_local Entry table[64] = {};
+  const uint32_t h = ((uint32_t)M * 2654435761u ^ (uint32_t)N * 40503u ^ (uint32_t)K * 2246822519u) >> 7;
+  Entry& e = table[h % 64];
+  const int cus = device_cu_count();
+  if (e.M != M || e.N != N || e.K != K || e.cus != cus) e = {M, N, K, cus, rows_make_plan(M, K, N, true)};
+  return e.plan;
+}
+
+}  // namespace
+
+double w4a16_wide_price(int M, int K, int N, bool ring);     // us of the 64-row tiles and (ring) the ring kernels
+
+// Whether this kernel is the one to take.
+//  - Up to 16 rows: the streaming kernel, except for groups of 64 and 32 on small layers, where four scale rows per K block
+//    keep it from its rate (4096 x 4096, groups of 64, 1 / 16 rows: 9.1 / 10.2 -> 7.8 / 8.3 us, 2048 x 2048 8.3 / 8.7 -> 6.5 / 6.7;
+//    4096 x 28672, bf16: 16.2 against 19.8).
+//  - 17..32 rows: there the streaming kernel takes two row tiles and stays ahead on groups of 128 while the layer is small
+//    (4096 x 6144, 20 / 28 rows: 8.9 / 9.3 against 9.6 / 9.9 us; 14336 x 4096 14.3 against 14.5; but 4096 x 28672 21.3 -> 18.8, 18944 x
+//    3584 16.8 -> 15.0, 8192 x 8192 15.2 -> 14.7; bf16, whose operands cost more here, from 100 million weights on).
+//  - Pre-scaled zero-points up to 64 rows: the streaming kernel, which uses z * s as it is.
+//  - To 128 rows: always.  Above: where its price is below that of the kernels with larger tiles, which read and dequantise the
+//    weights fewer times (their model prices them 5 % low against this one's).
+bool w4a16_rows_wanted(int M, int K, int N, int group_size, int zeros_kind, int dtype) {
+  const bool small = group_size % 128 != 0;
+  const long w = (long)K * N;
+  if (small && group_size != 64 && group_size != 32) return false;
+  if (M > 4096 || (size_t)M * K * 2 >= ((size_t)1 << 32)) return false;
+  if (zeros_kind == MI355Q_ZP_PRESCALED && M <= 64) return false;
+  if (M <= 16) return small && w <= (1L << 25);
+  if (M <= 32) return small || w >= (dtype == MI355Q_F16 ? 1L << 26 : 3L << 25);
+  if (M <= 128) return true;
+  return rows_plan(M, K, N).price < 0.95 * w4a16_wide_price(M, K, N, !small);
+}
+
+size_t w4a16_rows_workspace_bytes(int M, int K, int N) { return M <= 4096 ? rows_plan(M, K, N).bytes : 0; }
+
+// mt 0: the plan, unsplit where the workspace does not hold the partial sums; else 16 mt rows x 64 nt columns, K in `splits` ranges
+int w4a16_rows_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
+                      const void* bias, int M, int K, int N, int group_size, int dtype, void* workspace, size_t workspace_bytes,
+                      int mt, int nt, int splits, hipStream_t st) {
+  if (!mt) {
+    RowsPlan p = rows_plan(M, K, N);
+    if (p.bytes > (workspace ? workspace_bytes : 0)) p = rows_make_plan(M, K, N, false);
+    mt = p.mt;
+    nt = p.nt;
+    splits = p.splits;
+  }
+  splits = std::max(1, std::min(splits, K / 128));
+  if (splits > 1 && (!workspace || workspace_bytes < (size_t)splits * M * N * 4)) splits = 1;
+  MQ_REQUIRE((size_t)M * K * 2 < ((size_t)1 << 32), "w4a16_gemm: activation matrix %d x %d is 4 GiB or more", M, K);
+  MQ_REQUIRE(group_size % 128 == 0 || group_size == 64 || group_size == 32, "w4a16_gemm(rows): group size %d", group_size);
+  RowsArgs a = {};
+  a.out = (uint16_t*)out; a.x = (const uint16_t*)x; a.qw = (const u4*)qweight; a.scales = (const uint16_t*)scales;
+  a.zeros = (const char*)zeros; a.bias = (const uint16_t*)bias;
+  a.M = M; a.K = K; a.N = N;
+  const uint32_t gpk = group_size >= 128 ? (uint32_t)group_size / 128u : 1u;
+  a.gpk_magic = gpk > 1 ? (uint32_t)((((uint64_t)1 << 32) + gpk - 1) / gpk) : 0u;
+  a.partial = (float*)workspace;
+#define MQ_GPB(DT, ZK, GPB) return launch_rows_cfg<DT, ZK, GPB>(a, mt, nt, splits, bias, dtype, st)
+#define MQ_ZK(DT, ZK)                       \
+  do {                                      \
+    if (group_size == 64) MQ_GPB(DT, ZK, 2); \
+    if (group_size == 32) MQ_GPB(DT, ZK, 4); \
+    MQ_GPB(DT, ZK, 1);                      \
+  } while (0)
+#define MQ_DT(DT)                                                          \
+  do {                                                                     \
+    if (zeros_kind == MI355Q_ZP_PACKED) MQ_ZK(DT, MI355Q_ZP_PACKED);       \
+    if (zeros_kind == MI355Q_ZP_PRESCALED) MQ_ZK(DT, MI355Q_ZP_PRESCALED); \
+    MQ_ZK(DT, MI355Q_ZP_NONE);                                             \
+  } while (0)
+  if (dtype == MI355Q_F16) MQ_DT(MI355Q_F16);
+  MQ_DT(MI355Q_BF16);
+#undef MQ_DT
+#undef MQ_ZK
+#undef MQ_GPB
+}
+
+}  // namespace mi355q
