@@ -1,33 +1,32 @@
-// fp8-e4m3 block-scaled GEMM for more than 64 rows on the 128-deep fp8 MFMA of gfx950
-// (v_mfma_f32_16x16x128_f8f6f4, twice the rate of the 32-deep one), with the 128 x 128 block
-// scales applied to the fp32 partial sum of every K block.
+// fp8-e4m3 GEMMs for many rows on the 128-deep fp8 MFMA of gfx950 (v_mfma_f32_16x16x128_f8f6f4, twice the rate of the
+// 32-deep one): per-token x per-channel scales, 128 x 128 block scales, and 16-bit operands on the same tiles.
 //
-//   out[m, n] = sum_kb x_scale[m, kb] * w_scale[n / 128, kb] * sum_{k in block kb} x[m, k] * w[n, k]
+// Same machinery as the int8 GEMM next door: a workgroup owns a 256 x 128 output tile; K advances in LDS tiles of
+// 128 bytes per row, which is exactly one scale block and one MFMA deep; tiles go from global memory straight
+// into LDS (16 B per lane, no staging registers; 16-byte-chunk XOR swizzle, or chunk-major for kslab weights) in
+// three stages.
 //
-// Same machinery as the int8 GEMM next door: a workgroup of eight wavefronts
-// (4 x 2, each 64 rows of x by 64 rows of w) owns a 256 x 128 output tile; K
-// advances in LDS tiles of 128 bytes per row, which is exactly one scale block
-// and one MFMA deep; tiles go from global memory straight into LDS (16 B per
-// lane, no staging registers; 16-byte-chunk XOR swizzle, or chunk-major for
-// kslab weights) in three stages; operand reads are hand-written and
-// hand-waited for.  A K block's MFMA starts from zero and its result joins the
-// running sum multiplied by the block's scale.  128 columns are exactly one
-// scale block, so the weight scale of a tile and K block is a single number;
-// it and the activation scales of the K block (one per row) travel with the
-// tiles through LDS (4-byte direct-to-LDS copies).  Two wavefronts per SIMD
-// leave each 256 registers: 64 running sums, two sets of x operands, one set
-// of w operands that is re-read tile by tile behind the MFMAs (see `step`).
+// Per-token x per-channel scales (cutlass_scaled_mm on fp8 operands; fp8_pc_gemm_kernel): eight wavefronts (4 x 2,
+// each 64 rows of x by 64 rows of w) multiply and copy; operand reads are hand-written and hand-waited for.  Two
+// wavefronts per SIMD leave each 256 registers: 64 running sums, two sets of x operands, one set of w operands that is
+// re-read tile by tile behind the MFMAs (see `step`).  Every MFMA accumulates straight into the running sum, and the
+// epilogue multiplies by x_scale[m] (or one value) and w_scale[n] (or one value).  What bounds it is the clock that the
+// power limit leaves (a K block 0.75 us with random operands, 0.53 with zeros).
 //
-// PC variant (per-token x per-channel scales, cutlass_scaled_mm on fp8 operands): the scales live
-// outside the K sum, so every MFMA accumulates straight into the running sum, no scales travel
-// through LDS, and the epilogue multiplies by x_scale[m] (or one value) and w_scale[n] (or one value).
-//
-// OP16 variant (unquantised fp16 / bf16 experts at prefill token counts, grouped launches only): the
+// 16-bit operands (OP16: unquantised fp16 / bf16 experts at prefill token counts, grouped launches only): the
 // same tiles of 128 bytes per row hold 64 elements of 16 bits; a lane's two 16-byte chunks are the
 // operands of two 32-deep 16-bit MFMAs (chunk kq: elements 8 kq .. 8 kq + 7 of the first 32, chunk
 // 4 + kq: of the second 32), which take as long as the one 128-deep fp8 MFMA.  No scales anywhere.
 // The host passes K and the row strides in bytes.
+//
+// Block scales (fp8_block_gemm_kernel):
+//   out[m, n] = sum_kb x_scale[m, kb] * w_scale[n / 128, kb] * sum_{k in block kb} x[m, k] * w[n, k]
+// A K block's MFMA starts from zero and its result joins the running sum multiplied by the block's scale.  128 columns
+// are exactly one scale block, so the weight scale of a tile and K block is a single number; it and the
+// activation scales of the K block (one per row) travel with the tiles through LDS (4-byte direct-to-LDS copies).
 #include "common.h"
+
+#include <algorithm>
 
 namespace mi355q {
 int kcontig_fp8_pc_launch(void* out, const void* a, const void* w, const float* a_scale, int scale_per_row,
@@ -64,8 +63,8 @@ struct F8Args {
   const int32_t* npp;          // device scalar: padded id count
   const float* topk_weights;   // [numel] or null
   int numel, topk, E, max_blocks;
-  int block_rows;              // slot ids per align block: 256, or 128 (the upper half of every row tile is empty:
-                               // its wavefronts only copy, as in a dense launch of up to 128 rows)
+  int block_rows;              // slot ids per align block: 256, or 128 (16-bit operands: the upper half of every row
+                               // tile is empty, its wavefronts only copy, as in a dense launch of up to 128 rows)
   long w_stride, ws_stride;    // per expert: bytes of weights, floats of weight scales
 };
 
@@ -73,28 +72,55 @@ __device__ __forceinline__ void dma16(const void* gptr, void* lds_wave_base) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gptr,
                                    (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
 }
-// 64 x 4 B: lane l lands at base + 4 l
-__device__ __forceinline__ void dma4(const void* gptr, void* lds_wave_base) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gptr,
-                                   (__attribute__((address_space(3))) void*)lds_wave_base, 4, 0, 0);
-}
-
 typedef int i8v __attribute__((ext_vector_type(8)));
+
+// origin of an output tile of BM x 128 (split K: of an output tile and K range)
+template <bool GROUPED, int BM>
+__device__ __forceinline__ void f8_tile_origin(const F8Args& a, int mtiles, int ntiles_n, int ksplits, int tile, int& m0, int& n0) {
+  int tm, tn;
+  if (GROUPED) {
+    // block-major: neighbouring workgroups share a block's activation rows
+    tm = tile / ntiles_n;
+    tn = tile - tm * ntiles_n;
+  } else if (ksplits > 1) {
+    const int t = tile / ksplits;
+    tm = t % mtiles;
+    tn = t / mtiles;
+  } else if (a.n_panels_swizzle) {
+    // XCD x takes the weight panels tn = x, x + 8, ...; it sweeps them for a chunk of 8 row tiles
+    // (2048 rows of x: what its L2 can keep warm next to a panel) before the next chunk
+    const int x = tile & 7, j = tile >> 3;
+    const int P = ntiles_n >> 3, full = (mtiles >> 3) << 3;           // panels per XCD, row tiles in whole chunks
+    int tj;
+    if (j < full * P) {
+      const int c = j / (8 * P), r = j - c * 8 * P;
+      tj = r >> 3;
+      tm = c * 8 + (r & 7);
+    } else {
+      const int rem = mtiles - full, r = j - full * P;
+      tj = r / rem;
+      tm = full + r % rem;
+    }
+    tn = tj * 8 + x;
+  } else {
+    tm = tile % mtiles;
+    tn = tile / mtiles;
+  }
+  m0 = tm * BM;
+  n0 = tn * FTN;
+}
 
 // GROUPED: the fused-MoE grouped GEMM at prefill token counts.  Row tile b is align block b (256 slot
 // ids of expert expert_ids[b]): x rows and their scales are gathered through the ids (row id / topk),
 // weights and weight scales are the expert's, output row id gets the result (times its routing weight).
 // Blocks past num_tokens_post_pad do not exist (the tile count is read on the device); a block of an
 // expert outside [0, E) writes zeros.  No K ranges, no bias.
-template <int DT, bool PC, bool GROUPED = false, bool OP16 = false>
+template <int DT, bool OP16>
 __global__ void __launch_bounds__(F8_THREADS, 1)
-fp8_block_gemm_kernel(F8Args a) {
-  static_assert(!GROUPED || !PC || OP16, "the grouped form exists for block scales and for 16-bit operands");
-  static_assert(!OP16 || (PC && GROUPED), "16-bit operands: grouped launches, no scales");
+fp8_pc_gemm_kernel(F8Args a) {
+  constexpr bool GROUPED = OP16;                        // (16-bit operands: grouped launches only)
   constexpr int WN = 2, NI = 4, NJ = 4;                 // 4 x 2 wavefronts of 64 x 64
-  constexpr int X_BYTES = FTM * FTKB, W_BYTES = FTN * FTKB, XS_BYTES = FTM * 4;
-  constexpr int WS_BYTES = 256;                         // the tile's weight scale of a K block, 64 copies
-  constexpr int STAGE_BYTES = X_BYTES + W_BYTES + XS_BYTES + WS_BYTES;
+  constexpr int X_BYTES = FTM * FTKB, W_BYTES = FTN * FTKB, STAGE_BYTES = X_BYTES + W_BYTES;
   constexpr int XCOPIES = FTM / 8 / 8, WCOPIES = FTN / 8 / 8;       // 1 KiB copies per wavefront
   extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -111,55 +137,19 @@ fp8_block_gemm_kernel(F8Args a) {
   const int ksplits = (!GROUPED && a.ksplits > 1) ? a.ksplits : 1;
   const int total_tiles = mtiles * ntiles_n * ksplits;   // (split K: tile ids count (output tile, K range) pairs)
   if (GROUPED && (int)blockIdx.x >= total_tiles) return;  // (the grid is sized for the largest block count the ids can fill)
-  auto tile_origin = [&](int tile, int& m0, int& n0) {
-    int tm, tn;
-    if (GROUPED) {
-      // block-major: neighbouring workgroups share a block's activation rows
-      tm = tile / ntiles_n;
-      tn = tile - tm * ntiles_n;
-    } else if (ksplits > 1) {
-      const int t = tile / ksplits;
-      tm = t % mtiles;
-      tn = t / mtiles;
-    } else if (a.n_panels_swizzle) {
-      // XCD x takes the weight panels tn = x, x + 8, ...; it sweeps them for a chunk of 8 row tiles
-      // (2048 rows of x: what its L2 can keep warm next to a panel) before the next chunk
-      const int x = tile & 7, j = tile >> 3;
-      const int P = ntiles_n >> 3, full = (mtiles >> 3) << 3;           // panels per XCD, row tiles in whole chunks
-      int tj;
-      if (j < full * P) {
-        const int c = j / (8 * P), r = j - c * 8 * P;
-        tj = r >> 3;
-        tm = c * 8 + (r & 7);
-      } else {
-        const int rem = mtiles - full, r = j - full * P;
-        tj = r / rem;
-        tm = full + r % rem;
-      }
-      tn = tj * 8 + x;
-    } else {
-      tm = tile % mtiles;
-      tn = tile / mtiles;
-    }
-    m0 = tm * FTM;
-    n0 = tn * FTN;
-  };
+  auto tile_origin = [&](int tile, int& m0, int& n0) { f8_tile_origin<GROUPED, FTM>(a, mtiles, ntiles_n, ksplits, tile, m0, n0); };
 
   f4 acc[NI][NJ];
 
   // global -> LDS: lane = 8 * row + slot, slot p of row r receives chunk p ^ (r & 7); kslab weights
   // chunk-major (lane = 8 * position + row, position p of an odd 8-row group holding chunk p ^ 1)
   const int crow = lane >> 3, cchunk = (lane & 7) ^ (crow & 7);
-  uint32_t xo[XCOPIES], wo[WCOPIES], xso = 0;
-  int wsbase = 0;
+  uint32_t xo[XCOPIES], wo[WCOPIES];
   const uint8_t *xtile, *wtile;
-  const float* xsbase = a.x_scale;
-  const long xs_kstride = (!GROUPED && a.xs_t) ? a.xs_ld : 1;       // floats between the K blocks of a row's scale
   auto set_copy_tile = [&](int tile) {
     int m0, n0;
     tile_origin(tile, m0, n0);
     long ebytes = 0;
-    int escales = 0;
     if (GROUPED) {
       const int* ids = a.sorted_ids + (m0 / FTM) * a.block_rows;
 #pragma unroll
@@ -171,7 +161,6 @@ fp8_block_gemm_kernel(F8Args a) {
       int e = a.expert_ids[m0 / FTM];
       e = __builtin_amdgcn_readfirstlane((e < 0 || e >= a.E) ? 0 : e);     // (a foreign expert's block is computed and zeroed)
       ebytes = (long)e * a.w_stride;
-      escales = e * (int)a.ws_stride;
     } else {
 #pragma unroll
       for (int p = 0; p < XCOPIES; ++p) {
@@ -198,41 +187,21 @@ fp8_block_gemm_kernel(F8Args a) {
         wo[p] = (uint32_t)(r * a.ldw + 16 * cchunk);
       }
     }
-    // activation scales: wavefronts 0..3 copy 64 rows each (index in floats)
     // (split K: the tile's range starts kb0 K blocks into every row; 64 kslab rows interleave their K blocks)
     const int kb0 = ksplits > 1 ? (tile % ksplits) * (KB / ksplits) : 0;
-    if (!GROUPED && a.xs_t) {
-      // K block major: the 64 scales of a copy lie side by side (4 cache lines instead of 64)
-      xso = (uint32_t)min(m0 + 64 * (wave & 3) + lane, M - 1);
-      xsbase = a.xs_t + (long)kb0 * a.xs_ld;
-    } else if (GROUPED) {
-      const int id = a.sorted_ids[(m0 / FTM) * a.block_rows + ((64 * (wave & 3) + lane) & (a.block_rows - 1))];
-      xso = (uint32_t)(max(0, min(id, a.numel - 1)) / a.topk) * (uint32_t)KB;
-      xsbase = a.x_scale;
-    } else {
-      xso = (uint32_t)min(m0 + 64 * (wave & 3) + lane, M - 1) * (uint32_t)KB + (uint32_t)kb0;
-      xsbase = a.x_scale;
-    }
-    wsbase = escales + (n0 >> 7) * KB + kb0;       // wavefront 4 copies the tile's weight scale
     xtile = GROUPED ? a.x : a.x + (long)m0 * a.ldx + (long)kb0 * FTKB;
     wtile = a.w + ebytes + (a.w_kslab ? (long)kb0 * FTKB * 64 : (long)n0 * a.ldw + (long)kb0 * FTKB);
   };
-  constexpr int NSLOT = XCOPIES + WCOPIES + 1;
+  constexpr int NSLOT = XCOPIES + WCOPIES;
   auto copy_slot = [&](int s, int stage, int kt) {
     unsigned char* xs = lds + stage * STAGE_BYTES;
     if (s < XCOPIES) {
       dma16(xtile + (long)kt * FTKB + xo[s], xs + (wave + 8 * s) * 1024);
-    } else if (s < XCOPIES + WCOPIES) {
+    } else {
       const int p = s - XCOPIES;
       const long koff = (OP16 && a.w_kslab) ? (long)(kt >> 1) * 16384 + (kt & 1) * 512
                                             : (a.w_kslab ? (long)kt * FTKB * 64 : (long)kt * FTKB);
       dma16(wtile + koff + wo[p < WCOPIES ? p : 0], xs + X_BYTES + (wave + 8 * p) * 1024);
-    } else if (PC) {
-      // no scales inside the K sum
-    } else if (wave < 4) {
-      dma4(xsbase + xso + (long)kt * xs_kstride, xs + X_BYTES + W_BYTES + wave * 256);
-    } else if (wave == 4) {
-      dma4(a.w_scale + wsbase + kt, xs + X_BYTES + W_BYTES + XS_BYTES);
     }
   };
 
@@ -249,14 +218,12 @@ fp8_block_gemm_kernel(F8Args a) {
                        : lo[h];
   }
   const uint32_t xwave = wm * (16 * NJ) * FTKB, wwave = X_BYTES + wn * (16 * NI) * FTKB;
-  const uint32_t xsaddr = lds_base + X_BYTES + W_BYTES + (uint32_t)(wm * 64 + l16) * 4u;
-  // The operands of one K block: two 16-byte halves per 16-row tile.  The x tiles and the
-  // activation scales of this lane's four row tiles (rows wm * 64 + 16 j + l16) have two register
+  // The operands of one K block: two 16-byte halves per 16-row tile.  The x tiles have two register
   // sets that swap roles every K block.  The w tiles of rows 0..2 have one: the MFMAs walk the w
   // tiles in order, so tile i is re-read for the next K block as soon as its four MFMAs are under
   // way; only the last w tile, in use until the end of the K block, has two sets.  (Two full sets
   // would need 128 registers of the 256 a wavefront has at two wavefronts per SIMD.)
-  struct XOps { i4 bx[2][NJ]; float xs[NJ]; float ws; };
+  struct XOps { i4 bx[2][NJ]; };
   typedef i4 WTile[2];
   auto read_x = [&](XOps& f, int h, int j, uint32_t stage_off) {
     const uint32_t xb = lo[h] + stage_off + xwave;
@@ -273,14 +240,6 @@ fp8_block_gemm_kernel(F8Args a) {
         if (ii == i) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(t[h]) : "v"(wb), "n"(ii * 16 * FTKB));
     }
   };
-  auto read_xs = [&](XOps& f, uint32_t stage_off) {
-    if (PC) return;
-    const uint32_t ad = xsaddr + stage_off;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-      asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(f.xs[j]) : "v"(ad), "n"(j * 64));
-    asm volatile("ds_read_b32 %0, %1" : "=v"(f.ws) : "v"(lds_base + (uint32_t)(X_BYTES + W_BYTES + XS_BYTES) + stage_off));
-  };
   WTile w012[3];
   auto lds_wait = [&](XOps& f, WTile& w3) {
     // every register the reads of a step write, exactly once each
@@ -288,18 +247,12 @@ fp8_block_gemm_kernel(F8Args a) {
                  : "+v"(f.bx[0][0]), "+v"(f.bx[0][1]), "+v"(f.bx[0][2]), "+v"(f.bx[0][3]), "+v"(f.bx[1][0]),
                    "+v"(f.bx[1][1]), "+v"(f.bx[1][2]), "+v"(f.bx[1][3]), "+v"(w012[0][0]), "+v"(w012[0][1]),
                    "+v"(w012[1][0]), "+v"(w012[1][1]), "+v"(w012[2][0]), "+v"(w012[2][1]), "+v"(w3[0]),
-                   "+v"(w3[1]), "+v"(f.xs[0]), "+v"(f.xs[1]), "+v"(f.xs[2]), "+v"(f.xs[3]), "+v"(f.ws));
+                   "+v"(w3[1]));
   };
 
-  // One K block: one 128-deep MFMA per (w tile i, x tile j), started from zero; its result joins
-  // the running sum with the block's scale two MFMAs later, when the matrix pipe has delivered it.
-  // Between the MFMAs: the operand and scale reads of the next K block (a w tile one MFMA after
+  // One K block: one 128-deep MFMA per (w tile i, x tile j).  Between the MFMAs: the operand reads of the next K block (a w tile one MFMA after
   // the last one that used it) and the copy slots of the K block three ahead.
   auto step = [&](const XOps& cur, XOps& nxt, const WTile& w3cur, WTile& w3nxt, uint32_t rso, int cstage, int kt) {
-    float sc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) sc[j] = cur.xs[j] * cur.ws;
-    f4 ring[4];
     const bool odd_slots = wave < 4;
     int n = 0;
 #pragma unroll
@@ -317,36 +270,25 @@ fp8_block_gemm_kernel(F8Args a) {
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<b8>(a0), bitcast<b8>(cur.bx[0][j]), acc[i][j], 0, 0, 0);
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bitcast<b8>(a1), bitcast<b8>(cur.bx[1][j]), acc[i][j], 0, 0, 0);
           }
-        } else if (PC) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[i][j], 0, 0, 0, 0, 0, 0);
-        else ring[n & 3] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, (f4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-        if (!PC && n >= 2) {
-          const int pn = n - 2;
-          acc[pn / NJ][pn % NJ] += sc[pn % NJ] * ring[pn & 3];
-          // (pinned here: left alone, the compiler gives every MFMA a result tile of its own and sinks all
-          // sixty-four multiply-adds behind the last MFMA, where the matrix pipe waits for them)
-          asm volatile("" : "+v"(acc[pn / NJ][pn % NJ]));
+        } else {
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[i][j], 0, 0, 0, 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
         if (n == 0) read_w(w3nxt, 3, rso);
         if (n == 4) read_w(w012[0], 0, rso);
         if (n == 8) read_w(w012[1], 1, rso);
         if (n == 12) read_w(w012[2], 2, rso);
-        // x tiles: one read after each of MFMAs 1 2 3, 5 6 7, 9 10; the scales after 13
+        // x tiles: one read after each of MFMAs 1 2 3, 5 6 7, 9 10
         if ((n & 3) != 0 && n < 11) {
           const int r = n - 1 - (n >> 2);             // 0..7
           read_x(nxt, r >> 2, r & 3, rso);
         }
-        if (n == 13) read_xs(nxt, rso);
         // copy slot k after MFMA 2 k + 1 in wavefronts 0..3, after MFMA 2 k + 2 in wavefronts 4..7: the
         // address unit takes one copy (1 KiB) at a time, and eight in the same cycle queue up
         if (n >= 1 && n <= 2 * NSLOT && ((n & 1) != 0) == odd_slots) copy_slot((n - 1) >> 1, cstage, kt);
         __builtin_amdgcn_sched_barrier(0);
         ++n;
       }
-    if (!PC) {
-#pragma unroll
-      for (int pn = NI * NJ - 2; pn < NI * NJ; ++pn) acc[pn / NJ][pn % NJ] += sc[pn % NJ] * ring[pn & 3];
-    }
   };
   static_assert(NI == 4 && NJ == 4 && NSLOT <= 8, "the read and copy schedule is written for 16 MFMAs per K block");
 
@@ -373,9 +315,7 @@ fp8_block_gemm_kernel(F8Args a) {
     return kt;
   };
   auto wait_all_but_last_step = [&]() {
-    // copies per step and wavefront: 4 x + 2 w, and one of scales in wavefronts 0..4
-    if (!PC && wave <= 4) __builtin_amdgcn_s_waitcnt(0x0f77);  // vmcnt(7)
-    else __builtin_amdgcn_s_waitcnt(0x0f76);                   // vmcnt(6)
+    __builtin_amdgcn_s_waitcnt(0x0f76);            // vmcnt(6): 4 copies of x and 2 of w per step and wavefront
   };
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -392,7 +332,6 @@ fp8_block_gemm_kernel(F8Args a) {
 #pragma unroll
   for (int i = 0; i < 3; ++i) read_w(w012[i], i, 0);
   read_w(w3a, 3, 0);
-  read_xs(o0, 0);
   lds_wait(o0, w3a);
   __builtin_amdgcn_s_barrier();                    // nobody still reads element 0 when step 0 overwrites its stage
   int st = 0;                                      // stage of the current element
@@ -494,25 +433,23 @@ fp8_block_gemm_kernel(F8Args a) {
       for (int e = 0; e < 4; ++e) bia[i][e] = a.bias ? Elem<DT>::to_f32(((const uint16_t*)a.bias)[n + e]) : 0.0f;
     }
     float wsc[NI][4];
-    if (PC) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int n = n0 + wn * (16 * NI) + i * 16 + 4 * kq;
+    for (int i = 0; i < NI; ++i) {
+      const int n = n0 + wn * (16 * NI) + i * 16 + 4 * kq;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) wsc[i][e] = a.w_scale[(n + e) * a.ws_mul];
-      }
+      for (int e = 0; e < 4; ++e) wsc[i][e] = a.w_scale[(n + e) * a.ws_mul];
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       const int m = m0 + wm * (16 * NJ) + j * 16 + l16;
       if (m >= M) continue;
-      const float xsc = PC ? a.x_scale[(long)m * a.xs_mul] : 1.0f;
+      const float xsc = a.x_scale[(long)m * a.xs_mul];
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         const int n = n0 + wn * (16 * NI) + i * 16 + 4 * kq;
         float v[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = plus_bias(PC ? scaled_sum(acc[i][j][e], xsc, wsc[i][e]) : acc[i][j][e], bia[i][e]);
+        for (int e = 0; e < 4; ++e) v[e] = plus_bias(scaled_sum(acc[i][j][e], xsc, wsc[i][e]), bia[i][e]);
         u2 o;
         o.x = (uint32_t)Elem<DT>::from_f32(v[0]) | ((uint32_t)Elem<DT>::from_f32(v[1]) << 16);
         o.y = (uint32_t)Elem<DT>::from_f32(v[2]) | ((uint32_t)Elem<DT>::from_f32(v[3]) << 16);
@@ -525,6 +462,347 @@ fp8_block_gemm_kernel(F8Args a) {
   }
   // no copy may still be writing LDS when the workgroup retires
   __builtin_amdgcn_s_waitcnt(0x0f70);              // vmcnt(0)
+}
+
+// ---- 128 x 128 block scales ------------------------------------------------------------------------------------------
+// The same tiles and LDS images as above (BM = 256 rows of x, or 128 where there are no more), another division of work:
+// four wavefronts, one per SIMD with 256 registers, multiply BM / 2 x 64 each, and four copy.  Per K block every product
+// of the matrix pipe (32 clocks) joins the running sum by four multiply-adds with the block's scale, and what the
+// wavefronts that multiply issue besides -- a copy holds its wavefront up for as long as the address path is busy, 16 clocks
+// and more each -- comes on top: with eight wavefronts that did both a K block of 256 x 128 took 1.09 us, here 0.93 (0.57
+// without the multiply-adds; 0.45 the matrix pipe alone; 0.76 with operands of zeros: the rest is the clock, which the power
+// limit lowers).  x tiles of BM / 2 rows pass through four register slots; the last two x tiles of a K block are multiplied by
+// w tile, so that each w tile is read again for the next K block as soon as its last product is under way, and the
+// barrier lies before them, where the stage before has been read and the next one is needed.
+// (us, before -> here: K 7168 x N 4096 at 1537 / 2048 rows 71.6 -> 58.3 / 69.6 -> 60.3; K 2048 x N 7168 at 1537 45.8 -> 40.1;
+// K 4096 x N 28672 at 1024 153.7 -> 133.5; K 8192 x N 28672 at 2048 520 -> 469)
+__device__ __forceinline__ void f8_copy16(uint32_t voff, const void* sbase, uint32_t lds_addr) {
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+}
+// 64 x 4 B: lane l lands at base + 4 l
+__device__ __forceinline__ void f8_copy4(uint32_t voff, const void* sbase, uint32_t lds_addr) {
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+}
+// x, w, a scale per row (1 KiB) and the tile's weight scale, 64 times
+constexpr int f8_stage_bytes(int BM) { return BM * FTKB + FTN * FTKB + 1024 + 256; }
+
+template <int DT, bool GROUPED, int BM>
+__global__ void __launch_bounds__(F8_THREADS, 1)
+fp8_block_gemm_kernel(F8Args a) {
+  constexpr int WN = 2, NI = 4, NJ = BM / 32;           // 2 x 2 wavefronts of BM / 2 x 64 multiply, four copy
+  constexpr int X_BYTES = BM * FTKB, W_BYTES = FTN * FTKB, STAGE_BYTES = f8_stage_bytes(BM);
+  constexpr int XCOPIES = BM / 8 / 4, WCOPIES = FTN / 8 / 4;       // 1 KiB copies per copying wavefront
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3;
+  const bool copies = wave8 >= 4;
+  const int l16 = lane & 15, kq = lane >> 4;
+  const int wm = wave / WN, wn = wave % WN;
+  const int M = a.M, N = a.N, K = a.K, KB = K >> 7;
+
+  int mtiles = (M + BM - 1) / BM;
+  if (GROUPED) {
+    const int blocks = (*a.npp + BM - 1) / BM;
+    mtiles = __builtin_amdgcn_readfirstlane(blocks < a.max_blocks ? blocks : a.max_blocks);
+  }
+  const int ntiles_n = N / FTN;
+  const int ksplits = (!GROUPED && a.ksplits > 1) ? a.ksplits : 1;
+  const int total_tiles = mtiles * ntiles_n * ksplits;   // (split K: tile ids count (output tile, K range) pairs)
+  if (GROUPED && (int)blockIdx.x >= total_tiles) return;  // (the grid is sized for the largest block count the ids can fill)
+  auto tile_origin = [&](int tile, int& m0, int& n0) { f8_tile_origin<GROUPED, BM>(a, mtiles, ntiles_n, ksplits, tile, m0, n0); };
+
+  const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)lds);
+  const int nt = KB / ksplits;                     // K blocks per (output tile, K range)
+  // (kept in a register: read through the dispatch packet it is fetched again in every iteration)
+  const int gdim = __builtin_amdgcn_readfirstlane((int)gridDim.x);
+  int tile = blockIdx.x;
+  const int mytiles = (total_tiles - tile + gdim - 1) / gdim;
+  const int elements = mytiles * nt;               // K blocks this workgroup multiplies, over all its tiles
+
+  if (copies) {
+  // global -> LDS: lane = 8 * row + slot, slot p of row r receives chunk p ^ (r & 7); kslab weights
+  // chunk-major (lane = 8 * position + row, position p of an odd 8-row group holding chunk p ^ 1)
+  const int crow = lane >> 3, cchunk = (lane & 7) ^ (crow & 7);
+  uint32_t xo[XCOPIES], wo[WCOPIES], xso = 0;
+  int wsbase = 0;
+  const uint8_t *xtile, *wtile;
+  const float* xsbase = a.x_scale;
+  const long xs_kstride = (!GROUPED && a.xs_t) ? a.xs_ld : 1;       // floats between the K blocks of a row's scale
+  auto set_copy_tile = [&](int tile) {
+    int m0, n0;
+    tile_origin(tile, m0, n0);
+    long ebytes = 0;
+    int escales = 0;
+    if (GROUPED) {
+      const int* ids = a.sorted_ids + m0;
+#pragma unroll
+      for (int p = 0; p < XCOPIES; ++p) {
+        const int id = ids[(wave + 4 * p) * 8 + crow];
+        xo[p] = (uint32_t)(max(0, min(id, a.numel - 1)) / a.topk) * (uint32_t)a.ldx + (uint32_t)(16 * cchunk);   // pads read a valid row
+      }
+      int e = a.expert_ids[m0 / BM];
+      e = __builtin_amdgcn_readfirstlane((e < 0 || e >= a.E) ? 0 : e);     // (a foreign expert's block is computed and zeroed)
+      ebytes = (long)e * a.w_stride;
+      escales = e * (int)a.ws_stride;
+    } else {
+#pragma unroll
+      for (int p = 0; p < XCOPIES; ++p) {
+        const int r = (wave + 4 * p) * 8 + crow;
+        xo[p] = (uint32_t)((min(m0 + r, M - 1) - m0) * a.ldx + 16 * cchunk);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < WCOPIES; ++p) {
+      if (a.w_kslab) {
+        const uint32_t n = (uint32_t)(n0 + (wave + 4 * p) * 8 + (lane & 7));
+        const uint32_t c = (uint32_t)((lane >> 3) ^ (wave & 1));
+        wo[p] = ((n >> 6) * (uint32_t)(K >> 7) * 4u + ((n & 63u) >> 4)) * 2048u + (c & 1u) * 1024u +
+                ((c >> 1) * 16u + (n & 15u)) * 16u;
+      } else {
+        const int r = (wave + 4 * p) * 8 + crow;
+        wo[p] = (uint32_t)(r * a.ldw + 16 * cchunk);
+      }
+    }
+    // activation scales: 64 rows per copying wavefront, 128-row tiles twice (index in floats)
+    const int srow = (64 * wave + lane) & (BM - 1);
+    // (split K: the tile's range starts kb0 K blocks into every row; 64 kslab rows interleave their K blocks)
+    const int kb0 = ksplits > 1 ? (tile % ksplits) * (KB / ksplits) : 0;
+    if (!GROUPED && a.xs_t) {
+      // K block major: the 64 scales of a copy lie side by side (4 cache lines instead of 64)
+      xso = (uint32_t)min(m0 + srow, M - 1);
+      xsbase = a.xs_t + (long)kb0 * a.xs_ld;
+    } else if (GROUPED) {
+      const int id = a.sorted_ids[m0 + srow];
+      xso = (uint32_t)(max(0, min(id, a.numel - 1)) / a.topk) * (uint32_t)KB;
+      xsbase = a.x_scale;
+    } else {
+      xso = (uint32_t)min(m0 + srow, M - 1) * (uint32_t)KB + (uint32_t)kb0;
+      xsbase = a.x_scale;
+    }
+    wsbase = escales + (n0 >> 7) * KB + kb0;       // the first of them copies the tile's weight scale
+    xtile = GROUPED ? a.x : a.x + (long)m0 * a.ldx + (long)kb0 * FTKB;
+    wtile = a.w + ebytes + (a.w_kslab ? (long)kb0 * FTKB * 64 : (long)n0 * a.ldw + (long)kb0 * FTKB);
+  };
+    // the K block that the next copies are of; past the last one a re-read that nobody consumes
+    int kt = 0;
+    set_copy_tile(tile);
+    auto copy_stage = [&](int stage) {
+      const uint32_t xs = lds_base + (uint32_t)(stage * STAGE_BYTES);
+#pragma unroll
+      for (int p = 0; p < XCOPIES; ++p) f8_copy16(xo[p], xtile + (long)kt * FTKB, xs + (uint32_t)((wave + 4 * p) * 1024));
+      const long koff = a.w_kslab ? (long)kt * FTKB * 64 : (long)kt * FTKB;
+#pragma unroll
+      for (int p = 0; p < WCOPIES; ++p) f8_copy16(wo[p], wtile + koff, xs + (uint32_t)(X_BYTES + (wave + 4 * p) * 1024));
+      f8_copy4(xso * 4u, xsbase + (long)kt * xs_kstride, xs + (uint32_t)(X_BYTES + W_BYTES + wave * 256));
+      if (wave == 0) f8_copy4(0u, a.w_scale + wsbase + kt, xs + (uint32_t)(X_BYTES + W_BYTES + 1024));
+      if (++kt == nt) {
+        if (tile + gdim < total_tiles) {
+          tile += gdim;
+          kt = 0;
+          set_copy_tile(tile);
+        } else {
+          kt = nt - 1;
+        }
+      }
+    };
+    auto wait_all_but_last_stage = [&]() {
+      constexpr int NC = XCOPIES + WCOPIES + 1;
+      if (wave == 0) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(NC + 1) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(NC) : "memory");
+    };
+    copy_stage(0);
+    copy_stage(1);
+    int st = 2;
+    for (int g = 0; g <= elements; ++g) {
+      wait_all_but_last_stage();                   // element g has landed
+      __builtin_amdgcn_s_barrier();                // ... everybody's share of it, and nobody reads element g - 1 any more
+      copy_stage(st);
+      st = st == 2 ? 0 : st + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");   // no copy may still be writing LDS when the workgroup retires
+    return;
+  }
+
+  // no row of the (only) row tile in this wavefront's share: it keeps the workgroup's barriers
+  if (!GROUPED && mtiles == 1 && wm * (16 * NJ) >= M) {
+    for (int g = 0; g <= elements; ++g) __builtin_amdgcn_s_barrier();
+    return;
+  }
+
+  uint32_t xa[2], wa[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    xa[h] = (uint32_t)(wm * (16 * NJ) * FTKB + l16 * FTKB + (((4 * h + kq) ^ (l16 & 7)) * 16));
+    wa[h] = (uint32_t)(X_BYTES + wn * (16 * NI) * FTKB) +
+            (a.w_kslab ? (uint32_t)((l16 >> 3) * 1024 + (((4 * h + kq) ^ (l16 >> 3)) * 128) + (l16 & 7) * 16)
+                       : (uint32_t)(l16 * FTKB + (((4 * h + kq) ^ (l16 & 7)) * 16)));
+  }
+  const uint32_t xsa = (uint32_t)(X_BYTES + W_BYTES) + (uint32_t)(wm * (16 * NJ) + l16) * 4u;
+  struct Tile { i4 h[2]; };
+  f4 acc[NI][NJ], ring[4];
+  Tile w[NI], x[4];
+  float sc[NJ], xsn[NJ], wsn;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    w[i].h[0] = w[i].h[1] = x[i].h[0] = x[i].h[1] = (i4){0, 0, 0, 0};
+    ring[i] = (f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) sc[j] = 0.f;
+  auto read_x = [&](Tile& t, int j, uint32_t so) {
+    t.h[0] = *(const i4*)(lds + so + xa[0] + j * 2048);
+    t.h[1] = *(const i4*)(lds + so + xa[1] + j * 2048);
+  };
+  auto read_w = [&](Tile& t, int i, uint32_t so) {
+    t.h[0] = *(const i4*)(lds + so + wa[0] + i * 2048);
+    t.h[1] = *(const i4*)(lds + so + wa[1] + i * 2048);
+  };
+  // position p of a round: the last two x tiles of the K block before by w tile (p < 8), then the others of this one by x tile
+  auto pi = [](int p) constexpr { return p < 8 ? p >> 1 : (p - 8) & 3; };
+  auto pj = [](int p) constexpr { return p < 8 ? NJ - 2 + (p & 1) : (p - 8) >> 2; };
+  auto add = [&](int q) {                          // the product of position q joins the running sum
+    acc[pi(q)][pj(q)] += sc[pj(q)] * ring[q & 3];
+    // (pinned here: left alone, the compiler gives every MFMA a result tile of its own and sinks all
+    // multiply-adds behind the last MFMA, where the matrix pipe waits for them)
+    asm volatile("" : "+v"(acc[pi(q)][pj(q)]));
+  };
+  auto multiply = [&](int p) {
+    const int i = pi(p), j = pj(p);
+    const i4 a0 = w[i].h[0], a1 = w[i].h[1], b0 = x[j & 3].h[0], b1 = x[j & 3].h[1];
+    const i8v av = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+    const i8v bv = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
+    ring[p & 3] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, (f4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto epilogue = [&](int tile) {
+    int m0, n0;
+    tile_origin(tile, m0, n0);
+    // ---- epilogue: lane holds, per (w tile i, x tile j), output row m = .. + l16 and columns
+    // n = .. + 4 kq + {0..3}
+    if (ksplits > 1) {
+      // split K: the fp32 sums of this K range, nothing else; bias (and the scales that live outside the
+      // K sum) are the second launch's
+      float* const part = a.partial + (long)(tile % ksplits) * M * N;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int m = m0 + wm * (16 * NJ) + j * 16 + l16;
+        if (m >= M) continue;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) *(f4*)(part + (long)m * N + n0 + wn * (16 * NI) + i * 16 + 4 * kq) = acc[i][j];
+      }
+      return;
+    }
+    if (GROUPED) {
+      const int e = a.expert_ids[m0 / BM];
+      const bool foreign = e < 0 || e >= a.E;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int id = a.sorted_ids[m0 + wm * (16 * NJ) + j * 16 + l16];
+        if (id >= a.numel || id < 0) continue;
+        const float rw = foreign ? 0.0f : (a.topk_weights ? a.topk_weights[id] : 1.0f);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int n = n0 + wn * (16 * NI) + i * 16 + 4 * kq;
+          float v[4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = foreign ? 0.0f : acc[i][j][c] * rw;
+          u2 o;
+          o.x = (uint32_t)Elem<DT>::from_f32(v[0]) | ((uint32_t)Elem<DT>::from_f32(v[1]) << 16);
+          o.y = (uint32_t)Elem<DT>::from_f32(v[2]) | ((uint32_t)Elem<DT>::from_f32(v[3]) << 16);
+          *(u2*)((uint16_t*)a.out + (long)id * a.ldo + n) = o;
+        }
+      }
+      return;
+    }
+    float bia[NI][4];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int n = n0 + wn * (16 * NI) + i * 16 + 4 * kq;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bia[i][e] = a.bias ? Elem<DT>::to_f32(((const uint16_t*)a.bias)[n + e]) : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int m = m0 + wm * (16 * NJ) + j * 16 + l16;
+      if (m >= M) continue;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int n = n0 + wn * (16 * NI) + i * 16 + 4 * kq;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = plus_bias(acc[i][j][e], bia[i][e]);
+        u2 o;
+        o.x = (uint32_t)Elem<DT>::from_f32(v[0]) | ((uint32_t)Elem<DT>::from_f32(v[1]) << 16);
+        o.y = (uint32_t)Elem<DT>::from_f32(v[2]) | ((uint32_t)Elem<DT>::from_f32(v[3]) << 16);
+        *(u2*)((uint16_t*)a.out + (long)m * a.ldo + n) = o;
+      }
+    }
+  };
+
+  int st = 0, T = 0, done = -1;                    // done: the output tile whose last K block is still being multiplied
+  for (;;) {
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
+    const uint32_t so = (uint32_t)(st * STAGE_BYTES);
+    st = st == 2 ? 0 : st + 1;
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+      multiply(p);
+      add((p + 4 * NJ - 2) % (4 * NJ));
+      if (p == 0) read_x(x[0], 0, so);
+      if (p == 1) read_x(x[1], 1, so);
+      if (p >= 2 && (p & 1) == 0) read_w(w[(p >> 1) - 1], (p >> 1) - 1, so);
+      if (p == 3) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) xsn[j] = *(const float*)(lds + so + xsa + j * 64);
+        wsn = *(const float*)(lds + so + X_BYTES + W_BYTES + 1024);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    read_w(w[3], 3, so);
+    read_x(x[2], 2, so);
+    __builtin_amdgcn_sched_barrier(0);
+    if (T == 0) {
+      if (done >= 0) {
+        add(6);
+        add(7);
+        ring[2] = ring[3] = (f4){0.f, 0.f, 0.f, 0.f};
+        epilogue(done);
+      }
+      if (tile >= total_tiles) return;
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
+    }
+    const float sa = sc[NJ - 2], sb = sc[NJ - 1];     // (positions 6 and 7 still belong to the K block before)
+#pragma unroll
+    for (int p = 8; p < 4 * NJ; ++p) {
+      multiply(p);
+      if (p == 8) {
+        acc[3][NJ - 2] += sa * ring[2];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) sc[j] = xsn[j] * wsn;
+      } else if (p == 9) {
+        acc[3][NJ - 1] += sb * ring[3];
+      } else {
+        add(p - 2);
+      }
+      // x tile j of this K block into slot j & 3 once tile j - 4 (or the K block before's) is through
+      if (p == 9) read_x(x[3], 3, so);
+      if (NJ == 8 && p >= 12 && (p & 3) == 1 && p < 29) read_x(x[((p - 13) >> 2) & 3], 4 + ((p - 13) >> 2), so);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (++T == nt) {
+      T = 0;
+      done = tile;
+      tile += gdim;
+    }
+  }
 }
 
 // Second launch of a split: the ranges' sums added in range order (run-to-run identical), then the epilogue.
@@ -582,6 +860,14 @@ constexpr size_t F8_SPLITK_BYTES = (size_t)64 << 20;
 constexpr size_t F8_WS_OFFSET = (size_t)1 << 20;     // the first MiB of a workspace belongs to the W4A16 arrival counters
 
 }  // namespace
+
+// Rounds of the block-scale kernel, in units of a round of 256-row tiles: a K block of a 128-row tile takes 0.61 us, of a 256-row
+// tile 0.93, so the smaller ones pay where they fill a last round that the larger ones leave half empty (us, 128 against
+// 256 rows: K 2048 x N 7168 at 1537 rows 38.8 / 41.9, K 4096 x N 8192 at 1300 60.4 / 65.4; K 7168 x N 4096 at 1537 66.4 / 59.0).
+double f8_block_rounds(int M, int N, int bm) {
+  const long cus = std::max(8, device_cu_count() / 8 * 8), tiles = (long)((M + bm - 1) / bm) * (N / FTN);
+  return (double)((tiles + cus - 1) / cus) * (bm == 256 ? 1.0 : 0.65);
+}
 
 // K ranges for a shape: as many as put about one 256 x 128 tile on every CU, each at least eight K
 // blocks long, a divisor of the K block count, partial sums within 64 MiB.  1: no split.
@@ -659,36 +945,41 @@ int launch_f8_auto(F8Args& a, void* workspace, size_t workspace_bytes, hipStream
   return launch_f8<DT, PC>(a, st);
 }
 
-template <int DT, bool PC>
-int launch_f8(const F8Args& a, hipStream_t st) {
-  const int mtiles = (a.M + FTM - 1) / FTM, ntiles = a.N / FTN;
-  F8Args b = a;
-  const int ks = a.ksplits > 1 ? a.ksplits : 1;
-  b.n_panels_swizzle = (ntiles % 8 == 0 && ks == 1) ? 1 : 0;
-  const size_t shmem = 3 * (size_t)(FTM * FTKB + FTN * FTKB + FTM * 4 + 256);
-  static hipError_t attr = hipFuncSetAttribute((const void*)fp8_block_gemm_kernel<DT, PC>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+template <int DT, int BM, bool GROUPED = false>
+int launch_f8_block(const F8Args& a, int grid, hipStream_t st) {
+  const size_t shmem = 3 * (size_t)f8_stage_bytes(BM);
+  static hipError_t attr = hipFuncSetAttribute((const void*)fp8_block_gemm_kernel<DT, GROUPED, BM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   MQ_REQUIRE(attr == hipSuccess, "fp8 gemm: cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
-  int grid = mtiles * ntiles * ks, cus = device_cu_count() / 8 * 8;
-  if (cus >= 8 && grid > cus) grid = cus;
-  hipLaunchKernelGGL((fp8_block_gemm_kernel<DT, PC>), dim3(grid), dim3(F8_THREADS), shmem, st, b);
+  hipLaunchKernelGGL((fp8_block_gemm_kernel<DT, GROUPED, BM>), dim3((unsigned)grid), dim3(F8_THREADS), shmem, st, a);
   MQ_LAUNCH_CHECK("fp8 gemm");
   return 0;
 }
 
-template <int DT, bool OP16 = false>
-int launch_f8_grouped(const F8Args& a, hipStream_t st) {
-  const size_t shmem = 3 * (size_t)(FTM * FTKB + FTN * FTKB + FTM * 4 + 256);
-  static hipError_t attr = hipFuncSetAttribute((const void*)fp8_block_gemm_kernel<DT, OP16, true, OP16>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
-  MQ_REQUIRE(attr == hipSuccess, "moe_gemm(MFMA tiles): cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
-  long grid = (long)a.max_blocks * (a.N / FTN);
-  const long cus = device_cu_count();
-  if (grid > cus) grid = cus;
-  hipLaunchKernelGGL((fp8_block_gemm_kernel<DT, OP16, true, OP16>), dim3((unsigned)grid), dim3(F8_THREADS), shmem, st, a);
-  MQ_LAUNCH_CHECK("moe_gemm(MFMA tiles)");
+template <int DT, bool OP16>
+int launch_f8_pc(const F8Args& a, int grid, hipStream_t st) {
+  const size_t shmem = 3 * (size_t)(FTM * FTKB + FTN * FTKB);
+  static hipError_t attr = hipFuncSetAttribute((const void*)fp8_pc_gemm_kernel<DT, OP16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+  MQ_REQUIRE(attr == hipSuccess, "fp8 gemm: cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
+  hipLaunchKernelGGL((fp8_pc_gemm_kernel<DT, OP16>), dim3((unsigned)grid), dim3(F8_THREADS), shmem, st, a);
+  MQ_LAUNCH_CHECK("fp8 gemm");
   return 0;
 }
+
+template <int DT, bool PC>
+int launch_f8(const F8Args& a, hipStream_t st) {
+  const int ks = a.ksplits > 1 ? a.ksplits : 1;
+  const bool low = !PC && (a.M <= 128 || (ks == 1 && f8_block_rounds(a.M, a.N, 128) < f8_block_rounds(a.M, a.N, 256)));
+  const int bm = low ? 128 : 256, mtiles = (a.M + bm - 1) / bm, ntiles = a.N / FTN;
+  F8Args b = a;
+  b.n_panels_swizzle = (ntiles % 8 == 0 && ks == 1) ? 1 : 0;
+  int grid = mtiles * ntiles * ks, cus = device_cu_count() / 8 * 8;
+  if (cus >= 8 && grid > cus) grid = cus;
+  if constexpr (PC) return launch_f8_pc<DT, false>(b, grid, st);
+  else return low ? launch_f8_block<DT, 128>(b, grid, st) : launch_f8_block<DT, 256>(b, grid, st);
+}
+
+// grouped launches: as many workgroups as CUs at most (the number of filled blocks is read on the device)
+int f8_grouped_grid(const F8Args& a) { return (int)std::min<long>((long)a.max_blocks * (a.N / FTN), device_cu_count()); }
 
 }  // namespace
 
@@ -714,7 +1005,10 @@ int fp8_block_grouped_launch(void* out, const void* a, const void* w, const floa
   g.block_rows = block_size;
   g.w_stride = (long)N * K;
   g.ws_stride = (long)(N / 128) * (K / 128);
-  return out_dtype == MI355Q_F16 ? launch_f8_grouped<MI355Q_F16>(g, st) : launch_f8_grouped<MI355Q_BF16>(g, st);
+  const int grid = f8_grouped_grid(g);
+  if (block_size == 128)
+    return out_dtype == MI355Q_F16 ? launch_f8_block<MI355Q_F16, 128, true>(g, grid, st) : launch_f8_block<MI355Q_BF16, 128, true>(g, grid, st);
+  return out_dtype == MI355Q_F16 ? launch_f8_block<MI355Q_F16, 256, true>(g, grid, st) : launch_f8_block<MI355Q_BF16, 256, true>(g, grid, st);
 }
 
 // The same for unquantised fp16 / bf16 experts ([E, N, K] row-major, or the kslab order of 2-byte elements):
@@ -736,7 +1030,8 @@ int half_grouped_tile_launch(void* out, const void* a, const void* w, const floa
   g.numel = numel; g.topk = topk; g.E = E; g.max_blocks = max_blocks;
   g.block_rows = block_size;
   g.w_stride = 2L * N * K;
-  return dtype == MI355Q_F16 ? launch_f8_grouped<MI355Q_F16, true>(g, st) : launch_f8_grouped<MI355Q_BF16, true>(g, st);
+  const int grid = f8_grouped_grid(g);
+  return dtype == MI355Q_F16 ? launch_f8_pc<MI355Q_F16, true>(g, grid, st) : launch_f8_pc<MI355Q_BF16, true>(g, grid, st);
 }
 
 }  // namespace mi355q

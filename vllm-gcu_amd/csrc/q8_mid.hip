@@ -30,6 +30,7 @@ namespace mi355q {
 
 // K ranges of the 256-row tile kernels (1: none), and the int8 one's rounds in units of a round of 256 x 128 tiles
 int fp8_ksplits(int M, int N, int K);
+double f8_block_rounds(int M, int N, int bm);
 int int8_ksplits(int M, int N, int K);
 int int8_ksplits_wide(int M, int N, int K);
 double int8_tile_rounds(int M, int N);
@@ -351,7 +352,7 @@ constexpr Q8Price kPlainPrice = {3.4, 1.6, 1.55, {0.151, 0.232, 0.961}, {0.200, 
 struct TilePrice {
   double base, step, split, split_mn;
 };
-constexpr TilePrice kTilePrice[3] = {{0.4, 1.18, 6.6, 1.61}, {2.6, 0.881, 4.3, 1.70}, {7.2, 0.776, 0.9, 1.83}};
+constexpr TilePrice kTilePrice[3] = {{6.5, 0.95, 4.0, 1.61}, {2.6, 0.881, 4.3, 1.70}, {7.2, 0.776, 0.9, 1.83}};
 
 double with_stream(double t, double K, double N) {      // never faster than the weights arrive
   const double h = K * N / 5.05e6;
@@ -369,6 +370,7 @@ double tile_kernel_price(int mode, int M, int N, int K) {
   const long cus = device_cu_count();
   const TilePrice& p = kTilePrice[mode];
   double rounds = (double)(((long)((M + 255) / 256) * ((N + 127) / 128) * splits + cus - 1) / cus);
+  if (mode == Q8_BLOCK && splits == 1) rounds = std::min(f8_block_rounds(M, N, 128), f8_block_rounds(M, N, 256));
   if (mode == Q8_INT8 && splits == 1) {
     const int wide = int8_ksplits_wide(M, N, K);            // ranges of 256 x 256 tiles, one round
     rounds = wide ? 1 / 0.545 : int8_tile_rounds(M, N);
