@@ -6,7 +6,7 @@
 // wavefronts without rows, and the few tiles there are walk K at about 1 us per K block (sixteen MFMAs, as many
 // operand reads and sixty-four scale multiply-adds in a row per wavefront).  Here a workgroup of four wavefronts owns
 // a tile of 32 x 64 or 64 x 64, and two or three workgroups share a CU and fill each other's barrier and LDS waits (or
-// eight wavefronts own 128 x 128 rows, alone on it), so that every wavefront has rows and K is cut into fewer ranges,
+// twelve own 48 .. 128 rows x 128 columns, alone on it), so that every wavefront has rows and K is cut into fewer ranges,
 // there being two to eight times as many tiles.
 //
 // Every operand travels from global memory straight into a ring of LDS stages (one K block of 128 bytes per row each),
@@ -15,11 +15,11 @@
 // row after the other with an odd pitch.  kslab weights are the LDS image already: a copy is one contiguous KiB.
 //
 // Measured against the streamer / the 256-row tiles (us): fp8 block 2048 x 7168 at 48 / 128 / 256 / 512 rows 9.1 / 18.6 / 25.6 /
-// 26.7 -> 6.4 / 8.0 / 10.2 / 15.6, 7168 x 4096 17.6 / 21.9 / 28.9 / 36.3 -> 11.4 / 15.6 / 20.5 / 30.1; int8 3584 x 4608 16.1 /
-// 18.6 / 25.3 / 29.4 -> 7.7 / 9.6 / 13.9 / 21.3, 8192 x 8192 at 128 / 512: 26.0 / 51.8 -> 24.3 / 43.7.  What bounds it: HBM up to
+// 26.7 -> 6.4 / 8.0 / 9.0 / 13.7, 7168 x 4096 17.6 / 21.9 / 28.9 / 36.3 -> 11.4 / 15.6 / 20.5 / 26.9; int8 3584 x 4608 16.1 /
+// 18.6 / 25.3 / 29.4 -> 7.7 / 9.6 / 13.9 / 19.5, 8192 x 8192 at 512: 51.8 -> 48.2.  What bounds it: HBM up to
 // about 100 rows on large layers; the launch and the filling of the ring (4 us) on small ones; above, the step of a K block
-// (0.6 us for 128 x 128 with eight wavefronts: barrier, 12 operand reads, 4 copies and 8 .. 16 matrix instructions each --
-// taking out any one of the three saves a fifth), which is why the 256-row tiles win again from about 1000 rows.
+// (barrier, operand reads, copies and matrix instructions, none of which alone is more than half of it), which is why the
+// 256-row tiles win again from about 1000 rows.
 #include "common.h"
 
 #include <algorithm>
@@ -51,7 +51,6 @@ struct Q8Args {
   long ldx, ldo;
   int kper;                 // K blocks per range (blockIdx.y)
   int mtiles;
-  int xcds;                 // the column tiles are a multiple of the eight XCDs
   void* partial;            // split K: f32 / int32 sums [range][M][N]; null: write the output
 };
 
@@ -124,17 +123,11 @@ q8_mid_kernel(Q8Args a) {
   const int l16 = lane & 15, kq = lane >> 4;
   const int wm = wave / C::WN, wn = wave % C::WN;
   const int M = a.M, N = a.N, KB = a.K >> 7;
-  // consecutive workgroups go to the eight XCDs in turn: the row tiles of a column tile take ids of one residue, so
-  // that its weights pass through one L2
-  int tm, tn;
-  if (a.xcds) {
-    const int j = blockIdx.x >> 3;
-    tm = j % a.mtiles;
-    tn = j / a.mtiles * 8 + (blockIdx.x & 7);
-  } else {
-    tm = blockIdx.x % a.mtiles;
-    tn = blockIdx.x / a.mtiles;
-  }
+  // Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles, ordered by column, so that the
+  // row tiles of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
+  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
+  const int t = x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
+  const int tn = t / a.mtiles, tm = t - tn * a.mtiles;
   const int m0 = tm * C::BM, n0 = tn * C::BN;
   const int kb0 = blockIdx.y * a.kper, nk = min(KB - kb0, a.kper);
   const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)lds);
@@ -282,6 +275,198 @@ q8_mid_kernel(Q8Args a) {
   }
 }
 
+// ---- 48 .. 128 rows x 128 columns with wavefronts of their own for the copies ---------------------------------------------
+// Larger tiles copy fewer bytes per product, and there the address path (16 clocks and more per KiB) and the matrix pipe are
+// both busy enough that a wavefront must not wait for one to feed the other: per K range (two, whose sums meet in LDS) four
+// wavefronts multiply, each all rows of its 32 columns, and two copy.
+// (us, eight wavefronts that do both on 128 x 128 or four on 64 x 64 -> here; fp8 block 7168 x 4096 at 512 rows 31.4 -> 26.9,
+// 8192 x 8192 at 256 / 512 40.8 / 61.9 -> 33.6 / 52.5, 4096 x 6144 at 256 / 512 19.6 / 31.1 -> 16.3 / 24.7; int8 7168 x 4096 at 512
+// 31.5 -> 25.0, 14336 x 4096 at 256 36.0 -> 30.6)
+__device__ __forceinline__ void q8_copy16(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr), "s"(more) : "memory", "scc");
+}
+template <int OFF>
+__device__ __forceinline__ void q8_copy16_next(uint32_t voff, const void* sbase) {   // the same m0; the offset counts on both sides
+  asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
+}
+__device__ __forceinline__ void q8_copy4(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr), "s"(more) : "memory", "scc");
+}
+
+// 16 NJ rows x 128 columns
+template <int NJ_, bool BLOCK>
+struct Q8Wide {
+  static constexpr int NJ = NJ_, NI = 2, KS = 2, NW = 4, CW = KS * NW, THREADS = 64 * (CW + 2 * KS);
+  static constexpr int BM = 16 * NJ, BN = 64 * NI, SC = BLOCK ? (BM + 63) / 64 : 0;
+  static constexpr int X_BYTES = BM * 128, W_BYTES = BN * 128, S_OFF = X_BYTES + W_BYTES, STAGE = S_OFF + (BLOCK ? 256 * SC + 256 : 0);
+  static constexpr int NC = NJ + 4 * NI + SC;         // copies of a copying wavefront per stage
+  static constexpr int D = 159 * 1024 / (KS * STAGE), RING = D * STAGE;
+  static_assert((D - 1) * NC < 64 && D >= 2, "a ring, and copies in flight that the wait can count");
+};
+
+template <int MODE, int DT, typename C>
+__global__ void __launch_bounds__(C::THREADS, C::THREADS / 256)
+q8_wide_kernel(Q8Args a) {
+  constexpr int NJ = C::NJ, NI = C::NI, D = C::D, NW = C::NW;
+  typedef typename std::conditional<MODE == Q8_INT8, i4, f4>::type acc_t;
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool copies = wg >= C::CW;
+  const int wave = copies ? (wg - C::CW) % 2 : wg % NW, ks = copies ? (wg - C::CW) / 2 : wg / NW;
+  const int l16 = lane & 15, kq = lane >> 4;
+  const int M = a.M, N = a.N, KB = a.K >> 7;
+  // Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles, ordered by column, so that the
+  // row tiles of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
+  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
+  const int t = x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
+  const int tn = t / a.mtiles, tm = t - tn * a.mtiles;
+  const int m0 = tm * C::BM, n0 = tn * C::BN;
+  const int g0 = (int)blockIdx.y * a.kper, ng = min(KB - g0, a.kper);
+  const int nk = (ng + 1) / 2, mine = min(ng - ks * nk, nk);
+
+  acc_t acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = (acc_t){0, 0, 0, 0};
+
+  if (copies) {
+    uint32_t xo[NJ];
+#pragma unroll
+    for (int p = 0; p < NJ; ++p) {
+      const int r = (wave + 2 * p) * 8 + (lane >> 3);
+      xo[p] = (uint32_t)(min(m0 + r, M - 1) - m0) * (uint32_t)a.ldx + 16u * (uint32_t)((lane & 7) ^ (r & 7));
+    }
+    const uint32_t lane16 = (uint32_t)lane * 16u;
+    int kb = min(g0 + ks * nk, KB - 1);
+    const int klast = max(g0 + ks * nk + mine - 1, kb);
+    const uint8_t* xg = a.x + (long)m0 * a.ldx + (long)kb * 128;
+    const uint8_t* wgp = a.w + ((long)(n0 >> 6) * KB + kb) * 8192 + wave * 4096;
+    uint32_t so[C::SC ? C::SC : 1];
+    const float* sg = nullptr;
+    if (MODE == Q8_BLOCK) {
+#pragma unroll
+      for (int p = 0; p < C::SC; ++p) so[p] = wave == 0 ? (uint32_t)(min(m0 + 64 * p + lane, M - 1) - m0) * (uint32_t)KB * 4u : 0u;
+      sg = (wave == 0 ? a.x_scale + (long)m0 * KB : a.w_scale + (long)(n0 >> 7) * KB) + kb;
+    }
+    const uint32_t ring = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)lds) + ks * C::RING;
+    auto copy_stage = [&](int slot) {
+      const uint32_t sb = ring + (uint32_t)(slot * C::STAGE);
+#pragma unroll
+      for (int g = 0; g < NI; ++g) {
+        q8_copy16(lane16, wgp + (long)g * KB * 8192, sb, (uint32_t)(C::X_BYTES + g * 8192 + wave * 4096));
+        q8_copy16_next<1024>(lane16, wgp + (long)g * KB * 8192);
+        q8_copy16_next<2048>(lane16, wgp + (long)g * KB * 8192);
+        q8_copy16_next<3072>(lane16, wgp + (long)g * KB * 8192);
+      }
+#pragma unroll
+      for (int p = 0; p < NJ; ++p) q8_copy16(xo[p], xg, sb, (uint32_t)((wave + 2 * p) * 1024));
+      if constexpr (MODE == Q8_BLOCK) {
+#pragma unroll
+        for (int p = 0; p < C::SC; ++p) q8_copy4(so[p], sg, sb, (uint32_t)(C::S_OFF + (wave == 0 ? 256 * p : 256 * C::SC)));
+      }
+      if (kb < klast) {
+        ++kb;
+        xg += 128;
+        wgp += 8192;
+        if (MODE == Q8_BLOCK) ++sg;
+      }
+    };
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) copy_stage(d);
+    int slot = 0;
+    for (int i = 0; i < nk; ++i) {
+      asm volatile("s_waitcnt vmcnt(%0)" : : "n"((D - 2) * C::NC) : "memory");
+      __builtin_amdgcn_s_barrier();
+      copy_stage(slot == 0 ? D - 1 : slot - 1);
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+  } else {
+    uint32_t xa[2], wa[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int c = 4 * h + kq;
+      xa[h] = (uint32_t)(l16 * 128 + ((c ^ (l16 & 7)) * 16));
+      wa[h] = (uint32_t)(C::X_BYTES + wave * NI * 2048 + (c & 1) * 1024 + ((c >> 1) * 16 + l16) * 16);
+    }
+    int slot = 0;
+    for (int i = 0; i < nk; ++i) {
+      asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" : : : "memory");
+      if (i < mine) {
+        const unsigned char* st = lds + ks * C::RING + slot * C::STAGE;
+        i4 w[NI][2], x[NJ][2];
+        float xs[NJ], wsc = 1.0f;
+#pragma unroll
+        for (int t = 0; t < NI; ++t) {
+          w[t][0] = *(const i4*)(st + wa[0] + t * 2048);
+          w[t][1] = *(const i4*)(st + wa[1] + t * 2048);
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          x[j][0] = *(const i4*)(st + xa[0] + j * 2048);
+          x[j][1] = *(const i4*)(st + xa[1] + j * 2048);
+        }
+        if constexpr (MODE == Q8_BLOCK) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) xs[j] = *(const float*)(st + C::S_OFF + (16 * j + l16) * 4);
+          wsc = *(const float*)(st + C::S_OFF + 256 * C::SC);
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int t = 0; t < NI; ++t) {
+            if constexpr (MODE == Q8_INT8) {
+              acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[t][0], x[j][0], acc[t][j], 0, 0, 0);
+              acc[t][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w[t][1], x[j][1], acc[t][j], 0, 0, 0);
+            } else {
+              const i8v av = __builtin_shufflevector(w[t][0], w[t][1], 0, 1, 2, 3, 4, 5, 6, 7);
+              const i8v bv = __builtin_shufflevector(x[j][0], x[j][1], 0, 1, 2, 3, 4, 5, 6, 7);
+              if constexpr (MODE == Q8_PC) {
+                acc[t][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[t][j], 0, 0, 0, 0, 0, 0);
+              } else {
+                const f4 part = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, (f4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+                acc[t][j] += (xs[j] * wsc) * part;
+              }
+            }
+          }
+      }
+      slot = slot + 1 == D ? 0 : slot + 1;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+  }
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
+  // the two ranges' sums: each finishes half of the row tiles
+  constexpr int H = (NJ + 1) / 2;
+  static_assert(C::KS * NW * NI * H * 1024 <= C::KS * C::RING, "the exchange fits in the ring");
+  if (!copies) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      if ((j < H) != (ks == 0)) {
+#pragma unroll
+        for (int t = 0; t < NI; ++t) *(acc_t*)(lds + (((ks * NW + wave) * NI + t) * H + (j < H ? j : j - H)) * 1024 + lane * 16) = acc[t][j];
+      }
+  }
+  __syncthreads();
+  if (copies) return;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    if ((j < H) != (ks == 0)) continue;
+    const int m = m0 + j * 16 + l16;
+    if (m >= M) continue;
+#pragma unroll
+    for (int t = 0; t < NI; ++t) {
+      const acc_t sum = acc[t][j] + *(const acc_t*)(lds + ((((1 - ks) * NW + wave) * NI + t) * H + (j < H ? j : j - H)) * 1024 + lane * 16);
+      const int n = n0 + (wave * NI + t) * 16 + 4 * kq;
+      if (a.partial) *(acc_t*)((acc_t*)a.partial + (((long)blockIdx.y * M + m) * N + n) / 4) = sum;
+      else q8_finish<MODE, DT>(a, m, n, sum);
+    }
+  }
+}
+
 // second launch of a split: the ranges' sums in range order, then the epilogue
 template <int MODE, int DT>
 __global__ void __launch_bounds__(256)
@@ -297,9 +482,16 @@ q8_splitk_epilogue_kernel(Q8Args a, int splits, FastDiv quads) {
   q8_finish<MODE, DT>(a, (int)m, (int)nq * 4, s);
 }
 
+template <int MODE, int DT>
+int launch_q8_epilogue(const Q8Args& a, int splits, hipStream_t st) {
+  const FastDiv quads((uint32_t)(a.N / 4));
+  hipLaunchKernelGGL((q8_splitk_epilogue_kernel<MODE, DT>), dim3((unsigned)(((size_t)a.M * quads.d + 255) / 256)), dim3(256), 0, st, a, splits, quads);
+  MQ_LAUNCH_CHECK("q8 gemm (split-K epilogue)");
+  return 0;
+}
+
 typedef Q8Cfg<1, 4, 2, 1, 4> Q8T32;      // 32 x 64, 48 KiB of stages
 typedef Q8Cfg<2, 2, 2, 2, 4> Q8T64;      // 64 x 64, 64 KiB
-typedef Q8Cfg<2, 4, 4, 2, 4> Q8T128;     // 128 x 128, 128 KiB
 
 template <int MODE, typename C>
 size_t q8_lds(int kper) {
@@ -312,7 +504,6 @@ template <int MODE, int DT, typename C>
 int launch_q8(Q8Args a, int splits, hipStream_t st) {
   const int KB = a.K / 128;
   a.mtiles = (a.M + C::BM - 1) / C::BM;
-  a.xcds = (a.N / C::BN) % 8 == 0;
   a.kper = (KB + splits - 1) / splits;
   splits = (KB + a.kper - 1) / a.kper;                // no empty ranges
   if (splits <= 1) a.partial = nullptr;
@@ -322,45 +513,67 @@ int launch_q8(Q8Args a, int splits, hipStream_t st) {
   MQ_REQUIRE(attr == hipSuccess, "q8 gemm: cannot reserve LDS: %s", hipGetErrorString(attr));
   hipLaunchKernelGGL((q8_mid_kernel<MODE, DT, C>), dim3((unsigned)(a.mtiles * (a.N / C::BN)), (unsigned)splits), dim3(C::THREADS), shmem, st, a);
   MQ_LAUNCH_CHECK("q8 gemm");
-  if (splits > 1) {
-    const FastDiv quads((uint32_t)(a.N / 4));
-    hipLaunchKernelGGL((q8_splitk_epilogue_kernel<MODE, DT>), dim3((unsigned)(((size_t)a.M * quads.d + 255) / 256)), dim3(256), 0, st, a, splits, quads);
-    MQ_LAUNCH_CHECK("q8 gemm (split-K epilogue)");
-  }
-  return 0;
+  return splits > 1 ? launch_q8_epilogue<MODE, DT>(a, splits, st) : 0;
+}
+
+template <int MODE, int DT, int NJ>
+int launch_q8_wide(Q8Args a, int splits, hipStream_t st) {
+  typedef Q8Wide<NJ, MODE == Q8_BLOCK> C;
+  const int KB = a.K / 128;
+  a.mtiles = (a.M + C::BM - 1) / C::BM;
+  a.kper = (KB + splits - 1) / splits;
+  splits = (KB + a.kper - 1) / a.kper;                // no empty ranges
+  if (splits <= 1) a.partial = nullptr;
+  const size_t shmem = (size_t)C::KS * C::RING;
+  static hipError_t attr = hipFuncSetAttribute((const void*)q8_wide_kernel<MODE, DT, C>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+  MQ_REQUIRE(attr == hipSuccess, "q8 gemm: cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
+  hipLaunchKernelGGL((q8_wide_kernel<MODE, DT, C>), dim3((unsigned)(a.mtiles * (a.N / C::BN)), (unsigned)splits), dim3(C::THREADS), shmem, st, a);
+  MQ_LAUNCH_CHECK("q8 gemm");
+  return splits > 1 ? launch_q8_epilogue<MODE, DT>(a, splits, st) : 0;
 }
 
 template <int MODE, int DT>
-int launch_q8_tile(const Q8Args& a, int bm, int splits, hipStream_t st) {
-  if (bm == 32) return launch_q8<MODE, DT, Q8T32>(a, splits, st);
-  if (bm == 64) return launch_q8<MODE, DT, Q8T64>(a, splits, st);
-  return launch_q8<MODE, DT, Q8T128>(a, splits, st);
+int launch_q8_tile(const Q8Args& a, int tile, int splits, hipStream_t st) {
+  switch (tile) {
+    case 0: return launch_q8<MODE, DT, Q8T32>(a, splits, st);
+    case 1: return launch_q8<MODE, DT, Q8T64>(a, splits, st);
+    case 2: return launch_q8_wide<MODE, DT, 3>(a, splits, st);
+    case 3: return launch_q8_wide<MODE, DT, 4>(a, splits, st);
+    case 4: return launch_q8_wide<MODE, DT, 6>(a, splits, st);
+    default: return launch_q8_wide<MODE, DT, 8>(a, splits, st);
+  }
 }
 
 // ---- which tile, how many K ranges, or which other kernel ---------------------------------------------------
-// Prices in us, fitted on MI355X to 13,000 launches: fourteen layers from 1024 x 1024 to 8192 x 28672, 8 .. 1536 rows,
-// every tile and 1 .. 16 K ranges, weights rotated past the last-level cache.  A round of workgroups pays a step per K
-// block, more of it for every workgroup that shares the CU; the weight stream is a floor; a split pays for its second
-// launch and for the bytes of its partial sums.  The pick is within 2 % of the best launch on average.
-struct Q8Price {
-  double base, split, split_mn;            // launch and ramp; second launch; per million partial sums
-  double one[3], more[3];                  // step of one workgroup per CU, of each further one (tiles of 32, 64, 128 rows)
+// Prices in us, fitted on MI355X to 16,000 launches: twelve layers from 1024 x 3072 to 4096 x 28672, 20 .. 1536 rows,
+// every tile and 1 .. 12 K ranges, weights rotated past the last-level cache.  A round of workgroups pays a step per K
+// block (the wide tiles: per two), more of it for every workgroup that shares the CU and less on an empty chip; the weight
+// stream is a floor; a split pays for its second launch and for the bytes of its partial sums.  The pick is within 1.5 % of
+// the best launch on average.
+struct Q8Tile {
+  int bm, bn;
 };
-constexpr Q8Price kBlockPrice = {3.1, 2.3, 1.29, {0.200, 0.294, 0.973}, {0.185, 0.240, 0.474}};
-constexpr Q8Price kPlainPrice = {3.4, 1.6, 1.55, {0.151, 0.232, 0.961}, {0.200, 0.260, 0.190}};
+constexpr Q8Tile kTiles[6] = {{32, 64}, {64, 64}, {48, 128}, {64, 128}, {96, 128}, {128, 128}};
+struct Q8Price {
+  double base, wide, split, split_mn;      // launch and ramp; more of it for the wide tiles; second launch; per million partial sums
+  double stream, alone, round;             // bytes of weights per us; share of a step that an empty chip saves; per further round
+  double one[6], more[2];                  // step of one workgroup per CU; of each further one (the tiles of 64 columns)
+};
+constexpr Q8Price kBlockPrice = {2.74, 0.56, 1.96, 1.50, 4.83e6, 0.22, 1.47, {0.237, 0.313, 0.699, 0.795, 1.208, 1.364}, {0.096, 0.132}};
+constexpr Q8Price kPlainPrice = {3.16, 1.29, 1.60, 1.31, 4.88e6, 0.22, 2.08, {0.174, 0.249, 0.624, 0.731, 1.142, 1.307}, {0.127, 0.189}};
 // the 256-row tile kernels: base, step per K block of a round of 256 x 128 tiles, second launch, per million partial sums
 struct TilePrice {
   double base, step, split, split_mn;
 };
-constexpr TilePrice kTilePrice[3] = {{6.5, 0.95, 4.0, 1.61}, {2.6, 0.881, 4.3, 1.70}, {7.2, 0.776, 0.9, 1.83}};
+constexpr TilePrice kTilePrice[3] = {{4.95, 0.991, 0.8, 1.76}, {5.41, 0.825, 1.4, 1.89}, {8.06, 0.729, 0, 2.00}};
 
-double with_stream(double t, double K, double N) {      // never faster than the weights arrive
-  const double h = K * N / 5.05e6;
+double with_stream(double t, double K, double N, double rate) {      // never faster than the weights arrive
+  const double h = K * N / rate;
   return std::sqrt(std::sqrt(t * t * t * t + h * h * h * h));
 }
 
 struct Q8Plan {
-  int bm, splits;                          // bm 0: another kernel is ahead
+  int tile, splits;                        // tile -1: another kernel is ahead
   size_t bytes;                            // partial sums
 };
 
@@ -378,12 +591,12 @@ double tile_kernel_price(int mode, int M, int N, int K) {
   }
   double t = p.base + rounds * p.step * nk / splits;
   if (splits > 1) t += p.split + p.split_mn * 1e-6 * splits * M * N;
-  return with_stream(t, K, N);
+  return with_stream(t, K, N, 5.0e6);
 }
 
 Q8Plan q8_make_plan(int mode, int M, int N, int K) {
-  Q8Plan best = {0, 1, 0};
-  if (M <= 16 || K % 128 != 0 || N % 64 != 0 || (mode == Q8_BLOCK && N % 128 != 0)) return best;
+  Q8Plan best = {-1, 1, 0};
+  if (M <= 16 || M > 1536 || K % 128 != 0 || N % 64 != 0 || (mode == Q8_BLOCK && N % 128 != 0)) return best;
   // The weight streamer stays ahead up to 16 rows, and up to 32 where the weights are large enough for HBM alone to set
   // the pace (us at 32 rows, streamer / here: 8192 x 8192 15.4 / 17.0, 8192 x 28672 44.2 / 48.1, 5120 x 13824 16.2 / 15.4; but
   // 14336 x 4096 19.7 / 15.1, 7168 x 4096 11.4 / 10.9, 3584 x 4608 11.5 / 7.4).
@@ -392,31 +605,36 @@ Q8Plan q8_make_plan(int mode, int M, int N, int K) {
   const int KB = K / 128;
   const long cus = device_cu_count();
   double least = 1e30;
-  for (int c = 0; c < 3; ++c) {
-    const int bm = 32 << c, bn = c == 2 ? 128 : 64;
-    if (N % bn != 0 || (c > 0 && M <= bm / 2)) continue;
+  for (int c = 0; c < 6; ++c) {
+    const int bm = kTiles[c].bm, bn = kTiles[c].bn;
+    const bool wide = c >= 2;
+    if (N % bn != 0 || (c > 0 && M <= (bm > 64 ? bm - 32 : bm - 16))) continue;
     for (int s = 1; s <= 16; ++s) {
       const int kper = (KB + s - 1) / s, ranges = (KB + kper - 1) / kper;
       if (ranges != s || (s > 1 && kper < 8)) continue;
       const size_t bytes = s > 1 ? (size_t)s * M * N * 4 : 0;
       if (bytes > ((size_t)64 << 20)) continue;
-      size_t lds = c == 0 ? q8_lds<Q8_PC, Q8T32>(kper) : c == 1 ? q8_lds<Q8_PC, Q8T64>(kper) : q8_lds<Q8_PC, Q8T128>(kper);
-      if (mode == Q8_BLOCK) lds = c == 0 ? q8_lds<Q8_BLOCK, Q8T32>(kper) : c == 1 ? q8_lds<Q8_BLOCK, Q8T64>(kper) : q8_lds<Q8_BLOCK, Q8T128>(kper);
-      if (lds > 160 * 1024) continue;
-      const long res = std::min<long>(160 * 1024 / lds, 3);
+      long res = 1;
+      if (!wide) {
+        size_t lds = c == 0 ? q8_lds<Q8_PC, Q8T32>(kper) : q8_lds<Q8_PC, Q8T64>(kper);
+        if (mode == Q8_BLOCK) lds = c == 0 ? q8_lds<Q8_BLOCK, Q8T32>(kper) : q8_lds<Q8_BLOCK, Q8T64>(kper);
+        if (lds > 160 * 1024) continue;
+        res = std::min<long>(160 * 1024 / lds, 3);
+      }
       const long wgs = (long)((M + bm - 1) / bm) * (N / bn) * s, full = wgs / (res * cus), rest = wgs % (res * cus);
-      double steps = full * (p.one[c] + p.more[c] * (res - 1));
-      if (rest) steps += p.one[c] + p.more[c] * ((rest + cus - 1) / cus - 1);
-      double t = with_stream(steps * kper, K, N) + p.base;
+      const double more = wide ? 0 : p.more[c];
+      double steps = full * (p.one[c] + more * (res - 1));
+      if (rest) steps += p.one[c] * (1 - p.alone * (1 - (double)std::min(rest, cus) / cus)) + more * ((rest + cus - 1) / cus - 1);
+      double t = with_stream(steps * (wide ? (kper + 1) / 2 : kper), K, N, p.stream) + p.base + (wide ? p.wide : 0) + p.round * (full + (rest > 0) - 1);
       if (s > 1) t += p.split + p.split_mn * 1e-6 * s * M * N;
       if (t < least) {
         least = t;
-        best = {bm, s, bytes};
+        best = {c, s, bytes};
       }
     }
   }
   // the 256-row tiles from 65 rows on (below, half of their wavefronts and more have no rows)
-  if (best.bm && M > 64 && N % 128 == 0 && tile_kernel_price(mode, M, N, K) < 1.02 * least) best.bm = 0;
+  if (best.tile >= 0 && M > 64 && N % 128 == 0 && tile_kernel_price(mode, M, N, K) < 1.04 * least) best.tile = -1;
   return best;
 }
 
@@ -440,7 +658,7 @@ Q8Plan q8_plan(int mode, int M, int N, int K) {
 bool q8_mid_wanted(int mode, int M, int N, int K, size_t* bytes) {
   const Q8Plan p = q8_plan(mode, M, N, K);
   *bytes = p.bytes;
-  return p.bm != 0;
+  return p.tile >= 0;
 }
 
 // x_scale / w_scale: block scales (mode 0), or vectors / one value by their index multipliers (0: one value), null = 1 (int8)
@@ -448,16 +666,16 @@ int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float
                   int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* partial,
                   hipStream_t st) {
   const Q8Plan p = q8_plan(mode, M, N, K);
-  MQ_REQUIRE(p.bm && (p.splits == 1 || partial), "q8 gemm: no plan for M=%d N=%d K=%d", M, N, K);
+  MQ_REQUIRE(p.tile >= 0 && (p.splits == 1 || partial), "q8 gemm: no plan for M=%d N=%d K=%d", M, N, K);
   Q8Args a = {};
   a.out = out; a.x = (const uint8_t*)x; a.w = (const uint8_t*)w; a.x_scale = x_scale; a.w_scale = w_scale; a.bias = bias;
   a.xs_mul = xs_mul; a.ws_mul = ws_mul; a.bias_f32 = bias_f32;
   a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldo = ldo; a.partial = partial;
 #define MQ_Q8(MODE)                                                                                       \
   do {                                                                                                    \
-    if (out_dtype == MI355Q_F16) return launch_q8_tile<MODE, MI355Q_F16>(a, p.bm, p.splits, st);          \
-    if (out_dtype == MI355Q_BF16) return launch_q8_tile<MODE, MI355Q_BF16>(a, p.bm, p.splits, st);        \
-    if constexpr (MODE == Q8_INT8) return launch_q8_tile<MODE, MI355Q_F32>(a, p.bm, p.splits, st);        \
+    if (out_dtype == MI355Q_F16) return launch_q8_tile<MODE, MI355Q_F16>(a, p.tile, p.splits, st);          \
+    if (out_dtype == MI355Q_BF16) return launch_q8_tile<MODE, MI355Q_BF16>(a, p.tile, p.splits, st);        \
+    if constexpr (MODE == Q8_INT8) return launch_q8_tile<MODE, MI355Q_F32>(a, p.tile, p.splits, st);        \
     MQ_REQUIRE(false, "q8 gemm: bad out dtype %d", out_dtype);                                            \
   } while (0)
   if (mode == Q8_BLOCK) MQ_Q8(Q8_BLOCK);

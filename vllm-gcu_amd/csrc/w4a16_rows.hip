@@ -45,7 +45,7 @@ struct RowsArgs {
   int M, K, N;
   int kper;                   // K blocks per range (blockIdx.y)
   uint32_t gpk_magic;         // ceil(2^32 / K blocks per group), 0: a group is one K block or less
-  int mtiles, xcds;
+  int mtiles;
   float* partial;             // split K: f32 tiles [range][M][N]; null: write the output
 };
 
@@ -125,15 +125,11 @@ w4a16_rows_kernel(RowsArgs a) {
   const int wave = copies ? (wg - C::CW) % 2 : wg % NW, ks = copies ? (wg - C::CW) / 2 : wg / NW;
   const int c = lane & 15, kq = lane >> 4;
   const int M = a.M, N = a.N, K = a.K, G = K >> 7;
-  int tm, tn;
-  if (a.xcds) {                                       // the row tiles of a column tile on one XCD: its weights pass one L2
-    const int j = blockIdx.x >> 3;
-    tm = j % a.mtiles;
-    tn = j / a.mtiles * 8 + (blockIdx.x & 7);
-  } else {
-    tm = blockIdx.x % a.mtiles;
-    tn = blockIdx.x / a.mtiles;
-  }
+  // Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles, ordered by column, so that the
+  // row tiles of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
+  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
+  const int t = x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
+  const int tn = t / a.mtiles, tm = t - tn * a.mtiles;
   const int m0 = tm * C::BM;
   const int slab = tn * NW * NT >> 3, t0 = tn * NW * NT & 7;           // 128-column slab, first of the workgroup's 16-column tiles in it
   const int g0 = (int)blockIdx.y * a.kper, ng = min(G - g0, a.kper);   // K blocks of the workgroup
@@ -316,7 +312,6 @@ template <int DT, int ZK, typename C>
 int launch_rows(RowsArgs a, int splits, const void* bias, int dtype, hipStream_t st) {
   const int G = a.K / 128;
   a.mtiles = (a.M + C::BM - 1) / C::BM;
-  a.xcds = (a.N / C::BN) % 8 == 0;
   a.kper = (G + splits - 1) / splits;
   splits = (G + a.kper - 1) / a.kper;                 // no empty ranges
   if (splits <= 1) a.partial = nullptr;
@@ -346,12 +341,12 @@ struct RowsPrice {
   int mt, nt;
   double one, more;
 };
-constexpr RowsPrice kRows[] = {{2, 1, 0.419, 0.398}, {3, 1, 0.589, 0.480}, {4, 1, 0.716, 0}, {2, 2, 0.789, 0.578},
-                               {3, 2, 0.961, 0},     {4, 2, 1.147, 0},     {5, 2, 1.307, 0}, {6, 2, 1.520, 0}};
-constexpr double kRowsBase = 3.77, kRowsRound = 1.37, kRowsSplit = 2.36, kRowsSplitMN = 1.41;
+constexpr RowsPrice kRows[] = {{2, 1, 0.422, 0.388}, {3, 1, 0.600, 0.500}, {4, 1, 0.700, 0}, {2, 2, 0.773, 0.594},
+                               {3, 2, 0.956, 0},     {4, 2, 1.173, 0},     {5, 2, 1.333, 0}, {6, 2, 1.555, 0}};
+constexpr double kRowsBase = 3.57, kRowsRound = 1.10, kRowsSplit = 2.18, kRowsSplitMN = 1.56;
 constexpr double kRowsAlone = 0.283;        // share of a step that goes away as the chip empties (the caches and memory are shared)
-constexpr double kRowsSecond = 0.345;       // share of the second workgroup's price that grows with how many CUs hold two
-constexpr double kRowsStream = 4.12e6;      // bytes of weights per microsecond
+constexpr double kRowsSecond = 0.388;       // share of the second workgroup's price that grows with how many CUs hold two
+constexpr double kRowsStream = 4.23e6;      // bytes of weights per microsecond
 
 struct RowsPlan {
   int mt, nt, splits;
