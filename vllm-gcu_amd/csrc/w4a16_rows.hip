@@ -47,6 +47,13 @@ struct RowsArgs {
   uint32_t gpk_magic;         // ceil(2^32 / K blocks per group), 0: a group is one K block or less
   int mtiles;
   float* partial;             // split K: f32 tiles [range][M][N]; null: write the output
+  // grouped (fused-MoE) launches: blockIdx.y = block of sorted token slots, all of one expert
+  const int32_t* sorted_ids;    // slot ids, pads >= numel
+  const int32_t* expert_ids;    // [blocks]
+  const int32_t* npp;           // device scalar: slots after padding
+  const float* topk_weights;    // [numel] or null
+  int numel, topk, E, block;
+  long w_stride, s_stride, z_stride;   // bytes per expert
 };
 
 __device__ __forceinline__ void rows_dma16(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
@@ -112,9 +119,10 @@ struct RowsCfg {
   static_assert((D - 1) * NC < 64, "copies in flight that the wait can count");
 };
 
-template <int DT, int ZK, typename C>
-__global__ void __launch_bounds__(C::THREADS, (C::PAIR + 1) * C::THREADS / 256)
-w4a16_rows_kernel(RowsArgs a) {
+// The tile of rows m0 .. and column tile tn over K blocks g0 .. g0 + ng - 1.  GROUPED: rows are the slots ids[0 ..] of one
+// expert, gathered from row id / topk of x and stored to row id of the output, times the slot's routing weight.
+template <int DT, int ZK, typename C, bool GROUPED>
+__device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids, int m0, int tn, int g0, int ng) {
   typedef RowsMma<DT> MM;
   constexpr int MT = C::MT, NW = C::NW, NT = C::NT, KS = C::KS, GPB = C::GPB, D = C::D, STAGE = C::STAGE;
   // A operands one K step ahead where the registers are there (else the compiler places the reads, and spills nothing)
@@ -125,14 +133,7 @@ w4a16_rows_kernel(RowsArgs a) {
   const int wave = copies ? (wg - C::CW) % 2 : wg % NW, ks = copies ? (wg - C::CW) / 2 : wg / NW;
   const int c = lane & 15, kq = lane >> 4;
   const int M = a.M, N = a.N, K = a.K, G = K >> 7;
-  // Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles, ordered by column, so that the
-  // row tiles of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
-  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
-  const int t = x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
-  const int tn = t / a.mtiles, tm = t - tn * a.mtiles;
-  const int m0 = tm * C::BM;
   const int slab = tn * NW * NT >> 3, t0 = tn * NW * NT & 7;           // 128-column slab, first of the workgroup's 16-column tiles in it
-  const int g0 = (int)blockIdx.y * a.kper, ng = min(G - g0, a.kper);   // K blocks of the workgroup
   const int nk = (ng + KS - 1) / KS;                  // ... of each of its ranges (the last may hold fewer, even none)
   const int mine = min(ng - ks * nk, nk);
 
@@ -148,7 +149,8 @@ w4a16_rows_kernel(RowsArgs a) {
 #pragma unroll
     for (int p = 0; p < C::XC; ++p) {
       const int r = 4 * (wave + 2 * p) + (lane >> 4);
-      xo[p] = ((uint32_t)min(m0 + r, M - 1) * (uint32_t)K + 8u * (uint32_t)((lane & 15) ^ (r & 15))) * 2u;
+      const int row = GROUPED ? min(ids[r], a.numel - 1) / a.topk : min(m0 + r, M - 1);   // (pads read a valid row)
+      xo[p] = ((uint32_t)row * (uint32_t)K + 8u * (uint32_t)((lane & 15) ^ (r & 15))) * 2u;
     }
     const uint32_t lane16 = (uint32_t)lane * 16u;
     int kb = min(g0 + ks * nk, G - 1);                // the K block that the next copies are of
@@ -286,25 +288,68 @@ w4a16_rows_kernel(RowsArgs a) {
   constexpr int TPR = C::BN / 4;                      // threads per row
   const int q = tid % TPR, n = 128 * slab + 8 * (q / Q) + t0 + 4 * (q % Q);
   float bs[4] = {0.f, 0.f, 0.f, 0.f};
-  if (a.bias && !a.partial) {
+  if (!GROUPED && a.bias && !a.partial) {
     const uint2 bw = *(const uint2*)(a.bias + n);
     bs[0] = Elem<DT>::to_f32((uint16_t)(bw.x & 0xffffu)); bs[1] = Elem<DT>::to_f32((uint16_t)(bw.x >> 16));
     bs[2] = Elem<DT>::to_f32((uint16_t)(bw.y & 0xffffu)); bs[3] = Elem<DT>::to_f32((uint16_t)(bw.y >> 16));
   }
   for (int r = tid / TPR; r < C::BM; r += C::THREADS / TPR) {
-    const int m = m0 + r;
-    if (m >= M) break;
+    const int m = GROUPED ? ids[r] : m0 + r;
+    if (m >= (GROUPED ? a.numel : M)) {
+      if (GROUPED) continue;
+      break;
+    }
     f4 v = *(const f4*)(lds + r * EP + q * 16);
 #pragma unroll
     for (int k = 1; k < KS; ++k) v += *(const f4*)(lds + k * C::RING + r * EP + q * 16);
-    if (a.partial) {
+    if (!GROUPED && a.partial) {
       *(f4*)(a.partial + ((size_t)blockIdx.y * M + m) * N + n) = v;
     } else {
+      if (GROUPED && a.topk_weights) v *= a.topk_weights[m];
       uint2 o;
       o.x = (uint32_t)Elem<DT>::from_f32(v[0] + bs[0]) | ((uint32_t)Elem<DT>::from_f32(v[1] + bs[1]) << 16);
       o.y = (uint32_t)Elem<DT>::from_f32(v[2] + bs[2]) | ((uint32_t)Elem<DT>::from_f32(v[3] + bs[3]) << 16);
       *(uint2*)(a.out + (size_t)m * N + n) = o;
     }
+  }
+}
+
+template <int DT, int ZK, typename C>
+__global__ void __launch_bounds__(C::THREADS, (C::PAIR + 1) * C::THREADS / 256)
+w4a16_rows_kernel(RowsArgs a) {
+  // Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles, ordered by column, so that the
+  // row tiles of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
+  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
+  const int t = x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
+  const int tn = t / a.mtiles, tm = t - tn * a.mtiles;
+  const int g0 = (int)blockIdx.y * a.kper;
+  rows_tile<DT, ZK, C, false>(a, nullptr, tm * C::BM, tn, g0, min((a.K >> 7) - g0, a.kper));
+}
+
+// Blocks of up to 16 MAX slots: a block takes the tile of as many row tiles as hold real slots (they come first)
+template <int DT, int ZK, int GPB, int MAX>
+__global__ void __launch_bounds__(768, (RowsCfg<MAX, 2, GPB, ZK>::PAIR + 1) * 3)
+w4a16_rows_grouped_kernel(RowsArgs a) {
+  const int base = blockIdx.y * a.block;
+  if (base >= *a.npp) return;                         // block beyond the padded ids
+  const int32_t* const ids = a.sorted_ids + base;
+  const int lane = threadIdx.x & 63, tn = blockIdx.x;
+  const unsigned long long real = __ballot(lane < a.block && ids[min(lane, a.block - 1)] < a.numel);
+  if (!real) return;                                  // pads only
+  const long e = a.expert_ids[blockIdx.y];
+  if (e < 0 || e >= a.E) {                            // not one of this rank's experts: zero rows, no weights read
+    zero_block_columns(a.out, ids, a.block, a.numel, a.N, tn * 128, 128, 768);
+    return;
+  }
+  a.qw = (const u4*)((const char*)a.qw + e * a.w_stride);
+  a.scales = (const uint16_t*)((const char*)a.scales + e * a.s_stride);
+  if (a.zeros) a.zeros += e * a.z_stride;
+  const int tiles = __builtin_amdgcn_readfirstlane((64 - __builtin_clzll(real) + 15) >> 4), G = a.K >> 7;
+  if (tiles == 1) return rows_tile<DT, ZK, RowsCfg<1, 2, GPB, ZK>, true>(a, ids, 0, tn, 0, G);
+  if (MAX == 2 || tiles == 2) return rows_tile<DT, ZK, RowsCfg<2, 2, GPB, ZK>, true>(a, ids, 0, tn, 0, G);
+  if constexpr (MAX > 2) {
+    if (tiles == 3) return rows_tile<DT, ZK, RowsCfg<3, 2, GPB, ZK>, true>(a, ids, 0, tn, 0, G);
+    rows_tile<DT, ZK, RowsCfg<4, 2, GPB, ZK>, true>(a, ids, 0, tn, 0, G);
   }
 }
 
@@ -394,6 +439,19 @@ RowsPlan rows_plan(int M, int K, int N) {
   return e.plan;
 }
 
+template <int DT, int ZK, int GPB, int MAX>
+int launch_rows_grouped(const RowsArgs& a, int max_blocks, hipStream_t st) {
+  size_t shmem = 0;
+  for (size_t b : {(size_t)RowsCfg<1, 2, GPB, ZK>::RING, (size_t)RowsCfg<2, 2, GPB, ZK>::RING, MAX > 2 ? (size_t)RowsCfg<3, 2, GPB, ZK>::RING : 0,
+                   MAX > 2 ? (size_t)RowsCfg<4, 2, GPB, ZK>::RING : 0})
+    shmem = std::max(shmem, 2 * b);
+  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_rows_grouped_kernel<DT, ZK, GPB, MAX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+  MQ_REQUIRE(attr == hipSuccess, "moe_w4a16(rows): cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
+  hipLaunchKernelGGL((w4a16_rows_grouped_kernel<DT, ZK, GPB, MAX>), dim3((unsigned)(a.N / 128), (unsigned)max_blocks), dim3(768), shmem, st, a);
+  MQ_LAUNCH_CHECK("moe_w4a16(rows)");
+  return 0;
+}
+
 }  // namespace
 
 double w4a16_wide_price(int M, int K, int N, bool ring);     // us of the 64-row tiles and (ring) the ring kernels
@@ -462,6 +520,44 @@ int w4a16_rows_launch(void* out, const void* x, const int32_t* qweight, const vo
 #undef MQ_DT
 #undef MQ_ZK
 #undef MQ_GPB
+}
+
+// blocks of 32 or 64 slots of one expert, groups of 64 or multiples of 128
+int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
+                              const float* topk_weights, const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
+                              int numel, int topk, int block_size, int max_blocks, int E, int K, int N, int group_size, int dtype,
+                              hipStream_t st) {
+  MQ_REQUIRE(block_size == 32 || block_size == 64, "moe_w4a16(rows): blocks of 32 or 64 slots, got %d", block_size);
+  MQ_REQUIRE(group_size % 128 == 0 || group_size == 64, "moe_w4a16(rows): group size %d", group_size);
+  RowsArgs a = {};
+  a.out = (uint16_t*)out; a.x = (const uint16_t*)x; a.qw = (const u4*)qweight; a.scales = (const uint16_t*)scales;
+  a.zeros = (const char*)zeros;
+  a.M = numel; a.K = K; a.N = N;
+  const uint32_t gpk = group_size >= 128 ? (uint32_t)group_size / 128u : 1u;
+  a.gpk_magic = gpk > 1 ? (uint32_t)((((uint64_t)1 << 32) + gpk - 1) / gpk) : 0u;
+  a.sorted_ids = sorted_ids; a.expert_ids = expert_ids; a.npp = npp; a.topk_weights = topk_weights;
+  a.numel = numel; a.topk = topk; a.E = E; a.block = block_size;
+  a.w_stride = (long)K * N / 2;
+  a.s_stride = (long)(K / group_size) * N * 2;
+  a.z_stride = zeros_kind == MI355Q_ZP_PACKED ? (long)(K / group_size) * N / 2 : a.s_stride;
+#define MQ_MAX(DT, ZK, GPB)                                                                                               \
+  return block_size == 32 ? launch_rows_grouped<DT, ZK, GPB, 2>(a, max_blocks, st) : launch_rows_grouped<DT, ZK, GPB, 4>(a, max_blocks, st)
+#define MQ_ZK(DT, ZK)                         \
+  do {                                        \
+    if (group_size == 64) MQ_MAX(DT, ZK, 2);  \
+    MQ_MAX(DT, ZK, 1);                        \
+  } while (0)
+#define MQ_DT(DT)                                                          \
+  do {                                                                     \
+    if (zeros_kind == MI355Q_ZP_PACKED) MQ_ZK(DT, MI355Q_ZP_PACKED);       \
+    if (zeros_kind == MI355Q_ZP_PRESCALED) MQ_ZK(DT, MI355Q_ZP_PRESCALED); \
+    MQ_ZK(DT, MI355Q_ZP_NONE);                                             \
+  } while (0)
+  if (dtype == MI355Q_F16) MQ_DT(MI355Q_F16);
+  MQ_DT(MI355Q_BF16);
+#undef MQ_DT
+#undef MQ_ZK
+#undef MQ_MAX
 }
 
 }  // namespace mi355q

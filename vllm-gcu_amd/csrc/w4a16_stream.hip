@@ -671,31 +671,22 @@ int w4a16_stream_launch(void* out, const void* x, const int32_t* qweight, const 
   return 0;
 }
 
-// Fused-MoE grouped GEMM for blocks of 16 or 32 slots (decode-sized token counts): one launch over
+// Fused-MoE grouped GEMM for blocks of 16 slots (decode-sized token counts): one launch over
 // (tile groups, blocks); K is never split, so there is no workspace.
 template <int DT, int ZK>
-static void launch_grouped_nt(const StreamArgs& a, int mt, int nt, int blocks, hipStream_t st) {
+static void launch_grouped_nt(const StreamArgs& a, int nt, int blocks, hipStream_t st) {
   dim3 grid(a.N / 128 * (8 / nt), 1, blocks), block(256);
-#define MQ_GR_LAUNCH(MT, NT) hipLaunchKernelGGL((w4a16_stream_kernel<DT, MT, ZK, 4, NT, true>), grid, block, 0, st, a)
-  if (mt == 1) {
-    if (nt == 8) MQ_GR_LAUNCH(1, 8);
-    else if (nt == 4) MQ_GR_LAUNCH(1, 4);
-    else MQ_GR_LAUNCH(1, 2);
-  } else {
-    if (nt == 8) MQ_GR_LAUNCH(2, 8);
-    else if (nt == 4) MQ_GR_LAUNCH(2, 4);
-    else MQ_GR_LAUNCH(2, 2);
-  }
+#define MQ_GR_LAUNCH(NT) hipLaunchKernelGGL((w4a16_stream_kernel<DT, 1, ZK, 4, NT, true>), grid, block, 0, st, a)
+  if (nt == 8) MQ_GR_LAUNCH(8);
+  else if (nt == 4) MQ_GR_LAUNCH(4);
+  else MQ_GR_LAUNCH(2);
 #undef MQ_GR_LAUNCH
 }
 
 int w4a16_stream_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales,
                                 const void* zeros, int zeros_kind, const float* topk_weights,
                                 const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
-                                int numel, int topk, int block_size, int max_blocks, int E, int K, int N,
-                                int group_size, int dtype, hipStream_t st) {
-  MQ_REQUIRE(block_size == 16 || block_size == 32, "moe_w4a16(stream): blocks of 16 or 32 slots, got %d", block_size);
-  const int mt = block_size / 16;
+                                int numel, int topk, int max_blocks, int E, int K, int N, int group_size, int dtype, hipStream_t st) {
   MQ_REQUIRE(group_size % 128 == 0 && K % 128 == 0 && N % 128 == 0,
              "moe_w4a16(stream): K=%d, N=%d and group_size=%d must be multiples of 128", K, N, group_size);
   const int rows = numel / (topk > 0 ? topk : 1) + 1;
@@ -726,9 +717,9 @@ int w4a16_stream_grouped_launch(void* out, const void* x, const int32_t* qweight
   while (nt > 2 && (long)slabs * (8 / nt) * max_blocks < 2L * cus) nt >>= 1;
 #define MQ_GR_ZK(DT)                                                                          \
   do {                                                                                        \
-    if (zeros_kind == MI355Q_ZP_NONE) launch_grouped_nt<DT, MI355Q_ZP_NONE>(a, mt, nt, max_blocks, st);    \
-    else if (zeros_kind == MI355Q_ZP_PACKED) launch_grouped_nt<DT, MI355Q_ZP_PACKED>(a, mt, nt, max_blocks, st); \
-    else launch_grouped_nt<DT, MI355Q_ZP_PRESCALED>(a, mt, nt, max_blocks, st);               \
+    if (zeros_kind == MI355Q_ZP_NONE) launch_grouped_nt<DT, MI355Q_ZP_NONE>(a, nt, max_blocks, st);    \
+    else if (zeros_kind == MI355Q_ZP_PACKED) launch_grouped_nt<DT, MI355Q_ZP_PACKED>(a, nt, max_blocks, st); \
+    else launch_grouped_nt<DT, MI355Q_ZP_PRESCALED>(a, nt, max_blocks, st);               \
   } while (0)
   if (dtype == MI355Q_F16) MQ_GR_ZK(MI355Q_F16);
   else MQ_GR_ZK(MI355Q_BF16);

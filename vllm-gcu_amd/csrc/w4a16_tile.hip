@@ -596,11 +596,12 @@ hipError_t launch_small_groups_one(const TileArgs& a, int row_blocks, hipStream_
 }
 template <int DT, int MT, bool GROUPED>
 hipError_t launch_small_groups(const TileArgs& a, int zk, int gpb, int row_blocks, hipStream_t st) {
-  if (gpb == 2) {
-    if (zk == MI355Q_ZP_NONE) return launch_small_groups_one<DT, MI355Q_ZP_NONE, MT, GROUPED, 2>(a, row_blocks, st);
-    if (zk == MI355Q_ZP_PACKED) return launch_small_groups_one<DT, MI355Q_ZP_PACKED, MT, GROUPED, 2>(a, row_blocks, st);
-    return launch_small_groups_one<DT, MI355Q_ZP_PRESCALED, MT, GROUPED, 2>(a, row_blocks, st);
-  }
+  if constexpr (!(GROUPED && MT == 2))               // (blocks of 32 slots with groups of 64 never come here)
+    if (gpb == 2) {
+      if (zk == MI355Q_ZP_NONE) return launch_small_groups_one<DT, MI355Q_ZP_NONE, MT, GROUPED, 2>(a, row_blocks, st);
+      if (zk == MI355Q_ZP_PACKED) return launch_small_groups_one<DT, MI355Q_ZP_PACKED, MT, GROUPED, 2>(a, row_blocks, st);
+      return launch_small_groups_one<DT, MI355Q_ZP_PRESCALED, MT, GROUPED, 2>(a, row_blocks, st);
+    }
   if (zk == MI355Q_ZP_NONE) return launch_small_groups_one<DT, MI355Q_ZP_NONE, MT, GROUPED, 4>(a, row_blocks, st);
   if (zk == MI355Q_ZP_PACKED) return launch_small_groups_one<DT, MI355Q_ZP_PACKED, MT, GROUPED, 4>(a, row_blocks, st);
   return launch_small_groups_one<DT, MI355Q_ZP_PRESCALED, MT, GROUPED, 4>(a, row_blocks, st);
@@ -1048,8 +1049,12 @@ static int tile_launch_dense(void* out, const void* x, const int32_t* qweight, c
 int w4a16_stream_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales,
                                 const void* zeros, int zeros_kind, const float* topk_weights,
                                 const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
-                                int numel, int topk, int block_size, int max_blocks, int E, int K, int N,
-                                int group_size, int dtype, hipStream_t st);
+                                int numel, int topk, int max_blocks, int E, int K, int N, int group_size, int dtype, hipStream_t st);
+
+int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
+                              const float* topk_weights, const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
+                              int numel, int topk, int block_size, int max_blocks, int E, int K, int N, int group_size, int dtype,
+                              hipStream_t st);
 
 // Split-K plan of a grouped launch.  The host does not know how many blocks the alignment filled, so
 // the grid is estimated as every slot in a full block plus half a block of pads per expert.  A long K
@@ -1093,7 +1098,6 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
                          const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                          int numel, int topk, int block_size, int max_blocks, int E, int K, int N,
                          int group_size, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st) {
-  // groups of 64 and 32: the plain loop of the MFMA kernel at every block size
   const bool small_groups = group_size == 64 || group_size == 32;
   MQ_REQUIRE(group_size % 128 == 0 || (small_groups && !scales_f32 && !out_scale),
              "moe_w4a16: group_size=%d must be 32, 64 or a multiple of 128 (a multiple of 128 with fp32 scales)", group_size);
@@ -1101,13 +1105,20 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
              "moe_w4a16: activation matrix of %d rows x %d is 4 GiB or more", numel / (topk > 0 ? topk : 1), K);
   MQ_REQUIRE(block_size == 16 || block_size == 32 || block_size == 64 || block_size == 128,
              "moe_w4a16: block_size=%d must be 16, 32, 64 or 128", block_size);
-  // blocks of 16 or 32 slots (decode-sized token counts): the layer is bound by the experts' weights,
-  // which the streaming kernel reads faster than the MFMA tile kernel with one or two row tiles
+  // Blocks of 32 slots, and of 64 that are half empty on average over a long K: the kernel with copying wavefronts, which
+  // takes a block by the row tiles that hold slots.  (us per layer, before -> here: eight experts of 4096 x 28672 and 14336 x 4096 at
+  // 12 / 24 rows per expert, blocks of 32, 218 / 245 -> 176 / 189, at 32 / 48, blocks of 64, 245 / 246 -> 215 / 236; sixty of 2048 x 2816 and
+  // 1408 x 2048 at 17 / 26 rows, blocks of 32, 132 / 147 -> 94 / 103, but at 34, blocks of 64, 122 against 132.)
+  const bool plain = !scales_f32 && !out_scale;
+  if (plain && group_size != 32 && (block_size == 32 || (block_size == 64 && K >= 4096 && numel <= 48L * E)))
+    return w4a16_rows_grouped_launch(out, x, qweight, scales, zeros, zeros_kind, topk_weights, sorted_ids, expert_ids, npp, numel,
+                                     topk, block_size, max_blocks, E, K, N, group_size, dtype, st);
+  // blocks of 16 slots (decode-sized token counts): the layer is bound by the experts' weights,
+  // which the streaming kernel reads faster than the MFMA tile kernel with one row tile
   // (the grouped streaming kernel takes groups that are multiples of 128 only)
-  if (block_size <= 32 && !scales_f32 && !out_scale && !small_groups)
+  if (block_size == 16 && plain && !small_groups)
     return w4a16_stream_grouped_launch(out, x, qweight, scales, zeros, zeros_kind, topk_weights, sorted_ids,
-                                       expert_ids, npp, numel, topk, block_size, max_blocks, E, K, N, group_size,
-                                       dtype, st);
+                                       expert_ids, npp, numel, topk, max_blocks, E, K, N, group_size, dtype, st);
   TileArgs a = {};
   a.out = (uint16_t*)out;
   a.x = (const uint16_t*)x;
