@@ -770,7 +770,9 @@ fp8_block_gemm_kernel(F8Args a) {
       if (done >= 0) {
         add(6);
         add(7);
+        // the two adds below find products and scales of 0: a scale of the tile before may be infinite, and Inf * 0 is NaN
         ring[2] = ring[3] = (f4){0.f, 0.f, 0.f, 0.f};
+        sc[NJ - 2] = sc[NJ - 1] = 0.f;
         epilogue(done);
       }
       if (tile >= total_tiles) return;
