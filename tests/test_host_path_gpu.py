@@ -139,3 +139,46 @@ def test_declined_operands():
     assert h.w4a16(x, layer.qweight, layer.qzeros, layer.scales, g, None, 128) is None              # not verified yet
     with torch.enable_grad():
         assert h.w4a16(x.clone().requires_grad_(), *args) is None
+
+OPERATOR = {"gptq": "gptq_gemm_gcu", "awq": "awq_gemm_gcu", "int8 static": "dot_bias_quant", "int8 dynamic": "cutlass_scaled_mm",
+            "fp8 block": "linear_quant", "fp8 token": "cutlass_scaled_mm", "fp8 static": "cutlass_scaled_mm"}
+
+
+def _traced_or_refused(fn, a, b):
+    """torch.jit.trace of ``fn`` on ``a`` computes ``fn(b)`` too; -> False where torch refuses to trace (it does not take
+    operators whose schema writes to a plain ``Tensor!``).  What must not happen is a result recorded as a constant."""
+    try:
+        traced = torch.jit.trace(fn, (a,), check_trace=False)
+    except RuntimeError as e:
+        assert "observable data dependence" not in str(e)
+        return False
+    assert torch.equal(traced(b), fn(b)) and torch.equal(traced(a), fn(a))
+    return True
+
+
+@pytest.mark.parametrize("which", sorted(MAKE))
+def test_tracing_sees_the_operator(which):
+    print(f"case host path traced {which}", flush=True)
+    _, layer, apply = MAKE[which](which, torch.float16)
+    a, b = (torch.randn(5, K, device="cuda", dtype=torch.float16) for _ in range(2))
+    apply(layer, a, None)                                       # (may verify and convert)
+    traced = _traced_or_refused(lambda t: apply(layer, t, None) + t[:, :1], a, b)
+    assert traced or which not in ("gptq", "awq")
+
+
+@pytest.mark.parametrize("grouped", [True])
+def test_tracing_sees_the_routing(grouped):
+    from vllm_gcu_amd.kernels import fused_moe as fmoe
+    print(f"case host path traced routing grouped={grouped}", flush=True)
+    a, b = (torch.randn(5, 8, device="cuda") for _ in range(2))
+    for i in (0, 1):
+        _traced_or_refused(lambda g: fmoe.select_experts(g, g, 2, grouped, True, topk_group=2, num_expert_group=4)[i] + g[:, :2], a, b)
+
+
+@pytest.mark.parametrize("which", ["gptq", "awq"])
+def test_vmap(which):
+    print(f"case host path vmap {which}", flush=True)
+    _, layer, apply = MAKE[which](which, torch.float16)
+    x = torch.randn(3, 5, K, device="cuda", dtype=torch.float16)
+    want = torch.stack([apply(layer, t, None) for t in x])
+    assert torch.equal(torch.vmap(lambda t: apply(layer, t, None))(x), want)

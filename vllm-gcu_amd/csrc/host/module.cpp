@@ -3,8 +3,9 @@
 // Every function here is a fast path: it takes operands that the kernels can read as they are (GPU tensors,
 // contiguous, weights in this library's layouts, matching types and sizes), allocates the outputs and launches.
 // Anything else -- a conversion, a reference-layout weight, a tensor subclass or a mode that must see the
-// operator (tracing, functionalisation, gradients), a wrong size -- makes it return None before any work is
-// enqueued, and the Python caller goes on with its general path, which converts or raises.
+// operator (torch.jit tracing, functionalisation, functorch's transforms, gradients), a wrong size -- makes it return
+// None before any work is enqueued, and the Python caller goes on with its general path, which calls the operator, converts
+// or raises.
 #include <Python.h>
 
 #include <ATen/core/grad_mode.h>
@@ -41,9 +42,14 @@ constexpr c10::DispatchKeySet kSpecial({
     c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Batched,
     c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
 
+// what a thread turns on to see every operator: tracing records it, functorch runs it level by level
+constexpr c10::DispatchKeySet kWatching = kSpecial | c10::DispatchKeySet({
+    c10::DispatchKey::Tracer, c10::DispatchKey::FuncTorchVmapMode, c10::DispatchKey::FuncTorchDynamicLayerFrontMode,
+    c10::DispatchKey::FuncTorchDynamicLayerBackMode});
+
 bool modes_active() {
   const auto inc = c10::impl::tls_local_dispatch_key_set().included_;
-  return inc.has_any(kSpecial) || c10::impl::TorchDispatchModeTLS::any_modes_set();
+  return inc.has_any(kWatching) || c10::impl::TorchDispatchModeTLS::any_modes_set();
 }
 
 bool plain(const Tensor& t) {
