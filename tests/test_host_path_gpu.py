@@ -175,6 +175,41 @@ def test_tracing_sees_the_routing(grouped):
         _traced_or_refused(lambda g: fmoe.select_experts(g, g, 2, grouped, True, topk_group=2, num_expert_group=4)[i] + g[:, :2], a, b)
 
 
+@pytest.mark.parametrize("which", sorted(MAKE))
+def test_subclasses_and_function_modes_see_the_operator(which):
+    print(f"case host path overridden {which}", flush=True)
+    seen = []
+
+    class Seen(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    _, layer, apply = MAKE[which](which, torch.float16)
+    x = torch.randn(5, K, device="cuda", dtype=torch.float16)
+    want = [apply(layer, x, None) for _ in range(2)][-1]
+    got = apply(layer, x.as_subclass(Seen), None)
+    assert any(OPERATOR[which] in s for s in seen) and torch.equal(got.as_subclass(torch.Tensor), want)
+    seen.clear()
+    with Mode():
+        got = apply(layer, x, None)
+    assert any(OPERATOR[which] in s for s in seen) and torch.equal(got, want)
+    # a parameter class that leaves torch's functions alone, and a default device, are nothing to stand aside for
+    class Weight(torch.nn.Parameter):
+        pass
+    from vllm_gcu_amd.kernels import _runtime as rt
+    if which == "awq":
+        qw = Weight(layer.qweight.data, requires_grad=False)
+        with torch.device("cuda"):
+            assert torch.equal(rt.host.w4a16(x, qw, layer.qzeros, layer.scales, None, None, 128), want)
+
+
 @pytest.mark.parametrize("which", ["gptq", "awq"])
 def test_vmap(which):
     print(f"case host path vmap {which}", flush=True)

@@ -3,16 +3,18 @@
 // Every function here is a fast path: it takes operands that the kernels can read as they are (GPU tensors,
 // contiguous, weights in this library's layouts, matching types and sizes), allocates the outputs and launches.
 // Anything else -- a conversion, a reference-layout weight, a tensor subclass or a mode that must see the
-// operator (torch.jit tracing, functionalisation, functorch's transforms, gradients), a wrong size -- makes it return
-// None before any work is enqueued, and the Python caller goes on with its general path, which calls the operator, converts
-// or raises.
+// operator (torch.jit tracing, __torch_function__ and __torch_dispatch__ in classes and modes, functionalisation,
+// functorch's transforms, gradients), a wrong size -- makes it return None before any work is enqueued, and the
+// Python caller goes on with its general path, which calls the operator, converts or raises.
 #include <Python.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Device.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
@@ -47,9 +49,33 @@ constexpr c10::DispatchKeySet kWatching = kSpecial | c10::DispatchKeySet({
     c10::DispatchKey::Tracer, c10::DispatchKey::FuncTorchVmapMode, c10::DispatchKey::FuncTorchDynamicLayerFrontMode,
     c10::DispatchKey::FuncTorchDynamicLayerBackMode});
 
+// looked up when the module is loaded: the __torch_function__ of classes that leave torch's functions alone (parameters among
+// them), and the type of the mode behind torch.device(..) contexts and torch.set_default_device, which acts on the functions that
+// make tensors only
+PyObject* g_disabled_torch_function = nullptr;
+PyObject* g_device_context = nullptr;
+
+bool function_mode_active() {
+  using TLS = at::impl::PythonTorchFunctionTLS;
+  if (!at::impl::torch_function_mode_enabled()) return false;
+  for (int64_t i = 0; i < TLS::stack_len(); ++i)
+    if (reinterpret_cast<PyObject*>(Py_TYPE(TLS::get_stack_at(i)->ptr(getPyInterpreter()))) != g_device_context) return true;
+  return false;
+}
+
 bool modes_active() {
   const auto inc = c10::impl::tls_local_dispatch_key_set().included_;
-  return inc.has_any(kWatching) || c10::impl::TorchDispatchModeTLS::any_modes_set();
+  return inc.has_any(kWatching) || c10::impl::TorchDispatchModeTLS::any_modes_set() || function_mode_active();
+}
+
+// a tensor of a class whose __torch_function__ has to see the call
+bool overrides_torch_function(PyObject* o) {
+  static const Bytes name("__torch_function__");
+  if (THPVariable_CheckExact(o)) return false;
+  PyObject* f = PyObject_GetAttr(reinterpret_cast<PyObject*>(Py_TYPE(o)), name.o);
+  if (!f) PyErr_Clear();
+  Py_XDECREF(f);                   // (the class holds it)
+  return f != g_disabled_torch_function;
 }
 
 bool plain(const Tensor& t) {
@@ -60,7 +86,7 @@ bool plain(const Tensor& t) {
 const Tensor* as_tensor(PyObject* o) {
   if (!o || !THPVariable_Check(o)) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
-  return plain(t) ? &t : nullptr;
+  return plain(t) && !overrides_torch_function(o) ? &t : nullptr;
 }
 
 // None or no object -> an undefined tensor; false for anything a fast path does not take
@@ -184,7 +210,7 @@ bool g_idx_ok(PyObject* g, int64_t group) {
   if (!g || g == Py_None) return true;
   if (!THPVariable_Check(g)) return false;
   const Tensor& t = THPVariable_Unpack(g);
-  if (t.key_set().has_any(kSpecial)) return false;
+  if (t.key_set().has_any(kSpecial) || overrides_torch_function(g)) return false;
   if (t.numel() == 0) return true;
   PyObject** dict = _PyObject_GetDictPtr(g);
   PyObject* v = dict && *dict ? PyDict_GetItem(*dict, tag.o) : nullptr;
@@ -727,4 +753,14 @@ Scratch workspace(const Tensor& like, void* stream, size_t bytes) {
 
 }  // namespace mi355q_host
 
-PyMODINIT_FUNC PyInit__mi355q_host() { return PyModule_Create(&mi355q_host::kModule); }
+PyMODINIT_FUNC PyInit__mi355q_host() {
+  using namespace mi355q_host;
+  auto attribute = [](const char* module, const char* name) -> PyObject* {
+    const Ref m(PyImport_ImportModule(module));
+    return m.o ? PyObject_GetAttrString(m.o, name) : nullptr;
+  };
+  g_disabled_torch_function = attribute("torch._C", "_disabled_torch_function_impl");
+  g_device_context = attribute("torch.utils._device", "DeviceContext");
+  if (!g_disabled_torch_function || !g_device_context) return nullptr;
+  return PyModule_Create(&kModule);
+}
