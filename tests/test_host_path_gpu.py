@@ -166,7 +166,7 @@ def test_tracing_sees_the_operator(which):
     assert traced or which not in ("gptq", "awq")
 
 
-@pytest.mark.parametrize("grouped", [True])
+@pytest.mark.parametrize("grouped", [False, True])
 def test_tracing_sees_the_routing(grouped):
     from vllm_gcu_amd.kernels import fused_moe as fmoe
     print(f"case host path traced routing grouped={grouped}", flush=True)

@@ -536,11 +536,15 @@ def fused_topk(hidden_states: torch.Tensor, gating_output: torch.Tensor, topk: i
     rt.require_gpu(gating_output)
     if gating_output.numel() == 0:
         return topk_weights, topk_ids
-    # one launch: the kernel reads f16 / bf16 / f32 logits as they are and divides by the row sum
-    # itself (the reference's caller does both in separate PyTorch kernels)
     g = gating_output.contiguous()
     if g.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         g = g.float()
+    if torch.jit.is_tracing():
+        # (the call below is none that a trace could record)
+        topk_softmax(topk_weights, topk_ids, torch.empty_like(topk_ids), g)
+        return (topk_weights / topk_weights.sum(-1, keepdim=True) if renormalize else topk_weights), topk_ids
+    # one launch: the kernel reads f16 / bf16 / f32 logits as they are and divides by the row sum
+    # itself (the reference's caller does both in separate PyTorch kernels)
     with torch.cuda.device(g.device):
         _lib.call("mi355q_topk_softmax", topk_weights.data_ptr(), topk_ids.data_ptr(), None, g.data_ptr(),
                   M, g.shape[1], topk, int(bool(renormalize)), rt.dtype_code(g.dtype), rt.stream_ptr())
