@@ -30,7 +30,9 @@ enum {
   MI355Q_ZP_PACKED = 1,    /* int32 [K/g, N/8], nibble j of column c = z[g, 8c+j]   */
   MI355Q_ZP_PRESCALED = 2  /* activation-dtype [K/g, N] holding z*scale (the form   */
                            /* the reference's GPTQ loader produces,                 */
-                           /* vllm_gcu/kernels/quantization/rearrange.py:33-34)     */
+                           /* vllm_gcu/kernels/quantization/rearrange.py:33-34):    */
+                           /* w = q*scale - zeros, whatever zeros holds; a kernel   */
+                           /* may read z*scale of an integer z before its rounding  */
 };
 
 /* source formats understood by the int4 repack kernels */

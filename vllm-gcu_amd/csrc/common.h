@@ -91,6 +91,22 @@ template <> struct Elem<MI355Q_BF16> {
   static __device__ __forceinline__ uint16_t from_f32(float f) { return f32_to_bf16(f); }
 };
 
+// A pre-scaled zero-point zs (16 bits, as stored) of a group with scale s, for kernels whose operands are q - z with an integer
+// z: w = q s - zs is (q - z) s - rest.  Where zs is bit for bit an integer 0 .. 15 times s, as the loaders that pre-multiply make
+// it, rest is 0 (zs read before its rounding); any other zs is taken as given.  A scale of 0 has w = -zs.
+template <int DT>
+__device__ __forceinline__ float prescaled_zero(uint16_t zs, float s) {
+  return fminf(fmaxf(__builtin_rintf(Elem<DT>::to_f32(zs) / s), 0.0f), 15.0f);     // (0 / 0: 0)
+}
+// not 0: z times s is not zs (what the loops look at; the rest itself only where there is one)
+template <int DT>
+__device__ __forceinline__ uint32_t prescaled_differs(uint16_t zs, float z, float s) { return Elem<DT>::from_f32(z * s) ^ zs; }
+template <int DT>
+__device__ __forceinline__ float prescaled_rest(uint16_t zs, float s) {
+  const float z = prescaled_zero<DT>(zs, s), zf = Elem<DT>::to_f32(zs);
+  return z == 0.0f ? zf : prescaled_differs<DT>(zs, z, s) ? __builtin_fmaf(-z, s, zf) : 0.0f;
+}
+
 // Kernels whose accumulators alone fill 128+ registers call this once: an
 // inline-asm AGPR operand makes the compiler keep MFMA accumulators in the
 // accumulation half of the register file (AGPR-form MFMA) instead of using it

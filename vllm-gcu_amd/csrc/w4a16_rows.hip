@@ -18,7 +18,8 @@
 // (the compiler, which does not see them, waits for the LDS reads alone); they are waited for by hand.
 //
 // B operands are the exact integers q - z in the activation type and the group scale multiplies the fp32 partial sum of
-// each group, as in the 64-row tile kernel: the only rounding is that of the fp32 additions, for fp16 and bf16 alike.
+// each group, as in the 64-row tile kernel: the only rounding is that of the fp32 additions, for fp16 and bf16 alike.  What a
+// pre-scaled zero-point holds beyond an integer times the scale is taken off behind each K block.
 //
 // Measured (us, fp16, groups of 128, weights cold; before -> here): 4096 x 4096 at 48 / 96 / 192 rows 12.0 / 15.5 / 23.1 ->
 // 9.1 / 9.4 / 12.2; 4096 x 6144 at 64 / 128 / 256 15.9 / 20.5 / 28.2 -> 9.5 / 13.2 / 18.6; 4096 x 28672 at 48 / 64 / 96
@@ -211,6 +212,7 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
         u4 w[NT], av[2][MT];
         float sc[NT][GPB];
         _Float16 zlo[NT][GPB], zhi[NT][GPB];
+        uint32_t rests = 0;                             // not 0: a pre-scaled zero-point is no integer times the scale
         uint32_t zw[GPB];
 #pragma unroll
         for (int t = 0; t < NT; ++t) w[t] = *(const u4*)(st + C::W_OFF + (wave * NT + t) * 1024 + lane * 16);
@@ -224,10 +226,12 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
 #pragma unroll
           for (int g = 0; g < GPB; ++g) {
             sc[t][g] = Elem<DT>::to_f32(*(const uint16_t*)(st + C::S_OFF + 256 * g + (8 * c + tile) * 2));
-            if constexpr (ZK == MI355Q_ZP_PRESCALED) {   // z * s rounded to the activation type -> the integer z
-              const float zf = __builtin_rintf(Elem<DT>::to_f32(*(const uint16_t*)(st + C::Z_OFF + 256 * g + (8 * c + tile) * 2)) / sc[t][g]);
+            if constexpr (ZK == MI355Q_ZP_PRESCALED) {
+              const uint16_t zs = *(const uint16_t*)(st + C::Z_OFF + 256 * g + (8 * c + tile) * 2);
+              const float zf = prescaled_zero<DT>(zs, sc[t][g]);
               zlo[t][g] = (_Float16)(1024.0f + zf);
               zhi[t][g] = (_Float16)(64.0f + zf);
+              rests |= prescaled_differs<DT>(zs, zf, sc[t][g]);
             } else {                                     // fp16 bit patterns directly
               const uint32_t z = (zw[g] >> (4 * tile)) & 15u;
               zlo[t][g] = bitcast<_Float16>((uint16_t)(0x6400u | z));
@@ -261,6 +265,35 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
               for (int t = 0; t < NT; ++t) acc[mt][t] += sc[t][g] * part[mt][t];
+          }
+        }
+        if constexpr (ZK == MI355Q_ZP_PRESCALED) {
+          // (rare: a checkpoint whose zero-points are no integers) what they hold beyond them times the sum of the group's
+          // activations, one matrix instruction with a B operand of ones per K step.  Everything is read from LDS again, so
+          // that the loop above has its registers for itself.
+          if (__any(rests != 0)) {
+            asm volatile("" : : : "memory");
+            const uint32_t one = DT == MI355Q_F16 ? 0x3c003c00u : 0x3f803f80u;
+            const u4 ones = {one, one, one, one};
+#pragma unroll
+            for (int g = 0; g < GPB; ++g) {
+              float rest[NT];
+#pragma unroll
+              for (int t = 0; t < NT; ++t) {
+                const unsigned char* const q = st + 256 * g + (8 * c + t0 + wave * NT + t) * 2;
+                rest[t] = prescaled_rest<DT>(*(const uint16_t*)(q + C::Z_OFF), Elem<DT>::to_f32(*(const uint16_t*)(q + C::S_OFF)));
+              }
+#pragma unroll
+              for (int mt = 0; mt < MT; ++mt) {
+                f4 xs = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = g * (4 / GPB); s < (g + 1) * (4 / GPB); ++s) xs = MM::run(*(const u4*)(st + a_pos[s] + mt * 4096), ones, xs);
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                  if (rest[t] != 0.0f) acc[mt][t] -= rest[t] * xs;
+                asm volatile("" : : : "memory");
+              }
+            }
           }
         }
       }

@@ -294,17 +294,9 @@ w4a16_tile_kernel(TileArgs a) {
       sc = sreg;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        if (ZK == MI355Q_ZP_PRESCALED) {
-          const uint32_t zw = (t < 2) ? zsreg.x : zsreg.y;
-          // the loader pre-multiplied an integer zero-point by the scale
-          // (z * s rounded to the activation type): recover the integer
-          const float zf = __builtin_rintf(IO::to_f32((uint16_t)((t & 1) ? (zw >> 16) : (zw & 0xffffu))) / scale_of(sc, t));
-          zz[t] = (h2){(_Float16)(1024.0f + zf), (_Float16)(64.0f + zf)};
-        } else {
-          // fp16 bit patterns directly: 1024 + z = 0x6400 | z, 64 + z = 0x5400 | z << 4
-          const uint32_t z = (zreg >> (4 * t)) & 15u;
-          zz[t] = bitcast<h2>(0x54006400u | z | (z << 20));
-        }
+        // fp16 bit patterns directly: 1024 + z = 0x6400 | z, 64 + z = 0x5400 | z << 4
+        const uint32_t z = (zreg >> (4 * t)) & 15u;
+        zz[t] = bitcast<h2>(0x54006400u | z | (z << 20));
       }
     };
     const unsigned aoff = (wmh * MTW * 16 + c) * A_ROW + kq * 16;
@@ -399,6 +391,7 @@ w4a16_tile_kernel(TileArgs a) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) wcur[t] = wreg[t];
       float sc[GPB][4];
+      uint32_t rests = 0;                    // not 0: a pre-scaled zero-point is no integer times the scale
       h2 zz[GPB][4];
 #pragma unroll
       for (int sg = 0; sg < GPB; ++sg) {
@@ -411,9 +404,9 @@ w4a16_tile_kernel(TileArgs a) {
           float zf;
           if (ZK == MI355Q_ZP_PRESCALED) {
             const uint32_t zw = (t < 2) ? zsv.x : zsv.y;
-            // the loader pre-multiplied an integer zero-point by the scale
-            // (z * s rounded to the activation type): recover the integer
-            zf = __builtin_rintf(IO::to_f32((uint16_t)((t & 1) ? (zw >> 16) : (zw & 0xffffu))) / sc[sg][t]);
+            const uint16_t zs = (uint16_t)((t & 1) ? (zw >> 16) : (zw & 0xffffu));
+            zf = prescaled_zero<DT>(zs, sc[sg][t]);
+            rests |= prescaled_differs<DT>(zs, zf, sc[sg][t]);
           } else {
             zf = (float)((zv >> (4 * t)) & 15u);
           }
@@ -450,6 +443,35 @@ w4a16_tile_kernel(TileArgs a) {
           }
 #pragma unroll
           for (int t = 0; t < 4; ++t) acc[mt][t] += sc[sg][t] * part[t];
+        }
+      }
+      if constexpr (ZK == MI355Q_ZP_PRESCALED) {
+        // (rare: a checkpoint whose zero-points are no integers) what they hold beyond them times the sum of the group's
+        // activations, one matrix instruction with a B operand of ones per K step.  Everything is read again, so that the
+        // loop above has its registers for itself.
+        if (__any(rests != 0)) {
+          asm volatile("" : : : "memory");
+          const uint32_t one = DT == MI355Q_F16 ? 0x3c003c00u : 0x3f803f80u;
+          const vec ones = bitcast<vec>((u4){one, one, one, one});
+#pragma unroll
+          for (int sg = 0; sg < GPB; ++sg) {
+            const size_t q = (size_t)((128 * g) / a.gs + sg) * N + ncol;
+            float rest[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) rest[t] = prescaled_rest<DT>(((const uint16_t*)zeros)[q + t], IO::to_f32(scales[q + t]));
+#pragma unroll
+            for (int mt = 0; mt < MTW; ++mt) {
+              if (!tile_live(mt)) continue;
+              f4 xs = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+              for (int s = sg * (4 / GPB); s < (sg + 1) * (4 / GPB); ++s)
+                xs = MM::run(bitcast<vec>(*(const u4*)(abase + mt * 16 * A_ROW + s * 64)), ones, xs);
+#pragma unroll
+              for (int t = 0; t < 4; ++t)
+                if (rest[t] != 0.0f) acc[mt][t] -= rest[t] * xs;
+              asm volatile("" : : : "memory");
+            }
+          }
         }
       }
       // the other buffer was last read one iteration ago: every wavefront has
