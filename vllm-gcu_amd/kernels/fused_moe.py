@@ -40,10 +40,13 @@ def get_default_config(M: int, E: int, N: int, K: int, topk: int, dtype: Optiona
         # kernels with gathered rows instead of the weight-streaming kernel
         return {"BLOCK_SIZE_M": 256 if per_expert > _TILE_256_ROWS_PER_EXPERT else 128, "BLOCK_SIZE_N": 64,
                 "BLOCK_SIZE_K": 32, "GROUP_SIZE_M": 8}
-    # W4A16 experts (block_shape [0, group]) leave the blocks of 16 earlier: their kernel for blocks of 32 takes as many
-    # row tiles as a block has rows (us per layer with 16 / 32: eight experts of 4096 x 28672 at 16 rows per expert 209 / 176,
-    # sixty of 2048 x 2816 at 13 rows 87 / 89)
-    if per_expert <= (12 if block_shape is not None and block_shape[0] == 0 else 16):
+    # W4A16 experts leave the blocks of 16 earlier: their kernel for blocks of 32 takes as many row tiles as a block has rows
+    # (us per layer with 16 / 32 at 13 and at 16 rows per expert: eight experts of 4096 x 14336 168 / 170 and 195 / 179, sixty of
+    # 2048 x 1408 83 / 75 and 97 / 79, 128 of 2048 x 768 in bf16 102 / 101 and 120 / 106, groups of 64, eight of 4096 x 14336, 220 /
+    # 158 and 240 / 184).  Groups of 32 and W8A16 experts have other kernels (eight of 4096 x 14336: 257 / 292 and 274 / 297;
+    # 336 / 357 and 405 / 362)
+    rows_kernel = dtype == "int4_w4a16" and block_shape is not None and block_shape[1] != 32
+    if per_expert <= (12 if rows_kernel else 16):
         bm = 16
     elif per_expert <= 28:      # measured on the Mixtral-8x7B W4A16 layer: at 32 rows per expert on average
         bm = 32                 # half of the experts already need a second block of 32

@@ -60,6 +60,10 @@ class TritonExpertsPad:
     def quant_dtype(self):
         return self.quant_config.quant_dtype
 
+    @property
+    def config_dtype(self) -> Optional[str]:
+        return "int8_w8a8" if self.use_int8_w8a8 else "int4_w4a16" if self.use_int4_w4a16 else None
+
     def supports_chunking(self) -> bool:
         return True
 
@@ -87,8 +91,8 @@ class TritonExpertsPad:
         else:
             return False
         E, M, N, K, top_k = moe_problem_size(hidden_states, w1, w2, topk_ids, self.use_int4_w4a16)
-        config = get_default_config(M=M, E=E, N=N, K=K, topk=top_k, dtype="int8_w8a8" if self.use_int8_w8a8 else None,
-                                    is_marlin=False, block_shape=self.block_shape)
+        config = get_default_config(M=M, E=E, N=N, K=K, topk=top_k, dtype=self.config_dtype, is_marlin=False,
+                                    block_shape=self.block_shape)
         return rt.host.fused_experts(mode, group, config["BLOCK_SIZE_M"], hidden_states, w1, w2, w1_scale, w2_scale, w1_zp,
                                      w2_zp, topk_weights, topk_ids, output) is not None
 
@@ -105,8 +109,8 @@ class TritonExpertsPad:
             global_num_experts = E
         unquantised = w1.dtype == hidden_states.dtype and w1.dtype in (torch.float16, torch.bfloat16)
         config = get_default_config(M=num_tokens, E=E, N=N, K=K, topk=top_k_num,
-                                    dtype="int8_w8a8" if self.use_int8_w8a8 else "w16a16" if unquantised else None,
-                                    is_marlin=False, block_shape=self.block_shape)
+                                    dtype="w16a16" if unquantised else self.config_dtype, is_marlin=False,
+                                    block_shape=self.block_shape)
         act_dtype = workspace2.dtype
         # cache1 and cache3 share workspace2: cache1 is dead once cache2 exists
         cache1 = workspace2.reshape(-1)[:num_tokens * top_k_num * N].view(num_tokens, top_k_num, N)
