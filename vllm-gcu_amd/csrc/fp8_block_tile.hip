@@ -564,21 +564,22 @@ fp8_block_gemm_kernel(F8Args a) {
         wo[p] = (uint32_t)(r * a.ldw + 16 * cchunk);
       }
     }
-    // activation scales: 64 rows per copying wavefront, 128-row tiles twice (index in floats)
+    // activation scales: 64 rows per copying wavefront, 128-row tiles twice (32-bit index in floats from the tile's first row;
+    // grouped: from the matrix's, whose scales the entry point keeps below 2^27 bytes)
     const int srow = (64 * wave + lane) & (BM - 1);
     // (split K: the tile's range starts kb0 K blocks into every row; 64 kslab rows interleave their K blocks)
     const int kb0 = ksplits > 1 ? (tile % ksplits) * (KB / ksplits) : 0;
     if (!GROUPED && a.xs_t) {
       // K block major: the 64 scales of a copy lie side by side (4 cache lines instead of 64)
-      xso = (uint32_t)min(m0 + srow, M - 1);
-      xsbase = a.xs_t + (long)kb0 * a.xs_ld;
+      xso = (uint32_t)(min(m0 + srow, M - 1) - m0);
+      xsbase = a.xs_t + (long)kb0 * a.xs_ld + m0;
     } else if (GROUPED) {
       const int id = a.sorted_ids[m0 + srow];
       xso = (uint32_t)(max(0, min(id, a.numel - 1)) / a.topk) * (uint32_t)KB;
       xsbase = a.x_scale;
     } else {
-      xso = (uint32_t)min(m0 + srow, M - 1) * (uint32_t)KB + (uint32_t)kb0;
-      xsbase = a.x_scale;
+      xso = (uint32_t)((min(m0 + srow, M - 1) - m0) * KB);
+      xsbase = a.x_scale + (long)m0 * KB + kb0;
     }
     wsbase = escales + (n0 >> 7) * KB + kb0;       // the first of them copies the tile's weight scale
     xtile = GROUPED ? a.x : a.x + (long)m0 * a.ldx + (long)kb0 * FTKB;
