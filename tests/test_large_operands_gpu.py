@@ -44,3 +44,46 @@ def test_fp8_block_scales_of_four_gib(monkeypatch):
     for p in parts:
         want = (x[p].float() * xs[p].repeat_interleave(128, 1)) @ wf.t()
         torch.testing.assert_close(out[p].float(), want, rtol=1e-2, atol=1e-2 * want.std().item())
+
+
+# rows of 8192 pieces of 8 elements: this many of them in a launch whose pieces are counted with 31 bits
+D, PER_LAUNCH = 65536, 0x7fff0000 // 8192
+
+
+def _rows(make):
+    """A tensor of more rows than a launch takes and the slice around the border that is written and looked at."""
+    t = make(PER_LAUNCH + 40)
+    return t, slice(PER_LAUNCH - 2, PER_LAUNCH + 40)
+
+
+# the row count ends behind the border, and before it
+@pytest.mark.parametrize("count", [PER_LAUNCH + 20, PER_LAUNCH - 1])
+@pytest.mark.parametrize("which", ["silu_and_mul", "group_quant", "moe_sum"])
+def test_row_counts_over_several_launches(which, count):
+    print(f"case large {which} with a row count of {count}", flush=True)
+    _need({"silu_and_mul": 97, "group_quant": 50, "moe_sum": 66}[which])
+    wide = 2 * D if which == "silu_and_mul" else D
+    x, part = _rows(lambda n: torch.empty(n, wide, dtype=torch.float16, device="cuda"))
+    x[part] = torch.randn(x[part].shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(2)).half()
+    size = torch.tensor([count], dtype=torch.int32, device="cuda")
+    live = count - part.start
+    small = x[part].clone()
+    if which == "silu_and_mul":
+        out, want = torch.empty(x.shape[0], D, dtype=torch.float16, device="cuda"), torch.full((42, D), 7.0, dtype=torch.float16, device="cuda")
+        out[part] = 7.0
+        torch.ops._C.silu_and_mul_pad(out, x, size)
+        torch.ops._C.silu_and_mul(want[:live], small[:live])
+    elif which == "group_quant":
+        out, want = (torch.empty(n, D, dtype=torch.float8_e4m3fn, device="cuda") for n in (x.shape[0], 42))
+        out[part], want[:] = 7.0, 7.0
+        sc, wsc = torch.zeros(x.shape[0], D // 128, device="cuda"), torch.zeros(42, D // 128, device="cuda")
+        torch.ops._C.dynamic_per_token_group_fp8_quant_with_size(out, sc, x, size, 128)
+        torch.ops._C.dynamic_per_token_group_fp8_quant(want[:live], wsc[:live], small[:live], 128)
+        assert torch.equal(sc[part], wsc)
+        out, want = out.view(torch.uint8), want.view(torch.uint8)
+    else:
+        out, want = torch.empty(x.shape, dtype=torch.float16, device="cuda"), torch.full((42, D), 7.0, dtype=torch.float16, device="cuda")
+        out[part] = 7.0
+        torch.ops._moe_C.moe_sum_pad(out, x[:, None], size, 1, False)
+        want[:live] = small[:live]
+    assert torch.equal(out[part], want)

@@ -75,14 +75,19 @@ struct SharedDivisor {
   }
 };
 
+// Rows of this launch that count: `rows` of them, or up to the device's row count (times rows per count) less the `row0` rows of
+// the launches before this one.
+__device__ __forceinline__ uint32_t live_rows(uint32_t rows, const int* valid_rows, int rpc, long row0) {
+  return valid_rows ? (uint32_t)max(0L, min((long)rows, (long)max(0, *valid_rows) * rpc - row0)) : rows;
+}
+
 // ---- silu_and_mul: out[r, :d] = silu(x[r, :d]) * x[r, d:] -------------------
 // (row and piece of an item by multiplication: a 64-bit division per 16-byte piece was a quarter of these kernels'
 // instructions, and they are bound by issue as much as by HBM)
 template <int DT>
 __global__ void __launch_bounds__(256)
-silu_and_mul_kernel(uint16_t* out, const uint16_t* x, uint32_t rows, int d, FastDiv chunks, const int* valid_rows, int rpc) {
-  const long nrow = valid_rows ? min((long)rows, (long)max(0, *valid_rows) * rpc) : rows;
-  const uint32_t total = (uint32_t)nrow * chunks.d;
+silu_and_mul_kernel(uint16_t* out, const uint16_t* x, uint32_t rows, int d, FastDiv chunks, const int* valid_rows, int rpc, long row0) {
+  const uint32_t total = live_rows(rows, valid_rows, rpc, row0) * chunks.d;
   for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
     const uint32_t r = chunks.div(i), c = i - r * chunks.d;
     const uint16_t* xr = x + (size_t)r * 2 * d + 8 * c;
@@ -100,9 +105,8 @@ silu_and_mul_kernel(uint16_t* out, const uint16_t* x, uint32_t rows, int d, Fast
 template <int DT, bool SILU>
 __global__ void __launch_bounds__(256)
 group_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, uint32_t rows, int K, FastDiv chunks, int lpg,
-                       const int* valid_rows, int rpc) {
-  const long nrow = valid_rows ? min((long)rows, (long)max(0, *valid_rows) * rpc) : rows;
-  const uint32_t total = (uint32_t)nrow * chunks.d;     // 8-element pieces; lpg (a power of two <= 64) lanes per group
+                       const int* valid_rows, int rpc, long row0) {
+  const uint32_t total = live_rows(rows, valid_rows, rpc, row0) * chunks.d;     // 8-element pieces; lpg (a power of two <= 64) lanes per group
   const int lg = 31 - __clz(lpg);
   for (uint32_t i0 = blockIdx.x * 256; i0 < total; i0 += gridDim.x * 256) {
     const uint32_t i = i0 + threadIdx.x;
@@ -261,9 +265,8 @@ static_fp8_quant_kernel(uint8_t* out, const uint16_t* x, const float* scale, lon
 // ---- moe_sum: out[m, :] = sum_t in[m, t, :] in fp32 --------------------------
 template <int DT_IN, int DT_OUT>
 __global__ void __launch_bounds__(256)
-moe_sum_kernel(void* out, const uint16_t* in, uint32_t rows, int T, int K, FastDiv chunks, const int* valid_rows) {
-  const long nrow = valid_rows ? min((long)rows, (long)max(0, *valid_rows)) : rows;
-  const uint32_t total = (uint32_t)nrow * chunks.d;
+moe_sum_kernel(void* out, const uint16_t* in, uint32_t rows, int T, int K, FastDiv chunks, const int* valid_rows, long row0) {
+  const uint32_t total = live_rows(rows, valid_rows, 1, row0) * chunks.d;
   for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
     const long r = chunks.div(i);
     const int c = (int)(i - (uint32_t)r * chunks.d);
@@ -517,7 +520,6 @@ extern "C" int mi355q_silu_and_mul(void* out, const void* x, long rows, int d, i
   if (rows == 0) return 0;
   MQ_REQUIRE(out && x, "silu_and_mul: null pointer");
   MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "silu_and_mul: dtype %d must be f16 or bf16", dtype);
-  MQ_REQUIRE(!valid_rows || rows <= rows_per_launch(d / 8), "silu_and_mul: too many rows with a row count");
   hipStream_t st = as_stream(stream);
   const FastDiv chunks((uint32_t)(d / 8));
   for (long r0 = 0; r0 < rows; r0 += rows_per_launch(d / 8)) {
@@ -526,9 +528,9 @@ extern "C" int mi355q_silu_and_mul(void* out, const void* x, long rows, int d, i
     uint16_t* o = (uint16_t*)out + r0 * d;
     const uint16_t* xp = (const uint16_t*)x + r0 * 2 * d;
     if (dtype == MI355Q_F16)
-      hipLaunchKernelGGL((silu_and_mul_kernel<MI355Q_F16>), dim3(g), dim3(256), 0, st, o, xp, n, d, chunks, valid_rows, rows_per_count);
+      hipLaunchKernelGGL((silu_and_mul_kernel<MI355Q_F16>), dim3(g), dim3(256), 0, st, o, xp, n, d, chunks, valid_rows, rows_per_count, r0);
     else
-      hipLaunchKernelGGL((silu_and_mul_kernel<MI355Q_BF16>), dim3(g), dim3(256), 0, st, o, xp, n, d, chunks, valid_rows, rows_per_count);
+      hipLaunchKernelGGL((silu_and_mul_kernel<MI355Q_BF16>), dim3(g), dim3(256), 0, st, o, xp, n, d, chunks, valid_rows, rows_per_count, r0);
   }
   MQ_LAUNCH_CHECK("silu_and_mul");
   return 0;
@@ -545,7 +547,6 @@ extern "C" int mi355q_fp8_group_quant(uint8_t* out, float* scales, const void* x
              "fp8_group_quant: group_size=%d must be 64, 128, 256 or 512", group_size);
   MQ_REQUIRE(K % group_size == 0, "fp8_group_quant: K=%d must be a multiple of group_size=%d", K, group_size);
   MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "fp8_group_quant: dtype %d must be f16 or bf16", dtype);
-  MQ_REQUIRE(!valid_rows || rows <= rows_per_launch(K / 8), "fp8_group_quant: too many rows with a row count");
   hipStream_t st = as_stream(stream);
   const FastDiv chunks((uint32_t)(K / 8));
   const int lpg = group_size / 8;
@@ -558,13 +559,13 @@ extern "C" int mi355q_fp8_group_quant(uint8_t* out, float* scales, const void* x
     float* sc = scales + r0 * (K / group_size);
     const uint16_t* xp = (const uint16_t*)x + r0 * K * (fuse_silu_mul ? 2 : 1);
     if (fuse_silu_mul && f16)
-      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_F16, true>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count);
+      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_F16, true>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count, r0);
     else if (fuse_silu_mul)
-      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_BF16, true>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count);
+      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_BF16, true>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count, r0);
     else if (f16)
-      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_F16, false>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count);
+      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_F16, false>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count, r0);
     else
-      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_BF16, false>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count);
+      hipLaunchKernelGGL((group_fp8_quant_kernel<MI355Q_BF16, false>), dim3(g), dim3(256), 0, st, o, sc, xp, n, K, chunks, lpg, valid_rows, rows_per_count, r0);
   }
   MQ_LAUNCH_CHECK("fp8_group_quant");
   return 0;
@@ -622,7 +623,6 @@ extern "C" int mi355q_moe_sum(void* out, const void* in, long rows, int topk, in
   MQ_REQUIRE(in_dtype == MI355Q_F16 || in_dtype == MI355Q_BF16, "moe_sum: input dtype %d must be f16 or bf16", in_dtype);
   MQ_REQUIRE(out_dtype == in_dtype || out_dtype == MI355Q_F32, "moe_sum: output dtype %d must equal the input's or be f32", out_dtype);
   hipStream_t st = as_stream(stream);
-  MQ_REQUIRE(!valid_rows || rows <= rows_per_launch(K / 8), "moe_sum: too many rows with a row count");
   const FastDiv chunks((uint32_t)(K / 8));
   for (long r0 = 0; r0 < rows; r0 += rows_per_launch(K / 8)) {
     const uint32_t n = (uint32_t)std::min(rows - r0, rows_per_launch(K / 8));
@@ -630,13 +630,13 @@ extern "C" int mi355q_moe_sum(void* out, const void* in, long rows, int topk, in
     const uint16_t* p = (const uint16_t*)in + r0 * topk * K;
     void* o = (char*)out + r0 * K * (out_dtype == MI355Q_F32 ? 4 : 2);
     if (in_dtype == MI355Q_F16 && out_dtype == MI355Q_F16)
-      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F16>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows);
+      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F16>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0);
     else if (in_dtype == MI355Q_F16)
-      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F32>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows);
+      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F32>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0);
     else if (out_dtype == MI355Q_BF16)
-      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_BF16>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows);
+      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_BF16>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0);
     else
-      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_F32>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows);
+      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_F32>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0);
   }
   MQ_LAUNCH_CHECK("moe_sum");
   return 0;
