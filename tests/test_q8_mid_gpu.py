@@ -1,10 +1,9 @@
-"""The 8-bit kernel for a few dozen to some hundred rows (csrc/q8_mid.hip) through the operators that choose it:
-row counts around every tile edge, column counts that are and are not a multiple of eight column tiles, odd numbers of K
+"""The 8-bit kernel for a few dozen to 1536 rows (csrc/q8_mid.hip) through the operators that choose it:
+row counts around every tile edge and to the end of its range, column counts that are and are not a multiple of eight column tiles, odd numbers of K
 blocks, one and several K ranges, with and without bias.  int8 is exact; fp8 is compared with a float64 product."""
 import pytest
 import torch
 
-from vllm_gcu_amd import _lib
 from vllm_gcu_amd.kernels import _custom_ops as ops
 from vllm_gcu_amd.kernels import _runtime as rt
 from vllm_gcu_amd.kernels.quantization import rearrange
@@ -13,7 +12,9 @@ pytestmark = pytest.mark.gpu
 # (M, N, K): tiles of 32, 64 and 128 rows, with and without K ranges
 SHAPES = [(17, 64, 384), (31, 320, 128), (33, 512, 1152), (48, 1024, 7168), (63, 640, 640), (64, 4096, 2048), (65, 1024, 1024),
           (96, 3072, 3584), (127, 256, 4096), (129, 1024, 5120), (130, 4096, 7168), (200, 2048, 1408), (257, 4608, 3584),
-          (511, 4096, 4096), (512, 8192, 2048)]
+          (511, 4096, 4096), (512, 8192, 2048), (700, 512, 7168), (768, 1024, 4096), (1000, 3072, 3584), (1024, 4096, 4096),
+          (1300, 640, 2048), (1535, 1536, 3584), (1536, 2048, 2048)]
+BLOCK, SCALED, INT8 = 0, 1, 2            # kinds of mi355q_q8_mid_plan
 
 
 def _planned(kind, M, N, K):
@@ -25,7 +26,7 @@ def _planned(kind, M, N, K):
 @pytest.mark.parametrize("with_bias", [False, True])
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_int8(M, N, K, with_bias):
-    _planned(_lib.Q_INT8, M, N, K)
+    _planned(INT8, M, N, K)
     torch.manual_seed(M + N + K)
     x = torch.randint(-128, 128, (M, K), dtype=torch.int8, device="cuda")
     w = torch.randint(-128, 128, (N, K), dtype=torch.int8, device="cuda")
@@ -50,13 +51,13 @@ def test_fp8_block_and_scaled(M, N, K):
     xd = x.double().view(M, K // 128, 128) * xb.double()[..., None]
     wd = w.double().view(N // 128, 128, K // 128, 128) * wb.double()[:, None, :, None]
     want = xd.view(M, K) @ wd.view(N, K).t()
-    _planned(_lib.Q_FP8_BLOCK, M, N, K)
+    _planned(BLOCK, M, N, K)
     for bias in (None, torch.randn(N, device="cuda").bfloat16()):
         out = torch.full((M, N), float("nan"), device="cuda").bfloat16()
         torch.ops._C.linear_quant(out, x, wk, bias, xb, wb)
         ref = want if bias is None else want + bias.double()
         assert float((out.double() - ref).norm() / ref.norm()) < 3e-3        # one rounding to bf16
-    _planned(1, M, N, K)
+    _planned(SCALED, M, N, K)
     for xs, ws in ((torch.rand(M, 1, device="cuda") * 0.01, torch.rand(N, 1, device="cuda") * 0.01),
                    (torch.full((1,), 0.01, device="cuda"), torch.full((1,), 0.003, device="cuda"))):
         out = torch.full((M, N), float("nan"), device="cuda").half()

@@ -62,7 +62,8 @@ def test_tiles(mt, nt, K, N, g, splits, dtype, monkeypatch):
 
 @pytest.mark.parametrize("M,K,N,g", [(5, 1024, 1024, 64), (20, 4096, 16384, 128), (24, 2048, 512, 32), (33, 1024, 128, 128),
                                      (48, 4096, 1024, 128), (64, 2048, 4096, 128), (65, 3584, 512, 128), (96, 1024, 14336, 128),
-                                     (130, 2048, 1024, 64), (333, 1024, 2048, 128), (700, 1024, 1024, 128)])
+                                     (130, 2048, 1024, 64), (333, 1024, 2048, 128), (700, 1024, 1024, 128), (4095, 512, 128, 128),
+                                     (4096, 512, 128, 64), (4097, 512, 128, 64)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_automatic(M, K, N, g, dtype):
     """What the library takes by itself equals this kernel's result (its sums are exact on these inputs, so they prove
@@ -72,3 +73,28 @@ def test_automatic(M, K, N, g, dtype):
     want = torch.from_numpy(_want(q, z, s, x, g)).to(dtype)
     assert torch.equal(_run(q, z, s, x, g), want)
     assert torch.equal(_run(q, z, s, x, g, family=4), want)
+
+
+def test_activations_of_four_gib():
+    """The last row below 4 GiB of activations is addressed in 32 bits; from 4 GiB on the problem is refused."""
+    K, N, M = 1 << 24, 128, 127
+    print(f"case w4a16 rows M={M} K={K} N={N}", flush=True)
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 24 << 30:
+        pytest.skip("needs 24 GiB of GPU memory")
+    q, z, s, x = _case(1, M, 256, N, 128, torch.float16, exact=True)
+    packed = torch.zeros(K // 8, N, dtype=torch.int32, device="cuda")
+    packed[-32:] = torch.from_numpy(ow4.gptq_pack_weight(q)).cuda()
+    zeros = torch.zeros(K // 128, N // 8, dtype=torch.int32, device="cuda")
+    zeros[-2:] = torch.from_numpy(ow4.gptq_pack_zeros(z)).cuda()
+    w, zp = rearrange.rearrange_uint4_int32_gptq(packed, zeros)
+    del packed
+    scales = torch.ones(K // 128, N, dtype=torch.float16, device="cuda")
+    scales[-2:] = s.cuda()
+    xs = torch.zeros(M + 1, K, dtype=torch.float16, device="cuda")
+    xs[:M, -256:] = x.cuda()
+    got = ops.w4a16_gemm(xs[:M], w, scales, zp, None, 128, family=4)
+    assert torch.equal(got.cpu(), torch.from_numpy(_want(q, z, s, x, 128)).half())
+    for family in (0, 4):
+        with pytest.raises(RuntimeError, match="4 GiB"):
+            ops.w4a16_gemm(xs, w, scales, zp, None, 128, family=family)
