@@ -75,11 +75,11 @@ int mi355q_w4_unpack(const int32_t* packed, uint8_t* dst, int batch, int K, int 
  *   out[M, N] = x[M, K] @ ((q - z) * s)[K, N] (+ bias[N]),  fp32 accumulate.
  * x, out, scales, bias share `dtype` (F16 or BF16); qweight is the slab
  * layout; scales [K/g, N]; group_size a multiple of 32 dividing K that divides
- * 128 or is a multiple of it (or -1 for one group).  M <= 64 runs the split-K
- * streaming kernel, larger M the LDS-staged MFMA kernels (groups of 32, 64 and
- * multiples of 128; other sizes go through the streaming kernel 32 rows at a
- * time), which split K over two kernels when their grid would leave most of
- * the chip idle.  bf16 activations of 65 rows or more on outputs of about two million
+ * 128 or is a multiple of it (or -1 for one group).  Up to 16 or 32 rows (by
+ * the layer) run the split-K streaming kernel, more the LDS-staged MFMA kernels
+ * (groups of 32, 64 and multiples of 128; other sizes go through the streaming
+ * kernel 32 rows at a time), which split K over two kernels when their grid
+ * would leave most of the chip idle.  bf16 activations of 65 rows or more on outputs of about two million
  * elements or more are first stored in the workspace as fp16 rows, each times a
  * power of two of its own (exact), and take the fp16 kernels (group sizes that
  * are multiples of 128, zero-points not pre-scaled); with a workspace too small
@@ -97,13 +97,12 @@ int mi355q_w4a16_gemm(void* out, const void* x, const int32_t* qweight,
  * factor, bits 8..15 the tiles (of 16 columns) per workgroup of the streaming
  * kernel (1, 2, 4 or 8); 0 in a field = automatic.  family: 0 = auto,
  * 1 = streaming, 2 = MFMA tiles of 64 rows (with groups of 64 and 32 family
- * 4's where the library takes those by itself), 3 = MFMA workgroups of up to
- * 128 rows fed through a ring of LDS stages (fp16, group sizes that are
- * multiples of 128; there bits 8..15 of split_k = 1 or 4 select workgroups of
- * 128 or 512 columns instead of 256; bf16 above 64 rows with the full workspace: the rows staged as
- * fp16, workgroups of 256 or 512 columns), 4 = MFMA workgroups of 32..96
- * rows x 64 or 128 columns (split_k bits 8..15: rows / 16, 16..23: columns /
- * 64; 0 = the library's choice). */
+ * 4's where the library takes those by itself), 3 = MFMA workgroups of 128
+ * rows x 256 columns fed through a ring of LDS stages (fp16, group sizes that
+ * are multiples of 128; there bits 8..15 of split_k = 4 select 512 columns;
+ * bf16 above 64 rows with the full workspace: the rows staged as fp16),
+ * 4 = MFMA workgroups of 32..96 rows x 64 or 128 columns (split_k bits
+ * 8..15: rows / 16, 16..23: columns / 64; 0 = the library's choice). */
 int mi355q_w4a16_gemm_ex(void* out, const void* x, const int32_t* qweight,
                          const void* scales, const void* zeros, int zeros_kind,
                          const void* bias, int M, int K, int N, int group_size,

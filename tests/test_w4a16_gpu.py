@@ -352,8 +352,7 @@ def test_tile_gemm_zero_kinds_and_group_256(ops, rearrange, zero_reading):
 @pytest.mark.parametrize("M", [33, 64, 100, 128])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_narrow_tiles_mid_rows(ops, rearrange, M, dtype):
-    """33..128 rows on layers up to 8192 wide run 32-row x 64-column workgroups (one tile per wavefront,
-    two K blocks in flight), with K split up to four ways on a narrow layer: packed, absent and float
+    """33..128 rows forced through the 64-row tiles, with K split on a narrow layer: packed, absent and float
     zero-points, group 128 and 256, bias, ragged last row block, exact inputs bit for bit."""
     print(f"case narrow tiles M={M} {dtype}", flush=True)
     for K, N, g in ((4096, 512, 128), (1024, 1152, 256)):
@@ -384,10 +383,9 @@ def test_narrow_tiles_mid_rows(ops, rearrange, M, dtype):
                                            (2048, 2048, 384, 128, 0)])
 @pytest.mark.parametrize("tw", [2, 1, 4])
 def test_ring_gemm_parity(ops, rearrange, M, K, N, g, split, tw):
-    """The kernel that owns up to 128 rows per workgroup and streams K through a ring of LDS stages
+    """The kernel that owns 128 rows per workgroup and streams K through a ring of LDS stages
     (fp16; B operands are (q - z) * s rounded to fp16), with two 16-column tiles per wavefront
-    (workgroups of 256 columns), with one (128 columns) and with four (512 columns, always 128 rows
-    per workgroup): ragged M, a half-empty last column tile and workgroups with whole slabs past N,
+    (workgroups of 256 columns; asked for one, too) and with four (512 columns): ragged M, a half-empty last column tile and workgroups with whole slabs past N,
     several row blocks, K split with the separate reduction, groups of 256, bias; run-to-run
     identical; exact inputs bit for bit (every scale a power of two, so the fp16 weights are exact)."""
     print(f"case ring M={M} K={K} N={N} g={g} split={split} tiles per wavefront={tw}", flush=True)
@@ -422,9 +420,8 @@ def test_ring_gemm_zero_kinds(ops, rearrange, M, tw, zero_reading):
 
 
 def test_mid_rows_take_the_ring_kernel_where_k_is_long(ops, rearrange):
-    """33..128 rows on a layer whose workgroups walk ten K blocks or more: the dispatcher takes the ring
-    kernel with 128-column workgroups and splits K four ways here (64 column tiles on 256 CUs).  Sampled
-    columns against the oracle, the forced 64-row tile kernel beside it, run-to-run identical."""
+    """33..128 rows on a layer of long K, whichever kernel the dispatcher takes: against the oracle, the
+    forced 64-row tile kernel beside it, run-to-run identical."""
     M, K, N, g = 96, 5120, 8192, 128
     print(f"case ring auto M={M} K={K} N={N}", flush=True)
     q, z, s, x = make_case(21, M, K, N, g)

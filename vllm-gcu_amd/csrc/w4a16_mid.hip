@@ -1,19 +1,17 @@
 // W4A16 MFMA GEMM in which every operand reaches the CU through a ring of LDS stages (fp16).
 //
-// One workgroup per CU owns all rows of a block (16 MT, up to 128) of 512, 256 or 128 columns and walks K
-// (or its share of K) in blocks of 128.  Everything a K block needs -- the activation rows, the packed
+// One workgroup per CU owns the 128 rows of a block of 512 or 256 columns and walks K (or its share of
+// K) in blocks of 128.  Everything a K block needs -- the activation rows, the packed
 // weights, the group scales and zero-points -- is copied from global memory straight into a ring of LDS
 // stages (global_load_lds, 16 B per lane, no staging registers) several K blocks ahead; the ring is the
 // latency cover that a second workgroup per CU provides in the 64-row tile kernel.  Each of the eight
 // wavefronts (two per SIMD: one wavefront alone issues an instruction every five or six clocks, too
-// few for the matrix pipe) owns all row tiles of TW = 4, 2 or 1 of the 16-column tiles: no weight is
+// few for the matrix pipe) owns all row tiles of TW = 4 or 2 of the 16-column tiles: no weight is
 // dequantised twice.  B operands are scaled, (q - z) * s rounded to fp16 -- the dequantised weight the
 // operator is defined on -- so the matrix instructions accumulate in place.
 //
-// Three uses: above 128 rows (TW = 2 or 4, workgroups of 256 or 512 columns, row blocks in blockIdx.y)
-// where a round model prices it below the 64-row tiles, and from 33 to 128 rows (TW = 1, workgroups of
-// 128 columns: twice the workgroups, so K needs half the splits) where a workgroup walks ten K blocks
-// or more.  With TW = 4 an activation operand read from LDS feeds four matrix instructions instead of
+// Used above 128 rows (TW = 2 or 4, workgroups of 256 or 512 columns, row blocks in blockIdx.y) where a
+// round model prices it below the 64-row tiles.  With TW = 4 an activation operand read from LDS feeds four matrix instructions instead of
 // two -- the LDS reads per matrix instruction fall from 0.75 to 0.5 and the copies per column from a
 // 128-row block of activations per 256 columns to one per 512 -- at the price of a ring of two stages
 // instead of three and of registers: the 128 accumulators of the 8 x 4 tiles leave room for a ring of
@@ -47,10 +45,10 @@ struct MidArgs {
   const uint32_t* scale_max;  // [64] largest scale magnitude (bf16 bits) of 64 slices of the scales array
 };
 
-// TW: 16-column tiles per wavefront -- 2: a workgroup of 256 columns; 4: of 512 columns (128 rows only);
-// 1: of 128 columns (one slab), for launches of up to 128 rows, where 256-column workgroups are too few
-// to fill the chip without splitting K
-template <int MT, int TW>
+constexpr int MT = 8;                                 // row tiles of 16 per workgroup
+
+// TW: 16-column tiles per wavefront -- 2: a workgroup of 256 columns; 4: of 512 columns
+template <int TW>
 struct MidCfg {
   static constexpr int BM = 16 * MT;
   static constexpr int BNW = 128 * TW;                // columns per workgroup
@@ -59,7 +57,7 @@ struct MidCfg {
   static constexpr int SZ_OFF = A_BYTES + 8192 * TW;  // 8 wavefronts x (256 B of scales + 256 B of zero-points)
   static constexpr int STAGE = A_BYTES + 8192 * TW + 4096;
   static constexpr int D = (160 * 1024 - 1024) / STAGE < 6 ? (160 * 1024 - 1024) / STAGE : 6;   // stages in the ring
-  static constexpr int XC = MT >= 2 ? MT / 2 : 1;     // activation copies (4 rows each) per wavefront and stage
+  static constexpr int XC = MT / 2;                   // activation copies (4 rows each) per wavefront and stage
 };
 
 // 64 lanes x 16 B from saddr + voff into LDS at lds_addr + 16 * lane
@@ -109,11 +107,11 @@ __device__ __forceinline__ uint32_t mid_dequant_pair(uint32_t w, int p, _Float16
 // brings the largest of them into [2^10, 2^11) -- (q - z) s stays below fp16's largest number and a
 // scale 2^24 below the largest one still keeps all its bits; the epilogue undoes both powers of two
 // exactly (one ldexp per output) and rounds to bf16.
-template <int ZK, int MT, int TW, bool IOBF = false>
+template <int ZK, int TW, bool IOBF>
 __global__ void __launch_bounds__(512, 1)
 w4a16_mid_kernel(MidArgs a) {
   static_assert(!IOBF || ZK != MI355Q_ZP_PRESCALED, "pre-scaled zero-points stay with the bf16 kernel");
-  typedef MidCfg<MT, TW> C;
+  typedef MidCfg<TW> C;
   constexpr int D = C::D, STAGE = C::STAGE, XC = C::XC;
   constexpr bool HASZ = ZK != MI355Q_ZP_NONE;
   constexpr int NSLOT = XC + TW + 1;                  // copy slots per wavefront and stage (the last: scales + zeros)
@@ -127,10 +125,10 @@ w4a16_mid_kernel(MidArgs a) {
   const int m0 = blockIdx.y * C::BM;
   // N may end in the middle of a 256-column tile: the wavefronts of the missing slab work on the
   // previous one and their columns are never stored
-  const int wslab = TW == 4 ? wave >> 1 : TW == 2 ? wave >> 2 : 0;   // slab of the workgroup this wavefront works on
+  const int wslab = TW == 4 ? wave >> 1 : wave >> 2;                 // slab of the workgroup this wavefront works on
   const bool live = (blockIdx.x * TW + wslab) < (N >> 7);
   const int slab = live ? blockIdx.x * TW + wslab : (N >> 7) - 1;
-  const int t0 = TW == 4 ? (wave & 1) * 4 : TW == 2 ? (wave & 3) * 2 : wave;   // first of this wavefront's TW tiles of the slab
+  const int t0 = TW == 4 ? (wave & 1) * 4 : (wave & 3) * 2;          // first of this wavefront's TW tiles of the slab
   const int gb = (int)blockIdx.z * a.kper, ge = min(G, gb + a.kper);
   const uint32_t lds_base =
       __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)lds);
@@ -204,14 +202,12 @@ w4a16_mid_kernel(MidArgs a) {
   struct Sz { uint2 s; uint2 zs; uint32_t z; };
   auto read_sz = [&](Sz& q, int slot) {
     const unsigned char* p = lds + slot * STAGE + C::SZ_OFF + wave * 512;
-    // (one tile per wavefront: t0 may be odd, the 32-bit read starts at the even column below it)
-    const int te = t0 & ~1;
     if (TW == 4) q.s = *(const uint2*)(p + (8 * c + t0) * 2);
-    else q.s.x = *(const uint32_t*)(p + (8 * c + te) * 2) >> (16 * (t0 & 1));
+    else q.s.x = *(const uint32_t*)(p + (8 * c + t0) * 2);
     if (ZK == MI355Q_ZP_PACKED) q.z = *(const uint32_t*)(p + 256 + c * 4) >> (4 * t0);
     if (ZK == MI355Q_ZP_PRESCALED) {
       if (TW == 4) q.zs = *(const uint2*)(p + 256 + (8 * c + t0) * 2);
-      else q.zs.x = *(const uint32_t*)(p + 256 + (8 * c + te) * 2) >> (16 * (t0 & 1));
+      else q.zs.x = *(const uint32_t*)(p + 256 + (8 * c + t0) * 2);
     }
   };
   // per column tile: scale, 1024 + z, 64 + z, z * s
@@ -327,7 +323,7 @@ w4a16_mid_kernel(MidArgs a) {
 #pragma unroll
           for (int q = 0; q < NP; ++q) {
             if (q * MT / NP != mt) continue;
-            if (k++ % TW != (TW == 1 ? 0 : (t + 1) % TW)) continue;
+            if (k++ % TW != (t + 1) % TW) continue;
             const int tt = q >> 2, p = q & 3;
             bv[nxt][tt][p] = mid_dequant_pair<ZK>(st < 3 ? wc[tt][st + 1] : wn[tt][0], p, zlo[tt], zhi[tt], sc[tt], zsc[tt], dqk);
           }
@@ -356,15 +352,13 @@ w4a16_mid_kernel(MidArgs a) {
   constexpr int EP = C::BNW * 4 + 16;                  // bytes per tile row in LDS
   constexpr int HALVES = TW == 4 ? 2 : 1, MTH = MT / HALVES;
   static_assert(16 * MTH * EP <= D * STAGE, "the output tile fits in the ring");
-  // 4 columns per lane: a wavefront instruction covers part of a row, one row or two rows
-  constexpr int LPR = C::BNW / 4;                      // lanes per row
-  constexpr int RPI = LPR >= 64 ? 1 : 64 / LPR, IPR = LPR >= 64 ? LPR / 64 : 1;   // rows per instruction, instructions per row
+  constexpr int IPR = C::BNW / 256;                    // instructions per row, 4 columns per lane
   typedef Elem<IOBF ? MI355Q_BF16 : MI355Q_F16> IO;
   f4 bs[IPR];
 #pragma unroll
   for (int q = 0; q < IPR; ++q) {
     bs[q] = (f4){0.f, 0.f, 0.f, 0.f};
-    const int col = blockIdx.x * C::BNW + 4 * (lane % LPR) + 256 * q;
+    const int col = blockIdx.x * C::BNW + 4 * lane + 256 * q;
     if (a.bias && !a.partial && col < N) {
       const uint2 bw = *(const uint2*)(a.bias + col);
       bs[q] = (f4){IO::to_f32((uint16_t)(bw.x & 0xffffu)), IO::to_f32((uint16_t)(bw.x >> 16)),
@@ -382,24 +376,23 @@ w4a16_mid_kernel(MidArgs a) {
         for (int i = 0; i < 4; ++i) {
           const int mt = h * MTH + mh;
           unsigned char* q = base + (mh * 16 + 4 * kq + i) * EP;
-          if (TW == 4) *(f4*)q = (f4){acc[mt][0][i], acc[mt][1 % TW][i], acc[mt][2 % TW][i], acc[mt][3 % TW][i]};
-          else if (TW == 2) *(f2*)q = (f2){acc[mt][0][i], acc[mt][TW - 1][i]};
-          else *(float*)q = acc[mt][0][i];
+          if (TW == 4) *(f4*)q = (f4){acc[mt][0][i], acc[mt][1][i], acc[mt][2 % TW][i], acc[mt][3 % TW][i]};
+          else *(f2*)q = (f2){acc[mt][0][i], acc[mt][1][i]};
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int p = 0; p < 2 * MTH / RPI; ++p) {
-      const int r = RPI * (wave + 8 * p) + (LPR >= 64 ? 0 : lane / LPR), m = m0 + h * 16 * MTH + r;
+    for (int p = 0; p < 2 * MTH; ++p) {
+      const int r = wave + 8 * p, m = m0 + h * 16 * MTH + r;
       if (m >= M) break;
       // IOBF: the row's power of two and the scales' in one exponent
       int back = 0;
       if (IOBF) back = (int)((bitcast<uint32_t>(a.row_scale[m]) >> 23) & 255u) - 127 - sshift;
 #pragma unroll
       for (int q = 0; q < IPR; ++q) {
-        const int col = blockIdx.x * C::BNW + 4 * (lane % LPR) + 256 * q;
+        const int col = blockIdx.x * C::BNW + 4 * lane + 256 * q;
         if (col >= N) continue;
-        f4 v = *(const f4*)(lds + r * EP + (lane % LPR) * 16 + 1024 * q);
+        f4 v = *(const f4*)(lds + r * EP + lane * 16 + 1024 * q);
         if (IOBF) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = __builtin_ldexpf(v[e], back);
@@ -417,56 +410,31 @@ w4a16_mid_kernel(MidArgs a) {
   }
 }
 
-template <int ZK, int MT, int TW>
-int launch_mid(const MidArgs& a, int row_blocks, int splits, hipStream_t st) {
-  typedef MidCfg<MT, TW> C;
+template <int ZK, int TW, bool IOBF>
+int launch_mid(const MidArgs& a, int splits, hipStream_t st) {
+  typedef MidCfg<TW> C;
   const size_t shmem = (size_t)C::D * C::STAGE;
-  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_mid_kernel<ZK, MT, TW>,
+  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_mid_kernel<ZK, TW, IOBF>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   MQ_REQUIRE(attr == hipSuccess, "w4a16_gemm(mid): cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
-  dim3 grid((a.N + C::BNW - 1) / C::BNW, row_blocks, splits);
-  hipLaunchKernelGGL((w4a16_mid_kernel<ZK, MT, TW>), grid, dim3(512), shmem, st, a);
+  dim3 grid((a.N + C::BNW - 1) / C::BNW, (a.M + C::BM - 1) / C::BM, splits);
+  hipLaunchKernelGGL((w4a16_mid_kernel<ZK, TW, IOBF>), grid, dim3(512), shmem, st, a);
   MQ_LAUNCH_CHECK("w4a16_gemm(mid)");
   return 0;
 }
 
-// bf16 rows staged as fp16: 128-row workgroups of 256 or 512 columns, no K split
-template <int ZK, int TW>
-int launch_mid_iobf(const MidArgs& a, int row_blocks, hipStream_t st) {
-  typedef MidCfg<8, TW> C;
-  const size_t shmem = (size_t)C::D * C::STAGE;
-  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_mid_kernel<ZK, 8, TW, true>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
-  MQ_REQUIRE(attr == hipSuccess, "w4a16_gemm(mid): cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
-  dim3 grid((a.N + C::BNW - 1) / C::BNW, row_blocks, 1);
-  hipLaunchKernelGGL((w4a16_mid_kernel<ZK, 8, TW, true>), grid, dim3(512), shmem, st, a);
-  MQ_LAUNCH_CHECK("w4a16_gemm(mid, bf16 staged)");
-  return 0;
-}
-
-template <int ZK>
-int launch_mid_mt(const MidArgs& a, int mt, int tw, int row_blocks, int splits, hipStream_t st) {
-  if (tw == 4) return launch_mid<ZK, 8, 4>(a, row_blocks, splits, st);
-  if (tw == 1) {
-    if (mt <= 2) return launch_mid<ZK, 2, 1>(a, row_blocks, splits, st);
-    if (mt <= 4) return launch_mid<ZK, 4, 1>(a, row_blocks, splits, st);
-    return launch_mid<ZK, 8, 1>(a, row_blocks, splits, st);
-  }
-  if (mt <= 2) return launch_mid<ZK, 2, 2>(a, row_blocks, splits, st);
-  if (mt <= 4) return launch_mid<ZK, 4, 2>(a, row_blocks, splits, st);
-  return launch_mid<ZK, 8, 2>(a, row_blocks, splits, st);
+template <int ZK, bool IOBF>
+int launch_mid_tw(const MidArgs& a, int tw, int splits, hipStream_t st) {
+  return tw == 4 ? launch_mid<ZK, 4, IOBF>(a, splits, st) : launch_mid<ZK, 2, IOBF>(a, splits, st);
 }
 
 }  // namespace
 
-// Row tiles of 16 per workgroup for M rows: the smallest of 2, 4, 8 that holds them all, 8 beyond.
-static int mid_rows_mt(int M) { return M <= 32 ? 2 : M <= 64 ? 4 : 8; }
-
 // K splits: as many as still fit the chip in one round (one workgroup per CU), each at least four K
 // blocks long and the partial tiles within 64 MiB.
 int w4a16_mid_splits(int M, int K, int N, int tw) {
-  const int mt = mid_rows_mt(M), G = K / 128, bn = 128 * tw;
-  const long wgs = (long)((M + 16 * mt - 1) / (16 * mt)) * ((N + bn - 1) / bn);
+  const int G = K / 128, bn = 128 * tw;
+  const long wgs = (long)((M + 127) / 128) * ((N + bn - 1) / bn);
   const long cus = device_cu_count();
   long s = cus / wgs;
   if (s > G / 4) s = G / 4;
@@ -474,11 +442,6 @@ int w4a16_mid_splits(int M, int K, int N, int tw) {
   if (s < 1) s = 1;
   const int kper = (int)((G + s - 1) / s);
   return (G + kper - 1) / kper;
-}
-
-size_t w4a16_mid_workspace_bytes(int M, int K, int N) {
-  const int s = w4a16_mid_splits(M, K, N, 2);
-  return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
 }
 
 // fp16 activations, group sizes that are multiples of 128.  `splits` 0: the plan above.
@@ -489,7 +452,7 @@ int w4a16_mid_launch(void* out, const void* x, const int32_t* qweight, const voi
              "w4a16_gemm(mid): fp16 and group sizes that are multiples of 128 only (dtype %d, group %d)", dtype, group_size);
   MQ_REQUIRE((size_t)M * K * 2 < ((size_t)1 << 32), "w4a16_gemm: activation matrix %d x %d is 4 GiB or more", M, K);
   const int G = K / 128;
-  if (tw != 1 && tw != 4) tw = 2;
+  if (tw != 4) tw = 2;
   if (splits <= 0) splits = w4a16_mid_splits(M, K, N, tw);
   if (splits > G) splits = G;
   if (splits > 1 && (!workspace || workspace_bytes < (size_t)splits * M * N * sizeof(float))) splits = 1;
@@ -506,12 +469,10 @@ int w4a16_mid_launch(void* out, const void* x, const int32_t* qweight, const voi
   a.gpk = (uint32_t)group_size / 128u;
   a.gpk_magic = a.gpk > 1 ? (uint32_t)((((uint64_t)1 << 32) + a.gpk - 1) / a.gpk) : 0u;
   a.partial = splits > 1 ? (float*)workspace : nullptr;
-  const int mt = mid_rows_mt(M);
-  const int row_blocks = (M + 16 * mt - 1) / (16 * mt);
   int rc;
-  if (zeros_kind == MI355Q_ZP_NONE) rc = launch_mid_mt<MI355Q_ZP_NONE>(a, mt, tw, row_blocks, splits, st);
-  else if (zeros_kind == MI355Q_ZP_PACKED) rc = launch_mid_mt<MI355Q_ZP_PACKED>(a, mt, tw, row_blocks, splits, st);
-  else rc = launch_mid_mt<MI355Q_ZP_PRESCALED>(a, mt, tw, row_blocks, splits, st);
+  if (zeros_kind == MI355Q_ZP_NONE) rc = launch_mid_tw<MI355Q_ZP_NONE, false>(a, tw, splits, st);
+  else if (zeros_kind == MI355Q_ZP_PACKED) rc = launch_mid_tw<MI355Q_ZP_PACKED, false>(a, tw, splits, st);
+  else rc = launch_mid_tw<MI355Q_ZP_PRESCALED, false>(a, tw, splits, st);
   if (rc) return rc;
   if (splits > 1) return w4a16_splitk_reduce_launch(out, (const float*)workspace, bias, M, N, splits, dtype, st);
   return 0;
@@ -538,10 +499,8 @@ int w4a16_mid_launch_staged(void* out, const void* x16, const int32_t* qweight, 
   a.gpk_magic = a.gpk > 1 ? (uint32_t)((((uint64_t)1 << 32) + a.gpk - 1) / a.gpk) : 0u;
   a.row_scale = row_scale;
   a.scale_max = scale_max;
-  const int row_blocks = (M + 127) / 128;
-  if (zeros_kind == MI355Q_ZP_NONE)
-    return tw == 4 ? launch_mid_iobf<MI355Q_ZP_NONE, 4>(a, row_blocks, st) : launch_mid_iobf<MI355Q_ZP_NONE, 2>(a, row_blocks, st);
-  return tw == 4 ? launch_mid_iobf<MI355Q_ZP_PACKED, 4>(a, row_blocks, st) : launch_mid_iobf<MI355Q_ZP_PACKED, 2>(a, row_blocks, st);
+  return zeros_kind == MI355Q_ZP_NONE ? launch_mid_tw<MI355Q_ZP_NONE, true>(a, tw, 1, st)
+                                      : launch_mid_tw<MI355Q_ZP_PACKED, true>(a, tw, 1, st);
 }
 
 }  // namespace mi355q
