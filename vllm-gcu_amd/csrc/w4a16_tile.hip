@@ -643,18 +643,22 @@ hipError_t launch_zk(const TileArgs& a, int zk, int row_blocks, hipStream_t st) 
     // fp32 group scales: symmetric int4 experts only
     if (a.scales_f32) return launch_one<DT, MI355Q_ZP_NONE, MT, true, true>(a, row_blocks, st);
   }
-  if (zk == MI355Q_ZP_NONE) return launch_one<DT, MI355Q_ZP_NONE, MT, GROUPED>(a, row_blocks, st);
-  if (zk == MI355Q_ZP_PACKED) return launch_one<DT, MI355Q_ZP_PACKED, MT, GROUPED>(a, row_blocks, st);
-  return launch_one<DT, MI355Q_ZP_PRESCALED, MT, GROUPED>(a, row_blocks, st);
+  if constexpr (GROUPED && MT <= 2) {
+    return hipErrorInvalidValue;                     // (blocks of 16 and 32 slots with 16-bit scales run other kernels)
+  } else {
+    if (zk == MI355Q_ZP_NONE) return launch_one<DT, MI355Q_ZP_NONE, MT, GROUPED>(a, row_blocks, st);
+    if (zk == MI355Q_ZP_PACKED) return launch_one<DT, MI355Q_ZP_PACKED, MT, GROUPED>(a, row_blocks, st);
+    return launch_one<DT, MI355Q_ZP_PRESCALED, MT, GROUPED>(a, row_blocks, st);
+  }
 }
 
-template <int DT, bool GROUPED>
-hipError_t launch_mt(const TileArgs& a, int zk, int mt, int row_blocks, hipStream_t st) {
+template <int DT>
+hipError_t launch_blocks(const TileArgs& a, int zk, int mt, int row_blocks, hipStream_t st) {
   switch (mt) {
-    case 1: return launch_zk<DT, 1, GROUPED>(a, zk, row_blocks, st);
-    case 2: return launch_zk<DT, 2, GROUPED>(a, zk, row_blocks, st);
-    case 4: return launch_zk<DT, 4, GROUPED>(a, zk, row_blocks, st);
-    default: return launch_zk<DT, 8, GROUPED>(a, zk, row_blocks, st);
+    case 1: return launch_zk<DT, 1, true>(a, zk, row_blocks, st);
+    case 2: return launch_zk<DT, 2, true>(a, zk, row_blocks, st);
+    case 4: return launch_zk<DT, 4, true>(a, zk, row_blocks, st);
+    default: return launch_zk<DT, 8, true>(a, zk, row_blocks, st);
   }
 }
 
@@ -812,19 +816,13 @@ int w4a16_splitk_reduce_launch(void* out, const float* partial, const void* bias
 // bring the grid to about one workgroup per CU, at least 4 K blocks each, and
 // partial tiles of at most TILE_SPLITK_BYTES in total
 constexpr size_t TILE_SPLITK_BYTES = (size_t)64 << 20;
-static int tile_rows_mt(int M, int N) {
+static int tile_splits(int M, int K, int N) {
   // 64-row tiles for every dense shape: four wavefronts on the pipelined loop, two workgroups
   // per CU -- measured equal or faster than 128-row tiles of eight wavefronts from M = 65 to
   // 8192 (M = 2048: qkv 134 -> 112 us, gate_up 461 -> 449 us), fp16 and bf16
-  (void)M;
-  (void)N;
-  return 4;
-}
-static int tile_splits(int M, int K, int N) {
-  const int mt = tile_rows_mt(M, N), G = K / 128;
-  const long wgs = (long)((M + 16 * mt - 1) / (16 * mt)) * ((N + BN - 1) / BN);
-  // 64-row tiles run two workgroups per CU
-  const long target = (long)device_cu_count() * (mt == 4 ? 2 : 1);
+  const int G = K / 128;
+  const long wgs = (long)((M + 63) / 64) * ((N + BN - 1) / BN);
+  const long target = 2L * device_cu_count();
   long s;
   if (wgs * 5 >= target * 2) {
     // 40 % of a round or more (a wide layer at about a hundred rows: N 28672, M 128: 47 -> 43 us
@@ -832,12 +830,12 @@ static int tile_splits(int M, int K, int N) {
     // of the time of two that share one, so between 1/2 and 0.7 of a round over a long K three
     // splits (two even rounds of a third of K) beat one uneven round: K 14336, N 4096,
     // M 1100..1280: 203 -> 167..175 us; above that, and for K 4096, no split count gained.
-    if (mt != 4 || wgs * 10 > target * 7 || G < 64) return 1;
+    if (wgs * 10 > target * 7 || G < 64) return 1;
     s = 3;
   } else {
-    // 128-row tiles: the nearest count; 64-row tiles must all be resident at once (a second
-    // round of a few workgroups would double the time), so never above the target
-    s = mt == 4 ? target / wgs : (target + wgs / 2) / wgs;
+    // they must all be resident at once (a second round of a few workgroups would double the
+    // time), so never above the target
+    s = target / wgs;
   }
   if (s > G / 4) s = G / 4;
   while (s > 1 && (size_t)s * M * N * sizeof(float) > TILE_SPLITK_BYTES) --s;
@@ -1045,10 +1043,9 @@ static int tile_launch_dense(void* out, const void* x, const int32_t* qweight, c
   a.zeros = zeros;
   a.bias = (const uint16_t*)bias;
   a.M = M; a.K = K; a.N = N; a.gs = group_size;
-  const int mt = tile_rows_mt(M, N);
   const int G = K / 128;
   int splits = tile_splits(M, K, N);
-  const int row_blocks = (M + 16 * mt - 1) / (16 * mt);
+  const int row_blocks = (M + 63) / 64;
   if (splits > 1 && (!workspace || workspace_bytes < (size_t)splits * M * N * sizeof(float))) splits = 1;
   a.kper = (G + splits - 1) / splits;
   splits = (G + a.kper - 1) / a.kper;                // no empty splits
@@ -1060,8 +1057,8 @@ static int tile_launch_dense(void* out, const void* x, const int32_t* qweight, c
     e = (dtype == MI355Q_F16) ? launch_small_groups<MI355Q_F16, 4, false>(a, zeros_kind, 128 / group_size, row_blocks, st)
                               : launch_small_groups<MI355Q_BF16, 4, false>(a, zeros_kind, 128 / group_size, row_blocks, st);
   else
-    e = (dtype == MI355Q_F16) ? launch_mt<MI355Q_F16, false>(a, zeros_kind, mt, row_blocks, st)
-                              : launch_mt<MI355Q_BF16, false>(a, zeros_kind, mt, row_blocks, st);
+    e = (dtype == MI355Q_F16) ? launch_zk<MI355Q_F16, 4, false>(a, zeros_kind, row_blocks, st)
+                              : launch_zk<MI355Q_BF16, 4, false>(a, zeros_kind, row_blocks, st);
   MQ_REQUIRE(e == hipSuccess, "w4a16_gemm(tile): cannot reserve LDS: %s", hipGetErrorString(e));
   MQ_LAUNCH_CHECK("w4a16_gemm(tile)");
   if (splits > 1) return splitk_reduce_rows_launch(out, (const float*)workspace, bias, M, N, splits, dtype, st, row_scale);
@@ -1204,8 +1201,8 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
       e = (dtype == MI355Q_F16) ? launch_small_groups<MI355Q_F16, 8, true>(a, zeros_kind, gpb, max_blocks, st)
                                 : launch_small_groups<MI355Q_BF16, 8, true>(a, zeros_kind, gpb, max_blocks, st);
   } else {
-    e = (dtype == MI355Q_F16) ? launch_mt<MI355Q_F16, true>(a, zeros_kind, block_size / 16, max_blocks, st)
-                              : launch_mt<MI355Q_BF16, true>(a, zeros_kind, block_size / 16, max_blocks, st);
+    e = (dtype == MI355Q_F16) ? launch_blocks<MI355Q_F16>(a, zeros_kind, block_size / 16, max_blocks, st)
+                              : launch_blocks<MI355Q_BF16>(a, zeros_kind, block_size / 16, max_blocks, st);
   }
   MQ_REQUIRE(e == hipSuccess, "moe_w4a16: cannot reserve LDS: %s", hipGetErrorString(e));
   MQ_LAUNCH_CHECK("moe_w4a16");
