@@ -42,6 +42,7 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef int i4 __attribute__((ext_vector_type(4)));
+typedef int i8v __attribute__((ext_vector_type(8)));
 typedef int i16v __attribute__((ext_vector_type(16)));
 typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
@@ -130,6 +131,43 @@ __device__ __forceinline__ u4 buf_load16(rsrc_t r, uint32_t off) {
 __device__ __forceinline__ u4 buf_load16_nt(rsrc_t r, uint32_t off) {
   return bitcast<u4>(__builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 2));
 }
+
+// Copies straight from global memory into LDS, 64 lanes x 16 (or 4) bytes, no registers between: lane l lands at the
+// wavefront's LDS base + 16 l (4 l).  dma16 is the compiler's form, from an address per lane.  The others are inline
+// assembly, from a 32-bit byte offset per lane and a base per wavefront: the compiler does not see them, places its waits
+// for the LDS reads alone, and the kernel waits for the copies by hand (vmcnt).
+__device__ __forceinline__ void dma16(const void* gptr, void* lds_wave_base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gptr,
+                                   (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
+}
+__device__ __forceinline__ void lds_copy16(uint32_t voff, const void* sbase, uint32_t lds_addr) {
+  // (uniform by construction; inside a divergent region the compiler may otherwise keep it in a vector register)
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+}
+__device__ __forceinline__ void lds_copy4(uint32_t voff, const void* sbase, uint32_t lds_addr) {
+  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+}
+// to lds_addr + more, both in scalar registers already
+__device__ __forceinline__ void lds_copy16(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr), "s"(more) : "memory", "scc");
+}
+__device__ __forceinline__ void lds_copy4(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr), "s"(more) : "memory", "scc");
+}
+template <int OFF>
+__device__ __forceinline__ void lds_copy16_next(uint32_t voff, const void* sbase) {   // the m0 of the copy before; OFF counts on both sides
+  asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
+}
+
+// Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles (ordered by column), so that the row tiles
+// of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
+__device__ __forceinline__ int xcd_tile() {
+  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
+  return x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
+}
+
 // Wavefront reductions on the data-parallel-primitive path (lane shifts inside the vector ALU, no trip
 // through the LDS crossbar).  Every lane of the wavefront must be active.
 // Whole wavefront: an inclusive scan within each row of 16 lanes (shifts by 1, 2, 4, 8; lanes a shift
@@ -237,5 +275,21 @@ __device__ __forceinline__ float block_max(float x, float* red) {
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 int device_cu_count();
+
+// The plan of a shape, remembered per thread: a serving loop asks for the same few again and again, from the host path and
+// from the entry points.  `make` is a captureless lambda at one place in the source, so each has a table of its own.
+template <typename Make>
+auto cached_plan(int kind, int M, int N, int K, Make make) -> decltype(make(kind, M, N, K)) {
+  struct Entry {
+    int kind, M, N, K, cus;
+    decltype(make(kind, M, N, K)) plan;
+  };
+  static thread_local Entry table[64] = {};
+  const uint32_t h = ((uint32_t)M * 2654435761u ^ (uint32_t)N * 40503u ^ (uint32_t)K * 2246822519u ^ (uint32_t)kind) >> 7;
+  Entry& e = table[h % 64];
+  const int cus = device_cu_count();
+  if (e.M != M || e.N != N || e.K != K || e.kind != kind || e.cus != cus) e = {kind, M, N, K, cus, make(kind, M, N, K)};
+  return e.plan;
+}
 
 }  // namespace mi355q

@@ -68,12 +68,6 @@ struct F8Args {
   long w_stride, ws_stride;    // per expert: bytes of weights, floats of weight scales
 };
 
-__device__ __forceinline__ void dma16(const void* gptr, void* lds_wave_base) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gptr,
-                                   (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
-}
-typedef int i8v __attribute__((ext_vector_type(8)));
-
 // origin of an output tile of BM x 128 (split K: of an output tile and K range)
 template <bool GROUPED, int BM>
 __device__ __forceinline__ void f8_tile_origin(const F8Args& a, int mtiles, int ntiles_n, int ksplits, int tile, int& m0, int& n0) {
@@ -476,15 +470,6 @@ fp8_pc_gemm_kernel(F8Args a) {
 // barrier lies before them, where the stage before has been read and the next one is needed.
 // (us, before -> here: K 7168 x N 4096 at 1537 / 2048 rows 71.6 -> 58.3 / 69.6 -> 60.3; K 2048 x N 7168 at 1537 45.8 -> 40.1;
 // K 4096 x N 28672 at 1024 153.7 -> 133.5; K 8192 x N 28672 at 2048 520 -> 469)
-__device__ __forceinline__ void f8_copy16(uint32_t voff, const void* sbase, uint32_t lds_addr) {
-  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
-}
-// 64 x 4 B: lane l lands at base + 4 l
-__device__ __forceinline__ void f8_copy4(uint32_t voff, const void* sbase, uint32_t lds_addr) {
-  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
-}
 // x, w, a scale per row (1 KiB) and the tile's weight scale, 64 times
 constexpr int f8_stage_bytes(int BM) { return BM * FTKB + FTN * FTKB + 1024 + 256; }
 
@@ -591,12 +576,12 @@ fp8_block_gemm_kernel(F8Args a) {
     auto copy_stage = [&](int stage) {
       const uint32_t xs = lds_base + (uint32_t)(stage * STAGE_BYTES);
 #pragma unroll
-      for (int p = 0; p < XCOPIES; ++p) f8_copy16(xo[p], xtile + (long)kt * FTKB, xs + (uint32_t)((wave + 4 * p) * 1024));
+      for (int p = 0; p < XCOPIES; ++p) lds_copy16(xo[p], xtile + (long)kt * FTKB, xs + (uint32_t)((wave + 4 * p) * 1024));
       const long koff = a.w_kslab ? (long)kt * FTKB * 64 : (long)kt * FTKB;
 #pragma unroll
-      for (int p = 0; p < WCOPIES; ++p) f8_copy16(wo[p], wtile + koff, xs + (uint32_t)(X_BYTES + (wave + 4 * p) * 1024));
-      f8_copy4(xso * 4u, xsbase + (long)kt * xs_kstride, xs + (uint32_t)(X_BYTES + W_BYTES + wave * 256));
-      if (wave == 0) f8_copy4(0u, a.w_scale + wsbase + kt, xs + (uint32_t)(X_BYTES + W_BYTES + 1024));
+      for (int p = 0; p < WCOPIES; ++p) lds_copy16(wo[p], wtile + koff, xs + (uint32_t)(X_BYTES + (wave + 4 * p) * 1024));
+      lds_copy4(xso * 4u, xsbase + (long)kt * xs_kstride, xs + (uint32_t)(X_BYTES + W_BYTES + wave * 256));
+      if (wave == 0) lds_copy4(0u, a.w_scale + wsbase + kt, xs + (uint32_t)(X_BYTES + W_BYTES + 1024));
       if (++kt == nt) {
         if (tile + gdim < total_tiles) {
           tile += gdim;

@@ -54,20 +54,10 @@ struct Q8Args {
   void* partial;            // split K: f32 / int32 sums [range][M][N]; null: write the output
 };
 
-__device__ __forceinline__ void q8_dma16(uint32_t voff, const void* sbase, uint32_t lds_addr) {
-  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
-}
-__device__ __forceinline__ void q8_dma4(uint32_t voff, const void* sbase, uint32_t lds_addr) {
-  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
-}
 template <int N>
 __device__ __forceinline__ void q8_wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");   // (and no LDS read of the stage before is open)
 }
-
-typedef int i8v __attribute__((ext_vector_type(8)));
 
 // wavefronts WM x WN, each 16 NJ rows of x by 16 NI rows of w
 template <int WM_, int WN_, int NJ_, int NI_, int D_>
@@ -123,10 +113,7 @@ q8_mid_kernel(Q8Args a) {
   const int l16 = lane & 15, kq = lane >> 4;
   const int wm = wave / C::WN, wn = wave % C::WN;
   const int M = a.M, N = a.N, KB = a.K >> 7;
-  // Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles, ordered by column, so that the
-  // row tiles of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
-  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
-  const int t = x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
+  const int t = xcd_tile();
   const int tn = t / a.mtiles, tm = t - tn * a.mtiles;
   const int m0 = tm * C::BM, n0 = tn * C::BN;
   const int kb0 = blockIdx.y * a.kper, nk = min(KB - kb0, a.kper);
@@ -149,10 +136,10 @@ q8_mid_kernel(Q8Args a) {
     const int kb = min(i, nk - 1);                    // past the end: a re-read into a stage nobody reads
     const uint32_t sb = lds_base + (uint32_t)(slot * C::STAGE);
     if (p < C::XC) {
-      q8_dma16(xo[p < C::XC ? p : 0], xg + (long)kb * 128, sb + (uint32_t)((wave + C::WAVES * p) * 1024));
+      lds_copy16(xo[p < C::XC ? p : 0], xg + (long)kb * 128, sb + (uint32_t)((wave + C::WAVES * p) * 1024));
     } else {
       const int c = wave + C::WAVES * (p - C::XC);
-      q8_dma16(lane16, wg + ((long)(c >> 3) * KB + kb) * 8192 + (c & 7) * 1024, sb + (uint32_t)(C::X_BYTES + c * 1024));
+      lds_copy16(lane16, wg + ((long)(c >> 3) * KB + kb) * 8192 + (c & 7) * 1024, sb + (uint32_t)(C::X_BYTES + c * 1024));
     }
   };
   if (MODE == Q8_BLOCK) {
@@ -160,12 +147,12 @@ q8_mid_kernel(Q8Args a) {
     const int total = C::BM * pitch;
     for (int p0 = wave * 64; p0 < total; p0 += C::THREADS) {
       const int p = min(p0 + lane, total - 1), r = p / pitch, kb = min(p - r * pitch, nk - 1);
-      q8_dma4((uint32_t)((min(m0 + r, M - 1) - m0) * KB + kb) * 4u, a.x_scale + (long)m0 * KB + kb0,
+      lds_copy4((uint32_t)((min(m0 + r, M - 1) - m0) * KB + kb) * 4u, a.x_scale + (long)m0 * KB + kb0,
               lds_base + scales_off + (uint32_t)p0 * 4u);
     }
     const uint32_t ws_off = scales_off + (uint32_t)((total + 63) / 64 * 64) * 4u;
     for (int p0 = wave * 64; p0 < nk; p0 += C::THREADS)
-      q8_dma4((uint32_t)min(p0 + lane, nk - 1) * 4u, a.w_scale + (long)(n0 >> 7) * KB + kb0, lds_base + ws_off + (uint32_t)p0 * 4u);
+      lds_copy4((uint32_t)min(p0 + lane, nk - 1) * 4u, a.w_scale + (long)(n0 >> 7) * KB + kb0, lds_base + ws_off + (uint32_t)p0 * 4u);
   }
 #pragma unroll
   for (int d = 0; d < D; ++d)
@@ -282,16 +269,6 @@ q8_mid_kernel(Q8Args a) {
 // (us, eight wavefronts that do both on 128 x 128 or four on 64 x 64 -> here; fp8 block 7168 x 4096 at 512 rows 31.4 -> 26.9,
 // 8192 x 8192 at 256 / 512 40.8 / 61.9 -> 33.6 / 52.5, 4096 x 6144 at 256 / 512 19.6 / 31.1 -> 16.3 / 24.7; int8 7168 x 4096 at 512
 // 31.5 -> 25.0, 14336 x 4096 at 256 36.0 -> 30.6)
-__device__ __forceinline__ void q8_copy16(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
-  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr), "s"(more) : "memory", "scc");
-}
-template <int OFF>
-__device__ __forceinline__ void q8_copy16_next(uint32_t voff, const void* sbase) {   // the same m0; the offset counts on both sides
-  asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
-}
-__device__ __forceinline__ void q8_copy4(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
-  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr), "s"(more) : "memory", "scc");
-}
 
 // 16 NJ rows x 128 columns
 template <int NJ_, bool BLOCK>
@@ -315,10 +292,7 @@ q8_wide_kernel(Q8Args a) {
   const int wave = copies ? (wg - C::CW) % 2 : wg % NW, ks = copies ? (wg - C::CW) / 2 : wg / NW;
   const int l16 = lane & 15, kq = lane >> 4;
   const int M = a.M, N = a.N, KB = a.K >> 7;
-  // Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles, ordered by column, so that the
-  // row tiles of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
-  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
-  const int t = x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
+  const int t = xcd_tile();
   const int tn = t / a.mtiles, tm = t - tn * a.mtiles;
   const int m0 = tm * C::BM, n0 = tn * C::BN;
   const int g0 = (int)blockIdx.y * a.kper, ng = min(KB - g0, a.kper);
@@ -354,16 +328,16 @@ q8_wide_kernel(Q8Args a) {
       const uint32_t sb = ring + (uint32_t)(slot * C::STAGE);
 #pragma unroll
       for (int g = 0; g < NI; ++g) {
-        q8_copy16(lane16, wgp + (long)g * KB * 8192, sb, (uint32_t)(C::X_BYTES + g * 8192 + wave * 4096));
-        q8_copy16_next<1024>(lane16, wgp + (long)g * KB * 8192);
-        q8_copy16_next<2048>(lane16, wgp + (long)g * KB * 8192);
-        q8_copy16_next<3072>(lane16, wgp + (long)g * KB * 8192);
+        lds_copy16(lane16, wgp + (long)g * KB * 8192, sb, (uint32_t)(C::X_BYTES + g * 8192 + wave * 4096));
+        lds_copy16_next<1024>(lane16, wgp + (long)g * KB * 8192);
+        lds_copy16_next<2048>(lane16, wgp + (long)g * KB * 8192);
+        lds_copy16_next<3072>(lane16, wgp + (long)g * KB * 8192);
       }
 #pragma unroll
-      for (int p = 0; p < NJ; ++p) q8_copy16(xo[p], xg, sb, (uint32_t)((wave + 2 * p) * 1024));
+      for (int p = 0; p < NJ; ++p) lds_copy16(xo[p], xg, sb, (uint32_t)((wave + 2 * p) * 1024));
       if constexpr (MODE == Q8_BLOCK) {
 #pragma unroll
-        for (int p = 0; p < C::SC; ++p) q8_copy4(so[p], sg, sb, (uint32_t)(C::S_OFF + (wave == 0 ? 256 * p : 256 * C::SC)));
+        for (int p = 0; p < C::SC; ++p) lds_copy4(so[p], sg, sb, (uint32_t)(C::S_OFF + (wave == 0 ? 256 * p : 256 * C::SC)));
       }
       if (kb < klast) {
         ++kb;
@@ -638,19 +612,7 @@ Q8Plan q8_make_plan(int mode, int M, int N, int K) {
   return best;
 }
 
-// (a serving loop asks for the same few shapes again and again, from the host path and from the entry points)
-Q8Plan q8_plan(int mode, int M, int N, int K) {
-  struct Entry {
-    int mode, M, N, K, dev_cus;
-    Q8Plan plan;
-  };
-  static thread_local Entry table[64] = {};
-  const uint32_t h = ((uint32_t)M * 2654435761u ^ (uint32_t)N * 40503u ^ (uint32_t)K * 2246822519u ^ (uint32_t)mode) >> 7;
-  Entry& e = table[h % 64];
-  const int cus = device_cu_count();
-  if (e.M != M || e.N != N || e.K != K || e.mode != mode || e.dev_cus != cus) e = {mode, M, N, K, cus, q8_make_plan(mode, M, N, K)};
-  return e.plan;
-}
+Q8Plan q8_plan(int mode, int M, int N, int K) { return cached_plan(mode, M, N, K, [](int m, int M, int N, int K) { return q8_make_plan(m, M, N, K); }); }
 
 }  // namespace
 

@@ -60,16 +60,6 @@ struct MidCfg {
   static constexpr int XC = MT / 2;                   // activation copies (4 rows each) per wavefront and stage
 };
 
-// 64 lanes x 16 B from saddr + voff into LDS at lds_addr + 16 * lane
-__device__ __forceinline__ void dma16(uint32_t voff, const void* sbase, uint32_t lds_addr) {
-  // (uniform by construction; inside a divergent region the compiler may otherwise keep it in a vector register)
-  lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(voff), "s"(sbase), "s"(lds_addr)
-               : "memory");
-}
-
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
@@ -174,15 +164,15 @@ w4a16_mid_kernel(MidArgs a) {
     int gq = rot + min(i, nk - 1);                    // past the end: a re-read into a stage nobody reads
     gq = gb + (gq >= nk ? gq - nk : gq);
     if (s < XC) {
-      dma16(xo[s < XC ? s : 0], xg + (size_t)gq * 256, sb + (uint32_t)((wave + 8 * s) * 1024));
+      lds_copy16(xo[s < XC ? s : 0], xg + (size_t)gq * 256, sb + (uint32_t)((wave + 8 * s) * 1024));
     } else if (s < XC + TW) {
       const int t = s - XC;
-      dma16(lane16, wg + (size_t)gq * 8192 + t * 1024, sb + (uint32_t)(C::W_OFF + wave * 1024 * TW + t * 1024));
+      lds_copy16(lane16, wg + (size_t)gq * 8192 + t * 1024, sb + (uint32_t)(C::W_OFF + wave * 1024 * TW + t * 1024));
     } else {
       const uint32_t qrow = a.gpk_magic ? (uint32_t)(((uint64_t)(uint32_t)gq * a.gpk_magic) >> 32) : (uint32_t)gq;
       if (lane < 16) {
-        dma16(lane16, sg + (size_t)qrow * N * 2, sb + (uint32_t)(C::SZ_OFF + wave * 512));
-        if (HASZ) dma16(zlane, zg + (size_t)qrow * zrow, sb + (uint32_t)(C::SZ_OFF + wave * 512 + 256));
+        lds_copy16(lane16, sg + (size_t)qrow * N * 2, sb + (uint32_t)(C::SZ_OFF + wave * 512));
+        if (HASZ) lds_copy16(zlane, zg + (size_t)qrow * zrow, sb + (uint32_t)(C::SZ_OFF + wave * 512 + 256));
       }
     }
   };

@@ -57,14 +57,6 @@ struct RowsArgs {
   long w_stride, s_stride, z_stride;   // bytes per expert
 };
 
-__device__ __forceinline__ void rows_dma16(uint32_t voff, const void* sbase, uint32_t lds_addr, uint32_t more) {
-  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_addr), "s"(more) : "memory", "scc");
-}
-template <int OFF>
-__device__ __forceinline__ void rows_dma16_next(uint32_t voff, const void* sbase) {   // the same m0; the offset counts on both sides
-  asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
-}
-
 struct RowsDq {
   uint32_t magic, mlo, mhi;
 };
@@ -171,13 +163,13 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
     auto copy_stage = [&](int slot) {
       const uint32_t sb = ring + (uint32_t)(slot * STAGE);
 #pragma unroll
-      for (int p = 0; p < C::XC; ++p) rows_dma16(xo[p], xg, sb, (uint32_t)((wave + 2 * p) * 1024));
-      rows_dma16(lane16, qg, sb, (uint32_t)(C::W_OFF + wave * C::WC * 1024));
-      if constexpr (C::WC > 1) rows_dma16_next<1024>(lane16, qg);
-      if constexpr (C::WC > 2) rows_dma16_next<2048>(lane16, qg);
-      if constexpr (C::WC > 3) rows_dma16_next<3072>(lane16, qg);
+      for (int p = 0; p < C::XC; ++p) lds_copy16(xo[p], xg, sb, (uint32_t)((wave + 2 * p) * 1024));
+      lds_copy16(lane16, qg, sb, (uint32_t)(C::W_OFF + wave * C::WC * 1024));
+      if constexpr (C::WC > 1) lds_copy16_next<1024>(lane16, qg);
+      if constexpr (C::WC > 2) lds_copy16_next<2048>(lane16, qg);
+      if constexpr (C::WC > 3) lds_copy16_next<3072>(lane16, qg);
       const uint32_t row = GPB > 1 ? (uint32_t)kb * GPB : a.gpk_magic ? (uint32_t)(((uint64_t)kb * a.gpk_magic) >> 32) : (uint32_t)kb;
-      if (lane < szlanes) rows_dma16(szoff, szg + (size_t)row * szrow, sb, szlds);
+      if (lane < szlanes) lds_copy16(szoff, szg + (size_t)row * szrow, sb, szlds);
       if (kb < klast) {                               // (past the end: a re-read into a stage nobody reads)
         ++kb;
         xg += 256;
@@ -350,10 +342,7 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
 template <int DT, int ZK, typename C>
 __global__ void __launch_bounds__(C::THREADS, (C::PAIR + 1) * C::THREADS / 256)
 w4a16_rows_kernel(RowsArgs a) {
-  // Workgroups go to the eight XCDs in turn: XCD x takes the x-th eighth of the tiles, ordered by column, so that the
-  // row tiles of a column tile share one L2 and its weights pass it once, whatever the number of column tiles
-  const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;
-  const int t = x8 * share + min(x8, odd) + ((int)blockIdx.x >> 3);
+  const int t = xcd_tile();
   const int tn = t / a.mtiles, tm = t - tn * a.mtiles;
   const int g0 = (int)blockIdx.y * a.kper;
   rows_tile<DT, ZK, C, false>(a, nullptr, tm * C::BM, tn, g0, min((a.K >> 7) - g0, a.kper));
@@ -458,19 +447,7 @@ RowsPlan rows_make_plan(int M, int K, int N, bool split) {
   return best;
 }
 
-// (a serving loop asks for the same few shapes again and again, from the host path and from the entry points)
-RowsPlan rows_plan(int M, int K, int N) {
-  struct Entry {
-    int M, N, K, cus;
-    RowsPlan plan;
-  };
-  static thread_local Entry table[64] = {};
-  const uint32_t h = ((uint32_t)M * 2654435761u ^ (uint32_t)N * 40503u ^ (uint32_t)K * 2246822519u) >> 7;
-  Entry& e = table[h % 64];
-  const int cus = device_cu_count();
-  if (e.M != M || e.N != N || e.K != K || e.cus != cus) e = {M, N, K, cus, rows_make_plan(M, K, N, true)};
-  return e.plan;
-}
+RowsPlan rows_plan(int M, int K, int N) { return cached_plan(0, M, N, K, [](int, int M, int N, int K) { return rows_make_plan(M, K, N, true); }); }
 
 template <int DT, int ZK, int GPB, int MAX>
 int launch_rows_grouped(const RowsArgs& a, int max_blocks, hipStream_t st) {

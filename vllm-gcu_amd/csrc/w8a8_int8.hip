@@ -77,13 +77,6 @@ __device__ __forceinline__ float load_bias(const void* bias, int bias_f32, int n
   return Elem<DT == MI355Q_F32 ? MI355Q_F16 : DT>::to_f32(((const uint16_t*)bias)[n]);
 }
 
-// one wavefront instruction copies 64 x 16 B from global memory straight into
-// 1 KiB of LDS (lane l lands at base + 16 l); no registers, no LDS store
-__device__ __forceinline__ void dma16(const void* gptr, void* lds_wave_base) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gptr,
-                                   (__attribute__((address_space(3))) void*)lds_wave_base, 16, 0, 0);
-}
-
 // WM x WN wavefronts, each NJ x NI MFMA tiles of 16 x 16 (rows of x by rows of w)
 // GROUPED: the fused-MoE grouped GEMM at prefill token counts.  Row tile b is align block b (256 slot
 // ids of expert expert_ids[b]): x rows are gathered through the ids (row id / topk), weights and
