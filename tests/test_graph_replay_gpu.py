@@ -45,7 +45,7 @@ def _replay_against_eager(run, inputs, fresh_inputs, between=None, replays=3):
 @pytest.mark.parametrize("M", [16, 32, 128, 512])
 def test_w4a16_split_k_launches_replay(M):
     """K = 14336, N = 4096 (the down projection): split-K exchange between workgroups for up to 32
-    rows, narrow tiles with a reduction kernel at 128, wide tiles with one at 512."""
+    rows, K ranges with a reduction kernel at 128 and at 512."""
     from vllm_gcu_amd.kernels import _custom_ops as ops
     K, N, g = 14336, 4096, 128
     gen = torch.Generator(device="cpu").manual_seed(M)

@@ -2,7 +2,7 @@
 //
 // Why it exists: the kernels of a decode step take 3 .. 15 us each, and a Python wrapper of the same work
 // (attribute look-ups, views, the dispatcher calling back into Python, a ctypes call of twenty arguments)
-// took 20 .. 26 us per operator on the box's host core, so the GPU waited for the host.  Here an operator
+// took 20 .. 26 us per operator on an EPYC core, so the GPU waited for the host.  Here an operator
 // costs its allocation and its launch.
 #pragma once
 
