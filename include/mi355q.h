@@ -191,6 +191,9 @@ int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w, const flo
  * (kind 1) or mi355q_w8a8_int8_gemm_ws (kind 2) is called with *workspace_bytes bytes of workspace (0: none needed).
  * 1: it is, and those entry points are ahead of mi355q_kcontig_gemm; 0: it is not. */
 int mi355q_q8_mid_plan(int kind, int M, int N, int K, size_t* workspace_bytes);
+/* The work split of that plan: rows and columns of a workgroup's tile and K ranges (what a profile was taken on); all 0 where the
+ * plan answers 0. */
+int mi355q_q8_mid_tile(int kind, int M, int N, int K, int* rows, int* columns, int* k_ranges);
 
 /* ---- W8A8 int8 -------------------------------------------------------------
  * Replaces topsatenDotBiasQuant as called by cutlass_scaled_mm

@@ -4,16 +4,18 @@ blocks, one and several K ranges, with and without bias.  int8 is exact; fp8 is 
 import pytest
 import torch
 
+from test_q8_plans_cpu import tile
 from vllm_gcu_amd.kernels import _custom_ops as ops
 from vllm_gcu_amd.kernels import _runtime as rt
 from vllm_gcu_amd.kernels.quantization import rearrange
 
 pytestmark = pytest.mark.gpu
-# (M, N, K): tiles of 32, 64 and 128 rows, with and without K ranges
+# (M, N, K): tiles of every height, with and without K ranges
 SHAPES = [(17, 64, 384), (31, 320, 128), (33, 512, 1152), (48, 1024, 7168), (63, 640, 640), (64, 4096, 2048), (65, 1024, 1024),
           (96, 3072, 3584), (127, 256, 4096), (129, 1024, 5120), (130, 4096, 7168), (200, 2048, 1408), (257, 4608, 3584),
           (511, 4096, 4096), (512, 8192, 2048), (700, 512, 7168), (768, 1024, 4096), (1000, 3072, 3584), (1024, 4096, 4096),
-          (1300, 640, 2048), (1535, 1536, 3584), (1536, 2048, 2048)]
+          (1300, 640, 2048), (1535, 1536, 3584), (1536, 2048, 2048),
+          (257, 7168, 2048), (193, 4096, 14336), (385, 6656, 1536), (400, 7168, 2048), (513, 6656, 1536), (577, 6656, 1536), (640, 6656, 1536)]
 BLOCK, SCALED, INT8 = 0, 1, 2            # kinds of mi355q_q8_mid_plan
 
 
@@ -21,6 +23,11 @@ def _planned(kind, M, N, K):
     want = rt.host.q8_mid_plan(kind, M, N, K)
     print(f"case q8 mid kind={kind} M={M} N={N} K={K} workspace={want}", flush=True)
     assert want >= 0, "another kernel takes this shape: the case tests nothing"
+
+
+@pytest.mark.parametrize("kind", [BLOCK, SCALED, INT8])
+def test_the_shapes_take_every_tile(kind):
+    assert {tile(kind, *s)[0] for s in SHAPES if s[1] % 128 == 0} == {32, 48, 64, 80, 96, 112, 128, 144, 160}
 
 
 @pytest.mark.parametrize("with_bias", [False, True])
