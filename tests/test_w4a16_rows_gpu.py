@@ -75,6 +75,20 @@ def test_automatic(M, K, N, g, dtype):
     assert torch.equal(_run(q, z, s, x, g, family=4), want)
 
 
+@pytest.mark.parametrize("M,K,N,g,dtype", [(170, 28672, 8192, 128, torch.bfloat16), (1536, 4096, 6144, 64, torch.bfloat16),
+                                           (333, 7168, 9344, 64, torch.bfloat16), (700, 5120, 5120, 32, torch.bfloat16),
+                                           (256, 3584, 37888, 32, torch.float16), (700, 5120, 5120, 64, torch.float16)])
+def test_taken_where_the_tiles_loop_is_the_slow_one(M, K, N, g, dtype):
+    """The 64-row tiles run a slower loop for groups of 64 and 32 and for bf16 rows that are not staged as fp16; this kernel is 18 to 40 %
+    ahead of it at these shapes.  Sums in another order round differently, so equal bits say which kernel ran."""
+    print(f"case w4a16 slow loop M={M} K={K} N={N} g={g} {dtype}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    w, zp = (torch.randint(-2**31, 2**31, shape, dtype=torch.int32, device="cuda", generator=gen) for shape in ((K // 8, N), (K // g, N // 8)))
+    scales = (torch.rand(K // g, N, device="cuda", generator=gen) * 0.01).to(dtype)
+    x = torch.randn(M, K, device="cuda", generator=gen).to(dtype)
+    assert torch.equal(ops.w4a16_gemm(x, w, scales, zp, None, g), ops.w4a16_gemm(x, w, scales, zp, None, g, family=4))
+
+
 def test_activations_of_four_gib():
     """The last row below 4 GiB of activations is addressed in 32 bits; from 4 GiB on the problem is refused."""
     K, N, M = 1 << 24, 128, 127

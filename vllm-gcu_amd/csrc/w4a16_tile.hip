@@ -933,12 +933,21 @@ size_t w4a16_tile_fixed_bytes(int M, int K, int N) {
 // Room for the ring kernel's partial tiles: layers that a call with the fixed scratch takes have one plan, with and without a workspace
 constexpr size_t FIXED_BYTES = (size_t)31 << 20;
 static size_t ring_bytes(int M, int K, int N) { return w4a16_tile_fixed_bytes(M, K, N) <= FIXED_BYTES ? FIXED_BYTES : TILE_SPLITK_BYTES; }
-// the ring kernel's plan where it is the cheaper one (tw 0: the 64-row tiles)
-static MidPlan tile_ring_plan(int M, int K, int N, size_t bytes) {
+// The loop of the 64-row tiles that these operands take, beside the pipelined one (fp16 rows, or bf16 rows staged as fp16; groups of 128 and
+// more; zero-points packed or none) that tile_time_model prices, as a factor on its price.  The rows kernel, whose price has no such
+// factor, costs 5 .. 75 % more for some of them itself: that is divided out.  Medians of 1300 launches (13 layers, 144 .. 2048 rows).
+static double tile_loop_factor(int group_size, int zeros_kind, bool bf16) {
+  static constexpr double f[2][3][3] = {{{1.0, 1.0, 1.15}, {1.18, 1.18, 1.27}, {1.10, 1.25, 1.20}},       // fp16; groups of 128, 64, 32; none, packed, pre-scaled
+                                        {{1.24, 1.23, 1.31}, {1.23, 1.23, 1.39}, {1.24, 1.38, 1.50}}};    // bf16
+  return f[bf16][group_size == 32 ? 2 : group_size == 64 ? 1 : 0][zeros_kind];
+}
+constexpr double MAX_LOOP_FACTOR_RING = 1.15;        // of the operands that the ring kernel takes
+// the ring kernel's plan where it is the cheaper one (tw 0: the 64-row tiles); loop: the tiles' factor
+static MidPlan tile_ring_plan(int M, int K, int N, size_t bytes, double loop) {
   if (ring_allowed(M, K, N, false)) {
     MidPlan p = w4a16_mid_plan(M, K, N, ring_bytes(M, K, N));
     if (p.splits > 1 && (size_t)p.splits * M * N * sizeof(float) > bytes) p = w4a16_mid_plan(M, K, N, bytes);
-    if (p.price < tile_time_model(M, K, N)) return p;
+    if (p.price < loop * tile_time_model(M, K, N)) return p;
   }
   return {0, 0, 1, 0.0};
 }
@@ -949,19 +958,24 @@ static MidPlan staged_ring_plan(int M, int K, int N) {
   }
   return {0, 0, 1, 0.0};
 }
-double w4a16_wide_price(int M, int K, int N, bool ring, bool bf16) {
-  if (!ring) return tile_time_model(M, K, N);
-  const double tiles = bf16 ? staged_tile_price(M, K, N) : tile_time_model(M, K, N);
-  if (!ring_allowed(M, K, N, bf16)) return tiles;
-  const MidPlan p = w4a16_mid_plan(M, K, N, bf16 ? 0 : ring_bytes(M, K, N));
-  return std::min(tiles, bf16 ? staged_ring_price(M, K, p) : p.price);
+static bool bf16_stage_pays(int M, int N);
+static bool bf16_stage_takes(int group_size, int zeros_kind) { return group_size % 128 == 0 && zeros_kind != MI355Q_ZP_PRESCALED; }
+// us of the kernels with larger tiles than the rows kernel's: the price of what these operands run
+double w4a16_wide_price(int M, int K, int N, int group_size, int zeros_kind, bool bf16) {
+  if (bf16 && bf16_stage_pays(M, N) && bf16_stage_takes(group_size, zeros_kind)) {
+    const double tiles = staged_tile_price(M, K, N);
+    return ring_allowed(M, K, N, true) ? std::min(tiles, staged_ring_price(M, K, w4a16_mid_plan(M, K, N, 0))) : tiles;
+  }
+  const double tiles = tile_loop_factor(group_size, zeros_kind, bf16) * tile_time_model(M, K, N);
+  if (bf16 || group_size % 128 != 0 || !ring_allowed(M, K, N, false)) return tiles;
+  return std::min(tiles, w4a16_mid_plan(M, K, N, ring_bytes(M, K, N)).price);
 }
 
 size_t w4a16_tile_workspace_bytes(int M, int K, int N) {
   // (the choice between the kernels also depends on the dtype and the group size, which this
   // function does not see: room for whichever plan is larger)
   const int s = tile_splits(M, K, N);
-  const int sr = tile_ring_plan(M, K, N, (size_t)-1).splits;
+  const int sr = tile_ring_plan(M, K, N, (size_t)-1, MAX_LOOP_FACTOR_RING).splits;
   const int m = s > sr ? s : sr;
   return m > 1 ? (size_t)m * M * N * sizeof(float) : 0;
 }
@@ -1001,7 +1015,7 @@ constexpr int BF16_STAGE_NOT_TAKEN = -12345;
 int w4a16_bf16_staged_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros,
                              int zeros_kind, const void* bias, int M, int K, int N, int group_size, void* workspace,
                              size_t workspace_bytes, int force_tw, hipStream_t st) {
-  if (group_size % 128 != 0 || zeros_kind == MI355Q_ZP_PRESCALED || M <= 64 || !workspace ||
+  if (!bf16_stage_takes(group_size, zeros_kind) || M <= 64 || !workspace ||
       workspace_bytes <= BF16_STAGE_OFFSET + BF16_STAGE_SCALE_BYTES)
     return BF16_STAGE_NOT_TAKEN;
   // Rows per chunk for a staging area that starts `off` bytes into the workspace
@@ -1072,7 +1086,7 @@ int w4a16_tile_launch(void* out, const void* x, const int32_t* qweight, const vo
              "w4a16_gemm: the MFMA kernel needs a group size of 32, 64 or a multiple of 128, got %d", group_size);
   MQ_REQUIRE((size_t)M * K * 2 < ((size_t)1 << 32), "w4a16_gemm: activation matrix %d x %d is 4 GiB or more", M, K);
   if (allow_ring && dtype == MI355Q_F16 && !small_groups) {
-    const MidPlan p = tile_ring_plan(M, K, N, workspace ? workspace_bytes : 0);
+    const MidPlan p = tile_ring_plan(M, K, N, workspace ? workspace_bytes : 0, tile_loop_factor(group_size, zeros_kind, false));
     if (p.tw)
       return w4a16_mid_launch(out, x, qweight, scales, zeros, zeros_kind, bias, M, K, N, group_size, dtype,
                               workspace, workspace_bytes, p.splits, p.tw, p.mt, st);
