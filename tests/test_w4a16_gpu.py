@@ -314,6 +314,18 @@ def test_tile_gemm_split_k_small_grid(ops, rearrange, M, K, N):
     assert torch.equal(got.cpu(), torch.from_numpy(oracle(q, z, s, x, g, torch.float16)).to(torch.float16))
 
 
+@pytest.mark.parametrize("g,dtype", [(128, torch.float16), (128, torch.bfloat16), (64, torch.bfloat16), (32, torch.float16)])
+@pytest.mark.parametrize("M,N", [(8063, 1280), (8129, 1280), (14271, 2048), (14273, 2048)])
+def test_tile_gemm_in_either_order(ops, rearrange, M, N, g, dtype):
+    """Both sides of the rounds from which the tiles go in an order of their own, columns that are and are not a multiple of eight tiles;
+    exact inputs bit for bit."""
+    K = 256
+    print(f"case tile order M={M} K={K} N={N} g={g} {dtype}", flush=True)
+    q, z, s, x = make_case(M + N, M, K, N, g, exact=True)
+    got = run_gemm(ops, rearrange, q, z, s, x, g, dtype, family=2)
+    assert torch.equal(got.cpu(), torch.from_numpy(oracle(q, z, s, x, g, dtype)).to(dtype))
+
+
 def test_tile_gemm_three_way_split_between_half_and_full_round(ops, rearrange):
     # 288 output tiles over a long K (more than half of the 512 resident workgroups, fewer than 0.7
     # of them): K is split three ways; sampled rows against the oracle, exact inputs bit for bit

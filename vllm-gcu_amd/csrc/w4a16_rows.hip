@@ -486,14 +486,13 @@ bool w4a16_rows_wanted(int M, int K, int N, int group_size, int zeros_kind, int 
   if (M <= 16) return small && w <= (1L << 25);
   if (M <= 32) return small || w >= (dtype == MI355Q_F16 ? 1L << 26 : 3L << 25);
   if (M <= 128) return true;
-  // (the price, corrected for the size of the output and the rows by 255 launches with fp16 rows and 177 with bf16, rms errors 4.6 %; 3 % on the
-  // pipelined fp16 loop: of factors from 0.95 to 1.05 the ones above 1 had the best picks.  Elsewhere they do not: bf16 K 14336 x N 4096 at 900 /
-  // 1024 rows 136 / 149 us here, 131 / 135 on the staged tiles, 11008 x 4096 at 900 113 / 103; the other loops by 1300 launches, the picks
-  // within 0.2 % of the better kernel: bf16 with groups of 64 4096 x 6144 at 1536 100 here, 142 there, with groups of 32 117 / 180, bf16 rows
-  // that are not staged 28672 x 8192 at 170 102 / 124, fp16 with groups of 32 3584 x 37888 at 256 119 / 159.)
-  const bool bf16 = dtype == MI355Q_BF16, piped = !bf16 && !small && zeros_kind != MI355Q_ZP_PRESCALED;
+  // (the price, corrected for the size of the output and the rows by 255 launches with fp16 rows and 177 with bf16, rms errors 4.6 and 3 %.  The
+  // pick loses 0.1 / 0.2 % (fp16 / bf16) to the best of the three kernels over 23 layers at 144 .. 2048 rows, 11 % at worst, where prices tie.  The
+  // loops that are not pipelined by 1300 launches, 0.2 %: bf16 with groups of 64 4096 x 6144 at 1536 100 us here, 142 there, with groups of 32
+  // 117 / 180, bf16 rows that are not staged 28672 x 8192 at 170 102 / 124, fp16 with groups of 32 3584 x 37888 at 256 119 / 159.)
+  const bool bf16 = dtype == MI355Q_BF16;
   const double corrected = w4a16_rows_price(M, K, N) * (bf16 ? 1.023 + 14e-6 * M : 0.881 + 66e-6 * M) + 0.78e-6 * M * N;
-  return corrected < (piped ? 1.03 : 1.0) * w4a16_wide_price(M, K, N, group_size, zeros_kind, bf16);
+  return corrected < w4a16_wide_price(M, K, N, group_size, zeros_kind, bf16);
 }
 
 size_t w4a16_rows_workspace_bytes(int M, int K, int N) { return M <= 4096 ? rows_plan(M, K, N).bytes : 0; }

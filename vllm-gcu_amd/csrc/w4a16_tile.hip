@@ -42,7 +42,7 @@ struct TileArgs {
   const int* npp;             // device scalar: padded id count
   const float* topk_weights;  // [numel] or null
   int numel, topk, E;
-  TileOrder order;            // of the output tiles and splits (not the grouped launches')
+  TileOrder order;            // of the output tiles and splits (total 0: they are the grid's coordinates)
   // split-K: split z takes K blocks [z * kper, (z + 1) * kper) and writes an fp32 partial
   // tile to partial[z][M][N] (grouped: M = numel, rows indexed by slot id, routing weight not yet
   // applied); a second kernel adds the partials up
@@ -143,9 +143,12 @@ w4a16_tile_kernel(TileArgs a) {
   const int c = lane & 15, kq = lane >> 4;
   const int N = a.N, K = a.K, M = a.M;
   const int G = K >> 7;
-  int tm = 0, tn = 0, split = 0;
-  if (!GROUPED) a.order.locate(blockIdx.x, tm, tn, split);
-  const uint32_t by = GROUPED ? blockIdx.y : tm, bx = GROUPED ? blockIdx.x : tn, bz = GROUPED ? blockIdx.z : split;
+  uint32_t bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+  if (!GROUPED && a.order.total) {
+    int tm, tn, split;
+    a.order.locate(blockIdx.x, tm, tn, split);
+    bx = tn, by = tm, bz = split;
+  }
   const int m0 = by * BM;
   const u4* qw = a.qw;
   const uint16_t* scales = a.scales;
@@ -594,11 +597,17 @@ w4a16_grouped_reduce_kernel(uint16_t* out, const float* partial, const float* ro
   *(uint2*)(out + i) = o;
 }
 
-// grouped: (columns, blocks, splits); dense: one dimension in the order of tile_order
+// (columns, row blocks, splits), or one dimension in the order of tile_order for dense launches of several rounds.  Workgroups that are all
+// resident at once gain nothing by the order, and the grid's coordinates spread K ranges and columns over the XCDs: with the order
+// K 8192 x N 8192 at 400 rows, three splits, 80.8 us against 76.1 without, 8192 x 10240 at 512 106.9 / 102.9, 2048 x 28672 at 576 73.9 / 71.6.
+// Columns that are a multiple of eight are on one XCD each by the coordinates already, and the order's blocks of rows are ahead only from
+// some rounds on.  (20 layers, 144 .. 3072 rows, fp16 and bf16: 0.994 of the time by the coordinates, by the order always 0.998, and 1.13
+// at worst; at 2048 rows of 7168 x 9344 284 -> 270.)
 template <bool GROUPED>
 dim3 tile_grid(TileArgs& a, int row_blocks, int bm, int per_cu) {
   const int cols = (a.N + BN - 1) / BN, splits = ((a.K >> 7) + a.kper - 1) / a.kper;
-  if (GROUPED) return dim3(cols, row_blocks, splits);
+  const double rounds = (double)cols * row_blocks * splits / (per_cu * device_cu_count());
+  if (GROUPED || rounds < (cols % 8 ? 1.25 : 3.5)) return dim3(cols, row_blocks, splits);
   a.order = tile_order(row_blocks, cols, splits, (double)bm * a.kper * 256, (double)BN * a.kper * 64, per_cu);
   return dim3((unsigned)(cols * row_blocks * splits));
 }
@@ -960,11 +969,13 @@ static MidPlan staged_ring_plan(int M, int K, int N) {
 }
 static bool bf16_stage_pays(int M, int N);
 static bool bf16_stage_takes(int group_size, int zeros_kind) { return group_size % 128 == 0 && zeros_kind != MI355Q_ZP_PRESCALED; }
-// us of the kernels with larger tiles than the rows kernel's: the price of what these operands run
+// us of the kernels with larger tiles than the rows kernel's: the price of what these operands run, on the scale of that kernel's (staged bf16
+// rows: 2 % below, where the picks between them are best; of 0.96 .. 1.01 the upper ones took the rows kernel where the tiles are 4 .. 9 % ahead,
+// 12288 x 3072 at 1300 rows 115 against 130 us, 11008 x 4096 at 1024 110 / 115, 8192 x 10240 at 333 79 / 83)
 double w4a16_wide_price(int M, int K, int N, int group_size, int zeros_kind, bool bf16) {
   if (bf16 && bf16_stage_pays(M, N) && bf16_stage_takes(group_size, zeros_kind)) {
     const double tiles = staged_tile_price(M, K, N);
-    return ring_allowed(M, K, N, true) ? std::min(tiles, staged_ring_price(M, K, w4a16_mid_plan(M, K, N, 0))) : tiles;
+    return 0.98 * (ring_allowed(M, K, N, true) ? std::min(tiles, staged_ring_price(M, K, w4a16_mid_plan(M, K, N, 0))) : tiles);
   }
   const double tiles = tile_loop_factor(group_size, zeros_kind, bf16) * tile_time_model(M, K, N);
   if (bf16 || group_size % 128 != 0 || !ring_allowed(M, K, N, false)) return tiles;
