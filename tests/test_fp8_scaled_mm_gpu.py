@@ -190,6 +190,38 @@ def test_block_scales_of_the_activations_staged_k_block_major(M, K, N, kslab, mo
     np.testing.assert_allclose(staged.float().cpu().numpy(), want, rtol=RTOL, atol=RTOL * max(1.0, float(np.abs(want).max())))
 
 
+@pytest.mark.parametrize("M,K,N,turned", [(130, 5248, 10240, True), (130, 4736, 10240, False), (130, 5248, 10112, False), (333, 3200, 28672, True),
+                                          (200, 10496, 10240, True), (200, 5376, 10240, False), (256, 5120, 16512, True), (257, 5248, 10240, False), (1025, 3072, 11776, True), (1025, 2944, 8192, False)])
+def test_block_scales_are_turned_where_it_pays(M, K, N, turned):
+    """The tile kernel's own look at the scales: with room behind the partial sums they stand there K block major after the call, on
+    the deep and wide layers (one and several row tiles, and two K ranges, the fifth), and the output is that of a call without the room bit
+    for bit."""
+    from vllm_gcu_amd import _lib
+    from vllm_gcu_amd.kernels.quantization import rearrange
+    print(f"case fp8 block scales turned M={M} K={K} N={N}", flush=True)
+    torch.manual_seed(M + K + N)
+    x, w = ((torch.randn(r, K, device="cuda") * 40).to(torch.float8_e4m3fn) for r in (M, N))
+    xs, wsc = torch.rand(M, K // 128, device="cuda") + 0.5, torch.rand(N // 128, K // 128, device="cuda") + 0.5
+    need = _lib.load().mi355q_fp8_gemm_workspace_bytes(M, N, K) or 1 << 20
+    rows = (M + 15) // 16 * 16
+    mid = _lib.load().mi355q_q8_mid_plan(0, M, N, K, None)
+    for wt, ldw in ((w, K), (rearrange.to_kslab(w), 0))[:1 if mid else 2]:
+        outs = []
+        for room in (0, rows * (K // 128) * 4):
+            out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+            ws = torch.zeros(need + rows * (K // 128) * 4, dtype=torch.uint8, device="cuda")
+            _lib.call("mi355q_fp8_block_gemm_ws", out.data_ptr(), x.data_ptr(), wt.data_ptr(), xs.data_ptr(), wsc.data_ptr(), None, M, N, K, K, ldw,
+                      N, _lib.BF16, ws.data_ptr(), need + room, torch.cuda.current_stream().cuda_stream)
+            area = ws[need:].view(torch.float32).view(K // 128, rows)
+            assert torch.equal(area[:, :M], xs.t()) if turned and room else not area.any()
+            outs.append(out)
+        assert torch.equal(*outs)
+        xd = (x.double().view(M, -1, 128) * xs.double()[..., None]).view(M, K)
+        want = torch.cat([xd @ (b.double().view(-1, 128, K // 128, 128) * s.double()[:, None, :, None]).view(-1, K).t()
+                          for b, s in zip(w.split(2048), wsc.split(16))], 1)
+        assert float((outs[0].double() - want).norm() / want.norm()) < 3e-3          # one rounding to bf16
+
+
 @pytest.mark.parametrize("M", [1, 16, 128, 2048])
 def test_full_size_layer_sampled(M):
     """K = 8192, N = 28672 (one Llama-3-70B MLP projection): sampled rows and columns against the oracle, the whole

@@ -632,12 +632,14 @@ int launch_f8_auto(F8Args& a, void* workspace, size_t workspace_bytes, hipStream
   const int splits = fp8_ksplits(a.M, a.N, a.K);
   const bool split = splits > 1 && workspace && workspace_bytes >= F8_WS_OFFSET + (size_t)splits * a.M * a.N * sizeof(float);
   // (It pays where a row has more scales than the one cache line that 16 K blocks share and enough tiles read them again: a launch of 4 us
-  // against 0.1 us for a K block of a full round.  Measured, us, as they come -> K block major: K 8192 x N 28672 at 130 / 2048
-  // 59.5 / 492 -> 53.8 / 449, K 7168 x N 4096 at 1537 55.8 -> 52.5, K 4096 x N 14336 at 520 / 1000 50.2 / 76.3 -> 51.4 / 72.6, K 7168 x N 9344 at
-  // 300 / 520 37.3 / 51.6 -> 39.6 / 49.4, K 4096 x N 28672 at 130 33.4 -> 35.0, K 2048 x N 7168 at 1537 / 2048 34.5 / 40.9 -> 37.3 / 43.8.)
+  // against 0.1 us for a K block of a full round, 0.2 where all columns read the scales of one row tile.  Measured, us, as they
+  // come -> K block major: K 8192 x N 17664 at 100 / 250 rows 47.9 / 69.1 -> 44.9 / 59.3, K 8192 x N 28672 at 130 / 2048 59.5 / 492 -> 53.8 / 449, K 7168
+  // x N 4096 at 1537 55.8 -> 52.5, K 10368 x N 12288 at 193 56.4 -> 50.6; but K 6272 x N 10240 at 300 34.3 -> 36.1, K 7296 x N 7168 at 520
+  // 42.6 -> 45.9, K 4096 x N 28672 at 80 / 130 28.8 / 33.1 -> 30.8 / 33.4, K 2048 x N 7168 at 1537 / 2048 34.5 / 40.9 -> 37.3 / 43.8.  By this rule the
+  // launches of 20 layers at 80 .. 2048 rows are within 0.3 % of the better way, by the product of K blocks and tiles alone 1.5 %, 17 % at worst.)
   const long tiles = (long)((a.M + FTM - 1) / FTM) * (a.N / FTN);
   const int KB = a.K / FTKB;
-  if (MODE == T8_BLOCK && workspace && KB >= 24 && KB * tiles >= 11000) {
+  if (MODE == T8_BLOCK && workspace && ((a.M <= FTM && tiles >= 80 && KB / (split ? splits : 1) >= 40) || (KB >= 24 && KB * tiles >= 11000))) {
     // block scales: with room behind the partial sums, the activation scales are re-ordered K block major first
     const size_t off = F8_WS_OFFSET + (split ? (size_t)splits * a.M * a.N * sizeof(float) : 0);
     if (workspace_bytes >= off + fp8_scales_kmajor_bytes(a.M, a.K)) {
