@@ -71,3 +71,27 @@ def test_fp8_block_and_scaled(M, N, K):
         torch.ops._C.cutlass_scaled_mm(out, x, wk.t(), xs, ws, None)
         ref = (x.double() @ w.double().t()) * xs.double().view(-1, 1) * ws.double().view(1, -1)
         assert float((out.double() - ref).norm() / ref.norm()) < 1e-3
+
+
+@pytest.mark.parametrize("M,N,K", [(48, 1024, 7168), (193, 4096, 14336), (65, 1024, 1024), (385, 6656, 1536)])
+def test_other_output_types(M, N, K):
+    """fp8 with block scales to fp16 and int8 to fp32, with and without K ranges."""
+    from vllm_gcu_amd import _lib
+    _planned(BLOCK, M, N, K), _planned(INT8, M, N, K)
+    torch.manual_seed(M + N + K)
+    st = torch.cuda.current_stream().cuda_stream
+    ws = torch.zeros(80 << 20, dtype=torch.uint8, device="cuda")
+    x, w = ((torch.randn(r, K, device="cuda") * 40).to(torch.float8_e4m3fn) for r in (M, N))
+    xb, wb = torch.rand(M, K // 128, device="cuda") * 1e-4 + 1e-5, torch.rand(N // 128, K // 128, device="cuda") + 0.1
+    out = torch.full((M, N), float("nan"), device="cuda").half()
+    _lib.call("mi355q_fp8_block_gemm_ws", out.data_ptr(), x.data_ptr(), rearrange.to_kslab(w).data_ptr(), xb.data_ptr(), wb.data_ptr(), None, M, N, K, K,
+              0, N, _lib.F16, ws.data_ptr(), ws.numel(), st)
+    want = (x.double().view(M, -1, 128) * xb.double()[..., None]).view(M, K) @ (
+        w.double().view(N // 128, 128, K // 128, 128) * wb.double()[:, None, :, None]).view(N, K).t()
+    assert float((out.double() - want).norm() / want.norm()) < 1e-3
+    x, w = (torch.randint(-128, 128, (r, K), dtype=torch.int8, device="cuda") for r in (M, N))
+    xs, wsc = torch.rand(M, device="cuda") * 0.1, torch.rand(N, device="cuda") * 0.01
+    out = torch.full((M, N), float("nan"), device="cuda")
+    _lib.call("mi355q_w8a8_int8_gemm_ws", out.data_ptr(), None, x.data_ptr(), rearrange.to_kslab(w).data_ptr(), xs.data_ptr(), 1, wsc.data_ptr(), 1,
+              None, 1, M, N, K, K, 0, N, _lib.F32, ws.data_ptr(), ws.numel(), st)
+    assert torch.equal(out, (x.double() @ w.double().t()).float() * xs.view(-1, 1) * wsc)

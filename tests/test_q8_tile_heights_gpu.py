@@ -64,3 +64,23 @@ def test_fp8(M, N, K):
         _lib.call("mi355q_fp8_scaled_gemm_ws", out.data_ptr(), x.data_ptr(), wt.data_ptr(), xs.data_ptr(), 1, wsc.data_ptr(), 1, bias.data_ptr(),
                   M, N, K, K, ldw, N, BF16, ws.data_ptr(), ws.numel(), st)
         assert float((out.double() - scaled).norm() / scaled.norm()) < 3e-3
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_fp8_to_fp16(M, N, K):
+    """The same sums, stored as fp16: within one rounding of the float64 product."""
+    ws, st = _common(M, N, K)
+    x, w = ((torch.randn(r, K, device="cuda") * 40).to(torch.float8_e4m3fn) for r in (M, N))
+    xb, wb = torch.rand(M, K // 128, device="cuda") * 1e-4 + 1e-5, torch.rand(N // 128, K // 128, device="cuda") + 0.1
+    xs, wsc = torch.rand(M, device="cuda") * 1e-4, torch.rand(N, device="cuda")
+    xd = (x.double().view(M, K // 128, 128) * xb.double()[..., None]).view(M, K)
+    wd = (w.double().view(N // 128, 128, K // 128, 128) * wb.double()[:, None, :, None]).view(N, K)
+    want = xd @ wd.t(), (x.double() @ w.double().t()) * xs.double().view(-1, 1) * wsc.double().view(1, -1)
+    for wt, ldw in ((w, K), (rearrange.to_kslab(w), 0)):
+        outs = [torch.full((M, N), float("nan"), device="cuda").half() for _ in range(2)]
+        _lib.call("mi355q_fp8_block_gemm_ws", outs[0].data_ptr(), x.data_ptr(), wt.data_ptr(), xb.data_ptr(), wb.data_ptr(), None, M, N, K,
+                  K, ldw, N, F16, ws.data_ptr(), ws.numel(), st)
+        _lib.call("mi355q_fp8_scaled_gemm_ws", outs[1].data_ptr(), x.data_ptr(), wt.data_ptr(), xs.data_ptr(), 1, wsc.data_ptr(), 1, None,
+                  M, N, K, K, ldw, N, F16, ws.data_ptr(), ws.numel(), st)
+        for out, ref in zip(outs, want):
+            assert float((out.double() - ref).norm() / ref.norm()) < 1e-3

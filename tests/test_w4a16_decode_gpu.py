@@ -13,7 +13,8 @@ from vllm_gcu_amd.kernels.quantization import rearrange
 pytestmark = pytest.mark.gpu
 # (K, N, group): K blocks 1 .. 64, N on both sides of 256 tiles of 16 and of 32 columns
 SHAPES = [(128, 128, 128), (640, 1024, 128), (1024, 4096, 1024), (1152, 4224, 128), (2048, 384, 256), (2176, 8192, 128), (3072, 256, 1536),
-          (4096, 512, 128), (4096, 8320, 256), (4224, 1024, 128), (6144, 4352, 128), (8192, 512, 4096), (1024, 16384, 128), (2944, 8448, 128)]
+          (4096, 512, 128), (4096, 8320, 256), (4224, 1024, 128), (6144, 4352, 128), (8192, 512, 4096), (1024, 16384, 128), (2944, 8448, 128),
+          (1024, 8192, 256), (1280, 8320, 128), (3968, 4224, 128), (4352, 8320, 128), (6400, 4224, 128)]
 
 
 def _data(K, N, g, dtype, exact):
@@ -156,3 +157,63 @@ def test_unsorted_slots(E, K, N, ids_dtype, dtype):
                                                          None, idd.data_ptr(), int(ids_dtype == torch.int64), numel, topk, E, K, N, 1, code, st),
                            "moe_w4a16_unsorted")
                 assert torch.equal(glu[keep.cuda()], act[keep.cuda()]) and glu[~keep.cuda()].isnan().all() and not glu[keep.cuda()].isnan().any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["none", "packed", "pre-scaled"])
+@pytest.mark.parametrize("E,K,N,g", [(2, 1152, 256, 384), (1, 1152, 16384, 1152), (1, 640, 32768, 128), (4, 1152, 16384, 128), (4, 512, 16384, 256)])
+def test_unsorted_slots_of_every_form(E, K, N, g, kind, dtype):
+    """Every workgroup shape with up to nine K blocks (a wavefront then has several or none), groups of one to nine of them, each kind of
+    zero-points: the aligned launch against a float64 product, the unsorted one and SiLU of gate and up against it bit for bit."""
+    from vllm_gcu_amd import _lib
+    from vllm_gcu_amd.kernels import fused_moe
+    lib, code = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // 8, N), dtype=torch.int32, device="cuda", generator=gen)
+    s = (torch.rand(E, K // g, N, device="cuda", generator=gen) * 0.009 + 0.001).to(dtype)
+    zk, zp = _lib.ZP_NONE, None
+    dense = rearrange.unpack_slab(w).to(torch.float32).view(E, K // g, g, N)
+    if kind == "packed":
+        z = torch.randint(0, 16, (E, K // g, N), dtype=torch.uint8, device="cuda", generator=gen)
+        zk = _lib.ZP_PACKED
+        zp = torch.stack([rearrange.rearrange_uint4_int32_gptq(w[0], torch.from_numpy(ow4.gptq_pack_zeros(a.cpu().numpy())).cuda())[1] for a in z])
+        dense = (dense - z[:, :, None].float()) * s[:, :, None].float()
+    elif kind == "pre-scaled":                               # fractions of the scale, as they are
+        zk, zp = _lib.ZP_PRESCALED, (s.float() * torch.rand(s.shape, device="cuda", generator=gen) * 15).to(dtype)
+        dense = dense * s[:, :, None].float() - zp[:, :, None].float()
+    else:
+        dense = (dense - 8) * s[:, :, None].float()
+    dense = dense.view(E, K, N)
+    st = torch.cuda.current_stream().cuda_stream
+    for numel, topk in ((1, 1), (5, 1), (18, 2), (60, 1)):
+        print(f"case w4a16 unsorted {kind} E={E} K={K} N={N} g={g} numel={numel} {dtype}", flush=True)
+        ids = torch.randint(0, E, (numel // topk, topk), device="cuda", generator=gen)
+        if numel > 2:
+            ids.view(-1)[1], ids.view(-1)[-1] = -1, E
+        x = torch.randn(numel // topk, K, device="cuda", generator=gen).to(dtype)
+        rw = torch.rand(numel, device="cuda", generator=gen)
+        so, ex, n = fused_moe.moe_align_block_size(ids, 16, E)
+
+        def unsorted(weights, glu):
+            out = torch.full((numel, N // 2 if glu else N), float("nan"), dtype=dtype, device="cuda")
+            _lib.check(lib.mi355q_moe_w4a16_unsorted(out.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), None if zp is None else zp.data_ptr(),
+                                                     zk, g, None if weights is None else weights.data_ptr(), ids.data_ptr(), 1, numel, topk, E, K,
+                                                     N, glu, code, st), "moe_w4a16_unsorted")
+            return out
+        aligned = torch.full((numel, N), float("nan"), dtype=dtype, device="cuda")
+        _lib.check(lib.mi355q_moe_gemm(aligned.data_ptr(), x.data_ptr(), w.data_ptr(), None, s.data_ptr(), None if zp is None else zp.data_ptr(), zk, 0,
+                                       g, rw.data_ptr(), so.data_ptr(), ex.data_ptr(), n.data_ptr(), numel, topk, 16, ex.numel(), E, K, N, code,
+                                       code, 0, None, 0, st), "moe_gemm")
+        flat = ids.view(-1)
+        keep = (flat >= 0) & (flat < E)
+        got = unsorted(rw, 0)
+        assert torch.equal(got[keep], aligned[keep]) and got[~keep].isnan().all()
+        rows = keep.nonzero().view(-1).tolist()
+        want = torch.stack([(x[r // topk].double() @ dense[flat[r]].double()) * rw[r].double() for r in rows])
+        err = float((got[rows].double() - want).norm() / want.norm())
+        assert err < (1e-3 if dtype == torch.float16 else 6e-3)                          # one rounding to 16 bits
+        if zk != _lib.ZP_PRESCALED:
+            plain, glu = unsorted(None, 0), unsorted(None, 1)
+            act = torch.full((numel, N // 2), float("nan"), dtype=dtype, device="cuda")
+            _lib.check(lib.mi355q_silu_and_mul(act.data_ptr(), plain.data_ptr(), numel, N // 2, code, None, 1, st), "silu_and_mul")
+            assert torch.equal(glu[keep], act[keep]) and glu[~keep].isnan().all()

@@ -314,16 +314,24 @@ def test_tile_gemm_split_k_small_grid(ops, rearrange, M, K, N):
     assert torch.equal(got.cpu(), torch.from_numpy(oracle(q, z, s, x, g, torch.float16)).to(torch.float16))
 
 
-@pytest.mark.parametrize("g,dtype", [(128, torch.float16), (128, torch.bfloat16), (64, torch.bfloat16), (32, torch.float16)])
+@pytest.mark.parametrize("g,dtype", [(128, torch.float16), (128, torch.bfloat16), (64, torch.float16), (64, torch.bfloat16), (32, torch.float16),
+                                     (32, torch.bfloat16)])
 @pytest.mark.parametrize("M,N", [(8063, 1280), (8129, 1280), (14271, 2048), (14273, 2048)])
-def test_tile_gemm_in_either_order(ops, rearrange, M, N, g, dtype):
-    """Both sides of the rounds from which the tiles go in an order of their own, columns that are and are not a multiple of eight tiles;
-    exact inputs bit for bit."""
+def test_tile_gemm_in_either_order(ops, rearrange, M, N, g, dtype, monkeypatch):
+    """Both sides of the rounds from which the tiles go in an order of their own, columns that are and are not a multiple of eight tiles,
+    each loop of the kernel; exact inputs bit for bit."""
     K = 256
     print(f"case tile order M={M} K={K} N={N} g={g} {dtype}", flush=True)
     q, z, s, x = make_case(M + N, M, K, N, g, exact=True)
-    got = run_gemm(ops, rearrange, q, z, s, x, g, dtype, family=2)
-    assert torch.equal(got.cpu(), torch.from_numpy(oracle(q, z, s, x, g, dtype)).to(dtype))
+    want = torch.from_numpy(oracle(q, z, s, x, g, dtype)).to(dtype)
+    assert torch.equal(run_gemm(ops, rearrange, q, z, s, x, g, dtype, family=2).cpu(), want)
+    # z * s read as it is (exact with scales that are powers of two), and none
+    monkeypatch.setattr(ops, "_RECOVER_INTEGER_ZEROS", False)
+    w, _ = rearrange.rearrange_uint4_int32_gptq(dev(ow4.gptq_pack_weight(q)), None)
+    xs, sd = to_act(x, dtype).cuda(), to_act(s, dtype).cuda()
+    assert torch.equal(ops.w4a16_gemm(xs, w, sd, to_act(z * s, dtype).cuda(), None, g, family=2).cpu(), want)
+    got = ops.w4a16_gemm(xs, w, sd, None, None, g, family=2).cpu()
+    assert torch.equal(got, torch.from_numpy(oracle(q, None, s, x, g, dtype)).to(dtype))
 
 
 def test_tile_gemm_three_way_split_between_half_and_full_round(ops, rearrange):

@@ -40,6 +40,25 @@ def test_heights(K, N, g, dtype):
                     assert torch.equal(out.cpu(), want[:M])
 
 
+@pytest.mark.parametrize("dtype,kind", [(torch.float16, "none"), (torch.bfloat16, "none"), (torch.float16, "pre-scaled")])
+def test_heights_and_zero_points(dtype, kind, monkeypatch):
+    """No zero-points, and z * s in the activation type read as they are (fp16; bf16 rows with those are not staged)."""
+    monkeypatch.setattr(ops, "_RECOVER_INTEGER_ZEROS", False)
+    K, N, g = 768, 1408, 128
+    w, _, s, x, bias, _ = _data(K, N, g, 333, dtype)
+    q = rearrange.unpack_slab(w).cpu().numpy()
+    z = np.full((K // g, N), 8, dtype=np.uint8) if kind == "none" else np.random.default_rng(1).integers(0, 16, size=(K // g, N), dtype=np.uint8)
+    zs = None if kind == "none" else (torch.from_numpy(z).cuda() * s.float()).to(dtype)
+    want = torch.from_numpy(x.float().cpu().numpy() @ ow4.dequantize(q, z, s.float().cpu().numpy(), g) + bias.float().cpu().numpy()).to(dtype)
+    for mt in (5, 6, 7, 8):
+        for M in (16 * mt + 1, 333):
+            for tw in (2, 4):
+                print(f"case w4a16 ring {kind} rows={16 * mt} tw={tw} M={M} {dtype}", flush=True)
+                out = torch.full((M, N), float("nan"), dtype=dtype, device="cuda")
+                ops.w4a16_gemm(x[:M], w, s, zs, bias, g, family=3, split_k=1 | tw << 8 | mt << 16, out=out)
+                assert torch.equal(out.cpu(), want[:M])
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("K,N,g", CASES)
 def test_chosen(K, N, g, dtype):
