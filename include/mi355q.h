@@ -222,6 +222,10 @@ int mi355q_w8a8_int8_gemm(void* out, int32_t* acc_out, const int8_t* x, const in
  * rules of mi355q_w4a16_gemm's (its first MiB is left alone, so one buffer serves both); without
  * one, or with a smaller one, the unsplit launch runs. */
 size_t mi355q_w8a8_int8_workspace_bytes(int M, int N, int K);
+/* No counterpart in the reference.  What mi355q_w8a8_int8_gemm_ws launches for dense operands, no raw accumulators and a workspace of that size
+ * (or of mi355q_q8_mid_plan's): 0 = the kernel for a few dozen to some hundred rows (kslab weights), 1 = tiles of 128 .. 256 rows x 128
+ * columns, 2 = tiles of 256 rows x 128 .. 256 columns; and the K ranges it cuts K into. */
+int mi355q_w8a8_int8_plan(int M, int N, int K, int kslab, int* kernel, int* k_ranges);
 int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_t* x, const int8_t* w,
                              const float* x_scale, int x_scale_per_row, const float* w_scale,
                              int w_scale_per_col, const void* bias, int bias_f32, int M, int N, int K,

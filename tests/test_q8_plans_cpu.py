@@ -22,6 +22,21 @@ def test_every_tile_is_taken_somewhere(kind):
     assert rows == {0, 32, 48, 64, 80, 96, 112, 128, 144, 160}
 
 
+def int8_plan(M, N, K, kslab=True):
+    """(kernel, K ranges): 0 = csrc/q8_mid.hip, 1 = the tiles of csrc/fp8_block_tile.hip, 2 = the tiles of csrc/w8a8_int8.hip"""
+    kernel, ranges = c_int(), c_int()
+    _lib.call("mi355q_w8a8_int8_plan", M, N, K, kslab, byref(kernel), byref(ranges))
+    return kernel.value, ranges.value
+
+
+def test_the_int8_kernel_is_the_one_that_the_others_were_compared_with():
+    """Where the prices of the two tile kernels are close, the 8-bit kernel for some hundred rows gives way to the one that is launched: the
+    128-column tiles here (us, 8-bit kernel / 128-column tiles / 256 rows: K 3456 x N 20096 at 362 rows 49.6 / 42.1 / 44.9)."""
+    assert int8_plan(335, 19968, 3712) == (1, 1)
+    assert int8_plan(362, 20096, 3456) == (1, 1)
+    assert int8_plan(594, 26112, 1408) == (1, 1)
+
+
 def test_no_plan_outside_the_range():
     for M, N, K in ((16, 4096, 4096), (1537, 4096, 4096), (64, 4096 + 32, 4096)):
         assert tile(1, M, N, K) == (0, 0, 0)

@@ -842,11 +842,8 @@ static Int8Tiles int8_tile_plan(int M, int N) {
   return p;
 }
 
-// Prices in us: of this kernel's plan without K ranges (fitted to 80 shapes, rms error 9 %), and of the cheaper of it and the
-// 128-column tiles of the other 8-bit GEMMs (csrc/fp8_block_tile.hip), whose heights fit the rows and whose copies have
-// wavefronts of their own: they win unless tiles of 224 and 256 columns fill their rounds (us, here / there: K 8192 x N 28672 at 300 /
-// 640 / 900 / 2048 rows 101 / 91, 181 / 156, 193 / 219, 388 / 407; K 7168 x N 4096 at 1300 / 2048 70 / 42, 77 / 56; K 14336 x N 4096 at
-// 2048, two ranges, 120 / 100; K 2048 x N 7168 at 900 / 2048 30 / 22, 33 / 43).
+// Price in us of this kernel's plan, fitted to 80 launches without K ranges (rms error 9 %).  Its own ranges are close to it as well (us, priced /
+// measured: K 14336 x N 4096 at 2048 rows, two ranges, 127 / 120; K 23296 x N 9728 at 253, two, 90 / 91; K 26368 x N 8832 at 230 97 / 97).
 double int8_wide_price(int M, int N, int K) {
   const Int8Tiles p = int8_tile_plan(M, N);
   const int cus = device_cu_count(), mtiles = (M + TM - 1) / TM;
@@ -859,10 +856,23 @@ double int8_wide_price(int M, int N, int K) {
   if (p.split) part(N - p.split, p.tail_width);
   return t;
 }
-double int8_tile_price(int M, int N, int K) {
-  const double wide = int8_wide_price(M, N, K);
-  return N % 128 ? wide : std::min(wide, t8_price(2, M, N, K, int8_ksplits(M, N, K), nullptr));
+// This kernel or the 128-column tiles of the other 8-bit GEMMs (csrc/fp8_block_tile.hip), whose heights fit the rows and whose copies have
+// wavefronts of their own: they win unless tiles of 224 and 256 columns fill their rounds (us, here / there: K 8192 x N 28672 at 300 /
+// 640 / 900 / 2048 rows 101 / 91, 181 / 156, 193 / 219, 388 / 407; K 7168 x N 4096 at 1300 / 2048 70 / 42, 77 / 56; K 14336 x N 4096 at
+// 2048, two ranges, 120 / 100; K 2048 x N 7168 at 900 / 2048 30 / 22, 33 / 43).  Over 145 shapes whose two prices are within 16 % of each
+// other (cold weights, 65 .. 4096 rows) the pick is 0.7 % from the better kernel with 0.965, 2.2 % with 0.92 and 0.7 % with 1; where the
+// prices are 0.96 .. 1 apart the two kernels take the same time (0.993), and the lower price stands for either.
+struct Int8Pick {
+  bool tiles128;
+  double price;
+};
+static Int8Pick int8_pick(int M, int N, int K) {
+  return cached_plan(0, M, N, K, [](int, int M, int N, int K) {
+    const double wide = int8_wide_price(M, N, K), tiles = N % 128 ? 1e30 : t8_price(2, M, N, K, int8_ksplits(M, N, K), nullptr);
+    return Int8Pick{tiles < 0.965 * wide, std::min(tiles, wide)};
+  });
 }
+double int8_tile_price(int M, int N, int K) { return int8_pick(M, N, K).price; }
 
 namespace {
 
@@ -946,6 +956,20 @@ extern "C" size_t mi355q_w8a8_int8_workspace_bytes(int M, int N, int K) {
   return s > 1 ? I8_WS_OFFSET + (size_t)s * M * N * sizeof(int32_t) : 0;
 }
 
+extern "C" int mi355q_w8a8_int8_plan(int M, int N, int K, int kslab, int* kernel, int* k_ranges) {
+  MQ_REQUIRE(M > 0 && N > 0 && K > 0 && N % 4 == 0 && K % 128 == 0, "w8a8_int8_plan: bad shape M=%d N=%d K=%d", M, N, K);
+  MQ_REQUIRE(kernel && k_ranges, "w8a8_int8_plan: null pointer");
+  int rows, columns;
+  if (kslab && mi355q_q8_mid_tile(2, M, N, K, &rows, &columns, k_ranges) == 0 && rows > 0) {
+    *kernel = 0;
+    return 0;
+  }
+  *kernel = int8_pick(M, N, K).tiles128 ? 1 : 2;
+  *k_ranges = int8_ksplits(M, N, K);
+  if (*kernel == 2 && *k_ranges <= 1) *k_ranges = std::max(1, int8_ksplits_wide(M, N, K));
+  return 0;
+}
+
 extern "C" int mi355q_w8a8_int8_gemm(void* out, int32_t* acc_out, const int8_t* x, const int8_t* w,
                                      const float* x_scale, int x_scale_per_row, const float* w_scale,
                                      int w_scale_per_col, const void* bias, int bias_f32, int M, int N,
@@ -976,9 +1000,8 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
       (mid_bytes == 0 || (workspace && workspace_bytes >= I8_WS_OFFSET + mid_bytes)))
     return q8_mid_launch(2, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K, ldx,
                          ldo, out_dtype, mid_bytes ? (char*)workspace + I8_WS_OFFSET : nullptr, as_stream(stream));
-  const int ranges = int8_ksplits(M, N, K);
   if (N % 128 == 0 && !acc_out && (size_t)N * K < ((size_t)1 << 32) && (size_t)256 * (size_t)ldx < ((size_t)1 << 32) &&
-      (kslab || (size_t)128 * (size_t)ldw < ((size_t)1 << 32)) && t8_price(2, M, N, K, ranges, nullptr) < 0.92 * int8_wide_price(M, N, K))
+      (kslab || (size_t)128 * (size_t)ldw < ((size_t)1 << 32)) && int8_pick(M, N, K).tiles128)
     return int8_tile_launch(out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K,
                             ldx, ldw, ldo, out_dtype, workspace, workspace_bytes, as_stream(stream));
   I8Args a;
