@@ -95,3 +95,49 @@ def test_other_output_types(M, N, K):
     _lib.call("mi355q_w8a8_int8_gemm_ws", out.data_ptr(), None, x.data_ptr(), rearrange.to_kslab(w).data_ptr(), xs.data_ptr(), 1, wsc.data_ptr(), 1,
               None, 1, M, N, K, K, 0, N, _lib.F32, ws.data_ptr(), ws.numel(), st)
     assert torch.equal(out, (x.double() @ w.double().t()).float() * xs.view(-1, 1) * wsc)
+
+
+# 160 rows of 30 MB, 64 of 80 MB: further apart than 32 bits of bytes
+@pytest.mark.parametrize("M,N,K,ldx,kslab", [(160, 16512, 128, 30_000_000, True), (160, 16512, 128, 30_000_000, False),
+                                               (160, 260, 256, 30_000_000, False), (64, 16512, 128, 80_000_000, True)])
+def test_int8_rows_far_apart(M, N, K, ldx, kslab):
+    """Row strides at which the rows of a tile do not fit 32-bit offsets: the same outputs and sums as for dense rows."""
+    from vllm_gcu_amd import _lib
+    assert tile(INT8, 160, 16512, 128)[0] == 160
+    print(f"case q8 rows far apart M={M} N={N} K={K} ldx={ldx} kslab={kslab}", flush=True)
+    torch.manual_seed(M + N)
+    dense = torch.randint(-128, 128, (M, K), dtype=torch.int8, device="cuda")
+    w = torch.randint(-128, 128, (N, K), dtype=torch.int8, device="cuda")
+    wt, ldw = (rearrange.to_kslab(w), 0) if kslab else (w, K)
+    xs, wsc = torch.rand(M, device="cuda") * 0.1, torch.rand(N, device="cuda") * 0.01
+    x = torch.empty(M * ldx, dtype=torch.int8, device="cuda").as_strided((M, K), (ldx, 1))
+    x.copy_(dense)
+    ws, st = torch.zeros(80 << 20, dtype=torch.uint8, device="cuda"), torch.cuda.current_stream().cuda_stream
+    want = dense.double() @ w.double().t()
+    for acc in (None, torch.zeros(M, N, dtype=torch.int32, device="cuda")):
+        out = torch.full((M, N), float("nan"), device="cuda")
+        _lib.call("mi355q_w8a8_int8_gemm_ws", out.data_ptr(), None if acc is None else acc.data_ptr(), x.data_ptr(), wt.data_ptr(), xs.data_ptr(), 1,
+                  wsc.data_ptr(), 1, None, 0, M, N, K, ldx, ldw, N, _lib.F32, ws.data_ptr(), ws.numel(), st)
+        assert torch.equal(out, want.float() * xs.view(-1, 1) * wsc)
+        assert acc is None or torch.equal(acc, want.int())
+
+
+def test_fp8_rows_far_apart():
+    """The same for fp8: as many rows as fit are computed, more are refused."""
+    from vllm_gcu_amd import _lib
+    N, K, ldx = 16512, 128, 30_000_000
+    assert tile(SCALED, 140, N, K)[0] == 144 and tile(SCALED, 160, N, K)[0] == 160
+    w = rearrange.to_kslab((torch.randn(N, K, device="cuda") * 40).to(torch.float8_e4m3fn))
+    x = torch.empty(160 * ldx, dtype=torch.uint8, device="cuda").view(torch.float8_e4m3fn).as_strided((160, K), (ldx, 1))
+    x.copy_((torch.randn(160, K, device="cuda") * 40).to(torch.float8_e4m3fn))
+    dense, xs, wsc = x.contiguous(), torch.rand(160, device="cuda"), torch.rand(N, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+
+    def call(M, rows, stride):
+        out = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+        _lib.call("mi355q_fp8_scaled_gemm_ws", out.data_ptr(), rows.data_ptr(), w.data_ptr(), xs.data_ptr(), 1, wsc.data_ptr(), 1, None, M, N, K,
+                  stride, 0, N, _lib.BF16, None, 0, st)
+        return out
+    assert torch.equal(call(140, x, ldx), call(140, dense, K))
+    with pytest.raises(RuntimeError, match="fits neither kernel"):
+        call(160, x, ldx)

@@ -26,7 +26,7 @@ double t8_price(int mode, int M, int N, int K, int splits, int* height);
 int int8_tile_launch(void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale, int ws_mul,
                      const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldw, long ldo, int out_dtype,
                      void* workspace, size_t workspace_bytes, hipStream_t st);
-bool q8_mid_wanted(int mode, int M, int N, int K, size_t* bytes);
+bool q8_mid_wanted(int mode, int M, int N, int K, long ldx, size_t* bytes);
 int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
                   int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* partial,
                   hipStream_t st);
@@ -996,7 +996,7 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
   MQ_REQUIRE(ldo >= N && ldo % 4 == 0, "w8a8_int8_gemm: output row stride %ld must be >= N and a multiple of 4", ldo);
   MQ_REQUIRE(out_dtype >= MI355Q_F16 && out_dtype <= MI355Q_F32, "w8a8_int8_gemm: bad out dtype %d", out_dtype);
   size_t mid_bytes = 0;
-  if (kslab && !acc_out && (size_t)128 * (size_t)ldx < ((size_t)1 << 32) && q8_mid_wanted(2, M, N, K, &mid_bytes) &&
+  if (kslab && !acc_out && q8_mid_wanted(2, M, N, K, ldx, &mid_bytes) &&
       (mid_bytes == 0 || (workspace && workspace_bytes >= I8_WS_OFFSET + mid_bytes)))
     return q8_mid_launch(2, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K, ldx,
                          ldo, out_dtype, mid_bytes ? (char*)workspace + I8_WS_OFFSET : nullptr, as_stream(stream));
@@ -1004,6 +1004,17 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
       (kslab || (size_t)128 * (size_t)ldw < ((size_t)1 << 32)) && int8_pick(M, N, K).tiles128)
     return int8_tile_launch(out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K,
                             ldx, ldw, ldo, out_dtype, workspace, workspace_bytes, as_stream(stream));
+  // rows of a tile lie at 32-bit offsets from its first one: strides that a tile of 256 rows does not reach take as many rows as fit
+  const int fit = (int)std::max(1L, std::min((long)TM, ((1L << 32) - 1) / ldx));
+  if (fit < TM && M > fit) {
+    const size_t cell = out_dtype == MI355Q_F32 ? 4 : 2;
+    for (int m = 0; m < M; m += fit)
+      if (int rc = mi355q_w8a8_int8_gemm_ws((char*)out + (size_t)m * ldo * cell, acc_out ? acc_out + (size_t)m * N : nullptr, x + (size_t)m * ldx, w,
+                                            x_scale && x_scale_per_row ? x_scale + m : x_scale, x_scale_per_row, w_scale, w_scale_per_col, bias,
+                                            bias_f32, std::min(fit, M - m), N, K, ldx, ldw, ldo, out_dtype, workspace, workspace_bytes, stream))
+        return rc;
+    return 0;
+  }
   I8Args a;
   a.out = out; a.acc_out = acc_out; a.x = x; a.w = w; a.x_scale = x_scale; a.w_scale = w_scale;
   a.bias = bias; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldw = ldw; a.ldo = ldo; a.ldacc = N;
