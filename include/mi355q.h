@@ -195,6 +195,10 @@ int mi355q_q8_mid_plan(int kind, int M, int N, int K, size_t* workspace_bytes);
  * plan answers 0. */
 int mi355q_q8_mid_tile(int kind, int M, int N, int K, int* rows, int* columns, int* k_ranges);
 
+/* The rows of a tile (128 .. 256 x 128 columns) and the K ranges of the kernel for more rows (csrc/fp8_block_tile.hip; a workspace that holds
+ * the ranges) where it is the one that those entry points launch. */
+int mi355q_q8_tile_plan(int kind, int M, int N, int K, int* rows, int* k_ranges);
+
 /* ---- W8A8 int8 -------------------------------------------------------------
  * Replaces topsatenDotBiasQuant as called by cutlass_scaled_mm
  * (csrc/src/cutlass_scaled_mm.cpp:12-36) and dot_bias_quant

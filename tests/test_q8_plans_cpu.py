@@ -29,6 +29,19 @@ def int8_plan(M, N, K, kslab=True):
     return kernel.value, ranges.value
 
 
+def tile_plan(kind, M, N, K):
+    """(rows of a tile, K ranges) of the kernel for more rows, csrc/fp8_block_tile.hip"""
+    rows, ranges = c_int(), c_int()
+    _lib.call("mi355q_q8_tile_plan", kind, M, N, K, byref(rows), byref(ranges))
+    return rows.value, ranges.value
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_every_height_is_taken_somewhere(kind):
+    heights = {tile_plan(kind, M, N, K)[0] for K, N in LAYERS for M in range(65, 2049, 9) if tile(kind, M, N, K)[0] == 0}
+    assert heights == {128, 160, 192, 224, 256}
+
+
 def test_the_int8_kernel_is_the_one_that_the_others_were_compared_with():
     """Where the prices of the two tile kernels are close, the 8-bit kernel for some hundred rows gives way to the one that is launched: the
     128-column tiles here (us, 8-bit kernel / 128-column tiles / 256 rows: K 3456 x N 20096 at 362 rows 49.6 / 42.1 / 44.9)."""

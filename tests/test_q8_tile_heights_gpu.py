@@ -1,9 +1,11 @@
 """The 8-bit GEMMs on tiles of 128 .. 256 rows (csrc/fp8_block_tile.hip): row counts on both sides of every tile height, odd and
-even numbers of K blocks, one and several K ranges, row-major weights (which no other dense kernel takes at these rows) and
-kslab ones.  int8 is exact; fp8 is compared with a float64 product."""
+even numbers of K blocks, row-major weights (for int8 csrc/w8a8_int8.hip takes a few of them, for fp8 nothing else does at these rows); kslab
+weights, which csrc/q8_mid.hip takes at many of those shapes, at shapes that it leaves to every height, with one and with several K ranges.
+int8 is exact; fp8 is compared with a float64 product."""
 import pytest
 import torch
 
+from test_q8_plans_cpu import int8_plan, tile, tile_plan
 from vllm_gcu_amd import _lib
 from vllm_gcu_amd.kernels.quantization import rearrange
 
@@ -12,7 +14,20 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(m, 32768, k) for m, k in ((96, 128), (128, 256), (129, 384), (160, 128), (161, 256), (192, 384), (193, 128), (224, 640), (225, 256),
                                      (256, 384), (257, 128))]
 SHAPES += [(320, 16384, 256), (448, 16384, 384), (1537, 4096, 896), (700, 14336, 256), (130, 2048, 4096), (333, 1024, 6144), (1600, 128, 128)]
+# kslab weights: (rows of a tile, K ranges) -> shape
+SERVED = {(128, 1): (1800, 1024, 640), (160, 1): (1543, 2560, 640), (192, 1): (337, 11008, 640), (224, 1): (197, 16512, 640),
+          (256, 1): (455, 11008, 640), (128, 2): (1598, 128, 2048), (160, 5): (1540, 512, 5120), (192, 3): (1604, 1024, 3072),
+          (224, 4): (1923, 768, 4096), (256, 6): (1805, 640, 6144)}
+SHAPES += SERVED.values()
 F16, BF16, F32 = 0, 1, 2
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_kslab_weights_at_every_height(kind):
+    assert {h for h, _ in SERVED} == {128, 160, 192, 224, 256} == {h for h, ranges in SERVED if ranges > 1}
+    for plan, s in SERVED.items():
+        assert tile(kind, *s) == (0, 0, 0) and tile_plan(kind, *s) == plan
+        assert kind != 2 or int8_plan(*s) == (1, plan[1])
 
 
 def _common(M, N, K):

@@ -169,6 +169,38 @@ def test_int8_gemm_split_k_is_bit_identical(ops, M, K, N, splits, out_dtype):
     assert torch.equal(got, ops.cutlass_scaled_mm(xd, wd.t(), dev(xs), wsd, out_dtype, bias))
 
 
+@pytest.mark.parametrize("M,K,N,kslab,ranges", [(130, 2048, 260, False, 2), (64, 4096, 516, False, 4), (200, 8192, 1028, False, 8),
+                                                (1000, 3072, 772, False, 3), (2000, 4096, 192, True, 4), (1700, 2048, 1344, True, 2),
+                                                # two and three row tiles of 256 x 256
+                                                (257, 8192, 8196, False, 2), (520, 8192, 5636, False, 2)])
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_int8_k_ranges_of_the_256_row_tiles(ops, M, K, N, kslab, ranges, out_dtype):
+    """The shapes of the test above go to the 128-column tiles where their output is scaled; column counts that are no multiple of 128 do
+    not.  Scales of rows and columns, one of each and none, with and without bias of both types: exact."""
+    from test_q8_plans_cpu import int8_plan
+    from vllm_gcu_amd import _lib
+    from vllm_gcu_amd.kernels import _runtime as rt
+    from vllm_gcu_amd.kernels.quantization import rearrange
+    print(f"case i8 K ranges {M}x{K}x{N} {out_dtype}", flush=True)
+    assert int8_plan(M, N, K, kslab) == (2, ranges)
+    torch.manual_seed(M + K + N)
+    x = torch.randint(-128, 128, (M, K), dtype=torch.int8, device="cuda")
+    w = torch.randint(-128, 128, (N, K), dtype=torch.int8, device="cuda")
+    wt, ldw = (rearrange.to_kslab(w), 0) if kslab else (w, K)
+    xs, wsc = torch.rand(M, device="cuda") * 0.1, torch.rand(N, device="cuda") * 0.01
+    bias = torch.randn(N, device="cuda")
+    acc = (x.double() @ w.double().t()).float()              # below 2^53, rounded to fp32 once, as the kernel's conversion does
+    need = _lib.load().mi355q_w8a8_int8_workspace_bytes(M, N, K)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    for row, col, b in ((xs, wsc, None), (xs, wsc, bias), (xs[:1], wsc[:1], bias.to(out_dtype)), (None, None, bias)):
+        out = torch.full((M, N), float("nan"), device="cuda", dtype=out_dtype)
+        _lib.call("mi355q_w8a8_int8_gemm_ws", out.data_ptr(), None, x.data_ptr(), wt.data_ptr(), None if row is None else row.data_ptr(),
+                  int(row is xs), None if col is None else col.data_ptr(), int(col is wsc), None if b is None else b.data_ptr(),
+                  int(b is not None and b.dtype == torch.float32), M, N, K, K, ldw, N, rt.dtype_code(out_dtype), ws.data_ptr(), need, rt.stream_ptr())
+        want = acc if row is None else acc * row.view(-1, 1) * col.view(1, -1)
+        assert torch.equal(out, (want if b is None else want + b.float()).to(out_dtype))
+
+
 @pytest.mark.parametrize("M,N", [(2305, 2048), (4200, 1792), (2049, 4096)])
 def test_int8_gemm_more_than_eight_row_tiles(ops, M, N):
     # above 2048 rows the XCD-aware tile order walks the row tiles in chunks of eight (with a

@@ -38,6 +38,7 @@ SIGNATURES = {
                                       c_void_p, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_int,
                                       c_void_p]),
     "mi355q_w8a8_int8_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "mi355q_q8_tile_plan": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "mi355q_w8a8_int8_plan": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "mi355q_w8a8_int8_gemm_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
                                          c_void_p, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_int,

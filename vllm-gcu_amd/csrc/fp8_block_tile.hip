@@ -762,6 +762,15 @@ int half_grouped_tile_launch(void* out, const void* a, const void* w, const floa
 
 using namespace mi355q;
 
+extern "C" int mi355q_q8_tile_plan(int kind, int M, int N, int K, int* rows, int* k_ranges) {
+  MQ_REQUIRE(M > 0 && N > 0 && K > 0 && N % FTN == 0 && K % FTKB == 0 && kind >= 0 && kind <= 2, "q8_tile_plan: bad shape M=%d N=%d K=%d or kind %d", M,
+             N, K, kind);
+  MQ_REQUIRE(rows && k_ranges, "q8_tile_plan: null pointer");
+  *k_ranges = fp8_ksplits(M, N, K);
+  t8_price(kind, M, N, K, *k_ranges, rows);
+  return 0;
+}
+
 extern "C" size_t mi355q_fp8_gemm_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0) return 0;
   const int s = fp8_ksplits(M, N, K);
