@@ -174,7 +174,7 @@ int mi355q_fp8_scaled_gemm(void* out, const void* x, const void* w, const float*
  * launch (or, for the scaled GEMM on few tiles, the streaming kernel) runs.
  * mi355q_fp8_block_gemm_ws also uses ceil16(M) * (K / 128) * 4 bytes behind the partial sums (behind the first
  * MiB where nothing is split), when the workspace has them, from 24 K blocks of 128 on where K blocks x output
- * tiles of 256 x 128 are 11000 or more: the activation scales re-ordered K block major by a small launch of its own, so that a workgroup's
+ * tiles of 256 x 128 are 11000 or more, and up to 256 rows from 40 K blocks per range on with 80 tiles or more: the activation scales re-ordered K block major by a small launch of its own, so that a workgroup's
  * 256 scales of a K block are 1 KiB in a row instead of one value per cache line.  Same output bits. */
 size_t mi355q_fp8_gemm_workspace_bytes(int M, int N, int K);
 int mi355q_fp8_block_gemm_ws(void* out, const void* x, const void* w, const float* x_scale,

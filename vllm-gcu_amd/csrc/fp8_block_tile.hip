@@ -183,78 +183,78 @@ q8_tile_kernel(F8Args a) {
   const int elements = mytiles * nt;               // K blocks this workgroup multiplies, over all its tiles
 
   if (copies) {
-  // global -> LDS: lane = 8 * row + slot, slot p of row r receives chunk p ^ (r & 7); kslab weights
-  // chunk-major (lane = 8 * position + row, position p of an odd 8-row group holding chunk p ^ 1)
-  const int crow = lane >> 3, cchunk = (lane & 7) ^ (crow & 7);
-  uint32_t xo[XCOPIES], wo[WCOPIES], xso = 0;
-  int wsbase = 0;
-  const uint8_t *xtile, *wtile;
-  const float* xsbase = a.x_scale;
-  const long xs_kstride = (!GROUPED && a.xs_t) ? a.xs_ld : 1;       // floats between the K blocks of a row's scale
-  auto set_copy_tile = [&](int tile) {
-    int m0, n0, split;
-    tile_origin(tile, m0, n0, split);
-    long ebytes = 0;
-    int escales = 0;
-    if (GROUPED) {
-      const int* ids = a.sorted_ids + m0;
+    // global -> LDS: lane = 8 * row + slot, slot p of row r receives chunk p ^ (r & 7); kslab weights
+    // chunk-major (lane = 8 * position + row, position p of an odd 8-row group holding chunk p ^ 1)
+    const int crow = lane >> 3, cchunk = (lane & 7) ^ (crow & 7);
+    uint32_t xo[XCOPIES], wo[WCOPIES], xso = 0;
+    int wsbase = 0;
+    const uint8_t *xtile, *wtile;
+    const float* xsbase = a.x_scale;
+    const long xs_kstride = (!GROUPED && a.xs_t) ? a.xs_ld : 1;       // floats between the K blocks of a row's scale
+    auto set_copy_tile = [&](int tile) {
+      int m0, n0, split;
+      tile_origin(tile, m0, n0, split);
+      long ebytes = 0;
+      int escales = 0;
+      if (GROUPED) {
+        const int* ids = a.sorted_ids + m0;
 #pragma unroll
-      for (int p = 0; p < XCOPIES; ++p) {
-        const int id = ids[(wave + 4 * p) * 8 + crow];
-        xo[p] = (uint32_t)(max(0, min(id, a.numel - 1)) / a.topk) * (uint32_t)a.ldx + (uint32_t)(16 * cchunk);   // pads read a valid row
-      }
-      int e = a.expert_ids[m0 / BM];
-      e = __builtin_amdgcn_readfirstlane((e < 0 || e >= a.E) ? 0 : e);     // (a foreign expert's block is computed and zeroed)
-      ebytes = (long)e * a.w_stride;
-      escales = e * (int)a.ws_stride;
-    } else {
-#pragma unroll
-      for (int p = 0; p < XCOPIES; ++p) {
-        const int r = (wave + 4 * p) * 8 + crow;
-        xo[p] = (uint32_t)((min(m0 + r, M - 1) - m0) * a.ldx + 16 * cchunk);
-      }
-    }
-#pragma unroll
-    for (int p = 0; p < WCOPIES; ++p) {
-      if (MODE == T8_H16 && a.w_kslab) {
-        // 2-byte elements: a K block of the kslab order is 256 bytes per row = two of this kernel's K blocks; chunk c of
-        // K block h is vector c & 3 of lane quarter 2 h + (c >> 2)
-        const uint32_t n = (uint32_t)(n0 + (wave + 4 * p) * 8 + (lane & 7));
-        const uint32_t c = (uint32_t)((lane >> 3) ^ (wave & 1));
-        wo[p] = ((n >> 6) * (uint32_t)(K >> 8) * 4u + ((n & 63u) >> 4)) * 4096u + (c & 3u) * 1024u +
-                ((c >> 2) * 16u + (n & 15u)) * 16u;
-      } else if (a.w_kslab) {
-        const uint32_t n = (uint32_t)(n0 + (wave + 4 * p) * 8 + (lane & 7));
-        const uint32_t c = (uint32_t)((lane >> 3) ^ (wave & 1));
-        wo[p] = ((n >> 6) * (uint32_t)(K >> 7) * 4u + ((n & 63u) >> 4)) * 2048u + (c & 1u) * 1024u +
-                ((c >> 1) * 16u + (n & 15u)) * 16u;
+        for (int p = 0; p < XCOPIES; ++p) {
+          const int id = ids[(wave + 4 * p) * 8 + crow];
+          xo[p] = (uint32_t)(max(0, min(id, a.numel - 1)) / a.topk) * (uint32_t)a.ldx + (uint32_t)(16 * cchunk);   // pads read a valid row
+        }
+        int e = a.expert_ids[m0 / BM];
+        e = __builtin_amdgcn_readfirstlane((e < 0 || e >= a.E) ? 0 : e);     // (a foreign expert's block is computed and zeroed)
+        ebytes = (long)e * a.w_stride;
+        escales = e * (int)a.ws_stride;
       } else {
-        const int r = (wave + 4 * p) * 8 + crow;
-        wo[p] = (uint32_t)(r * a.ldw + 16 * cchunk);
+#pragma unroll
+        for (int p = 0; p < XCOPIES; ++p) {
+          const int r = (wave + 4 * p) * 8 + crow;
+          xo[p] = (uint32_t)((min(m0 + r, M - 1) - m0) * a.ldx + 16 * cchunk);
+        }
       }
-    }
-    // activation scales: 64 rows per copying wavefront, 128-row tiles twice (32-bit index in floats from the tile's first row;
-    // grouped: from the matrix's, whose scales the entry point keeps below 2^27 bytes)
-    const int srow = min(64 * wave + lane, BM - 1);
-    // (split K: the tile's range starts kb0 K blocks into every row; 64 kslab rows interleave their K blocks)
-    const int kb0 = ksplits > 1 ? split * (KB / ksplits) : 0;
-    if (!BLOCK) {
-    } else if (a.xs_t && !GROUPED) {
-      // K block major: the 64 scales of a copy lie side by side (4 cache lines instead of 64)
-      xso = (uint32_t)(min(m0 + srow, M - 1) - m0);
-      xsbase = a.xs_t + (long)kb0 * a.xs_ld + m0;
-    } else if (GROUPED) {
-      const int id = a.sorted_ids[m0 + srow];
-      xso = (uint32_t)(max(0, min(id, a.numel - 1)) / a.topk) * (uint32_t)KB;
-      xsbase = a.x_scale;
-    } else {
-      xso = (uint32_t)((min(m0 + srow, M - 1) - m0) * KB);
-      xsbase = a.x_scale + (long)m0 * KB + kb0;
-    }
-    wsbase = escales + (n0 >> 7) * KB + kb0;       // the first of them copies the tile's weight scale
-    xtile = GROUPED ? a.x : a.x + (long)m0 * a.ldx + (long)kb0 * FTKB;
-    wtile = a.w + ebytes + (a.w_kslab ? (long)kb0 * FTKB * 64 : (long)n0 * a.ldw + (long)kb0 * FTKB);
-  };
+#pragma unroll
+      for (int p = 0; p < WCOPIES; ++p) {
+        if (MODE == T8_H16 && a.w_kslab) {
+          // 2-byte elements: a K block of the kslab order is 256 bytes per row = two of this kernel's K blocks; chunk c of
+          // K block h is vector c & 3 of lane quarter 2 h + (c >> 2)
+          const uint32_t n = (uint32_t)(n0 + (wave + 4 * p) * 8 + (lane & 7));
+          const uint32_t c = (uint32_t)((lane >> 3) ^ (wave & 1));
+          wo[p] = ((n >> 6) * (uint32_t)(K >> 8) * 4u + ((n & 63u) >> 4)) * 4096u + (c & 3u) * 1024u +
+                  ((c >> 2) * 16u + (n & 15u)) * 16u;
+        } else if (a.w_kslab) {
+          const uint32_t n = (uint32_t)(n0 + (wave + 4 * p) * 8 + (lane & 7));
+          const uint32_t c = (uint32_t)((lane >> 3) ^ (wave & 1));
+          wo[p] = ((n >> 6) * (uint32_t)(K >> 7) * 4u + ((n & 63u) >> 4)) * 2048u + (c & 1u) * 1024u +
+                  ((c >> 1) * 16u + (n & 15u)) * 16u;
+        } else {
+          const int r = (wave + 4 * p) * 8 + crow;
+          wo[p] = (uint32_t)(r * a.ldw + 16 * cchunk);
+        }
+      }
+      // activation scales: 64 rows per copying wavefront, 128-row tiles twice (32-bit index in floats from the tile's first row;
+      // grouped: from the matrix's, whose scales the entry point keeps below 2^27 bytes)
+      const int srow = min(64 * wave + lane, BM - 1);
+      // (split K: the tile's range starts kb0 K blocks into every row; 64 kslab rows interleave their K blocks)
+      const int kb0 = ksplits > 1 ? split * (KB / ksplits) : 0;
+      if (!BLOCK) {
+      } else if (a.xs_t && !GROUPED) {
+        // K block major: the 64 scales of a copy lie side by side (4 cache lines instead of 64)
+        xso = (uint32_t)(min(m0 + srow, M - 1) - m0);
+        xsbase = a.xs_t + (long)kb0 * a.xs_ld + m0;
+      } else if (GROUPED) {
+        const int id = a.sorted_ids[m0 + srow];
+        xso = (uint32_t)(max(0, min(id, a.numel - 1)) / a.topk) * (uint32_t)KB;
+        xsbase = a.x_scale;
+      } else {
+        xso = (uint32_t)((min(m0 + srow, M - 1) - m0) * KB);
+        xsbase = a.x_scale + (long)m0 * KB + kb0;
+      }
+      wsbase = escales + (n0 >> 7) * KB + kb0;       // the first of them copies the tile's weight scale
+      xtile = GROUPED ? a.x : a.x + (long)m0 * a.ldx + (long)kb0 * FTKB;
+      wtile = a.w + ebytes + (a.w_kslab ? (long)kb0 * FTKB * 64 : (long)n0 * a.ldw + (long)kb0 * FTKB);
+    };
     // the K block that the next copies are of; past the last one a re-read that nobody consumes
     int kt = 0;
     set_copy_tile(tile);
@@ -343,10 +343,10 @@ q8_tile_kernel(F8Args a) {
   auto pj = [](int p) constexpr { return p < 8 ? NJ - 2 + (p & 1) : (p - 8) >> 2; };
   auto add = [&](int q) {                          // the product of position q joins the running sum
     if constexpr (BLOCK) {
-    acc[pi(q)][pj(q)] += sc[pj(q)] * ring[q & 3];
-    // (pinned here: left alone, the compiler gives every MFMA a result tile of its own and sinks all
-    // multiply-adds behind the last MFMA, where the matrix pipe waits for them)
-    asm volatile("" : "+v"(acc[pi(q)][pj(q)]));
+      acc[pi(q)][pj(q)] += sc[pj(q)] * ring[q & 3];
+      // (pinned here: left alone, the compiler gives every MFMA a result tile of its own and sinks all
+      // multiply-adds behind the last MFMA, where the matrix pipe waits for them)
+      asm volatile("" : "+v"(acc[pi(q)][pj(q)]));
     }
   };
   auto multiply = [&](int p) {
@@ -619,10 +619,10 @@ int fp8_split_min_rows(int N, int K, int splits) {
   return 64;
 }
 
-// with a workspace that holds the plan's partial sums: K ranges side by side; else the plain launch
 // bytes of the K block major copy of the activation scales (rows padded to whole 64-byte lines)
 size_t fp8_scales_kmajor_bytes(long rows, int K) { return (size_t)((rows + 15) / 16 * 16) * (K / FTKB) * sizeof(float); }
 
+// with a workspace that holds the plan's partial sums: K ranges side by side; else the plain launch
 template <int DT, int MODE>
 int launch_f8_auto(F8Args& a, void* workspace, size_t workspace_bytes, hipStream_t st) {
   a.ksplits = 1;
@@ -858,7 +858,7 @@ extern "C" int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w
     a.out = out; a.x = (const uint8_t*)x; a.w = (const uint8_t*)w; a.x_scale = x_scale; a.w_scale = w_scale;
     a.bias = bias; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldw = ldw; a.ldo = ldo;
     a.w_kslab = kslab ? 1 : 0;
-      a.xs_mul = x_scale_per_row ? 1 : 0;
+    a.xs_mul = x_scale_per_row ? 1 : 0;
     a.ws_mul = w_scale_per_col ? 1 : 0;
     if (out_dtype == MI355Q_F16) return launch_f8_auto<MI355Q_F16, T8_PC>(a, workspace, workspace_bytes, as_stream(stream));
     return launch_f8_auto<MI355Q_BF16, T8_PC>(a, workspace, workspace_bytes, as_stream(stream));

@@ -346,7 +346,7 @@ def _scaled_int8_mm(out, x, weight, x_scale, w_scale, bias, acc_out=None):
             bias = bias.to(torch.float32)
             bias_f32 = 1
         bias = bias.contiguous()
-    # kslab weights at some hundred rows: the kernel between the weight streamer and the 256-row tiles
+    # kslab weights at some hundred rows: the kernel between the weight streamer and the tiles of 128 to 256 rows
     mid = rt.host.q8_mid_plan(_lib.Q_INT8, M, N, K) if ldw == 0 and acc_out is None and _INT8_STREAM_MAX_M == 64 else -1
     stream_rows = 0 if mid >= 0 else rt.host.int8_stream_rows(K, N, _INT8_STREAM_MAX_M)
     # (row-major [N, K] weights: the tile kernel with its K ranges is level with the streaming kernel on
