@@ -17,9 +17,9 @@ def tile(kind, M, N, K):
 
 @pytest.mark.parametrize("kind", [0, 1, 2])
 def test_every_tile_is_taken_somewhere(kind):
-    """What is built is also chosen: fp8 with block scales, fp8 and int8 with scales outside the K sum."""
+    """What is built is also chosen: fp8 with block scales (which alone has 144 and 160 rows), fp8 and int8 with scales outside the K sum."""
     rows = {tile(kind, M, N, K)[0] for K, N in LAYERS for M in range(17, 1537)}
-    assert rows == {0, 32, 48, 64, 80, 96, 112, 128, 144, 160}
+    assert rows == {0, 32, 48, 64, 80, 96, 112, 128} | ({144, 160} if kind == 0 else set())
 
 
 def int8_plan(M, N, K, kslab=True):
