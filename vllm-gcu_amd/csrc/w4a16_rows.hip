@@ -487,7 +487,8 @@ bool w4a16_rows_wanted(int M, int K, int N, int group_size, int zeros_kind, int 
   if (M <= 32) return small || w >= (dtype == MI355Q_F16 ? 1L << 26 : 3L << 25);
   if (M <= 128) return true;
   // (the price, corrected for the size of the output and the rows by 255 launches with fp16 rows and 177 with bf16, rms errors 4.6 and 3 %.  The
-  // pick loses 0.1 / 0.2 % (fp16 / bf16) to the best of the three kernels over 23 layers at 144 .. 2048 rows, 11 % at worst, where prices tie.  The
+  // pick loses 0.1 / 0.2 % (fp16 / bf16) to the best of the three kernels over 23 layers at 144 .. 2048 rows, 15 % at worst, where prices
+  // tie: fp16 5120 x 13824 at 200 rows 53.7 us on the tiles, 46.1 here; 3584 x 37888 at 144 59.5 / 64.  The
   // loops that are not pipelined by 1300 launches, 0.2 %: bf16 with groups of 64 4096 x 6144 at 1536 100 us here, 142 there, with groups of 32
   // 117 / 180, bf16 rows that are not staged 28672 x 8192 at 170 102 / 124, fp16 with groups of 32 3584 x 37888 at 256 119 / 159.)
   const bool bf16 = dtype == MI355Q_BF16;
