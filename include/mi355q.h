@@ -405,6 +405,14 @@ int mi355q_moe_gemm(void* out, const void* a, const void* w, const float* a_scal
 int mi355q_moe_w4a16_unsorted(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
                               int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64, int numel, int topk,
                               int E, int K, int N, int silu_and_mul, int dtype, void* stream);
+/* The second GEMM of a fused-MoE layer over up to 64 unaligned slots (a [rows * topk, K], one row per slot) and the sum of each token's
+ * slots, out [rows, N]: what mi355q_moe_w4a16_unsorted with topk_weights and mi355q_moe_sum make one after the other, but for the order
+ * of the fp32 additions along K, which is cut into ranges whose f32 sums go through the workspace
+ * (mi355q_moe_w4a16_unsorted_sum_bytes). */
+size_t mi355q_moe_w4a16_unsorted_sum_bytes(int numel, int E, int K, int N);
+int mi355q_moe_w4a16_unsorted_sum(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
+                                  int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64, int rows, int topk,
+                                  int E, int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 /* Dense calls of the same kernels (quant_mode 1..4), replacing topsatenLinearQuant
  * as called by linear_quant (csrc/src/linear_quant.cpp:16-95, fp8 block-scaled
  * C = sum_kb (A_kb B_kb^T) As Bs) and by weight_only_quant

@@ -217,3 +217,34 @@ def test_unsorted_slots_of_every_form(E, K, N, g, kind, dtype):
             act = torch.full((numel, N // 2), float("nan"), dtype=dtype, device="cuda")
             _lib.check(lib.mi355q_silu_and_mul(act.data_ptr(), plain.data_ptr(), numel, N // 2, code, None, 1, st), "silu_and_mul")
             assert torch.equal(glu[keep], act[keep]) and glu[~keep].isnan().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("E,K,N,rows,topk,ranges", [(8, 6272, 4096, 2, 2, 2), (8, 6144, 4096, 3, 2, 4), (8, 3072, 4096, 3, 2, 2), (8, 2944, 4096, 3, 2, 1),
+                                                    (16, 6272, 3072, 16, 2, 2), (3, 256, 512, 64, 1, 1), (60, 384, 256, 10, 6, 1)])
+def test_unsorted_sum(E, K, N, rows, topk, ranges, dtype):
+    """The second GEMM whose K ranges and slots are added by one launch: the bits of the GEMM and moe_sum one after the other where every
+    sum along K is exact, for the ranges the shape is cut into (also uneven ones)."""
+    from vllm_gcu_amd import _lib
+    lib, g, numel = _lib.load(), 128, rows * topk
+    code = _lib.F16 if dtype == torch.float16 else _lib.BF16
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // 8, N), dtype=torch.int32, device="cuda", generator=gen)
+    zp = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // g, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    s = (2.0 ** torch.randint(-9, -6, (E, K // g, N), device="cuda", generator=gen)).to(dtype)
+    x = torch.randint(-4, 5, (numel, K), device="cuda", generator=gen).to(dtype)
+    rw = torch.rand(numel, device="cuda", generator=gen)
+    ids = torch.randint(0, E, (rows, topk), device="cuda", generator=gen, dtype=torch.int32)
+    st = torch.cuda.current_stream().cuda_stream
+    need = lib.mi355q_moe_w4a16_unsorted_sum_bytes(numel, E, K, N)
+    assert need == ranges * numel * N * 4
+    ws = torch.full((need // 4,), float("nan"), device="cuda")
+    got, want = (torch.full((rows, N), float("nan"), dtype=dtype, device="cuda") for _ in range(2))
+    slots = torch.empty(numel, N, dtype=dtype, device="cuda")
+    common = (w.data_ptr(), s.data_ptr(), zp.data_ptr(), _lib.ZP_PACKED, g, rw.data_ptr(), ids.data_ptr(), 0)
+    _lib.check(lib.mi355q_moe_w4a16_unsorted_sum(got.data_ptr(), x.data_ptr(), *common, rows, topk, E, K, N, code, ws.data_ptr(), need, st),
+               "moe_w4a16_unsorted_sum")
+    _lib.check(lib.mi355q_moe_w4a16_unsorted(slots.data_ptr(), x.data_ptr(), *common, numel, 1, E, K, N, 0, code, st), "moe_w4a16_unsorted")
+    _lib.check(lib.mi355q_moe_sum(want.data_ptr(), slots.data_ptr(), rows, topk, N, code, code, None, st), "moe_sum")
+    assert torch.equal(got, want)
+    assert lib.mi355q_moe_w4a16_unsorted_sum(got.data_ptr(), x.data_ptr(), *common, rows, topk, E, K, N, code, ws.data_ptr(), need - 4, st) != 0

@@ -605,6 +605,11 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
   }
   const int64_t blocks = (numel + E * (block - 1)) / block;
   const bool quant = mode != kW4;
+  // A wavefront's worth of slots in blocks of 16: the GEMMs sort them themselves, and the first applies the gate, where its launch counts:
+  // sixty experts of 2048 x 2816 at 1 / 8 / 16 tokens 32.2 / 39.9 / 51.2 -> 29.5 / 37.8 / 49.3 us, sixteen of 3072 x 8192 at 3 / 16 39.2 / 63.7 ->
+  // 36.7 / 62.7; eight of 4096 x 28672 at 1 / 5 / 16 48.6 / 103.2 / 132.5 and 47.5 / 104.1 / 132.4: two streams of weights instead of one.
+  const bool unsorted = mode == kW4 && block == 16 && numel <= 64 && group % 128 == 0 && K % 128 == 0 && N % 128 == 0 && I % 128 == 0;
+  const bool gate = unsorted && N * K <= (1 << 26), ids64 = ids.scalar_type() == at::kLong;
   // one allocation: quantised inputs of both GEMMs with their scales, the three intermediate matrices, the alignment
   int64_t total = 0;
   auto room = [&total](int64_t bytes) {
@@ -618,6 +623,8 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
   const int64_t o_c2 = room(mode == kFp8 ? 0 : numel * I * 2);
   const int64_t o_q2 = room(quant ? numel * I : 0), o_s2 = room(quant ? numel * s_cols2 * 4 : 0);
   const int64_t o_sorted = room((numel + E * (block - 1)) * 4), o_eid = room(blocks * 4), o_npp = room(4);
+  const size_t sums = unsorted ? mi355q_moe_w4a16_unsorted_sum_bytes(numel, E, I, K) : 0;      // of the second GEMM's K ranges
+  const int64_t o_sums = room(sums);
   const size_t need = std::max(mi355q_moe_gemm_workspace_bytes(mode, numel, block, blocks, E, K, N),
                                mi355q_moe_gemm_workspace_bytes(mode, numel, block, blocks, E, I, K));
   const OnDevice on(x);
@@ -642,11 +649,6 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
     else if (mode == kInt8)
       check(mi355q_dynamic_int8_quant(reinterpret_cast<int8_t*>(b + o_q1), s1, x.data_ptr(), M, K, code, nullptr, stream),
             "dynamic_int8_quant");
-    // A wavefront's worth of slots in blocks of 16: the GEMMs sort them themselves, and the first applies the gate, where its launch counts:
-    // sixty experts of 2048 x 2816 at 1 / 8 / 16 tokens 32.2 / 39.9 / 51.2 -> 29.5 / 37.8 / 49.3 us, sixteen of 3072 x 8192 at 3 / 16 39.2 / 63.7 ->
-    // 36.7 / 62.7; eight of 4096 x 28672 at 1 / 5 / 16 48.6 / 103.2 / 132.5 and 47.5 / 104.1 / 132.4: two streams of weights instead of one.
-    const bool unsorted = mode == kW4 && block == 16 && numel <= 64 && group % 128 == 0 && K % 128 == 0 && N % 128 == 0 && I % 128 == 0;
-    const bool gate = unsorted && N * K <= (1 << 26), ids64 = ids.scalar_type() == at::kLong;
     if (!unsorted)
       check(mi355q_moe_align_block_size(ids.data_ptr(), ids64, numel, T, nullptr, E, block, nullptr, sorted, eid, npp, stream), "moe_align_block_size");
     if (unsorted)
@@ -667,17 +669,18 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
     if (mode == kInt8)
       check(mi355q_dynamic_int8_quant(reinterpret_cast<int8_t*>(b + o_q2), s2, b + o_c2, numel, I, code, nullptr, stream),
             "dynamic_int8_quant");
-    if (unsorted)
-      check(mi355q_moe_w4a16_unsorted(b + o_c1, b + o_c2, static_cast<const int32_t*>(w2.data_ptr()), s2p->data_ptr(), ptr(z2),
-                                      z2.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, group, static_cast<const float*>(tw.data_ptr()),
-                                      ids.data_ptr(), ids64, numel, 1, E, I, K, 0, code, stream),
-            "moe_w4a16_unsorted");
-    else
+    if (unsorted) {
+      check(mi355q_moe_w4a16_unsorted_sum(out.data_ptr(), b + o_c2, static_cast<const int32_t*>(w2.data_ptr()), s2p->data_ptr(), ptr(z2),
+                                          z2.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, group, static_cast<const float*>(tw.data_ptr()),
+                                          ids.data_ptr(), ids64, M, T, E, I, K, code, b + o_sums, sums, stream),
+            "moe_w4a16_unsorted_sum");
+    } else {
       check(mi355q_moe_gemm(b + o_c1, quant ? b + o_q2 : b + o_c2, w2.data_ptr(), quant ? s2 : nullptr, s2p->data_ptr(), ptr(z2),
-                          z2.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, mode, group, static_cast<const float*>(tw.data_ptr()), sorted,
-                          eid, npp, numel, 1, block, blocks, E, I, K, act, code, quant, ws.p, ws.bytes, stream),
-          "moe_gemm");
-    check(mi355q_moe_sum(out.data_ptr(), b + o_c1, M, T, K, code, code, nullptr, stream), "moe_sum");
+                           z2.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, mode, group, static_cast<const float*>(tw.data_ptr()), sorted,
+                           eid, npp, numel, 1, block, blocks, E, I, K, act, code, quant, ws.p, ws.bytes, stream),
+            "moe_gemm");
+      check(mi355q_moe_sum(out.data_ptr(), b + o_c1, M, T, K, code, code, nullptr, stream), "moe_sum");
+    }
   }
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS

@@ -41,6 +41,8 @@ struct DecodeArgs {
   int numel, topk, E;
   int id_step, id_bits;         // launches without an alignment: sorted_ids are the slots' experts, int32 per id, bits of an expert
   long w_stride, s_stride, z_stride;   // bytes per expert
+  int kper;                     // K blocks per range (blockIdx.y)
+  float* partial;               // f32 sums [range][numel][N], without the routing weights; null: write the output
 };
 
 template <int DT> struct DecodeMma;
@@ -334,9 +336,9 @@ w4a16_decode_grouped_kernel(DecodeArgs a) {
                                 (uint32_t)a.qrows * (ZK == MI355Q_ZP_PRESCALED ? N * 2u : (N >> 1)));
   const rsrc_t xres = make_rsrc(a.x, (uint32_t)a.M * K * 2u);
   const uint32_t wlane = (uint32_t)(t0 * 64 + lane) * 16u;
-  const int nb = (G - wave + W - 1) / W;
+  const int g0 = (int)blockIdx.y * a.kper + wave, nb = (min(G - (int)blockIdx.y * a.kper, a.kper) - wave + W - 1) / W;
   auto load = [&](Block& b, int i) {
-    const int g = wave + W * min(i, nb);
+    const int g = g0 + W * min(i, nb);
     const uint32_t oob = i < nb ? 0u : 0x80000000u;            // past the last block: zeros, no traffic
 #pragma unroll
     for (int t = 0; t < NT; ++t) b.w[t] = buf_load16_nt(GLU && t >= CT ? upres : wres, wlane + (uint32_t)g * 8192u + oob + (t % CT) * 1024);
@@ -367,7 +369,7 @@ w4a16_decode_grouped_kernel(DecodeArgs a) {
     for (int j = 0; j < XN; ++j) xlane[j] = ((uint32_t)(min(slot_id(4 * j + kq), a.numel - 1) / a.topk) * (uint32_t)K + 8u * c) * 2u;   // (pads read a valid row)
     u4 xv[XN];
     auto load_x = [&](int i) {
-      const uint32_t at = (uint32_t)(wave + W * min(i, nb)) * 256u + (i < nb ? 0u : 0x80000000u);
+      const uint32_t at = (uint32_t)(g0 + W * min(i, nb)) * 256u + (i < nb ? 0u : 0x80000000u);
 #pragma unroll
       for (int j = 0; j < XN; ++j) xv[j] = buf_load16(xres, xlane[j] + at);
     };
@@ -439,14 +441,29 @@ w4a16_decode_grouped_kernel(DecodeArgs a) {
   const int q0 = wave * CW, ri = q0 / NT, tc = q0 % NT;
   const int id = slot_id(4 * kq + ri);
   if (id >= a.numel) return;
-  const float rw = a.topk_weights ? a.topk_weights[id] : 1.0f;
   float fin[CW];
 #pragma unroll
   for (int t = 0; t < CW; ++t) {
     float v = red[0][q0 + t][lane];
 #pragma unroll
     for (int w = 1; w < W; ++w) v += red[w][q0 + t][lane];
-    fin[t] = a.topk_weights ? v * rw : v;
+    fin[t] = v;
+  }
+  if (a.partial) {
+    float* const p = a.partial + ((size_t)blockIdx.y * a.numel + id) * N + ncol + tc;
+    if constexpr (CW % 4 == 0) {
+#pragma unroll
+      for (int t = 0; t < CW; t += 4) *(f4*)(p + t) = (f4){fin[t], fin[t + 1], fin[t + 2], fin[t + 3]};
+    } else {
+#pragma unroll
+      for (int t = 0; t < CW; ++t) p[t] = fin[t];
+    }
+    return;
+  }
+  if (a.topk_weights) {
+    const float rw = a.topk_weights[id];
+#pragma unroll
+    for (int t = 0; t < CW; ++t) fin[t] *= rw;
   }
   store_row<DT, CW>(a.out + (size_t)id * N + ncol + tc, nullptr, fin);
 }
@@ -543,10 +560,57 @@ GroupedPlan grouped_plan(int numel, int max_blocks, int E, int N) {
   return {8, 4};
 }
 
+// K ranges of the second GEMM.  Quarters of a slab with fewer than three workgroups per CU leave CUs with one more than others, and a CU
+// takes no more than its 25 GB/s from memory: half or a quarter of K each, their sums added by the launch that adds the slots, even that out.  (us
+// for the layer, fp16, 1 / 2 / 4 ranges; eight experts of 4096 x 28672 and 14336 x 4096 at 2 / 3 / 5 tokens, 211 / 282 / 378 workgroups 80.7 / 97.7 /
+// 104.2, 77.8 / 96.2 / 100.6, 78.6 / 92.4 / 100.5; sixteen of 3072 x 12288 and 6144 x 3072 at 4 / 16 / 32 51.2 / 85.2 / 95.4, 50.8 / 82.9 / 95.0,
+// 49.3 / 83.6 / 96.2.  Whole slabs and short K lose: eight experts at 16 tokens 136 / 141 / 145, sixty of 1408 x 2048 at 4 31.3 / 34.4 / 36.1.)
+int sum_ranges(int numel, int E, int K, int N) {
+  const GroupedPlan p = grouped_plan(numel, std::min(numel, (numel + E * 15) / 16), E, N);
+  if (p.nt != 4) return 1;
+  const long cus = device_cu_count();
+  const double wgs = N / 64 * E * (1.0 - std::pow(1.0 - 1.0 / E, numel));
+  const int s = wgs > 3 * cus ? 1 : wgs > 2 * cus || wgs <= cus ? 2 : 4;
+  return std::min(s, K / 128 >= 48 ? 4 : K / 128 >= 24 ? 2 : 1);
+}
+
+// out[m, n] = sum over a token's slots of the slot's sum over the K ranges times its routing weight, rounded to the output type as
+// the grouped GEMM and moe_sum round it one after the other.  (Bound by its launch; f32 sums from the GEMM cost nothing next to rounded ones:
+// eight experts of 4096 x 14336 at 16 / 32 tokens, one range, 139 / 146 -> 136 / 142 us for the layer.)
+template <int DT, int S>
+__global__ void __launch_bounds__(256)
+moe_range_sum_kernel(uint16_t* out, const float* partial, const float* topk_weights, uint32_t rows, int T, FastDiv quads) {
+  const uint32_t q = blockIdx.x * 256 + threadIdx.x;
+  if (q >= rows * quads.d) return;
+  const uint32_t m = quads.div(q), n = q - m * quads.d;
+  const size_t step = (size_t)rows * T * quads.d;
+  f4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < T; ++t) {
+    const f4* const p = (const f4*)partial + ((size_t)m * T + t) * quads.d + n;
+    f4 v[S];
+#pragma unroll
+    for (int r = 0; r < S; ++r) v[r] = p[r * step];
+    const float rw = topk_weights[m * T + t];
+#pragma unroll
+    for (int r = 1; r < S; ++r) v[0] += v[r];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float p = v[0][e] * rw;
+      asm volatile("" : "+v"(p));                      // (a product of its own, as the GEMM's: not one that is rounded to 16 bits at once)
+      acc[e] += Elem<DT>::to_f32(Elem<DT>::from_f32(p));
+    }
+  }
+  u2 o;
+  o.x = (uint32_t)Elem<DT>::from_f32(acc[0]) | ((uint32_t)Elem<DT>::from_f32(acc[1]) << 16);
+  o.y = (uint32_t)Elem<DT>::from_f32(acc[2]) | ((uint32_t)Elem<DT>::from_f32(acc[3]) << 16);
+  ((u2*)out)[q] = o;
+}
+
 template <int DT, int ZK, bool IDS, bool GLU = false>
 void launch_grouped(const DecodeArgs& a, GroupedPlan p, int blocks, hipStream_t st) {
+  const int ranges = (a.K / 128 + a.kper - 1) / a.kper;
 #define MQ_G(NT, W) \
-  if (p.nt == NT && p.w == W) hipLaunchKernelGGL((w4a16_decode_grouped_kernel<DT, ZK, NT, W, IDS, GLU>), dim3(a.N / 128 * (8 / NT), 1, blocks), dim3(64 * W), 0, st, a)
+  if (p.nt == NT && p.w == W) hipLaunchKernelGGL((w4a16_decode_grouped_kernel<DT, ZK, NT, W, IDS, GLU>), dim3(a.N / 128 * (8 / NT), ranges, blocks), dim3(64 * W), 0, st, a)
   MQ_G(8, 4); MQ_G(8, 8); MQ_G(4, 4);
   if constexpr (GLU) {
     MQ_G(4, 8);
@@ -560,7 +624,8 @@ void launch_grouped(const DecodeArgs& a, GroupedPlan p, int blocks, hipStream_t 
 // expert_ids null: sorted_ids are the experts of the slots themselves, id_step words apart.  glu: out [numel, N / 2] (packed zero-points or none)
 int w4a16_decode_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
                                 const float* topk_weights, const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
-                                int numel, int topk, int max_blocks, int E, int K, int N, int group_size, int dtype, hipStream_t st, int id_step = 1, bool glu = false) {
+                                int numel, int topk, int max_blocks, int E, int K, int N, int group_size, int dtype, hipStream_t st, int id_step = 1, bool glu = false,
+                                int kper = 0, float* partial = nullptr) {
   MQ_REQUIRE(group_size % 128 == 0 && K % 128 == 0 && N % 128 == 0,
              "moe_w4a16(decode): K=%d, N=%d and group_size=%d must be multiples of 128", K, N, group_size);
   const int rows = numel / (topk > 0 ? topk : 1) + 1;
@@ -581,6 +646,8 @@ int w4a16_decode_grouped_launch(void* out, const void* x, const int32_t* qweight
   a.w_stride = (long)K * N / 2;
   a.s_stride = (long)(K / group_size) * N * 2;
   a.z_stride = zeros_kind == MI355Q_ZP_PACKED ? (long)(K / group_size) * N / 2 : a.s_stride;
+  a.kper = kper > 0 ? kper : K / 128;
+  a.partial = partial;
   GroupedPlan p = grouped_plan(numel, max_blocks, E, N);
   if (glu && p.nt == 2) p.nt = 4;                    // (pairs of tiles)
 #define MQ_IDS(DT, ZK)                                                       \
@@ -622,4 +689,45 @@ extern "C" int mi355q_moe_w4a16_unsorted(void* out, const void* a, const int32_t
              "moe_w4a16_unsorted: SiLU of gate and up takes N=%d in two halves of whole slabs, zero-points that are not pre-scaled and no routing weights", N);
   return w4a16_decode_grouped_launch(out, a, w, w_scale, w_zeros, zeros_kind, topk_weights, (const int32_t*)topk_ids, nullptr, nullptr, numel, topk,
                                      std::min(numel, (numel + E * 15) / 16), E, K, N, group_size, dtype, as_stream(stream), ids_are_int64 ? 2 : 1, silu_and_mul != 0);
+}
+
+extern "C" size_t mi355q_moe_w4a16_unsorted_sum_bytes(int numel, int E, int K, int N) {
+  return numel > 0 && E > 0 && K > 0 && N > 0 ? (size_t)sum_ranges(numel, E, K, N) * numel * N * sizeof(float) : 0;
+}
+
+extern "C" int mi355q_moe_w4a16_unsorted_sum(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
+                                             int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64, int rows, int topk,
+                                             int E, int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  MQ_REQUIRE(rows >= 0 && topk > 0 && rows <= 64 / topk && E > 0 && K > 0 && N > 0, "moe_w4a16_unsorted_sum: bad shape rows=%d topk=%d E=%d K=%d N=%d", rows,
+             topk, E, K, N);
+  if (rows == 0) return 0;
+  MQ_REQUIRE(out && a && w && w_scale && topk_ids && topk_weights && workspace, "moe_w4a16_unsorted_sum: null pointer");
+  MQ_REQUIRE(zeros_kind >= MI355Q_ZP_NONE && zeros_kind <= MI355Q_ZP_PRESCALED && (zeros_kind == MI355Q_ZP_NONE || w_zeros),
+             "moe_w4a16_unsorted_sum: zeros_kind %d", zeros_kind);
+  MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "moe_w4a16_unsorted_sum: dtype %d", dtype);
+  MQ_REQUIRE(group_size > 0 && K % group_size == 0 && (size_t)N * K < ((size_t)1 << 31), "moe_w4a16_unsorted_sum: group_size=%d K=%d N=%d", group_size, K, N);
+  const int numel = rows * topk, G = K / 128;
+  int s = sum_ranges(numel, E, K, N);
+  MQ_REQUIRE(workspace_bytes >= (size_t)s * numel * N * sizeof(float), "moe_w4a16_unsorted_sum: workspace of %zu bytes", workspace_bytes);
+  const int kper = (G + s - 1) / s;
+  MQ_REQUIRE((G + kper - 1) / kper == s, "moe_w4a16_unsorted_sum: %d K blocks in %d ranges", G, s);
+  hipStream_t st = as_stream(stream);
+  const int rc = w4a16_decode_grouped_launch(nullptr, a, w, w_scale, w_zeros, zeros_kind, nullptr, (const int32_t*)topk_ids, nullptr, nullptr, numel, 1,
+                                             std::min(numel, (numel + E * 15) / 16), E, K, N, group_size, dtype, st, ids_are_int64 ? 2 : 1, false, kper,
+                                             (float*)workspace);
+  if (rc) return rc;
+  const FastDiv quads((uint32_t)(N / 4));
+  const dim3 grid((unsigned)(((size_t)rows * (N / 4) + 255) / 256));
+#define MQ_S(DT, S) \
+  if (s == S) hipLaunchKernelGGL((moe_range_sum_kernel<DT, S>), grid, dim3(256), 0, st, (uint16_t*)out, (const float*)workspace, topk_weights, (uint32_t)rows, topk, quads)
+#define MQ_DT(DT)                                      \
+  do {                                                 \
+    MQ_S(DT, 1); MQ_S(DT, 2); MQ_S(DT, 4);             \
+  } while (0)
+  if (dtype == MI355Q_F16) MQ_DT(MI355Q_F16);
+  else MQ_DT(MI355Q_BF16);
+#undef MQ_DT
+#undef MQ_S
+  MQ_LAUNCH_CHECK("moe_w4a16_unsorted_sum");
+  return 0;
 }

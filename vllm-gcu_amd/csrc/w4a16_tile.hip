@@ -1154,7 +1154,8 @@ static int tile_launch_dense(void* out, const void* x, const int32_t* qweight, c
 int w4a16_decode_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales,
                                 const void* zeros, int zeros_kind, const float* topk_weights,
                                 const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
-                                int numel, int topk, int max_blocks, int E, int K, int N, int group_size, int dtype, hipStream_t st, int id_step, bool glu);
+                                int numel, int topk, int max_blocks, int E, int K, int N, int group_size, int dtype, hipStream_t st, int id_step, bool glu,
+                                int kper, float* partial);
 int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
                               const float* topk_weights, const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                               int numel, int topk, int block_size, int max_blocks, int E, int K, int N, int group_size, int dtype,
@@ -1221,7 +1222,7 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   // launches reads faster than the tile kernel with one row tile (it takes groups that are multiples of 128 only).
   if (block_size == 16 && plain && !small_groups)
     return w4a16_decode_grouped_launch(out, x, qweight, scales, zeros, zeros_kind, topk_weights, sorted_ids,
-                                       expert_ids, npp, numel, topk, max_blocks, E, K, N, group_size, dtype, st, 1, false);
+                                       expert_ids, npp, numel, topk, max_blocks, E, K, N, group_size, dtype, st, 1, false, 0, nullptr);
   TileArgs a = {};
   a.out = (uint16_t*)out;
   a.x = (const uint16_t*)x;
