@@ -413,6 +413,12 @@ size_t mi355q_moe_w4a16_unsorted_sum_bytes(int numel, int E, int K, int N);
 int mi355q_moe_w4a16_unsorted_sum(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
                                   int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64, int rows, int topk,
                                   int E, int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+/* mi355q_moe_gemm with quant_mode 1 whose columns are gate and up, and mi355q_fp8_group_quant with fuse_silu_mul over groups of 128 of its
+ * result in act_dtype, in one launch and bit for bit: out e4m3fn [numel, N / 2], out_scales [numel, N / 256].  Blocks of 16, 32 or 64 slots,
+ * N % 256 == 0. */
+int mi355q_moe_fp8_gate_up_quant(uint8_t* out, float* out_scales, const void* a, const void* w, const float* a_scale, const float* w_scale,
+                                 const int32_t* sorted_token_ids, const int32_t* expert_ids, const int32_t* num_tokens_post_pad, int numel,
+                                 int topk, int block_size, int max_blocks, int E, int K, int N, int act_dtype, int w_layout, void* stream);
 /* Dense calls of the same kernels (quant_mode 1..4), replacing topsatenLinearQuant
  * as called by linear_quant (csrc/src/linear_quant.cpp:16-95, fp8 block-scaled
  * C = sum_kb (A_kb B_kb^T) As Bs) and by weight_only_quant

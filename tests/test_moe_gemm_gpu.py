@@ -875,3 +875,40 @@ def test_grouped_split_k_leaves_rows_of_dropped_ids_alone(fmoe, ops, rearrange):
         want = (x[t].float().numpy() @ ow4.dequantize(q[e], z[e], s[e].astype(np.float32), 128)) * tw[t, 0]
         np.testing.assert_allclose(got[t], want, rtol=RTOL, atol=ATOL)
     assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block", [16, 32, 64])
+@pytest.mark.parametrize("E,K,N,numel,topk", [(1, 128, 256, 1, 1), (3, 384, 512, 50, 2), (8, 1024, 768, 300, 6), (5, 256, 4096, 64, 1)])
+def test_fp8_gate_up_quant(E, K, N, numel, topk, block, dtype):
+    """The first fp8 expert GEMM with the gate and the group quantiser in its epilogue: codes and scales bit for bit those of the GEMM and
+    the quantiser one after the other, for both weight orders, ragged blocks, foreign experts (zeros) and an expert whose sums are zero."""
+    from vllm_gcu_amd import _lib
+    from vllm_gcu_amd.kernels import fused_moe
+    from vllm_gcu_amd.kernels.quantization import rearrange
+    lib, code, st = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device="cuda").manual_seed(E * K + N + block)
+    x = (torch.randn(numel // topk, K, device="cuda", generator=gen) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)
+    xs = torch.rand(numel // topk, K // 128, device="cuda", generator=gen) * 0.01 + 1e-4
+    w = (torch.randn(E, N, K, device="cuda", generator=gen) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)
+    ws = torch.rand(E, N // 128, K // 128, device="cuda", generator=gen) * 1e-3 + 1e-5
+    ws[0] = 0 if E > 1 else ws[0]
+    ids = torch.randint(0, E, (numel // topk, topk), device="cuda", generator=gen, dtype=torch.int32)
+    so, ex, npp = fused_moe.moe_align_block_size(ids, block, E)
+    if E > 2:
+        ex[1] = -1                                           # as an expert map makes of an expert of another rank
+    I = N // 2
+    for layout in (0, 1):
+        wk = rearrange.to_kslab(w) if layout else w
+        sums = torch.full((numel, N), float("nan"), dtype=dtype, device="cuda")
+        want, got = (torch.full((numel, I), 77, dtype=torch.uint8, device="cuda") for _ in range(2))
+        want_s, got_s = (torch.full((numel, I // 128), float("nan"), device="cuda") for _ in range(2))
+        _lib.check(lib.mi355q_moe_gemm(sums.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), ws.data_ptr(), None, 0, 1, 128, None,
+                                       so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, topk, block, ex.numel(), E, K, N, _lib.F16, code,
+                                       layout, None, 0, st), "moe_gemm")
+        _lib.check(lib.mi355q_fp8_group_quant(want.data_ptr(), want_s.data_ptr(), sums.data_ptr(), numel, I, 128, 1, code, None, 1, st),
+                   "fp8_group_quant")
+        _lib.check(lib.mi355q_moe_fp8_gate_up_quant(got.data_ptr(), got_s.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), ws.data_ptr(),
+                                                    so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, topk, block, ex.numel(), E, K, N, code,
+                                                    layout, st), "moe_fp8_gate_up_quant")
+        assert torch.equal(got, want) and torch.equal(got_s, want_s) and not got_s.isnan().any()

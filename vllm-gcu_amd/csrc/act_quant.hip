@@ -11,7 +11,6 @@
 namespace mi355q {
 namespace {
 
-constexpr float FP8_MAX = 448.0f;
 
 template <int DT> struct E16 { typedef Elem<DT> T; };
 
@@ -31,11 +30,6 @@ __device__ __forceinline__ u4 pack8(const float* f) {
     v[i] = (uint32_t)Elem<DT>::from_f32(f[2 * i]) | ((uint32_t)Elem<DT>::from_f32(f[2 * i + 1]) << 16);
   return v;
 }
-template <int DT>
-__device__ __forceinline__ float round_act(float f) {
-  return Elem<DT>::to_f32(Elem<DT>::from_f32(f));
-}
-
 // 8 floats (already within +-448) -> 8 e4m3fn codes, round to nearest even
 __device__ __forceinline__ u2 to_fp8x8(const float* y) {
   u2 r;
@@ -48,28 +42,6 @@ __device__ __forceinline__ u2 to_fp8x8(const float* y) {
   r.y = (uint32_t)w1;
   return r;
 }
-
-__device__ __forceinline__ float clamp448(float y) { return fminf(fmaxf(y, -FP8_MAX), FP8_MAX); }
-
-// a / s for many a and one s, with the result of the IEEE division: the reciprocal estimate and
-// its Newton step are made once per divisor, the quotient estimate and its two residual
-// corrections once per dividend -- the same fused multiply-adds the division expands to, without
-// the operand scaling that only matters when s, 1 / s, a / s or a residual leave the normal range.
-// For the dynamic scales here s = max(absmax, 1e-10) / 448 is normal, |a / s| <= 448, and a
-// residual can only underflow where the quotient is far below the smallest fp8 step.
-struct SharedDivisor {
-  float s, y;
-  __device__ __forceinline__ explicit SharedDivisor(float s_) : s(s_) {
-    const float y0 = __builtin_amdgcn_rcpf(s_);
-    y = __builtin_fmaf(__builtin_fmaf(-s_, y0, 1.0f), y0, y0);
-  }
-  __device__ __forceinline__ float div(float a) const {
-    const float q0 = a * y;
-    const float q1 = __builtin_fmaf(__builtin_fmaf(-s, q0, a), y, q0);
-    // the division's own last instruction: signed zeros, infinities and NaN as IEEE has them
-    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-s, q1, a), y, q1), s, a);
-  }
-};
 
 // Rows of this launch that count: `rows` of them, or up to the device's row count (times rows per count) less the `row0` rows of
 // the launches before this one.

@@ -241,6 +241,34 @@ __device__ __forceinline__ float silu_mul(float a, float b) {
   return a * (1.0f / (1.0f + expf(-a))) * b;      // left * sigmoid(left) * right
 }
 
+constexpr float FP8_MAX = 448.0f;
+template <int DT>
+__device__ __forceinline__ float round_act(float f) {
+  return Elem<DT>::to_f32(Elem<DT>::from_f32(f));
+}
+
+__device__ __forceinline__ float clamp448(float y) { return fminf(fmaxf(y, -FP8_MAX), FP8_MAX); }
+
+// a / s for many a and one s, with the result of the IEEE division: the reciprocal estimate and
+// its Newton step are made once per divisor, the quotient estimate and its two residual
+// corrections once per dividend -- the same fused multiply-adds the division expands to, without
+// the operand scaling that only matters when s, 1 / s, a / s or a residual leave the normal range.
+// For the dynamic scales here s = max(absmax, 1e-10) / 448 is normal, |a / s| <= 448, and a
+// residual can only underflow where the quotient is far below the smallest fp8 step.
+struct SharedDivisor {
+  float s, y;
+  __device__ __forceinline__ explicit SharedDivisor(float s_) : s(s_) {
+    const float y0 = __builtin_amdgcn_rcpf(s_);
+    y = __builtin_fmaf(__builtin_fmaf(-s_, y0, 1.0f), y0, y0);
+  }
+  __device__ __forceinline__ float div(float a) const {
+    const float q0 = a * y;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-s, q0, a), y, q0);
+    // the division's own last instruction: signed zeros, infinities and NaN as IEEE has them
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-s, q1, a), y, q1), s, a);
+  }
+};
+
 // Launch shape of the kernels that hold one row of K elements of 16 bits in registers (8 per lane and piece) between
 // two passes over it: threads per row and pieces per lane.  Four pieces per lane at most where there are rows
 // enough to fill the chip; with fewer rows than that a row is spread over more wavefronts, because the launch then

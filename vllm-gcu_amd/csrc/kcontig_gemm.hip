@@ -50,6 +50,8 @@ struct KcArgs {
   const float* topk_weights;
   int numel, topk, block_size, E;
   long w_stride, ws_stride;    // per-expert strides (elements)
+  uint8_t* q_out;              // GLUQ: e4m3fn codes [numel, N / 2] and their scales [numel, N / 256]
+  float* q_scales;
 };
 
 template <int MODE> struct Kc;
@@ -119,9 +121,16 @@ __device__ __forceinline__ void s8x16_to_bf16(const u4& v, u4& lo, u4& hi) {
 // NI (KS only): 16-column tiles per workgroup, 4, 2 or 1 -- a layer of a few thousand columns has only 64
 // to 128 groups of 64 columns, a quarter to half of the CUs; with 32 or 16 columns per workgroup every
 // CU streams a share of the weights (and reads the activations once more per workgroup).
-template <int MODE, int ODT, int MT, bool GROUPED, bool KS = false, int NI = 4>
+// GLUQ (grouped fp8): the columns are gate and up.  Two wavefronts take 128 gate columns, which are one group of the quantiser that
+// follows, and two the up columns that go with them; what leaves the workgroup is silu(gate) * up as e4m3fn codes and one scale per row, bit
+// for bit what mi355q_fp8_group_quant makes of the rounded sums.  Its launch is saved, and the sums' stores and reads, which cost this
+// kernel more than their bytes: they are scattered rows in between the weight stream.  (us for the layer, before -> here: 256 experts of
+// 7168 x 4096 and 2048 x 7168, 256 tokens 1813 -> 1783, of which the GEMM 1113 -> 1095; 128 of 3456 x 3328 and 1664 x 3456, 26 tokens 279 -> 275; 128
+// of 2176 x 3072 and 1536 x 2176, 4 tokens 70.5 -> 68.4.)
+template <int MODE, int ODT, int MT, bool GROUPED, bool KS = false, int NI = 4, bool GLUQ = false>
 __global__ void __launch_bounds__(256, 1)
 kcontig_gemm_kernel(KcArgs a) {
+  static_assert(!GLUQ || (MODE == KC_FP8_BLOCK && GROUPED && !KS), "gate and up of fp8 experts");
   static_assert(NI == 4 || (KS && (NI == 1 || NI == 2)), "narrow column groups exist for the K-split form only");
   typedef Kc<MODE> T;
   typedef typename T::acc_t acc_t;
@@ -152,12 +161,21 @@ kcontig_gemm_kernel(KcArgs a) {
     for (int j = 0; j < MT; ++j) tok[j] = a.sorted_ids[m0 + 16 * j + r16];   // (the array is padded to whole blocks)
     if (m0 >= npp) return;
     if (expert < 0 || expert >= a.E) {             // not one of this rank's experts: zero rows, no weights read
+      if constexpr (GLUQ) {                          // the codes and the scale of a group of zeros
+        for (int i = tid; i < BM * 32; i += 256) {
+          const int id = a.sorted_ids[m0 + (i >> 5)];
+          if (id >= a.numel) continue;
+          *(uint32_t*)(a.q_out + (size_t)id * (N >> 1) + 128 * blockIdx.x + 4 * (i & 31)) = 0u;
+          if ((i & 31) == 0) a.q_scales[(size_t)id * (N >> 8) + blockIdx.x] = 1e-10f / FP8_MAX;
+        }
+        return;
+      }
       const int col0 = blockIdx.x * 256;
       zero_block_columns((uint16_t*)a.out, a.sorted_ids + m0, BM, a.numel, N, col0, min(256, N - col0), 256);
       return;
     }
   }
-  const int n0 = KS ? blockIdx.x * (16 * NI) : blockIdx.x * 256 + wave * 64;
+  const int n0 = KS ? blockIdx.x * (16 * NI) : GLUQ ? (wave >> 1) * (N >> 1) + blockIdx.x * 128 + (wave & 1) * 64 : blockIdx.x * 256 + wave * 64;
   if (n0 >= N) return;
   // Operands are addressed through buffer descriptors: a 32-bit lane offset plus a scalar K-block offset
   // per load (no 64-bit address arithmetic in the loop; the host checks that one expert's weights, the
@@ -374,6 +392,67 @@ kcontig_gemm_kernel(KcArgs a) {
         if (kb >= KB) break;
       }
     }
+  }
+
+  if constexpr (GLUQ) {
+    // a lane holds the same rows and columns of gate and up as the lane of the wavefront two further: gate wavefronts finish
+    // column tiles 0 and 1, up wavefronts 2 and 3
+    __shared__ u2 trade[4][2 * MT][64];
+    __shared__ float largest[4][16 * MT];
+    const bool up = wave >= 2;
+    u2 kept[2 * MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f4 v = bitcast<f4>(acc[i][j]);
+        u2 o;
+        o.x = (uint32_t)Elem<ODT>::from_f32(v[0]) | ((uint32_t)Elem<ODT>::from_f32(v[1]) << 16);
+        o.y = (uint32_t)Elem<ODT>::from_f32(v[2]) | ((uint32_t)Elem<ODT>::from_f32(v[3]) << 16);
+        if (up == (i < 2)) trade[wave][2 * j + (i & 1)][lane] = o;
+        else kept[2 * j + (i & 1)] = o;
+      }
+    __syncthreads();
+    float y[2 * MT][4];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      float mx = 0.f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u2 other = trade[wave ^ 2][2 * j + h][lane], own = kept[2 * j + h], g = up ? other : own, u = up ? own : other;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t gw = e < 2 ? g.x : g.y, uw = e < 2 ? u.x : u.y;
+          const float gate = Elem<ODT>::to_f32((uint16_t)((e & 1) ? gw >> 16 : gw & 0xffffu)), upv = Elem<ODT>::to_f32((uint16_t)((e & 1) ? uw >> 16 : uw & 0xffffu));
+          const float v = round_act<ODT>(silu_mul(gate, upv));
+          y[2 * j + h][e] = v;
+          mx = fmaxf(mx, fabsf(v));
+        }
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      if (q == 0) largest[wave][16 * j + r16] = mx;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      const int r = 16 * j + r16, id = tok[j];
+      if (id >= a.numel) continue;
+      const float s = fmaxf(fmaxf(fmaxf(largest[0][r], largest[1][r]), fmaxf(largest[2][r], largest[3][r])), 1e-10f) / FP8_MAX;
+      const SharedDivisor by_s(s);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float c[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[e] = clamp448(by_s.div(y[2 * j + h][e]));
+        int w = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], 0, false);
+        w = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], w, true);
+        const int col = 128 * blockIdx.x + (wave & 1) * 64 + 16 * ((up ? 2 : 0) + h) + 4 * q;
+        *(uint32_t*)(a.q_out + (size_t)id * (N >> 1) + col) = (uint32_t)w;
+      }
+      if (wave == 0 && q == 0) a.q_scales[(size_t)id * (N >> 8) + blockIdx.x] = s;
+    }
+    return;
   }
 
   acc_t fin[MT];
@@ -737,6 +816,43 @@ extern "C" int mi355q_moe_gemm(void* out, const void* a, const void* w, const fl
   int rc = launch_mode<true>(g, mode, out_dtype, pick_mt(rows_per_wg), row_blocks, st);
   if (rc) return rc;
   MQ_LAUNCH_CHECK("moe_gemm");
+  return 0;
+}
+
+extern "C" int mi355q_moe_fp8_gate_up_quant(uint8_t* out, float* out_scales, const void* a, const void* w, const float* a_scale, const float* w_scale,
+                                            const int32_t* sorted_token_ids, const int32_t* expert_ids, const int32_t* num_tokens_post_pad, int numel,
+                                            int topk, int block_size, int max_blocks, int E, int K, int N, int act_dtype, int w_layout, void* stream) {
+  MQ_REQUIRE(numel >= 0 && topk > 0 && E > 0 && K > 0 && N > 0, "moe_fp8_gate_up_quant: bad shape");
+  if (numel == 0 || max_blocks == 0) return 0;
+  MQ_REQUIRE(out && out_scales && a && w && a_scale && w_scale && sorted_token_ids && expert_ids && num_tokens_post_pad, "moe_fp8_gate_up_quant: null pointer");
+  MQ_REQUIRE(K % 128 == 0 && N % 256 == 0, "moe_fp8_gate_up_quant: K=%d must be a multiple of 128 and N=%d of 256", K, N);
+  MQ_REQUIRE(block_size == 16 || block_size == 32 || block_size == 64, "moe_fp8_gate_up_quant: blocks of 16, 32 or 64 slots, got %d", block_size);
+  MQ_REQUIRE(act_dtype == MI355Q_F16 || act_dtype == MI355Q_BF16, "moe_fp8_gate_up_quant: dtype %d", act_dtype);
+  MQ_REQUIRE(w_layout == 0 || w_layout == 1, "moe_fp8_gate_up_quant: weight layout %d", w_layout);
+  MQ_REQUIRE((size_t)N * K * 2 < ((size_t)1 << 32) && ((size_t)numel / topk + 1) * K * 2 < ((size_t)1 << 32),
+             "moe_fp8_gate_up_quant: one expert's weights and the activations must each stay below 4 GiB (N=%d K=%d, %d slots)", N, K, numel);
+  KcArgs g = {};
+  g.a = a; g.w = w; g.a_scale = a_scale; g.w_scale = w_scale;
+  g.M = numel; g.N = N; g.K = K; g.kslab = w_layout;
+  g.sc_row = g.sc_col = 1;
+  g.sorted_ids = sorted_token_ids; g.expert_ids = expert_ids; g.npp = num_tokens_post_pad;
+  g.numel = numel; g.topk = topk; g.block_size = block_size; g.E = E;
+  g.w_stride = (long)N * K;
+  g.ws_stride = (long)(N / 128) * (K / 128);
+  g.q_out = out;
+  g.q_scales = out_scales;
+  const dim3 grid(N / 256, max_blocks), block(256);
+  hipStream_t st = as_stream(stream);
+#define MQ_MT(DT)                                                                                                                        \
+  do {                                                                                                                                   \
+    if (block_size == 16) hipLaunchKernelGGL((kcontig_gemm_kernel<KC_FP8_BLOCK, DT, 1, true, false, 4, true>), grid, block, 0, st, g);      \
+    else if (block_size == 32) hipLaunchKernelGGL((kcontig_gemm_kernel<KC_FP8_BLOCK, DT, 2, true, false, 4, true>), grid, block, 0, st, g); \
+    else hipLaunchKernelGGL((kcontig_gemm_kernel<KC_FP8_BLOCK, DT, 4, true, false, 4, true>), grid, block, 0, st, g);                       \
+  } while (0)
+  if (act_dtype == MI355Q_F16) MQ_MT(MI355Q_F16);
+  else MQ_MT(MI355Q_BF16);
+#undef MQ_MT
+  MQ_LAUNCH_CHECK("moe_fp8_gate_up_quant");
   return 0;
 }
 
