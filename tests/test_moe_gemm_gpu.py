@@ -912,3 +912,50 @@ def test_fp8_gate_up_quant(E, K, N, numel, topk, block, dtype):
                                                     so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, topk, block, ex.numel(), E, K, N, code,
                                                     layout, st), "moe_fp8_gate_up_quant")
         assert torch.equal(got, want) and torch.equal(got_s, want_s) and not got_s.isnan().any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("E,K,N,rows,plans", [(3, 512, 256, 34, ["rows"]), (16, 1536, 1536, 30, ["rows"]), (16, 1664, 1024, 70, ["rows"]),
+                                              (64, 256, 1024, 70, [1]), (4, 4096, 256, 75, [6]), (2, 6528, 1024, 200, [6]), (8, 7168, 1024, 100, [4]),
+                                              (16, 4096, 3072, 128, [1]), (1, 384, 4096, 256, ["rows"])])
+def test_grouped_w4a16_plans_of_blocks_of_64(fmoe, E, K, N, rows, plans, dtype):
+    """Every way blocks of 64 slots are taken -- the kernel with copying wavefronts, tiles unsplit and with K in several, also uneven, ranges --
+    and foreign experts and dropped ids in each: sums that are exact in fp32 against a float64 product, to the last bit."""
+    import ctypes
+    from vllm_gcu_amd import _lib
+    from vllm_gcu_amd.kernels.quantization import rearrange
+    lib, code, st, g = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream, 128
+    numel = E * rows
+    kernel, ranges = ctypes.c_int(), ctypes.c_int()
+    _lib.check(lib.mi355q_moe_w4a16_plan(numel, E, K, N, g, _lib.ZP_PACKED, code, ctypes.byref(kernel), ctypes.byref(ranges)), "plan")
+    taken = "rows" if kernel.value else ranges.value
+    print(f"case blocks of 64 E={E} K={K} N={N} rows={rows} {dtype}: {taken}", flush=True)
+    if dtype == torch.float16:
+        assert taken in plans
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // 8, N), dtype=torch.int32, device="cuda", generator=gen)
+    z = torch.randint(0, 16, (E, K // g, N), dtype=torch.uint8, device="cuda", generator=gen)
+    zp = torch.stack([rearrange.rearrange_uint4_int32_gptq(w[0], torch.from_numpy(ow4.gptq_pack_zeros(a.cpu().numpy())).cuda())[1] for a in z])
+    s = (2.0 ** torch.randint(-8, -5, (E, K // g, N), device="cuda", generator=gen)).to(dtype)
+    x = torch.randint(-3, 4, (numel, K), device="cuda", generator=gen).to(dtype)
+    rw = 2.0 ** torch.randint(-2, 2, (numel,), device="cuda", generator=gen).float()
+    ids = torch.randint(0, E, (numel, 1), device="cuda", generator=gen, dtype=torch.int32)
+    ids[3], ids[numel - 1] = E + 1, -1                       # in no block
+    so, ex, npp = fmoe.moe_align_block_size(ids, 64, E)
+    if E > 4:
+        ex[1] = -1                                           # an expert of another rank
+    of = torch.full((numel,), -2, device="cuda")
+    real = so[:int(npp)].view(-1, 64)
+    for b in range(real.shape[0]):
+        of[real[b][real[b] < numel].long()] = int(ex[b])
+    need = lib.mi355q_moe_gemm_workspace_bytes(0, numel, 64, ex.numel(), E, K, N)
+    ws = torch.full((need // 4 + 1,), float("nan"), device="cuda")
+    out = torch.full((numel, N), 7.0, dtype=dtype, device="cuda")
+    _lib.check(lib.mi355q_moe_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), None, s.data_ptr(), zp.data_ptr(), _lib.ZP_PACKED, 0, g,
+                                   rw.data_ptr(), so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, 1, 64, ex.numel(), E, K, N, code, code, 0,
+                                   ws.data_ptr(), need, st), "moe_gemm")
+    dense = (rearrange.unpack_slab(w).view(E, K // g, g, N).double() - z[:, :, None].double()) * s[:, :, None].double()
+    assert (out[of == -2] == 7.0).all() and (out[of == -1] == 0).all()
+    for e in range(E):
+        r = (of == e).nonzero().view(-1)
+        assert torch.equal(out[r], ((x[r].double() @ dense[e].view(K, N)) * rw[r, None].double()).to(dtype))

@@ -14,6 +14,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace mi355q {
 
@@ -148,6 +149,11 @@ w4a16_tile_kernel(TileArgs a) {
     int tm, tn, split;
     a.order.locate(blockIdx.x, tm, tn, split);
     bx = tn, by = tm, bz = split;
+  }
+  if (GROUPED) {                                     // (column and K range, block)
+    const uint32_t cols = (N + BN - 1) / BN;
+    bz = bx / cols;
+    bx -= bz * cols;
   }
   const int m0 = by * BM;
   const u4* qw = a.qw;
@@ -607,7 +613,11 @@ template <bool GROUPED>
 dim3 tile_grid(TileArgs& a, int row_blocks, int bm, int per_cu) {
   const int cols = (a.N + BN - 1) / BN, splits = ((a.K >> 7) + a.kper - 1) / a.kper;
   const double rounds = (double)cols * row_blocks * splits / (per_cu * device_cu_count());
-  if (GROUPED || rounds < (cols % 8 ? 1.25 : 3.5)) return dim3(cols, row_blocks, splits);
+  // grouped: the blocks last.  Of those the ids could fill most are empty, and workgroups that leave at once in between the others turn the CUs
+  // that the next ones go to: with the K ranges last eight blocks of 14336 x 4096 in two ranges, 256 workgroups, took 112 us, two of them on a CU
+  // and many CUs without any, and 77 us so
+  if (GROUPED) return dim3(cols * splits, row_blocks);
+  if (rounds < (cols % 8 ? 1.25 : 3.5)) return dim3(cols, row_blocks, splits);
   a.order = tile_order(row_blocks, cols, splits, (double)bm * a.kper * 256, (double)BN * a.kper * 64, per_cu);
   return dim3((unsigned)(cols * row_blocks * splits));
 }
@@ -1161,39 +1171,85 @@ int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, 
                               int numel, int topk, int block_size, int max_blocks, int E, int K, int N, int group_size, int dtype,
                               hipStream_t st);
 
-// Split-K plan of a grouped launch.  The host does not know how many blocks the alignment filled, so
-// the grid is estimated as every slot in a full block plus half a block of pads per expert.  A long K
-// with a narrow N (the second expert GEMM of a gated MLP) leaves the chip part empty and makes its few
-// workgroups very long; K is split until about two and a half workgroups per resident slot exist,
-// keeping at least 16 K blocks per split (Mixtral-8x7B layer, 512 tokens, second GEMM: 4 splits
-// measured best of 1..7; every further split adds 17 MB of partial tiles).
-static int grouped_splits(int numel, int block_size, int max_blocks, int E, int K, int N) {
-  if (block_size != 64) return 1;                  // the 64-row pipelined kernel only
+// Blocks of 64 slots: the tiles of this file with K in ranges, or the kernel with copying wavefronts (w4a16_rows.hip), which takes a block by
+// the row tiles that hold slots and gives a workgroup 128 columns and a CU to itself.  By prices in us, fitted to what every way took at 446
+// launches over 90 expert shapes (8 to 64 experts, K 1024 .. 14336, N 1024 .. 28672) at 29 .. 255 rows per expert, fp16 and bf16, weights
+// cold.  The blocks are those that evenly spread slots fill.  A CU that has one of the tiles takes 1.18 us for a K block, with two of
+// them 1.59; more rounds than one cost what they fill, and most of a round for its last workgroups.  Tiles on the loop that is not
+// pipelined (bf16 rows that are not staged, groups below 128, pre-scaled zero-points) take 1.39 times as long.
+// The pick is 0.3 % behind the best way on average (10 of the 446 by more than 5 %, 14 % at worst), where the tiles in one range are 12 % behind, the
+// other kernel is 12 %, and two and a half workgroups per slot, as before, were 7 %.  us, before -> here: 16 experts of 2688 x 1024 at
+// 30 / 64 / 100 rows each 27.9 / 29.4 / 29.8 -> 16.1 / 19.9 / 22.6 (bf16 at 40 40.9 -> 18.4), of 7168 x 1536 at 50 / 128 / 256 51.0 / 94.3 / 143.8 ->
+// 37.5 / 73.1 / 118.7, of 4096 x 3072 at 64 / 128 / 200 68.9 / 90.7 / 129.4 -> 59.9 / 75.3 / 108.8.
+struct BlocksPlan {
+  bool rows;                                       // w4a16_rows_grouped_launch
+  int splits;
+};
+static double expected_blocks(int numel, int E, int block) {
+  const double r = (double)numel / E, sd = std::sqrt(2 * r * (1 - 1.0 / E)) + 1e-9;
+  double sum = 0;
+  for (int k = 0; k * (double)block < r + 8 * sd; ++k) sum += 0.5 * std::erfc((k * (double)block + 0.5 - r) / sd);
+  return std::max(1.0, E * sum);
+}
+static BlocksPlan make_blocks_plan(int flags, int numel, int E, int K, int N) {
+  const bool plain = flags & 1, rows = flags & 2;  // plain: the loop that is not pipelined; rows: that kernel takes these operands
   const int G = K / 128;
-  long blocks = (numel + block_size - 1) / block_size + (E + 1) / 2;
-  if (blocks > max_blocks) blocks = max_blocks;
-  const long wgs = blocks * ((N + BN - 1) / BN), slots = 2L * device_cu_count();
-  if (wgs >= 2 * slots || G < 32) return 1;
-  long s = (5 * slots / 2 + wgs - 1) / wgs;
-  if (s > G / 16) s = G / 16;
-  while (s > 1 && (size_t)s * numel * N * sizeof(float) > TILE_SPLITK_BYTES * 2) --s;
-  return s < 1 ? 1 : (int)s;
+  const double blocks = expected_blocks(numel, E, 64), cus = device_cu_count(), weights = (double)std::min(blocks, (double)E) * K * N / 2;
+  const double slow = plain ? 1.39 : 1.0, stage = (flags & 4) && !plain ? 13.4 : 0;   // stage: the pass that makes the rows fp16
+  auto with_stream = [weights](double t) { const double h = weights / 3.8e6; return std::sqrt(std::sqrt(t * t * t * t + h * h * h * h)); };
+  BlocksPlan best = {false, 1};
+  double least = 1e30;
+  for (int s = 1; s <= 6; ++s) {
+    const int kper = (G + s - 1) / s;
+    if (s > 1 && (G / s < 4 || (G + kper - 1) / kper != s || (size_t)s * numel * N * sizeof(float) > TILE_SPLITK_BYTES * 2)) continue;
+    const double one = (kper * 1.18 + 5.2) * slow, two = (kper * 1.59 + 9.5) * slow;
+    const double r = blocks * ((N + BN - 1) / BN) * s / (2 * cus) - 0.02, full = std::floor(r);
+    double t = r <= 0.5 ? one : r <= 1 ? two : two * (0.29 * r + 0.71 * (full + (r - full <= 0.5 ? one / two : 1)));
+    t = with_stream(t + 2.5 + stage + (s > 1 ? 6.0 + 0.9e-6 * s * numel * N : 0));
+    if (t < least) least = t, best = {false, s};
+  }
+  if (rows && N % 128 == 0) {
+    const double tiles = std::max(numel / 16.0 + 0.5 * std::min((double)E, blocks), blocks), r = blocks * (N / 128) / cus - 0.03;
+    const double t = (G + 1) / 2 * (0.77 + 0.08 * tiles / blocks) * (flags & 4 ? 1.17 : 1.0) + 6.05;
+    if ((r <= 1 ? 1 : 0.06 * r + 0.94 * std::ceil(r)) * t + 0.5 < least) best = {true, 1};
+  }
+  return best;
+}
+struct BlocksPlans {
+  BlocksPlan of[8];                                // by flags
+};
+static BlocksPlans blocks_plans(int numel, int E, int K, int N) {
+  return cached_plan(E, numel, N, K, [](int E, int M, int N, int K) {
+    BlocksPlans p;
+    for (int f = 0; f < 8; ++f) p.of[f] = make_blocks_plan(f, M, E, K, N);
+    return p;
+  });
 }
 // bf16 activations of a grouped launch staged as fp16 rows (blocks of 64 slots, outputs of two million
 // elements or more): the area follows the partial tiles of the launch's split-K plan
 static bool grouped_stage_pays(int numel, int block_size, int N) {
   return block_size == 64 && (long)numel * N >= (1L << 21);
 }
+static BlocksPlan blocks_plan(int numel, int E, int K, int N, int group_size, int zeros_kind, int dtype) {
+  const bool bf16 = dtype == MI355Q_BF16, pipelined = group_size % 128 == 0 && zeros_kind != MI355Q_ZP_PRESCALED && (!bf16 || grouped_stage_pays(numel, 64, N));
+  return blocks_plans(numel, E, K, N).of[(pipelined ? 0 : 1) | (group_size != 32 ? 2 : 0) | (bf16 ? 4 : 0)];
+}
 static size_t grouped_partial_bytes(int splits, int numel, int N) {
   return splits > 1 ? (((size_t)splits * numel * N * sizeof(float)) + 255) & ~(size_t)255 : 0;
 }
+// (neither the dtype nor topk nor the zero-points are known here: room for each of the plans, with bf16 rows of one slot each beside the
+// partial tiles while both stay within 128 MiB; a larger workspace is used when it is there)
 size_t w4a16_grouped_workspace_bytes(int numel, int block_size, int max_blocks, int E, int K, int N) {
-  const int s = grouped_splits(numel, block_size, max_blocks, E, K, N);
-  size_t need = s > 1 ? (size_t)s * numel * N * sizeof(float) : 0;
-  // (neither the dtype nor topk is known here: room for bf16 rows of one slot each)
-  // (asked for while everything stays within 128 MiB; a larger workspace is used when it is there)
-  const size_t staged = grouped_partial_bytes(s, numel, N) + BF16_STAGE_SCALE_BYTES + (size_t)numel * K * 2;
-  if (grouped_stage_pays(numel, block_size, N) && staged <= 2 * BF16_STAGE_BYTES) need = staged;
+  if (block_size != 64) return 0;
+  const BlocksPlans plans = blocks_plans(numel, E, K, N);
+  size_t need = 0;
+  for (int f = 0; f < 8; ++f) {
+    if (plans.of[f].rows) continue;
+    const int s = plans.of[f].splits;
+    need = std::max(need, s > 1 ? (size_t)s * numel * N * sizeof(float) : 0);
+    const size_t staged = grouped_partial_bytes(s, numel, N) + BF16_STAGE_SCALE_BYTES + (size_t)numel * K * 2;
+    if ((f & 4) && !(f & 1) && grouped_stage_pays(numel, block_size, N) && staged <= 2 * BF16_STAGE_BYTES) need = std::max(need, staged);
+  }
   return need;
 }
 
@@ -1210,12 +1266,13 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
              "moe_w4a16: activation matrix of %d rows x %d is 4 GiB or more", numel / (topk > 0 ? topk : 1), K);
   MQ_REQUIRE(block_size == 16 || block_size == 32 || block_size == 64 || block_size == 128,
              "moe_w4a16: block_size=%d must be 16, 32, 64 or 128", block_size);
-  // Blocks of 32 slots, and of 64 that are half empty on average over a long K: the kernel with copying wavefronts, which
-  // takes a block by the row tiles that hold slots.  (us per layer, before -> here: eight experts of 4096 x 28672 and 14336 x 4096 at
-  // 12 / 24 rows per expert, blocks of 32, 218 / 245 -> 176 / 189, at 32 / 48, blocks of 64, 245 / 246 -> 215 / 236; sixty of 2048 x 2816 and
-  // 1408 x 2048 at 17 / 26 rows, blocks of 32, 132 / 147 -> 94 / 103, but at 34, blocks of 64, 122 against 132.)
+  // Blocks of 32 slots, and of 64 where that is the cheaper one: the kernel with copying wavefronts.  (us per layer, before -> here: eight experts
+  // of 4096 x 28672 and 14336 x 4096 at 12 / 24 rows per expert, blocks of 32, 218 / 245 -> 176 / 189; sixty of 2048 x 2816 and
+  // 1408 x 2048 at 17 / 26 rows, blocks of 32, 132 / 147 -> 94 / 103.)
   const bool plain = !scales_f32 && !out_scale;
-  if (plain && group_size != 32 && (block_size == 32 || (block_size == 64 && K >= 4096 && numel <= 48L * E)))
+  BlocksPlan plan = {block_size == 32, 1};
+  if (block_size == 64 && plain) plan = blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype);
+  if (plain && group_size != 32 && plan.rows)
     return w4a16_rows_grouped_launch(out, x, qweight, scales, zeros, zeros_kind, topk_weights, sorted_ids, expert_ids, npp, numel,
                                      topk, block_size, max_blocks, E, K, N, group_size, dtype, st);
   // Blocks of 16 slots (decode-sized token counts): the layer is bound by the experts' weights, which the kernel for decode
@@ -1237,7 +1294,7 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   a.sorted_ids = sorted_ids; a.expert_ids = expert_ids; a.npp = npp; a.topk_weights = topk_weights;
   a.numel = numel; a.topk = topk; a.E = E;
   const int G = K / 128;
-  int splits = (scales_f32 || out_scale) ? 1 : grouped_splits(numel, block_size, max_blocks, E, K, N);
+  int splits = plan.splits;
   if (splits > 1 && (!workspace || workspace_bytes < (size_t)splits * numel * N * sizeof(float))) splits = 1;
   a.kper = (G + splits - 1) / splits;
   splits = (G + a.kper - 1) / a.kper;              // no empty splits
@@ -1308,3 +1365,13 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
 }
 
 }  // namespace mi355q
+
+extern "C" int mi355q_moe_w4a16_plan(int numel, int E, int K, int N, int group_size, int zeros_kind, int dtype, int* rows_kernel, int* k_ranges) {
+  using namespace mi355q;
+  MQ_REQUIRE(numel > 0 && E > 0 && K > 0 && N > 0 && group_size > 0, "moe_w4a16_plan: bad shape numel=%d E=%d K=%d N=%d", numel, E, K, N);
+  MQ_REQUIRE(rows_kernel && k_ranges, "moe_w4a16_plan: null pointer");
+  const BlocksPlan p = blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype);
+  *rows_kernel = p.rows;
+  *k_ranges = p.splits;
+  return 0;
+}
