@@ -169,8 +169,9 @@ int mi355q_fp8_scaled_gemm(void* out, const void* x, const void* w, const float*
  * only where the split launch is ahead of the weight-streaming kernel) K is cut into ranges of
  * whole K blocks that run side by side, and a second launch adds their fp32 sums in range order and
  * applies bias (and, for the scaled GEMM, the scales): run-to-run identical, and equal to the unsplit
- * launch up to the order of the fp32 additions.  The workspace follows the rules of
- * mi355q_w4a16_gemm's (its first MiB is left alone); without one, or with a smaller one, the unsplit
+ * launch up to the order of the fp32 additions.  (Small tiles with few ranges add them in the first launch, by arrival counters
+ * in the first 64 KiB of the workspace.)  The workspace follows the rules of
+ * mi355q_w4a16_gemm's: zero-filled once, and its first MiB is as it was after every call; without one, or with a smaller one, the unsplit
  * launch (or, for the scaled GEMM on few tiles, the streaming kernel) runs.
  * mi355q_fp8_block_gemm_ws also uses ceil16(M) * (K / 128) * 4 bytes behind the partial sums (behind the first
  * MiB where nothing is split), when the workspace has them, from 24 K blocks of 128 on where K blocks x output
@@ -223,8 +224,8 @@ int mi355q_w8a8_int8_gemm(void* out, int32_t* acc_out, const int8_t* x, const in
  * workspace (0 = this shape is not split) K is cut into ranges that run side by side, and a second
  * launch adds their int32 sums and applies the scales and the bias: integer sums, so the result --
  * acc_out included -- is bit for bit that of the call without workspace.  The workspace follows the
- * rules of mi355q_w4a16_gemm's (its first MiB is left alone, so one buffer serves both); without
- * one, or with a smaller one, the unsplit launch runs. */
+ * rules of mi355q_w4a16_gemm's (zero-filled once; its first MiB, where small tiles count the ranges that have arrived, is as it was after
+ * every call, so one buffer serves both); without one, or with a smaller one, the unsplit launch runs. */
 size_t mi355q_w8a8_int8_workspace_bytes(int M, int N, int K);
 /* No counterpart in the reference.  What mi355q_w8a8_int8_gemm_ws launches for dense operands, no raw accumulators and a workspace of that size
  * (or of mi355q_q8_mid_plan's): 0 = the kernel for a few dozen to some hundred rows (kslab weights), 1 = tiles of 128 .. 256 rows x 128

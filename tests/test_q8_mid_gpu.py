@@ -145,3 +145,46 @@ def test_fp8_rows_far_apart():
     assert torch.equal(call(160, x, ldx), call(160, dense, K))
     with pytest.raises(RuntimeError, match="fits neither kernel"):
         call(160, x, 40_000_000)
+
+
+# (kind, M, N, K) -> rows of the 64 column tile and K ranges: sums added in the kernel (up to 56 KiB of other ranges) or by a second launch
+RANGES = [(SCALED, 17, 128, 2304, 32, 2), (INT8, 47, 3072, 7936, 32, 5), (SCALED, 32, 512, 2816, 32, 3), (BLOCK, 63, 128, 5120, 32, 5),
+          (INT8, 49, 192, 10624, 32, 11),
+          (SCALED, 33, 64, 7808, 32, 8), (BLOCK, 129, 128, 10880, 32, 11), (INT8, 65, 2048, 10752, 64, 4), (SCALED, 49, 3072, 4736, 64, 4),
+          (BLOCK, 50, 3072, 3456, 64, 3), (SCALED, 129, 1024, 10240, 64, 5)]
+
+
+@pytest.mark.parametrize("kind,M,N,K,rows,ranges", RANGES)
+def test_k_ranges_leave_the_counters_at_zero(kind, M, N, K, rows, ranges):
+    """Products and sums that are exact, over a workspace whose first MiB is zero and whose rest is not, twice: the output to the bit, the
+    counters as they were."""
+    from vllm_gcu_amd import _lib
+    if N % 128 == 0:
+        assert tile(kind, M, N, K) == (rows, 64, ranges)
+    need = rt.host.q8_mid_plan(kind, M, N, K)
+    print(f"case q8 ranges kind={kind} M={M} N={N} K={K} workspace={need}", flush=True)
+    assert need > 1 << 20
+    torch.manual_seed(M + N + K)
+    ws = torch.full((need,), 0xff, dtype=torch.uint8, device="cuda")
+    ws[:1 << 20] = 0
+    x, w = (torch.randint(-3, 4, (r, K), device="cuda").to(torch.int8 if kind == INT8 else torch.float8_e4m3fn) for r in (M, N))
+    wk, st = rearrange.to_kslab(w), torch.cuda.current_stream().cuda_stream
+    xs = 2.0 ** torch.randint(-2, 3, (M, K // 128) if kind == BLOCK else (M, 1), device="cuda").float()
+    sc = 2.0 ** torch.randint(-2, 3, (N // 128, K // 128) if kind == BLOCK else (N, 1), device="cuda").float()
+    if kind == BLOCK:
+        xd, wd = x.double() * xs.double().repeat_interleave(128, 1), w.double() * sc.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    else:
+        xd, wd = x.double() * xs.double(), w.double() * sc.double()
+    want = (xd @ wd.t()).bfloat16()
+    for _ in range(2):
+        out = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+        if kind == INT8:
+            _lib.call("mi355q_w8a8_int8_gemm_ws", out.data_ptr(), None, x.data_ptr(), wk.data_ptr(), xs.data_ptr(), 1, sc.data_ptr(), 1, None, 0,
+                      M, N, K, K, 0, N, _lib.BF16, ws.data_ptr(), need, st)
+        elif kind == SCALED:
+            _lib.call("mi355q_fp8_scaled_gemm_ws", out.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), 1, sc.data_ptr(), 1, None, M, N, K,
+                      K, 0, N, _lib.BF16, ws.data_ptr(), need, st)
+        else:
+            _lib.call("mi355q_fp8_block_gemm_ws", out.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), sc.data_ptr(), None, M, N, K, K, 0, N,
+                      _lib.BF16, ws.data_ptr(), need, st)
+        assert torch.equal(out, want) and not ws[:1 << 20].any()

@@ -36,7 +36,7 @@ int kcontig_fp8_pc_launch(void* out, const void* a, const void* w, const float* 
                           int out_dtype, int w_layout, hipStream_t st);
 bool q8_mid_wanted(int mode, int M, int N, int K, long ldx, size_t* bytes);
 int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
-                  int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* partial,
+                  int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* workspace,
                   hipStream_t st);
 namespace {
 
@@ -802,7 +802,7 @@ extern "C" int mi355q_fp8_block_gemm_ws(void* out, const void* x, const void* w,
   size_t mid_bytes = 0;
   if (kslab && q8_mid_wanted(0, M, N, K, ldx, &mid_bytes) && (mid_bytes == 0 || (workspace && workspace_bytes >= F8_WS_OFFSET + mid_bytes)))
     return q8_mid_launch(0, out, x, w, x_scale, 0, w_scale, 0, bias, 0, M, N, K, ldx, ldo, out_dtype,
-                         mid_bytes ? (char*)workspace + F8_WS_OFFSET : nullptr, as_stream(stream));
+                         workspace, as_stream(stream));
   F8Args a = {};
   a.out = out; a.x = (const uint8_t*)x; a.w = (const uint8_t*)w; a.x_scale = x_scale; a.w_scale = w_scale;
   a.bias = bias; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldw = ldw; a.ldo = ldo;
@@ -840,7 +840,7 @@ extern "C" int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w
       (out_dtype == MI355Q_F16 || out_dtype == MI355Q_BF16) && q8_mid_wanted(1, M, N, K, ldx, &mid_bytes) &&
       (mid_bytes == 0 || (workspace && workspace_bytes >= F8_WS_OFFSET + mid_bytes)))
     return q8_mid_launch(1, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, 0, M, N, K, ldx, ldo,
-                         out_dtype, mid_bytes ? (char*)workspace + F8_WS_OFFSET : nullptr, as_stream(stream));
+                         out_dtype, workspace, as_stream(stream));
   // the MFMA tile kernel from 65 rows on when its 256 x 128 tiles fill a good part of the chip; below
   // (and for shapes it does not take) the weight-streaming kernel, which wants dense operands
   const long tiles = (long)((M + FTM - 1) / FTM) * (N / FTN);

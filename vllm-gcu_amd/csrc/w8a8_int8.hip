@@ -28,7 +28,7 @@ int int8_tile_launch(void* out, const void* x, const void* w, const float* x_sca
                      void* workspace, size_t workspace_bytes, hipStream_t st);
 bool q8_mid_wanted(int mode, int M, int N, int K, long ldx, size_t* bytes);
 int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
-                  int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* partial,
+                  int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* workspace,
                   hipStream_t st);
 namespace {
 
@@ -999,7 +999,7 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
   if (kslab && !acc_out && q8_mid_wanted(2, M, N, K, ldx, &mid_bytes) &&
       (mid_bytes == 0 || (workspace && workspace_bytes >= I8_WS_OFFSET + mid_bytes)))
     return q8_mid_launch(2, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K, ldx,
-                         ldo, out_dtype, mid_bytes ? (char*)workspace + I8_WS_OFFSET : nullptr, as_stream(stream));
+                         ldo, out_dtype, workspace, as_stream(stream));
   if (N % 128 == 0 && !acc_out && (size_t)N * K < ((size_t)1 << 32) && (size_t)256 * (size_t)ldx < ((size_t)1 << 32) &&
       (kslab || (size_t)128 * (size_t)ldw < ((size_t)1 << 32)) && int8_pick(M, N, K).tiles128)
     return int8_tile_launch(out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K,
