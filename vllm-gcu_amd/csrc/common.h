@@ -241,6 +241,22 @@ __device__ __forceinline__ float silu_mul(float a, float b) {
   return a * (1.0f / (1.0f + expf(-a))) * b;      // left * sigmoid(left) * right
 }
 
+// what silu_and_mul stores for a gate and an up column that are 16 bits already
+template <int DT>
+__device__ __forceinline__ uint16_t silu_mul16(uint16_t gate, uint16_t up) {
+  if constexpr (DT == MI355Q_F16) {
+    uint32_t h;                                      // (its product with the up column is rounded to fp16 at once)
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(h) : "v"(silu_mul(Elem<DT>::to_f32(gate), 1.0f)), "v"((uint32_t)up));
+    return (uint16_t)h;
+  } else {
+    return Elem<DT>::from_f32(silu_mul(Elem<DT>::to_f32(gate), Elem<DT>::to_f32(up)));
+  }
+}
+template <int DT>
+__device__ __forceinline__ uint32_t silu_mul16x2(uint32_t gate, uint32_t up) {
+  return (uint32_t)silu_mul16<DT>((uint16_t)gate, (uint16_t)up) | ((uint32_t)silu_mul16<DT>((uint16_t)(gate >> 16), (uint16_t)(up >> 16)) << 16);
+}
+
 constexpr float FP8_MAX = 448.0f;
 template <int DT>
 __device__ __forceinline__ float round_act(float f) {

@@ -423,16 +423,7 @@ w4a16_decode_grouped_kernel(DecodeArgs a) {
       float vg = red[0][g][lane], vu = red[0][u][lane];
 #pragma unroll
       for (int w = 1; w < W; ++w) vg += red[w][g][lane], vu += red[w][u][lane];
-      const uint16_t up = Elem<DT>::from_f32(vu);
-      const float gate = Elem<DT>::to_f32(Elem<DT>::from_f32(vg));
-      if constexpr (DT == MI355Q_F16) {
-        // (the operator's product with the up column is rounded to fp16 at once)
-        uint32_t h;
-        asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(h) : "v"(silu_mul(gate, 1.0f)), "v"((uint32_t)up));
-        fin[t] = Elem<DT>::to_f32((uint16_t)h);
-      } else {
-        fin[t] = silu_mul(gate, Elem<DT>::to_f32(up));
-      }
+      fin[t] = Elem<DT>::to_f32(silu_mul16<DT>(Elem<DT>::from_f32(vg), Elem<DT>::from_f32(vu)));
     }
     store_row<DT, CP>(a.out + (size_t)id * (N >> 1) + ncol + tc, nullptr, fin);
     return;

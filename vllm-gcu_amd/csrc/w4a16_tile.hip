@@ -124,7 +124,9 @@ template <> struct TileMma<MI355Q_BF16> {
 // IOBF (with DT = fp16; grouped: the multiplier belongs to the row the slot was gathered from): the activations are bf16 rows that a pass before this kernel scaled by a
 // power of two each and stored as fp16 (exact: eight mantissa bits into eleven); scales, pre-scaled
 // zero-points, bias and output are bf16, and the epilogue multiplies each row by its power of two.
-template <int DT, int ZK, int MT, bool GROUPED, int WM, bool SF32 = false, int GPB = 1, bool IOBF = false>
+// GLU (grouped blocks of 64): the columns are gate and up; a workgroup takes 128 of each that go together, gates in its first two
+// wavefronts, and stores what silu_and_mul makes of the sums it would have stored ([numel, N / 2]).  K ranges store sums as ever.
+template <int DT, int ZK, int MT, bool GROUPED, int WM, bool SF32 = false, int GPB = 1, bool IOBF = false, bool GLU = false>
 __global__ void __launch_bounds__(256 * WM, WM == 1 ? 2 : 1)
 w4a16_tile_kernel(TileArgs a) {
   typedef TileMma<DT> MM;
@@ -132,6 +134,7 @@ w4a16_tile_kernel(TileArgs a) {
   static_assert(!IOBF || (DT == MI355Q_F16 && MT == 4 && WM == 1), "bf16 in and out around the fp16 loop: 64-row tiles");
   typedef Elem<IOBF ? MI355Q_BF16 : DT> IO;       // the type of scales, pre-scaled zero-points, bias and output
   static_assert(MT % WM == 0, "row tiles split evenly over the wavefront rows");
+  static_assert(!GLU || (GROUPED && MT == 4 && WM == 1 && !SF32 && GPB == 1), "blocks of 64 slots");
   constexpr int BM = 16 * MT;
   constexpr int MTW = MT / WM;                    // row tiles per wavefront
   constexpr int NTHR = 256 * WM;
@@ -177,6 +180,8 @@ w4a16_tile_kernel(TileArgs a) {
           if (id < a.numel)
             *(f4*)(a.partial + ((size_t)bz * a.numel + id) * N + col0 + 4 * piece) = (f4){0.f, 0.f, 0.f, 0.f};
         }
+      } else if (GLU) {
+        zero_block_columns(a.out, a.sorted_ids + m0, BM, a.numel, N >> 1, bx * 128, 128, NTHR);
       } else {
         zero_block_columns(a.out, a.sorted_ids + m0, BM, a.numel, N, col0, ncols, NTHR);
       }
@@ -205,8 +210,8 @@ w4a16_tile_kernel(TileArgs a) {
   auto tile_live = [&](int mt) { return !GROUPED || ((live_tiles >> (wmh * MTW + mt)) & 1); };
   // N may end in the middle of the 256-column tile: the two wavefronts of a
   // missing slab compute on the previous one and skip the epilogue
-  const bool live = (bx * 2 + (wave >> 1)) < (N >> 7);
-  const int slab = live ? bx * 2 + (wave >> 1) : (N >> 7) - 1;
+  const bool live = GLU || (bx * 2 + (wave >> 1)) < (N >> 7);
+  const int slab = GLU ? bx + (wave >> 1) * (N >> 8) : live ? bx * 2 + (wave >> 1) : (N >> 7) - 1;
   const int t0 = (wave & 1) * 4;
   const int ncol = 128 * slab + 8 * c + t0;          // first of this lane's 4 columns
 
@@ -502,6 +507,48 @@ w4a16_tile_kernel(TileArgs a) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) bs[t] = IO::to_f32(a.bias[ncol + t]);
   }
+  if constexpr (GLU) {
+    if (!a.partial) {
+      // gate wavefronts finish the upper half of the rows, up wavefronts the lower one: each leaves the other half in LDS, rounded as it
+      // would have been stored
+      constexpr int H = MTW / 2;
+      const int up = wave >> 1;
+      uint2* const mail = (uint2*)lds + lane;
+      auto packed = [&](int mt, int i) {
+        const int m = tok[mt * 16 + 4 * kq + i];
+        float rw = 1.0f;
+        if (IOBF && m < a.numel) rw = a.row_scale[a.topk == 1 ? m : m / a.topk];
+        uint2 o;
+        o.x = (uint32_t)IO::from_f32(acc[mt][0][i] * rw + 0.f) | ((uint32_t)IO::from_f32(acc[mt][1][i] * rw + 0.f) << 16);
+        o.y = (uint32_t)IO::from_f32(acc[mt][2][i] * rw + 0.f) | ((uint32_t)IO::from_f32(acc[mt][3][i] * rw + 0.f) << 16);
+        return o;
+      };
+      uint2 own[MTW][4];
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) own[mt][i] = packed(mt, i);
+      __syncthreads();                                 // (nobody reads activations any more)
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if ((mt >= H) != (up == 1)) mail[((wave * H + mt % H) * 4 + i) * 64] = own[mt][i];
+      __syncthreads();
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if ((mt >= H) != (up == 1)) continue;
+          const int m = tok[mt * 16 + 4 * kq + i];
+          const uint2 other = mail[(((wave ^ 2) * H + mt % H) * 4 + i) * 64];
+          const uint2 g = up ? other : own[mt][i], u = up ? own[mt][i] : other;
+          constexpr int IODT = IOBF ? MI355Q_BF16 : DT;
+          if (m < a.numel) *(uint2*)(a.out + (size_t)m * (N >> 1) + bx * 128 + 8 * c + t0) = make_uint2(silu_mul16x2<IODT>(g.x, u.x), silu_mul16x2<IODT>(g.y, u.y));
+        }
+      return;
+    }
+  }
 #pragma unroll
   for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
@@ -571,36 +618,45 @@ w4a16_splitk_reduce_kernel(uint16_t* out, const float* partial, const uint16_t* 
 // The same for a grouped launch: the rows are visited through the aligned id list, so a slot id that the
 // alignment dropped (an expert outside [0, E), a row past the valid count) -- whose partial rows no
 // split wrote -- is left alone, exactly as the unsplit launch leaves it.
-template <int DT>
+// GLU: gate and up columns, out [numel, N / 2] as silu_and_mul makes it.
+template <int DT, bool GLU>
 __global__ void __launch_bounds__(256)
 w4a16_grouped_reduce_kernel(uint16_t* out, const float* partial, const float* row_weight,
                             const int32_t* sorted_ids, const int32_t* npp, int numel, int N, int splits,
                             const float* row_scale, int topk) {
-  const int n4 = N >> 2;
+  const int NO = GLU ? N >> 1 : N, n4 = NO >> 2;
   const long t = (long)blockIdx.x * 256 + threadIdx.x;
   const long p = t / n4;
   if (p >= *npp) return;
   const int id = sorted_ids[p];
   if (id >= numel || id < 0) return;
   const long MN = (long)numel * N;
-  const long i = (long)id * N + (t - p * n4) * 4;
-  f4 v = *(const f4*)(partial + i);
-  int s = 1;
-  for (; s + 3 < splits; s += 4) {
-    const f4 p0 = *(const f4*)(partial + (size_t)s * MN + i), p1 = *(const f4*)(partial + (size_t)(s + 1) * MN + i);
-    const f4 p2 = *(const f4*)(partial + (size_t)(s + 2) * MN + i), p3 = *(const f4*)(partial + (size_t)(s + 3) * MN + i);
-    v += p0;
-    v += p1;
-    v += p2;
-    v += p3;
+  const int n = (int)(t - p * n4) * 4;
+  auto stored = [&](long i) {
+    f4 v = *(const f4*)(partial + i);
+    int s = 1;
+    for (; s + 3 < splits; s += 4) {
+      const f4 p0 = *(const f4*)(partial + (size_t)s * MN + i), p1 = *(const f4*)(partial + (size_t)(s + 1) * MN + i);
+      const f4 p2 = *(const f4*)(partial + (size_t)(s + 2) * MN + i), p3 = *(const f4*)(partial + (size_t)(s + 3) * MN + i);
+      v += p0;
+      v += p1;
+      v += p2;
+      v += p3;
+    }
+    for (; s < splits; ++s) v += *(const f4*)(partial + (size_t)s * MN + i);
+    if (row_weight) v *= row_weight[id];
+    if (row_scale) v *= row_scale[id / topk];        // bf16 rows staged as fp16: the gathered row's power of two
+    uint2 o;
+    o.x = (uint32_t)Elem<DT>::from_f32(v[0]) | ((uint32_t)Elem<DT>::from_f32(v[1]) << 16);
+    o.y = (uint32_t)Elem<DT>::from_f32(v[2]) | ((uint32_t)Elem<DT>::from_f32(v[3]) << 16);
+    return o;
+  };
+  uint2 o = stored((long)id * N + n);
+  if (GLU) {
+    const uint2 u = stored((long)id * N + NO + n);
+    o = make_uint2(silu_mul16x2<DT>(o.x, u.x), silu_mul16x2<DT>(o.y, u.y));
   }
-  for (; s < splits; ++s) v += *(const f4*)(partial + (size_t)s * MN + i);
-  if (row_weight) v *= row_weight[id];
-  if (row_scale) v *= row_scale[id / topk];          // bf16 rows staged as fp16: the gathered row's power of two
-  uint2 o;
-  o.x = (uint32_t)Elem<DT>::from_f32(v[0]) | ((uint32_t)Elem<DT>::from_f32(v[1]) << 16);
-  o.y = (uint32_t)Elem<DT>::from_f32(v[2]) | ((uint32_t)Elem<DT>::from_f32(v[3]) << 16);
-  *(uint2*)(out + i) = o;
+  *(uint2*)(out + (size_t)id * NO + n) = o;
 }
 
 // (columns, row blocks, splits), or one dimension in the order of tile_order for dense launches of several rounds.  Workgroups that are all
@@ -711,6 +767,23 @@ hipError_t launch_iobf(TileArgs a, int zk, int row_blocks, hipStream_t st) {
     hipLaunchKernelGGL((w4a16_tile_kernel<MI355Q_F16, MI355Q_ZP_PACKED, 4, GROUPED, 1, false, 1, true>), grid, block, shmem, st, a);
   }
   return hipSuccess;
+}
+
+// blocks of 64 slots, gate and up in one; (fp16 loop: fp16, or staged bf16 rows)
+template <int DT, int ZK, bool IOBF>
+hipError_t launch_glu_one(TileArgs a, int row_blocks, hipStream_t st) {
+  const dim3 grid = tile_grid<true>(a, row_blocks, 64, 2), block(256);
+  const size_t shmem = 2 * 64 * A_ROW;
+  static_assert(2 * 64 * A_ROW >= 16 * 1024, "the exchange of the halves");
+  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_tile_kernel<DT, ZK, 4, true, 1, false, 1, IOBF, true>,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((w4a16_tile_kernel<DT, ZK, 4, true, 1, false, 1, IOBF, true>), grid, block, shmem, st, a);
+  return hipSuccess;
+}
+template <int DT, bool IOBF>
+hipError_t launch_glu(const TileArgs& a, int zk, int row_blocks, hipStream_t st) {
+  return zk == MI355Q_ZP_NONE ? launch_glu_one<DT, MI355Q_ZP_NONE, IOBF>(a, row_blocks, st) : launch_glu_one<DT, MI355Q_ZP_PACKED, IOBF>(a, row_blocks, st);
 }
 
 // One workgroup per row of bf16 activations: the row's largest magnitude fixes a power of two 2^e that
@@ -1253,12 +1326,17 @@ size_t w4a16_grouped_workspace_bytes(int numel, int block_size, int max_blocks, 
   return need;
 }
 
+// whether gate and up columns can be made the gated ones where they are summed
+static bool w4a16_gates(const BlocksPlan& plan, int block_size, int N, int group_size, int zeros_kind) {
+  return block_size == 64 && !plan.rows && N % 256 == 0 && group_size % 128 == 0 && zeros_kind != MI355Q_ZP_PRESCALED;
+}
+
 int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales,
                          const float* scales_f32, const float* out_scale,
                          const void* zeros, int zeros_kind, const float* topk_weights,
                          const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                          int numel, int topk, int block_size, int max_blocks, int E, int K, int N,
-                         int group_size, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st) {
+                         int group_size, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st, bool glu) {
   const bool small_groups = group_size == 64 || group_size == 32;
   MQ_REQUIRE(group_size % 128 == 0 || (small_groups && !scales_f32 && !out_scale),
              "moe_w4a16: group_size=%d must be 32, 64 or a multiple of 128 (a multiple of 128 with fp32 scales)", group_size);
@@ -1272,6 +1350,7 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   const bool plain = !scales_f32 && !out_scale;
   BlocksPlan plan = {block_size == 32, 1};
   if (block_size == 64 && plain) plan = blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype);
+  MQ_REQUIRE(!glu || w4a16_gates(plan, block_size, N, group_size, zeros_kind), "moe_w4a16_gate_up: not for these operands");
   if (plain && group_size != 32 && plan.rows)
     return w4a16_rows_grouped_launch(out, x, qweight, scales, zeros, zeros_kind, topk_weights, sorted_ids, expert_ids, npp, numel,
                                      topk, block_size, max_blocks, E, K, N, group_size, dtype, st);
@@ -1326,7 +1405,10 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   a.s_stride = (long)(K / group_size) * N;
   a.z_stride = zeros_kind == MI355Q_ZP_PACKED ? (long)(K / group_size) * (N / 8) : (long)(K / group_size) * N;
   hipError_t e;
-  if (staged) {
+  if (glu) {
+    e = staged ? launch_glu<MI355Q_F16, true>(a, zeros_kind, max_blocks, st)
+        : dtype == MI355Q_F16 ? launch_glu<MI355Q_F16, false>(a, zeros_kind, max_blocks, st) : launch_glu<MI355Q_BF16, false>(a, zeros_kind, max_blocks, st);
+  } else if (staged) {
     e = launch_iobf<true>(a, zeros_kind, max_blocks, st);
   } else if (small_groups) {
     const int gpb = 128 / group_size;
@@ -1351,14 +1433,16 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   if (splits > 1) {
     // the reduction walks the aligned id list (at most max_blocks * block_size positions, cut at *npp on
     // the device): rows of ids that the alignment dropped have no partial tiles and are not touched
-    const long threads = (long)max_blocks * block_size * (N / 4);
+    const long threads = (long)max_blocks * block_size * ((glu ? N / 2 : N) / 4);
     const unsigned blocks = (unsigned)((threads + 255) / 256);
-    if (dtype == MI355Q_F16)
-      hipLaunchKernelGGL((w4a16_grouped_reduce_kernel<MI355Q_F16>), dim3(blocks), dim3(256), 0, st, (uint16_t*)out,
-                         (const float*)workspace, topk_weights, sorted_ids, npp, numel, N, splits, (const float*)nullptr, 1);
-    else
-      hipLaunchKernelGGL((w4a16_grouped_reduce_kernel<MI355Q_BF16>), dim3(blocks), dim3(256), 0, st, (uint16_t*)out,
-                         (const float*)workspace, topk_weights, sorted_ids, npp, numel, N, splits, a.row_scale, topk);
+#define MQ_REDUCE(DT, GLU)                                                                                                             \
+  hipLaunchKernelGGL((w4a16_grouped_reduce_kernel<DT, GLU>), dim3(blocks), dim3(256), 0, st, (uint16_t*)out, (const float*)workspace,    \
+                     topk_weights, sorted_ids, npp, numel, N, splits, a.row_scale, topk)
+    if (dtype == MI355Q_F16 && glu) MQ_REDUCE(MI355Q_F16, true);
+    else if (dtype == MI355Q_F16) MQ_REDUCE(MI355Q_F16, false);
+    else if (glu) MQ_REDUCE(MI355Q_BF16, true);
+    else MQ_REDUCE(MI355Q_BF16, false);
+#undef MQ_REDUCE
     MQ_LAUNCH_CHECK("moe_w4a16(split-K reduce)");
   }
   return 0;
@@ -1374,4 +1458,25 @@ extern "C" int mi355q_moe_w4a16_plan(int numel, int E, int K, int N, int group_s
   *rows_kernel = p.rows;
   *k_ranges = p.splits;
   return 0;
+}
+
+extern "C" int mi355q_moe_w4a16_gates(int numel, int block_size, int E, int K, int N, int group_size, int zeros_kind, int dtype) {
+  using namespace mi355q;
+  if (numel <= 0 || E <= 0 || K <= 0 || K % 128 != 0 || N <= 0 || group_size <= 0 || block_size != 64) return 0;
+  return w4a16_gates(blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype), block_size, N, group_size, zeros_kind);
+}
+
+extern "C" int mi355q_moe_w4a16_gate_up(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
+                                        int group_size, const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                                        const int32_t* num_tokens_post_pad, int numel, int topk, int block_size, int max_blocks, int E, int K,
+                                        int N, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace mi355q;
+  MQ_REQUIRE(numel >= 0 && topk > 0 && E > 0 && K > 0 && N > 0, "moe_w4a16_gate_up: bad shape numel=%d topk=%d E=%d K=%d N=%d", numel, topk, E, K, N);
+  if (numel == 0 || max_blocks == 0) return 0;
+  MQ_REQUIRE(out && a && w && w_scale && sorted_token_ids && expert_ids && num_tokens_post_pad, "moe_w4a16_gate_up: null pointer");
+  MQ_REQUIRE(zeros_kind == MI355Q_ZP_NONE || w_zeros, "moe_w4a16_gate_up: zero-points missing");
+  MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "moe_w4a16_gate_up: dtype %d", dtype);
+  MQ_REQUIRE(K % 128 == 0 && group_size > 0 && K % group_size == 0, "moe_w4a16_gate_up: K=%d group_size=%d", K, group_size);
+  return w4a16_grouped_launch(out, a, w, w_scale, nullptr, nullptr, w_zeros, zeros_kind, nullptr, sorted_token_ids, expert_ids, num_tokens_post_pad,
+                              numel, topk, block_size, max_blocks, E, K, N, group_size, dtype, workspace, workspace_bytes, as_stream(stream), true);
 }
