@@ -403,9 +403,9 @@ int mi355q_moe_gemm(void* out, const void* a, const void* w, const float* a_scal
                     int max_blocks, int E, int K, int N, int act_dtype, int out_dtype, int w_layout,
                     void* workspace, size_t workspace_bytes, void* stream);
 /* mi355q_moe_gemm with quant_mode 0 for columns that are gate and up: out is [numel, N / 2] and gets, bit for bit, what mi355q_silu_and_mul
- * makes of that result.  Where mi355q_moe_w4a16_gates answers 1: blocks of 64 slots that the tile kernel takes, N % 256 == 0, groups that
- * are multiples of 128, zero-points not pre-scaled; elsewhere it is an error.  Same workspace. */
-int mi355q_moe_w4a16_gates(int numel, int block_size, int E, int K, int N, int group_size, int zeros_kind, int dtype);
+ * makes of that result.  Where mi355q_moe_w4a16_gates answers 1: blocks of 16, 32 and 64 slots, N % 256 == 0, groups that are multiples of
+ * 128, zero-points not pre-scaled; elsewhere it is an error.  Same workspace. */
+int mi355q_moe_w4a16_gates(int block_size, int K, int N, int group_size, int zeros_kind);
 int mi355q_moe_w4a16_gate_up(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind, int group_size,
                              const int32_t* sorted_token_ids, const int32_t* expert_ids, const int32_t* num_tokens_post_pad, int numel, int topk,
                              int block_size, int max_blocks, int E, int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream);

@@ -962,20 +962,23 @@ def test_grouped_w4a16_plans_of_blocks_of_64(fmoe, E, K, N, rows, plans, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("E,K,N,rows,packed", [(64, 256, 1024, 70, True), (4, 4096, 256, 75, True), (16, 4096, 3072, 128, False), (2, 6528, 1024, 200, False),
-                                               (1, 128, 512, 64, True), (16, 4096, 3072, 50, True), (3, 640, 2816, 260, True)])
-def test_w4a16_gate_up(fmoe, E, K, N, rows, packed, dtype):
-    """Gate and up columns made the gated ones where they are summed, on tiles and behind K ranges, rows staged as fp16 or not, with foreign
-    experts and dropped ids: bit for bit the GEMM and silu_and_mul."""
+@pytest.mark.parametrize("block,E,K,N,rows,packed,way", [
+    (64, 64, 256, 1024, 70, True, 1), (64, 4, 4096, 256, 75, True, 6), (64, 16, 4096, 3072, 128, False, 1), (64, 2, 6528, 1024, 200, False, 6),
+    (64, 1, 128, 512, 64, True, None), (64, 16, 1664, 1024, 70, True, "rows"), (64, 3, 640, 2816, 260, False, None), (64, 3, 512, 256, 34, True, "rows"),
+    (32, 8, 1408, 2816, 20, True, None), (32, 3, 128, 256, 70, False, None), (32, 60, 384, 512, 17, True, None),
+    (16, 9, 1408, 2816, 9, True, None), (16, 64, 256, 256, 6, False, None), (16, 3, 4096, 1024, 40, True, None)])
+def test_w4a16_gate_up(fmoe, block, E, K, N, rows, packed, way, dtype):
+    """Gate and up columns made the gated ones where they are summed -- decode kernel, copying wavefronts at every height, tiles and K ranges,
+    rows staged as fp16 or not -- with foreign experts and dropped ids: bit for bit the GEMM and silu_and_mul."""
     import ctypes
     from vllm_gcu_amd import _lib
     lib, code, st, g, topk = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream, 128, 2
-    numel, kind = E * rows, _lib.ZP_PACKED if packed else _lib.ZP_NONE
+    numel, kind = E * rows // topk * topk, _lib.ZP_PACKED if packed else _lib.ZP_NONE
     kernel, ranges = ctypes.c_int(), ctypes.c_int()
     _lib.check(lib.mi355q_moe_w4a16_plan(numel, E, K, N, g, kind, code, ctypes.byref(kernel), ctypes.byref(ranges)), "plan")
-    gates = lib.mi355q_moe_w4a16_gates(numel, 64, E, K, N, g, kind, code)
-    print(f"case gate and up E={E} K={K} N={N} rows={rows} {dtype}: rows kernel {kernel.value} ranges {ranges.value} gates {gates}", flush=True)
-    assert gates == (not kernel.value)
+    print(f"case gate and up block={block} E={E} K={K} N={N} rows={rows} {dtype}: rows kernel {kernel.value} ranges {ranges.value}", flush=True)
+    assert lib.mi355q_moe_w4a16_gates(block, K, N, g, kind) and not lib.mi355q_moe_w4a16_gates(block, K, N + 128, g, kind)
+    assert way is None or dtype != torch.float16 or way == ("rows" if kernel.value else ranges.value)
     gen = torch.Generator(device="cuda").manual_seed(E + K + N)
     w = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // 8, N), dtype=torch.int32, device="cuda", generator=gen)
     z = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // g, N // 8), dtype=torch.int32, device="cuda", generator=gen) if packed else None
@@ -984,19 +987,15 @@ def test_w4a16_gate_up(fmoe, E, K, N, rows, packed, dtype):
     x[1] *= 60.0                                             # gates far on both sides
     ids = torch.randint(0, E, (numel // topk, topk), device="cuda", generator=gen, dtype=torch.int32)
     ids[1, 0], ids[-1, -1] = E + 1, -1                       # in no block
-    so, ex, npp = fmoe.moe_align_block_size(ids, 64, E)
+    so, ex, npp = fmoe.moe_align_block_size(ids, block, E)
     if E > 4:
         ex[1] = -1                                           # an expert of another rank
-    need = lib.mi355q_moe_gemm_workspace_bytes(0, numel, 64, ex.numel(), E, K, N)
+    need = lib.mi355q_moe_gemm_workspace_bytes(0, numel, block, ex.numel(), E, K, N)
     ws = torch.full((need // 4 + 1,), float("nan"), device="cuda")
     args = (x.data_ptr(), w.data_ptr())
-    zp, tail = None if z is None else z.data_ptr(), (so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, topk, 64, ex.numel(), E, K, N)
+    zp, tail = None if z is None else z.data_ptr(), (so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, topk, block, ex.numel(), E, K, N)
     got = torch.full((numel, N // 2), 7.0, dtype=dtype, device="cuda")
-    rc = lib.mi355q_moe_w4a16_gate_up(got.data_ptr(), *args, s.data_ptr(), zp, kind, g, *tail, code, ws.data_ptr(), need, st)
-    if not gates:
-        assert rc != 0
-        return
-    _lib.check(rc, "moe_w4a16_gate_up")
+    _lib.check(lib.mi355q_moe_w4a16_gate_up(got.data_ptr(), *args, s.data_ptr(), zp, kind, g, *tail, code, ws.data_ptr(), need, st), "moe_w4a16_gate_up")
     sums, want = torch.zeros(numel, N, dtype=dtype, device="cuda"), torch.empty(numel, N // 2, dtype=dtype, device="cuda")
     _lib.check(lib.mi355q_moe_gemm(sums.data_ptr(), *args, None, s.data_ptr(), zp, kind, 0, g, None, *tail, code, code, 0, ws.data_ptr(), need, st), "moe_gemm")
     _lib.check(lib.mi355q_silu_and_mul(want.data_ptr(), sums.data_ptr(), numel, N // 2, code, None, 1, st), "silu_and_mul")

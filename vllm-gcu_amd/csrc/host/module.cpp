@@ -610,8 +610,7 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
   // 36.7 / 62.7; eight of 4096 x 28672 at 1 / 5 / 16 48.6 / 103.2 / 132.5 and 47.5 / 104.1 / 132.4: two streams of weights instead of one.
   const bool unsorted = mode == kW4 && block == 16 && numel <= 64 && group % 128 == 0 && K % 128 == 0 && N % 128 == 0 && I % 128 == 0;
   const bool gate = unsorted && N * K <= (1 << 26), ids64 = ids.scalar_type() == at::kLong;
-  const bool tiles_gate = mode == kW4 && !unsorted && K % 128 == 0 &&
-                          mi355q_moe_w4a16_gates(numel, block, E, K, N, group, z1.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, dtype_code(dt));
+  const bool sorted_gate = mode == kW4 && !unsorted && mi355q_moe_w4a16_gates(block, K, N, group, z1.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE);
   const bool gate_up = mode == kFp8 && block <= 64 && N % 256 == 0;       // the first GEMM applies the gate and quantises
   // one allocation: quantised inputs of both GEMMs with their scales, the three intermediate matrices, the alignment
   int64_t total = 0;
@@ -663,7 +662,7 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
       check(mi355q_moe_fp8_gate_up_quant(reinterpret_cast<uint8_t*>(b + o_q2), s2, b + o_q1, w1.data_ptr(), s1, static_cast<const float*>(s1p->data_ptr()),
                                          sorted, eid, npp, numel, T, block, blocks, E, K, N, code, 1, stream),
             "moe_fp8_gate_up_quant");
-    else if (tiles_gate)
+    else if (sorted_gate)
       check(mi355q_moe_w4a16_gate_up(b + o_c2, x.data_ptr(), static_cast<const int32_t*>(w1.data_ptr()), s1p->data_ptr(), ptr(z1),
                                      z1.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, group, sorted, eid, npp, numel, T, block, blocks, E, K, N, code,
                                      ws.p, ws.bytes, stream),
@@ -677,7 +676,7 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
     } else if (mode == kFp8)
       check(mi355q_fp8_group_quant(reinterpret_cast<uint8_t*>(b + o_q2), s2, b + o_c1, numel, I, 128, 1, code, nullptr, 1, stream),
             "fp8_group_quant");
-    else if (!gate && !tiles_gate)
+    else if (!gate && !sorted_gate)
       check(mi355q_silu_and_mul(b + o_c2, b + o_c1, numel, I, code, nullptr, 1, stream), "silu_and_mul");
     if (mode == kInt8)
       check(mi355q_dynamic_int8_quant(reinterpret_cast<int8_t*>(b + o_q2), s2, b + o_c2, numel, I, code, nullptr, stream),

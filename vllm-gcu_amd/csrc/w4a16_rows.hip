@@ -97,12 +97,16 @@ template <> struct RowsMma<MI355Q_BF16> {
 };
 
 // 16 MT rows x 64 NT columns; KS = 2 K ranges with NW wavefronts that compute and two that copy, and a ring of LDS stages,
-// each.  GPB: quantisation groups per K block (1 for group sizes that are multiples of 128, 2 / 4 for 64 / 32)
-template <int MT_, int NT_, int GPB_, int ZK>
+// each.  GPB: quantisation groups per K block (1 for group sizes that are multiples of 128, 2 / 4 for 64 / 32).  GLU: half of the
+// columns are gate and half the up columns that go with them, with the scales and zero-points of both slabs in a stage.
+template <int MT_, int NT_, int GPB_, int ZK, bool GLU_ = false>
 struct RowsCfg {
+  static constexpr bool GLU = GLU_;
+  static_assert(!GLU || (NT_ == 2 && GPB_ == 1), "64 and 64 columns, one group");
   static constexpr int MT = MT_, NW = 4, NT = NT_, KS = 2, GPB = GPB_;
   static constexpr int BM = 16 * MT, BN = 16 * NW * NT, CW = NW * KS, THREADS = 64 * (CW + 2 * KS);
-  static constexpr int A_BYTES = BM * 256, W_BYTES = 1024 * NW * NT, S_BYTES = 256 * GPB, Z_BYTES = (ZK == MI355Q_ZP_PRESCALED ? 256 : 64) * GPB;
+  static constexpr int A_BYTES = BM * 256, W_BYTES = 1024 * NW * NT, HV = GLU ? 2 : 1,
+                       S_BYTES = 256 * GPB * HV, Z_BYTES = (ZK == MI355Q_ZP_PRESCALED ? 256 : 64) * GPB * HV;
   static constexpr int W_OFF = A_BYTES, S_OFF = W_OFF + W_BYTES, Z_OFF = S_OFF + S_BYTES, STAGE = Z_OFF + Z_BYTES;
   static constexpr int XC = A_BYTES / 2048, WC = NW * NT / 2, NC = XC + WC + 1;   // copies of a copying wavefront per stage
   // two workgroups per CU where two stages fit so (deeper rings did not gain: the copies are bound by their rate)
@@ -126,7 +130,9 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
   const int wave = copies ? (wg - C::CW) % 2 : wg % NW, ks = copies ? (wg - C::CW) / 2 : wg / NW;
   const int c = lane & 15, kq = lane >> 4;
   const int M = a.M, N = a.N, K = a.K, G = K >> 7;
-  const int slab = tn * NW * NT >> 3, t0 = tn * NW * NT & 7;           // 128-column slab, first of the workgroup's 16-column tiles in it
+  constexpr bool GLU = C::GLU;
+  // 128-column slab (GLU: of the gate columns; the up columns' is N / 256 further), first of the workgroup's 16-column tiles in it
+  const int slab = GLU ? tn >> 1 : tn * NW * NT >> 3, t0 = GLU ? 4 * (tn & 1) : tn * NW * NT & 7;
   const int nk = (ng + KS - 1) / KS;                  // ... of each of its ranges (the last may hold fewer, even none)
   const int mine = min(ng - ks * nk, nk);
 
@@ -149,14 +155,15 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
     int kb = min(g0 + ks * nk, G - 1);                // the K block that the next copies are of
     const int klast = max(g0 + ks * nk + mine - 1, kb);
     const char* xg = (const char*)a.x + (size_t)kb * 256;
-    const char* qg = (const char*)a.qw + ((size_t)slab * G + kb) * 8192 + (t0 + wave * C::WC) * 1024;
+    const char* qg = (const char*)a.qw + ((size_t)(slab + (GLU ? wave * (N >> 8) : 0)) * G + kb) * 8192 + (t0 + (GLU ? 0 : wave * C::WC)) * 1024;
     // the first wavefront of the range copies the scales, the second the zero-points (without any, the scales again: both
     // have the same number of copies to wait for)
     const bool packed = ZK == MI355Q_ZP_PACKED && wave == 1, zwave = ZK != MI355Q_ZP_NONE && wave == 1;
     const uint32_t szrow = packed ? (uint32_t)N / 2 : (uint32_t)N * 2;
-    const uint32_t szoff = packed ? (uint32_t)(lane & 3) * 16u + (uint32_t)(lane >> 2) * szrow
-                                  : (uint32_t)(lane & 15) * 16u + (uint32_t)(lane >> 4) * szrow;
-    const int szlanes = packed ? 4 * GPB : 16 * GPB;
+    const uint32_t sznext = GLU ? szrow / 2 : szrow;     // from one group's row to the next one's, or from gate to up
+    const uint32_t szoff = packed ? (uint32_t)(lane & 3) * 16u + (uint32_t)(lane >> 2) * sznext
+                                  : (uint32_t)(lane & 15) * 16u + (uint32_t)(lane >> 4) * sznext;
+    const int szlanes = (packed ? 4 : 16) * GPB * C::HV;
     const char* const szg = zwave ? a.zeros + (packed ? 64 : 256) * slab : (const char*)a.scales + 256 * slab;
     const uint32_t szlds = zwave ? C::Z_OFF : C::S_OFF;
     const uint32_t ring = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char*)lds) + ks * C::RING;
@@ -209,15 +216,16 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
 #pragma unroll
         for (int t = 0; t < NT; ++t) w[t] = *(const u4*)(st + C::W_OFF + (wave * NT + t) * 1024 + lane * 16);
 #pragma unroll
-        for (int g = 0; g < GPB; ++g) zw[g] = ZK == MI355Q_ZP_PACKED ? *(const uint32_t*)(st + C::Z_OFF + 64 * g + c * 4) : 0x88888888u;
+        for (int g = 0; g < GPB; ++g)
+          zw[g] = ZK == MI355Q_ZP_PACKED ? *(const uint32_t*)(st + C::Z_OFF + 64 * (GLU ? wave >> 1 : g) + c * 4) : 0x88888888u;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) av[0][mt] = *(const u4*)(st + a_pos[0] + mt * 4096);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          const int tile = t0 + wave * NT + t;
+          const int tile = t0 + (GLU ? wave & 1 : wave) * NT + t;
 #pragma unroll
           for (int g = 0; g < GPB; ++g) {
-            sc[t][g] = Elem<DT>::to_f32(*(const uint16_t*)(st + C::S_OFF + 256 * g + (8 * c + tile) * 2));
+            sc[t][g] = Elem<DT>::to_f32(*(const uint16_t*)(st + C::S_OFF + 256 * (GLU ? wave >> 1 : g) + (8 * c + tile) * 2));
             if constexpr (ZK == MI355Q_ZP_PRESCALED) {
               const uint16_t zs = *(const uint16_t*)(st + C::Z_OFF + 256 * g + (8 * c + tile) * 2);
               const float zf = prescaled_zero<DT>(zs, sc[t][g]);
@@ -310,6 +318,25 @@ __device__ __forceinline__ void rows_tile(const RowsArgs& a, const int32_t* ids,
           *(float*)(lds + ks * C::RING + (mt * 16 + 4 * kq + i) * EP + (TC * c + wave * NT + t) * 4) = acc[mt][t][i];
   }
   __syncthreads();
+  if constexpr (GLU) {
+    // tile columns 8 c .. are four gate and the four up columns that go with them
+    const int gc = tid % 16;
+    for (int r = tid / 16; r < C::BM; r += C::THREADS / 16) {
+      const int m = ids[r];
+      if (m >= a.numel) continue;
+      uint2 o[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        f4 v = *(const f4*)(lds + r * EP + (2 * gc + h) * 16);
+#pragma unroll
+        for (int k = 1; k < KS; ++k) v += *(const f4*)(lds + k * C::RING + r * EP + (2 * gc + h) * 16);
+        o[h].x = (uint32_t)Elem<DT>::from_f32(v[0] + 0.f) | ((uint32_t)Elem<DT>::from_f32(v[1] + 0.f) << 16);
+        o[h].y = (uint32_t)Elem<DT>::from_f32(v[2] + 0.f) | ((uint32_t)Elem<DT>::from_f32(v[3] + 0.f) << 16);
+      }
+      *(uint2*)(a.out + (size_t)m * (N >> 1) + 128 * slab + 8 * gc + t0) = make_uint2(silu_mul16x2<DT>(o[0].x, o[1].x), silu_mul16x2<DT>(o[0].y, o[1].y));
+    }
+    return;
+  }
   constexpr int TPR = C::BN / 4;                      // threads per row
   const int q = tid % TPR, n = 128 * slab + 8 * (q / Q) + t0 + 4 * (q % Q);
   float bs[4] = {0.f, 0.f, 0.f, 0.f};
@@ -348,9 +375,11 @@ w4a16_rows_kernel(RowsArgs a) {
   rows_tile<DT, ZK, C, false>(a, nullptr, tm * C::BM, tn, g0, min((a.K >> 7) - g0, a.kper));
 }
 
-// Blocks of up to 16 MAX slots: a block takes the tile of as many row tiles as hold real slots (they come first)
-template <int DT, int ZK, int GPB, int MAX>
-__global__ void __launch_bounds__(768, (RowsCfg<MAX, 2, GPB, ZK>::PAIR + 1) * 3)
+// Blocks of up to 16 MAX slots: a block takes the tile of as many row tiles as hold real slots (they come first).  GLU: the columns are gate
+// and up, and what is stored ([numel, N / 2]) is what silu_and_mul makes of the sums that would have been: its pass and half of the stores are
+// saved (us for a whole layer, 86 .. 224 of which 4 .. 7 were that pass: 79.0 -> 74.9, 111.6 -> 107.3, 171.7 -> 168.4).
+template <int DT, int ZK, int GPB, int MAX, bool GLU>
+__global__ void __launch_bounds__(768, (RowsCfg<MAX, 2, GPB, ZK, GLU>::PAIR + 1) * 3)
 w4a16_rows_grouped_kernel(RowsArgs a) {
   const int base = blockIdx.y * a.block;
   if (base >= *a.npp) return;                         // block beyond the padded ids
@@ -360,18 +389,19 @@ w4a16_rows_grouped_kernel(RowsArgs a) {
   if (!real) return;                                  // pads only
   const long e = a.expert_ids[blockIdx.y];
   if (e < 0 || e >= a.E) {                            // not one of this rank's experts: zero rows, no weights read
-    zero_block_columns(a.out, ids, a.block, a.numel, a.N, tn * 128, 128, 768);
+    if (GLU) zero_block_columns(a.out, ids, a.block, a.numel, a.N >> 1, tn * 64, 64, 768);
+    else zero_block_columns(a.out, ids, a.block, a.numel, a.N, tn * 128, 128, 768);
     return;
   }
   a.qw = (const u4*)((const char*)a.qw + e * a.w_stride);
   a.scales = (const uint16_t*)((const char*)a.scales + e * a.s_stride);
   if (a.zeros) a.zeros += e * a.z_stride;
   const int tiles = __builtin_amdgcn_readfirstlane((64 - __builtin_clzll(real) + 15) >> 4), G = a.K >> 7;
-  if (tiles == 1) return rows_tile<DT, ZK, RowsCfg<1, 2, GPB, ZK>, true>(a, ids, 0, tn, 0, G);
-  if (MAX == 2 || tiles == 2) return rows_tile<DT, ZK, RowsCfg<2, 2, GPB, ZK>, true>(a, ids, 0, tn, 0, G);
+  if (tiles == 1) return rows_tile<DT, ZK, RowsCfg<1, 2, GPB, ZK, GLU>, true>(a, ids, 0, tn, 0, G);
+  if (MAX == 2 || tiles == 2) return rows_tile<DT, ZK, RowsCfg<2, 2, GPB, ZK, GLU>, true>(a, ids, 0, tn, 0, G);
   if constexpr (MAX > 2) {
-    if (tiles == 3) return rows_tile<DT, ZK, RowsCfg<3, 2, GPB, ZK>, true>(a, ids, 0, tn, 0, G);
-    rows_tile<DT, ZK, RowsCfg<4, 2, GPB, ZK>, true>(a, ids, 0, tn, 0, G);
+    if (tiles == 3) return rows_tile<DT, ZK, RowsCfg<3, 2, GPB, ZK, GLU>, true>(a, ids, 0, tn, 0, G);
+    rows_tile<DT, ZK, RowsCfg<4, 2, GPB, ZK, GLU>, true>(a, ids, 0, tn, 0, G);
   }
 }
 
@@ -449,15 +479,15 @@ RowsPlan rows_make_plan(int M, int K, int N, bool split) {
 
 RowsPlan rows_plan(int M, int K, int N) { return cached_plan(0, M, N, K, [](int, int M, int N, int K) { return rows_make_plan(M, K, N, true); }); }
 
-template <int DT, int ZK, int GPB, int MAX>
+template <int DT, int ZK, int GPB, int MAX, bool GLU = false>
 int launch_rows_grouped(const RowsArgs& a, int max_blocks, hipStream_t st) {
   size_t shmem = 0;
-  for (size_t b : {(size_t)RowsCfg<1, 2, GPB, ZK>::RING, (size_t)RowsCfg<2, 2, GPB, ZK>::RING, MAX > 2 ? (size_t)RowsCfg<3, 2, GPB, ZK>::RING : 0,
-                   MAX > 2 ? (size_t)RowsCfg<4, 2, GPB, ZK>::RING : 0})
+  for (size_t b : {(size_t)RowsCfg<1, 2, GPB, ZK, GLU>::RING, (size_t)RowsCfg<2, 2, GPB, ZK, GLU>::RING, MAX > 2 ? (size_t)RowsCfg<3, 2, GPB, ZK, GLU>::RING : 0,
+                   MAX > 2 ? (size_t)RowsCfg<4, 2, GPB, ZK, GLU>::RING : 0})
     shmem = std::max(shmem, 2 * b);
-  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_rows_grouped_kernel<DT, ZK, GPB, MAX>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_rows_grouped_kernel<DT, ZK, GPB, MAX, GLU>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   MQ_REQUIRE(attr == hipSuccess, "moe_w4a16(rows): cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
-  hipLaunchKernelGGL((w4a16_rows_grouped_kernel<DT, ZK, GPB, MAX>), dim3((unsigned)(a.N / 128), (unsigned)max_blocks), dim3(768), shmem, st, a);
+  hipLaunchKernelGGL((w4a16_rows_grouped_kernel<DT, ZK, GPB, MAX, GLU>), dim3((unsigned)(a.N / 128), (unsigned)max_blocks), dim3(768), shmem, st, a);
   MQ_LAUNCH_CHECK("moe_w4a16(rows)");
   return 0;
 }
@@ -544,7 +574,7 @@ int w4a16_rows_launch(void* out, const void* x, const int32_t* qweight, const vo
 int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
                               const float* topk_weights, const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                               int numel, int topk, int block_size, int max_blocks, int E, int K, int N, int group_size, int dtype,
-                              hipStream_t st) {
+                              hipStream_t st, bool glu) {
   MQ_REQUIRE(block_size == 32 || block_size == 64, "moe_w4a16(rows): blocks of 32 or 64 slots, got %d", block_size);
   MQ_REQUIRE(group_size % 128 == 0 || group_size == 64, "moe_w4a16(rows): group size %d", group_size);
   RowsArgs a = {};
@@ -558,6 +588,16 @@ int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, 
   a.w_stride = (long)K * N / 2;
   a.s_stride = (long)(K / group_size) * N * 2;
   a.z_stride = zeros_kind == MI355Q_ZP_PACKED ? (long)(K / group_size) * N / 2 : a.s_stride;
+#define MQ_GLU(DT, ZK)                                                                                                                  \
+  return block_size == 32 ? launch_rows_grouped<DT, ZK, 1, 2, true>(a, max_blocks, st) : launch_rows_grouped<DT, ZK, 1, 4, true>(a, max_blocks, st)
+  if (glu) {
+    MQ_REQUIRE(group_size % 128 == 0 && N % 256 == 0 && zeros_kind != MI355Q_ZP_PRESCALED, "moe_w4a16(rows): gate and up of N=%d, group size %d", N, group_size);
+    if (dtype == MI355Q_F16 && zeros_kind == MI355Q_ZP_PACKED) MQ_GLU(MI355Q_F16, MI355Q_ZP_PACKED);
+    if (dtype == MI355Q_F16) MQ_GLU(MI355Q_F16, MI355Q_ZP_NONE);
+    if (zeros_kind == MI355Q_ZP_PACKED) MQ_GLU(MI355Q_BF16, MI355Q_ZP_PACKED);
+    MQ_GLU(MI355Q_BF16, MI355Q_ZP_NONE);
+  }
+#undef MQ_GLU
 #define MQ_MAX(DT, ZK, GPB)                                                                                               \
   return block_size == 32 ? launch_rows_grouped<DT, ZK, GPB, 2>(a, max_blocks, st) : launch_rows_grouped<DT, ZK, GPB, 4>(a, max_blocks, st)
 #define MQ_ZK(DT, ZK)                         \
