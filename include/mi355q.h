@@ -303,6 +303,10 @@ int mi355q_moe_align_block_size(const void* topk_ids, int ids_are_int64, int num
                                 const int32_t* valid_rows, int num_experts, int block_size,
                                 const int32_t* expert_map, int32_t* sorted_token_ids,
                                 int32_t* expert_ids, int32_t* num_tokens_post_pad, void* stream);
+/* mi355q_fp8_group_quant (groups of 128, rows [rows, K]) and mi355q_moe_align_block_size (no expert map, no valid count) in one launch. */
+int mi355q_moe_align_fp8_quant(uint8_t* q, float* q_scales, const void* x, long rows, int K, int dtype, const void* topk_ids, int ids_are_int64,
+                               int numel, int topk, int num_experts, int block_size, int32_t* sorted_token_ids, int32_t* expert_ids,
+                               int32_t* num_tokens_post_pad, void* stream);
 
 /* ---- activation glue --------------------------------------------------------
  * silu_and_mul / silu_and_mul_pad (csrc/src/silu_and_mul.cpp:29-109,

@@ -342,3 +342,31 @@ def test_valid_token_count_is_read_on_the_device_under_graph_replay(ops):
         assert (out[n:] == -1.0).all(), n       # rows past the count are left alone
         assert torch.equal(q.view(torch.uint8)[:n], full_q[:n]), n
         assert (q.view(torch.uint8)[n:] == 0x7f).all(), n
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K,T,E,B", [(1, 128, 1, 1, 16), (1, 7168, 8, 256, 16), (3, 1024, 6, 64, 32), (9, 384, 2, 8, 64), (257, 2048, 8, 256, 16),
+                                       (2100, 1152, 2, 16, 128), (64, 128, 4, 963, 16)])
+def test_moe_align_fp8_quant(M, K, T, E, B, dtype):
+    """One launch for the alignment and the rows' quantisation: every output bit of the two."""
+    from vllm_gcu_amd import _lib
+    print(f"case align and quant M={M} K={K} T={T} E={E} B={B} {dtype}", flush=True)
+    lib, code, st = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device="cuda").manual_seed(M + K + E)
+    x = (torch.randn(M, K, device="cuda", generator=gen) * 3).to(dtype)
+    x[0, :128] = 0
+    for ids in (torch.randint(0, E, (M, T), device="cuda", generator=gen), torch.randint(-1, E + 1, (M, T), device="cuda", generator=gen).int()):
+        wide, cap = int(ids.dtype == torch.int64), M * T + E * (B - 1)
+        outs = []
+        for fused in (False, True):
+            q, sc = torch.full((M, K), 0x55, dtype=torch.uint8, device="cuda"), torch.full((M, K // 128), float("nan"), device="cuda")
+            so, ex, npp = (torch.full((n,), -7, dtype=torch.int32, device="cuda") for n in (cap, cap // B, 1))
+            if fused:
+                _lib.check(lib.mi355q_moe_align_fp8_quant(q.data_ptr(), sc.data_ptr(), x.data_ptr(), M, K, code, ids.data_ptr(), wide, M * T, T, E, B,
+                                                          so.data_ptr(), ex.data_ptr(), npp.data_ptr(), st), "moe_align_fp8_quant")
+            else:
+                _lib.check(lib.mi355q_fp8_group_quant(q.data_ptr(), sc.data_ptr(), x.data_ptr(), M, K, 128, 0, code, None, 1, st), "fp8_group_quant")
+                _lib.check(lib.mi355q_moe_align_block_size(ids.data_ptr(), wide, M * T, T, None, E, B, None, so.data_ptr(), ex.data_ptr(),
+                                                           npp.data_ptr(), st), "moe_align_block_size")
+            outs.append((q, sc, so, ex, npp))
+        assert all(torch.equal(a, b) for a, b in zip(*outs))

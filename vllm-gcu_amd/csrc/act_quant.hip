@@ -4,7 +4,7 @@
 // fp32 arithmetic, one pass over the data.  Every kernel takes an optional
 // device int32 `valid_rows` so padded (graph-captured) batches skip dead rows
 // without a host synchronisation.
-#include "common.h"
+#include "moe_align.h"
 
 #include <algorithm>
 
@@ -71,12 +71,10 @@ silu_and_mul_kernel(uint16_t* out, const uint16_t* x, uint32_t rows, int d, Fast
 // ---- per-token-group fp8 quantisation (optionally fused behind SiLU-gate) ---
 // A group of `gs` elements is handled by gs/8 adjacent lanes (gs in 64,128,256,512).
 template <int DT, bool SILU>
-__global__ void __launch_bounds__(256)
-group_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, uint32_t rows, int K, FastDiv chunks, int lpg,
-                       const int* valid_rows, int rpc, long row0) {
-  const uint32_t total = live_rows(rows, valid_rows, rpc, row0) * chunks.d;     // 8-element pieces; lpg (a power of two <= 64) lanes per group
+__device__ __forceinline__ void group_fp8_quant(uint8_t* out, float* scales, const uint16_t* x, uint32_t total, int K, const FastDiv& chunks, int lpg,
+                                                uint32_t first, uint32_t step) {
   const int lg = 31 - __clz(lpg);
-  for (uint32_t i0 = blockIdx.x * 256; i0 < total; i0 += gridDim.x * 256) {
+  for (uint32_t i0 = first; i0 < total; i0 += step) {
     const uint32_t i = i0 + threadIdx.x;
     const bool live = i < total;
     const uint32_t r = live ? chunks.div(i) : 0, c = live ? i - r * chunks.d : 0;
@@ -108,6 +106,25 @@ group_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, uint32_t 
       if ((c & (lpg - 1)) == 0) scales[i >> lg] = s;
     }
   }
+}
+template <int DT, bool SILU>
+__global__ void __launch_bounds__(256)
+group_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, uint32_t rows, int K, FastDiv chunks, int lpg,
+                       const int* valid_rows, int rpc, long row0) {
+  const uint32_t total = live_rows(rows, valid_rows, rpc, row0) * chunks.d;     // 8-element pieces; lpg (a power of two <= 64) lanes per group
+  group_fp8_quant<DT, SILU>(out, scales, x, total, K, chunks, lpg, blockIdx.x * 256, gridDim.x * 256);
+}
+
+// The two things that fp8 experts need before their first GEMM and that do not need each other, side by side: the first workgroup aligns
+// the slots, the others quantise the rows.  (The alignment is one workgroup's latency, 6 us alone, the rows 5 at 256 x 7168.  us, the whole layer, two
+// launches -> here: 43.4 -> 41.2, 91.0 -> 88.2, 260.4 -> 257.7, 1739.9 -> 1735.3.)
+template <int DT, typename IdT>
+__global__ void __launch_bounds__(ALIGN_WAVES * 64)
+moe_align_fp8_quant_kernel(uint8_t* out, float* scales, const uint16_t* x, uint32_t total, int K, FastDiv chunks, const IdT* topk_ids, int numel,
+                           int top, int E, int B, int* sorted_ids, int cap, int* expert_ids, int nblocks, int* npp) {
+  extern __shared__ int sm[];
+  if (blockIdx.x == 0) return moe_align_ids(topk_ids, numel, top, (const int*)nullptr, E, B, (const int*)nullptr, sorted_ids, cap, expert_ids, nblocks, npp, sm);
+  group_fp8_quant<DT, false>(out, scales, x, total, K, chunks, 16, (blockIdx.x - 1) * (ALIGN_WAVES * 64), (gridDim.x - 1) * (ALIGN_WAVES * 64));
 }
 
 // ---- per-token fp8 (one workgroup per row) and static fp8 --------------------
@@ -667,5 +684,35 @@ extern "C" int mi355q_rms_norm(void* out, float* out_scales, const void* x, void
     else launch_rms<MI355Q_BF16, false>(quant_mode, grid, st, out, out_scales, xp, rp, wp, scale, eps, K, group_size);
   }
   MQ_LAUNCH_CHECK("rms_norm");
+  return 0;
+}
+
+extern "C" int mi355q_moe_align_fp8_quant(uint8_t* q, float* q_scales, const void* x, long rows, int K, int dtype, const void* topk_ids,
+                                          int ids_are_int64, int numel, int topk, int num_experts, int block_size, int32_t* sorted_token_ids,
+                                          int32_t* expert_ids, int32_t* num_tokens_post_pad, void* stream) {
+  MQ_REQUIRE(rows > 0 && K > 0 && K % 128 == 0 && numel > 0 && num_experts > 0 && block_size > 0 && topk > 0,
+             "moe_align_fp8_quant: bad arguments rows=%ld K=%d numel=%d E=%d block=%d topk=%d", rows, K, numel, num_experts, block_size, topk);
+  MQ_REQUIRE(q && q_scales && x && topk_ids && sorted_token_ids && expert_ids && num_tokens_post_pad, "moe_align_fp8_quant: null pointer");
+  MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "moe_align_fp8_quant: dtype %d must be f16 or bf16", dtype);
+  const size_t shmem = moe_align_lds(num_experts);
+  if (rows > rows_per_launch(K / 8) || shmem > 64 * 1024 || num_experts > 1024) {      // (refused there, or too many rows for one launch)
+    if (int rc = mi355q_fp8_group_quant(q, q_scales, x, rows, K, 128, 0, dtype, nullptr, 1, stream)) return rc;
+    return mi355q_moe_align_block_size(topk_ids, ids_are_int64, numel, topk, nullptr, num_experts, block_size, nullptr, sorted_token_ids, expert_ids,
+                                       num_tokens_post_pad, stream);
+  }
+  const uint32_t total = (uint32_t)rows * (uint32_t)(K / 8);
+  const unsigned grid = 1 + (unsigned)std::min<long>(((long)total + 1023) / 1024, (long)device_cu_count() * 8);
+  const int cap = numel + num_experts * (block_size - 1);
+  const FastDiv chunks((uint32_t)(K / 8));
+#define MQ_FRONT(DT, ID)                                                                                                                    \
+  hipLaunchKernelGGL((moe_align_fp8_quant_kernel<DT, ID>), dim3(grid), dim3(ALIGN_WAVES * 64), shmem, as_stream(stream), q, q_scales,          \
+                     (const uint16_t*)x, total, K, chunks, (const ID*)topk_ids, numel, topk, num_experts, block_size, sorted_token_ids, cap,    \
+                     expert_ids, cap / block_size, num_tokens_post_pad)
+  if (dtype == MI355Q_F16 && ids_are_int64) MQ_FRONT(MI355Q_F16, long);
+  else if (dtype == MI355Q_F16) MQ_FRONT(MI355Q_F16, int);
+  else if (ids_are_int64) MQ_FRONT(MI355Q_BF16, long);
+  else MQ_FRONT(MI355Q_BF16, int);
+#undef MQ_FRONT
+  MQ_LAUNCH_CHECK("moe_align_fp8_quant");
   return 0;
 }

@@ -646,12 +646,13 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
             *npp = reinterpret_cast<int32_t*>(b + o_npp);
     float *s1 = reinterpret_cast<float*>(b + o_s1), *s2 = reinterpret_cast<float*>(b + o_s2);
     if (mode == kFp8)
-      check(mi355q_fp8_group_quant(reinterpret_cast<uint8_t*>(b + o_q1), s1, x.data_ptr(), M, K, 128, 0, code, nullptr, 1, stream),
-            "fp8_group_quant");
+      check(mi355q_moe_align_fp8_quant(reinterpret_cast<uint8_t*>(b + o_q1), s1, x.data_ptr(), M, K, code, ids.data_ptr(), ids64, numel, T, E, block,
+                                       sorted, eid, npp, stream),
+            "moe_align_fp8_quant");
     else if (mode == kInt8)
       check(mi355q_dynamic_int8_quant(reinterpret_cast<int8_t*>(b + o_q1), s1, x.data_ptr(), M, K, code, nullptr, stream),
             "dynamic_int8_quant");
-    if (!unsorted)
+    if (!unsorted && mode != kFp8)
       check(mi355q_moe_align_block_size(ids.data_ptr(), ids64, numel, T, nullptr, E, block, nullptr, sorted, eid, npp, stream), "moe_align_block_size");
     if (unsorted)
       check(mi355q_moe_w4a16_unsorted(b + (gate ? o_c2 : o_c1), x.data_ptr(), static_cast<const int32_t*>(w1.data_ptr()), s1p->data_ptr(), ptr(z1),
