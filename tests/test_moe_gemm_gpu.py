@@ -1002,3 +1002,38 @@ def test_w4a16_gate_up(fmoe, block, E, K, N, rows, packed, way, dtype):
     in_block = torch.zeros(numel + 1, dtype=torch.bool, device="cuda")
     in_block[so[:int(npp)].long().clamp(max=numel)] = True
     assert torch.equal(got[in_block[:numel]], want[in_block[:numel]]) and (got[~in_block[:numel]] == 7.0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block,E,K,N,rows,ranges", [(64, 4, 4096, 256, 74, 6), (64, 2, 6528, 1024, 200, 6), (64, 8, 7168, 1024, 100, 4),
+                                                     (64, 8, 14336, 4096, 128, None), (64, 16, 4096, 3072, 128, 1), (64, 8, 3072, 1152, 70, None),
+                                                     (32, 8, 1408, 2048, 18, None), (16, 8, 1408, 2048, 10, None)])
+def test_w4a16_down_sum(fmoe, block, E, K, N, rows, ranges, dtype):
+    """The second GEMM and the sum over a token's slots, in one launch behind K ranges and in two without, with an expert of another rank:
+    bit for bit the two calls."""
+    import ctypes
+    from vllm_gcu_amd import _lib
+    lib, code, st, g, topk = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream, 128, 2
+    numel = E * rows
+    kernel, taken = ctypes.c_int(), ctypes.c_int()
+    _lib.check(lib.mi355q_moe_w4a16_plan(numel, E, K, N, g, _lib.ZP_PACKED, code, ctypes.byref(kernel), ctypes.byref(taken)), "plan")
+    print(f"case down and sum block={block} E={E} K={K} N={N} rows={rows} {dtype}: rows kernel {kernel.value} ranges {taken.value}", flush=True)
+    assert ranges is None or dtype != torch.float16 or taken.value == ranges
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w, z = (torch.randint(-2 ** 31, 2 ** 31 - 1, (E, r, c), dtype=torch.int32, device="cuda", generator=gen) for r, c in ((K // 8, N), (K // g, N // 8)))
+    s = (torch.rand(E, K // g, N, device="cuda", generator=gen) * 0.01 + 0.001).to(dtype)
+    x, rw = torch.randn(numel, K, device="cuda", generator=gen).to(dtype), torch.rand(numel, device="cuda", generator=gen)
+    ids = torch.randint(0, E, (numel // topk, topk), device="cuda", generator=gen, dtype=torch.int32)
+    so, ex, npp = fmoe.moe_align_block_size(ids, block, E)
+    ex[1] = -1                                               # an expert of another rank
+    need = lib.mi355q_moe_gemm_workspace_bytes(0, numel, block, ex.numel(), E, K, N)
+    ws = torch.full((need // 4 + 1,), float("nan"), device="cuda")
+    rows_out, out, want = (torch.full((n, N), float("nan"), dtype=dtype, device="cuda") for n in (numel, numel // topk, numel // topk))
+    _lib.check(lib.mi355q_moe_w4a16_down_sum(out.data_ptr(), rows_out.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(),
+                                             _lib.ZP_PACKED, g, rw.data_ptr(), so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel // topk, topk, block,
+                                             ex.numel(), E, K, N, code, ws.data_ptr(), need, st), "moe_w4a16_down_sum")
+    _lib.check(lib.mi355q_moe_gemm(rows_out.data_ptr(), x.data_ptr(), w.data_ptr(), None, s.data_ptr(), z.data_ptr(), _lib.ZP_PACKED, 0, g, rw.data_ptr(),
+                                   so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, 1, block, ex.numel(), E, K, N, code, code, 0, ws.data_ptr(), need,
+                                   st), "moe_gemm")
+    _lib.check(lib.mi355q_moe_sum(want.data_ptr(), rows_out.data_ptr(), numel // topk, topk, N, code, code, None, st), "moe_sum")
+    assert torch.equal(out, want) and not out.isnan().any()

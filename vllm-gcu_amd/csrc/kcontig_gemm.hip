@@ -674,7 +674,8 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
                          const void* zeros, int zeros_kind, const float* topk_weights,
                          const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                          int numel, int topk, int block_size, int max_blocks, int E, int K, int N,
-                         int group_size, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st, bool glu = false);
+                         int group_size, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st, bool glu = false,
+                         struct MoeSum* sum = nullptr);
 size_t w4a16_grouped_workspace_bytes(int numel, int block_size, int max_blocks, int E, int K, int N);
 int int8_grouped_launch(void* out, const void* a, const void* w, const float* a_scale, int a_scale_per_row,
                         const float* w_scale, const float* topk_weights, const int32_t* sorted_ids,

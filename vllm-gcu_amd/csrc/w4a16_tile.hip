@@ -1241,6 +1241,8 @@ int w4a16_decode_grouped_launch(void* out, const void* x, const int32_t* qweight
                                 const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                                 int numel, int topk, int max_blocks, int E, int K, int N, int group_size, int dtype, hipStream_t st, int id_step, bool glu,
                                 int kper, float* partial);
+int moe_range_sum_launch(void* out, const float* partial, const float* topk_weights, const float* row_scale, int rows, int topk, int N, int ranges,
+                         int dtype, hipStream_t st);
 int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
                               const float* topk_weights, const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                               int numel, int topk, int block_size, int max_blocks, int E, int K, int N, int group_size, int dtype,
@@ -1333,12 +1335,20 @@ static bool w4a16_gates(int block_size, int N, int group_size, int zeros_kind) {
   return (block_size == 16 || block_size == 32 || block_size == 64) && N % 256 == 0 && group_size % 128 == 0 && zeros_kind != MI355Q_ZP_PRESCALED;
 }
 
+// sum: the launch is of the second GEMM, and where its K ranges are added up anyway, so are the topk slots of a token ([rows, N] at sum->out;
+// out is not written then)
+struct MoeSum {
+  void* out;
+  int topk;
+  bool done;
+};
+
 int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales,
                          const float* scales_f32, const float* out_scale,
                          const void* zeros, int zeros_kind, const float* topk_weights,
                          const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                          int numel, int topk, int block_size, int max_blocks, int E, int K, int N,
-                         int group_size, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st, bool glu) {
+                         int group_size, int dtype, void* workspace, size_t workspace_bytes, hipStream_t st, bool glu, MoeSum* sum) {
   const bool small_groups = group_size == 64 || group_size == 32;
   MQ_REQUIRE(group_size % 128 == 0 || (small_groups && !scales_f32 && !out_scale),
              "moe_w4a16: group_size=%d must be 32, 64 or a multiple of 128 (a multiple of 128 with fp32 scales)", group_size);
@@ -1432,6 +1442,10 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   }
   MQ_REQUIRE(e == hipSuccess, "moe_w4a16: cannot reserve LDS: %s", hipGetErrorString(e));
   MQ_LAUNCH_CHECK("moe_w4a16");
+  if (splits > 1 && sum && topk == 1 && topk_weights) {
+    sum->done = true;
+    return moe_range_sum_launch(sum->out, (const float*)workspace, topk_weights, a.row_scale, numel / sum->topk, sum->topk, N, splits, dtype, st);
+  }
   if (splits > 1) {
     // the reduction walks the aligned id list (at most max_blocks * block_size positions, cut at *npp on
     // the device): rows of ids that the alignment dropped have no partial tiles and are not touched
@@ -1478,5 +1492,25 @@ extern "C" int mi355q_moe_w4a16_gate_up(void* out, const void* a, const int32_t*
   MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "moe_w4a16_gate_up: dtype %d", dtype);
   MQ_REQUIRE(K % 128 == 0 && group_size > 0 && K % group_size == 0, "moe_w4a16_gate_up: K=%d group_size=%d", K, group_size);
   return w4a16_grouped_launch(out, a, w, w_scale, nullptr, nullptr, w_zeros, zeros_kind, nullptr, sorted_token_ids, expert_ids, num_tokens_post_pad,
-                              numel, topk, block_size, max_blocks, E, K, N, group_size, dtype, workspace, workspace_bytes, as_stream(stream), true);
+                              numel, topk, block_size, max_blocks, E, K, N, group_size, dtype, workspace, workspace_bytes, as_stream(stream), true, nullptr);
+}
+
+extern "C" int mi355q_moe_w4a16_down_sum(void* out, void* rows_scratch, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros,
+                                         int zeros_kind, int group_size, const float* topk_weights, const int32_t* sorted_token_ids,
+                                         const int32_t* expert_ids, const int32_t* num_tokens_post_pad, int rows, int topk, int block_size,
+                                         int max_blocks, int E, int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace mi355q;
+  MQ_REQUIRE(rows >= 0 && topk > 0 && E > 0 && K > 0 && N > 0, "moe_w4a16_down_sum: bad shape rows=%d topk=%d E=%d K=%d N=%d", rows, topk, E, K, N);
+  if (rows == 0) return 0;
+  MQ_REQUIRE(out && rows_scratch && topk_weights, "moe_w4a16_down_sum: null pointer");
+  MQ_REQUIRE((long)rows * topk < (1L << 31), "moe_w4a16_down_sum: %d rows of %d slots", rows, topk);
+  MQ_REQUIRE(a && w && w_scale && sorted_token_ids && expert_ids && num_tokens_post_pad, "moe_w4a16_down_sum: null pointer");
+  MQ_REQUIRE(block_size >= 16 && block_size % 16 == 0 && K % 128 == 0 && N % 128 == 0, "moe_w4a16_down_sum: block_size=%d K=%d N=%d", block_size, K, N);
+  MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "moe_w4a16_down_sum: dtype %d", dtype);
+  MoeSum sum = {out, topk, false};
+  if (int rc = w4a16_grouped_launch(rows_scratch, a, w, w_scale, nullptr, nullptr, w_zeros, zeros_kind, topk_weights, sorted_token_ids, expert_ids,
+                                    num_tokens_post_pad, rows * topk, 1, block_size, max_blocks, E, K, N, group_size <= 0 ? K : group_size, dtype,
+                                    workspace, workspace_bytes, as_stream(stream), false, &sum))
+    return rc;
+  return sum.done ? 0 : mi355q_moe_sum(out, rows_scratch, rows, topk, N, dtype, dtype, nullptr, stream);
 }
