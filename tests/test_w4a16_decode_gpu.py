@@ -248,3 +248,12 @@ def test_unsorted_sum(E, K, N, rows, topk, ranges, dtype):
     _lib.check(lib.mi355q_moe_sum(want.data_ptr(), slots.data_ptr(), rows, topk, N, code, code, None, st), "moe_sum")
     assert torch.equal(got, want)
     assert lib.mi355q_moe_w4a16_unsorted_sum(got.data_ptr(), x.data_ptr(), *common, rows, topk, E, K, N, code, ws.data_ptr(), need - 4, st) != 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,N,g", [(8320, 2048, 128), (10240, 3072, 1024), (10368, 4096, 128), (12288, 2048, 256), (12416, 3072, 128), (14336, 4096, 128),
+                                   (10240, 4352, 128), (8448, 8192, 256)])
+def test_deep_k(K, N, g, dtype):
+    """Five to seven K blocks of a wavefront, on either side of the depths where it takes them, one and two tiles."""
+    test_rows_1_to_16(K, N, g, dtype)
+    test_exact(K, N, g, dtype)

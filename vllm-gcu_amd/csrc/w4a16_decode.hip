@@ -473,10 +473,16 @@ struct DecodePlan {
 };
 DecodePlan decode_plan(int M, int K, int N) {
   const int G = K / 128, cus = device_cu_count();
-  if (M > 16 || G > (M > 8 ? 32 : 64)) return {0, 0, 0};
+  if (M > 16 || G > (M > 8 ? 32 : 112)) return {0, 0, 0};
   int nt = 1;
   while (nt <= 4 && N / 16 / nt > cus) nt *= 2;
   if (nt > (M > 8 ? 2 : 4) || (nt == 4 && G > 48)) return {0, 0, 0};
+  // Deep K: as many K blocks of a wavefront as its registers hold, where most CUs have a tile.  (us, the streaming kernel with its exchange
+  // between K ranges -> here, fp16, at 1 / 4 rows: 8704 x 4096 8.1 / 8.7 -> 7.1 / 7.2, 14336 x 4096 10.2 / 10.7 -> 9.7 / 9.6, 10240 x 8192
+  // 12.8 / 12.2 -> 11.3 / 11.2, 8704 x 2048 7.0 / 7.5 -> 6.3 / 6.7; at 8 rows 8704 x 4096 8.7 -> 8.3.  Behind: 16384 x 8192 at 1 16.5 / 23, 13824 x 5120 11.1 /
+  // 13.4, both beyond the registers, 14336 x 4096 at 8 10.6 / 11.1, 8704 x 2048 at 8, bf16, 7.4 / 8.0; 14336 x 2048 at 2, bf16, 8.2 / 8.2.)
+  const int wgs = N / 16 / nt;
+  if (G > 64 && (nt == 4 || 2 * wgs < cus || G > (M > 4 || nt == 2 ? 80 : 4 * wgs < 3 * cus ? 96 : 112) || (M > 4 && 4 * wgs < 3 * cus))) return {0, 0, 0};
   const int w = G <= 16 || (G <= 32 && M <= 8 && nt <= 2) ? 8 : 16;
   return {nt, w, (G + w - 1) / w};
 }
@@ -490,6 +496,10 @@ void launch_plan(const DecodePlan& p, const DecodeArgs& a, hipStream_t st) {
     MQ_D(8, 3, 1); MQ_D(8, 4, 1); MQ_D(16, 4, 1);
     MQ_D(8, 3, 2); MQ_D(8, 4, 2); MQ_D(16, 4, 2);
     MQ_D(8, 1, 4); MQ_D(8, 2, 4); MQ_D(16, 2, 4);
+    MQ_D(16, 5, 1); MQ_D(16, 5, 2);
+    if constexpr (NT == 1) {
+      MQ_D(16, 6, 1); MQ_D(16, 7, 1);
+    }
   } else {
     MQ_D(16, 2, 1); MQ_D(16, 2, 2);
   }
