@@ -430,7 +430,7 @@ int mi355q_moe_w4a16_unsorted(void* out, const void* a, const int32_t* w, const 
 /* The second GEMM of a fused-MoE layer over up to 64 unaligned slots (a [rows * topk, K], one row per slot) and the sum of each token's
  * slots, out [rows, N]: what mi355q_moe_w4a16_unsorted with topk_weights and mi355q_moe_sum make one after the other, but for the order
  * of the fp32 additions along K, which is cut into ranges whose f32 sums go through the workspace
- * (mi355q_moe_w4a16_unsorted_sum_bytes). */
+ * (mi355q_moe_w4a16_unsorted_sum_bytes).  Slots of ids outside [0, E) add nothing. */
 size_t mi355q_moe_w4a16_unsorted_sum_bytes(int numel, int E, int K, int N);
 int mi355q_moe_w4a16_unsorted_sum(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
                                   int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64, int rows, int topk,

@@ -250,6 +250,37 @@ def test_unsorted_sum(E, K, N, rows, topk, ranges, dtype):
     assert lib.mi355q_moe_w4a16_unsorted_sum(got.data_ptr(), x.data_ptr(), *common, rows, topk, E, K, N, code, ws.data_ptr(), need - 4, st) != 0
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("E,K,N,rows,topk", [(8, 6144, 4096, 3, 2), (8, 2944, 4096, 3, 2), (5, 384, 256, 64, 1), (60, 384, 256, 10, 6)])
+def test_unsorted_sum_without_slots_of_no_expert(E, K, N, rows, topk, dtype, wide):
+    """Slots of ids outside [0, E) add nothing, whatever the workspace held: the bits of the GEMM into zeroed rows and moe_sum."""
+    from vllm_gcu_amd import _lib
+    print(f"case unsorted sum, dropped slots E={E} K={K} N={N} rows={rows} topk={topk} {dtype} wide={wide}", flush=True)
+    lib, g, numel = _lib.load(), 128, rows * topk
+    code = _lib.F16 if dtype == torch.float16 else _lib.BF16
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // 8, N), dtype=torch.int32, device="cuda", generator=gen)
+    zp = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // g, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    s = (2.0 ** torch.randint(-9, -6, (E, K // g, N), device="cuda", generator=gen)).to(dtype)
+    x = torch.randint(-4, 5, (numel, K), device="cuda", generator=gen).to(dtype)
+    rw = torch.rand(numel, device="cuda", generator=gen)
+    ids = torch.randint(0, E, (rows, topk), device="cuda", generator=gen, dtype=torch.int64 if wide else torch.int32)
+    ids[0, 0], ids[-1, :], ids[1, -1] = E, -1, E + 3
+    rw[0] = float("nan")                                     # (of a slot that adds nothing)
+    st = torch.cuda.current_stream().cuda_stream
+    need = lib.mi355q_moe_w4a16_unsorted_sum_bytes(numel, E, K, N)
+    ws = torch.full((need // 4,), float("nan"), device="cuda")
+    got, want = (torch.full((rows, N), float("nan"), dtype=dtype, device="cuda") for _ in range(2))
+    slots = torch.zeros(numel, N, dtype=dtype, device="cuda")
+    common = (w.data_ptr(), s.data_ptr(), zp.data_ptr(), _lib.ZP_PACKED, g, rw.data_ptr(), ids.data_ptr(), wide)
+    _lib.check(lib.mi355q_moe_w4a16_unsorted_sum(got.data_ptr(), x.data_ptr(), *common, rows, topk, E, K, N, code, ws.data_ptr(), need, st),
+               "moe_w4a16_unsorted_sum")
+    _lib.check(lib.mi355q_moe_w4a16_unsorted(slots.data_ptr(), x.data_ptr(), *common, numel, 1, E, K, N, 0, code, st), "moe_w4a16_unsorted")
+    _lib.check(lib.mi355q_moe_sum(want.data_ptr(), slots.data_ptr(), rows, topk, N, code, code, None, st), "moe_sum")
+    assert torch.equal(got, want) and (got[-1] == 0).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("K,N,g", [(8320, 2048, 128), (10240, 3072, 1024), (10368, 4096, 128), (12288, 2048, 256), (12416, 3072, 128), (14336, 4096, 128),
                                    (10240, 4352, 128), (8448, 8192, 256)])

@@ -582,10 +582,12 @@ int sum_ranges(int numel, int E, int K, int N) {
 // the grouped GEMM and moe_sum round it one after the other.  (Bound by its launch; f32 sums from the GEMM cost nothing next to rounded ones:
 // eight experts of 4096 x 14336 at 16 / 32 tokens, one range, 139 / 146 -> 136 / 142 us for the layer; at 256 / 512, where blocks of 64 slots have
 // K ranges and each had a launch of its own for their sums, 331 / 506 -> 327 / 501.)
-// row_scale: of bf16 rows staged as fp16, or null.
+// row_scale: of bf16 rows staged as fp16, or null.  ids: the slots' experts, id_step words apart, or null: a slot of an id outside [0, E) is in no
+// block, nobody wrote its sums, and it adds nothing.
 template <int DT, int S>
 __global__ void __launch_bounds__(256)
-moe_range_sum_kernel(uint16_t* out, const float* partial, const float* topk_weights, const float* row_scale, uint32_t rows, int T, FastDiv quads) {
+moe_range_sum_kernel(uint16_t* out, const float* partial, const float* topk_weights, const float* row_scale, const int32_t* ids, int id_step, uint32_t E,
+                     uint32_t rows, int T, FastDiv quads) {
   const uint32_t q = blockIdx.x * 256 + threadIdx.x;
   if (q >= rows * quads.d) return;
   const uint32_t m = quads.div(q), n = q - m * quads.d;
@@ -597,6 +599,7 @@ moe_range_sum_kernel(uint16_t* out, const float* partial, const float* topk_weig
 #pragma unroll
     for (int r = 0; r < S; ++r) v[r] = p[r * step];
     const float rw = topk_weights[m * T + t];
+    const bool counts = !ids || (uint32_t)ids[(m * T + t) * id_step] < E;
 #pragma unroll
     for (int r = 1; r < S; ++r) v[0] += v[r];
 #pragma unroll
@@ -604,7 +607,7 @@ moe_range_sum_kernel(uint16_t* out, const float* partial, const float* topk_weig
       float p = v[0][e] * rw;
       if (row_scale) p *= row_scale[m * T + t];
       asm volatile("" : "+v"(p));                      // (a product of its own, as the GEMM's: not one that is rounded to 16 bits at once)
-      acc[e] += Elem<DT>::to_f32(Elem<DT>::from_f32(p));
+      acc[e] += counts ? Elem<DT>::to_f32(Elem<DT>::from_f32(p)) : 0.f;
     }
   }
   u2 o;
@@ -680,12 +683,13 @@ int w4a16_decode_grouped_launch(void* out, const void* x, const int32_t* qweight
 }
 
 // out [rows, N] from f32 sums [ranges][rows * topk][N]; up to six ranges
-int moe_range_sum_launch(void* out, const float* partial, const float* topk_weights, const float* row_scale, int rows, int topk, int N, int ranges,
-                         int dtype, hipStream_t st) {
+int moe_range_sum_launch(void* out, const float* partial, const float* topk_weights, const float* row_scale, const int32_t* ids, int id_step, int E, int rows,
+                         int topk, int N, int ranges, int dtype, hipStream_t st) {
   const FastDiv quads((uint32_t)(N / 4));
   const dim3 grid((unsigned)(((size_t)rows * (N / 4) + 255) / 256));
 #define MQ_S(DT, S) \
-  if (ranges == S) hipLaunchKernelGGL((moe_range_sum_kernel<DT, S>), grid, dim3(256), 0, st, (uint16_t*)out, partial, topk_weights, row_scale, (uint32_t)rows, topk, quads)
+  if (ranges == S) hipLaunchKernelGGL((moe_range_sum_kernel<DT, S>), grid, dim3(256), 0, st, (uint16_t*)out, partial, topk_weights, row_scale, ids, id_step, (uint32_t)E, \
+                                       (uint32_t)rows, topk, quads)
 #define MQ_DT(DT)                                                             \
   do {                                                                        \
     MQ_S(DT, 1); MQ_S(DT, 2); MQ_S(DT, 3); MQ_S(DT, 4); MQ_S(DT, 5); MQ_S(DT, 6); \
@@ -744,5 +748,5 @@ extern "C" int mi355q_moe_w4a16_unsorted_sum(void* out, const void* a, const int
                                              std::min(numel, (numel + E * 15) / 16), E, K, N, group_size, dtype, st, ids_are_int64 ? 2 : 1, false, kper,
                                              (float*)workspace);
   if (rc) return rc;
-  return moe_range_sum_launch(out, (const float*)workspace, topk_weights, nullptr, rows, topk, N, s, dtype, as_stream(stream));
+  return moe_range_sum_launch(out, (const float*)workspace, topk_weights, nullptr, (const int32_t*)topk_ids, ids_are_int64 ? 2 : 1, E, rows, topk, N, s, dtype, st);
 }

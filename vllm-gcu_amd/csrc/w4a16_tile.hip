@@ -1241,8 +1241,8 @@ int w4a16_decode_grouped_launch(void* out, const void* x, const int32_t* qweight
                                 const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                                 int numel, int topk, int max_blocks, int E, int K, int N, int group_size, int dtype, hipStream_t st, int id_step, bool glu,
                                 int kper, float* partial);
-int moe_range_sum_launch(void* out, const float* partial, const float* topk_weights, const float* row_scale, int rows, int topk, int N, int ranges,
-                         int dtype, hipStream_t st);
+int moe_range_sum_launch(void* out, const float* partial, const float* topk_weights, const float* row_scale, const int32_t* ids, int id_step, int E, int rows,
+                         int topk, int N, int ranges, int dtype, hipStream_t st);
 int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
                               const float* topk_weights, const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                               int numel, int topk, int block_size, int max_blocks, int E, int K, int N, int group_size, int dtype,
@@ -1444,7 +1444,7 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   MQ_LAUNCH_CHECK("moe_w4a16");
   if (splits > 1 && sum && topk == 1 && topk_weights) {
     sum->done = true;
-    return moe_range_sum_launch(sum->out, (const float*)workspace, topk_weights, a.row_scale, numel / sum->topk, sum->topk, N, splits, dtype, st);
+    return moe_range_sum_launch(sum->out, (const float*)workspace, topk_weights, a.row_scale, nullptr, 1, E, numel / sum->topk, sum->topk, N, splits, dtype, st);
   }
   if (splits > 1) {
     // the reduction walks the aligned id list (at most max_blocks * block_size positions, cut at *npp on
