@@ -414,12 +414,18 @@ int mi355q_moe_w4a16_gate_up(void* out, const void* a, const int32_t* w, const v
                              const int32_t* sorted_token_ids, const int32_t* expert_ids, const int32_t* num_tokens_post_pad, int numel, int topk,
                              int block_size, int max_blocks, int E, int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 /* mi355q_moe_gemm with quant_mode 0 on a [rows * topk, K] with the routing weights, into rows_scratch [rows * topk, N], and mi355q_moe_sum of
- * it into out [rows, N], bit for bit; where the GEMM cuts K into ranges, their sums are added in one launch with the token's (and
- * rows_scratch is not written).  Same workspace. */
+ * it into out [rows, N], bit for bit; rows of slots that no block holds are added as the caller left them.  Same workspace. */
 int mi355q_moe_w4a16_down_sum(void* out, void* rows_scratch, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
                               int group_size, const float* topk_weights, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                               const int32_t* num_tokens_post_pad, int rows, int topk, int block_size, int max_blocks, int E, int K, int N, int dtype,
                               void* workspace, size_t workspace_bytes, void* stream);
+/* The same for an alignment without expert map and valid count, with the ids [rows * topk] that were aligned: slots of ids outside [0, E) add
+ * nothing, the others give the same bits.  Where the GEMM cuts K into ranges, their sums are added in one launch with the token's (and
+ * rows_scratch is not written).  Same workspace. */
+int mi355q_moe_w4a16_down_sum_ids(void* out, void* rows_scratch, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
+                                  int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64, const int32_t* sorted_token_ids,
+                                  const int32_t* expert_ids, const int32_t* num_tokens_post_pad, int rows, int topk, int block_size, int max_blocks, int E,
+                                  int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream);
 /* mi355q_moe_gemm with quant_mode 0 for up to 64 slots (numel) that are not aligned: topk_ids [numel] are the experts of the slots, a
  * launch of mi355q_moe_align_block_size less.  Groups that are multiples of 128; act and output dtype are one.  Slots of ids outside
  * [0, E) are not written.  Bit for bit the result of mi355q_moe_gemm on blocks of 16.  silu_and_mul: the columns are gate and up, out is

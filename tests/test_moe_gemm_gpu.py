@@ -1029,11 +1029,59 @@ def test_w4a16_down_sum(fmoe, block, E, K, N, rows, ranges, dtype):
     need = lib.mi355q_moe_gemm_workspace_bytes(0, numel, block, ex.numel(), E, K, N)
     ws = torch.full((need // 4 + 1,), float("nan"), device="cuda")
     rows_out, out, want = (torch.full((n, N), float("nan"), dtype=dtype, device="cuda") for n in (numel, numel // topk, numel // topk))
-    _lib.check(lib.mi355q_moe_w4a16_down_sum(out.data_ptr(), rows_out.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(),
-                                             _lib.ZP_PACKED, g, rw.data_ptr(), so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel // topk, topk, block,
-                                             ex.numel(), E, K, N, code, ws.data_ptr(), need, st), "moe_w4a16_down_sum")
+    _lib.check(lib.mi355q_moe_w4a16_down_sum_ids(out.data_ptr(), rows_out.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(),
+                                                 _lib.ZP_PACKED, g, rw.data_ptr(), ids.data_ptr(), 0, so.data_ptr(), ex.data_ptr(), npp.data_ptr(),
+                                                 numel // topk, topk, block, ex.numel(), E, K, N, code, ws.data_ptr(), need, st),
+               "moe_w4a16_down_sum_ids")
     _lib.check(lib.mi355q_moe_gemm(rows_out.data_ptr(), x.data_ptr(), w.data_ptr(), None, s.data_ptr(), z.data_ptr(), _lib.ZP_PACKED, 0, g, rw.data_ptr(),
                                    so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, 1, block, ex.numel(), E, K, N, code, code, 0, ws.data_ptr(), need,
                                    st), "moe_gemm")
     _lib.check(lib.mi355q_moe_sum(want.data_ptr(), rows_out.data_ptr(), numel // topk, topk, N, code, code, None, st), "moe_sum")
     assert torch.equal(out, want) and not out.isnan().any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block,E,K,N,rows,topk", [(64, 4, 4096, 256, 74, 2), (64, 8, 7168, 1024, 100, 2), (64, 8, 14336, 4096, 128, 2), (64, 16, 4096, 3072, 128, 2),
+                                                   (64, 3, 4096, 512, 100, 3), (32, 8, 1408, 2048, 18, 2), (16, 8, 1408, 2048, 10, 2)])
+def test_w4a16_down_sum_of_slots_in_no_block(fmoe, block, E, K, N, rows, topk, dtype):
+    """Slots of ids outside [0, E), which no block holds, with and without K ranges, whatever the workspace held: rows that moe_gemm leaves as they are
+    and moe_sum adds, or, given the ids, nothing."""
+    from vllm_gcu_amd import _lib
+    print(f"case down and sum, dropped slots block={block} E={E} K={K} N={N} rows={rows} {dtype}", flush=True)
+    lib, code, st, g = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream, 128
+    tokens = E * rows // topk
+    numel = tokens * topk
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w, z = (torch.randint(-2 ** 31, 2 ** 31 - 1, (E, r, c), dtype=torch.int32, device="cuda", generator=gen) for r, c in ((K // 8, N), (K // g, N // 8)))
+    s = (torch.rand(E, K // g, N, device="cuda", generator=gen) * 0.01 + 0.001).to(dtype)
+    x, rw = torch.randn(numel, K, device="cuda", generator=gen).to(dtype), torch.rand(numel, device="cuda", generator=gen)
+    ids = torch.randint(0, E, (tokens, topk), device="cuda", generator=gen, dtype=torch.int32)
+    ids[0, 0], ids[3, -1], ids[-1, :] = -1, E, E + 7
+    so, ex, npp = fmoe.moe_align_block_size(ids, block, E)
+    need = lib.mi355q_moe_gemm_workspace_bytes(0, numel, block, ex.numel(), E, K, N)
+    ws = torch.full((need // 4 + 1,), float("nan"), device="cuda")
+    scratch = torch.randn(numel, N, device="cuda", generator=gen).to(dtype)
+    tail = (w.data_ptr(), s.data_ptr(), z.data_ptr(), _lib.ZP_PACKED, g, rw.data_ptr(), so.data_ptr(), ex.data_ptr(), npp.data_ptr())
+    out, want = (torch.full((tokens, N), float("nan"), dtype=dtype, device="cuda") for _ in range(2))
+    rows_out = scratch.clone()
+    _lib.check(lib.mi355q_moe_gemm(rows_out.data_ptr(), x.data_ptr(), w.data_ptr(), None, s.data_ptr(), z.data_ptr(), _lib.ZP_PACKED, 0, g, rw.data_ptr(),
+                                   so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, 1, block, ex.numel(), E, K, N, code, code, 0, ws.data_ptr(), need,
+                                   st), "moe_gemm")
+    dropped = ((ids < 0) | (ids >= E)).view(-1)
+    assert torch.equal(rows_out[dropped], scratch[dropped])
+    _lib.check(lib.mi355q_moe_sum(want.data_ptr(), rows_out.data_ptr(), tokens, topk, N, code, code, None, st), "moe_sum")
+    ws.fill_(float("nan"))
+    _lib.check(lib.mi355q_moe_w4a16_down_sum(out.data_ptr(), scratch.data_ptr(), x.data_ptr(), *tail, tokens, topk, block, ex.numel(), E, K, N, code,
+                                             ws.data_ptr(), need, st), "moe_w4a16_down_sum")
+    assert torch.equal(out, want)
+    want.fill_(float("nan"))
+    rows_out[dropped] = 0
+    _lib.check(lib.mi355q_moe_sum(want.data_ptr(), rows_out.data_ptr(), tokens, topk, N, code, code, None, st), "moe_sum")
+    for of in (ids, ids.long()):
+        ws.fill_(float("nan"))
+        scratch.fill_(float("nan"))
+        out.fill_(float("nan"))
+        _lib.check(lib.mi355q_moe_w4a16_down_sum_ids(out.data_ptr(), scratch.data_ptr(), x.data_ptr(), *tail[:6], of.data_ptr(), of.dtype == torch.int64,
+                                                     *tail[6:], tokens, topk, block, ex.numel(), E, K, N, code, ws.data_ptr(), need, st),
+                   "moe_w4a16_down_sum_ids")
+        assert torch.equal(out, want) and (out[-1] == 0).all()

@@ -248,19 +248,35 @@ static_fp8_quant_kernel(uint8_t* out, const uint16_t* x, const float* scale, lon
 }
 
 // ---- moe_sum: out[m, :] = sum_t in[m, t, :] in fp32 --------------------------
-template <int DT_IN, int DT_OUT>
+// IDS: without the slots whose id, id_step words apart, is outside [0, E).  Two slots are on their way at a time there: the ids are one more line
+// to wait for, 0.4 us of a layer of 68 where a slot's row and id were waited for before the next one's.
+template <int DT_IN, int DT_OUT, bool IDS>
 __global__ void __launch_bounds__(256)
-moe_sum_kernel(void* out, const uint16_t* in, uint32_t rows, int T, int K, FastDiv chunks, const int* valid_rows, long row0) {
+moe_sum_kernel(void* out, const uint16_t* in, uint32_t rows, int T, int K, FastDiv chunks, const int* valid_rows, long row0, const int32_t* ids, int id_step,
+               uint32_t E) {
   const uint32_t total = live_rows(rows, valid_rows, 1, row0) * chunks.d;
   for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
     const long r = chunks.div(i);
     const int c = (int)(i - (uint32_t)r * chunks.d);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int t = 0; t < T; ++t) {
-      float v[8];
-      unpack8<DT_IN>(*(const u4*)(in + (r * T + t) * K + 8 * c), v);
+    constexpr int U = IDS ? 2 : 1;
+    for (int t = 0; t < T; t += U) {
+      u4 x[U];
+      int id[U];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] += v[e];
+      for (int u = 0; u < U; ++u) {
+        const long slot = r * T + min(t + u, T - 1);
+        x[u] = *(const u4*)(in + slot * K + 8 * c);
+        if (IDS) id[u] = ids[slot * id_step];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float v[8];
+        unpack8<DT_IN>(x[u], v);
+        const uint32_t keep = !IDS ? 0xffffffffu : t + u < T ? slot_mask(id[u], E) : 0u;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += bitcast<float>(bitcast<uint32_t>(v[e]) & keep);
+      }
     }
     if (DT_OUT == MI355Q_F32) {
       float* o = (float*)out + r * K + 8 * c;
@@ -487,6 +503,40 @@ inline unsigned grid_for(long items) {
 }
 
 }  // namespace
+
+// ids null: every slot counts
+int moe_sum_launch(void* out, const void* in, long rows, int topk, int K, int in_dtype, int out_dtype, const int32_t* valid_rows, const int32_t* ids,
+                   int id_step, int E, hipStream_t st) {
+  MQ_REQUIRE(rows >= 0 && topk > 0 && K > 0 && K % 8 == 0, "moe_sum: bad shape rows=%ld topk=%d K=%d (K %% 8 == 0)", rows, topk, K);
+  if (rows == 0) return 0;
+  MQ_REQUIRE(out && in, "moe_sum: null pointer");
+  MQ_REQUIRE(in_dtype == MI355Q_F16 || in_dtype == MI355Q_BF16, "moe_sum: input dtype %d must be f16 or bf16", in_dtype);
+  MQ_REQUIRE(out_dtype == in_dtype || out_dtype == MI355Q_F32, "moe_sum: output dtype %d must equal the input's or be f32", out_dtype);
+  MQ_REQUIRE(!ids || out_dtype == in_dtype, "moe_sum: with ids the output dtype %d must equal the input's", out_dtype);
+  const FastDiv chunks((uint32_t)(K / 8));
+  for (long r0 = 0; r0 < rows; r0 += rows_per_launch(K / 8)) {
+    const uint32_t n = (uint32_t)std::min(rows - r0, rows_per_launch(K / 8));
+    const unsigned g = grid_for((long)n * (K / 8));
+    const uint16_t* p = (const uint16_t*)in + r0 * topk * K;
+    void* o = (char*)out + r0 * K * (out_dtype == MI355Q_F32 ? 4 : 2);
+    const int32_t* const id = ids ? ids + r0 * topk * id_step : nullptr;
+#define MQ_SUM(IN, OUT, IDS) \
+  hipLaunchKernelGGL((moe_sum_kernel<IN, OUT, IDS>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0, id, id_step, (uint32_t)E)
+    if (in_dtype == MI355Q_F16) {
+      if (ids) MQ_SUM(MI355Q_F16, MI355Q_F16, true);
+      else if (out_dtype == MI355Q_F16) MQ_SUM(MI355Q_F16, MI355Q_F16, false);
+      else MQ_SUM(MI355Q_F16, MI355Q_F32, false);
+    } else {
+      if (ids) MQ_SUM(MI355Q_BF16, MI355Q_BF16, true);
+      else if (out_dtype == MI355Q_BF16) MQ_SUM(MI355Q_BF16, MI355Q_BF16, false);
+      else MQ_SUM(MI355Q_BF16, MI355Q_F32, false);
+    }
+#undef MQ_SUM
+  }
+  MQ_LAUNCH_CHECK("moe_sum");
+  return 0;
+}
+
 }  // namespace mi355q
 
 using namespace mi355q;
@@ -602,29 +652,7 @@ extern "C" int mi355q_fp8_static_quant(uint8_t* out, const void* x, const float*
 
 extern "C" int mi355q_moe_sum(void* out, const void* in, long rows, int topk, int K, int in_dtype,
                               int out_dtype, const int32_t* valid_rows, void* stream) {
-  MQ_REQUIRE(rows >= 0 && topk > 0 && K > 0 && K % 8 == 0, "moe_sum: bad shape rows=%ld topk=%d K=%d (K %% 8 == 0)", rows, topk, K);
-  if (rows == 0) return 0;
-  MQ_REQUIRE(out && in, "moe_sum: null pointer");
-  MQ_REQUIRE(in_dtype == MI355Q_F16 || in_dtype == MI355Q_BF16, "moe_sum: input dtype %d must be f16 or bf16", in_dtype);
-  MQ_REQUIRE(out_dtype == in_dtype || out_dtype == MI355Q_F32, "moe_sum: output dtype %d must equal the input's or be f32", out_dtype);
-  hipStream_t st = as_stream(stream);
-  const FastDiv chunks((uint32_t)(K / 8));
-  for (long r0 = 0; r0 < rows; r0 += rows_per_launch(K / 8)) {
-    const uint32_t n = (uint32_t)std::min(rows - r0, rows_per_launch(K / 8));
-    const unsigned g = grid_for((long)n * (K / 8));
-    const uint16_t* p = (const uint16_t*)in + r0 * topk * K;
-    void* o = (char*)out + r0 * K * (out_dtype == MI355Q_F32 ? 4 : 2);
-    if (in_dtype == MI355Q_F16 && out_dtype == MI355Q_F16)
-      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F16>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0);
-    else if (in_dtype == MI355Q_F16)
-      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_F16, MI355Q_F32>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0);
-    else if (out_dtype == MI355Q_BF16)
-      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_BF16>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0);
-    else
-      hipLaunchKernelGGL((moe_sum_kernel<MI355Q_BF16, MI355Q_F32>), dim3(g), dim3(256), 0, st, o, p, n, topk, K, chunks, valid_rows, r0);
-  }
-  MQ_LAUNCH_CHECK("moe_sum");
-  return 0;
+  return moe_sum_launch(out, in, rows, topk, K, in_dtype, out_dtype, valid_rows, nullptr, 1, 0, as_stream(stream));
 }
 
 // ---- fp8-e4m3fn -> f16 / bf16, exact (every e4m3fn value is representable in both) ----

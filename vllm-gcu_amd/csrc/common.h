@@ -257,6 +257,12 @@ __device__ __forceinline__ uint32_t silu_mul16x2(uint32_t gate, uint32_t up) {
   return (uint32_t)silu_mul16<DT>((uint16_t)gate, (uint16_t)up) | ((uint32_t)silu_mul16<DT>((uint16_t)(gate >> 16), (uint16_t)(up >> 16)) << 16);
 }
 
+// all ones for a slot of one of the E experts, zero for one that no block holds (no comparison: behind a branch the slot's sums would be asked for
+// only when its id has arrived)
+__device__ __forceinline__ uint32_t slot_mask(int32_t id, int32_t E) {
+  return (uint32_t)((id - E) & ~id) >> 31 ? 0xffffffffu : 0u;
+}
+
 constexpr float FP8_MAX = 448.0f;
 template <int DT>
 __device__ __forceinline__ float round_act(float f) {

@@ -688,10 +688,10 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
                                           ids.data_ptr(), ids64, M, T, E, I, K, code, b + o_sums, sums, stream),
             "moe_w4a16_unsorted_sum");
     } else if (mode == kW4) {
-      check(mi355q_moe_w4a16_down_sum(out.data_ptr(), b + o_c1, b + o_c2, static_cast<const int32_t*>(w2.data_ptr()), s2p->data_ptr(), ptr(z2),
-                                      z2.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, group, static_cast<const float*>(tw.data_ptr()), sorted, eid,
-                                      npp, M, T, block, blocks, E, I, K, code, ws.p, ws.bytes, stream),
-            "moe_w4a16_down_sum");
+      check(mi355q_moe_w4a16_down_sum_ids(out.data_ptr(), b + o_c1, b + o_c2, static_cast<const int32_t*>(w2.data_ptr()), s2p->data_ptr(), ptr(z2),
+                                          z2.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, group, static_cast<const float*>(tw.data_ptr()),
+                                          ids.data_ptr(), ids64, sorted, eid, npp, M, T, block, blocks, E, I, K, code, ws.p, ws.bytes, stream),
+            "moe_w4a16_down_sum_ids");
     } else {
       check(mi355q_moe_gemm(b + o_c1, b + o_q2, w2.data_ptr(), s2, s2p->data_ptr(), nullptr, MI355Q_ZP_NONE, mode, group, static_cast<const float*>(tw.data_ptr()), sorted,
                            eid, npp, numel, 1, block, blocks, E, I, K, act, code, quant, ws.p, ws.bytes, stream),

@@ -582,8 +582,8 @@ int sum_ranges(int numel, int E, int K, int N) {
 // the grouped GEMM and moe_sum round it one after the other.  (Bound by its launch; f32 sums from the GEMM cost nothing next to rounded ones:
 // eight experts of 4096 x 14336 at 16 / 32 tokens, one range, 139 / 146 -> 136 / 142 us for the layer; at 256 / 512, where blocks of 64 slots have
 // K ranges and each had a launch of its own for their sums, 331 / 506 -> 327 / 501.)
-// row_scale: of bf16 rows staged as fp16, or null.  ids: the slots' experts, id_step words apart, or null: a slot of an id outside [0, E) is in no
-// block, nobody wrote its sums, and it adds nothing.
+// row_scale: of bf16 rows staged as fp16, or null.  ids: the slots' experts, id_step words apart: a slot of an id outside [0, E) is in no block,
+// nobody wrote its sums, and it adds nothing.
 template <int DT, int S>
 __global__ void __launch_bounds__(256)
 moe_range_sum_kernel(uint16_t* out, const float* partial, const float* topk_weights, const float* row_scale, const int32_t* ids, int id_step, uint32_t E,
@@ -593,21 +593,32 @@ moe_range_sum_kernel(uint16_t* out, const float* partial, const float* topk_weig
   const uint32_t m = quads.div(q), n = q - m * quads.d;
   const size_t step = (size_t)rows * T * quads.d;
   f4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int t = 0; t < T; ++t) {
-    const f4* const p = (const f4*)partial + ((size_t)m * T + t) * quads.d + n;
-    f4 v[S];
+  for (int t = 0; t < T; t += 2) {                     // two slots on their way at a time
+    f4 v[2][S];
+    float rw[2], rs[2];
+    uint32_t keep[2];
 #pragma unroll
-    for (int r = 0; r < S; ++r) v[r] = p[r * step];
-    const float rw = topk_weights[m * T + t];
-    const bool counts = !ids || (uint32_t)ids[(m * T + t) * id_step] < E;
+    for (int u = 0; u < 2; ++u) {
+      const uint32_t slot = m * T + min(t + u, T - 1);
+      const f4* const p = (const f4*)partial + (size_t)slot * quads.d + n;
 #pragma unroll
-    for (int r = 1; r < S; ++r) v[0] += v[r];
+      for (int r = 0; r < S; ++r) v[u][r] = p[r * step];
+      rw[u] = topk_weights[slot];
+      rs[u] = row_scale ? row_scale[slot] : 1.f;
+      const uint32_t mask = slot_mask(ids[slot * id_step], E);
+      keep[u] = t + u < T ? mask : 0u;
+    }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float p = v[0][e] * rw;
-      if (row_scale) p *= row_scale[m * T + t];
-      asm volatile("" : "+v"(p));                      // (a product of its own, as the GEMM's: not one that is rounded to 16 bits at once)
-      acc[e] += counts ? Elem<DT>::to_f32(Elem<DT>::from_f32(p)) : 0.f;
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int r = 1; r < S; ++r) v[u][0] += v[u][r];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float p = v[u][0][e] * rw[u];
+        if (row_scale) p *= rs[u];
+        asm volatile("" : "+v"(p));                    // (a product of its own, as the GEMM's: not one that is rounded to 16 bits at once)
+        acc[e] += bitcast<float>(bitcast<uint32_t>(Elem<DT>::to_f32(Elem<DT>::from_f32(p))) & keep[u]);
+      }
     }
   }
   u2 o;

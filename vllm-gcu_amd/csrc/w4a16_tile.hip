@@ -1243,6 +1243,8 @@ int w4a16_decode_grouped_launch(void* out, const void* x, const int32_t* qweight
                                 int kper, float* partial);
 int moe_range_sum_launch(void* out, const float* partial, const float* topk_weights, const float* row_scale, const int32_t* ids, int id_step, int E, int rows,
                          int topk, int N, int ranges, int dtype, hipStream_t st);
+int moe_sum_launch(void* out, const void* in, long rows, int topk, int K, int in_dtype, int out_dtype, const int32_t* valid_rows, const int32_t* ids,
+                   int id_step, int E, hipStream_t st);
 int w4a16_rows_grouped_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
                               const float* topk_weights, const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp,
                               int numel, int topk, int block_size, int max_blocks, int E, int K, int N, int group_size, int dtype,
@@ -1336,10 +1338,12 @@ static bool w4a16_gates(int block_size, int N, int group_size, int zeros_kind) {
 }
 
 // sum: the launch is of the second GEMM, and where its K ranges are added up anyway, so are the topk slots of a token ([rows, N] at sum->out;
-// out is not written then)
+// out is not written then).  ids: the slots' experts, id_step words apart: a slot of an id outside [0, E) is in no block and adds nothing.
 struct MoeSum {
   void* out;
   int topk;
+  const int32_t* ids;
+  int id_step;
   bool done;
 };
 
@@ -1444,7 +1448,7 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   MQ_LAUNCH_CHECK("moe_w4a16");
   if (splits > 1 && sum && topk == 1 && topk_weights) {
     sum->done = true;
-    return moe_range_sum_launch(sum->out, (const float*)workspace, topk_weights, a.row_scale, nullptr, 1, E, numel / sum->topk, sum->topk, N, splits, dtype, st);
+    return moe_range_sum_launch(sum->out, (const float*)workspace, topk_weights, a.row_scale, sum->ids, sum->id_step, E, numel / sum->topk, sum->topk, N, splits, dtype, st);
   }
   if (splits > 1) {
     // the reduction walks the aligned id list (at most max_blocks * block_size positions, cut at *npp on
@@ -1500,17 +1504,34 @@ extern "C" int mi355q_moe_w4a16_down_sum(void* out, void* rows_scratch, const vo
                                          const int32_t* expert_ids, const int32_t* num_tokens_post_pad, int rows, int topk, int block_size,
                                          int max_blocks, int E, int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream) {
   using namespace mi355q;
+  MQ_REQUIRE(rows >= 0 && topk > 0 && (long)rows * topk < (1L << 31), "moe_w4a16_down_sum: %d rows of %d slots", rows, topk);
+  if (rows == 0) return 0;
+  MQ_REQUIRE(out && topk_weights, "moe_w4a16_down_sum: null pointer");
+  MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "moe_w4a16_down_sum: dtype %d", dtype);
+  // (which rows the GEMM leaves alone only the ids tell: the two calls)
+  if (int rc = mi355q_moe_gemm(rows_scratch, a, w, nullptr, w_scale, w_zeros, zeros_kind, 0, group_size, topk_weights, sorted_token_ids, expert_ids,
+                               num_tokens_post_pad, rows * topk, 1, block_size, max_blocks, E, K, N, dtype, dtype, 0, workspace, workspace_bytes, stream))
+    return rc;
+  return mi355q_moe_sum(out, rows_scratch, rows, topk, N, dtype, dtype, nullptr, stream);
+}
+
+extern "C" int mi355q_moe_w4a16_down_sum_ids(void* out, void* rows_scratch, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros,
+                                             int zeros_kind, int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64,
+                                             const int32_t* sorted_token_ids, const int32_t* expert_ids, const int32_t* num_tokens_post_pad, int rows,
+                                             int topk, int block_size, int max_blocks, int E, int K, int N, int dtype, void* workspace,
+                                             size_t workspace_bytes, void* stream) {
+  using namespace mi355q;
   MQ_REQUIRE(rows >= 0 && topk > 0 && E > 0 && K > 0 && N > 0, "moe_w4a16_down_sum: bad shape rows=%d topk=%d E=%d K=%d N=%d", rows, topk, E, K, N);
   if (rows == 0) return 0;
-  MQ_REQUIRE(out && rows_scratch && topk_weights, "moe_w4a16_down_sum: null pointer");
+  MQ_REQUIRE(out && rows_scratch && topk_weights && topk_ids, "moe_w4a16_down_sum: null pointer");
   MQ_REQUIRE((long)rows * topk < (1L << 31), "moe_w4a16_down_sum: %d rows of %d slots", rows, topk);
   MQ_REQUIRE(a && w && w_scale && sorted_token_ids && expert_ids && num_tokens_post_pad, "moe_w4a16_down_sum: null pointer");
   MQ_REQUIRE(block_size >= 16 && block_size % 16 == 0 && K % 128 == 0 && N % 128 == 0, "moe_w4a16_down_sum: block_size=%d K=%d N=%d", block_size, K, N);
   MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "moe_w4a16_down_sum: dtype %d", dtype);
-  MoeSum sum = {out, topk, false};
+  MoeSum sum = {out, topk, (const int32_t*)topk_ids, ids_are_int64 ? 2 : 1, false};
   if (int rc = w4a16_grouped_launch(rows_scratch, a, w, w_scale, nullptr, nullptr, w_zeros, zeros_kind, topk_weights, sorted_token_ids, expert_ids,
                                     num_tokens_post_pad, rows * topk, 1, block_size, max_blocks, E, K, N, group_size <= 0 ? K : group_size, dtype,
                                     workspace, workspace_bytes, as_stream(stream), false, &sum))
     return rc;
-  return sum.done ? 0 : mi355q_moe_sum(out, rows_scratch, rows, topk, N, dtype, dtype, nullptr, stream);
+  return sum.done ? 0 : moe_sum_launch(out, rows_scratch, rows, topk, N, dtype, dtype, nullptr, sum.ids, sum.id_step, E, as_stream(stream));
 }
