@@ -23,6 +23,11 @@ extern "C" {
 
 /* element types of activations / outputs */
 enum { MI355Q_F16 = 0, MI355Q_BF16 = 1, MI355Q_F32 = 2 };
+/* OR-ed into the out_dtype of mi355q_fp8_block_gemm_ws, mi355q_fp8_scaled_gemm_ws and mi355q_w8a8_int8_gemm_ws: the first 64 KiB of the workspace
+ * are zero (zero-filled once, as for mi355q_w4a16_gemm).  Small tiles with few K ranges are then added in the first launch, by arrival
+ * counters there that are zero again after every call.  Without it the first MiB of the workspace is neither read nor written and a second
+ * launch adds the ranges. */
+enum { MI355Q_ZEROED_COUNTERS = 0x100 };
 
 /* how zero-points are handed to the W4A16 kernels */
 enum {
@@ -169,10 +174,9 @@ int mi355q_fp8_scaled_gemm(void* out, const void* x, const void* w, const float*
  * only where the split launch is ahead of the weight-streaming kernel) K is cut into ranges of
  * whole K blocks that run side by side, and a second launch adds their fp32 sums in range order and
  * applies bias (and, for the scaled GEMM, the scales): run-to-run identical, and equal to the unsplit
- * launch up to the order of the fp32 additions.  (Small tiles with few ranges add them in the first launch, by arrival counters
- * in the first 64 KiB of the workspace.)  The workspace follows the rules of
- * mi355q_w4a16_gemm's: zero-filled once, and its first MiB is as it was after every call; without one, or with a smaller one, the unsplit
- * launch (or, for the scaled GEMM on few tiles, the streaming kernel) runs.
+ * launch up to the order of the fp32 additions.  The workspace follows the rules of
+ * mi355q_w4a16_gemm's, but its first MiB is left alone (with MI355Q_ZEROED_COUNTERS: as it was after every call); without one, or with a
+ * smaller one, the unsplit launch (or, for the scaled GEMM on few tiles, the streaming kernel) runs.
  * mi355q_fp8_block_gemm_ws also uses ceil16(M) * (K / 128) * 4 bytes behind the partial sums (behind the first
  * MiB where nothing is split), when the workspace has them, from 24 K blocks of 128 on where K blocks x output
  * tiles of 256 x 128 are 11000 or more, and up to 256 rows from 40 K blocks per range on with 80 tiles or more: the activation scales re-ordered K block major by a small launch of its own, so that a workgroup's
@@ -224,8 +228,8 @@ int mi355q_w8a8_int8_gemm(void* out, int32_t* acc_out, const int8_t* x, const in
  * workspace (0 = this shape is not split) K is cut into ranges that run side by side, and a second
  * launch adds their int32 sums and applies the scales and the bias: integer sums, so the result --
  * acc_out included -- is bit for bit that of the call without workspace.  The workspace follows the
- * rules of mi355q_w4a16_gemm's (zero-filled once; its first MiB, where small tiles count the ranges that have arrived, is as it was after
- * every call, so one buffer serves both); without one, or with a smaller one, the unsplit launch runs. */
+ * rules of mi355q_w4a16_gemm's (its first MiB is left alone, with MI355Q_ZEROED_COUNTERS it is as it was after every call, so one buffer
+ * serves both); without one, or with a smaller one, the unsplit launch runs. */
 size_t mi355q_w8a8_int8_workspace_bytes(int M, int N, int K);
 /* No counterpart in the reference.  What mi355q_w8a8_int8_gemm_ws launches for dense operands, no raw accumulators and a workspace of that size
  * (or of mi355q_q8_mid_plan's): 0 = the kernel for a few dozen to some hundred rows (kslab weights), 1 = tiles of 128 .. 256 rows x 128

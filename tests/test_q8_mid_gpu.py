@@ -186,3 +186,42 @@ def test_k_ranges_leave_the_counters_at_zero(kind, M, N, K, plan):
             _lib.call("mi355q_fp8_block_gemm_ws", out.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), sc.data_ptr(), None, M, N, K, K, 0, N,
                       _lib.BF16, ws.data_ptr(), need, st)
         assert torch.equal(out, want) and not ws[:1 << 20].any()
+
+
+@pytest.mark.parametrize("zeroed", [True, False])
+@pytest.mark.parametrize("kind,M,N,K,plan", RANGES)
+def test_k_ranges_leave_the_first_mib_as_it_was(kind, M, N, K, plan, zeroed):
+    """Products and sums that are exact, twice, over a workspace that nobody cleared but for, where the call says so, the counters: the output to
+    the bit, the counters at zero, and without them the first MiB neither read nor written."""
+    from vllm_gcu_amd import _lib
+    assert plan is None or tile(kind, M, N, K) == plan
+    need = rt.host.q8_mid_plan(kind, M, N, K)
+    print(f"case q8 ranges kind={kind} M={M} N={N} K={K} workspace={need} zeroed={zeroed}", flush=True)
+    assert need > 1 << 20
+    torch.manual_seed(M + N + K)
+    ws = torch.randint(0, 256, (need,), dtype=torch.uint8, device="cuda")
+    ws[1 << 20:] = 0xff
+    if zeroed:
+        ws[:1 << 16] = 0
+    before, code = ws[:1 << 20].clone(), _lib.BF16 | (_lib.ZEROED_COUNTERS if zeroed else 0)
+    x, w = (torch.randint(-3, 4, (r, K), device="cuda").to(torch.int8 if kind == INT8 else torch.float8_e4m3fn) for r in (M, N))
+    wk, st = rearrange.to_kslab(w), torch.cuda.current_stream().cuda_stream
+    xs = 2.0 ** torch.randint(-2, 3, (M, K // 128) if kind == BLOCK else (M, 1), device="cuda").float()
+    sc = 2.0 ** torch.randint(-2, 3, (N // 128, K // 128) if kind == BLOCK else (N, 1), device="cuda").float()
+    if kind == BLOCK:
+        xd, wd = x.double() * xs.double().repeat_interleave(128, 1), w.double() * sc.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    else:
+        xd, wd = x.double() * xs.double(), w.double() * sc.double()
+    want = (xd @ wd.t()).bfloat16()
+    for _ in range(2):
+        out = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+        if kind == INT8:
+            _lib.call("mi355q_w8a8_int8_gemm_ws", out.data_ptr(), None, x.data_ptr(), wk.data_ptr(), xs.data_ptr(), 1, sc.data_ptr(), 1, None, 0,
+                      M, N, K, K, 0, N, code, ws.data_ptr(), need, st)
+        elif kind == SCALED:
+            _lib.call("mi355q_fp8_scaled_gemm_ws", out.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), 1, sc.data_ptr(), 1, None, M, N, K,
+                      K, 0, N, code, ws.data_ptr(), need, st)
+        else:
+            _lib.call("mi355q_fp8_block_gemm_ws", out.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), sc.data_ptr(), None, M, N, K, K, 0, N,
+                      code, ws.data_ptr(), need, st)
+        assert torch.equal(out, want) and torch.equal(ws[:1 << 20], before)

@@ -11,6 +11,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmi355q.so")
 
 F16, BF16, F32 = 0, 1, 2
+ZEROED_COUNTERS = 0x100
 ZP_NONE, ZP_PACKED, ZP_PRESCALED = 0, 1, 2
 W4_SRC_GPTQ, W4_SRC_AWQ, W4_SRC_REF_KN, W4_SRC_REF_NK, W4_SRC_REF_KN_G64S = 0, 1, 2, 3, 4
 Q_W4A16, Q_FP8_BLOCK, Q_INT8, Q_NONE, Q_W8A16, Q_W4_F32SCALE = 0, 1, 2, 3, 4, 5

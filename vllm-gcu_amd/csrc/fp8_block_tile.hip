@@ -37,7 +37,7 @@ int kcontig_fp8_pc_launch(void* out, const void* a, const void* w, const float* 
 bool q8_mid_wanted(int mode, int M, int N, int K, long ldx, size_t* bytes);
 int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
                   int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* workspace,
-                  hipStream_t st);
+                  bool zeroed, hipStream_t st);
 namespace {
 
 constexpr int FTM = 256, FTN = 128, FTKB = 128;
@@ -787,6 +787,8 @@ extern "C" int mi355q_fp8_block_gemm_ws(void* out, const void* x, const void* w,
                                         const float* w_scale, const void* bias, int M, int N, int K, long ldx,
                                         long ldw, long ldo, int out_dtype, void* workspace, size_t workspace_bytes,
                                         void* stream) {
+  const int zeroed = out_dtype & MI355Q_ZEROED_COUNTERS;
+  out_dtype ^= zeroed;
   MQ_REQUIRE(M >= 0 && N > 0 && K > 0, "fp8_block_gemm: bad shape M=%d N=%d K=%d", M, N, K);
   if (M == 0) return 0;
   MQ_REQUIRE(out && x && w && x_scale && w_scale, "fp8_block_gemm: null pointer");
@@ -802,7 +804,7 @@ extern "C" int mi355q_fp8_block_gemm_ws(void* out, const void* x, const void* w,
   size_t mid_bytes = 0;
   if (kslab && q8_mid_wanted(0, M, N, K, ldx, &mid_bytes) && (mid_bytes == 0 || (workspace && workspace_bytes >= F8_WS_OFFSET + mid_bytes)))
     return q8_mid_launch(0, out, x, w, x_scale, 0, w_scale, 0, bias, 0, M, N, K, ldx, ldo, out_dtype,
-                         workspace, as_stream(stream));
+                         workspace, zeroed != 0, as_stream(stream));
   F8Args a = {};
   a.out = out; a.x = (const uint8_t*)x; a.w = (const uint8_t*)w; a.x_scale = x_scale; a.w_scale = w_scale;
   a.bias = bias; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldw = ldw; a.ldo = ldo;
@@ -826,6 +828,8 @@ extern "C" int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w
                                          int x_scale_per_row, const float* w_scale, int w_scale_per_col,
                                          const void* bias, int M, int N, int K, long ldx, long ldw, long ldo,
                                          int out_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  const int zeroed = out_dtype & MI355Q_ZEROED_COUNTERS;
+  out_dtype ^= zeroed;
   MQ_REQUIRE(M >= 0 && N > 0 && K > 0, "fp8_scaled_gemm: bad shape M=%d N=%d K=%d", M, N, K);
   if (M == 0) return 0;
   MQ_REQUIRE(out && x && w && x_scale && w_scale, "fp8_scaled_gemm: null pointer");
@@ -840,7 +844,7 @@ extern "C" int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w
       (out_dtype == MI355Q_F16 || out_dtype == MI355Q_BF16) && q8_mid_wanted(1, M, N, K, ldx, &mid_bytes) &&
       (mid_bytes == 0 || (workspace && workspace_bytes >= F8_WS_OFFSET + mid_bytes)))
     return q8_mid_launch(1, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, 0, M, N, K, ldx, ldo,
-                         out_dtype, workspace, as_stream(stream));
+                         out_dtype, workspace, zeroed != 0, as_stream(stream));
   // the MFMA tile kernel from 65 rows on when its 256 x 128 tiles fill a good part of the chip; below
   // (and for shapes it does not take) the weight-streaming kernel, which wants dense operands
   const long tiles = (long)((M + FTM - 1) / FTM) * (N / FTN);

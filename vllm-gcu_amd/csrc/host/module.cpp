@@ -297,7 +297,7 @@ void int8_mm(const Int8Mm& m, const Tensor& q, const Tensor& xs, const Tensor& o
   }
   check(mi355q_w8a8_int8_gemm_ws(out.data_ptr(), nullptr, static_cast<const int8_t*>(q.data_ptr()),
                                  static_cast<const int8_t*>(m.w.data_ptr()), xp, xp && xs.numel() > 1, wp, 1, ptr(m.bias), 0, M,
-                                 m.N, m.K, m.K, 0, m.N, dtype_code(m.out_dtype), ws.p, ws.bytes, stream),
+                                 m.N, m.K, m.K, 0, m.N, dtype_code(m.out_dtype) | MI355Q_ZEROED_COUNTERS, ws.p, ws.bytes, stream),
         "w8a8_int8_gemm");
 }
 
@@ -450,8 +450,8 @@ PyObject* py_fp8_block_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
     out = empty(with_last(x, N), od, x);
     const float *xp = static_cast<const float*>(xs.data_ptr()), *wp = static_cast<const float*>(st->data_ptr());
     if (need >= 0)
-      check(mi355q_fp8_block_gemm_ws(out.data_ptr(), q.data_ptr(), wt->data_ptr(), xp, wp, nullptr, M, N, K, K, 0, N, dtype_code(od),
-                                     ws.p, ws.bytes, stream),
+      check(mi355q_fp8_block_gemm_ws(out.data_ptr(), q.data_ptr(), wt->data_ptr(), xp, wp, nullptr, M, N, K, K, 0, N,
+                                     dtype_code(od) | MI355Q_ZEROED_COUNTERS, ws.p, ws.bytes, stream),
             "fp8_block_gemm");
     else
       check(mi355q_kcontig_gemm(out.data_ptr(), q.data_ptr(), wt->data_ptr(), xp, wp, nullptr, 1, 128, M, K, N, MI355Q_F16,
@@ -501,7 +501,7 @@ PyObject* py_fp8_scaled_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
     out = empty(with_last(x, N), x.scalar_type(), x);
     check(mi355q_fp8_scaled_gemm_ws(out.data_ptr(), q.data_ptr(), wt->data_ptr(), static_cast<const float*>(xs.data_ptr()),
                                     per_row && M > 1, static_cast<const float*>(st->data_ptr()), st->numel() > 1, ptr(bias), M, N, K,
-                                    K, 0, N, dt, ws.p, ws.bytes, stream),
+                                    K, 0, N, dt | MI355Q_ZEROED_COUNTERS, ws.p, ws.bytes, stream),
           "fp8_scaled_gemm");
   }
   return THPVariable_Wrap(std::move(out));

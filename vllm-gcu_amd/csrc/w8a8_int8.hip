@@ -29,7 +29,7 @@ int int8_tile_launch(void* out, const void* x, const void* w, const float* x_sca
 bool q8_mid_wanted(int mode, int M, int N, int K, long ldx, size_t* bytes);
 int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
                   int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* workspace,
-                  hipStream_t st);
+                  bool zeroed, hipStream_t st);
 namespace {
 
 constexpr int TM = 256, TKB = 128;                // tile rows of x, bytes of K per LDS tile row
@@ -983,6 +983,8 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
                                         int w_scale_per_col, const void* bias, int bias_f32, int M, int N,
                                         int K, long ldx, long ldw, long ldo, int out_dtype, void* workspace,
                                         size_t workspace_bytes, void* stream) {
+  const int zeroed = out_dtype & MI355Q_ZEROED_COUNTERS;
+  out_dtype ^= zeroed;
   MQ_REQUIRE(M >= 0 && N > 0 && K > 0, "w8a8_int8_gemm: bad shape M=%d N=%d K=%d", M, N, K);
   if (M == 0) return 0;
   MQ_REQUIRE(out && x && w, "w8a8_int8_gemm: null pointer");
@@ -999,7 +1001,7 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
   if (kslab && !acc_out && q8_mid_wanted(2, M, N, K, ldx, &mid_bytes) &&
       (mid_bytes == 0 || (workspace && workspace_bytes >= I8_WS_OFFSET + mid_bytes)))
     return q8_mid_launch(2, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K, ldx,
-                         ldo, out_dtype, workspace, as_stream(stream));
+                         ldo, out_dtype, workspace, zeroed != 0, as_stream(stream));
   if (N % 128 == 0 && !acc_out && (size_t)N * K < ((size_t)1 << 32) && (size_t)256 * (size_t)ldx < ((size_t)1 << 32) &&
       (kslab || (size_t)128 * (size_t)ldw < ((size_t)1 << 32)) && int8_pick(M, N, K).tiles128)
     return int8_tile_launch(out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K,
@@ -1011,7 +1013,7 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
     for (int m = 0; m < M; m += fit)
       if (int rc = mi355q_w8a8_int8_gemm_ws((char*)out + (size_t)m * ldo * cell, acc_out ? acc_out + (size_t)m * N : nullptr, x + (size_t)m * ldx, w,
                                             x_scale && x_scale_per_row ? x_scale + m : x_scale, x_scale_per_row, w_scale, w_scale_per_col, bias,
-                                            bias_f32, std::min(fit, M - m), N, K, ldx, ldw, ldo, out_dtype, workspace, workspace_bytes, stream))
+                                            bias_f32, std::min(fit, M - m), N, K, ldx, ldw, ldo, out_dtype | zeroed, workspace, workspace_bytes, stream))
         return rc;
     return 0;
   }

@@ -370,7 +370,7 @@ def _scaled_int8_mm(out, x, weight, x_scale, w_scale, bias, acc_out=None):
         wsp = rt.workspace(x.device, need) if need else None
         _lib.call("mi355q_w8a8_int8_gemm_ws", out2.data_ptr(), rt.ptr(acc_out), x2.data_ptr(), w.data_ptr(),
                   rt.ptr(xs), xs_row, rt.ptr(ws), ws_col, rt.ptr(bias), bias_f32, M, N, K,
-                  x2.stride(0), ldw, out2.stride(0), rt.dtype_code(out.dtype), rt.ptr(wsp),
+                  x2.stride(0), ldw, out2.stride(0), rt.dtype_code(out.dtype) | _lib.ZEROED_COUNTERS, rt.ptr(wsp),
                   0 if wsp is None else wsp.numel(), rt.stream_ptr())
 
 
@@ -425,7 +425,7 @@ def _scaled_fp8_mm(out, x, weight, x_scale, w_scale, bias):
         wsp = rt.workspace(x.device, need) if need else None
         _lib.call("mi355q_fp8_scaled_gemm_ws", out2.data_ptr(), x2.data_ptr(), w.data_ptr(), xs.data_ptr(),
                   int(xs.numel() > 1), ws.data_ptr(), int(ws.numel() > 1), rt.ptr(bias), M, N, K,
-                  x2.stride(0), ldw, out2.stride(0), rt.dtype_code(out.dtype), rt.ptr(wsp),
+                  x2.stride(0), ldw, out2.stride(0), rt.dtype_code(out.dtype) | _lib.ZEROED_COUNTERS, rt.ptr(wsp),
                   0 if wsp is None else wsp.numel(), rt.stream_ptr())
 
 
@@ -938,7 +938,7 @@ def _linear_quant_impl(out, lhs, rhs, bias, lhs_scale, rhs_scale):
             wsp = rt.workspace(lhs.device, total) if total else None
             _lib.call("mi355q_fp8_block_gemm_ws", out.data_ptr(), a2.data_ptr(), rhs.data_ptr(), xs.data_ptr(),
                       ws.data_ptr(), rt.ptr(b), M, N, K, K, 0 if rearrange.is_kslab(rhs) else K, N,
-                      rt.dtype_code(out.dtype), rt.ptr(wsp), 0 if wsp is None else wsp.numel(), rt.stream_ptr())
+                      rt.dtype_code(out.dtype) | _lib.ZEROED_COUNTERS, rt.ptr(wsp), 0 if wsp is None else wsp.numel(), rt.stream_ptr())
         return
     _kcontig(out, lhs, rhs, lhs_scale.to(torch.float32).reshape(-1, lhs_scale.shape[-1]).contiguous(),
              rhs_scale.to(torch.float32).contiguous(), bias, _lib.Q_FP8_BLOCK, 128)
