@@ -401,9 +401,11 @@ int mi355q_moe_sum(void* out, const void* in, long rows, int topk, int K, int in
  */
 size_t mi355q_moe_gemm_workspace_bytes(int quant_mode, int numel, int block_size, int max_blocks, int E,
                                        int K, int N);
-/* What mi355q_moe_gemm takes for quant_mode 0 on blocks of 64 slots: the kernel with copying wavefronts, or tiles with K in k_ranges (where
- * the workspace holds their sums). */
+/* What mi355q_moe_gemm takes for quant_mode 0 on blocks of 64 slots with a workspace of that size: the kernel with copying wavefronts, or
+ * tiles with K in k_ranges; and (scratch 0) without one, or with one that does not hold the ranges. */
 int mi355q_moe_w4a16_plan(int numel, int E, int K, int N, int group_size, int zeros_kind, int dtype, int* rows_kernel, int* k_ranges);
+int mi355q_moe_w4a16_plan_scratch(int numel, int E, int K, int N, int group_size, int zeros_kind, int dtype, int scratch, int* rows_kernel,
+                                  int* k_ranges);
 int mi355q_moe_gemm(void* out, const void* a, const void* w, const float* a_scale, const void* w_scale,
                     const void* w_zeros, int zeros_kind, int quant_mode, int group_size,
                     const float* topk_weights, const int32_t* sorted_token_ids, const int32_t* expert_ids,

@@ -1085,3 +1085,31 @@ def test_w4a16_down_sum_of_slots_in_no_block(fmoe, block, E, K, N, rows, topk, d
                                                      *tail[6:], tokens, topk, block, ex.numel(), E, K, N, code, ws.data_ptr(), need, st),
                    "moe_w4a16_down_sum_ids")
         assert torch.equal(out, want) and (out[-1] == 0).all()
+
+
+@pytest.mark.parametrize("room", ["none", "less than the ranges"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("E,K,N,rows", [(4, 7168, 256, 40), (2, 6528, 1024, 200), (1, 4096, 640, 83)])
+def test_grouped_w4a16_without_room_for_k_ranges(fmoe, E, K, N, rows, dtype, room):
+    """Blocks of 64 slots whose plan cuts K, without a workspace or with one that does not hold the ranges: sums that are exact in fp32 against a
+    float64 product, to the last bit."""
+    from vllm_gcu_amd import _lib
+    from vllm_gcu_amd.kernels.quantization import rearrange
+    print(f"case blocks of 64, workspace {room}, E={E} K={K} N={N} rows={rows} {dtype}", flush=True)
+    lib, code, st, g, numel = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream, 128, E * rows
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // 8, N), dtype=torch.int32, device="cuda", generator=gen)
+    s = (2.0 ** torch.randint(-8, -5, (E, K // g, N), device="cuda", generator=gen)).to(dtype)
+    x = torch.randint(-3, 4, (numel, K), device="cuda", generator=gen).to(dtype)
+    ids = torch.randint(0, E, (numel, 1), device="cuda", generator=gen, dtype=torch.int32)
+    so, ex, npp = fmoe.moe_align_block_size(ids, 64, E)
+    assert lib.mi355q_moe_gemm_workspace_bytes(0, numel, 64, ex.numel(), E, K, N) >= 2 * numel * N * 4
+    ws = torch.full((numel * N,), float("nan"), device="cuda") if room != "none" else None
+    out = torch.full((numel, N), float("nan"), dtype=dtype, device="cuda")
+    _lib.check(lib.mi355q_moe_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), None, s.data_ptr(), None, _lib.ZP_NONE, 0, g, None, so.data_ptr(),
+                                   ex.data_ptr(), npp.data_ptr(), numel, 1, 64, ex.numel(), E, K, N, code, code, 0,
+                                   None if ws is None else ws.data_ptr(), 0 if ws is None else numel * N * 4, st), "moe_gemm")
+    dense = (rearrange.unpack_slab(w).view(E, K // g, g, N).double() - 8) * s[:, :, None].double()
+    for e in range(E):
+        r = (ids[:, 0] == e).nonzero().view(-1)
+        assert torch.equal(out[r], (x[r].double() @ dense[e].view(K, N)).to(dtype))

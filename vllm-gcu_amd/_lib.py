@@ -82,6 +82,7 @@ SIGNATURES = {
     "mi355q_moe_w4a16_unsorted_sum_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "mi355q_moe_w4a16_unsorted_sum": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
                                               c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "mi355q_moe_w4a16_plan_scratch": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "mi355q_moe_w4a16_plan": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "mi355q_moe_w4a16_gates": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "mi355q_moe_w4a16_gate_up": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int,

@@ -1270,15 +1270,16 @@ static double expected_blocks(int numel, int E, int block) {
   for (int k = 0; k * (double)block < r + 8 * sd; ++k) sum += 0.5 * std::erfc((k * (double)block + 0.5 - r) / sd);
   return std::max(1.0, E * sum);
 }
-static BlocksPlan make_blocks_plan(int flags, int numel, int E, int K, int N) {
-  const bool plain = flags & 1, rows = flags & 2;  // plain: the loop that is not pipelined; rows: that kernel takes these operands
+static BlocksPlan make_blocks_plan(int flags, double blocks, int numel, int E, int K, int N) {
+  // plain: the loop that is not pipelined; rows: that kernel takes these operands; whole: nowhere to put the sums of K ranges
+  const bool plain = flags & 1, rows = flags & 2, whole = flags & 8;
   const int G = K / 128;
-  const double blocks = expected_blocks(numel, E, 64), cus = device_cu_count(), weights = (double)std::min(blocks, (double)E) * K * N / 2;
+  const double cus = device_cu_count(), weights = (double)std::min(blocks, (double)E) * K * N / 2;
   const double slow = plain ? 1.39 : 1.0, stage = (flags & 4) && !plain ? 13.4 : 0;   // stage: the pass that makes the rows fp16
   auto with_stream = [weights](double t) { const double h = weights / 3.8e6; return std::sqrt(std::sqrt(t * t * t * t + h * h * h * h)); };
   BlocksPlan best = {false, 1};
   double least = 1e30;
-  for (int s = 1; s <= 6; ++s) {
+  for (int s = 1; s <= (whole ? 1 : 6); ++s) {
     const int kper = (G + s - 1) / s;
     if (s > 1 && (G / s < 4 || (G + kper - 1) / kper != s || (size_t)s * numel * N * sizeof(float) > TILE_SPLITK_BYTES * 2)) continue;
     const double one = (kper * 1.18 + 5.2) * slow, two = (kper * 1.59 + 9.5) * slow;
@@ -1295,12 +1296,13 @@ static BlocksPlan make_blocks_plan(int flags, int numel, int E, int K, int N) {
   return best;
 }
 struct BlocksPlans {
-  BlocksPlan of[8];                                // by flags
+  BlocksPlan of[16];                               // by flags
 };
 static BlocksPlans blocks_plans(int numel, int E, int K, int N) {
   return cached_plan(E, numel, N, K, [](int E, int M, int N, int K) {
     BlocksPlans p;
-    for (int f = 0; f < 8; ++f) p.of[f] = make_blocks_plan(f, M, E, K, N);
+    const double blocks = expected_blocks(M, E, 64);
+    for (int f = 0; f < 16; ++f) p.of[f] = make_blocks_plan(f, blocks, M, E, K, N);
     return p;
   });
 }
@@ -1309,9 +1311,12 @@ static BlocksPlans blocks_plans(int numel, int E, int K, int N) {
 static bool grouped_stage_pays(int numel, int block_size, int N) {
   return block_size == 64 && (long)numel * N >= (1L << 21);
 }
-static BlocksPlan blocks_plan(int numel, int E, int K, int N, int group_size, int zeros_kind, int dtype) {
-  const bool bf16 = dtype == MI355Q_BF16, pipelined = group_size % 128 == 0 && zeros_kind != MI355Q_ZP_PRESCALED && (!bf16 || grouped_stage_pays(numel, 64, N));
-  return blocks_plans(numel, E, K, N).of[(pipelined ? 0 : 1) | (group_size != 32 ? 2 : 0) | (bf16 ? 4 : 0)];
+// scratch: the caller's workspace holds what w4a16_grouped_workspace_bytes asks for; without it nothing is cut or staged.  (Tiles whose ranges had
+// no room ran in one: us without a workspace, one expert of 11776 x 12544 at 43 rows 98.6 -> 41, four of 7168 x 4096 at 40 62.7 -> 30.)
+static BlocksPlan blocks_plan(int numel, int E, int K, int N, int group_size, int zeros_kind, int dtype, bool scratch) {
+  const bool bf16 = dtype == MI355Q_BF16;
+  const bool pipelined = group_size % 128 == 0 && zeros_kind != MI355Q_ZP_PRESCALED && (!bf16 || (scratch && grouped_stage_pays(numel, 64, N)));
+  return blocks_plans(numel, E, K, N).of[(pipelined ? 0 : 1) | (group_size != 32 ? 2 : 0) | (bf16 ? 4 : 0) | (scratch ? 0 : 8)];
 }
 static size_t grouped_partial_bytes(int splits, int numel, int N) {
   return splits > 1 ? (((size_t)splits * numel * N * sizeof(float)) + 255) & ~(size_t)255 : 0;
@@ -1365,7 +1370,12 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   // 1408 x 2048 at 17 / 26 rows, blocks of 32, 132 / 147 -> 94 / 103.)
   const bool plain = !scales_f32 && !out_scale;
   BlocksPlan plan = {block_size == 32, 1};
-  if (block_size == 64 && plain) plan = blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype);
+  if (block_size == 64 && plain) {
+    plan = blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype, true);
+    if (workspace ? plan.splits > 1 && workspace_bytes < (size_t)plan.splits * numel * N * sizeof(float)
+                  : w4a16_grouped_workspace_bytes(numel, block_size, max_blocks, E, K, N) > 0)
+      plan = blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype, false);
+  }
   MQ_REQUIRE(!glu || w4a16_gates(block_size, N, group_size, zeros_kind), "moe_w4a16_gate_up: not for these operands");
   if (plain && group_size != 32 && plan.rows)
     return w4a16_rows_grouped_launch(out, x, qweight, scales, zeros, zeros_kind, topk_weights, sorted_ids, expert_ids, npp, numel,
@@ -1390,7 +1400,6 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
   a.numel = numel; a.topk = topk; a.E = E;
   const int G = K / 128;
   int splits = plan.splits;
-  if (splits > 1 && (!workspace || workspace_bytes < (size_t)splits * numel * N * sizeof(float))) splits = 1;
   a.kper = (G + splits - 1) / splits;
   splits = (G + a.kper - 1) / a.kper;              // no empty splits
   a.partial = splits > 1 ? (float*)workspace : nullptr;
@@ -1471,10 +1480,15 @@ int w4a16_grouped_launch(void* out, const void* x, const int32_t* qweight, const
 }  // namespace mi355q
 
 extern "C" int mi355q_moe_w4a16_plan(int numel, int E, int K, int N, int group_size, int zeros_kind, int dtype, int* rows_kernel, int* k_ranges) {
+  return mi355q_moe_w4a16_plan_scratch(numel, E, K, N, group_size, zeros_kind, dtype, 1, rows_kernel, k_ranges);
+}
+
+extern "C" int mi355q_moe_w4a16_plan_scratch(int numel, int E, int K, int N, int group_size, int zeros_kind, int dtype, int scratch, int* rows_kernel,
+                                             int* k_ranges) {
   using namespace mi355q;
   MQ_REQUIRE(numel > 0 && E > 0 && K > 0 && N > 0 && group_size > 0, "moe_w4a16_plan: bad shape numel=%d E=%d K=%d N=%d", numel, E, K, N);
   MQ_REQUIRE(rows_kernel && k_ranges, "moe_w4a16_plan: null pointer");
-  const BlocksPlan p = blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype);
+  const BlocksPlan p = blocks_plan(numel, E, K, N, group_size, zeros_kind, dtype, scratch != 0);
   *rows_kernel = p.rows;
   *k_ranges = p.splits;
   return 0;
