@@ -199,6 +199,10 @@ int mi355q_q8_mid_plan(int kind, int M, int N, int K, size_t* workspace_bytes);
 /* The work split of that plan: rows and columns of a workgroup's tile and K ranges (what a profile was taken on); all 0 where the
  * plan answers 0. */
 int mi355q_q8_mid_tile(int kind, int M, int N, int K, int* rows, int* columns, int* k_ranges);
+/* The same by the kernel that runs, with (scratch 1) a workspace that is large enough or without one: tile 0 / 1 = 32 x 32 / 32 x 64 with rings of
+ * six stages, 2 / 3 = 64 x 64 / 32 x 64 with four, 4 .. 11 = 48, 64 .. 160 rows x 128 columns, -1 = another kernel takes the call; its K
+ * ranges (0 then); whether it adds them itself when the call has MI355Q_ZEROED_COUNTERS. */
+int mi355q_q8_mid_way(int kind, int M, int N, int K, int scratch, int* tile, int* k_ranges, int* in_kernel);
 
 /* The rows of a tile (128 .. 256 x 128 columns) and the K ranges of the kernel for more rows (csrc/fp8_block_tile.hip; a workspace that holds
  * the ranges) where it is the one that those entry points launch. */

@@ -4,7 +4,7 @@ blocks, one and several K ranges, with and without bias.  int8 is exact; fp8 is 
 import pytest
 import torch
 
-from test_q8_plans_cpu import tile
+from test_q8_plans_cpu import NO_ROOM, tile
 from vllm_gcu_amd.kernels import _custom_ops as ops
 from vllm_gcu_amd.kernels import _runtime as rt
 from vllm_gcu_amd.kernels.quantization import rearrange
@@ -225,3 +225,22 @@ def test_k_ranges_leave_the_first_mib_as_it_was(kind, M, N, K, plan, zeroed):
             _lib.call("mi355q_fp8_block_gemm_ws", out.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), sc.data_ptr(), None, M, N, K, K, 0, N,
                       code, ws.data_ptr(), need, st)
         assert torch.equal(out, want) and torch.equal(ws[:1 << 20], before)
+
+
+@pytest.mark.parametrize("kind,M,N,K", NO_ROOM)
+def test_without_room_for_k_ranges(kind, M, N, K):
+    """Shapes whose plan cuts K, through the entry points without a workspace: sums that are exact, to the bit."""
+    from vllm_gcu_amd import _lib
+    print(f"case q8 without a workspace kind={kind} M={M} N={N} K={K}", flush=True)
+    torch.manual_seed(M + N + K)
+    x, w = (torch.randint(-3, 4, (r, K), device="cuda").to(torch.int8 if kind == INT8 else torch.float8_e4m3fn) for r in (M, N))
+    wk, st = rearrange.to_kslab(w), torch.cuda.current_stream().cuda_stream
+    xs, sc = (torch.ones(r, K // 128 if kind == BLOCK else 1, device="cuda") for r in (M, N // 128 if kind == BLOCK else N))
+    out = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+    if kind == INT8:
+        _lib.call("mi355q_w8a8_int8_gemm", out.data_ptr(), None, x.data_ptr(), wk.data_ptr(), xs.data_ptr(), 1, sc.data_ptr(), 1, None, 0, M, N, K, K, 0,
+                  N, _lib.BF16, st)
+    else:
+        _lib.call("mi355q_fp8_block_gemm", out.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), sc.data_ptr(), None, M, N, K, K, 0, N, _lib.BF16,
+                  st)
+    assert torch.equal(out, (x.double() @ w.double().t()).bfloat16())

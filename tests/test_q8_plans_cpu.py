@@ -55,3 +55,30 @@ def test_no_plan_outside_the_range():
         assert tile(1, M, N, K) == (0, 0, 0)
     with pytest.raises(RuntimeError, match="bad shape"):
         tile(3, 64, 4096, 4096)
+
+
+def way(kind, M, N, K, scratch=1):
+    """(tile, K ranges, added in the kernel)"""
+    out = [c_int() for _ in range(3)]
+    _lib.call("mi355q_q8_mid_way", kind, M, N, K, scratch, *(byref(v) for v in out))
+    return out[0].value, out[1].value, bool(out[2].value)
+
+
+NO_ROOM = [(0, 23, 768, 1792), (0, 28, 512, 1664), (0, 20, 896, 1536), (2, 17, 512, 2304), (2, 30, 320, 2432), (2, 22, 1216, 2688), (2, 76, 128, 2688)]
+
+
+# us without a workspace, tiles of 256 rows / here: 9.4 / 6.0, 8.9 / 5.7, 8.7 / 5.6, 11.2 / 6.2, 14.7 / 6.2, 15.8 / 6.4, 13.4 / 6.1
+@pytest.mark.parametrize("kind,M,N,K", NO_ROOM)
+def test_ranges_without_room_do_not_lose_the_kernel(kind, M, N, K):
+    tile_, ranges, _ = way(kind, M, N, K)
+    assert tile_ in (0, 1) and ranges > 1
+    assert way(kind, M, N, K, 0) == (3, 1, False)
+
+
+def test_what_needs_no_room_is_the_same_without():
+    for kind in range(3):
+        for K, N in LAYERS:
+            for M in range(1, 1600, 7):
+                w = way(kind, M, N, K)
+                without = way(kind, M, N, K, 0)
+                assert without == w if w[1] <= 1 else without[1] <= 1

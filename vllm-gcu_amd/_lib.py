@@ -34,6 +34,7 @@ SIGNATURES = {
     "mi355q_w4a16_gemm_noalloc": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                                           c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "mi355q_q8_mid_plan": (c_int, [c_int, c_int, c_int, c_int, c_void_p]),
+    "mi355q_q8_mid_way": (c_int, [c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "mi355q_q8_mid_tile": (c_int, [c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "mi355q_w8a8_int8_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int,
                                       c_void_p, c_int, c_int, c_int, c_int, c_long, c_long, c_long, c_int,
