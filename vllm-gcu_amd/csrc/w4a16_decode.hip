@@ -749,8 +749,10 @@ extern "C" int mi355q_moe_w4a16_unsorted_sum(void* out, const void* a, const int
              "moe_w4a16_unsorted_sum: zeros_kind %d", zeros_kind);
   MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "moe_w4a16_unsorted_sum: dtype %d", dtype);
   MQ_REQUIRE(group_size > 0 && K % group_size == 0 && (size_t)N * K < ((size_t)1 << 31), "moe_w4a16_unsorted_sum: group_size=%d K=%d N=%d", group_size, K, N);
+  MQ_REQUIRE(K % 128 == 0 && N % 128 == 0 && group_size % 128 == 0, "moe_w4a16_unsorted_sum: K=%d, N=%d and group_size=%d must be multiples of 128", K, N,
+             group_size);
   const int numel = rows * topk, G = K / 128;
-  int s = sum_ranges(numel, E, K, N);
+  const int s = sum_ranges(numel, E, K, N);
   MQ_REQUIRE(workspace_bytes >= (size_t)s * numel * N * sizeof(float), "moe_w4a16_unsorted_sum: workspace of %zu bytes", workspace_bytes);
   const int kper = (G + s - 1) / s;
   MQ_REQUIRE((G + kper - 1) / kper == s, "moe_w4a16_unsorted_sum: %d K blocks in %d ranges", G, s);
