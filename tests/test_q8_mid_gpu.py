@@ -4,7 +4,7 @@ blocks, one and several K ranges, with and without bias.  int8 is exact; fp8 is 
 import pytest
 import torch
 
-from test_q8_plans_cpu import NO_ROOM, tile
+from test_q8_plans_cpu import NO_ROOM, tile, way
 from vllm_gcu_amd.kernels import _custom_ops as ops
 from vllm_gcu_amd.kernels import _runtime as rt
 from vllm_gcu_amd.kernels.quantization import rearrange
@@ -188,22 +188,31 @@ def test_k_ranges_leave_the_counters_at_zero(kind, M, N, K, plan):
         assert torch.equal(out, want) and not ws[:1 << 20].any()
 
 
+# with RANGES and SHAPES: every tile of every kind whole, with ranges that the kernel adds and with ranges that a second launch adds, where the plans
+# have such launches (test_q8_plans_cpu.py looks whether they are all here)
+MORE = [(BLOCK, 17, 128, 14336), (BLOCK, 129, 1152, 3968), (BLOCK, 121, 2432, 10240), (BLOCK, 129, 128, 2048), (BLOCK, 207, 1152, 9088),
+        (BLOCK, 129, 128, 9088), (BLOCK, 97, 2176, 8192), (BLOCK, 339, 2176, 6400), (BLOCK, 1285, 3072, 384), (BLOCK, 1450, 3072, 384),
+        (SCALED, 17, 64, 14336), (SCALED, 129, 64, 2048), (SCALED, 33, 4096, 14336), (SCALED, 129, 64, 9088), (SCALED, 129, 1408, 14336),
+        (SCALED, 152, 1408, 14336), (INT8, 33, 1408, 5120), (INT8, 129, 1152, 3968), (INT8, 106, 2432, 6400), (INT8, 129, 64, 3072), (INT8, 70, 1024, 8192),
+        (INT8, 97, 3072, 9088), (INT8, 482, 2432, 10880)]
+
+
 @pytest.mark.parametrize("zeroed", [True, False])
-@pytest.mark.parametrize("kind,M,N,K,plan", RANGES)
+@pytest.mark.parametrize("kind,M,N,K,plan", RANGES + [(*m, None) for m in MORE])
 def test_k_ranges_leave_the_first_mib_as_it_was(kind, M, N, K, plan, zeroed):
-    """Products and sums that are exact, twice, over a workspace that nobody cleared but for, where the call says so, the counters: the output to
+    """Products and sums that are exact, in two output types, over a workspace that nobody cleared but for, where the call says so, the counters: the output to
     the bit, the counters at zero, and without them the first MiB neither read nor written."""
     from vllm_gcu_amd import _lib
     assert plan is None or tile(kind, M, N, K) == plan
     need = rt.host.q8_mid_plan(kind, M, N, K)
-    print(f"case q8 ranges kind={kind} M={M} N={N} K={K} workspace={need} zeroed={zeroed}", flush=True)
-    assert need > 1 << 20
+    print(f"case q8 ranges kind={kind} M={M} N={N} K={K} workspace={need} zeroed={zeroed} way={way(kind, M, N, K)}", flush=True)
+    assert need > 1 << 20 or (need == 0 and way(kind, M, N, K)[1] == 1)
     torch.manual_seed(M + N + K)
-    ws = torch.randint(0, 256, (need,), dtype=torch.uint8, device="cuda")
+    ws = torch.randint(0, 256, (max(need, 1 << 20),), dtype=torch.uint8, device="cuda")
     ws[1 << 20:] = 0xff
     if zeroed:
         ws[:1 << 16] = 0
-    before, code = ws[:1 << 20].clone(), _lib.BF16 | (_lib.ZEROED_COUNTERS if zeroed else 0)
+    before, flag = ws[:1 << 20].clone(), _lib.ZEROED_COUNTERS if zeroed else 0
     x, w = (torch.randint(-3, 4, (r, K), device="cuda").to(torch.int8 if kind == INT8 else torch.float8_e4m3fn) for r in (M, N))
     wk, st = rearrange.to_kslab(w), torch.cuda.current_stream().cuda_stream
     xs = 2.0 ** torch.randint(-2, 3, (M, K // 128) if kind == BLOCK else (M, 1), device="cuda").float()
@@ -212,9 +221,9 @@ def test_k_ranges_leave_the_first_mib_as_it_was(kind, M, N, K, plan, zeroed):
         xd, wd = x.double() * xs.double().repeat_interleave(128, 1), w.double() * sc.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
     else:
         xd, wd = x.double() * xs.double(), w.double() * sc.double()
-    want = (xd @ wd.t()).bfloat16()
-    for _ in range(2):
-        out = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+    want = xd @ wd.t()
+    for dtype in (torch.bfloat16, torch.float32 if kind == INT8 else torch.float16):
+        out, code = torch.full((M, N), float("nan"), dtype=dtype, device="cuda"), rt.dtype_code(dtype) | flag
         if kind == INT8:
             _lib.call("mi355q_w8a8_int8_gemm_ws", out.data_ptr(), None, x.data_ptr(), wk.data_ptr(), xs.data_ptr(), 1, sc.data_ptr(), 1, None, 0,
                       M, N, K, K, 0, N, code, ws.data_ptr(), need, st)
@@ -224,7 +233,7 @@ def test_k_ranges_leave_the_first_mib_as_it_was(kind, M, N, K, plan, zeroed):
         else:
             _lib.call("mi355q_fp8_block_gemm_ws", out.data_ptr(), x.data_ptr(), wk.data_ptr(), xs.data_ptr(), sc.data_ptr(), None, M, N, K, K, 0, N,
                       code, ws.data_ptr(), need, st)
-        assert torch.equal(out, want) and torch.equal(ws[:1 << 20], before)
+        assert torch.equal(out, want.to(dtype)) and torch.equal(ws[:1 << 20], before)
 
 
 @pytest.mark.parametrize("kind,M,N,K", NO_ROOM)

@@ -82,3 +82,22 @@ def test_what_needs_no_room_is_the_same_without():
                 w = way(kind, M, N, K)
                 without = way(kind, M, N, K, 0)
                 assert without == w if w[1] <= 1 else without[1] <= 1
+
+
+def _launches(shapes):
+    for kind, M, N, K in shapes:
+        t, ranges, in_kernel = way(kind, M, N, K)
+        if t >= 0:
+            yield kind, t, "whole" if ranges == 1 else "added in the kernel" if in_kernel else "second launch"
+
+
+def test_every_launch_of_the_plans_is_among_the_shapes_that_are_run():
+    """(kind, tile, how its K ranges are added): what the plans of a wide range of layers take against what the GPU tests run."""
+    import test_q8_mid_gpu as gpu
+    wide = LAYERS + [(K, N) for N in (64, 128, 192, 256, 384, 640, 1024, 1152, 1408, 2176, 2432, 3072, 4096)
+                     for K in (384, 1024, 1408, 2048, 3072, 3968, 5120, 6400, 8192, 9088, 10240, 10880, 14336)]
+    rows = [*range(17, 130), *range(130, 1537, 11)]
+    planned = set(_launches((kind, M, N, K) for kind in range(3) for K, N in wide if kind or N % 128 == 0 for M in rows))
+    run = set(_launches([(kind, *s) for kind in range(3) for s in gpu.SHAPES if kind == gpu.INT8 or s[1] % 128 == 0] +
+                        [s[:4] for s in gpu.RANGES] + gpu.MORE))
+    assert len(planned) > 50 and planned <= run, sorted(planned - run)
