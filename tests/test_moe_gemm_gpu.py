@@ -1113,3 +1113,49 @@ def test_grouped_w4a16_without_room_for_k_ranges(fmoe, E, K, N, rows, dtype, roo
     for e in range(E):
         r = (ids[:, 0] == e).nonzero().view(-1)
         assert torch.equal(out[r], (x[r].double() @ dense[e].view(K, N)).to(dtype))
+
+
+def _w4_layer(E, H, I, tokens, topk, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(E + H + I + tokens)
+    w1, w2 = (torch.randint(-2 ** 31, 2 ** 31 - 1, (E, r // 8, c), dtype=torch.int32, device="cuda", generator=gen) for r, c in ((H, 2 * I), (I, H)))
+    s1, s2 = ((torch.rand(E, r // 128, c, device="cuda", generator=gen) * 0.002 + 0.001).to(dtype) for r, c in ((H, 2 * I), (I, H)))
+    x = (torch.randn(tokens, H, device="cuda", generator=gen) * 0.1).to(dtype)
+    ids = torch.randint(0, E, (tokens, topk), device="cuda", generator=gen, dtype=torch.int32)
+    return x, w1, w2, s1, s2, torch.rand(tokens, topk, device="cuda", generator=gen), ids
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("E,H,I,tokens,topk,block", [(8, 512, 6144, 5, 2, 16), (60, 512, 256, 40, 4, 16), (8, 1024, 512, 60, 2, 32), (8, 512, 4096, 300, 2, 64)])
+def test_fused_experts_slots_of_no_expert_add_nothing(E, H, I, tokens, topk, block, dtype):
+    """The whole W4A16 layer on the library's own path, with ids outside [0, E), over scratch that holds NaN: as with those slots' weights at 0."""
+    from vllm_gcu_amd.kernels import _runtime as rt
+    print(f"case fused w4a16, dropped slots E={E} H={H} I={I} tokens={tokens} topk={topk} block={block} {dtype}", flush=True)
+    x, w1, w2, s1, s2, tw, ids = _w4_layer(E, H, I, tokens, topk, dtype)
+    dropped = torch.zeros_like(ids, dtype=torch.bool)
+    dropped[0, 0], dropped[1, -1], dropped[-1, :] = True, True, True
+    outs = []
+    for out_of in (False, True):
+        rt.workspace(x.device, 1)[1 << 20:].fill_(0xff)
+        del_me = torch.full((tokens * topk * (2 * I + H) * 4 + (1 << 22),), 0xff, dtype=torch.uint8, device="cuda")
+        del del_me
+        out = torch.full_like(x, float("nan"))
+        these = torch.where(dropped, torch.where(ids % 2 == 0, -1, E + 2).int(), ids) if out_of else ids
+        assert rt.host.fused_experts(0, 128, block, x, w1, w2, s1, s2, None, None, tw if out_of else tw * ~dropped, these, out)
+        outs.append(out.float())
+    assert (outs[1][-1] == 0).all() and outs[0].norm() > 0
+    assert float((outs[0] - outs[1]).norm() / outs[0].norm()) < 1e-5
+
+
+@pytest.mark.parametrize("E,H,I,tokens,topk,block", [(8, 512, 4096, 300, 2, 64), (8, 512, 4096, 60, 2, 16), (60, 512, 2048, 10, 4, 16)])
+def test_fused_experts_hold_no_rows_that_nobody_writes(E, H, I, tokens, topk, block):
+    """Where the first GEMM leaves gated columns there are no gate and up columns in the scratch."""
+    from vllm_gcu_amd.kernels import _runtime as rt
+    x, w1, w2, s1, s2, tw, ids = _w4_layer(E, H, I, tokens, topk, torch.float16)
+    out, numel = torch.empty_like(x), tokens * topk
+    for _ in range(2):                                       # (the first call allocates the stream's workspace)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        assert rt.host.fused_experts(0, 128, block, x, w1, w2, s1, s2, None, None, tw, ids, out)
+        held = torch.cuda.max_memory_allocated() - before
+    assert held < numel * (I + H) * 2 + 4 * numel * H * 4 + (1 << 17) and held < numel * 2 * I * 2

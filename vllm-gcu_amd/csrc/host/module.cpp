@@ -621,7 +621,8 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
   };
   const int64_t s_cols1 = mode == kFp8 ? K / 128 : 1, s_cols2 = mode == kFp8 ? I / 128 : 1;
   const int64_t o_q1 = room(quant ? M * K : 0), o_s1 = room(quant ? M * s_cols1 * 4 : 0);
-  const int64_t o_c1 = room(std::max(numel * N, numel * K) * 2);             // first GEMM, then (dead by then) the second one
+  // first GEMM, unless it leaves gated columns, then (dead by then) the second one, unless its sums are f32
+  const int64_t o_c1 = room(std::max(gate || sorted_gate || gate_up ? 0 : numel * N, unsorted ? 0 : numel * K) * 2);
   const int64_t o_c2 = room(mode == kFp8 ? 0 : numel * I * 2);
   const int64_t o_q2 = room(quant ? numel * I : 0), o_s2 = room(quant ? numel * s_cols2 * 4 : 0);
   const int64_t o_sorted = room((numel + E * (block - 1)) * 4), o_eid = room(blocks * 4), o_npp = room(4);
@@ -673,11 +674,10 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
                           s1p->data_ptr(), ptr(z1), z1.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE, mode, group, nullptr, sorted, eid,
                           npp, numel, T, block, blocks, E, K, N, act, code, quant, ws.p, ws.bytes, stream),
           "moe_gemm");
-    if (gate_up) {
-    } else if (mode == kFp8)
+    if (mode == kFp8 && !gate_up)
       check(mi355q_fp8_group_quant(reinterpret_cast<uint8_t*>(b + o_q2), s2, b + o_c1, numel, I, 128, 1, code, nullptr, 1, stream),
             "fp8_group_quant");
-    else if (!gate && !sorted_gate)
+    else if (mode != kFp8 && !gate && !sorted_gate)
       check(mi355q_silu_and_mul(b + o_c2, b + o_c1, numel, I, code, nullptr, 1, stream), "silu_and_mul");
     if (mode == kInt8)
       check(mi355q_dynamic_int8_quant(reinterpret_cast<int8_t*>(b + o_q2), s2, b + o_c2, numel, I, code, nullptr, stream),
