@@ -1159,3 +1159,93 @@ def test_fused_experts_hold_no_rows_that_nobody_writes(E, H, I, tokens, topk, bl
         assert rt.host.fused_experts(0, 128, block, x, w1, w2, s1, s2, None, None, tw, ids, out)
         held = torch.cuda.max_memory_allocated() - before
     assert held < numel * (I + H) * 2 + 4 * numel * H * 4 + (1 << 17) and held < numel * 2 * I * 2
+
+
+def _same(a, b):
+    return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0, 1.0, -1.0), b.nan_to_num(0.0, 1.0, -1.0)) and torch.equal(a.isinf(), b.isinf())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block,E,K,N,rows", [(64, 4, 4096, 256, 75), (64, 16, 1664, 1024, 70), (64, 64, 256, 1024, 70), (32, 8, 1408, 2816, 20),
+                                              (16, 9, 1408, 2816, 9)])
+def test_w4a16_epilogues_pass_infinities_and_nan(fmoe, block, E, K, N, rows, dtype):
+    """Rows with an infinity of either sign, a NaN and the largest finite value: the gated columns and the sums over slots as the separate
+    launches make them, and no other row touched by them."""
+    from vllm_gcu_amd import _lib
+    print(f"case w4a16 epilogues, inf and nan block={block} E={E} K={K} N={N} rows={rows} {dtype}", flush=True)
+    lib, code, st, g, topk = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream, 128, 2
+    tokens = E * rows // topk
+    numel = tokens * topk
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w, z = (torch.randint(-2 ** 31, 2 ** 31 - 1, (E, r, c), dtype=torch.int32, device="cuda", generator=gen) for r, c in ((K // 8, N), (K // g, N // 8)))
+    s = (torch.rand(E, K // g, N, device="cuda", generator=gen) * 0.01 + 0.001).to(dtype)
+    ids = torch.randint(0, E, (tokens, topk), device="cuda", generator=gen, dtype=torch.int32)
+    so, ex, npp = fmoe.moe_align_block_size(ids, block, E)
+    need = lib.mi355q_moe_gemm_workspace_bytes(0, numel, block, ex.numel(), E, K, N)
+    ws = torch.full((need // 4 + 1,), float("nan"), device="cuda")
+    special = [float("inf"), -float("inf"), float("nan"), torch.finfo(dtype).max]
+    blocks = (so.data_ptr(), ex.data_ptr(), npp.data_ptr())
+
+    def gemm(x, slots_per_row, weights):
+        out = torch.full((numel, N), float("nan"), dtype=dtype, device="cuda")
+        _lib.check(lib.mi355q_moe_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), None, s.data_ptr(), z.data_ptr(), _lib.ZP_PACKED, 0, g, weights, *blocks,
+                                       numel, slots_per_row, block, ex.numel(), E, K, N, code, code, 0, ws.data_ptr(), need, st), "moe_gemm")
+        return out
+    x = torch.randn(tokens, K, device="cuda", generator=gen).to(dtype)
+    for i, v in enumerate(special):
+        x[2 * i + 1, 37 * i + 5] = v
+    got, want = (torch.full((numel, N // 2), 7.0, dtype=dtype, device="cuda") for _ in range(2))
+    _lib.check(lib.mi355q_moe_w4a16_gate_up(got.data_ptr(), x.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(), _lib.ZP_PACKED, g, *blocks, numel, topk,
+                                            block, ex.numel(), E, K, N, code, ws.data_ptr(), need, st), "moe_w4a16_gate_up")
+    _lib.check(lib.mi355q_silu_and_mul(want.data_ptr(), gemm(x, topk, None).data_ptr(), numel, N // 2, code, None, 1, st), "silu_and_mul")
+    plain = torch.ones(tokens, dtype=torch.bool, device="cuda")
+    plain[[1, 3, 5, 7]] = False
+    assert _same(got, want) and got[plain.repeat_interleave(topk)].isfinite().all() and not got.isfinite().all()
+
+    y, rw = torch.randn(numel, K, device="cuda", generator=gen).to(dtype), torch.rand(numel, device="cuda", generator=gen)
+    for i, v in enumerate(special):
+        y[5 * i + 2, 37 * i + 5] = v
+    rw[30], rw[33] = float("inf"), float("nan")
+    out, want = (torch.full((tokens, N), 7.0, dtype=dtype, device="cuda") for _ in range(2))
+    scratch = torch.empty(numel, N, dtype=dtype, device="cuda")
+    _lib.check(lib.mi355q_moe_w4a16_down_sum_ids(out.data_ptr(), scratch.data_ptr(), y.data_ptr(), w.data_ptr(), s.data_ptr(), z.data_ptr(),
+                                                 _lib.ZP_PACKED, g, rw.data_ptr(), ids.data_ptr(), 0, *blocks, tokens, topk, block, ex.numel(), E, K, N,
+                                                 code, ws.data_ptr(), need, st), "moe_w4a16_down_sum_ids")
+    _lib.check(lib.mi355q_moe_sum(want.data_ptr(), gemm(y, 1, rw.data_ptr()).data_ptr(), tokens, topk, N, code, code, None, st), "moe_sum")
+    plain[:] = True
+    plain[[i // topk for i in (2, 7, 12, 17, 30, 33)]] = False
+    assert _same(out, want) and out[plain].isfinite().all() and not out.isfinite().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block", [16, 32, 64])
+def test_fp8_gate_up_quant_passes_infinities_and_nan(fmoe, block, dtype):
+    """A row with a NaN, one whose scale is an infinity and one whose scale is a NaN: codes and scales of the GEMM and the quantiser, and no other
+    row touched by them."""
+    from vllm_gcu_amd import _lib
+    print(f"case fp8 gate and up, inf and nan block={block} {dtype}", flush=True)
+    lib, code, st = _lib.load(), _lib.F16 if dtype == torch.float16 else _lib.BF16, torch.cuda.current_stream().cuda_stream
+    E, K, N, tokens, topk = 4, 384, 512, 40, 2
+    numel, I = tokens * topk, N // 2
+    gen = torch.Generator(device="cuda").manual_seed(block)
+    x = (torch.randn(tokens, K, device="cuda", generator=gen) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)
+    x.view(torch.uint8)[3, 17] = 0x7f
+    xs = torch.rand(tokens, K // 128, device="cuda", generator=gen) * 0.01 + 1e-4
+    xs[9, 1], xs[11, 0] = float("inf"), float("nan")
+    w = (torch.randn(E, N, K, device="cuda", generator=gen) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)
+    ws = torch.rand(E, N // 128, K // 128, device="cuda", generator=gen) * 1e-3 + 1e-5
+    ids = torch.randint(0, E, (tokens, topk), device="cuda", generator=gen, dtype=torch.int32)
+    so, ex, npp = fmoe.moe_align_block_size(ids, block, E)
+    sums = torch.full((numel, N), float("nan"), dtype=dtype, device="cuda")
+    want, got = (torch.full((numel, I), 77, dtype=torch.uint8, device="cuda") for _ in range(2))
+    want_s, got_s = (torch.full((numel, I // 128), 7.0, device="cuda") for _ in range(2))
+    blocks = (so.data_ptr(), ex.data_ptr(), npp.data_ptr(), numel, topk, block, ex.numel(), E, K, N)
+    _lib.check(lib.mi355q_moe_gemm(sums.data_ptr(), x.data_ptr(), w.data_ptr(), xs.data_ptr(), ws.data_ptr(), None, 0, 1, 128, None, *blocks, _lib.F16,
+                                   code, 0, None, 0, st), "moe_gemm")
+    _lib.check(lib.mi355q_fp8_group_quant(want.data_ptr(), want_s.data_ptr(), sums.data_ptr(), numel, I, 128, 1, code, None, 1, st), "fp8_group_quant")
+    _lib.check(lib.mi355q_moe_fp8_gate_up_quant(got.data_ptr(), got_s.data_ptr(), x.data_ptr(), w.data_ptr(), xs.data_ptr(), ws.data_ptr(), *blocks, code,
+                                                0, st), "moe_fp8_gate_up_quant")
+    assert torch.equal(got, want) and _same(got_s, want_s)
+    plain = torch.ones(tokens, dtype=torch.bool, device="cuda")
+    plain[[3, 9, 11]] = False
+    assert sums[plain.repeat_interleave(topk)].isfinite().all() and not sums.isfinite().all() and got_s[plain.repeat_interleave(topk)].isfinite().all()

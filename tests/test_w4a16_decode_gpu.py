@@ -250,6 +250,43 @@ def test_unsorted_sum(E, K, N, rows, topk, ranges, dtype):
     assert lib.mi355q_moe_w4a16_unsorted_sum(got.data_ptr(), x.data_ptr(), *common, rows, topk, E, K, N, code, ws.data_ptr(), need - 4, st) != 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("E,K,N,rows,topk", [(8, 6144, 4096, 6, 2), (8, 2944, 4096, 6, 2), (60, 384, 256, 10, 6)])
+def test_unsorted_sum_passes_infinities_and_nan(E, K, N, rows, topk, dtype):
+    """Rows with an infinity of either sign, a NaN and the largest finite value, and an infinite weight: what the GEMM and moe_sum make of them (exact
+    sums elsewhere), and no other token touched by them."""
+    from vllm_gcu_amd import _lib
+    print(f"case unsorted sum, inf and nan E={E} K={K} N={N} rows={rows} topk={topk} {dtype}", flush=True)
+    lib, g, numel = _lib.load(), 128, rows * topk
+    code = _lib.F16 if dtype == torch.float16 else _lib.BF16
+    gen = torch.Generator(device="cuda").manual_seed(E + K + N)
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, K // 8, N), dtype=torch.int32, device="cuda", generator=gen)
+    s = (2.0 ** torch.randint(-9, -6, (E, K // g, N), device="cuda", generator=gen)).to(dtype)
+    x = torch.randint(-4, 5, (numel, K), device="cuda", generator=gen).to(dtype)
+    for i, v in enumerate((float("inf"), -float("inf"), float("nan"), torch.finfo(dtype).max)):
+        x[topk * i, 61 * i + 3] = v                          # tokens 0 .. 3
+    rw = torch.rand(numel, device="cuda", generator=gen)
+    rw[topk * 4] = float("inf")                              # token 4
+    ids, st = torch.randint(0, E, (rows, topk), device="cuda", generator=gen, dtype=torch.int32), torch.cuda.current_stream().cuda_stream
+    need = lib.mi355q_moe_w4a16_unsorted_sum_bytes(numel, E, K, N)
+    ws = torch.full((need // 4,), float("nan"), device="cuda")
+    got, want = (torch.full((rows, N), 7.0, dtype=dtype, device="cuda") for _ in range(2))
+    slots = torch.empty(numel, N, dtype=dtype, device="cuda")
+    common = (w.data_ptr(), s.data_ptr(), None, _lib.ZP_NONE, g, rw.data_ptr(), ids.data_ptr(), 0)
+    _lib.check(lib.mi355q_moe_w4a16_unsorted_sum(got.data_ptr(), x.data_ptr(), *common, rows, topk, E, K, N, code, ws.data_ptr(), need, st),
+               "moe_w4a16_unsorted_sum")
+    _lib.check(lib.mi355q_moe_w4a16_unsorted(slots.data_ptr(), x.data_ptr(), *common, numel, 1, E, K, N, 0, code, st), "moe_w4a16_unsorted")
+    _lib.check(lib.mi355q_moe_sum(want.data_ptr(), slots.data_ptr(), rows, topk, N, code, code, None, st), "moe_sum")
+    assert not got[:3].isfinite().all() and not got[4].isfinite().all()
+    for t in range(rows):
+        if t == 3:                                           # (sums that are not exact: 2^16 and more beside small products)
+            assert torch.equal(got[t].isfinite(), want[t].isfinite())
+            fin = want[t].isfinite()
+            assert torch.allclose(got[t][fin].double(), want[t][fin].double(), rtol=1e-2)
+        else:
+            assert torch.equal(got[t].nan_to_num(11.0, 12.0, 13.0), want[t].nan_to_num(11.0, 12.0, 13.0)) and (t < 5 or got[t].isfinite().all())
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("E,K,N,rows,topk", [(8, 6144, 4096, 3, 2), (8, 2944, 4096, 3, 2), (5, 384, 256, 64, 1), (60, 384, 256, 10, 6)])
