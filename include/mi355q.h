@@ -117,6 +117,10 @@ int mi355q_w4a16_gemm_ex(void* out, const void* x, const int32_t* qweight,
                          int dtype, void* workspace, size_t workspace_bytes,
                          int split_k, int family, void* stream);
 
+/* No counterpart in the reference.  The unsplit kernel for up to 16 rows (csrc/w4a16_decode.hip) on the current device: 16-column tiles per
+ * workgroup, its wavefronts and the K blocks of 128 that each holds; all 0 where the streaming kernel takes the shape. */
+int mi355q_w4a16_decode_plan(int M, int K, int N, int* tiles, int* wavefronts, int* k_blocks);
+
 /* No counterpart in the reference (the vendor GEMM chooses its own launch).  The work split the streaming
  * kernel takes for M <= 64 rows of a shape on the current device: 16-column tiles per workgroup (1, 2, 4
  * or 8) and the number of K ranges that separate workgroups sum through the workspace.  (Small layers of up to

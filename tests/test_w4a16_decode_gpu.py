@@ -1,5 +1,5 @@
 """The W4A16 kernels for up to 16 rows (csrc/w4a16_decode.hip), through the library's own choice, over small layers -- 1, 2 and 4 column
-tiles per workgroup, 8 and 16 wavefronts, one to four K blocks each (the last ones without a block), row counts around each load of
+tiles per workgroup, 8 and 16 wavefronts, one to seven K blocks each (the last ones without a block), row counts around each load of
 four rows, groups of 128 to K, zero-points and none, bias, exact inputs bit for bit, and a row of infinities -- and over blocks of 16
 slots of a fused-MoE layer."""
 import numpy as np
@@ -15,6 +15,9 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(128, 128, 128), (640, 1024, 128), (1024, 4096, 1024), (1152, 4224, 128), (2048, 384, 256), (2176, 8192, 128), (3072, 256, 1536),
           (4096, 512, 128), (4096, 8320, 256), (4224, 1024, 128), (6144, 4352, 128), (8192, 512, 4096), (1024, 16384, 128), (2944, 8448, 128),
           (1024, 8192, 256), (1280, 8320, 128), (3968, 4224, 128), (4352, 8320, 128), (6400, 4224, 128)]
+# K blocks 65 .. 112: five to seven of a wavefront, on either side of the rows where it takes them (test_w4a16_decode_cpu.py has the plans)
+DEEP = [(8320, 2048, 128), (10240, 3072, 1024), (10368, 4096, 128), (12288, 2048, 256), (12416, 3072, 128), (14336, 4096, 128), (10240, 4352, 128),
+        (8448, 8192, 256)]
 
 
 def _data(K, N, g, dtype, exact):
@@ -319,8 +322,7 @@ def test_unsorted_sum_without_slots_of_no_expert(E, K, N, rows, topk, dtype, wid
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("K,N,g", [(8320, 2048, 128), (10240, 3072, 1024), (10368, 4096, 128), (12288, 2048, 256), (12416, 3072, 128), (14336, 4096, 128),
-                                   (10240, 4352, 128), (8448, 8192, 256)])
+@pytest.mark.parametrize("K,N,g", DEEP)
 def test_deep_k(K, N, g, dtype):
     """Five to seven K blocks of a wavefront, on either side of the depths where it takes them, one and two tiles."""
     test_rows_1_to_16(K, N, g, dtype)

@@ -78,6 +78,7 @@ SIGNATURES = {
     "mi355q_moe_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                                 c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                                 c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "mi355q_w4a16_decode_plan": (c_int, [c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "mi355q_moe_w4a16_unsorted": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
                                           c_int, c_int, c_int, c_int, c_int, c_void_p]),
     "mi355q_moe_w4a16_unsorted_sum_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),

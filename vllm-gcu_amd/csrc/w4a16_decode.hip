@@ -717,6 +717,16 @@ int moe_range_sum_launch(void* out, const float* partial, const float* topk_weig
 
 using namespace mi355q;
 
+extern "C" int mi355q_w4a16_decode_plan(int M, int K, int N, int* tiles, int* wavefronts, int* k_blocks) {
+  MQ_REQUIRE(M > 0 && K > 0 && N > 0 && K % 128 == 0 && N % 128 == 0, "w4a16_decode_plan: bad shape M=%d K=%d N=%d", M, K, N);
+  MQ_REQUIRE(tiles && wavefronts && k_blocks, "w4a16_decode_plan: null pointer");
+  const DecodePlan p = decode_plan(M, K, N);
+  *tiles = p.nt;
+  *wavefronts = p.w;
+  *k_blocks = p.b;
+  return 0;
+}
+
 extern "C" int mi355q_moe_w4a16_unsorted(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
                                          int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64, int numel,
                                          int topk, int E, int K, int N, int silu_and_mul, int dtype, void* stream) {
