@@ -165,7 +165,7 @@ w4a16_decode_kernel(DecodeArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, kq = lane >> 4;
   constexpr int TG = 8 / NT;
-  const int slab = blockIdx.x / TG, t0 = (blockIdx.x % TG) * NT;
+  const int group = xcd_tile(), slab = group / TG, t0 = (group % TG) * NT;
   const int G = a.K >> 7, N = a.N, K = a.K;
   const int ncol8 = 128 * slab + 8 * c, ncol = ncol8 + t0;
   constexpr int RED = W * 4 * NT * 64 * 4, XL = W * 1024 * XN;    // x: 16 lanes to a row, four rows per load
@@ -281,7 +281,7 @@ w4a16_decode_grouped_kernel(DecodeArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, kq = lane >> 4;
   constexpr int CT = GLU ? NT / 2 : NT, TG = 8 / CT; // tiles in a slab, tile groups of a slab
-  const int slab = blockIdx.x / TG, t0 = (blockIdx.x % TG) * CT;
+  const int group = xcd_tile(), slab = group / TG, t0 = (group % TG) * CT;
   const int G = a.K >> 7, N = a.N, K = a.K;
   __shared__ int block_ids[IDS ? 16 : 1];
   const int32_t* const ids = a.sorted_ids + 16 * blockIdx.z;

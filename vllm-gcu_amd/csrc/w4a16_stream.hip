@@ -192,7 +192,9 @@ w4a16_stream_kernel(StreamArgs a) {
   const int c = lane & 15, kq = lane >> 4;
   constexpr int TG = 8 / NT;                          // tile groups per slab
   constexpr int HW = NT >= 2 ? NT / 2 : 1;            // packed 16-bit pairs per lane
-  const int slab = blockIdx.x / TG, t0 = (blockIdx.x % TG) * NT, split = blockIdx.y;
+  // parts of a slab on one XCD; behind more than two K ranges they were 0 .. 4 % slower so (14336 x 4096 at 32 rows 14.5 -> 15.1), and
+  // whole slabs have nothing to share
+  const int group = NT < 8 && gridDim.y <= 2 ? xcd_tile() : (int)blockIdx.x, slab = group / TG, t0 = (group % TG) * NT, split = blockIdx.y;
   const int G = a.K >> 7;
   const int per = a.per;
   const int gb = split * per;
