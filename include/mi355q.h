@@ -195,6 +195,15 @@ int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w, const flo
                               const void* bias, int M, int N, int K, long ldx, long ldw, long ldo,
                               int out_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
+/* No counterpart in the reference.  An 8-bit layer with kslab weights (N % 64 == 0, K % 128 == 0) on a few 16-bit rows, quantised in the same
+ * launch: kind 1 = fp8 with a scale per token (quant 1), kind 2 = int8 with a scale per token (quant 1) or per input channel (quant 2: x_scale
+ * [K] in x's type).  Bit for bit mi355q_fp8_token_quant, mi355q_dynamic_int8_quant or mi355q_static_int8_quant_typed and the GEMM on their
+ * codes.  w_scale f32 [N] or one value, bias [N] or null; x, bias and out in `dtype` (f16 or bf16), x, weights and scales aligned to 16
+ * bytes, out and bias to 8.  No workspace, nothing allocated.  _takes: 1 where the call is covered (up to 16 rows, some thousand elements). */
+int mi355q_q8_quant_gemm_takes(int kind, int quant, int M, int N, int K);
+int mi355q_q8_quant_gemm(void* out, const void* x, const void* w, const void* x_scale, const float* w_scale, int w_scale_per_col,
+                         const void* bias, int kind, int quant, int M, int N, int K, int dtype, void* stream);
+
 /* No counterpart in the reference.  Whether an 8-bit layer in the kslab order with M rows is taken by the kernel for
  * a few dozen to some hundred rows (csrc/q8_mid.hip) when mi355q_fp8_block_gemm_ws (kind 0), mi355q_fp8_scaled_gemm_ws
  * (kind 1) or mi355q_w8a8_int8_gemm_ws (kind 2) is called with *workspace_bytes bytes of workspace (0: none needed).

@@ -1,0 +1,128 @@
+"""The 8-bit kernel for up to 16 rows (csrc/q8_decode.hip): K of one block, of fewer blocks than wavefronts, of whole and ragged rounds of the ring; columns for
+one to eight tiles per workgroup with a last workgroup that is not full; every quantiser.  Rows quantised in the kernel give, bit for bit, what
+the quantiser's launch and the GEMM on its codes give, and codes are held to a float64 product."""
+import pytest
+import torch
+
+from vllm_gcu_amd import _lib
+from vllm_gcu_amd.kernels.quantization import rearrange
+
+pytestmark = pytest.mark.gpu
+DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
+FP8, INT8 = 1, 2                         # kinds of mi355q_q8_quant_gemm
+TOKEN, CHANNEL = 1, 2                    # its quantisers
+# (M, N, K)
+ROWS = [(1, 64, 128), (3, 192, 640), (16, 4096, 1024), (8, 4160, 1920), (5, 8256, 1152), (1, 12352, 1408), (1, 64, 2048), (7, 4096, 2176), (2, 4160, 4096),
+        (4, 8192, 4096), (1, 16384, 7168), (2, 16448, 3712), (1, 28672, 2048), (1, 3584, 18944), (1, 320, 20480)]
+CODES = [(1, 64, 2048), (16, 4096, 2048), (9, 4160, 2176), (16, 8256, 3712), (12, 12352, 5120), (3, 16448, 7168), (8, 4096, 14336), (7, 3584, 18560), (2, 64, 65536)]
+
+
+def _p(t):
+    return t.data_ptr() if t is not None else None
+
+
+def _check(rc):
+    torch.cuda.synchronize()
+    _lib.check(rc, "q8_decode test")
+
+
+def _stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+def _weights(kind, N, K, gen):
+    if kind == INT8:
+        return torch.randint(-128, 128, (N, K), dtype=torch.int8, device="cuda", generator=gen)
+    return (torch.randn(N, K, device="cuda", generator=gen) * 40).to(torch.float8_e4m3fn)
+
+
+def _codes_gemm(lib, kind, out, q, w, kslab, xs, ws, bias, M, N, K, dtype):
+    if kind == INT8:
+        return lib.mi355q_kcontig_gemm(_p(out), _p(q), _p(w), _p(xs), _p(ws), _p(bias), 2, 0, M, K, N, DT[dtype], DT[dtype], int(kslab), _stream())
+    return lib.mi355q_fp8_scaled_gemm(_p(out), _p(q), _p(w), _p(xs), int(xs.numel() > 1), _p(ws), int(ws.numel() > 1), _p(bias), M, N, K, K,
+                                      0 if kslab else K, N, DT[dtype], _stream())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind,quant", [(INT8, TOKEN), (INT8, CHANNEL), (FP8, TOKEN)])
+@pytest.mark.parametrize("M,N,K", ROWS)
+def test_rows_are_quantised_as_by_the_launch_of_their_own(M, N, K, kind, quant, dtype):
+    print(f"case q8 decode rows M={M} N={N} K={K} kind={kind} quant={quant} {dtype}", flush=True)
+    lib = _lib.load()
+    assert lib.mi355q_q8_quant_gemm_takes(kind, quant, M, N, K)
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, device="cuda", generator=gen).to(dtype)
+    x[M - 1, K - 1], x[0, 0] = 37.0, -0.0
+    if M > 2:
+        x[1] = 0.0                                              # a row of zeros
+        x[2, 5] = float("inf")                                  # reaches its own row only
+    if M > 3:
+        x[3, 7] = float("nan")
+    w = rearrange.to_kslab(_weights(kind, N, K, gen))
+    cs = (torch.rand(K, device="cuda", generator=gen) * 0.05 + 0.01).to(dtype)
+    bias = torch.randn(N, device="cuda", generator=gen).to(dtype) if M % 2 else None
+    ws = torch.rand(N if M != 2 or kind == INT8 else 1, device="cuda", generator=gen) * 0.01
+    q = torch.empty(M, K, dtype=torch.int8, device="cuda")
+    xs = torch.empty(M, device="cuda") if quant == TOKEN else None
+    if quant == CHANNEL:
+        _check(lib.mi355q_static_int8_quant_typed(_p(q), _p(x), _p(cs), DT[dtype], 1, M, K, DT[dtype], _stream()))
+    elif kind == INT8:
+        _check(lib.mi355q_dynamic_int8_quant(_p(q), _p(xs), _p(x), M, K, DT[dtype], None, _stream()))
+    else:
+        _check(lib.mi355q_fp8_token_quant(_p(q), _p(xs), _p(x), M, K, DT[dtype], None, _stream()))
+    want, got = (torch.full((M, N), float("nan"), device="cuda").to(dtype) for _ in range(2))
+    _check(_codes_gemm(lib, kind, want, q, w, True, xs, ws, bias, M, N, K, dtype))
+    _check(lib.mi355q_q8_quant_gemm(_p(got), _p(x), _p(w), _p(cs) if quant == CHANNEL else None, _p(ws), int(ws.numel() > 1), _p(bias), kind, quant, M, N,
+                                    K, DT[dtype], _stream()))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert torch.isfinite(got[[r for r in range(M) if r not in (2, 3)]]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", [0, FP8, INT8])                # 0: block scales
+@pytest.mark.parametrize("M,N,K", CODES)
+def test_codes(M, N, K, kind, dtype):
+    print(f"case q8 decode codes M={M} N={N} K={K} kind={kind} {dtype}", flush=True)
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = _weights(kind, M, K, gen)
+    w = _weights(kind, N, K, gen)
+    bias = torch.randn(N, device="cuda", generator=gen).to(dtype) if M % 2 else None
+    outs = []
+    if kind == 0:
+        xs, ws = torch.rand(M, K // 128, device="cuda", generator=gen) + 0.1, torch.rand((N + 127) // 128, K // 128, device="cuda", generator=gen) * 1e-4
+        want, size = torch.zeros(M, N, dtype=torch.float64, device="cuda"), torch.zeros(M, N, dtype=torch.float64, device="cuda")
+        for b in range(K // 128):
+            xb, wb, sb = x[:, 128 * b:128 * b + 128].double(), w[:, 128 * b:128 * b + 128].double().t(), xs[:, b:b + 1].double() * ws[:, b].double().repeat_interleave(128)[:N]
+            want += (xb @ wb) * sb
+            size += (xb.abs() @ wb.abs()) * sb
+    else:
+        xs, ws = (torch.rand(M, device="cuda", generator=gen) + 1) * 0.05, (torch.rand(N, device="cuda", generator=gen) + 1) * 5e-4
+        want, size = ((a @ b.t()) * xs.double()[:, None] * ws.double() for a, b in ((x.double(), w.double()), (x.double().abs(), w.double().abs())))
+    if bias is not None:
+        want = want + bias.double()
+    for kslab in (True, False):
+        out = torch.full((M, N), float("nan"), device="cuda").to(dtype)
+        wk = rearrange.to_kslab(w) if kslab else w
+        if kind == 0:
+            _check(lib.mi355q_kcontig_gemm(_p(out), _p(x), _p(wk), _p(xs), _p(ws), _p(bias), 1, 128, M, K, N, DT[dtype], DT[dtype], int(kslab), _stream()))
+        else:
+            _check(_codes_gemm(lib, kind, out, x, wk, kslab, xs, ws, bias, M, N, K, dtype))
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    # one rounding to 16 bits, and matrix instructions that align 32 products and the running sum to the largest of them: at most 33 units of 2^-24 of
+    # what the magnitudes of all products add up to (at random a small part of that: the norms)
+    eps = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    err = (outs[0].double() - want).abs()
+    assert (err <= eps * want.abs() + (K / 32 * 33 * 2.0 ** -24) * size).all()
+    assert err.norm() <= 0.75 * eps * want.norm()              # (uniform rounding alone: eps / sqrt(3) at most)
+
+
+def test_what_is_not_covered_is_an_error():
+    lib = _lib.load()
+    takes = lib.mi355q_q8_quant_gemm_takes
+    assert not takes(INT8, TOKEN, 17, 4096, 128) and not takes(INT8, TOKEN, 5, 4096, 4096) and not takes(FP8, CHANNEL, 1, 4096, 4096)
+    assert not takes(FP8, TOKEN, 1, 4096 + 32, 4096) and not takes(INT8, TOKEN, 1, 4096, 4096 + 64) and not takes(0, TOKEN, 1, 4096, 4096)
+    x = torch.zeros(17 * 4096, dtype=torch.float16, device="cuda")
+    assert lib.mi355q_q8_quant_gemm(_p(x), _p(x), _p(x), None, _p(x), 1, None, INT8, TOKEN, 17, 128, 128, DT[x.dtype], _stream()) != 0
+    assert lib.mi355q_q8_quant_gemm(_p(x), _p(x) + 2, _p(x), None, _p(x), 1, None, INT8, TOKEN, 1, 128, 128, DT[x.dtype], _stream()) != 0

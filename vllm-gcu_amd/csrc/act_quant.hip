@@ -5,6 +5,7 @@
 // device int32 `valid_rows` so padded (graph-captured) batches skip dead rows
 // without a host synchronisation.
 #include "moe_align.h"
+#include "rows8.h"
 
 #include <algorithm>
 
@@ -15,14 +16,6 @@ namespace {
 template <int DT> struct E16 { typedef Elem<DT> T; };
 
 template <int DT>
-__device__ __forceinline__ void unpack8(const u4& v, float* f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = Elem<DT>::to_f32((uint16_t)(v[i] & 0xffffu));
-    f[2 * i + 1] = Elem<DT>::to_f32((uint16_t)(v[i] >> 16));
-  }
-}
-template <int DT>
 __device__ __forceinline__ u4 pack8(const float* f) {
   u4 v;
 #pragma unroll
@@ -30,19 +23,6 @@ __device__ __forceinline__ u4 pack8(const float* f) {
     v[i] = (uint32_t)Elem<DT>::from_f32(f[2 * i]) | ((uint32_t)Elem<DT>::from_f32(f[2 * i + 1]) << 16);
   return v;
 }
-// 8 floats (already within +-448) -> 8 e4m3fn codes, round to nearest even
-__device__ __forceinline__ u2 to_fp8x8(const float* y) {
-  u2 r;
-  int w0 = 0, w1 = 0;
-  w0 = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], w0, false);
-  w0 = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], w0, true);
-  w1 = __builtin_amdgcn_cvt_pk_fp8_f32(y[4], y[5], w1, false);
-  w1 = __builtin_amdgcn_cvt_pk_fp8_f32(y[6], y[7], w1, true);
-  r.x = (uint32_t)w0;
-  r.y = (uint32_t)w1;
-  return r;
-}
-
 // Rows of this launch that count: `rows` of them, or up to the device's row count (times rows per count) less the `row0` rows of
 // the launches before this one.
 __device__ __forceinline__ uint32_t live_rows(uint32_t rows, const int* valid_rows, int rpc, long row0) {
@@ -153,17 +133,15 @@ token_fp8_quant_row_kernel(uint8_t* out, float* scales, const uint16_t* x, int K
     for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(y[e]));
   }
   mx = block_max(mx, red);
-  const float s = fmaxf(mx, 1e-10f) / FP8_MAX;
-  if (threadIdx.x == 0) scales[row] = s;
-  const SharedDivisor by_s(s);
+  const RowFp8 q(mx);
+  if (threadIdx.x == 0) scales[row] = q.scale;
 #pragma unroll
   for (int i = 0; i < P; ++i) {
     const int c = threadIdx.x + nt * i;
     float y[8];
     unpack8<DT>(v[i], y);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = clamp448(by_s.div(y[e]));
-    if (c < chunks) *(u2*)(out + row * K + 8 * c) = to_fp8x8(y);
+    const u2 codes = q.codes(y);
+    if (c < chunks) *(u2*)(out + row * K + 8 * c) = codes;
   }
 }
 

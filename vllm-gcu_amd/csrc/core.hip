@@ -1,7 +1,7 @@
 // Library-wide state: thread-local error text, ABI version, device queries.
 #include "common.h"
 
-#include <mutex>
+#include <atomic>
 
 namespace mi355q {
 
@@ -14,19 +14,18 @@ void set_error(const char* fmt, ...) {
   va_end(ap);
 }
 
+// (asked several times on the way to a launch of a few microseconds: a look-up without a lock; two threads that find nothing store the same)
 int device_cu_count() {
-  static int cached[64];
-  static std::mutex mu;
+  static std::atomic<int> cached[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  std::lock_guard<std::mutex> lk(mu);
-  if (cached[dev] == 0) {
+  int cus = cached[dev].load(std::memory_order_relaxed);
+  if (cus == 0) {
     hipDeviceProp_t p;
-    cached[dev] = (hipGetDeviceProperties(&p, dev) == hipSuccess && p.multiProcessorCount > 0)
-                      ? p.multiProcessorCount
-                      : 256;
+    cus = (hipGetDeviceProperties(&p, dev) == hipSuccess && p.multiProcessorCount > 0) ? p.multiProcessorCount : 256;
+    cached[dev].store(cus, std::memory_order_relaxed);
   }
-  return cached[dev];
+  return cus;
 }
 
 }  // namespace mi355q

@@ -309,6 +309,13 @@ size_t int8_scratch(const Int8Mm& m, int64_t M, int64_t top, bool& mid) {
   return M <= int8_stream_rows(m.K, m.N, top) ? 0 : mi355q_w8a8_int8_workspace_bytes(M, m.N, m.K);
 }
 
+// Whether a call of a few rows goes to the kernel that quantises them itself (kind and quantiser of mi355q_q8_quant_gemm)
+bool quantises(int kind, int quant, int64_t M, int64_t N, int64_t K, const Tensor& x, const Tensor& c_scale, const Tensor& w, const Tensor& ws,
+               const Tensor& bias) {
+  const auto off = [](const Tensor& t, uintptr_t a) { return reinterpret_cast<uintptr_t>(ptr(t)) % a != 0; };
+  return M <= 16 && mi355q_q8_quant_gemm_takes(kind, quant, M, N, K) && !off(x, 16) && !off(c_scale, 16) && !off(w, 16) && !off(ws, 16) && !off(bias, 8);
+}
+
 // (layer, x, bias, top): quantise with the layer's per-channel in_scales, multiply with out_scales
 PyObject* py_w8a8_static_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
   HANDLE_TH_ERRORS
@@ -326,11 +333,17 @@ PyObject* py_w8a8_static_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
   const int64_t M = x.numel() / m.K;
   const OnDevice on(x);
   void* stream = on.stream();
-  bool mid;
-  const size_t need = int8_scratch(m, M, top, mid);
-  const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
   Tensor out;
-  {
+  if (m.out_dtype == x.scalar_type() && quantises(2, 2, M, m.N, m.K, x, *it, m.w, m.ws, m.bias)) {
+    const NoGil free_gil;
+    out = empty(with_last(x, m.N), m.out_dtype, x);
+    check(mi355q_q8_quant_gemm(out.data_ptr(), x.data_ptr(), m.w.data_ptr(), it->data_ptr(), static_cast<const float*>(m.ws.data_ptr()), 1,
+                               ptr(m.bias), 2, 2, M, m.N, m.K, dtype_code(m.out_dtype), stream),
+          "q8_quant_gemm");
+  } else {
+    bool mid;
+    const size_t need = int8_scratch(m, M, top, mid);
+    const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
     const NoGil free_gil;
     const Tensor q = empty({M, m.K}, at::kChar, x);
     out = empty(with_last(x, m.N), m.out_dtype, x);
@@ -359,11 +372,17 @@ PyObject* py_int8_dynamic_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
   const int64_t M = x.numel() / m.K;
   const OnDevice on(x);
   void* stream = on.stream();
-  bool mid;
-  const size_t need = int8_scratch(m, M, top, mid);
-  const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
   Tensor out;
-  {
+  if (quantises(2, 1, M, m.N, m.K, x, Tensor(), m.w, m.ws, m.bias)) {
+    const NoGil free_gil;
+    out = empty(with_last(x, m.N), m.out_dtype, x);
+    check(mi355q_q8_quant_gemm(out.data_ptr(), x.data_ptr(), m.w.data_ptr(), nullptr, static_cast<const float*>(m.ws.data_ptr()), 1, ptr(m.bias),
+                               2, 1, M, m.N, m.K, dtype_code(m.out_dtype), stream),
+          "q8_quant_gemm");
+  } else {
+    bool mid;
+    const size_t need = int8_scratch(m, M, top, mid);
+    const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
     const NoGil free_gil;
     const Tensor q = empty({M, m.K}, at::kChar, x), xs = empty({M}, at::kFloat, x);
     out = empty(with_last(x, m.N), m.out_dtype, x);
@@ -479,12 +498,18 @@ PyObject* py_fp8_scaled_layer(PyObject*, PyObject* const* a, Py_ssize_t) {
     return no();
   const OnDevice on(x);
   void* stream = on.stream();
-  size_t need = 0;
-  if (!mi355q_q8_mid_plan(1, M, N, K, &need)) need = mi355q_fp8_gemm_workspace_bytes(M, N, K);
-  const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
   const int dt = dtype_code(x.scalar_type());
   Tensor out;
-  {
+  if (!xs.defined() && quantises(1, 1, M, N, K, x, Tensor(), *wt, *st, bias)) {
+    const NoGil free_gil;
+    out = empty(with_last(x, N), x.scalar_type(), x);
+    check(mi355q_q8_quant_gemm(out.data_ptr(), x.data_ptr(), wt->data_ptr(), nullptr, static_cast<const float*>(st->data_ptr()), st->numel() > 1,
+                               ptr(bias), 1, 1, M, N, K, dt, stream),
+          "q8_quant_gemm");
+  } else {
+    size_t need = 0;
+    if (!mi355q_q8_mid_plan(1, M, N, K, &need)) need = mi355q_fp8_gemm_workspace_bytes(M, N, K);
+    const Scratch ws = need ? workspace(x, stream, need) : Scratch{nullptr, 0};
     const NoGil free_gil;
     const Tensor q = empty({M, K}, at::kFloat8_e4m3fn, x);
     const bool per_row = !xs.defined();

@@ -17,7 +17,7 @@
 // are read from LDS, and the copy of the tile after next is in flight.  The
 // weights take the A operand slot so that each lane ends up with 4 consecutive
 // output columns (one 8-byte store).
-#include "common.h"
+#include "rows8.h"
 
 #include <algorithm>
 
@@ -508,28 +508,6 @@ __device__ __forceinline__ float ld_half(uint16_t raw) {
   return Elem<DT == MI355Q_F32 ? MI355Q_F16 : DT>::to_f32(raw);
 }
 
-__device__ __forceinline__ int8_t sat_rne_s8(float y) {
-  y = __builtin_rintf(y);                       // round half to even
-  y = fminf(fmaxf(y, -128.0f), 127.0f);
-  return (int8_t)(int)y;
-}
-
-// the 8 values of a piece of 16-bit elements
-template <int DT>
-__device__ __forceinline__ void unpack_half8(const u4& v, float* f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[2 * i] = ld_half<DT>((uint16_t)(v[i] & 0xffffu));
-    f[2 * i + 1] = ld_half<DT>((uint16_t)(v[i] >> 16));
-  }
-}
-__device__ __forceinline__ u2 pack_s8x8(const float* y) {
-  uint32_t q[2] = {0u, 0u};
-#pragma unroll
-  for (int e = 0; e < 8; ++e) q[e >> 2] |= ((uint32_t)(uint8_t)sat_rne_s8(y[e])) << (8 * (e & 3));
-  return (u2){q[0], q[1]};
-}
-
 // one workgroup per token row: absmax -> scale = absmax / 127 -> q = rne(x * (127 / absmax)).  The row is read once,
 // P pieces of 16 bytes per lane with all loads in flight together, and quantised from registers: bound by HBM at
 // prefill sizes (the loop below reads every row twice, one piece at a time).
@@ -551,24 +529,20 @@ dynamic_int8_quant_row_kernel(int8_t* out, float* scales, const uint16_t* x, int
 #pragma unroll
   for (int i = 0; i < P; ++i) {
     float y[8];
-    unpack_half8<DT>(v[i], y);
+    unpack8<DT>(v[i], y);
 #pragma unroll
     for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(y[e]));
   }
   mx = block_max(mx, red);
-  if (threadIdx.x == 0) scales[row] = mx / 127.0f;
-  const float inv = 127.0f / mx;                // inf for an all-zero row
+  const RowInt8 q(mx);
+  if (threadIdx.x == 0) scales[row] = q.scale;
 #pragma unroll
   for (int i = 0; i < P; ++i) {
     const int c = threadIdx.x + nt * i;
     float y[8];
-    unpack_half8<DT>(v[i], y);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      y[e] *= inv;
-      if (y[e] != y[e]) y[e] = 0.f;             // 0 * inf
-    }
-    if (c < chunks) *(u2*)(out + row * K + 8 * c) = pack_s8x8(y);
+    unpack8<DT>(v[i], y);
+    const u2 codes = q.codes(y);
+    if (c < chunks) *(u2*)(out + row * K + 8 * c) = codes;
   }
 }
 
@@ -637,13 +611,11 @@ static_int8_quant_vec_kernel(int8_t* out, const uint16_t* x, const void* scale, 
 #pragma unroll
     for (int e = 0; e < 4; ++e) s[e] = a[e], s[4 + e] = b[e];
   } else {
-    unpack_half8<DT>(*(const u4*)((const uint16_t*)scale + 8 * c), s);
+    unpack8<DT>(*(const u4*)((const uint16_t*)scale + 8 * c), s);
   }
   float y[8];
-  unpack_half8<DT>(v, y);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) y[e] *= Elem<DT>::to_f32(Elem<DT>::from_f32(1.0f / s[e]));
-  *(u2*)(out + 8 * i) = pack_s8x8(y);
+  unpack8<DT>(v, y);
+  *(u2*)(out + 8 * i) = static_int8_codes<DT>(y, s);
 }
 
 template <int DT, int SDT>
