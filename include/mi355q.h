@@ -464,6 +464,17 @@ size_t mi355q_moe_w4a16_unsorted_sum_bytes(int numel, int E, int K, int N);
 int mi355q_moe_w4a16_unsorted_sum(void* out, const void* a, const int32_t* w, const void* w_scale, const void* w_zeros, int zeros_kind,
                                   int group_size, const float* topk_weights, const void* topk_ids, int ids_are_int64, int rows, int topk,
                                   int E, int K, int N, int dtype, void* workspace, size_t workspace_bytes, void* stream);
+/* No counterpart in the reference.  The fp8 experts of a few tokens -- both GEMMs, the gate and the sum over a token's slots -- from 16-bit rows x
+ * [M, K] and the router's ids [M, topk] (int32 or int64), without alignment and quantisers: kslab weights w1 [E, 2 I, K], w2 [E, K, I] with
+ * block scales f32 [E, 2 I / 128, K / 128], [E, K / 128, I / 128]; out [M, K] may be x.  Slots whose id is outside [0, E) add nothing.  Sums as
+ * mi355q_moe_fp8_gate_up_quant and mi355q_moe_gemm make them, K blocks in another order.  _bytes: of the workspace (any contents), 0 where a call is not
+ * covered (up to four tokens and 64 slots, K and I multiples of 128 up to 32768); _wanted: 1 where it is ahead of the sorted launches.
+ * Operands aligned to 16 bytes. */
+size_t mi355q_moe_fp8_unsorted_bytes(int M, int topk, int E, int K, int I);
+int mi355q_moe_fp8_unsorted_wanted(int M, int topk, int E, int K, int I);
+int mi355q_moe_fp8_unsorted(void* out, const void* x, const void* w1, const float* w1_scale, const void* w2, const float* w2_scale,
+                            const float* topk_weights, const void* topk_ids, int ids_are_int64, int M, int topk, int E, int K, int I,
+                            int dtype, void* workspace, size_t workspace_bytes, void* stream);
 /* mi355q_moe_gemm with quant_mode 1 whose columns are gate and up, and mi355q_fp8_group_quant with fuse_silu_mul over groups of 128 of its
  * result in act_dtype, in one launch and bit for bit: out e4m3fn [numel, N / 2], out_scales [numel, N / 256].  Blocks of 16, 32 or 64 slots,
  * N % 256 == 0. */

@@ -33,6 +33,10 @@ SIGNATURES = {
     "mi355q_w4a16_noalloc_scratch_bytes": (c_size_t, []),
     "mi355q_w4a16_gemm_noalloc": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                                           c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "mi355q_moe_fp8_unsorted_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "mi355q_moe_fp8_unsorted_wanted": (c_int, [c_int, c_int, c_int, c_int, c_int]),
+    "mi355q_moe_fp8_unsorted": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
+                                        c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "mi355q_q8_quant_gemm_takes": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "mi355q_q8_quant_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int,
                                      c_int, c_int, c_void_p]),

@@ -628,13 +628,30 @@ PyObject* py_fused_experts(PyObject*, PyObject* const* a, Py_ssize_t) {
     if (mode == kFp8 && group != 128) return no();
     if (mode == kInt8) group = 1;
   }
+  const bool ids64 = ids.scalar_type() == at::kLong;
+  if (mode == kFp8 && M <= 4 && mi355q_moe_fp8_unsorted_wanted(M, T, E, K, I)) {
+    const auto at16 = [](const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+    if (at16(x) && at16(out) && at16(w1) && at16(w2)) {
+      const size_t bytes = mi355q_moe_fp8_unsorted_bytes(M, T, E, K, I);
+      const OnDevice on(x);
+      {
+        const NoGil free_gil;
+        const Tensor buf = empty({static_cast<int64_t>(bytes)}, at::kByte, x);
+        check(mi355q_moe_fp8_unsorted(out.data_ptr(), x.data_ptr(), w1.data_ptr(), static_cast<const float*>(s1p->data_ptr()), w2.data_ptr(),
+                                      static_cast<const float*>(s2p->data_ptr()), static_cast<const float*>(tw.data_ptr()), ids.data_ptr(), ids64, M, T,
+                                      E, K, I, dtype_code(dt), buf.data_ptr(), bytes, on.stream()),
+              "moe_fp8_unsorted");
+      }
+      Py_RETURN_TRUE;
+    }
+  }
   const int64_t blocks = (numel + E * (block - 1)) / block;
   const bool quant = mode != kW4;
   // A wavefront's worth of slots in blocks of 16: the GEMMs sort them themselves, and the first applies the gate, where its launch counts:
   // sixty experts of 2048 x 2816 at 1 / 8 / 16 tokens 32.2 / 39.9 / 51.2 -> 29.5 / 37.8 / 49.3 us, sixteen of 3072 x 8192 at 3 / 16 39.2 / 63.7 ->
   // 36.7 / 62.7; eight of 4096 x 28672 at 1 / 5 / 16 48.6 / 103.2 / 132.5 and 47.5 / 104.1 / 132.4: two streams of weights instead of one.
   const bool unsorted = mode == kW4 && block == 16 && numel <= 64 && group % 128 == 0 && K % 128 == 0 && N % 128 == 0 && I % 128 == 0;
-  const bool gate = unsorted && N * K <= (1 << 26), ids64 = ids.scalar_type() == at::kLong;
+  const bool gate = unsorted && N * K <= (1 << 26);
   const bool sorted_gate = mode == kW4 && !unsorted && mi355q_moe_w4a16_gates(block, K, N, group, z1.defined() ? MI355Q_ZP_PACKED : MI355Q_ZP_NONE);
   const bool gate_up = mode == kFp8 && block <= 64 && N % 256 == 0;       // the first GEMM applies the gate and quantises
   // one allocation: quantised inputs of both GEMMs with their scales, the three intermediate matrices, the alignment

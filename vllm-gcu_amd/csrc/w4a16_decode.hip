@@ -14,7 +14,7 @@
 // Measured (us, graph replays, weights warm in the last-level cache / cold, the streaming kernel -> here, fp16, groups of 128): 4096 x 4096 at
 // 1 / 4 / 16 rows 5.0 / 5.6 / 5.6 -> 3.5 / 3.5 / 4.7 warm, 6.1 / 6.1 / 6.3 -> 4.0 / 4.1 / 5.4 cold; 4096 x 6144 at 1 / 16 6.0 / 6.2 -> 4.5 / 5.8 and
 // 6.7 / 6.9 -> 5.2 / 6.6; 8192 x 8192 at 1 / 8 9.5 / 9.9 -> 8.0 / 8.7 and 10.9 / 10.7 -> 8.4 / 9.2; 1024 x 1024 at 1 2.8 -> 2.3.
-#include "common.h"
+#include "moe_slots.h"
 
 #include <algorithm>
 #include <cmath>
@@ -289,30 +289,14 @@ w4a16_decode_grouped_kernel(DecodeArgs a) {
   long e;
   int real;                                          // slots up to the last that is no pad
   if constexpr (IDS) {
-    int mine = lane < a.numel ? a.sorted_ids[lane * a.id_step] : -1;
-    if (mine >= a.E) mine = -1;
-    unsigned long long same = __ballot(mine >= 0);
-    for (int b = 0; b < a.id_bits; ++b) {
-      const bool bit = (mine >> b) & 1;
-      const unsigned long long set = __ballot(bit);
-      same &= bit ? set : ~set;
-    }
-    const unsigned long long below = (1ull << lane) - 1ull;
-    const int slots = mine >= 0 ? __popcll(same) : 0, rank = __popcll(same & below);
-    int first = 0;                                   // block of the expert's first 16 slots
-#pragma unroll
-    for (int n = 0; n < 64; n += 16) first += __popcll(__ballot(rank == 0 && slots > n) & below);
-    const int z = (int)blockIdx.z;
-    const unsigned long long found = __ballot(mine >= 0 && rank == 0 && z >= first && z < first + (slots + 15) / 16);
-    if (!found) return;                              // (as every wavefront of the workgroup)
-    const int owner = __builtin_amdgcn_readfirstlane(__ffsll(found) - 1);
-    e = __builtin_amdgcn_readlane(mine, owner);
-    const int chunk = z - __builtin_amdgcn_readlane(first, owner);
-    real = min(16, __builtin_amdgcn_readlane(slots, owner) - 16 * chunk);
+    const SlotBlock b = find_slot_block<4>(a.sorted_ids, a.id_step, a.id_bits, a.numel, a.E, (int)blockIdx.z, lane);
+    if (!b.real) return;                             // (as every wavefront of the workgroup)
+    e = b.expert;
+    real = b.real;
     if (wave == 0) {
       if (lane < 16) block_ids[lane] = a.numel;
       __builtin_amdgcn_wave_barrier();
-      if (mine == (int)e && rank >> 4 == chunk) block_ids[rank & 15] = lane;
+      if (holds_lane<4>(b)) block_ids[b.rank & 15] = lane;
     }
     __syncthreads();
   } else {
