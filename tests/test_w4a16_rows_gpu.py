@@ -60,6 +60,20 @@ def test_tiles(mt, nt, K, N, g, splits, dtype, monkeypatch):
     assert torch.equal(_run(q, z, s, x, g, **kw), torch.from_numpy(_want(q, z, s, x, g)).to(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("g", [128, 32])
+@pytest.mark.parametrize("mt,nt", [(2, 1), (3, 1), (2, 2)])
+def test_one_and_two_workgroups_per_cu(mt, nt, g, dtype):
+    """The tiles that fit twice on a CU have a ring for it and another for a launch of no more workgroups than CUs (test_tiles' are all of those): on both
+    sides of the line, with fewer K blocks than either ring has stages and with more."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for K, tiles in ((128, cus), (128, cus + 2), (1152, cus), (1152, cus + 2)):
+        M, N = 16 * mt - 3, tiles * 64 * nt
+        print(f"case w4a16 rows {16 * mt}x{64 * nt} M={M} K={K} N={N} g={g} {dtype}", flush=True)
+        q, z, s, x = _case(K + mt, M, K, N, g, dtype, exact=True)
+        assert torch.equal(_run(q, z, s, x, g, family=4, split_k=1 | mt << 8 | nt << 16), torch.from_numpy(_want(q, z, s, x, g)).to(dtype))
+
+
 @pytest.mark.parametrize("M,K,N,g", [(5, 1024, 1024, 64), (20, 4096, 16384, 128), (24, 2048, 512, 32), (33, 1024, 128, 128),
                                      (48, 4096, 1024, 128), (64, 2048, 4096, 128), (65, 3584, 512, 128), (96, 1024, 14336, 128),
                                      (130, 2048, 1024, 64), (333, 1024, 2048, 128), (700, 1024, 1024, 128), (4095, 512, 128, 128),

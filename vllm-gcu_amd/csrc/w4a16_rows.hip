@@ -24,6 +24,9 @@
 // Measured (us, fp16, groups of 128, weights cold; before -> here): 4096 x 4096 at 48 / 96 / 192 rows 12.0 / 15.5 / 23.1 ->
 // 9.1 / 9.4 / 12.2; 4096 x 6144 at 64 / 128 / 256 15.9 / 20.5 / 28.2 -> 9.5 / 13.2 / 18.6; 4096 x 28672 at 48 / 64 / 96
 // 29.9 / 32.7 / 41.7 -> 20.3 / 23.2 / 29.1; 14336 x 4096 at 48 / 96 / 192 20.3 / 27.5 / 39.0 -> 16.3 / 21.9 / 31.7.
+// A workgroup without another one on its CU takes a ring of three stages in place of two, and the tiles up to 128 rows are priced for it (before -> since):
+// 4096 x 6144 at 96 15.4 -> 11.9; 8192 x 8192 at 40 / 96 18.1 / 29.8 -> 16.1 / 21.8; 4096 x 12288 at 48 16.1 -> 12.9; 5120 x 13824 at 40 19.7 -> 15.5;
+// 11008 x 4096 at 48 / 112 16.5 / 21.8 -> 14.3 / 23.4; 4096 x 28672 at 24 19.4 -> 17.1; bf16 8192 x 8192 at 48 / 96 21.2 / 29.9 -> 18.1 / 25.0.
 #include "common.h"
 
 #include <algorithm>
@@ -99,7 +102,8 @@ template <> struct RowsMma<MI355Q_BF16> {
 // 16 MT rows x 64 NT columns; KS = 2 K ranges with NW wavefronts that compute and two that copy, and a ring of LDS stages,
 // each.  GPB: quantisation groups per K block (1 for group sizes that are multiples of 128, 2 / 4 for 64 / 32).  GLU: half of the
 // columns are gate and half the up columns that go with them, with the scales and zero-points of both slabs in a stage.
-template <int MT_, int NT_, int GPB_, int ZK, bool GLU_ = false>
+// LONE: the ring of a workgroup that has its CU for itself.
+template <int MT_, int NT_, int GPB_, int ZK, bool GLU_ = false, bool LONE_ = false>
 struct RowsCfg {
   static constexpr bool GLU = GLU_;
   static_assert(!GLU || (NT_ == 2 && GPB_ == 1), "64 and 64 columns, one group");
@@ -109,9 +113,11 @@ struct RowsCfg {
                        S_BYTES = 256 * GPB * HV, Z_BYTES = (ZK == MI355Q_ZP_PRESCALED ? 256 : 64) * GPB * HV;
   static constexpr int W_OFF = A_BYTES, S_OFF = W_OFF + W_BYTES, Z_OFF = S_OFF + S_BYTES, STAGE = Z_OFF + Z_BYTES;
   static constexpr int XC = A_BYTES / 2048, WC = NW * NT / 2, NC = XC + WC + 1;   // copies of a copying wavefront per stage
-  // two workgroups per CU where two stages fit so (deeper rings did not gain: the copies are bound by their rate)
-  static constexpr int PAIR = 2 * KS * STAGE <= 80 * 1024 ? 1 : 0, ROOM = (PAIR ? 80 : 159) * 1024 / (KS * STAGE);
-  static constexpr int D = ROOM < 4 ? ROOM : 4, RING = D * STAGE;
+  // two workgroups per CU where two stages fit so.  (With two workgroups deeper rings did not gain: the copies are bound by their rate.  One alone has a stage
+  // of each range on its way then, and gains by another, but not by a third)
+  static constexpr int MOST = LONE_ ? 3 : 4;
+  static constexpr int PAIR = !LONE_ && 2 * KS * STAGE <= 80 * 1024 ? 1 : 0, ROOM = (PAIR ? 80 : 159) * 1024 / (KS * STAGE);
+  static constexpr int D = ROOM < MOST ? ROOM : MOST, RING = D * STAGE;
   static_assert(XC * 2048 == A_BYTES && WC * 2 == NW * NT && WC <= 4 && D >= 2, "whole copies, a ring");
   static_assert((D - 1) * NC < 64, "copies in flight that the wait can count");
 };
@@ -423,27 +429,49 @@ int launch_rows(RowsArgs a, int splits, const void* bias, int dtype, hipStream_t
 
 template <int DT, int ZK, int GPB>
 int launch_rows_cfg(const RowsArgs& a, int mt, int nt, int splits, const void* bias, int dtype, hipStream_t st) {
-#define MQ_CFG(MT, NT) if (mt == MT && nt == NT) return launch_rows<DT, ZK, RowsCfg<MT, NT, GPB, ZK>>(a, splits, bias, dtype, st)
-  MQ_CFG(2, 1); MQ_CFG(3, 1); MQ_CFG(4, 1);
-  MQ_CFG(2, 2); MQ_CFG(3, 2); MQ_CFG(4, 2); MQ_CFG(5, 2); MQ_CFG(6, 2);
+  // no more workgroups than CUs: LONE, but for 32 x 128 with bf16, whose arithmetic fills the wait (us, there / here: 4096 x 28672 at 20 rows 17.5 / 18.7, 14336 x 8192 at 18
+  // 21.4 / 22.0, 3584 x 18944 at 24 16.6 / 17.0; only 8192 x 28672 and 5120 x 27648 below 21 rows gain, 37.9 / 34.7)
+  const bool lone = (long)((a.M + 16 * mt - 1) / (16 * mt)) * (a.N / (64 * nt)) * splits <= device_cu_count();
+#define MQ_CFG(MT, NT)                                                                                                                  \
+  if (mt == MT && nt == NT) {                                                                                                           \
+    if constexpr (RowsCfg<MT, NT, GPB, ZK>::PAIR && (NT == 1 || DT == MI355Q_F16))                                                      \
+      if (lone) return launch_rows<DT, ZK, RowsCfg<MT, NT, GPB, ZK, false, true>>(a, splits, bias, dtype, st);                          \
+    return launch_rows<DT, ZK, RowsCfg<MT, NT, GPB, ZK>>(a, splits, bias, dtype, st);                                                   \
+  }
+  MQ_CFG(2, 1) MQ_CFG(3, 1) MQ_CFG(4, 1)
+  MQ_CFG(2, 2) MQ_CFG(3, 2) MQ_CFG(4, 2) MQ_CFG(5, 2) MQ_CFG(6, 2)
 #undef MQ_CFG
   MQ_REQUIRE(false, "w4a16_gemm(rows): no tile of %d x %d", 16 * mt, 64 * nt);
 }
 
 // ---- the choice of tile and K split: the cheapest by a price model in microseconds.  Per tile: a K block of each of its two
-// ranges, for a workgroup alone on its CU and added for a second one beside it (tiles of 64 columns and 32 x 128 fit two).
-// Fitted to 3400 measurements (15 layer shapes, 20..2048 rows, 1..12 ranges, weights cold in the caches; rms error 5 %); the tile
-// taken by it is within 2 % of the best one on average over those points.
+// ranges, for a workgroup with its CU for itself (`lone`, where that is another ring than that of two), else for the first one on its CU and added for a
+// second one beside it (tiles of 64 columns and 32 x 128 fit two).  Above 128 rows, where the other kernels' prices are compared with this one: fitted to 3400
+// measurements (15 layer shapes, 20..2048 rows, 1..12 ranges, weights cold in the caches; rms error 5 %), without rings of their own for lone workgroups.  Up to
+// 128 rows: to the launches of 42 layers with each type (18 .. 128 rows, up to eight ranges, cold weights; rms errors 6 and 5 %); the tile taken by it loses 0.5 / 0.3 %
+// (fp16 / bf16) to the best one on average, and 14 / 10 % at worst (by the prices above 128 rows 1.0 / 1.8 %, and 18 / 25 %).
 struct RowsPrice {
   int mt, nt;
-  double one, more;
+  double one, more, lone;
 };
-constexpr RowsPrice kRows[] = {{2, 1, 0.422, 0.388}, {3, 1, 0.600, 0.500}, {4, 1, 0.700, 0}, {2, 2, 0.773, 0.594},
-                               {3, 2, 0.956, 0},     {4, 2, 1.173, 0},     {5, 2, 1.333, 0}, {6, 2, 1.555, 0}};
-constexpr double kRowsBase = 3.57, kRowsRound = 1.10, kRowsSplit = 2.18, kRowsSplitMN = 1.56;
-constexpr double kRowsAlone = 0.283;        // share of a step that goes away as the chip empties (the caches and memory are shared)
-constexpr double kRowsSecond = 0.388;       // share of the second workgroup's price that grows with how many CUs hold two
-constexpr double kRowsStream = 4.23e6;      // bytes of weights per microsecond
+struct RowsModel {
+  RowsPrice tiles[8];
+  double base, round, split, split_mn;
+  double alone;               // share of a step that goes away as the chip empties (the caches and memory are shared)
+  double second;              // share of the second workgroup's price that grows with how many CUs hold two
+  double stream;              // bytes of weights per microsecond
+};
+constexpr RowsModel kRows[3] = {
+    {{{2, 1, 0.422, 0.388, 0.422}, {3, 1, 0.600, 0.500, 0.600}, {4, 1, 0.700, 0, 0}, {2, 2, 0.773, 0.594, 0.773},
+      {3, 2, 0.956, 0, 0}, {4, 2, 1.173, 0, 0}, {5, 2, 1.333, 0, 0}, {6, 2, 1.555, 0, 0}},
+     3.57, 1.10, 2.18, 1.56, 0.283, 0.388, 4.23e6},
+    {{{2, 1, 0.344, 0.544, 0.436}, {3, 1, 0.866, 0.413, 0.554}, {4, 1, 0.757, 0, 0}, {2, 2, 0.587, 0.911, 0.780},
+      {3, 2, 0.982, 0, 0}, {4, 2, 1.253, 0, 0}, {5, 2, 1.414, 0, 0}, {6, 2, 1.605, 0, 0}},
+     3.29, 1.44, 1.66, 2.11, 0.199, 0.236, 4.71e6},
+    {{{2, 1, 0.464, 0.522, 0.511}, {3, 1, 0.605, 0.541, 0.640}, {4, 1, 0.750, 0, 0}, {2, 2, 0.597, 1.143, 0.908},
+      {3, 2, 1.137, 0, 0}, {4, 2, 1.258, 0, 0}, {5, 2, 1.519, 0, 0}, {6, 2, 1.599, 0, 0}},
+     4.05, 1.45, 1.79, 1.95, 0.155, 0.149, 4.04e6}};
+const RowsModel& rows_model(int M, bool bf16) { return kRows[M > 128 ? 0 : bf16 ? 2 : 1]; }
 
 struct RowsPlan {
   int mt, nt, splits;
@@ -451,12 +479,12 @@ struct RowsPlan {
   double price;
 };
 
-RowsPlan rows_make_plan(int M, int K, int N, bool split) {
+RowsPlan rows_make_plan(const RowsModel& m, int M, int K, int N, bool split) {
   RowsPlan best = {0, 0, 1, 0, 1e30};
   const int KB = K / 128;
   const long cus = device_cu_count();
-  const double stream = std::pow((double)K * N / 2 / kRowsStream, 4);
-  for (const RowsPrice& p : kRows) {
+  const double stream = std::pow((double)K * N / 2 / m.stream, 4);
+  for (const RowsPrice& p : m.tiles) {
     const int bm = 16 * p.mt, bn = 64 * p.nt;
     if (p.mt > 2 && M <= bm - 16) continue;
     const long tiles = (long)((M + bm - 1) / bm) * (N / bn), res = p.more > 0 ? 2 : 1;
@@ -466,18 +494,28 @@ RowsPlan rows_make_plan(int M, int K, int N, bool split) {
       const size_t bytes = s > 1 ? (size_t)s * M * N * 4 : 0;
       if (bytes > ((size_t)31 << 20)) continue;       // (fits the fixed scratch of callers that cannot allocate, too)
       const long full = tiles * s / (res * cus), rest = tiles * s % (res * cus);
+      const double one = p.lone > 0 && tiles * s <= cus ? p.lone : p.one;
       double steps = full * (p.one + p.more * (res - 1));
-      if (rest) steps += p.one * (1 - kRowsAlone * (1 - (double)std::min(rest, cus) / cus));
-      if (rest > cus) steps += p.more * ((double)(rest - cus) / cus * kRowsSecond + 1 - kRowsSecond);
-      double t = std::sqrt(std::sqrt(std::pow(steps * ((kper + 1) / 2), 4) + stream)) + kRowsBase + kRowsRound * (full + (rest > 0) - 1);
-      if (s > 1) t += kRowsSplit + kRowsSplitMN * 1e-6 * s * M * N;
+      if (rest) steps += one * (1 - m.alone * (1 - (double)std::min(rest, cus) / cus));
+      if (rest > cus) steps += p.more * ((double)(rest - cus) / cus * m.second + 1 - m.second);
+      double t = std::sqrt(std::sqrt(std::pow(steps * ((kper + 1) / 2), 4) + stream)) + m.base + m.round * (full + (rest > 0) - 1);
+      if (s > 1) t += m.split + m.split_mn * 1e-6 * s * M * N;
       if (t < best.price) best = {p.mt, p.nt, s, bytes, t};
     }
   }
   return best;
 }
 
-RowsPlan rows_plan(int M, int K, int N) { return cached_plan(0, M, N, K, [](int, int M, int N, int K) { return rows_make_plan(M, K, N, true); }); }
+// of fp16 and of bf16 (together: whoever sizes a workspace asks for both)
+struct RowsPlans {
+  RowsPlan of[2];
+};
+RowsPlans rows_plans(int M, int K, int N) {
+  return cached_plan(0, M, N, K, [](int, int M, int N, int K) {
+    const RowsPlan f16 = rows_make_plan(rows_model(M, false), M, K, N, true);
+    return RowsPlans{{f16, M > 128 ? f16 : rows_make_plan(rows_model(M, true), M, K, N, true)}};
+  });
+}
 
 template <int DT, int ZK, int GPB, int MAX, bool GLU = false>
 int launch_rows_grouped(const RowsArgs& a, int max_blocks, hipStream_t st) {
@@ -494,16 +532,17 @@ int launch_rows_grouped(const RowsArgs& a, int max_blocks, hipStream_t st) {
 
 }  // namespace
 
-double w4a16_rows_price(int M, int K, int N) { return rows_plan(M, K, N).price; }
+double w4a16_rows_price(int M, int K, int N) { return rows_plans(M, K, N).of[0].price; }
 double w4a16_wide_price(int M, int K, int N, int group_size, int zeros_kind, bool bf16);     // us of the 64-row tiles and the ring kernels
 
 // Whether this kernel is the one to take.
 //  - Up to 16 rows: the streaming kernel, except for groups of 64 and 32 on small layers, where four scale rows per K block
 //    keep it from its rate (4096 x 4096, groups of 64, 1 / 16 rows: 9.1 / 10.2 -> 7.8 / 8.3 us, 2048 x 2048 8.3 / 8.7 -> 6.5 / 6.7;
 //    4096 x 28672, bf16: 16.2 against 19.8).
-//  - 17..32 rows: there the streaming kernel takes two row tiles and stays ahead on groups of 128 while the layer is small
-//    (4096 x 6144, 20 / 28 rows: 8.9 / 9.3 against 9.6 / 9.9 us; 14336 x 4096 14.3 against 14.5; but 4096 x 28672 21.3 -> 18.8, 18944 x
-//    3584 16.8 -> 15.0, 8192 x 8192 15.2 -> 14.7; bf16, whose operands cost more here, from 100 million weights on).
+//  - 17..32 rows: there the streaming kernel takes two row tiles and stays ahead on groups of 128 while the layer is small in both directions (us at 24 rows, fp16,
+//    there / here: 4096 x 6144 8.8 / 9.3, 2048 x 7168 6.0 / 6.5, 4096 x 4096 8.3 / 8.2; from 8192 columns 1408 x 19328 10.3 / 8.2, 4096 x 12288 11.8 / 11.0, 2560 x 8960
+//    8.3 / 7.7; from K 5120 6144 x 2048 8.6 / 7.6, 14336 x 4096 14.7 / 13.3, 5248 x 3840 8.9 / 8.7), and with bf16, whose operands cost more here, up to 100 million
+//    weights or 16384 columns (4096 x 12288 11.9 / 12.5, 14336 x 4096 14.3 / 14.5; 2432 x 18944 14.6 / 13.5).
 //  - Pre-scaled zero-points up to 64 rows: the streaming kernel, which uses z * s as it is.
 //  - To 128 rows: always.  Above: where its price is below that of the kernels with larger tiles, which read and dequantise the
 //    weights fewer times, as those operands run there.
@@ -514,7 +553,7 @@ bool w4a16_rows_wanted(int M, int K, int N, int group_size, int zeros_kind, int 
   if (M > 4096 || (size_t)M * K * 2 >= ((size_t)1 << 32)) return false;
   if (zeros_kind == MI355Q_ZP_PRESCALED && M <= 64) return false;
   if (M <= 16) return small && w <= (1L << 25);
-  if (M <= 32) return small || w >= (dtype == MI355Q_F16 ? 1L << 26 : 3L << 25);
+  if (M <= 32) return small || (dtype == MI355Q_F16 ? N >= 8192 || K >= 5120 : N >= 16384 || w >= 3L << 25);
   if (M <= 128) return true;
   // (the price, corrected for the size of the output and the rows by 255 launches with fp16 rows and 177 with bf16, rms errors 4.6 and 3 %.  The
   // pick loses 0.1 / 0.2 % (fp16 / bf16) to the best of the three kernels over 23 layers at 144 .. 2048 rows, 15 % at worst, where prices
@@ -526,15 +565,21 @@ bool w4a16_rows_wanted(int M, int K, int N, int group_size, int zeros_kind, int 
   return corrected < w4a16_wide_price(M, K, N, group_size, zeros_kind, bf16);
 }
 
-size_t w4a16_rows_workspace_bytes(int M, int K, int N) { return M <= 4096 ? rows_plan(M, K, N).bytes : 0; }
+// (of either type)
+size_t w4a16_rows_workspace_bytes(int M, int K, int N) {
+  if (M > 4096) return 0;
+  const RowsPlans p = rows_plans(M, K, N);
+  return std::max(p.of[0].bytes, p.of[1].bytes);
+}
 
 // mt 0: the plan, unsplit where the workspace does not hold the partial sums; else 16 mt rows x 64 nt columns, K in `splits` ranges
 int w4a16_rows_launch(void* out, const void* x, const int32_t* qweight, const void* scales, const void* zeros, int zeros_kind,
                       const void* bias, int M, int K, int N, int group_size, int dtype, void* workspace, size_t workspace_bytes,
                       int mt, int nt, int splits, hipStream_t st) {
   if (!mt) {
-    RowsPlan p = rows_plan(M, K, N);
-    if (p.bytes > (workspace ? workspace_bytes : 0)) p = rows_make_plan(M, K, N, false);
+    const bool bf16 = dtype == MI355Q_BF16;
+    RowsPlan p = rows_plans(M, K, N).of[bf16];
+    if (p.bytes > (workspace ? workspace_bytes : 0)) p = rows_make_plan(rows_model(M, bf16), M, K, N, false);
     mt = p.mt;
     nt = p.nt;
     splits = p.splits;
