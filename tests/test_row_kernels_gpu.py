@@ -78,3 +78,53 @@ def test_silu_and_sum_index_arithmetic(rows, d):
         g = out.float().view(rows, d // 128, 128)
         assert torch.equal(s, over(g.abs().amax(-1).clamp_min(1e-10), 448.0))
         assert torch.equal(q.view(torch.uint8), (g / s[..., None]).clamp(-448, 448).view(rows, d).to(torch.float8_e4m3fn).view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_group_fp8_codes_of_every_pair(dtype):
+    """Every value against every largest magnitude of its group's binade that there is (the division depends on the fractions alone): the code is that of
+    the IEEE quotient.  An infinity in the group makes zeros of the rest, with their signs."""
+    bits = 10 if dtype == torch.float16 else 7
+    one = 0x3C00 if dtype == torch.float16 else 0x3F80
+    print(f"case group fp8 codes of every pair {dtype}", flush=True)
+    n = 1 << bits
+    small = torch.arange(-10 * n, n, device="cuda") + one                  # ten binades below and that of the largest
+    small = torch.where(small % 2 == 1, small | 0x8000, small)
+    for m0 in range(0, n, 256):
+        mx = torch.arange(m0, min(m0 + 256, n), device="cuda") + one
+        groups = (small.numel() + 126) // 127
+        x = torch.zeros(mx.numel(), groups, 128, dtype=torch.int32, device="cuda")
+        x[:, :, 1:] = torch.nn.functional.pad(small, (0, groups * 127 - small.numel())).view(groups, 127)
+        x[:, :, 1:] = torch.where((x[:, :, 1:] & 0x7FFF) > mx[:, None, None], mx[:, None, None].int(), x[:, :, 1:])
+        x[:, :, 0] = mx[:, None]
+        x = x.to(torch.int16).view(dtype).view(mx.numel(), -1)
+        q, s = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device="cuda"), torch.empty(mx.numel(), groups, device="cuda")
+        torch.ops._C.dynamic_per_token_group_fp8_quant(q, s, x, 128)
+        assert torch.equal(s, over(x.view(mx.numel(), groups, 128)[:, :, 0].float(), 448.0))
+        want = (x.float().view(mx.numel(), groups, 128) / s[:, :, None]).clamp(-448, 448).to(torch.float8_e4m3fn)
+        assert torch.equal(q.view(torch.uint8), want.view(torch.uint8).view(q.shape))
+    x = torch.randn(1, 128, device="cuda").to(dtype)
+    x[0, 5], x[0, 7] = float("inf"), -0.0
+    q, s = torch.empty(1, 128, dtype=torch.float8_e4m3fn, device="cuda"), torch.empty(1, 1, device="cuda")
+    torch.ops._C.dynamic_per_token_group_fp8_quant(q, s, x, 128)
+    rest = torch.arange(128, device="cuda") != 5
+    assert s.isinf().all() and torch.equal(q.view(torch.uint8)[0, rest], (torch.signbit(x[0, rest]).to(torch.uint8) * 128))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_silu_of_every_gate(dtype):
+    """Every gate there is, also those whose sigmoid is no normal number, against the product in 64 bits: half a unit of the type's last place, and 2^-20
+    for the exponential, the reciprocal and the products in fp32; the smallest step of the type; and where the exponential is beyond fp32, 2^128 and more, a
+    sigmoid of 0 in place of up to 2^-128."""
+    print(f"case silu of every gate {dtype}", flush=True)
+    gate = torch.arange(65536, device="cuda").to(torch.int32).to(torch.int16).view(dtype)
+    gate = gate[gate.float().isfinite()].view(1, -1)
+    gate = gate[:, :gate.numel() // 8 * 8]
+    x = torch.cat([gate, torch.ones_like(gate)], dim=1).contiguous()
+    y = torch.empty_like(gate)
+    torch.ops._C.silu_and_mul(y, x)
+    a = gate.double()
+    want = a / (1 + torch.exp(-a))
+    digits, least = (11, 2.0 ** -24) if dtype == torch.float16 else (8, 2.0 ** -126)
+    bound = want.abs() * (2.0 ** -digits + 2.0 ** -20) + least + a.abs() * 2.0 ** -128
+    assert ((y.double() - want).abs() <= bound).all()

@@ -1,7 +1,10 @@
 // Elementwise glue between the GEMMs: SiLU-gate, fp8-e4m3fn activation
 // quantisers (per token group, per token, static), the fused SiLU-gate + group
-// quantiser, and the top-k sum.  All are HBM-bound: 16-byte loads per lane,
-// fp32 arithmetic, one pass over the data.  Every kernel takes an optional
+// quantiser, and the top-k sum: 16-byte loads per lane,
+// fp32 arithmetic, one pass over the data.  The sum, the plain gate and the per-token quantisers are HBM-bound; norm and gate with group codes were bound by
+// their instructions (33 and 61 per element), of which conversions in pairs, a maximum and a division of three instructions each and a reciprocal of
+// as many are left (us, bf16, rows 1537 / 4096 x 7168: norm + codes 11.5 / 24.4 -> 9.9 / 20.4, gate + codes 15.9 / 36.5 -> 11.7 / 28.1, codes alone
+// 7.0 / 16.1 -> 6.2 / 14.9).  Every kernel takes an optional
 // device int32 `valid_rows` so padded (graph-captured) batches skip dead rows
 // without a host synchronisation.
 #include "moe_align.h"
@@ -42,8 +45,7 @@ silu_and_mul_kernel(uint16_t* out, const uint16_t* x, uint32_t rows, int d, Fast
     float a[8], b[8], y[8];
     unpack8<DT>(*(const u4*)xr, a);
     unpack8<DT>(*(const u4*)(xr + d), b);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = silu_mul(a[e], b[e]);
+    silu_mul8(a, b, y);
     *(u4*)(out + (size_t)r * d + 8 * c) = pack8<DT>(y);
   }
 }
@@ -65,14 +67,15 @@ __device__ __forceinline__ void group_fp8_quant(uint8_t* out, float* scales, con
       unpack8<DT>(*(const u4*)xr, a);
       unpack8<DT>(*(const u4*)(xr + K), b);
       // the unfused sequence stores the gate output in the activation dtype
+      silu_mul8(a, b, y);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = round_act<DT>(silu_mul(a[e], b[e]));
+      for (int e = 0; e < 8; e += 2) round_act2<DT>(y[e], y[e + 1]);
     } else {
       unpack8<DT>(*(const u4*)(x + (size_t)r * K + 8 * c), y);
     }
     float mx = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(y[e]));
+    for (int e = 0; e < 8; e += 2) mx = SILU ? max_abs2(mx, y[e], y[e + 1]) : fmaxf(fmaxf(mx, fabsf(y[e])), fabsf(y[e + 1]));
     if (!live) mx = 0.f;
     mx = lane_group_max(mx, lpg);
     const float s = fmaxf(mx, 1e-10f) / FP8_MAX;
@@ -338,15 +341,10 @@ rms_norm_kernel(void* out, float* out_scales, const uint16_t* x, uint16_t* resid
         if ((c % lpg) == 0) out_scales[row * (K / gs) + c / lpg] = sg;
       }
     } else {
-      uint32_t lo = 0, hi = 0;
+      float q[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float a = fminf(fmaxf(__builtin_rintf(v[e] * qs), -128.f), 127.f);
-        float b = fminf(fmaxf(__builtin_rintf(v[4 + e] * qs), -128.f), 127.f);
-        lo |= ((uint32_t)(int)a & 0xffu) << (8 * e);
-        hi |= ((uint32_t)(int)b & 0xffu) << (8 * e);
-      }
-      if (live) *(u2*)((uint8_t*)out + row * K + 8 * c) = (u2){lo, hi};
+      for (int e = 0; e < 8; ++e) q[e] = v[e] * qs;
+      if (live) *(u2*)((uint8_t*)out + row * K + 8 * c) = pack_s8x8(q);
     }
   }
 }
@@ -408,7 +406,12 @@ rms_norm_row_kernel(void* out, float* out_scales, const uint16_t* x, uint16_t* r
     unpack8<DT>(xv[i], y);
     unpack8<DT>(wv[i], w);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = round_act<DT>(round_act<DT>(y[e] * rs) * w[e]);
+    for (int e = 0; e < 8; e += 2) {
+      y[e] *= rs, y[e + 1] *= rs;
+      round_act2<DT>(y[e], y[e + 1]);
+      y[e] *= w[e], y[e + 1] *= w[e + 1];
+      round_act2<DT>(y[e], y[e + 1]);
+    }
     if (QM == 0) {
       if (live[i]) *(u4*)((uint16_t*)out + row * K + 8 * c) = pack8<DT>(y);
     } else if (QM == 1) {
@@ -419,7 +422,7 @@ rms_norm_row_kernel(void* out, float* out_scales, const uint16_t* x, uint16_t* r
     } else if (QM == 2) {
       float mx = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(y[e]));
+      for (int e = 0; e < 8; e += 2) mx = max_abs2(mx, y[e], y[e + 1]);
       if (!live[i]) mx = 0.f;
       mx = lane_group_max(mx, lpg);
       const float sg = fmaxf(mx, 1e-10f) / FP8_MAX;
@@ -432,15 +435,10 @@ rms_norm_row_kernel(void* out, float* out_scales, const uint16_t* x, uint16_t* r
         if ((c & (lpg - 1)) == 0) out_scales[(row * chunks + c) >> (31 - __clz(lpg))] = sg;
       }
     } else {
-      uint32_t lo = 0, hi = 0;
+      float q[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float a = fminf(fmaxf(__builtin_rintf(y[e] * qs), -128.f), 127.f);
-        float b = fminf(fmaxf(__builtin_rintf(y[4 + e] * qs), -128.f), 127.f);
-        lo |= ((uint32_t)(int)a & 0xffu) << (8 * e);
-        hi |= ((uint32_t)(int)b & 0xffu) << (8 * e);
-      }
-      if (live[i]) *(u2*)((uint8_t*)out + row * K + 8 * c) = (u2){lo, hi};
+      for (int e = 0; e < 8; ++e) q[e] = y[e] * qs;
+      if (live[i]) *(u2*)((uint8_t*)out + row * K + 8 * c) = pack_s8x8(q);
     }
   }
 }

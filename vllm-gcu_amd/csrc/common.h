@@ -200,18 +200,19 @@ __device__ __forceinline__ float wave_sum(float x) {
   MQ_DPP_REDUCE(v, 0, op_fadd_bits);
   return __int_as_float(v);
 }
-// max over aligned groups of `lanes` lanes (a power of two, 2 .. 64), the result in every lane of the
+// max of values of at least 0 (no NaN) over aligned groups of `lanes` lanes (a power of two, 2 .. 64), the result in every lane of the
 // group: swaps inside quads, mirrors of the half row and of the row of 16 lanes, LDS shuffles only
-// for what crosses rows
+// for what crosses rows.  (As integers, which order such floats alike: an instruction a step.)
 __device__ __forceinline__ float lane_group_max(float x, int lanes) {
   int v = __float_as_int(x);
-  if (lanes >= 2) v = op_fmax_bits(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));    // quad_perm [1,0,3,2]
-  if (lanes >= 4) v = op_fmax_bits(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));    // quad_perm [2,3,0,1]
-  if (lanes >= 8) v = op_fmax_bits(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false));   // row_half_mirror
-  if (lanes >= 16) v = op_fmax_bits(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false));  // row_mirror
-  float m = __int_as_float(v);
-  for (int o = 16; o < lanes; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
-  return m;
+  if (lanes >= 2) v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));             // quad_perm [1,0,3,2]
+  if (lanes >= 4) v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));             // quad_perm [2,3,0,1]
+  if (lanes >= 8) v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false));            // row_half_mirror
+  if (lanes >= 16) {
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false));                          // row_mirror
+    for (int o = 16; o < lanes; o <<= 1) v = max(v, __shfl_xor(v, o));
+  }
+  return __int_as_float(v);
 }
 
 // Fused-MoE grouped GEMMs: a block whose expert id lies outside [0, E) -- a non-local expert under an
@@ -245,6 +246,29 @@ __device__ __forceinline__ float silu_mul(float a, float b) {
   return a * (1.0f / (1.0f + expf(-a))) * b;      // left * sigmoid(left) * right
 }
 
+// ... of eight of each, to the same bits.  An estimate and its Newton step are the correctly rounded reciprocal of every float from 1 to 2^126 (all of them were
+// compared with the division, which takes ten instructions for these three); gates below -87, whose reciprocal is no normal number, take the division.
+__device__ __forceinline__ void silu_mul8(const float* a, const float* b, float* y) {
+  float s[8], r[8], m = 1.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) s[e] = 1.0f + expf(-a[e]);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) m = fmaxf(m, s[e]);
+  if (__any(m > 0x1p126f)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = 1.0f / s[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float r0 = __builtin_amdgcn_rcpf(s[e]);
+      r[e] = __builtin_fmaf(__builtin_fmaf(-s[e], r0, 1.0f), r0, r0);
+    }
+  }
+  // (here, so that the last product is rounded to fp16 at once, as the single ones are)
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] = a[e] * r[e] * b[e];
+}
+
 // what silu_and_mul stores for a gate and an up column that are 16 bits already
 template <int DT>
 __device__ __forceinline__ uint16_t silu_mul16(uint16_t gate, uint16_t up) {
@@ -275,23 +299,44 @@ __device__ __forceinline__ float round_act(float f) {
 
 __device__ __forceinline__ float clamp448(float y) { return fminf(fmaxf(y, -FP8_MAX), FP8_MAX); }
 
-// a / s for many a and one s, with the result of the IEEE division: the reciprocal estimate and
-// its Newton step are made once per divisor, the quotient estimate and its two residual
-// corrections once per dividend -- the same fused multiply-adds the division expands to, without
-// the operand scaling that only matters when s, 1 / s, a / s or a residual leave the normal range.
-// For the dynamic scales here s = max(absmax, 1e-10) / 448 is normal, |a / s| <= 448, and a
-// residual can only underflow where the quotient is far below the smallest fp8 step.
+// Two values rounded to the activation type (bf16: one conversion for both, which the compiler would take apart again).
+template <int DT>
+__device__ __forceinline__ void round_act2(float& a, float& b) {
+  if constexpr (DT == MI355Q_BF16) {
+    uint32_t v;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(v) : "v"(a), "v"(b));
+    a = bitcast<float>(v << 16);
+    b = bitcast<float>(v & 0xffff0000u);
+  } else {
+    a = round_act<DT>(a);
+    b = round_act<DT>(b);
+  }
+}
+
+// max(m, |a|, |b|) without the operands' NaNs, of results of arithmetic or conversions.  (In one instruction: fmaxf of values whose bits were
+// moved about makes the compiler quiet NaNs first, which those results never need.)
+__device__ __forceinline__ float max_abs2(float m, float a, float b) {
+  float r;
+  asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
+  return r;
+}
+
+// a / s for many a and one s, with the result of the IEEE division, for what the quantisers divide: a of 16 bits, s = max(largest |a|, 1e-10) / 448.
+// The correctly rounded reciprocal is made once per divisor (an estimate and its Newton step), per dividend the quotient estimate and its
+// correction by the exact residual.  s is normal and |a / s| <= 448; a residual can only underflow where the quotient is far below the smallest fp8 step.  (That
+// one correction is enough is known for every pair of 16-bit values there is: all of them give the division's fp8 code.)  An infinite s, of a group with an
+// infinity, makes zeros of what is finite and NaN of the infinities; the residual is taken as s q - a, whose zero leaves the sign of a zero quotient alone.
 struct SharedDivisor {
   float s, y;
-  __device__ __forceinline__ explicit SharedDivisor(float s_) : s(s_) {
-    const float y0 = __builtin_amdgcn_rcpf(s_);
-    y = __builtin_fmaf(__builtin_fmaf(-s_, y0, 1.0f), y0, y0);
+  __device__ __forceinline__ explicit SharedDivisor(float s_) {
+    const float y0 = __builtin_amdgcn_rcpf(s_), y1 = __builtin_fmaf(__builtin_fmaf(-s_, y0, 1.0f), y0, y0);
+    const bool finite = s_ < __builtin_inff();
+    s = finite ? s_ : 0.0f;
+    y = finite ? y1 : 0.0f;
   }
   __device__ __forceinline__ float div(float a) const {
-    const float q0 = a * y;
-    const float q1 = __builtin_fmaf(__builtin_fmaf(-s, q0, a), y, q0);
-    // the division's own last instruction: signed zeros, infinities and NaN as IEEE has them
-    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-s, q1, a), y, q1), s, a);
+    const float q = a * y;
+    return __builtin_fmaf(-__builtin_fmaf(q, s, -a), y, q);
   }
 };
 

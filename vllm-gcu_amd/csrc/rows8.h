@@ -28,29 +28,30 @@ __device__ __forceinline__ u2 to_fp8x8(const float* y) {
   return r;
 }
 
-__device__ __forceinline__ int8_t sat_rne_s8(float y) {
-  y = __builtin_rintf(y);                       // round half to even
-  y = fminf(fmaxf(y, -128.0f), 127.0f);
-  return (int8_t)(int)y;
+// Rounded to even and saturated to int8, in the low byte: the sum with 1.5 * 2^23 has no bits for a fraction.  (NaN: -128.)
+__device__ __forceinline__ uint32_t rne_s8_byte(float y) { return bitcast<uint32_t>(__builtin_amdgcn_fmed3f(y, -128.0f, 127.0f) + 12582912.0f); }
+__device__ __forceinline__ int8_t sat_rne_s8(float y) { return (int8_t)rne_s8_byte(y); }
+// the low bytes of four words
+__device__ __forceinline__ uint32_t low_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  return __builtin_amdgcn_perm(__builtin_amdgcn_perm(d, c, 0x0c0c0400u), __builtin_amdgcn_perm(b, a, 0x0c0c0400u), 0x05040100u);
 }
 __device__ __forceinline__ u2 pack_s8x8(const float* y) {
-  uint32_t q[2] = {0u, 0u};
-#pragma unroll
-  for (int e = 0; e < 8; ++e) q[e >> 2] |= ((uint32_t)(uint8_t)sat_rne_s8(y[e])) << (8 * (e & 3));
-  return (u2){q[0], q[1]};
+  return (u2){low_bytes(rne_s8_byte(y[0]), rne_s8_byte(y[1]), rne_s8_byte(y[2]), rne_s8_byte(y[3])),
+              low_bytes(rne_s8_byte(y[4]), rne_s8_byte(y[5]), rne_s8_byte(y[6]), rne_s8_byte(y[7]))};
 }
 
 // 8 values of a row with the largest magnitude mx -> codes of the per-token int8 quantiser, and the row's scale
 struct RowInt8 {
   float scale, inv;
   __device__ __forceinline__ explicit RowInt8(float mx) : scale(mx / 127.0f), inv(127.0f / mx) {}   // (inv: inf for an all-zero row)
-  __device__ __forceinline__ u2 codes(float* y) const {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      y[e] *= inv;
-      if (y[e] != y[e]) y[e] = 0.f;             // 0 * inf
-    }
-    return pack_s8x8(y);
+  // (NaN, also of 0 * inf: 0, which the conversion makes of it by itself; it saturates as well)
+  __device__ __forceinline__ uint32_t code(float y) const {
+    int i;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(__builtin_rintf(y * inv)));
+    return (uint32_t)min(max(i, -128), 127);
+  }
+  __device__ __forceinline__ u2 codes(const float* y) const {
+    return (u2){low_bytes(code(y[0]), code(y[1]), code(y[2]), code(y[3])), low_bytes(code(y[4]), code(y[5]), code(y[6]), code(y[7]))};
   }
 };
 // ... of the per-token fp8 quantiser
