@@ -207,7 +207,8 @@ int mi355q_q8_quant_gemm(void* out, const void* x, const void* w, const void* x_
 /* No counterpart in the reference.  Whether an 8-bit layer in the kslab order with M rows is taken by the kernel for
  * a few dozen to some hundred rows (csrc/q8_mid.hip) when mi355q_fp8_block_gemm_ws (kind 0), mi355q_fp8_scaled_gemm_ws
  * (kind 1) or mi355q_w8a8_int8_gemm_ws (kind 2) is called with *workspace_bytes bytes of workspace (0: none needed).
- * 1: it is, and those entry points are ahead of mi355q_kcontig_gemm; 0: it is not. */
+ * 1: it is, and those entry points are ahead of mi355q_kcontig_gemm; 0: it is not.  (Up to 64 dense rows that fit LDS whole, some 128 thousand elements, are
+ * multiplied by the kernel for fewer rows, csrc/q8_decode.hip, by either entry point where it is ahead.) */
 int mi355q_q8_mid_plan(int kind, int M, int N, int K, size_t* workspace_bytes);
 /* The work split of that plan: rows and columns of a workgroup's tile and K ranges (what a profile was taken on); all 0 where the
  * plan answers 0. */

@@ -1,4 +1,4 @@
-"""The 8-bit kernel for up to 16 rows (csrc/q8_decode.hip): K of one block, of fewer blocks than wavefronts, of whole and ragged rounds of the ring; columns for
+"""The 8-bit kernel for few rows (csrc/q8_decode.hip): K of one block, of fewer blocks than wavefronts, of whole and ragged rounds of the ring; columns for
 one to eight tiles per workgroup with a last workgroup that is not full; every quantiser.  Rows quantised in the kernel give, bit for bit, what
 the quantiser's launch and the GEMM on its codes give, and codes are held to a float64 product."""
 import pytest
@@ -14,6 +14,11 @@ TOKEN, CHANNEL = 1, 2                    # its quantisers
 # (M, N, K)
 ROWS = [(1, 64, 128), (3, 192, 640), (16, 4096, 1024), (8, 4160, 1920), (5, 8256, 1152), (1, 12352, 1408), (1, 64, 2048), (7, 4096, 2176), (2, 4160, 4096),
         (4, 8192, 4096), (1, 16384, 7168), (2, 16448, 3712), (1, 28672, 2048), (1, 3584, 18944), (1, 320, 20480)]
+# of 17 .. 64 rows: two, three and four row tiles, the last one full and with one row, for one to eight column tiles, the rows up to all of LDS; kinds
+MORE = [(17, 64, 1024, (0, FP8, INT8)), (32, 4096, 4096, (0,)), (28, 4096, 4096, (INT8,)), (23, 4096, 4096, (FP8,)), (24, 4224, 3712, (0,)), (32, 4160, 2048, (INT8,)),
+        (31, 8256, 1024, (INT8,)), (29, 12352, 1152, (INT8,)), (18, 16512, 7168, (0, FP8, INT8)), (32, 16512, 4096, (0, FP8, INT8)), (25, 13824, 5120, (0, FP8, INT8)),
+        (33, 320, 1024, (INT8,)), (48, 4096, 2048, (0,)), (40, 4096, 3200, (0,)), (40, 4096, 1408, (0, INT8)), (47, 4160, 1024, (INT8,)), (36, 4224, 3328, (0, INT8)),
+        (33, 12352, 3328, (INT8,)), (48, 16384, 1024, (INT8,)), (49, 4224, 1024, (INT8,)), (64, 8192, 1024, (INT8,)), (64, 8256, 1024, (INT8,))]
 CODES = [(1, 64, 2048), (16, 4096, 2048), (9, 4160, 2176), (16, 8256, 3712), (12, 12352, 5120), (3, 16448, 7168), (8, 4096, 14336), (7, 3584, 18560), (2, 64, 65536)]
 
 
@@ -78,11 +83,7 @@ def test_rows_are_quantised_as_by_the_launch_of_their_own(M, N, K, kind, quant, 
     assert torch.isfinite(got[[r for r in range(M) if r not in (2, 3)]]).all()
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("kind", [0, FP8, INT8])                # 0: block scales
-@pytest.mark.parametrize("M,N,K", CODES)
-def test_codes(M, N, K, kind, dtype):
-    print(f"case q8 decode codes M={M} N={N} K={K} kind={kind} {dtype}", flush=True)
+def _hold_codes(M, N, K, kind, dtype, layouts):
     lib = _lib.load()
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
     x = _weights(kind, M, K, gen)
@@ -101,7 +102,7 @@ def test_codes(M, N, K, kind, dtype):
         want, size = ((a @ b.t()) * xs.double()[:, None] * ws.double() for a, b in ((x.double(), w.double()), (x.double().abs(), w.double().abs())))
     if bias is not None:
         want = want + bias.double()
-    for kslab in (True, False):
+    for kslab in layouts:
         out = torch.full((M, N), float("nan"), device="cuda").to(dtype)
         wk = rearrange.to_kslab(w) if kslab else w
         if kind == 0:
@@ -109,13 +110,47 @@ def test_codes(M, N, K, kind, dtype):
         else:
             _check(_codes_gemm(lib, kind, out, x, wk, kslab, xs, ws, bias, M, N, K, dtype))
         outs.append(out)
-    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(outs[0], outs[-1])
     # one rounding to 16 bits, and matrix instructions that align 32 products and the running sum to the largest of them: at most 33 units of 2^-24 of
     # what the magnitudes of all products add up to (at random a small part of that: the norms)
     eps = 2.0 ** (-11 if dtype == torch.float16 else -8)
     err = (outs[0].double() - want).abs()
     assert (err <= eps * want.abs() + (K / 32 * 33 * 2.0 ** -24) * size).all()
     assert err.norm() <= 0.75 * eps * want.norm()              # (uniform rounding alone: eps / sqrt(3) at most)
+    return x, w, xs, ws, bias, outs[0]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", [0, FP8, INT8])                # 0: block scales
+@pytest.mark.parametrize("M,N,K", CODES)
+def test_codes(M, N, K, kind, dtype):
+    print(f"case q8 decode codes M={M} N={N} K={K} kind={kind} {dtype}", flush=True)
+    _hold_codes(M, N, K, kind, dtype, (True, False))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind,M,N,K", [(k, *c[:3]) for c in MORE for k in c[3] if k or c[1] % 128 == 0])
+def test_codes_of_up_to_64_rows(M, N, K, kind, dtype):
+    """... also through the entry points that choose between this kernel and the tiles, with and without a workspace: the same bits (the tiles add
+    in another order)."""
+    print(f"case q8 decode codes M={M} N={N} K={K} kind={kind} {dtype}", flush=True)
+    lib = _lib.load()
+    x, w, xs, ws, bias, want = _hold_codes(M, N, K, kind, dtype, (True,))
+    wk, room = rearrange.to_kslab(w), torch.zeros(80 << 20, dtype=torch.uint8, device="cuda")
+    for scratch in (room, None):
+        if not lib.mi355q_q8_mid_plan(kind, M, N, K, None):
+            continue
+        out, tail = torch.full((M, N), float("nan"), device="cuda").to(dtype), (DT[dtype], _p(scratch), 0 if scratch is None else scratch.numel(), _stream())
+        if kind == 0:
+            _check(lib.mi355q_fp8_block_gemm_ws(_p(out), _p(x), _p(wk), _p(xs), _p(ws), _p(bias), M, N, K, K, 0, N, *tail))
+        elif kind == FP8:
+            _check(lib.mi355q_fp8_scaled_gemm_ws(_p(out), _p(x), _p(wk), _p(xs), 1, _p(ws), 1, _p(bias), M, N, K, K, 0, N, *tail))
+        else:
+            _check(lib.mi355q_w8a8_int8_gemm_ws(_p(out), None, _p(x), _p(wk), _p(xs), 1, _p(ws), 1, _p(bias), 0, M, N, K, K, 0, N, *tail))
+        if scratch is not None:
+            assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        else:                                                   # (the tall tiles may be ahead without room)
+            assert (out.double() - want.double()).norm() <= 4e-3 * want.double().norm()
 
 
 def test_what_is_not_covered_is_an_error():

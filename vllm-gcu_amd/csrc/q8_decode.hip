@@ -1,4 +1,4 @@
-// 8-bit GEMM for up to 16 rows: fp8 with 128 x 128 block scales, fp8 with per-token x per-channel scales, int8.  Where the rows are few
+// 8-bit GEMM for up to 16 rows, and up to 64 where they are short: fp8 with 128 x 128 block scales, fp8 with per-token x per-channel scales, int8.  Where the rows are few
 // thousand elements it takes them as 16-bit values and quantises them itself.
 //
 // What bounds such a call: HBM on layers of 60 MB and more, and below that what is not overlapped -- the launch, one trip to memory, the sums of the
@@ -13,6 +13,8 @@
 // kcontig_gemm_kernel -> here): 2048 x 2048 at 1 / 16 rows 3.4 / 4.0 -> 2.9 / 3.1, rows 5.3 -> 3.0; 4096 x 4096 at 1 / 8 5.5 / 5.7 -> 4.7 / 4.8, rows at 1 / 4
 // 7.5 / 7.9 -> 4.7 / 6.1; 3584 x 4608 at 16 7.7 -> 5.5; 14336 x 4096 at 1 / 4 13.3 / 12.9 -> 11.2 / 11.1, rows at 1 16.0 -> 12.3; 18944 x 3584 at 1 16.5 -> 13.1, rows
 // 19.8 -> 15.3; 8192 x 10240 at 1 / 8 18.7 / 19.1 -> 17.1 / 16.5; 4096 x 28672 at 1 21.7 -> 21.4, rows 23.9 -> 21.4.
+// From 17 rows on the weights of a workgroup are multiplied by two, three or four tiles of rows; what it takes is then the copy of the rows, which every
+// workgroup makes in whole (the figures stand with the rule, q8_decode_tiles).
 #include "rows8.h"
 
 #include <type_traits>
@@ -45,11 +47,11 @@ __device__ __forceinline__ void qd_lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// NI tiles of 16 columns, W wavefronts, BPR K blocks of each on their way
-template <int MODE, int SRC, int DT, int NI, int W, int BPR>
+// NI tiles of 16 columns, W wavefronts, BPR K blocks of each on their way, MT tiles of 16 rows
+template <int MODE, int SRC, int DT, int NI, int W, int BPR, int MT>
 __global__ void __launch_bounds__(64 * W, 2)
 q8_decode_kernel(QdArgs a) {
-  static_assert(NI <= W, "a wavefront finishes one tile at most");
+  static_assert(NI <= W, "the tiles that a wavefront finishes are of the same columns");
   static_assert(SRC == QD_CODES || MODE != QD_BLOCK, "rows for block scales come quantised");
   static_assert(SRC != QD_CHANNEL || MODE == QD_INT8, "scales per column are int8's");
   typedef typename std::conditional<MODE == QD_INT8, i4, f4>::type acc_t;
@@ -72,18 +74,26 @@ q8_decode_kernel(QdArgs a) {
     if (SRC == QD_CHANNEL) cv[p] = ((const u4*)a.c_scale)[i - (int)(a.row_pieces.div((uint32_t)i) * a.row_pieces.d)];
   }
   if (SRC == QD_TOKEN && tid < 16) row_max[tid] = 0u;
-  const int nt = n0 + 16 * wave + 4 * q;                     // columns of the outputs that this lane stores (wave < NI)
-  const bool stores = wave < NI && nt < N;
+  // tiles wave, wave + W of the NI x MT (columns first): the columns, and the rows, of the outputs that this lane stores
+  constexpr int FIN = (NI * MT + W - 1) / W;
+  const int nt = n0 + 16 * (wave % NI) + 4 * q;
+  const bool stores = wave < NI * MT && nt < N;
+  auto stored_row = [&](int f) { return 16 * ((wave + W * f) / NI) + r16; };
   f4 ws = {1.f, 1.f, 1.f, 1.f};
   uint2 bs = {0u, 0u};
-  float xs = 1.0f;
+  float xs[FIN];
+#pragma unroll
+  for (int f = 0; f < FIN; ++f) xs[f] = 1.0f;
   if (stores) {
     if (MODE != QD_BLOCK) {
       if (a.sc_col) ws = *(const f4*)(a.w_scale + nt);
       else ws = (f4){a.w_scale[0], a.w_scale[0], a.w_scale[0], a.w_scale[0]};
     }
     if (a.bias) bs = *(const uint2*)(a.bias + nt);
-    if (SRC == QD_CODES && MODE != QD_BLOCK && a.x_scale) xs = a.x_scale[min(r16, M - 1) * a.sc_row];
+    if (SRC == QD_CODES && MODE != QD_BLOCK && a.x_scale) {
+#pragma unroll
+      for (int f = 0; f < FIN; ++f) xs[f] = a.x_scale[min(stored_row(f), M - 1) * a.sc_row];
+    }
   }
   // block scales of x and of the columns, into LDS behind x: thread t holds values t, t + 64 W
   const int s_total = M * KB;
@@ -166,36 +176,43 @@ q8_decode_kernel(QdArgs a) {
       if (tid + p * THREADS < s_total) xs_l[tid + p * THREADS] = sv[p];
     if (tid < KB) ws_l[tid] = wsv;
   }
+  static_assert(SRC != QD_TOKEN || MT == 1, "sixteen largest magnitudes");
   if (SRC == QD_TOKEN && stores)
-    xs = MODE == QD_INT8 ? RowInt8(bitcast<float>(row_max[r16])).scale : RowFp8(bitcast<float>(row_max[r16])).scale;
+    xs[0] = MODE == QD_INT8 ? RowInt8(bitcast<float>(row_max[r16])).scale : RowFp8(bitcast<float>(row_max[r16])).scale;
   qd_lds_barrier();
 
-  // ---- K blocks wave, wave + 16, ..
-  acc_t acc[NI];
+  // ---- K blocks wave, wave + W, ..
+  acc_t acc[MT][NI];
 #pragma unroll
-  for (int t = 0; t < NI; ++t) acc[t] = (acc_t){0, 0, 0, 0};
-  const int row = min(r16, M - 1);
+  for (int j = 0; j < MT; ++j)
+#pragma unroll
+    for (int t = 0; t < NI; ++t) acc[j][t] = (acc_t){0, 0, 0, 0};
+  int row[MT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j) row[j] = min(16 * j + r16, M - 1);
   auto multiply = [&](int b, int kb) {
-    const u4 x0 = *(const u4*)(lds + chunk_at(kb, row, 2 * q)), x1 = *(const u4*)(lds + chunk_at(kb, row, 2 * q + 1));
-    const u4 xo[2] = {x0, x1};
-    const float sc = MODE == QD_BLOCK ? xs_l[row * KB + kb] * ws_l[kb] : 1.0f;
 #pragma unroll
-    for (int t = 0; t < NI; ++t) {
-      if constexpr (MODE == QD_INT8) {
+    for (int j = 0; j < MT; ++j) {
+      const u4 xo[2] = {*(const u4*)(lds + chunk_at(kb, row[j], 2 * q)), *(const u4*)(lds + chunk_at(kb, row[j], 2 * q + 1))};
+      const float sc = MODE == QD_BLOCK ? xs_l[row[j] * KB + kb] * ws_l[kb] : 1.0f;
 #pragma unroll
-        for (int v = 0; v < 2; ++v) acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bitcast<i4>(w[b][t][v]), bitcast<i4>(xo[v]), acc[t], 0, 0, 0);
-      } else {
-        f4 part = MODE == QD_BLOCK ? (f4){0.f, 0.f, 0.f, 0.f} : acc[t];
+      for (int t = 0; t < NI; ++t) {
+        if constexpr (MODE == QD_INT8) {
 #pragma unroll
-        for (int v = 0; v < 2; ++v) {
-          const u4 wv = w[b][t][v];
-          part = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)((unsigned long)wv[0] | ((unsigned long)wv[1] << 32)),
-                                                            (long)((unsigned long)xo[v][0] | ((unsigned long)xo[v][1] << 32)), part, 0, 0, 0);
-          part = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)((unsigned long)wv[2] | ((unsigned long)wv[3] << 32)),
-                                                            (long)((unsigned long)xo[v][2] | ((unsigned long)xo[v][3] << 32)), part, 0, 0, 0);
+          for (int v = 0; v < 2; ++v) acc[j][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bitcast<i4>(w[b][t][v]), bitcast<i4>(xo[v]), acc[j][t], 0, 0, 0);
+        } else {
+          f4 part = MODE == QD_BLOCK ? (f4){0.f, 0.f, 0.f, 0.f} : acc[j][t];
+#pragma unroll
+          for (int v = 0; v < 2; ++v) {
+            const u4 wv = w[b][t][v];
+            part = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)((unsigned long)wv[0] | ((unsigned long)wv[1] << 32)),
+                                                              (long)((unsigned long)xo[v][0] | ((unsigned long)xo[v][1] << 32)), part, 0, 0, 0);
+            part = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)((unsigned long)wv[2] | ((unsigned long)wv[3] << 32)),
+                                                              (long)((unsigned long)xo[v][2] | ((unsigned long)xo[v][3] << 32)), part, 0, 0, 0);
+          }
+          if constexpr (MODE == QD_BLOCK) acc[j][t] += sc * part;
+          else acc[j][t] = part;
         }
-        if constexpr (MODE == QD_BLOCK) acc[t] += sc * part;
-        else acc[t] = part;
       }
     }
   };
@@ -216,23 +233,30 @@ q8_decode_kernel(QdArgs a) {
   qd_lds_barrier();                                          // everybody has read x
   acc_t* const red = (acc_t*)lds;
 #pragma unroll
-  for (int t = 0; t < NI; ++t) red[(wave * NI + t) * 64 + lane] = acc[t];
+  for (int j = 0; j < MT; ++j)
+#pragma unroll
+    for (int t = 0; t < NI; ++t) red[(wave * NI * MT + j * NI + t) * 64 + lane] = acc[j][t];
   qd_lds_barrier();
-  if (!stores || r16 >= M) return;
-  acc_t sum = red[wave * 64 + lane];
+  if (!stores) return;
 #pragma unroll
-  for (int s = 1; s < W; ++s) sum += red[(s * NI + wave) * 64 + lane];
-  float v[4];
+  for (int f = 0; f < FIN; ++f) {
+    const int m = stored_row(f);
+    if (m >= M) return;
+    acc_t sum = red[(wave + W * f) * 64 + lane];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v[e] = MODE == QD_BLOCK ? (float)sum[e] : scaled_sum((float)sum[e], xs, ws[e]);
-    const uint32_t bw = e < 2 ? bs.x : bs.y;
-    if (a.bias) v[e] = plus_bias(v[e], Elem<DT>::to_f32((uint16_t)((e & 1) ? bw >> 16 : bw & 0xffffu)));
+    for (int s = 1; s < W; ++s) sum += red[(s * NI * MT + wave + W * f) * 64 + lane];
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = MODE == QD_BLOCK ? (float)sum[e] : scaled_sum((float)sum[e], xs[f], ws[e]);
+      const uint32_t bw = e < 2 ? bs.x : bs.y;
+      if (a.bias) v[e] = plus_bias(v[e], Elem<DT>::to_f32((uint16_t)((e & 1) ? bw >> 16 : bw & 0xffffu)));
+    }
+    u2 o;
+    o.x = (uint32_t)Elem<DT>::from_f32(v[0]) | ((uint32_t)Elem<DT>::from_f32(v[1]) << 16);
+    o.y = (uint32_t)Elem<DT>::from_f32(v[2]) | ((uint32_t)Elem<DT>::from_f32(v[3]) << 16);
+    *(u2*)((uint16_t*)a.out + (size_t)m * N + nt) = o;
   }
-  u2 o;
-  o.x = (uint32_t)Elem<DT>::from_f32(v[0]) | ((uint32_t)Elem<DT>::from_f32(v[1]) << 16);
-  o.y = (uint32_t)Elem<DT>::from_f32(v[2]) | ((uint32_t)Elem<DT>::from_f32(v[3]) << 16);
-  *(u2*)((uint16_t*)a.out + (size_t)r16 * N + nt) = o;
 }
 
 // column tiles per workgroup: one workgroup per CU
@@ -243,19 +267,28 @@ int qd_tiles(int N) {
   return 0;
 }
 size_t qd_lds_bytes(int mode, int M, int K, int ni, int waves) {
-  const size_t x = (size_t)M * K + (mode == QD_BLOCK ? ((size_t)M * (K / 128) + K / 128) * 4 : 0), sums = (size_t)waves * ni * 1024;
+  const size_t x = (size_t)M * K + (mode == QD_BLOCK ? ((size_t)M * (K / 128) + K / 128) * 4 : 0), sums = (size_t)waves * ni * ((M + 15) / 16) * 1024;
   return x > sums ? x : sums;
 }
 // (with four wavefronts K blocks are added in the order of kcontig_gemm_kernel, which takes codes of so short a K)
 int qd_waves(int K) { return K < 2048 ? 4 : 8; }
 
-template <int MODE, int SRC, int DT, int NI, int W, int BPR>
-int launch_qd(const QdArgs& a, hipStream_t st) {
-  static hipError_t attr = hipFuncSetAttribute((const void*)q8_decode_kernel<MODE, SRC, DT, NI, W, BPR>, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
+template <int MODE, int SRC, int DT, int NI, int W, int BPR, int MT>
+int launch_qd_rows(const QdArgs& a, hipStream_t st) {
+  static hipError_t attr = hipFuncSetAttribute((const void*)q8_decode_kernel<MODE, SRC, DT, NI, W, BPR, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
   MQ_REQUIRE(attr == hipSuccess, "q8_decode: cannot reserve LDS: %s", hipGetErrorString(attr));
-  hipLaunchKernelGGL((q8_decode_kernel<MODE, SRC, DT, NI, W, BPR>), dim3((a.N + 16 * NI - 1) / (16 * NI)), dim3(64 * W), qd_lds_bytes(MODE, a.M, a.K, NI, W), st, a);
+  hipLaunchKernelGGL((q8_decode_kernel<MODE, SRC, DT, NI, W, BPR, MT>), dim3((a.N + 16 * NI - 1) / (16 * NI)), dim3(64 * W), qd_lds_bytes(MODE, a.M, a.K, NI, W), st, a);
   MQ_LAUNCH_CHECK("q8_decode");
   return 0;
+}
+template <int MODE, int SRC, int DT, int NI, int W, int BPR>
+int launch_qd(const QdArgs& a, hipStream_t st) {
+  if constexpr (SRC == QD_CODES) {
+    if constexpr (MODE == QD_INT8 && (NI == 2 || NI == 4)) if (a.M > 48) return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 4>(a, st);
+    if constexpr (MODE == QD_INT8 ? NI <= 4 : MODE == QD_BLOCK && NI <= 2) if (a.M > 32) return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 3>(a, st);
+    if (a.M > 16) return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 2>(a, st);
+  }
+  return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 1>(a, st);
 }
 template <int MODE, int SRC, int DT, int NI, int W>
 int launch_qd_ring(const QdArgs& a, hipStream_t st) {
@@ -284,12 +317,36 @@ int launch_qd_waves(const QdArgs& a, int tiles, hipStream_t st) {
 
 }  // namespace
 
-// Column tiles per workgroup where codes of M rows go here, 0 where they do not.  Below 2048 kcontig_gemm_kernel is ahead (1024 x 4096 at one row 3.0 us against 3.5); rows fill LDS at 128 KiB, and with
-// two column tiles per workgroup its wavefronts catch up from 96 KiB on (8192 x 8192 at 16 rows 12.2 us against 12.9).
-int q8_decode_tiles(int M, int N, int K) {
-  if (M < 1 || M > 16 || K % 128 != 0 || K < 2048 || K > 65536 || N % 16 != 0 || (long)M * K > 128 * 1024 || (size_t)N * K >= ((size_t)1 << 31)) return 0;
-  const int tiles = qd_tiles(N);
-  return tiles == 2 && M * K > 96 * 1024 ? 0 : tiles;
+// Column tiles per workgroup where codes of M rows go here, 0 where they do not.  The rows fill LDS at 128 KiB.
+//  - Up to 16 rows: below K 2048 kcontig_gemm_kernel is ahead (1024 x 4096 at one row 3.0 us against 3.5), and with two column tiles per workgroup its
+//    wavefronts catch up from 96 KiB on (8192 x 8192 at 16 rows 12.2 us against 12.9).
+//  - 17 .. 64 rows, against q8_mid_kernel, which reads a share of the rows for every 32 or 64 columns and walks K through a barrier per block: 22 layers of K 1024 .. 7168 at nine
+//    numbers of rows, with weights from memory and from the last-level cache.  From memory this is ahead nearly everywhere (1.0 .. 1.7 times); from the cache the copy of all rows into every
+//    workgroup costs more than the weights, so the lines are where that pays less than 3 %.  (us, from memory, there / here, and the ratio from the cache: block scales 2048 x 2048 at 20 6.0 /
+//    3.5, 1.68, 2048 x 7168 at 24 / 48 6.2 / 5.3, 1.23, 6.9 / 6.5, 1.02, 4096 x 12288 at 24 13.2 / 12.6, 0.95; int8 4096 x 4096 at 24 7.8 / 6.0, 1.10, 3584 x 4608 at 20 7.2 / 6.2, 1.00, 4096 x 6144 at 24
+//    8.3 / 7.3, 0.91, 2048 x 11008 at 24 / 48 8.3 / 6.9, 1.09, 10.4 / 7.9, 1.07; per channel 4096 x 4096 at 20 / 32 7.9 / 5.9, 1.39, 8.0 / 7.0, 0.97, 3072 x 4608 at 24 6.6 / 6.3, 0.92.)
+//  - 17 .. 32 rows of large layers, against the streamer (5120 x 13824 at 24, int8 16.2 / 15.0 and 1.08; 4096 x 28672 at 32 25.1 / 22.6 and 1.11).
+int q8_decode_tiles(int mode, int M, int N, int K) {
+  if (M < 1 || M > 64 || K % 128 != 0 || K > 65536 || N % 16 != 0 || (long)M * K > 128 * 1024 || (size_t)N * K >= ((size_t)1 << 31)) return 0;
+  const int tiles = qd_tiles(N), rows = (M + 15) / 16;
+  if (M <= 16) return K < 2048 || (tiles == 2 && M * K > 96 * 1024) ? 0 : tiles;
+  if (K < 1024) return 0;
+  if (M <= 32 && N >= 12288 && (long)K * N >= (1L << 26)) return tiles;
+  if (tiles > 4) return 0;
+  int most = 0;                                              // KiB of rows
+  if (mode == QD_BLOCK) {
+    if (rows == 2) most = tiles == 1 ? 128 : tiles == 2 ? 100 : 0;
+    else if (rows == 3 && tiles <= 2) most = M <= 40 || K <= 2048 ? 128 : 0;
+  } else if (mode == QD_PC) {
+    most = tiles == 1 && rows == 2 ? 96 : 0;
+  } else if (rows == 2) {
+    most = tiles == 1 ? 112 : tiles == 2 ? (K <= 2048 ? 64 : 0) : 96;
+  } else if (rows == 3) {
+    most = tiles == 1 ? (M <= 40 ? 96 : 0) : tiles == 2 ? 120 : 112;
+  } else {
+    most = tiles >= 2 ? 64 : 0;
+  }
+  return M * K <= most * 1024 ? tiles : 0;
 }
 
 // (the loads and stores of its widths)
