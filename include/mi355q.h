@@ -107,7 +107,9 @@ int mi355q_w4a16_gemm(void* out, const void* x, const int32_t* qweight,
  * 4's where the library takes those by itself), 3 = MFMA workgroups of 128
  * rows x 256 columns fed through a ring of LDS stages (fp16, group sizes that
  * are multiples of 128; there bits 8..15 of split_k = 4 select 512 columns, and
- * bits 16..23 = 5, 6 or 7 select 80, 96 or 112 rows; bf16 above 64
+ * bits 16..23 = 5, 6 or 7 select 80, 96 or 112 rows, with 512 columns and
+ * bits 16..23 = 8 bits 24..30 the workgroups per column tile where some of
+ * 112 and some of 128 rows make that many; bf16 above 64
  * rows with the full workspace: the rows staged as fp16),
  * 4 = MFMA workgroups of 32..96 rows x 64 or 128 columns (split_k bits
  * 8..15: rows / 16, 16..23: columns / 64; 0 = the library's choice). */

@@ -40,6 +40,20 @@ def test_heights(K, N, g, dtype):
                     assert torch.equal(out.cpu(), want[:M])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,N,g", CASES)
+def test_two_heights(K, N, g, dtype):
+    """Workgroups of 128 rows first and of 112 after them: one of either, rows that end inside the last one, K splits; a number of them that does not
+    come out (9 for 1300 rows: all of 128)."""
+    w, zp, s, x, bias, want = _data(K, N, g, 1300, dtype)
+    for M, rows in ((225, 2), (239, 2), (240, 2), (352, 3), (368, 3), (1237, 11), (1300, 11), (1300, 9)):
+        for split in (1, 3) if dtype == torch.float16 else (1,):
+            print(f"case w4a16 ring two heights rows={rows} split={split} M={M} K={K} N={N} {dtype}", flush=True)
+            out = torch.full((M, N), float("nan"), dtype=dtype, device="cuda")
+            ops.w4a16_gemm(x[:M], w, s, zp, bias, g, family=3, split_k=split | 4 << 8 | 8 << 16 | rows << 24, out=out)
+            assert torch.equal(out.cpu(), want[:M])
+
+
 @pytest.mark.parametrize("dtype,kind", [(torch.float16, "none"), (torch.bfloat16, "none"), (torch.float16, "pre-scaled")])
 def test_heights_and_zero_points(dtype, kind, monkeypatch):
     """No zero-points, and z * s in the activation type read as they are (fp16; bf16 rows with those are not staged)."""

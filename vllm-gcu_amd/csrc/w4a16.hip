@@ -135,7 +135,7 @@ extern "C" int mi355q_w4a16_gemm_ex(void* out, const void* x, const int32_t* qwe
     const int rc = w4a16_bf16_staged_launch(out, x, qweight, scales, zeros, zeros_kind, bias, M, K, N, group_size,
                                             ws_ok ? (char*)workspace + TILE_WS_OFFSET : nullptr,
                                             ws_ok ? workspace_bytes - TILE_WS_OFFSET : 0,
-                                            (((split_k >> 8) & 0xff) == 4 ? 4 : 2) | (split_k & 0xff0000), as_stream(stream));
+                                            (((split_k >> 8) & 0xff) == 4 ? 4 : 2) | (split_k & 0x7fff0000), as_stream(stream));
     MQ_REQUIRE(rc != -12345,
                "w4a16_gemm: the ring kernels are fp16 kernels; bf16 rows reach them through a workspace of "
                "mi355q_w4a16_workspace_bytes() bytes, above 64 rows, with group sizes that are multiples of 128 and "
@@ -146,7 +146,7 @@ extern "C" int mi355q_w4a16_gemm_ex(void* out, const void* x, const int32_t* qwe
   if (family == 3)
     return w4a16_mid_launch(out, x, qweight, scales, zeros, zeros_kind, bias, M, K, N, group_size, dtype,
                             ws_ok ? (char*)workspace + TILE_WS_OFFSET : nullptr,
-                            ws_ok ? workspace_bytes - TILE_WS_OFFSET : 0, split_k & 0xff, (split_k >> 8) & 0xff, (split_k >> 16) & 0xff ? (split_k >> 16) & 0xff : 8, as_stream(stream));
+                            ws_ok ? workspace_bytes - TILE_WS_OFFSET : 0, split_k & 0xff, (split_k >> 8) & 0xff, (split_k >> 16) & 0xff ? (split_k >> 16) & 0x7fff : 8, as_stream(stream));
   return w4a16_tile_launch(out, x, qweight, scales, zeros, zeros_kind, bias, M, K, N, group_size, dtype,
                            ws_ok ? (char*)workspace + TILE_WS_OFFSET : nullptr,
                            ws_ok ? workspace_bytes - TILE_WS_OFFSET : 0, caller_family == 0, as_stream(stream));

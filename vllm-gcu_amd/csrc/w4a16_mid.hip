@@ -46,6 +46,7 @@ struct MidArgs {
   TileOrder order;            // of the output tiles and splits
   uint32_t gpk, gpk_magic;    // K blocks per group and ceil(2^32 / gpk)
   float* partial;             // split K: fp32 tiles [split][M][N]; null: write the output
+  int tall;                   // MIX kernels: the first workgroups' row tiles are one higher than the others'
   // IOBF kernels (bf16 rows staged as fp16 times a power of two each; scales, bias and output bf16):
   const float* row_scale;     // [M] the power of two each staged row has to be multiplied back by
   const uint32_t* scale_max;  // [64] largest scale magnitude (bf16 bits) of 64 slices of the scales array
@@ -102,8 +103,9 @@ __device__ __forceinline__ uint32_t mid_dequant_pair(uint32_t w, int p, _Float16
 // scale 2^24 below the largest one still keeps all its bits; the epilogue undoes both powers of two
 // exactly (one ldexp per output) and rounds to bf16.
 template <int ZK, int TW, int MT, bool IOBF>
-__global__ void __launch_bounds__(512, 1)
-w4a16_mid_kernel(MidArgs a) {
+__device__ __forceinline__ void mid_tile(MidArgs a, const int m0, const int tn, const int split) {   // (by value: by reference the copies' addresses are made anew for every K block.  As the kernel itself
+  // this was 4 .. 5 % slower with five and six row tiles of 512 columns, 4096 x 28672 at 333 rows 87.2 us, here 83.6)
+  extern __shared__ __align__(16) unsigned char lds[];
   static_assert(!IOBF || ZK != MI355Q_ZP_PRESCALED, "pre-scaled zero-points stay with the bf16 kernel");
   typedef MidCfg<TW, MT> C;
   constexpr int D = C::D, STAGE = C::STAGE, XC = C::XC;
@@ -111,14 +113,10 @@ w4a16_mid_kernel(MidArgs a) {
   constexpr int NSLOT = XC + TW + 1;                  // copy slots per wavefront and stage (the last: scales + zeros)
   constexpr int NC = XC + TW + 1 + (HASZ ? 1 : 0);    // copy instructions per wavefront and stage
   static_assert((D - 1) * NC <= 63, "vmcnt is a 6-bit counter");
-  extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, kq = lane >> 4;
   const int N = a.N, K = a.K, M = a.M, G = K >> 7;
-  int tm, tn, split;
-  a.order.locate(blockIdx.x, tm, tn, split);
-  const int m0 = tm * C::BM;
   // N may end in the middle of a 256-column tile: the wavefronts of the missing slab work on the
   // previous one and their columns are never stored
   const int wslab = TW == 4 ? wave >> 1 : wave >> 2;                 // slab of the workgroup this wavefront works on
@@ -407,24 +405,56 @@ w4a16_mid_kernel(MidArgs a) {
   }
 }
 
-template <int ZK, int TW, int MT, bool IOBF>
-int launch_mid(MidArgs a, int splits, hipStream_t st) {
+// MIX: workgroups of MT row tiles for the first rows and of MT - 1 for the others
+template <int ZK, int TW, int MT, bool IOBF, bool MIX>
+__global__ void __launch_bounds__(512, 1)
+w4a16_mid_kernel(MidArgs a) {
+  int tm, tn, split;
+  a.order.locate(blockIdx.x, tm, tn, split);
+  if constexpr (MIX) {
+    if (tm >= a.tall) {
+      mid_tile<ZK, TW, MT - 1, IOBF>(a, 16 * (a.tall + tm * (MT - 1)), tn, split);
+      return;
+    }
+  }
+  mid_tile<ZK, TW, MT, IOBF>(a, 16 * MT * tm, tn, split);
+}
+
+template <int ZK, int TW, int MT, bool IOBF, bool MIX>
+int launch_mid(MidArgs a, int mtiles, int splits, hipStream_t st) {
   typedef MidCfg<TW, MT> C;
-  const size_t shmem = (size_t)C::D * C::STAGE;
-  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_mid_kernel<ZK, TW, MT, IOBF>,
+  typedef MidCfg<TW, MIX ? MT - 1 : MT> L;
+  const size_t shmem = std::max((size_t)C::D * C::STAGE, (size_t)L::D * L::STAGE);
+  static hipError_t attr = hipFuncSetAttribute((const void*)w4a16_mid_kernel<ZK, TW, MT, IOBF, MIX>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   MQ_REQUIRE(attr == hipSuccess, "w4a16_gemm(mid): cannot reserve %zu bytes of LDS: %s", shmem, hipGetErrorString(attr));
-  const int mtiles = (a.M + C::BM - 1) / C::BM, ntiles = (a.N + C::BNW - 1) / C::BNW;
+  const int ntiles = (a.N + C::BNW - 1) / C::BNW;
   a.order = tile_order(mtiles, ntiles, splits, (double)C::BM * a.kper * 256, (double)C::BNW * a.kper * 64);
-  hipLaunchKernelGGL((w4a16_mid_kernel<ZK, TW, MT, IOBF>), dim3((unsigned)(mtiles * ntiles * splits)), dim3(512), shmem, st, a);
+  hipLaunchKernelGGL((w4a16_mid_kernel<ZK, TW, MT, IOBF, MIX>), dim3((unsigned)(mtiles * ntiles * splits)), dim3(512), shmem, st, a);
   MQ_LAUNCH_CHECK("w4a16_gemm(mid)");
   return 0;
 }
+template <int ZK, int TW, int MT, bool IOBF>
+int launch_mid_rows(MidArgs a, int mixed, int splits, hipStream_t st) {
+  if constexpr (TW == 4 && MT == 8)
+    if (mixed) {
+      a.tall = (a.M + 15) / 16 - mixed * (MT - 1);
+      return launch_mid<ZK, TW, MT, IOBF, true>(a, mixed, splits, st);
+    }
+  return launch_mid<ZK, TW, MT, IOBF, false>(a, (a.M + 16 * MT - 1) / (16 * MT), splits, st);
+}
 
+// mt: row tiles of a workgroup; from bit 8 on the workgroups per column tile, where some of them take one row tile less (0: none does).  Of 512 columns and
+// eight row tiles, where layers of several rounds go.
+bool mid_mixes(int M, int tw, int mt, int mixed) {
+  const int S = (M + 15) / 16;
+  return tw == 4 && mt == 8 && mixed * (mt - 1) < S && S < mixed * mt;
+}
 template <int ZK, bool IOBF>
 int launch_mid_tw(const MidArgs& a, int tw, int mt, int splits, hipStream_t st) {
-#define MQ_MID(MT) case MT: return tw == 4 ? launch_mid<ZK, 4, MT, IOBF>(a, splits, st) : launch_mid<ZK, 2, MT, IOBF>(a, splits, st)
-  switch (mt) {
+  const int mixed = mid_mixes(a.M, tw, mt & 255, mt >> 8) ? mt >> 8 : 0;
+#define MQ_MID(MT) case MT: return tw == 4 ? launch_mid_rows<ZK, 4, MT, IOBF>(a, mixed, splits, st) : launch_mid_rows<ZK, 2, MT, IOBF>(a, mixed, splits, st)
+  switch (mt & 255) {
     MQ_MID(5);
     MQ_MID(6);
     MQ_MID(7);
@@ -454,25 +484,39 @@ struct MidPrice {
 };
 static constexpr MidPrice kMid[2] = {{0.391, 0.1518, 0.498, 0.1003, 0.047, 4.89, 2.44, 0.00330, 2.10, 0.98},
                                      {1.041, 0.2372, 1.211, 0.1730, -0.034, 7.09, 2.40, 0.00409, 1.05, 0.92}};
+constexpr double kMixed = 1.02;      // what their price has to be below the others' by
 static MidPlan make_mid_plan(int M, int K, int N, size_t bytes) {
-  const int G = K / 128, cus = device_cu_count();
+  const int G = K / 128, cus = device_cu_count(), S = (M + 15) / 16;
   MidPlan best = {2, 8, 1, 1e30};
-  for (int tw = 2; tw <= 4; tw += 2)
-    for (int mt = 5; mt <= 8; ++mt) {
-      const int tiles = ((M + 16 * mt - 1) / (16 * mt)) * ((N + 128 * tw - 1) / (128 * tw));
-      const MidPrice& p = kMid[tw == 4];
-      const double odd = p.odd * (mt & 1), full = p.full + p.full_mt * mt + odd, lone = p.lone + p.lone_mt * mt + odd;
-      for (int s = 1; s <= 8 && (s == 1 || ((long)tiles * (s - 1) < 6L * cus && G / s >= 4 && (size_t)s * M * N * sizeof(float) <= bytes)); ++s) {
-        const int kper = (G + s - 1) / s;
-        if (s > 1 && (s - 1) * kper >= G) continue;    // an empty split
-        const int wgs = tiles * s, rounds = wgs / cus;
-        const double rest = (double)(wgs - rounds * cus) / cus;
-        double t = kper * (rounds * full + (rest > 0 ? lone + (full - lone) * rest * rest : 0.0)) * (1 + p.power * mt * std::min(rounds, 6)) +
-                   p.round * (rounds + (rest > 0)) + p.base;
-        if (s > 1) t += p.split + p.split_mn * 1e-6 * s * M * N;
-        if (t < best.price) best = {tw, mt, s, t};
+  double least = 1e30;
+  // rows: workgroups per column tile, `mean` row tiles high; mixed: some of mt and some of mt - 1
+  auto offer = [&](int tw, int mt, int rows, double mean, bool mixed) {
+    const int tiles = rows * ((N + 128 * tw - 1) / (128 * tw));
+    const MidPrice& p = kMid[tw == 4];
+    const double odd = p.odd * (mixed ? 0.5 : mt & 1), full = p.full + p.full_mt * mean + odd, lone = p.lone + p.lone_mt * mean + odd;
+    for (int s = 1; s <= 8 && (s == 1 || ((long)tiles * (s - 1) < 6L * cus && G / s >= 4 && (size_t)s * M * N * sizeof(float) <= bytes)); ++s) {
+      const int kper = (G + s - 1) / s;
+      if (s > 1 && (s - 1) * kper >= G) continue;    // an empty split
+      const int wgs = tiles * s, rounds = wgs / cus;
+      const double rest = (double)(wgs - rounds * cus) / cus;
+      double t = kper * (rounds * full + (rest > 0 ? lone + (full - lone) * rest * rest : 0.0)) * (1 + p.power * mean * std::min(rounds, 6)) +
+                 p.round * (rounds + (rest > 0)) + p.base;
+      if (s > 1) t += p.split + p.split_mn * 1e-6 * s * M * N;
+      if (mixed) t = kMixed * t + kper * p.full_mt * (mt - mean);     // (a CU with one high workgroup more than the others)
+      if (t < least) {
+        least = t;
+        best = {tw, mixed ? mt | rows << 8 : mt, s, mixed ? best.price : t};
       }
     }
+  };
+  for (int tw = 2; tw <= 4; tw += 2)
+    for (int mt = 5; mt <= 8; ++mt) offer(tw, mt, (M + 16 * mt - 1) / (16 * mt), mt, false);
+  // (the price stays that of the even ones: other kernels are chosen by it, whose operands are exact, and what is rounded to fp16 shall not
+  // depend on how the rows are dealt out)
+  // Even rounds by workgroups of 7 and 8 row tiles, up to three rounds: a chip that is full for longer runs into its power limit and gains nothing.  (us, all of one
+  // height -> here: 3584 x 37888 at 700 rows 190.2 -> 185.4, 4096 x 28672 at 1024 / 1537, bf16, 219.4 / 340.2 -> 216.1 / 334.4, 8192 x 28672 at 1024 424.2 -> 418.2; in four rounds
+  // 4096 x 28672 at 2048 430.6 / 435.3.  Of 256 columns, and 6 and 7 or 5 and 6 row tiles: within 1 % on average.)
+  for (int rows = S / 8 + 1; rows <= 127 && mid_mixes(M, 4, 8, rows) && (long)rows * ((N + 511) / 512) <= 3L * cus; ++rows) offer(4, 8, rows, (double)S / rows, true);
   return best;
 }
 // (bytes: 0, what a fixed scratch of 32 MiB leaves, or 64 MiB, but for callers with less than the library asked for)
@@ -492,9 +536,9 @@ int w4a16_mid_launch(void* out, const void* x, const int32_t* qweight, const voi
   MQ_REQUIRE((size_t)M * K * 2 < ((size_t)1 << 32), "w4a16_gemm: activation matrix %d x %d is 4 GiB or more", M, K);
   const int G = K / 128;
   if (tw != 4) tw = 2;
-  if (mt < 5 || mt > 8) mt = 8;
+  if ((mt & 255) < 5 || (mt & 255) > 8) mt = 8;
   if (splits <= 0) {
-    const long wgs = (long)((M + 16 * mt - 1) / (16 * mt)) * ((N + 128 * tw - 1) / (128 * tw));
+    const long wgs = (long)((M + 16 * (mt & 255) - 1) / (16 * (mt & 255))) * ((N + 128 * tw - 1) / (128 * tw));
     splits = (int)std::min<long>(device_cu_count() / wgs, G / 4);
     while (splits > 1 && (size_t)splits * M * N * sizeof(float) > ((size_t)64 << 20)) --splits;
     if (splits < 1) splits = 1;
