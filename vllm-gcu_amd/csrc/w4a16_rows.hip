@@ -26,7 +26,7 @@
 // 29.9 / 32.7 / 41.7 -> 20.3 / 23.2 / 29.1; 14336 x 4096 at 48 / 96 / 192 20.3 / 27.5 / 39.0 -> 16.3 / 21.9 / 31.7.
 // A workgroup without another one on its CU takes a ring of three stages in place of two, and the tiles up to 128 rows are priced for it (before -> since):
 // 4096 x 6144 at 96 15.4 -> 11.9; 8192 x 8192 at 40 / 96 18.1 / 29.8 -> 16.1 / 21.8; 4096 x 12288 at 48 16.1 -> 12.9; 5120 x 13824 at 40 19.7 -> 15.5;
-// 11008 x 4096 at 48 / 112 16.5 / 21.8 -> 14.3 / 23.4; 4096 x 28672 at 24 19.4 -> 17.1; bf16 8192 x 8192 at 48 / 96 21.2 / 29.9 -> 18.1 / 25.0.
+// 11008 x 4096 at 48 16.5 -> 14.3; 4096 x 28672 at 24 19.4 -> 17.1; bf16 8192 x 8192 at 48 / 96 21.2 / 29.9 -> 18.1 / 25.0.
 #include "common.h"
 
 #include <algorithm>
@@ -448,8 +448,10 @@ int launch_rows_cfg(const RowsArgs& a, int mt, int nt, int splits, const void* b
 // ranges, for a workgroup with its CU for itself (`lone`, where that is another ring than that of two), else for the first one on its CU and added for a
 // second one beside it (tiles of 64 columns and 32 x 128 fit two).  Above 128 rows, where the other kernels' prices are compared with this one: fitted to 3400
 // measurements (15 layer shapes, 20..2048 rows, 1..12 ranges, weights cold in the caches; rms error 5 %), without rings of their own for lone workgroups.  Up to
-// 128 rows: to the launches of 42 layers with each type (18 .. 128 rows, up to eight ranges, cold weights; rms errors 6 and 5 %); the tile taken by it loses 0.5 / 0.3 %
-// (fp16 / bf16) to the best one on average, and 14 / 10 % at worst (by the prices above 128 rows 1.0 / 1.8 %, and 18 / 25 %).
+// 128 rows: to the launches of 42 layers with each type (18 .. 128 rows, up to eight ranges, weights from memory; rms errors 6 and 5 %), and with fp16 then moved until the
+// tiles taken over 34 layers were right with weights from memory and from the Infinity Cache both, K ranges charged 0.2 us for their second launch (3584 x 37888
+// at 33 rows, by the first fit and now: 31.3 / 32.1 us from memory, 33.2 / 27.9 from the cache).  The tile taken loses 0.2 / 0.2 % (fp16 / bf16) to the best one on average,
+// 7 % at worst, and against the prices above 128 rows gains 3.6 / 3.1 % from memory and 1.6 / 1.3 % from the cache.
 struct RowsPrice {
   int mt, nt;
   double one, more, lone;
@@ -465,9 +467,9 @@ constexpr RowsModel kRows[3] = {
     {{{2, 1, 0.422, 0.388, 0.422}, {3, 1, 0.600, 0.500, 0.600}, {4, 1, 0.700, 0, 0}, {2, 2, 0.773, 0.594, 0.773},
       {3, 2, 0.956, 0, 0}, {4, 2, 1.173, 0, 0}, {5, 2, 1.333, 0, 0}, {6, 2, 1.555, 0, 0}},
      3.57, 1.10, 2.18, 1.56, 0.283, 0.388, 4.23e6},
-    {{{2, 1, 0.344, 0.544, 0.436}, {3, 1, 0.866, 0.413, 0.554}, {4, 1, 0.757, 0, 0}, {2, 2, 0.587, 0.911, 0.780},
-      {3, 2, 0.982, 0, 0}, {4, 2, 1.253, 0, 0}, {5, 2, 1.414, 0, 0}, {6, 2, 1.605, 0, 0}},
-     3.29, 1.44, 1.66, 2.11, 0.199, 0.236, 4.71e6},
+    {{{2, 1, 0.332, 0.643, 0.458}, {3, 1, 0.705, 0.364, 0.589}, {4, 1, 0.736, 0, 0}, {2, 2, 0.650, 0.672, 0.872},
+      {3, 2, 0.959, 0, 0}, {4, 2, 1.135, 0, 0}, {5, 2, 1.232, 0, 0}, {6, 2, 1.545, 0, 0}},
+     3.37, 1.25, 1.66, 2.97, 0.175, 0.249, 4.39e6},
     {{{2, 1, 0.464, 0.522, 0.511}, {3, 1, 0.605, 0.541, 0.640}, {4, 1, 0.750, 0, 0}, {2, 2, 0.597, 1.143, 0.908},
       {3, 2, 1.137, 0, 0}, {4, 2, 1.258, 0, 0}, {5, 2, 1.519, 0, 0}, {6, 2, 1.599, 0, 0}},
      4.05, 1.45, 1.79, 1.95, 0.155, 0.149, 4.04e6}};
@@ -541,8 +543,10 @@ double w4a16_wide_price(int M, int K, int N, int group_size, int zeros_kind, boo
 //    4096 x 28672, bf16: 16.2 against 19.8).
 //  - 17..32 rows: there the streaming kernel takes two row tiles and stays ahead on groups of 128 while the layer is small in both directions (us at 24 rows, fp16,
 //    there / here: 4096 x 6144 8.8 / 9.3, 2048 x 7168 6.0 / 6.5, 4096 x 4096 8.3 / 8.2; from 8192 columns 1408 x 19328 10.3 / 8.2, 4096 x 12288 11.8 / 11.0, 2560 x 8960
-//    8.3 / 7.7; from K 5120 6144 x 2048 8.6 / 7.6, 14336 x 4096 14.7 / 13.3, 5248 x 3840 8.9 / 8.7), and with bf16, whose operands cost more here, up to 100 million
-//    weights or 16384 columns (4096 x 12288 11.9 / 12.5, 14336 x 4096 14.3 / 14.5; 2432 x 18944 14.6 / 13.5).
+//    8.3 / 7.7; from K 5120 5248 x 3840 8.9 / 8.7), and with bf16, whose operands cost more here, up to 16384 columns (4096 x 12288 11.9 / 12.5; 2432 x 18944
+//    14.6 / 13.5).  K ranges here are a second launch, which the streaming kernel does without: 3 us more of host time in a call (3.3 -> 6.1, 7168 x 2560 at 30), so they have to
+//    be worth that.  14336 x 4096 14.7 / 13.3 and 6144 x 2048 8.6 / 7.6 are not (a whole layer of 2560 x 14336 and 7168 x 2560 at 30, launched call by call, 39.4 -> 41.7);
+//    the largest layers are (from 67 million weights with fp16, 100 million with bf16).
 //  - Pre-scaled zero-points up to 64 rows: the streaming kernel, which uses z * s as it is.
 //  - To 128 rows: always.  Above: where its price is below that of the kernels with larger tiles, which read and dequantise the
 //    weights fewer times, as those operands run there.
@@ -553,7 +557,11 @@ bool w4a16_rows_wanted(int M, int K, int N, int group_size, int zeros_kind, int 
   if (M > 4096 || (size_t)M * K * 2 >= ((size_t)1 << 32)) return false;
   if (zeros_kind == MI355Q_ZP_PRESCALED && M <= 64) return false;
   if (M <= 16) return small && w <= (1L << 25);
-  if (M <= 32) return small || (dtype == MI355Q_F16 ? N >= 8192 || K >= 5120 : N >= 16384 || w >= 3L << 25);
+  if (M <= 32) {
+    const bool bf = dtype == MI355Q_BF16;
+    if (small || w >= (bf ? 3L << 25 : 1L << 26)) return true;
+    return (bf ? N >= 16384 : N >= 8192 || K >= 5120) && rows_plans(M, K, N).of[bf].splits == 1;
+  }
   if (M <= 128) return true;
   // (the price, corrected for the size of the output and the rows by 255 launches with fp16 rows and 177 with bf16, rms errors 4.6 and 3 %.  The
   // pick loses 0.1 / 0.2 % (fp16 / bf16) to the best of the three kernels over 23 layers at 144 .. 2048 rows, 15 % at worst, where prices
