@@ -103,6 +103,18 @@ def test_taken_where_the_tiles_loop_is_the_slow_one(M, K, N, g, dtype):
     assert torch.equal(ops.w4a16_gemm(x, w, scales, zp, None, g), ops.w4a16_gemm(x, w, scales, zp, None, g, family=4))
 
 
+@pytest.mark.parametrize("M,K,N,dtype,family", [(17, 2560, 14336, torch.float16, 4), (32, 1408, 19328, torch.float16, 4), (24, 7168, 2560, torch.float16, 1),
+                                                (32, 14080, 4352, torch.float16, 1), (30, 14336, 4096, torch.bfloat16, 1), (24, 2432, 18944, torch.bfloat16, 4)])
+def test_17_to_32_rows_without_a_second_launch(M, K, N, dtype, family):
+    """Wide layers come here unsplit; those that K ranges would serve stay with the streaming kernel, one launch (K in another order, so equal bits say which ran)."""
+    print(f"case w4a16 17..32 rows M={M} K={K} N={N} {dtype}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    w, zp = (torch.randint(-2**31, 2**31, shape, dtype=torch.int32, device="cuda", generator=gen) for shape in ((K // 8, N), (K // 128, N // 8)))
+    scales = (torch.rand(K // 128, N, device="cuda", generator=gen) * 0.01).to(dtype)
+    x = torch.randn(M, K, device="cuda", generator=gen).to(dtype)
+    assert torch.equal(ops.w4a16_gemm(x, w, scales, zp, None, 128), ops.w4a16_gemm(x, w, scales, zp, None, 128, family=family))
+
+
 def test_activations_of_four_gib():
     """The last row below 4 GiB of activations is addressed in 32 bits; from 4 GiB on the problem is refused."""
     K, N, M = 1 << 24, 128, 127
