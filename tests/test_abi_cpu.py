@@ -50,3 +50,16 @@ def test_ops_fail_loudly_on_cpu_tensors():
     s = torch.ones(1, 128, dtype=torch.float16)
     with pytest.raises((RuntimeError, NotImplementedError)):
         ops.gptq_gemm_gcu(x, w, torch.empty(0, dtype=torch.int32), s, torch.empty(0, dtype=torch.int32), 4, None, 128)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 24])
+@pytest.mark.parametrize("K", [1024, 4096])
+@pytest.mark.parametrize("quant_mode", [1, 2])               # fp8 with block scales, int8
+def test_kcontig_gemm_refuses_other_outputs_than_16_bits(quant_mode, K, M):
+    """Whichever kernel the rows would go to."""
+    from vllm_gcu_amd import _lib
+    lib = _lib.load()
+    for out_dtype in (_lib.F32, 7, -1, _lib.BF16 | _lib.ZEROED_COUNTERS):
+        for layout in (0, 1):
+            rc = lib.mi355q_kcontig_gemm(4096, 4096, 4096, 4096, 4096, None, quant_mode, 128, M, K, 4096, _lib.F16, out_dtype, layout, None)
+            assert rc != 0 and b"unsupported mode" in lib.mi355q_last_error()

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from vllm_gcu_amd import _lib
+from vllm_gcu_amd.kernels import _custom_ops as ops
 from vllm_gcu_amd.kernels.quantization import rearrange
 
 pytestmark = pytest.mark.gpu
@@ -161,3 +162,18 @@ def test_what_is_not_covered_is_an_error():
     x = torch.zeros(17 * 4096, dtype=torch.float16, device="cuda")
     assert lib.mi355q_q8_quant_gemm(_p(x), _p(x), _p(x), None, _p(x), 1, None, INT8, TOKEN, 17, 128, 128, DT[x.dtype], _stream()) != 0
     assert lib.mi355q_q8_quant_gemm(_p(x), _p(x) + 2, _p(x), None, _p(x), 1, None, INT8, TOKEN, 1, 128, 128, DT[x.dtype], _stream()) != 0
+
+
+@pytest.mark.parametrize("M", [1, 16, 24])
+def test_fp32_outputs_are_refused(M):
+    """... by the operators that reach this kernel, and nothing is written."""
+    print(f"case q8 decode fp32 output M={M}", flush=True)
+    N, K = 4096, 4096
+    x, w = torch.ones(M, K, device="cuda").to(torch.float8_e4m3fn), rearrange.to_kslab(torch.ones(N, K, device="cuda").to(torch.float8_e4m3fn))
+    out, xs, ws = torch.full((M, N), 7.0, device="cuda"), torch.ones(M, K // 128, device="cuda"), torch.ones(N // 128, K // 128, device="cuda")
+    with pytest.raises(RuntimeError, match="unsupported mode"):
+        torch.ops._C.linear_quant(out, x, w, None, xs, ws)
+    with pytest.raises(RuntimeError, match="unsupported mode"):
+        ops.w8a8_block_fp8_matmul(x, w, xs, ws, [128, 128], torch.float32)
+    torch.cuda.synchronize()
+    assert (out == 7.0).all()

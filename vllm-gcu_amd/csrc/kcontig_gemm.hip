@@ -902,7 +902,9 @@ extern "C" int mi355q_kcontig_gemm(void* out, const void* a, const void* w, cons
   } else {
     MQ_REQUIRE(false, "kcontig_gemm: unknown quant_mode %d", quant_mode);
   }
-  if (const int tiles = (mode == KC_FP8_BLOCK || mode == KC_INT8) && (M <= 16 || w_layout) && q8_decode_reads(a, w, w_scale, bias, out)
+  // (16-bit outputs; launch_mode refuses the others)
+  if (const int tiles = (mode == KC_FP8_BLOCK || mode == KC_INT8) && (out_dtype == MI355Q_F16 || out_dtype == MI355Q_BF16) && (M <= 16 || w_layout) &&
+                                q8_decode_reads(a, w, w_scale, bias, out)
                             ? q8_decode_tiles(mode == KC_INT8 ? 2 : 0, M, N, K) : 0)
     return q8_decode_launch(tiles, mode == KC_INT8 ? 2 : 0, 0, out, a, w, a_scale, 1, nullptr, (const float*)w_scale, 1, bias, M, N, K, w_layout, out_dtype,
                             as_stream(stream));

@@ -366,6 +366,7 @@ static int quant_tiles(int mode, int quant, int M, int N, int K) {
 
 int q8_decode_launch(int tiles, int mode, int src, void* out, const void* x, const void* w, const float* x_scale, int sc_row, const void* c_scale,
                      const float* w_scale, int sc_col, const void* bias, int M, int N, int K, int kslab, int dtype, hipStream_t st) {
+  MQ_REQUIRE(dtype == MI355Q_F16 || dtype == MI355Q_BF16, "q8_decode: output dtype %d must be f16 or bf16", dtype);
   QdArgs a = {};
   a.out = out; a.x = x; a.w = (const uint8_t*)w; a.x_scale = x_scale; a.c_scale = (const uint16_t*)c_scale; a.w_scale = w_scale;
   a.bias = (const uint16_t*)bias;
