@@ -206,17 +206,18 @@ int mi355q_q8_quant_gemm_takes(int kind, int quant, int M, int N, int K);
 int mi355q_q8_quant_gemm(void* out, const void* x, const void* w, const void* x_scale, const float* w_scale, int w_scale_per_col,
                          const void* bias, int kind, int quant, int M, int N, int K, int dtype, void* stream);
 
-/* No counterpart in the reference.  Whether an 8-bit layer in the kslab order with M rows is taken by the kernel for
- * a few dozen to some hundred rows (csrc/q8_mid.hip) when mi355q_fp8_block_gemm_ws (kind 0), mi355q_fp8_scaled_gemm_ws
+/* No counterpart in the reference.  Whether an 8-bit layer in the kslab order with M rows is taken by the kernels for
+ * a few dozen to some hundred rows (csrc/q8_mid.hip, and csrc/q8_decode.hip up to 64 rows that fit LDS whole, some 128 thousand elements) when mi355q_fp8_block_gemm_ws (kind 0), mi355q_fp8_scaled_gemm_ws
  * (kind 1) or mi355q_w8a8_int8_gemm_ws (kind 2) is called with *workspace_bytes bytes of workspace (0: none needed).
- * 1: it is, and those entry points are ahead of mi355q_kcontig_gemm; 0: it is not.  (Up to 64 dense rows that fit LDS whole, some 128 thousand elements, are
- * multiplied by the kernel for fewer rows, csrc/q8_decode.hip, by either entry point where it is ahead.) */
+ * 1: it is, and those entry points are ahead of mi355q_kcontig_gemm; 0: it is not.  The kernel for few rows uses no workspace and takes dense rows,
+ * 16-bit outputs, a bias in the output's type and operands aligned to 16 bytes (out and bias: 8), by mi355q_kcontig_gemm as well; the bytes
+ * are what the calls of the same sizes that it does not take can use. */
 int mi355q_q8_mid_plan(int kind, int M, int N, int K, size_t* workspace_bytes);
-/* The work split of that plan: rows and columns of a workgroup's tile and K ranges (what a profile was taken on); all 0 where the
- * plan answers 0. */
+/* The work split of that plan, for operands as the kernel for few rows takes them: rows and columns of a workgroup's tile and K ranges (what a
+ * profile was taken on); all 0 where the plan answers 0. */
 int mi355q_q8_mid_tile(int kind, int M, int N, int K, int* rows, int* columns, int* k_ranges);
 /* The same by the kernel that runs, with (scratch 1) a workspace that is large enough or without one: tile 0 / 1 = 32 x 32 / 32 x 64 with rings of
- * six stages, 2 / 3 = 64 x 64 / 32 x 64 with four, 4 .. 11 = 48, 64 .. 160 rows x 128 columns, -1 = another kernel takes the call; its K
+ * six stages, 2 / 3 = 64 x 64 / 32 x 64 with four, 4 .. 11 = 48, 64 .. 160 rows x 128 columns, 12 = the kernel for few rows, -1 = another kernel takes the call; its K
  * ranges (0 then); whether it adds them itself when the call has MI355Q_ZEROED_COUNTERS. */
 int mi355q_q8_mid_way(int kind, int M, int N, int K, int scratch, int* tile, int* k_ranges, int* in_kernel);
 
@@ -252,7 +253,7 @@ int mi355q_w8a8_int8_gemm(void* out, int32_t* acc_out, const int8_t* x, const in
  * serves both); without one, or with a smaller one, the unsplit launch runs. */
 size_t mi355q_w8a8_int8_workspace_bytes(int M, int N, int K);
 /* No counterpart in the reference.  What mi355q_w8a8_int8_gemm_ws launches for dense operands, no raw accumulators and a workspace of that size
- * (or of mi355q_q8_mid_plan's): 0 = the kernel for a few dozen to some hundred rows (kslab weights), 1 = tiles of 128 .. 256 rows x 128
+ * (or of mi355q_q8_mid_plan's): 0 = the kernels of mi355q_q8_mid_plan (kslab weights), 1 = tiles of 128 .. 256 rows x 128
  * columns, 2 = tiles of 256 rows x 128 .. 256 columns; and the K ranges it cuts K into. */
 int mi355q_w8a8_int8_plan(int M, int N, int K, int kslab, int* kernel, int* k_ranges);
 int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_t* x, const int8_t* w,

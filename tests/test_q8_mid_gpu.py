@@ -11,7 +11,7 @@ from vllm_gcu_amd.kernels.quantization import rearrange
 
 pytestmark = pytest.mark.gpu
 # (M, N, K): tiles of every height, with and without K ranges
-SHAPES = [(17, 64, 384), (31, 320, 128), (33, 512, 1152), (48, 1024, 7168), (63, 640, 640), (64, 4096, 2048), (65, 1024, 1024),
+SHAPES = [(17, 64, 384), (31, 320, 128), (33, 512, 4096), (48, 1024, 7168), (63, 640, 640), (64, 4096, 2048), (65, 1024, 1024),
           (96, 3072, 3584), (127, 256, 4096), (129, 1024, 5120), (130, 4096, 7168), (200, 2048, 1408), (257, 4608, 3584),
           (511, 4096, 4096), (512, 8192, 2048), (700, 512, 7168), (768, 1024, 4096), (1000, 3072, 3584), (1024, 4096, 4096),
           (1300, 640, 2048), (1535, 1536, 3584), (1536, 2048, 2048),
@@ -19,12 +19,13 @@ SHAPES = [(17, 64, 384), (31, 320, 128), (33, 512, 1152), (48, 1024, 7168), (63,
           # with K ranges; 144 and 160 rows with block scales
           (65, 1920, 3968), (66, 5504, 6272), (36, 8448, 3456), (84, 8576, 7552), (195, 2816, 6400), (131, 5504, 5888), (151, 5504, 6016)]
 BLOCK, SCALED, INT8 = 0, 1, 2            # kinds of mi355q_q8_mid_plan
+FEW = 12                                 # the kernel for few rows (csrc/q8_decode.hip) among the tiles of mi355q_q8_mid_way
 
 
 def _planned(kind, M, N, K):
     want = rt.host.q8_mid_plan(kind, M, N, K)
     print(f"case q8 mid kind={kind} M={M} N={N} K={K} workspace={want}", flush=True)
-    assert want >= 0, "another kernel takes this shape: the case tests nothing"
+    assert want >= 0 and way(kind, M, N, K)[0] < FEW, "another kernel takes this shape: the case tests nothing"
 
 
 @pytest.mark.parametrize("kind", [BLOCK, SCALED, INT8])
@@ -148,8 +149,8 @@ def test_fp8_rows_far_apart():
 
 
 # (kind, M, N, K) -> tile and K ranges: sums added in the kernel (up to 56 KiB of other ranges) or by a second launch
-RANGES = [(BLOCK, 31, 128, 2048, (32, 32, 3)), (INT8, 32, 128, 3328, (32, 32, 5)), (SCALED, 47, 128, 3968, (32, 32, 6)), (BLOCK, 100, 1024, 3584, (32, 32, 2)),
-          (SCALED, 47, 128, 10880, (32, 32, 15)), (INT8, 49, 128, 11648, (32, 32, 16)), (INT8, 17, 192, 10624, None), (BLOCK, 33, 1408, 3712, (32, 64, 5)),
+RANGES = [(BLOCK, 54, 1152, 2560, (32, 32, 3)), (INT8, 46, 768, 7936, (32, 32, 5)), (SCALED, 47, 128, 3968, (32, 32, 6)), (BLOCK, 100, 1024, 3584, (32, 32, 2)),
+          (SCALED, 47, 128, 10880, (32, 32, 15)), (INT8, 49, 128, 11648, (32, 32, 16)), (INT8, 17, 192, 10624, None), (BLOCK, 33, 1408, 4224, (32, 64, 5)),
           (BLOCK, 33, 896, 8832, (32, 64, 9)), (SCALED, 100, 2176, 4480, (64, 64, 3)), (SCALED, 129, 1024, 5120, (64, 64, 5)), (INT8, 129, 128, 10880, (32, 64, 11))]
 
 
@@ -194,7 +195,9 @@ MORE = [(BLOCK, 17, 128, 14336), (BLOCK, 129, 1152, 3968), (BLOCK, 121, 2432, 10
         (BLOCK, 129, 128, 9088), (BLOCK, 97, 2176, 8192), (BLOCK, 339, 2176, 6400), (BLOCK, 1285, 3072, 384), (BLOCK, 1450, 3072, 384),
         (SCALED, 17, 64, 14336), (SCALED, 129, 64, 2048), (SCALED, 33, 4096, 14336), (SCALED, 129, 64, 9088), (SCALED, 129, 1408, 14336),
         (SCALED, 152, 1408, 14336), (INT8, 33, 1408, 5120), (INT8, 129, 1152, 3968), (INT8, 106, 2432, 6400), (INT8, 129, 64, 3072), (INT8, 70, 1024, 8192),
-        (INT8, 97, 3072, 9088), (INT8, 482, 2432, 10880)]
+        (INT8, 97, 3072, 9088), (INT8, 482, 2432, 10880),
+        # the kernel for few rows; an int8 layer of it to fp32, which is the tile's, with ranges
+        (BLOCK, 33, 512, 1152), (SCALED, 24, 1024, 2048), (INT8, 33, 512, 1152), (INT8, 32, 128, 3328)]
 
 
 @pytest.mark.parametrize("zeroed", [True, False])
@@ -240,6 +243,7 @@ def test_k_ranges_leave_the_first_mib_as_it_was(kind, M, N, K, plan, zeroed):
 def test_without_room_for_k_ranges(kind, M, N, K):
     """Shapes whose plan cuts K, through the entry points without a workspace: sums that are exact, to the bit."""
     from vllm_gcu_amd import _lib
+    assert way(kind, M, N, K, 0)[0] < FEW
     print(f"case q8 without a workspace kind={kind} M={M} N={N} K={K}", flush=True)
     torch.manual_seed(M + N + K)
     x, w = (torch.randint(-3, 4, (r, K), device="cuda").to(torch.int8 if kind == INT8 else torch.float8_e4m3fn) for r in (M, N))

@@ -34,10 +34,9 @@ namespace mi355q {
 int kcontig_fp8_pc_launch(void* out, const void* a, const void* w, const float* a_scale, int scale_per_row,
                           const float* w_scale, int scale_per_col, const void* bias, int M, int K, int N,
                           int out_dtype, int w_layout, hipStream_t st);
-bool q8_mid_takes(int mode, int M, int N, int K, long ldx, const void* workspace, size_t workspace_bytes);
-int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
-                  int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* workspace,
-                  size_t workspace_bytes, bool zeroed, hipStream_t st);
+bool q8_mid_call(int& rc, int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
+                 int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* workspace,
+                 size_t workspace_bytes, bool zeroed, hipStream_t st);
 namespace {
 
 constexpr int FTM = 256, FTN = 128, FTKB = 128;
@@ -801,9 +800,10 @@ extern "C" int mi355q_fp8_block_gemm_ws(void* out, const void* x, const void* w,
              "fp8_block_gemm: operands too large for 32-bit tile offsets (M=%d N=%d K=%d)", M, N, K);
   MQ_REQUIRE(ldo >= N && ldo % 4 == 0, "fp8_block_gemm: output row stride %ld must be >= N and a multiple of 4", ldo);
   MQ_REQUIRE(out_dtype == MI355Q_F16 || out_dtype == MI355Q_BF16, "fp8_block_gemm: bad out dtype %d", out_dtype);
-  if (kslab && q8_mid_takes(0, M, N, K, ldx, workspace, workspace_bytes))
-    return q8_mid_launch(0, out, x, w, x_scale, 0, w_scale, 0, bias, 0, M, N, K, ldx, ldo, out_dtype,
-                         workspace, workspace_bytes, zeroed != 0, as_stream(stream));
+  int rc = 0;
+  if (kslab && q8_mid_call(rc, 0, out, x, w, x_scale, 0, w_scale, 0, bias, 0, M, N, K, ldx, ldo, out_dtype, workspace, workspace_bytes, zeroed != 0,
+                           as_stream(stream)))
+    return rc;
   F8Args a = {};
   a.out = out; a.x = (const uint8_t*)x; a.w = (const uint8_t*)w; a.x_scale = x_scale; a.w_scale = w_scale;
   a.bias = bias; a.M = M; a.N = N; a.K = K; a.ldx = ldx; a.ldw = ldw; a.ldo = ldo;
@@ -838,9 +838,11 @@ extern "C" int mi355q_fp8_scaled_gemm_ws(void* out, const void* x, const void* w
   MQ_REQUIRE(!kslab || N % 64 == 0, "fp8_scaled_gemm: weights in the kslab order need N=%d %% 64 == 0", N);
   MQ_REQUIRE(ldx >= K && (kslab || ldw >= K) && ldo >= N,
              "fp8_scaled_gemm: row strides (%ld, %ld, %ld) must cover K=%d / N=%d", ldx, ldw, ldo, K, N);
-  if (kslab && ldx % 16 == 0 && ldo % 4 == 0 && q8_mid_takes(1, M, N, K, ldx, workspace, workspace_bytes))
-    return q8_mid_launch(1, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, 0, M, N, K, ldx, ldo,
-                         out_dtype, workspace, workspace_bytes, zeroed != 0, as_stream(stream));
+  int rc = 0;
+  if (kslab && ldx % 16 == 0 && ldo % 4 == 0 &&
+      q8_mid_call(rc, 1, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, 0, M, N, K, ldx, ldo, out_dtype, workspace,
+                  workspace_bytes, zeroed != 0, as_stream(stream)))
+    return rc;
   // the MFMA tile kernel from 65 rows on when its 256 x 128 tiles fill a good part of the chip; below
   // (and for shapes it does not take) the weight-streaming kernel, which wants dense operands
   const long tiles = (long)((M + FTM - 1) / FTM) * (N / FTN);

@@ -26,10 +26,9 @@ double t8_price(int mode, int M, int N, int K, int splits, int* height);
 int int8_tile_launch(void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale, int ws_mul,
                      const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldw, long ldo, int out_dtype,
                      void* workspace, size_t workspace_bytes, hipStream_t st);
-bool q8_mid_takes(int mode, int M, int N, int K, long ldx, const void* workspace, size_t workspace_bytes);
-int q8_mid_launch(int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
-                  int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* workspace,
-                  size_t workspace_bytes, bool zeroed, hipStream_t st);
+bool q8_mid_call(int& rc, int mode, void* out, const void* x, const void* w, const float* x_scale, int xs_mul, const float* w_scale,
+                 int ws_mul, const void* bias, int bias_f32, int M, int N, int K, long ldx, long ldo, int out_dtype, void* workspace,
+                 size_t workspace_bytes, bool zeroed, hipStream_t st);
 namespace {
 
 constexpr int TM = 256, TKB = 128;                // tile rows of x, bytes of K per LDS tile row
@@ -969,9 +968,10 @@ extern "C" int mi355q_w8a8_int8_gemm_ws(void* out, int32_t* acc_out, const int8_
              "w8a8_int8_gemm: kslab weights need N=%d %% 64 == 0 and fewer than 4 Gi elements", N);
   MQ_REQUIRE(ldo >= N && ldo % 4 == 0, "w8a8_int8_gemm: output row stride %ld must be >= N and a multiple of 4", ldo);
   MQ_REQUIRE(out_dtype >= MI355Q_F16 && out_dtype <= MI355Q_F32, "w8a8_int8_gemm: bad out dtype %d", out_dtype);
-  if (kslab && !acc_out && q8_mid_takes(2, M, N, K, ldx, workspace, workspace_bytes))
-    return q8_mid_launch(2, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K, ldx,
-                         ldo, out_dtype, workspace, workspace_bytes, zeroed != 0, as_stream(stream));
+  int rc = 0;
+  if (kslab && !acc_out && q8_mid_call(rc, 2, out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K, ldx,
+                                       ldo, out_dtype, workspace, workspace_bytes, zeroed != 0, as_stream(stream)))
+    return rc;
   if (N % 128 == 0 && !acc_out && (size_t)N * K < ((size_t)1 << 32) && (size_t)256 * (size_t)ldx < ((size_t)1 << 32) &&
       (kslab || (size_t)128 * (size_t)ldw < ((size_t)1 << 32)) && int8_pick(M, N, K).tiles128)
     return int8_tile_launch(out, x, w, x_scale, x_scale_per_row ? 1 : 0, w_scale, w_scale_per_col ? 1 : 0, bias, bias_f32, M, N, K,
