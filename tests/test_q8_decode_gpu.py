@@ -176,3 +176,27 @@ def test_fp32_outputs_are_refused(M):
         ops.w8a8_block_fp8_matmul(x, w, xs, ws, [128, 128], torch.float32)
     torch.cuda.synchronize()
     assert (out == 7.0).all()
+
+
+@pytest.mark.parametrize("M,N,K,kslab,taken", [(1, 6144, 2560, True, False), (4, 8192, 2048, True, False), (8, 8192, 2048, True, True), (8, 7168, 4096, True, False),
+                                               (4, 6080, 4096, True, True), (4, 12288, 4096, True, False), (5, 12288, 4096, True, True), (1, 4096, 16384, False, True),
+                                               (2, 8192, 8192, False, False), (2, 8192, 6144, False, True), (8, 10240, 4096, False, False), (16, 12544, 4096, False, True),
+                                               (16, 14336, 4096, False, False), (1, 16384, 3712, False, True), (1, 20480, 8192, False, True)])
+def test_which_block_scaled_calls_of_up_to_16_rows_come_here(M, N, K, kslab, taken):
+    """Scales that lie 4 bytes off are not for this kernel, and the other one adds K in another order: the same bits say that it ran with the scales in place, too."""
+    print(f"case q8 decode who M={M} N={N} K={K} kslab={kslab}", flush=True)
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = _weights(0, M, K, gen), _weights(0, N, K, gen)
+    w = rearrange.to_kslab(w) if kslab else w
+    xs, blocks = torch.rand(M, K // 128, device="cuda", generator=gen) + 0.1, (N + 127) // 128 * (K // 128)
+    room = torch.empty(blocks + 1, device="cuda")
+    scales = torch.rand(blocks, device="cuda", generator=gen) * 1e-4
+    outs = []
+    for ws in (room[:-1].copy_(scales), room[1:]):
+        ws.copy_(scales)
+        out = torch.full((M, N), float("nan"), device="cuda").half()
+        _check(lib.mi355q_kcontig_gemm(_p(out), _p(x), _p(w), _p(xs), _p(ws), None, 1, 128, M, K, N, _lib.F16, _lib.F16, int(kslab), _stream()))
+        outs.append(out)
+    assert torch.equal(*outs) != taken
+    assert (outs[0].double() - outs[1].double()).norm() <= 2.0 ** -11 * outs[1].double().norm()

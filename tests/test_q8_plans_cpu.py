@@ -97,6 +97,12 @@ def test_the_plans_state_the_kernel_for_few_rows(kind, M, N, K):
     assert way(kind, 65, N, K)[0] not in (-1, 12)
 
 
+@pytest.mark.parametrize("kind,M,N,K", [(0, 36, 8192, 3200), (0, 40, 5248, 3200), (2, 24, 8320, 3584), (2, 32, 9216, 2176), (2, 17, 9216, 3072)])
+def test_rows_that_the_tiles_are_ahead_on(kind, M, N, K):
+    """us, the kernel for few rows / the tiles, the weights in the cache: 8.6 / 7.9, 7.9 / 7.9, 8.6 / 7.7, 6.8 / 6.6, 7.8 / 7.5."""
+    assert way(kind, M, N, K)[0] in range(12)
+
+
 def _launches(shapes):
     for kind, M, N, K in shapes:
         t, ranges, in_kernel = way(kind, M, N, K)

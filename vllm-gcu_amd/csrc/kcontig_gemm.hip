@@ -690,7 +690,7 @@ int fp8_block_grouped_launch(void* out, const void* a, const void* w, const floa
 int half_grouped_tile_launch(void* out, const void* a, const void* w, const float* topk_weights,
                              const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* npp, int numel, int topk,
                              int block_size, int max_blocks, int E, int K, int N, int dtype, int w_kslab, hipStream_t st);
-int q8_decode_tiles(int mode, int M, int N, int K);
+int q8_decode_tiles(int mode, int M, int N, int K, bool kslab);
 bool q8_decode_reads(const void* x, const void* w, const void* w_scale, const void* bias, const void* out);
 int q8_decode_launch(int tiles, int mode, int src, void* out, const void* x, const void* w, const float* x_scale, int sc_row, const void* c_scale,
                      const float* w_scale, int sc_col, const void* bias, int M, int N, int K, int kslab, int dtype, hipStream_t st);
@@ -700,7 +700,7 @@ int q8_decode_launch(int tiles, int mode, int src, void* out, const void* x, con
 int kcontig_fp8_pc_launch(void* out, const void* a, const void* w, const float* a_scale, int scale_per_row,
                           const float* w_scale, int scale_per_col, const void* bias, int M, int K, int N,
                           int out_dtype, int w_layout, hipStream_t st) {
-  if (const int tiles = (M <= 16 || w_layout) && q8_decode_reads(a, w, w_scale, bias, out) ? q8_decode_tiles(1, M, N, K) : 0)
+  if (const int tiles = q8_decode_reads(a, w, w_scale, bias, out) ? q8_decode_tiles(1, M, N, K, w_layout != 0) : 0)
     return q8_decode_launch(tiles, 1, 0, out, a, w, a_scale, scale_per_row ? 1 : 0, nullptr, w_scale, scale_per_col ? 1 : 0, bias, M, N, K, w_layout, out_dtype, st);
   KcArgs g = {};
   g.out = out; g.a = a; g.w = w; g.a_scale = a_scale; g.w_scale = w_scale; g.bias = bias;
@@ -903,9 +903,9 @@ extern "C" int mi355q_kcontig_gemm(void* out, const void* a, const void* w, cons
     MQ_REQUIRE(false, "kcontig_gemm: unknown quant_mode %d", quant_mode);
   }
   // (16-bit outputs; launch_mode refuses the others)
-  if (const int tiles = (mode == KC_FP8_BLOCK || mode == KC_INT8) && (out_dtype == MI355Q_F16 || out_dtype == MI355Q_BF16) && (M <= 16 || w_layout) &&
+  if (const int tiles = (mode == KC_FP8_BLOCK || mode == KC_INT8) && (out_dtype == MI355Q_F16 || out_dtype == MI355Q_BF16) &&
                                 q8_decode_reads(a, w, w_scale, bias, out)
-                            ? q8_decode_tiles(mode == KC_INT8 ? 2 : 0, M, N, K) : 0)
+                            ? q8_decode_tiles(mode == KC_INT8 ? 2 : 0, M, N, K, w_layout != 0) : 0)
     return q8_decode_launch(tiles, mode == KC_INT8 ? 2 : 0, 0, out, a, w, a_scale, 1, nullptr, (const float*)w_scale, 1, bias, M, N, K, w_layout, out_dtype,
                             as_stream(stream));
   int mt = pick_mt(M < 64 ? M : 64);

@@ -318,29 +318,40 @@ int launch_qd_waves(const QdArgs& a, int tiles, hipStream_t st) {
 }  // namespace
 
 // Column tiles per workgroup where codes of M rows go here, 0 where they do not.  The rows fill LDS at 128 KiB.
-//  - Up to 16 rows: below K 2048 kcontig_gemm_kernel is ahead (1024 x 4096 at one row 3.0 us against 3.5), and with two column tiles per workgroup its
-//    wavefronts catch up from 96 KiB on (8192 x 8192 at 16 rows 12.2 us against 12.9).
+//  - Up to 16 rows, against kcontig_gemm_kernel, 1700 launches with weights from memory and from the cache: below K 2048 that is ahead (1024 x 4096 at one row
+//    3.0 us against 3.5), and with two column tiles per workgroup its wavefronts catch up from 96 KiB on (8192 x 8192 at 16 rows 12.2 us against 12.9).  Block scales: from 6144
+//    columns on it has 32 columns to a workgroup as well, and is up to 9 % ahead over K 2560 .. 16384 (one row), and 64 from 12288 (up to 5 %, to four rows).
+//    Row-major weights, a tile of which is sixteen pieces K bytes apart: with two or four column tiles and a long K that is ahead (there / here, one row: block scales
+//    16384 x 8192 0.75, 12288 x 8192 0.88, 4096 x 14336 0.89, 8192 x 16384 0.80; scales outside 8192 x 16384 0.89, 12288 x 14336 0.92), with one and eight column tiles
+//    at no K (1.04 and more).
 //  - 17 .. 64 rows, against q8_mid_kernel, which reads a share of the rows for every 32 or 64 columns and walks K through a barrier per block: 22 layers of K 1024 .. 7168 at nine
 //    numbers of rows, with weights from memory and from the last-level cache.  From memory this is ahead nearly everywhere (1.0 .. 1.7 times); from the cache the copy of all rows into every
-//    workgroup costs more than the weights, so the lines are where that pays less than 3 %.  (us, from memory, there / here, and the ratio from the cache: block scales 2048 x 2048 at 20 6.0 /
+//    workgroup costs more than the weights, so the lines are where that pays less than 4 %.  (us, from memory, there / here, and the ratio from the cache: block scales 2048 x 2048 at 20 6.0 /
 //    3.5, 1.68, 2048 x 7168 at 24 / 48 6.2 / 5.3, 1.23, 6.9 / 6.5, 1.02, 4096 x 12288 at 24 13.2 / 12.6, 0.95; int8 4096 x 4096 at 24 7.8 / 6.0, 1.10, 3584 x 4608 at 20 7.2 / 6.2, 1.00, 4096 x 6144 at 24
-//    8.3 / 7.3, 0.91, 2048 x 11008 at 24 / 48 8.3 / 6.9, 1.09, 10.4 / 7.9, 1.07; per channel 4096 x 4096 at 20 / 32 7.9 / 5.9, 1.39, 8.0 / 7.0, 0.97, 3072 x 4608 at 24 6.6 / 6.3, 0.92.)
+//    8.3 / 7.3, 0.91, 2048 x 11008 at 24 / 48 8.3 / 6.9, 1.09, 10.4 / 7.9, 1.07; per channel 4096 x 4096 at 20 / 32 7.9 / 5.9, 1.39, 8.0 / 7.0, 0.97, 3072 x 4608 at 24 6.6 / 6.3, 0.92;
+//    block scales at 40 rows 3200 x 8192 0.92, from the cache 0.90, 3200 x 5120 1.00, 1.00; int8 at 24 3584 x 8320 1.15, 0.91, at 28 3072 x 11264 1.12, 1.00.)
 //  - 17 .. 32 rows of large layers, against the streamer (5120 x 13824 at 24, int8 16.2 / 15.0 and 1.08; 4096 x 28672 at 32 25.1 / 22.6 and 1.11).
-int q8_decode_tiles(int mode, int M, int N, int K) {
+int q8_decode_tiles(int mode, int M, int N, int K, bool kslab) {
   if (M < 1 || M > 64 || K % 128 != 0 || K > 65536 || N % 16 != 0 || (long)M * K > 128 * 1024 || (size_t)N * K >= ((size_t)1 << 31)) return 0;
   const int tiles = qd_tiles(N), rows = (M + 15) / 16;
-  if (M <= 16) return K < 2048 || (tiles == 2 && M * K > 96 * 1024) ? 0 : tiles;
-  if (K < 1024) return 0;
+  if (M <= 16) {
+    bool no = K < 2048 || (tiles == 2 && M * K > 96 * 1024);
+    if (kslab) no |= mode == QD_BLOCK && ((tiles == 2 && N >= 6144 && (K > 2048 || M <= 4)) || (tiles == 4 && N >= 12288 && M <= 4));
+    else if (tiles == 2) no |= mode == QD_BLOCK && K > 6144 && M <= 4;
+    else if (tiles == 4) no |= mode == QD_BLOCK ? K >= 4096 && (M <= 8 || N > 12544) : K >= 8192 && N > 12544;
+    return no ? 0 : tiles;
+  }
+  if (!kslab || K < 1024) return 0;
   if (M <= 32 && N >= 12288 && (long)K * N >= (1L << 26)) return tiles;
   if (tiles > 4) return 0;
   int most = 0;                                              // KiB of rows
   if (mode == QD_BLOCK) {
     if (rows == 2) most = tiles == 1 ? 128 : tiles == 2 ? 100 : 0;
-    else if (rows == 3 && tiles <= 2) most = M <= 40 || K <= 2048 ? 128 : 0;
+    else if (rows == 3 && tiles <= 2) most = K <= 2048 || (M <= 40 && N <= 5120) ? 128 : 0;
   } else if (mode == QD_PC) {
     most = tiles == 1 && rows == 2 ? 96 : 0;
   } else if (rows == 2) {
-    most = tiles == 1 ? 112 : tiles == 2 ? (K <= 2048 ? 64 : 0) : 96;
+    most = tiles == 1 ? 112 : tiles == 2 ? (K <= 2048 ? 64 : 0) : K <= 2048 || N >= 11008 ? 96 : 0;
   } else if (rows == 3) {
     most = tiles == 1 ? (M <= 40 ? 96 : 0) : tiles == 2 ? 120 : 112;
   } else {
