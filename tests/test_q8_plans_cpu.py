@@ -2,6 +2,7 @@
 from ctypes import byref, c_int
 
 import pytest
+import torch
 
 from vllm_gcu_amd import _lib
 
@@ -120,3 +121,32 @@ def test_every_launch_of_the_plans_is_among_the_shapes_that_are_run():
     run = set(_launches([(kind, *s) for kind in range(3) for s in gpu.SHAPES if kind == gpu.INT8 or s[1] % 128 == 0] +
                         [s[:4] for s in gpu.RANGES] + gpu.MORE))
     assert len(planned) > 50 and planned <= run, sorted(planned - run)
+
+
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="launches on addresses that are none")
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_the_kernel_for_few_rows_is_built_for_every_call_it_is_chosen_for(kind):
+    """Every launch that the rules ask for, codes in both weight layouts and rows quantised in the launch: without a GPU each ends at the device, not at a launch that
+    is not there."""
+    lib = _lib.load()
+    columns = [64, 320, 4096, 4224, 6144, 8192, 8320, 11008, 12288, 12544, 14336, 16384, 16512, 20480, 28672, 32768]
+    seen = set()
+
+    def ends_at_the_device(rc):
+        error = lib.mi355q_last_error().decode()
+        assert rc != 0 and "device" in error, error
+        seen.add("few" if "q8_decode" in error else "other")
+    for N in columns:
+        for K in [*range(128, 8192, 128), 10240, 16384, 20480, 28672, 65536]:
+            if N * K >= 1 << 31:
+                continue
+            for M in (1, 2, 3, 5, 8, 9, 16, 17, 20, 24, 25, 32, 33, 36, 40, 41, 48, 49, 56, 64):
+                for kslab in (0, 1) if M <= 16 else (1,):
+                    if kind == 1:
+                        ends_at_the_device(lib.mi355q_fp8_scaled_gemm(4096, 4096, 4096, 4096, 1, 4096, 1, None, M, N, K, K, 0 if kslab else K, N, _lib.BF16, None))
+                    else:
+                        ends_at_the_device(lib.mi355q_kcontig_gemm(4096, 4096, 4096, 4096, 4096, None, 1 + kind // 2, 128, M, K, N, _lib.F16, _lib.BF16, kslab, None))
+                for quant in (1, 2):
+                    if lib.mi355q_q8_quant_gemm_takes(kind, quant, M, N, K):
+                        ends_at_the_device(lib.mi355q_q8_quant_gemm(4096, 4096, 4096, 4096, 4096, 1, None, kind, quant, M, N, K, _lib.BF16, None))
+    assert seen == {"few", "other"}

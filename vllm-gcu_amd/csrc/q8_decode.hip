@@ -52,6 +52,7 @@ template <int MODE, int SRC, int DT, int NI, int W, int BPR, int MT>
 __global__ void __launch_bounds__(64 * W, 2)
 q8_decode_kernel(QdArgs a) {
   static_assert(NI <= W, "the tiles that a wavefront finishes are of the same columns");
+  static_assert(NI * BPR <= QD_RING, "a longer ring was slower");
   static_assert(SRC == QD_CODES || MODE != QD_BLOCK, "rows for block scales come quantised");
   static_assert(SRC != QD_CHANNEL || MODE == QD_INT8, "scales per column are int8's");
   typedef typename std::conditional<MODE == QD_INT8, i4, f4>::type acc_t;
@@ -216,7 +217,7 @@ q8_decode_kernel(QdArgs a) {
       }
     }
   };
-  const int mine = (KB - wave + W - 1) / W;    // (16 K blocks at least: none is negative)
+  const int mine = (KB - wave + W - 1) / W;    // (one K block at least, and wave < W: none is negative)
   int i = 0;
   for (; i + BPR < mine; i += BPR) {
 #pragma unroll
@@ -273,22 +274,36 @@ size_t qd_lds_bytes(int mode, int M, int K, int ni, int waves) {
 // (with four wavefronts K blocks are added in the order of kcontig_gemm_kernel, which takes codes of so short a K)
 int qd_waves(int K) { return K < 2048 ? 4 : 8; }
 
+// What q8_decode_tiles and quant_tiles can ask for, and is built.  Codes of up to 16 rows and rows for eight wavefronts have two K blocks to a wavefront at least, rows for
+// four (K below 2048) four at most; taller rows are as deep as their KiB allow; and the large layers of 17 .. 32 rows have four or eight column tiles and four K
+// blocks to a wavefront at least.
+constexpr bool qd_built(int mode, int src, int ni, int waves, int bpr, int mt) {
+  if (src != QD_CODES) return mt == 1 && (waves == 4 ? ni < 8 && bpr <= 4 : ni == 8 || bpr > 1);
+  if (mt == 1 || ni == 8) return mt <= 2 && (ni == 8 || bpr > 1);
+  if (mt == 2) return ni == 1 || (ni == 2 ? mode == QD_BLOCK || (mode == QD_INT8 && bpr <= 2) : mode == QD_INT8 || bpr == 2);
+  if (mt == 3) return bpr <= 4 && (mode == QD_INT8 || (mode == QD_BLOCK && ni <= 2));
+  return mode == QD_INT8 && ni >= 2 && bpr <= 2;
+}
+
 template <int MODE, int SRC, int DT, int NI, int W, int BPR, int MT>
 int launch_qd_rows(const QdArgs& a, hipStream_t st) {
-  static hipError_t attr = hipFuncSetAttribute((const void*)q8_decode_kernel<MODE, SRC, DT, NI, W, BPR, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
-  MQ_REQUIRE(attr == hipSuccess, "q8_decode: cannot reserve LDS: %s", hipGetErrorString(attr));
-  hipLaunchKernelGGL((q8_decode_kernel<MODE, SRC, DT, NI, W, BPR, MT>), dim3((a.N + 16 * NI - 1) / (16 * NI)), dim3(64 * W), qd_lds_bytes(MODE, a.M, a.K, NI, W), st, a);
-  MQ_LAUNCH_CHECK("q8_decode");
-  return 0;
+  if constexpr (qd_built(MODE, SRC, NI, W, BPR, MT)) {
+    static hipError_t attr = hipFuncSetAttribute((const void*)q8_decode_kernel<MODE, SRC, DT, NI, W, BPR, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
+    MQ_REQUIRE(attr == hipSuccess, "q8_decode: cannot reserve LDS: %s", hipGetErrorString(attr));
+    hipLaunchKernelGGL((q8_decode_kernel<MODE, SRC, DT, NI, W, BPR, MT>), dim3((a.N + 16 * NI - 1) / (16 * NI)), dim3(64 * W), qd_lds_bytes(MODE, a.M, a.K, NI, W), st, a);
+    MQ_LAUNCH_CHECK("q8_decode");
+    return 0;
+  }
+  MQ_REQUIRE(false, "q8_decode: M=%d N=%d K=%d is not covered", a.M, a.N, a.K);
 }
 template <int MODE, int SRC, int DT, int NI, int W, int BPR>
 int launch_qd(const QdArgs& a, hipStream_t st) {
-  if constexpr (SRC == QD_CODES) {
-    if constexpr (MODE == QD_INT8 && (NI == 2 || NI == 4)) if (a.M > 48) return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 4>(a, st);
-    if constexpr (MODE == QD_INT8 ? NI <= 4 : MODE == QD_BLOCK && NI <= 2) if (a.M > 32) return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 3>(a, st);
-    if (a.M > 16) return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 2>(a, st);
+  switch ((a.M + 15) / 16) {
+    case 1: return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 1>(a, st);
+    case 2: return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 2>(a, st);
+    case 3: return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 3>(a, st);
+    default: return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 4>(a, st);
   }
-  return launch_qd_rows<MODE, SRC, DT, NI, W, BPR, 1>(a, st);
 }
 template <int MODE, int SRC, int DT, int NI, int W>
 int launch_qd_ring(const QdArgs& a, hipStream_t st) {
@@ -304,9 +319,7 @@ int launch_qd_tiles(const QdArgs& a, int tiles, hipStream_t st) {
     case 1: return launch_qd_ring<MODE, SRC, DT, 1, W>(a, st);
     case 2: return launch_qd_ring<MODE, SRC, DT, 2, W>(a, st);
     case 4: return launch_qd_ring<MODE, SRC, DT, 4, W>(a, st);
-    default:
-      if constexpr (W >= 8) return launch_qd_ring<MODE, SRC, DT, 8, W>(a, st);
-      MQ_REQUIRE(false, "q8_decode: N=%d, K=%d is not covered", a.N, a.K);
+    default: return launch_qd_ring<MODE, SRC, DT, 8, W>(a, st);
   }
 }
 template <int MODE, int SRC, int DT>
