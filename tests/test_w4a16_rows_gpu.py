@@ -103,6 +103,15 @@ def test_taken_where_the_tiles_loop_is_the_slow_one(M, K, N, g, dtype):
     assert torch.equal(ops.w4a16_gemm(x, w, scales, zp, None, g), ops.w4a16_gemm(x, w, scales, zp, None, g, family=4))
 
 
+@pytest.mark.parametrize("N", [7168, 8192])
+@pytest.mark.parametrize("M", [16, 24])
+def test_streaming_kernel_halves_of_slabs_in_two_ranges(M, N):
+    """Dealt out to the XCDs by slabs, and in turn where they fill the chip: every column is written either way."""
+    print(f"case w4a16 stream halves M={M} N={N}", flush=True)
+    q, z, s, x = _case(M + N, M, 1024, N, 128, torch.float16, exact=True)
+    assert torch.equal(_run(q, z, s, x, 128, family=1, split_k=2 | 4 << 8), torch.from_numpy(_want(q, z, s, x, 128)).half())
+
+
 @pytest.mark.parametrize("M,K,N,dtype,family", [(17, 2560, 14336, torch.float16, 4), (32, 1408, 19328, torch.float16, 4), (24, 7168, 2560, torch.float16, 1),
                                                 (32, 14080, 4352, torch.float16, 1), (30, 14336, 4096, torch.bfloat16, 1), (24, 2432, 18944, torch.bfloat16, 4)])
 def test_17_to_32_rows_without_a_second_launch(M, K, N, dtype, family):

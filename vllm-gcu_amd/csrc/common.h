@@ -165,7 +165,7 @@ __device__ __forceinline__ void lds_copy16_next(uint32_t voff, const void* sbase
 // of a column tile share one L2 and its weights pass it once, whatever the number of column tiles.  Column tiles that are parts of one
 // block of the weights' layout (8 KiB of a slab or of a kslab group) belong on one XCD for the same reason: dealt out in turn, eight L2s take
 // pieces of 1 .. 4 KiB out of every block, with its scales (us at one row, weights out of the caches, in turn -> here: int8 8192 x 8192 16.1 -> 12.7,
-// 8192 x 10240 21.5 -> 18.6, 4096 x 4096 6.0 -> 5.4; W4A16 4096 x 6144 5.9 -> 5.3, 8192 x 8192 at 1 / 16 9.7 / 11.9 -> 8.9 / 10.6; a layer of 64 experts of
+// 8192 x 10240 21.5 -> 18.6, 4096 x 4096 6.0 -> 5.4; W4A16 4096 x 6144 5.9 -> 5.3, 8192 x 8192 at 1 9.7 -> 8.9; a layer of 64 experts of
 // 2048 x 2048, six to a token, at 4 tokens 31.0 -> 29.2).
 __device__ __forceinline__ int xcd_tile() {
   const int share = (int)gridDim.x >> 3, odd = gridDim.x & 7, x8 = blockIdx.x & 7;

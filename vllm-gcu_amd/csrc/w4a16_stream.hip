@@ -30,6 +30,7 @@ struct StreamArgs {
   int splits;
   int per;           // K blocks per split: ceil(K / 128 / splits) (host-side: no division in the kernel's prologue)
   int qrows;         // K / gs
+  int one_xcd;       // the parts of a slab go to one XCD
   float* partial;    // [splits][16*MT][N]
   int* counters;     // four per blockIdx.x (<= N/16 workgroups, one per wavefront), zero between launches
 };
@@ -192,9 +193,7 @@ w4a16_stream_kernel(StreamArgs a) {
   const int c = lane & 15, kq = lane >> 4;
   constexpr int TG = 8 / NT;                          // tile groups per slab
   constexpr int HW = NT >= 2 ? NT / 2 : 1;            // packed 16-bit pairs per lane
-  // parts of a slab on one XCD; behind more than two K ranges they were 0 .. 4 % slower so (14336 x 4096 at 32 rows 14.5 -> 15.1), and
-  // whole slabs have nothing to share
-  const int group = NT < 8 && gridDim.y <= 2 ? xcd_tile() : (int)blockIdx.x, slab = group / TG, t0 = (group % TG) * NT, split = blockIdx.y;
+  const int group = NT < 8 && a.one_xcd ? xcd_tile() : (int)blockIdx.x, slab = group / TG, t0 = (group % TG) * NT, split = blockIdx.y;
   const int G = a.K >> 7;
   const int per = a.per;
   const int gb = split * per;
@@ -602,6 +601,9 @@ int w4a16_stream_launch(void* out, const void* x, const int32_t* qweight, const 
   a.splits = splits;
   a.per = (G + splits - 1) / splits;
   a.qrows = K / group_size;
+  // (behind more than two K ranges they were 0 .. 4 % slower so, 14336 x 4096 at 32 rows 14.5 -> 15.1; and halves in two ranges that fill the chip up to 5 %, 8192 columns,
+  // us so / in turn at 32 rows: K 6144 13.8 / 13.1, 8192, bf16, 15.5 / 14.9, where those of 6144 and 7168 columns gain 2 to 3 %.  Whole slabs have nothing to share)
+  a.one_xcd = splits <= 2 && !(plan.nt == 4 && splits == 2 && N / 64 * 2 >= device_cu_count());
   a.partial = nullptr;
   a.counters = nullptr;
   if (splits > 1) {
