@@ -175,8 +175,10 @@ kcontig_gemm_kernel(KcArgs a) {
       return;
     }
   }
-  // (KS: parts of a group of 64 columns on one XCD; whole groups in turn, 8192 x 28672 at 8 rows 37.5 us against 39.2)
-  const int n0 = KS ? (NI < 4 ? xcd_tile() : (int)blockIdx.x) * (16 * NI) : GLUQ ? (wave >> 1) * (N >> 1) + blockIdx.x * 128 + (wave & 1) * 64 : blockIdx.x * 256 + wave * 64;
+  // (KS: parts of a group of 64 columns on one XCD; whole groups in turn, 8192 x 28672 at 8 rows 37.5 us against 39.2, and 16-bit weights from the second
+  // round of workgroups on, 2 .. 5 %, bytes there within 2 % either way)
+  const bool one_xcd = NI < 4 && (T::WBYTES < 2 || gridDim.x <= 256);
+  const int n0 = KS ? (one_xcd ? xcd_tile() : (int)blockIdx.x) * (16 * NI) : GLUQ ? (wave >> 1) * (N >> 1) + blockIdx.x * 128 + (wave & 1) * 64 : blockIdx.x * 256 + wave * 64;
   if (n0 >= N) return;
   // Operands are addressed through buffer descriptors: a 32-bit lane offset plus a scalar K-block offset
   // per load (no 64-bit address arithmetic in the loop; the host checks that one expert's weights, the
