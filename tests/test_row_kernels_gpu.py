@@ -1,9 +1,13 @@
 """The row-in-registers quantisers and norms at the edges of their launch shapes: rows that end inside a piece, one
 piece short of and past a whole number of pieces, fewer and more rows than the rule's steps, rows too long for
 registers and rows whose address or length needs the one-element loops."""
+import ctypes
+import os
+
 import pytest
 import torch
 
+from vllm_gcu_amd import _lib
 from vllm_gcu_amd.kernels import _custom_ops  # noqa: F401  (registers the ops)
 
 pytestmark = pytest.mark.gpu
@@ -82,8 +86,8 @@ def test_silu_and_sum_index_arithmetic(rows, d):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_group_fp8_codes_of_every_pair(dtype):
-    """Every value against every largest magnitude of its group's binade that there is (the division depends on the fractions alone): the code is that of
-    the IEEE quotient.  An infinity in the group makes zeros of the rest, with their signs."""
+    """Every fraction against every largest one, over the ten binades whose codes are normal (test_short_forms_give_the_bits_of_the_plain_ones has all pairs): the code is that
+    of the IEEE quotient, as torch has it.  An infinity in the group makes zeros of the rest, with their signs."""
     bits = 10 if dtype == torch.float16 else 7
     one = 0x3C00 if dtype == torch.float16 else 0x3F80
     print(f"case group fp8 codes of every pair {dtype}", flush=True)
@@ -128,3 +132,17 @@ def test_silu_of_every_gate(dtype):
     digits, least = (11, 2.0 ** -24) if dtype == torch.float16 else (8, 2.0 ** -126)
     bound = want.abs() * (2.0 ** -digits + 2.0 ** -20) + least + a.abs() * 2.0 ** -128
     assert ((y.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("what,dtype", [("reciprocal", torch.float16), ("gate", torch.float16), ("gate", torch.bfloat16), ("codes", torch.float16), ("codes", torch.bfloat16)])
+def test_short_forms_give_the_bits_of_the_plain_ones(what, dtype):
+    """On the GPU, over every operand: the reciprocal of three instructions from 1 to 2^126; the gate of eight with every gate and up value there is; the fp8 codes of every
+    value against every largest magnitude of a row."""
+    print(f"case short forms {what} {dtype}", flush=True)
+    check = ctypes.CDLL(os.path.join(os.path.dirname(_lib.LIB_PATH), "libmi355q_bench.so")).mi355q_bench_check_arithmetic
+    check.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    wrong = torch.zeros(1, dtype=torch.int64, device="cuda")
+    assert check(["reciprocal", "gate", "codes"].index(what), {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}[dtype], wrong.data_ptr(),
+                 torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert wrong.item() == 0

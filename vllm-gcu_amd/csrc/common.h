@@ -246,8 +246,13 @@ __device__ __forceinline__ float silu_mul(float a, float b) {
   return a * (1.0f / (1.0f + expf(-a))) * b;      // left * sigmoid(left) * right
 }
 
-// ... of eight of each, to the same bits.  An estimate and its Newton step are the correctly rounded reciprocal of every float from 1 to 2^126 (all of them were
-// compared with the division, which takes ten instructions for these three); gates below -87, whose reciprocal is no normal number, take the division.
+// An estimate and its Newton step: the correctly rounded reciprocal of every float from 1 to 2^126, in three instructions where the division takes ten
+__device__ __forceinline__ float short_reciprocal(float s) {
+  const float y = __builtin_amdgcn_rcpf(s);
+  return __builtin_fmaf(__builtin_fmaf(-s, y, 1.0f), y, y);
+}
+// ... of eight of each, to the same bits for every gate and up value of 16 bits; gates below -87, whose reciprocal is no normal number, take the division.  (This and the
+// codes below are compared with the plain forms over all operands, csrc/bench/arith.hip.)
 __device__ __forceinline__ void silu_mul8(const float* a, const float* b, float* y) {
   float s[8], r[8], m = 1.0f;
 #pragma unroll
@@ -259,10 +264,7 @@ __device__ __forceinline__ void silu_mul8(const float* a, const float* b, float*
     for (int e = 0; e < 8; ++e) r[e] = 1.0f / s[e];
   } else {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float r0 = __builtin_amdgcn_rcpf(s[e]);
-      r[e] = __builtin_fmaf(__builtin_fmaf(-s[e], r0, 1.0f), r0, r0);
-    }
+    for (int e = 0; e < 8; ++e) r[e] = short_reciprocal(s[e]);
   }
   // (here, so that the last product is rounded to fp16 at once, as the single ones are)
 #pragma unroll
@@ -323,16 +325,15 @@ __device__ __forceinline__ float max_abs2(float m, float a, float b) {
 
 // a / s for many a and one s, with the result of the IEEE division, for what the quantisers divide: a of 16 bits, s = max(largest |a|, 1e-10) / 448.
 // The correctly rounded reciprocal is made once per divisor (an estimate and its Newton step), per dividend the quotient estimate and its
-// correction by the exact residual.  s is normal and |a / s| <= 448; a residual can only underflow where the quotient is far below the smallest fp8 step.  (That
-// one correction is enough is known for every pair of 16-bit values there is: all of them give the division's fp8 code.)  An infinite s, of a group with an
+// correction by the exact residual.  s is normal and |a / s| <= 448; a residual can only underflow where the quotient is far below the smallest fp8 step.  (One
+// correction is enough: every pair of finite 16-bit values gives the division's fp8 code.)  An infinite s, of a group with an
 // infinity, makes zeros of what is finite and NaN of the infinities; the residual is taken as s q - a, whose zero leaves the sign of a zero quotient alone.
 struct SharedDivisor {
   float s, y;
   __device__ __forceinline__ explicit SharedDivisor(float s_) {
-    const float y0 = __builtin_amdgcn_rcpf(s_), y1 = __builtin_fmaf(__builtin_fmaf(-s_, y0, 1.0f), y0, y0);
     const bool finite = s_ < __builtin_inff();
     s = finite ? s_ : 0.0f;
-    y = finite ? y1 : 0.0f;
+    y = finite ? short_reciprocal(s_) : 0.0f;
   }
   __device__ __forceinline__ float div(float a) const {
     const float q = a * y;
