@@ -472,7 +472,7 @@ int mi355q_moe_w4a16_unsorted_sum(void* out, const void* a, const int32_t* w, co
  * [M, K] and the router's ids [M, topk] (int32 or int64), without alignment and quantisers: kslab weights w1 [E, 2 I, K], w2 [E, K, I] with
  * block scales f32 [E, 2 I / 128, K / 128], [E, K / 128, I / 128]; out [M, K] may be x.  Slots whose id is outside [0, E) add nothing.  Sums as
  * mi355q_moe_fp8_gate_up_quant and mi355q_moe_gemm make them, K blocks in another order.  _bytes: of the workspace (any contents), 0 where a call is not
- * covered (up to four tokens and 64 slots, K and I multiples of 128 up to 32768); _wanted: 1 where it is ahead of the sorted launches.
+ * covered (up to four tokens and 64 slots, K and I multiples of 128, of which four rows, or as many as there are slots, fit 128 KiB as bytes); _wanted: 1 where it is ahead of the sorted launches.
  * Operands aligned to 16 bytes. */
 size_t mi355q_moe_fp8_unsorted_bytes(int M, int topk, int E, int K, int I);
 int mi355q_moe_fp8_unsorted_wanted(int M, int topk, int E, int K, int I);

@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 # tokens, slots per token, experts, K, I
 SHAPES = [(1, 1, 1, 128, 128), (1, 8, 128, 2304, 1152), (2, 6, 64, 1024, 640), (4, 2, 4, 384, 512), (3, 8, 256, 7168, 2048), (3, 3, 3, 640, 256), (4, 8, 16, 2176, 384),
-          (4, 4, 40, 4096, 1024), (2, 2, 2, 32768, 128), (1, 16, 64, 8320, 2432), (4, 16, 128, 2560, 896)]
+          (4, 4, 40, 4096, 1024), (2, 2, 2, 32768, 128), (1, 16, 64, 8320, 2432), (4, 16, 128, 2560, 896),
+          (1, 1, 2, 131072, 128), (1, 2, 2, 128, 65536), (1, 1, 2, 256, 65664)]
 
 
 def _quantise(x):
@@ -74,6 +75,7 @@ def test_what_is_not_covered():
     lib = _lib.load()
     need = lib.mi355q_moe_fp8_unsorted_bytes
     assert need(5, 1, 8, 1024, 1024) == 0 and need(4, 17, 128, 1024, 1024) == 0 and need(1, 1, 8, 1024 + 64, 1024) == 0 and need(4, 1, 8, 32768 + 128, 128) == 0
+    assert need(1, 2, 8, 65536, 128) and not need(1, 2, 8, 65536 + 128, 128) and need(1, 1, 8, 128, 131072) and not need(1, 1, 8, 128, 131072 + 128)
     assert lib.mi355q_moe_fp8_unsorted_wanted(1, 8, 256, 7168, 2048) and not lib.mi355q_moe_fp8_unsorted_wanted(4, 8, 256, 7168, 2048)
     x = torch.zeros(1024, dtype=torch.uint8, device="cuda").data_ptr()
     assert lib.mi355q_moe_fp8_unsorted(x, x, x, x, x, x, x, x, 0, 1, 1, 1, 128, 128, _lib.BF16, x, 8, None) != 0         # workspace too small
