@@ -15,7 +15,7 @@
 // 19.8 -> 15.3; 8192 x 10240 at 1 / 8 18.7 / 19.1 -> 17.1 / 16.5; 4096 x 28672 at 1 21.7 -> 21.4, rows 23.9 -> 21.4.
 // From 17 rows on the weights of a workgroup are multiplied by two, three or four tiles of rows; what it takes is then the copy of the rows, which every
 // workgroup makes in whole (the figures stand with the rule, q8_decode_tiles).
-#include "rows8.h"
+#include "q8_few.h"
 
 #include <type_traits>
 
@@ -39,20 +39,12 @@ struct QdArgs {
 };
 
 constexpr int qd_pieces(int src, int waves) { return src == QD_CODES ? 16 : 40 / waves; }   // of x that a thread holds
-constexpr int QD_RING = 8;                                   // tiles of 16 columns x one K block that a wavefront has on their way at most
-// (barriers of LDS traffic alone: the weights stay on their way over them)
-__device__ __forceinline__ void qd_lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // NI tiles of 16 columns, W wavefronts, BPR K blocks of each on their way, MT tiles of 16 rows
 template <int MODE, int SRC, int DT, int NI, int W, int BPR, int MT>
 __global__ void __launch_bounds__(64 * W, 2)
 q8_decode_kernel(QdArgs a) {
   static_assert(NI <= W, "the tiles that a wavefront finishes are of the same columns");
-  static_assert(NI * BPR <= QD_RING, "a longer ring was slower");
   static_assert(SRC == QD_CODES || MODE != QD_BLOCK, "rows for block scales come quantised");
   static_assert(SRC != QD_CHANNEL || MODE == QD_INT8, "scales per column are int8's");
   typedef typename std::conditional<MODE == QD_INT8, i4, f4>::type acc_t;
@@ -112,27 +104,17 @@ q8_decode_kernel(QdArgs a) {
 #pragma unroll
   for (int t = 0; t < NI; ++t) {
     const int n = n0 + 16 * t;
-    woff[t] = n >= N ? 0x80000000u : a.kslab ? (uint32_t)((((n >> 6) * KB) * 4 + ((n >> 4) & 3)) * 2048 + lane * 16) : (uint32_t)((n + r16) * K + 32 * q);
+    woff[t] = n >= N ? FEW_NONE : a.kslab ? few_kslab_offset(n, KB, lane) : (uint32_t)((n + r16) * K + 32 * q);
   }
-  u4 w[BPR][NI][2];
-  auto ask = [&](int b, int kb) {                            // (past the last K block: an offset beyond the buffer, no traffic)
-    const uint32_t none = kb < KB ? 0u : 0x80000000u;
-    const int at = kb < KB ? kb * (int)kstride : 0;
-#pragma unroll
-    for (int t = 0; t < NI; ++t)
-#pragma unroll
-      for (int v = 0; v < 2; ++v)
-        w[b][t][v] = bitcast<u4>(__builtin_amdgcn_raw_buffer_load_b128(wres, (int)(woff[t] | none), at + v * (int)vstride, 2));
-  };
+  FewWeights<NI, BPR> ring;
+  auto ask = [&](int b, int kb) { ring.ask(b, wres, woff, kb, KB, kstride, vstride); };
 #pragma unroll
   for (int b = 0; b < BPR; ++b) ask(b, wave + W * b);
   __builtin_amdgcn_sched_barrier(0);
 
-  // ---- x into LDS as codes.  Chunk c of row r's K block lies at position (c >> 1 | (c & 1) << 2) ^ (r & 7), so that the sixteen rows and
-  // four lane quarters of an operand read fall on different banks
-  auto chunk_at = [&](int kb, int r, int c) { return (uint32_t)((kb * M + r) * 128 + (((c >> 1) | ((c & 1) << 2)) ^ (r & 7)) * 16); };
+  // ---- x into LDS as codes
   if (SRC == QD_TOKEN) {
-    qd_lds_barrier();                                        // row_max is cleared
+    few_lds_barrier();                                        // row_max is cleared
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
       if (p * THREADS >= total) break;
@@ -144,7 +126,7 @@ q8_decode_kernel(QdArgs a) {
       mx = lane_group_max(mx, 16);                           // (a row is a whole number of sixteen pieces)
       if ((lane & 15) == 0 && i < total) atomicMax(&row_max[a.row_pieces.div((uint32_t)i)], bitcast<uint32_t>(mx));
     }
-    qd_lds_barrier();
+    few_lds_barrier();
   }
 #pragma unroll
   for (int p = 0; p < PIECES; ++p) {
@@ -152,7 +134,7 @@ q8_decode_kernel(QdArgs a) {
     const int i = tid + p * THREADS;
     const int r = (int)a.row_pieces.div((uint32_t)min(i, total - 1)), c = i - r * (int)a.row_pieces.d;
     if (SRC == QD_CODES) {
-      if (i < total) *(u4*)(lds + chunk_at(c >> 3, r, c & 7)) = xv[p];
+      if (i < total) *(u4*)(lds + few_chunk_at(M, c >> 3, r, c & 7)) = xv[p];
     } else {
       float y[8];
       unpack8<DT>(xv[p], y);
@@ -166,7 +148,7 @@ q8_decode_kernel(QdArgs a) {
       } else {
         codes = RowFp8(bitcast<float>(row_max[r])).codes(y);
       }
-      if (i < total) *(u2*)(lds + chunk_at(c >> 4, r, (c & 15) >> 1) + (c & 1) * 8) = codes;
+      if (i < total) *(u2*)(lds + few_chunk_at(M, c >> 4, r, (c & 15) >> 1) + (c & 1) * 8) = codes;
     }
   }
   float* const xs_l = (float*)(lds + (size_t)M * K);         // [row][K block], then the columns' scales
@@ -180,7 +162,7 @@ q8_decode_kernel(QdArgs a) {
   static_assert(SRC != QD_TOKEN || MT == 1, "sixteen largest magnitudes");
   if (SRC == QD_TOKEN && stores)
     xs[0] = MODE == QD_INT8 ? RowInt8(bitcast<float>(row_max[r16])).scale : RowFp8(bitcast<float>(row_max[r16])).scale;
-  qd_lds_barrier();
+  few_lds_barrier();
 
   // ---- K blocks wave, wave + W, ..
   acc_t acc[MT][NI];
@@ -194,58 +176,37 @@ q8_decode_kernel(QdArgs a) {
   auto multiply = [&](int b, int kb) {
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
-      const u4 xo[2] = {*(const u4*)(lds + chunk_at(kb, row[j], 2 * q)), *(const u4*)(lds + chunk_at(kb, row[j], 2 * q + 1))};
+      const FewOperand x(lds, M, kb, row[j], q);
       const float sc = MODE == QD_BLOCK ? xs_l[row[j] * KB + kb] * ws_l[kb] : 1.0f;
 #pragma unroll
       for (int t = 0; t < NI; ++t) {
         if constexpr (MODE == QD_INT8) {
 #pragma unroll
-          for (int v = 0; v < 2; ++v) acc[j][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bitcast<i4>(w[b][t][v]), bitcast<i4>(xo[v]), acc[j][t], 0, 0, 0);
+          for (int v = 0; v < 2; ++v) acc[j][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bitcast<i4>(ring.w[b][t][v]), bitcast<i4>(x.v[v]), acc[j][t], 0, 0, 0);
+        } else if constexpr (MODE == QD_BLOCK) {
+          acc[j][t] += sc * few_fp8_products(ring.w[b][t], x, (f4){0.f, 0.f, 0.f, 0.f});
         } else {
-          f4 part = MODE == QD_BLOCK ? (f4){0.f, 0.f, 0.f, 0.f} : acc[j][t];
-#pragma unroll
-          for (int v = 0; v < 2; ++v) {
-            const u4 wv = w[b][t][v];
-            part = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)((unsigned long)wv[0] | ((unsigned long)wv[1] << 32)),
-                                                              (long)((unsigned long)xo[v][0] | ((unsigned long)xo[v][1] << 32)), part, 0, 0, 0);
-            part = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)((unsigned long)wv[2] | ((unsigned long)wv[3] << 32)),
-                                                              (long)((unsigned long)xo[v][2] | ((unsigned long)xo[v][3] << 32)), part, 0, 0, 0);
-          }
-          if constexpr (MODE == QD_BLOCK) acc[j][t] += sc * part;
-          else acc[j][t] = part;
+          acc[j][t] = few_fp8_products(ring.w[b][t], x, acc[j][t]);
         }
       }
     }
   };
-  const int mine = (KB - wave + W - 1) / W;    // (one K block at least, and wave < W: none is negative)
-  int i = 0;
-  for (; i + BPR < mine; i += BPR) {
-#pragma unroll
-    for (int b = 0; b < BPR; ++b) {
-      multiply(b, wave + W * (i + b));
-      ask(b, wave + W * (i + b + BPR));
-    }
-  }
-#pragma unroll
-  for (int b = 0; b < BPR; ++b)
-    if (i + b < mine) multiply(b, wave + W * (i + b));
+  few_walk<BPR, W>(KB, wave, multiply, ask);
 
   // ---- the wavefronts' sums, in wavefront order
-  qd_lds_barrier();                                          // everybody has read x
+  few_lds_barrier();                                          // everybody has read x
   acc_t* const red = (acc_t*)lds;
 #pragma unroll
   for (int j = 0; j < MT; ++j)
 #pragma unroll
     for (int t = 0; t < NI; ++t) red[(wave * NI * MT + j * NI + t) * 64 + lane] = acc[j][t];
-  qd_lds_barrier();
+  few_lds_barrier();
   if (!stores) return;
 #pragma unroll
   for (int f = 0; f < FIN; ++f) {
     const int m = stored_row(f);
     if (m >= M) return;
-    acc_t sum = red[(wave + W * f) * 64 + lane];
-#pragma unroll
-    for (int s = 1; s < W; ++s) sum += red[(s * NI * MT + wave + W * f) * 64 + lane];
+    const acc_t sum = few_sum<W>(red, NI * MT, wave + W * f, lane);
     float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {

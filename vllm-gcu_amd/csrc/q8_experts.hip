@@ -12,7 +12,7 @@
 // -> 25.8 / 35.5 / 42.5; 128 of 4096 / 1024 45.0 / 49.1 / 61.6 -> 26.6 / 41.5 / 57.8; 256 of 7168 / 2048 at 1 74.8 -> 64.2; six to a token, 128 of 6144 / 512 at 1 / 2 / 3
 // 48.3 / 53.9 / 56.8 -> 23.2 / 37.2 / 48.1.
 #include "moe_slots.h"
-#include "rows8.h"
+#include "q8_few.h"
 
 #include <algorithm>
 #include <cmath>
@@ -37,12 +37,6 @@ struct QeArgs {
 };
 
 constexpr int QE_W = 8, QE_PIECES = 4, SHIFT = 2;            // (a token has an expert once: a block of four slots takes all rows that four tokens give it)
-
-__device__ __forceinline__ void qe_lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // GATED: x holds gate and up, and what is quantised is what silu_and_mul makes of them; else the rows of the slots' tokens.  NI tiles of 16 columns,
 // eight wavefronts that take the K blocks in turn, BPR K blocks of each on their way; blocks of 2^SHIFT slots.
@@ -85,25 +79,14 @@ q8_experts_kernel(QeArgs a) {
   const rsrc_t wres = make_rsrc(a.w + (size_t)blk.expert * N * K, (uint32_t)N * (uint32_t)K);
   uint32_t woff[NI];
 #pragma unroll
-  for (int t = 0; t < NI; ++t) {
-    const int n = n0 + 16 * t;
-    woff[t] = n >= N ? 0x80000000u : (uint32_t)((((n >> 6) * KB) * 4 + ((n >> 4) & 3)) * 2048 + lane * 16);
-  }
-  u4 w[BPR][NI][2];
-  auto ask = [&](int b, int kb) {                            // (past the last K block: an offset beyond the buffer, no traffic)
-    const uint32_t none = kb < KB ? 0u : 0x80000000u;
-    const int at = kb < KB ? kb * 8192 : 0;
-#pragma unroll
-    for (int t = 0; t < NI; ++t)
-#pragma unroll
-      for (int v = 0; v < 2; ++v) w[b][t][v] = bitcast<u4>(__builtin_amdgcn_raw_buffer_load_b128(wres, (int)(woff[t] | none), at + v * 1024, 2));
-  };
+  for (int t = 0; t < NI; ++t) woff[t] = n0 + 16 * t >= N ? FEW_NONE : few_kslab_offset(n0 + 16 * t, KB, lane);
+  FewWeights<NI, BPR> ring;
+  auto ask = [&](int b, int kb) { ring.ask(b, wres, woff, kb, KB, 8192, 1024); };
 #pragma unroll
   for (int b = 0; b < BPR; ++b) ask(b, wave + QE_W * b);
   __builtin_amdgcn_sched_barrier(0);
 
-  // ---- rows into LDS as codes with a scale per 128 values (sixteen lanes): positions as in q8_decode_kernel
-  auto chunk_at = [&](int kb, int r, int c) { return (uint32_t)((kb * R + r) * 128 + (((c >> 1) | ((c & 1) << 2)) ^ (r & 7)) * 16); };
+  // ---- rows into LDS as codes with a scale per 128 values (sixteen lanes)
   float* const xs_l = (float*)(lds + (size_t)R * K);         // [row][K block], then the columns' scales
   float* const ws_l = xs_l + R * KB;
   auto quantise = [&](int p, int first) {
@@ -122,7 +105,7 @@ q8_experts_kernel(QeArgs a) {
     const RowFp8 by(lane_group_max(mx, 16));                 // (a row is a whole number of sixteen pieces)
     const u2 codes = by.codes(y);
     if (i < total) {
-      *(u2*)(lds + chunk_at(c >> 4, r, (c & 15) >> 1) + (c & 1) * 8) = codes;
+      *(u2*)(lds + few_chunk_at(R, c >> 4, r, (c & 15) >> 1) + (c & 1) * 8) = codes;
       if ((c & 15) == 0) xs_l[r * KB + (c >> 4)] = by.scale;
     }
   };
@@ -136,7 +119,7 @@ q8_experts_kernel(QeArgs a) {
     quantise(0, first);
   }
   for (int i = tid; i < KB; i += THREADS) ws_l[i] = i == tid ? wsv : wsc[i];
-  qe_lds_barrier();
+  few_lds_barrier();
 
   // ---- K blocks wave, wave + 8, ..
   f4 acc[NI];
@@ -144,45 +127,21 @@ q8_experts_kernel(QeArgs a) {
   for (int t = 0; t < NI; ++t) acc[t] = (f4){0.f, 0.f, 0.f, 0.f};
   const int row = min(r16, R - 1);
   auto multiply = [&](int b, int kb) {
-    const u4 xo[2] = {*(const u4*)(lds + chunk_at(kb, row, 2 * q)), *(const u4*)(lds + chunk_at(kb, row, 2 * q + 1))};
+    const FewOperand x(lds, R, kb, row, q);
     const float sc = xs_l[row * KB + kb] * ws_l[kb];
 #pragma unroll
-    for (int t = 0; t < NI; ++t) {
-      f4 part = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int v = 0; v < 2; ++v) {
-        const u4 wv = w[b][t][v];
-        part = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)((unsigned long)wv[0] | ((unsigned long)wv[1] << 32)),
-                                                          (long)((unsigned long)xo[v][0] | ((unsigned long)xo[v][1] << 32)), part, 0, 0, 0);
-        part = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8((long)((unsigned long)wv[2] | ((unsigned long)wv[3] << 32)),
-                                                          (long)((unsigned long)xo[v][2] | ((unsigned long)xo[v][3] << 32)), part, 0, 0, 0);
-      }
-      acc[t] += sc * part;
-    }
+    for (int t = 0; t < NI; ++t) acc[t] += sc * few_fp8_products(ring.w[b][t], x, (f4){0.f, 0.f, 0.f, 0.f});
   };
-  const int mine = (KB - wave + QE_W - 1) / QE_W;
-  int i = 0;
-  for (; i + BPR < mine; i += BPR) {
-#pragma unroll
-    for (int b = 0; b < BPR; ++b) {
-      multiply(b, wave + QE_W * (i + b));
-      ask(b, wave + QE_W * (i + b + BPR));
-    }
-  }
-#pragma unroll
-  for (int b = 0; b < BPR; ++b)
-    if (i + b < mine) multiply(b, wave + QE_W * (i + b));
+  few_walk<BPR, QE_W>(KB, wave, multiply, ask);
 
   // ---- the wavefronts' sums, in wavefront order
-  qe_lds_barrier();                                          // everybody has read x
+  few_lds_barrier();                                          // everybody has read x
   f4* const red = (f4*)lds;
 #pragma unroll
   for (int t = 0; t < NI; ++t) red[(wave * NI + t) * 64 + lane] = acc[t];
-  qe_lds_barrier();
+  few_lds_barrier();
   if (!stores || r16 >= R) return;
-  f4 sum = red[wave * 64 + lane];
-#pragma unroll
-  for (int s = 1; s < QE_W; ++s) sum += red[(s * NI + wave) * 64 + lane];
+  const f4 sum = few_sum<QE_W>(red, NI, wave, lane);
   const int slot = slot_of[r16];
   const float rw = a.topk_weights ? a.topk_weights[slot] : 1.0f;
   u2 o;
