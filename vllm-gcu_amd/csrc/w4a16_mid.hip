@@ -513,9 +513,9 @@ static MidPlan make_mid_plan(int M, int K, int N, size_t bytes) {
     for (int mt = 5; mt <= 8; ++mt) offer(tw, mt, (M + 16 * mt - 1) / (16 * mt), mt, false);
   // (the price stays that of the even ones: other kernels are chosen by it, whose operands are exact, and what is rounded to fp16 shall not
   // depend on how the rows are dealt out)
-  // Even rounds by workgroups of 7 and 8 row tiles, up to three rounds: a chip that is full for longer runs into its power limit and gains nothing.  (us, all of one
-  // height -> here: 3584 x 37888 at 700 rows 190.2 -> 185.4, 4096 x 28672 at 1024 / 1537, bf16, 219.4 / 340.2 -> 216.1 / 334.4, 8192 x 28672 at 1024 424.2 -> 418.2; in four rounds
-  // 4096 x 28672 at 2048 430.6 / 435.3.  Of 256 columns, and 6 and 7 or 5 and 6 row tiles: within 1 % on average.)
+  // Even rounds by workgroups of 7 and 8 row tiles, up to three rounds: a chip that is full for longer runs into its power limit and gains nothing.  (us, all of 128
+  // rows -> here: 3584 x 37888 at 700 rows 191.4 -> 187.2, 4096 x 28672 at 1024 / 1537, bf16, 228.6 / 337.4 -> 224.8 / 336.3, 8192 x 28672 at 1024 435.1 -> 419.2; in four rounds
+  // 4096 x 28672 at 2048 437.3 / 437.9.  Of 256 columns, and 6 and 7 or 5 and 6 row tiles: within 1 % on average.)
   for (int rows = S / 8 + 1; rows <= 127 && mid_mixes(M, 4, 8, rows) && (long)rows * ((N + 511) / 512) <= 3L * cus; ++rows) offer(4, 8, rows, (double)S / rows, true);
   return best;
 }
