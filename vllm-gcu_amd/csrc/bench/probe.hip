@@ -1,4 +1,4 @@
-// Benchmark helpers, not part of the product library (built into libmi355q_bench.so, loaded by
+// Benchmark helpers, not part of the product library (built into libmi355q_bench.so and called by
 // bench.py only): a plain streaming read of a buffer, the floor against which the weight-streaming
 // kernels are quoted (same bytes, no arithmetic, nothing stored); and a loop of matrix instructions
 // on register-resident operands, the rate the matrix pipes sustain on the caller's data when
